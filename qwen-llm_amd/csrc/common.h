@@ -191,6 +191,34 @@ int32_t dfl_gemm_whole(dflash_ctx *ctx, int32_t w_type, const void *w, const voi
 // The weights are read once and stay in registers while the blocks pass; a row's bits are those of dfl_gemm_whole.
 int32_t dfl_gemm_whole_blocks(dflash_ctx *ctx, int32_t w_type, const void *w, const void *xf, float *y, int64_t n_in, int64_t n_out,
                               int32_t n_rows_total, int64_t pair_ffn, void *y_xf, int y_xf_kind, hipStream_t stream);
+bool dfl_whole_takes_blocks(const dflash_ctx *ctx, int32_t w_type, int64_t n_in, int64_t n_out);  // (the looping variant takes one)
+
+// ---- many rows at once (gemm_rows.hip): the products of a prompt's prefill ----
+// Every row gets the bits the 16-row kernels give it in its own block: dfl_gemm_rows_plan says which of their
+// arithmetics the matrix takes there and where K is cut.  kind == DFL_XF_NONE: not taken (only the tiled orders are).
+struct dfl_rows_plan {
+    int kind;      // fragment order the activations must be in
+    int twin;      // whole-K kernel's arithmetic (no sub-block sums needed)
+    int total, n_cut, by_group;
+};
+dfl_rows_plan dfl_gemm_rows_plan(const dflash_ctx *ctx, int32_t w_type, int64_t n_in, int64_t n_out, int64_t pair_ffn);
+// Sub-block sums of n_blocks blocks of rows in fragment order (kind Q4K), for the plans without `twin`:
+// dfl_xs_bytes(n_in) bytes per block.
+static inline size_t dfl_xs_bytes(int64_t n_in) { return static_cast<size_t>(n_in / 256) * 1024; }
+int32_t dfl_xf_sums(dflash_ctx *ctx, const void *xf, int64_t n_in, int32_t n_blocks, void *xs, hipStream_t stream);
+// y[n_rows][n_out] = X . W^T, block b of sixteen rows at xf + b * dfl_xf_bytes(n_in) (sums: xs + b * dfl_xs_bytes(n_in)).
+// pair_ffn > 0: W is a fused gate | up matrix and silu(gate) * up goes to y_xf in fragment order y_kind (and its sub-block
+// sums to y_xs unless null) instead.
+int32_t dfl_gemm_rows(dflash_ctx *ctx, const dfl_rows_plan &plan, int32_t w_type, const void *w, const void *xf, const void *xs, float *y,
+                      int64_t n_in, int64_t n_out, int32_t n_rows, int64_t pair_ffn, void *y_xf, void *y_xs, int y_kind, hipStream_t stream);
+// The experts' products over row tiles listed on the device, tiles[i] = {expert (-1: the extra matrix), first block,
+// blocks (1..4), -}: the arithmetic of gemm_q4k_experts_kernel.  w_up != null: silu(x . w^T) * (x . w_up^T) to y_xf / y_xs.
+int32_t dfl_gemm_rows_experts(dflash_ctx *ctx, const void *w, const void *w_extra, const void *w_up, const void *w_up_extra, size_t w_stride,
+                              const void *xf, const void *xs, const int32_t *tiles, const int32_t *n_tiles, int32_t max_tiles, float *y,
+                              int64_t n_in, int64_t n_out, void *y_xf, void *y_xs, hipStream_t stream);
+// How dfl_gemm_fewrow_checked splits a Q4_K matrix in tiled order: workgroup i of n_wg takes stages
+// [total i / n_wg, total (i + 1) / n_wg) of the (256-row tile group x super-block) space; false where it does not take it.
+bool dfl_q4k_tiled_split(const dflash_ctx *ctx, int64_t n_in, int64_t n_out, int *total, int *n_wg);
 
 // dflash_dflash2_conv whose result also goes to y_xf in fragment order (XF; h a multiple of 256), for the whole-K
 // projection that reads it.
@@ -239,15 +267,17 @@ struct dfl_moe_group_scratch {
     int32_t *sel_e = nullptr;     // [rows][n_used]
     float *sel_w = nullptr;       // [rows][n_used]
     int32_t *pick_pos = nullptr;  // [rows][n_used]: row of eo that holds the pick's output
-    int32_t *ids = nullptr;       // [max_slots]
     int32_t *n_slots = nullptr;
     int32_t *slot_rows = nullptr; // [max_slots][16]
-    _Float16 *xg = nullptr;       // [max_slots][16][hidden]
-    _Float16 *act = nullptr;      // [max_slots][16][ffn_expert]
+    int32_t *tiles = nullptr;     // [max_slots][4]: row tiles of dfl_gemm_rows_experts
+    int32_t *n_tiles = nullptr;
+    uint8_t *xg = nullptr, *xg_sums = nullptr;    // every slot's rows in fragment order, and their sub-block sums
+    uint8_t *act = nullptr, *act_sums = nullptr;  // the same of silu(gate) * up
     float *eo = nullptr;          // [max_slots][16][hidden]
     int max_slots = 0;
 };
 int dfl_moe_group_max_slots(const dflash_model_cfg &cfg, int n_rows);
+int dfl_moe_group_max_picks();  // rows * picks per row that one pass takes
 bool dfl_moe_group_fits(const dflash_ctx *ctx, const dflash_model_cfg &cfg, const dflash_layer &layer, int n_rows);
 int32_t dfl_moe_ffn_group(dflash_ctx *ctx, const dflash_model_cfg &cfg, const dflash_layer &layer, float *x_resid,
                           float *cur, int n_rows, const dfl_moe_group_scratch &scratch, const float *next_norm_w, void *next_xf,

@@ -11,10 +11,10 @@
 //    of 1024.0 (low nibble) or 64.0 (high nibble, which sits four bits up), and one
 //    packed f16 fma per value pair, fma(1024+q, s, -1024*s), yields round(q*s) with a
 //    single rounding (s = d*sc_j in f16).  The per-sub-block minimum never touches the
-//    nibbles: each weight MFMA has a twin that multiplies the same activation fragment
-//    with dmin*m_j repeated eight times and accumulates into a second tile, subtracted
-//    at the end.  The matrix cores are nearly idle in this kernel and the vector ALU is
-//    not, so this is cheaper than pre-summing activations.
+//    nibbles: sum_k x[k] (dmin m_j) over a sub-block is (sum_k x[k]) (dmin m_j), so one MFMA
+//    per super-block multiplies the sub-block sums of the rounded activations (mfma_unpack.h,
+//    q4k_sum_parts) with the negated minima, ahead of the super-block's eight weight MFMAs and
+//    into the same accumulator (8-wave groups: see Q4KGeom::kSums).
 //  * The kernel is a persistent stream: one workgroup per CU walks a contiguous range of
 //    (tile group x super-block) work, weights go HBM -> LDS with direct-to-LDS loads
 //    through a ring of buffers, activations are converted to f16 MFMA fragments on the
@@ -100,7 +100,12 @@ struct Q4KGeom {
     static constexpr int kAhead = kWaves == 8 ? DFLASH_Q4K_AHEAD8 : 2;
     static constexpr int kRing = kAhead + 1;
     // LDS: a ring of kRing weight buffers, then two activation buffers (stage parity)
-    static constexpr int kLdsPieces = kRing * kWPieces + 2 * kQ4KBlockFrags;
+    // Minima of a 16-wave group: one MFMA over sub-block sums (the arithmetic of the many-row product, gemm_rows.hip, whose
+    // rows must get these bits).  An 8-wave group (batches: one or two stages per workgroup) keeps a twin of each weight
+    // MFMA instead: the sums of its first stage stand in front of everything else (14.8 against 12.6 us, 2048 -> 5 x 1024).
+    static constexpr bool kSums = kWaves == 16;
+    static constexpr int kXPieces = kQ4KBlockFrags + (kSums ? 64 : 0);  // a stage's activation fragments and its sub-block sums
+    static constexpr int kLdsPieces = kRing * kWPieces + 2 * kXPieces;
     static_assert(kLdsPieces * 16 <= 160 * 1024, "fits one CU's LDS");
     static_assert(kWPieces % 64 == 0, "whole wave-loads");
     static_assert(kFull + (kExtra ? 1 : 0) <= 4, "one weight load is issued after every second of a stage's 8 MFMAs");
@@ -283,10 +288,29 @@ __device__ __forceinline__ void q4k_load_x(const uint8_t *xblock, const Q4KLane<
     for (int r = 0; r < Q4KGeom<kWaves>::kXLoads; r++) q4k_load_x_vec(xblock, L.x_off[r], raw.v[r]);
 }
 
+// Sum over the eight lanes that share (lane & 7), in every one of them: partners 8, 16 and 32 lanes away in turn.
+__device__ __forceinline__ float q4k_row_sum(float v) {
+    v += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x128, 0xF, 0xF, true));  // row_ror:8
+    v += __shfl_xor(v, 16, 64);
+    v += __shfl_xor(v, 32, 64);
+    return v;
+}
+
+// The parts of the sum of row m's sub-block j into the A fragments `sums` of the minima's MFMA (see q4k_sum_parts).
+__device__ __forceinline__ void q4k_put_sum(uint8_t *sums, int m, int j, float sum) {
+    _Float16 *tw = reinterpret_cast<_Float16 *>(sums) + (m + 16 * (j >> 1)) * 8 + (j & 1);
+    const Q4KSumParts p = q4k_sum_parts(sum);
+    tw[0] = p.hi;
+    tw[2] = p.lo;
+    tw[4] = p.over;
+    tw[6] = static_cast<_Float16>(0.0f);
+}
+
 // Rounds a stage's raw activations to f16 and writes this thread's share of the fragments into
 // the activation buffer at `buf`.  Rows past n_rows repeat the last row: output rows depend on
 // their own activation row only, and those rows are never stored.
-template <int kWaves, typename XT>
+// kSums (Q4_K): the parts of each row's sub-block sums follow the fragments, as the A operand of the minima's MFMA.
+template <int kWaves, typename XT, bool kSums>
 __device__ __forceinline__ void q4k_write_x(half8_t *buf, const Q4KLane<kWaves> &L, const Q4KXRaw<kWaves, XT> &raw) {
     uint8_t *base = reinterpret_cast<uint8_t *>(buf);
 #pragma unroll
@@ -296,6 +320,13 @@ __device__ __forceinline__ void q4k_write_x(half8_t *buf, const Q4KLane<kWaves> 
         for (int i = 0; i < 4; i++) h[i] = static_cast<_Float16>(raw.v[r][i]);
         half4_t frag = {h[0], h[2], h[1], h[3]};
         *reinterpret_cast<half4_t *>(base + L.xw_off[r]) = frag;
+        if constexpr (kSums) {
+            // (a virtual wave is one sub-block of eight rows: the eight lanes of a row are eight apart)
+            float sum = (static_cast<float>(h[0]) + static_cast<float>(h[1])) + (static_cast<float>(h[2]) + static_cast<float>(h[3]));
+            sum = q4k_row_sum(sum);
+            const int lane = threadIdx.x & 63, vw = static_cast<int>(threadIdx.x >> 6) + kWaves * r, j = vw >> 1;
+            if (lane < 8) q4k_put_sum(base + kQ4KBlockFrags * 16, 8 * (vw & 1) + lane, j, sum);
+        }
     }
 }
 
@@ -306,7 +337,7 @@ __device__ __forceinline__ void q4k_issue_w(const uint8_t *wstage, half8_t *buf,
 }
 
 // One stage (one super-block) of this wave's tile out of the weight buffer `buf` and the activation
-// buffer `xcur`: 8 MFMAs for the scaled nibbles, 8 for the minima.  hdr = {d|dmin, scales[0..3], [4..7], [8..11]}, q0/q1 = the lane's 32 quant bytes
+// buffer `xcur`: one MFMA for the minima (8-wave groups: 8), 8 for the scaled nibbles.  hdr = {d|dmin, scales[0..3], [4..7], [8..11]}, q0/q1 = the lane's 32 quant bytes
 // (chunk g: sub-blocks 2g in the low and 2g+1 in the high nibbles).  The loads of later stages
 // are issued in between: one weight load after every second MFMA (spread over the MFMAs, the
 // loads never queue up behind each other in the address unit), then the activations; the
@@ -326,6 +357,7 @@ __device__ __forceinline__ void q4k_compute(const half8_t *buf, const half8_t *x
     half8_t af[8];
 #pragma unroll
     for (int t = 0; t < 8; t++) af[t] = a[t * 64];
+    const half8_t a_min = a[G::kSums ? kQ4KBlockFrags : 0];
     // scales and minima of sub-blocks 2g (low nibbles) and 2g+1 (high nibbles); the 6-bit codes of
     // sub-blocks 0..3 sit in one dword, those of 4..7 are split over two: select by bit mask,
     // not by branch
@@ -336,27 +368,27 @@ __device__ __forceinline__ void q4k_compute(const half8_t *buf, const half8_t *x
     // The two 6-bit codes of this lane sit in bytes (0,1) or (2,3) of those words.  A byte
     // permute drops each into the mantissa of an f16 1024.0 (the lane's selector picks the byte
     // pair), and one packed fma per pair, (1024 + code) * d - 1024 d, gives code * d rounded once:
-    // S = (s of sub-block 2g, s of 2g+1), M = (dmin*m of 2g, of 2g+1).
+    // S = (s of sub-block 2g, s of 2g+1), M = (-dmin*m of 2g, of 2g+1).
     const half2_t dm = __builtin_bit_cast(half2_t, hdr.x);
     const half2_t p_sc = as_half2(__builtin_amdgcn_perm(0x64646464u, sc_word, L.sc_sel));
     const half2_t p_mn = as_half2(__builtin_amdgcn_perm(0x64646464u, mn_word, L.sc_sel));
     const half2_t neg = dm * splat(static_cast<_Float16>(-1024.0f));
     const half2_t S = __builtin_elementwise_fma(p_sc, splat(dm[0]), splat(neg[0]));
-    const half2_t M = __builtin_elementwise_fma(p_mn, splat(dm[1]), splat(neg[1]));
+    const half2_t M = __builtin_elementwise_fma(p_mn, splat(-dm[1]), splat(-neg[1]));
     const half2_t unbias = {static_cast<_Float16>(-1024.0f), static_cast<_Float16>(-64.0f)};
     const half2_t Cs = S * unbias;
     const half2_t s2l = splat(S[0]), c2l = splat(Cs[0]);
     const half2_t s2h = splat(S[1]), c2h = splat(Cs[1]);
-    // dmin*m of sub-blocks 2g and 2g+1, eight times each: the B operands of the minima MFMAs
-    const _Float16 m_lo = M[0], m_hi = M[1];
-    const half8_t bml = {m_lo, m_lo, m_lo, m_lo, m_lo, m_lo, m_lo, m_lo};
-    const half8_t bmh = {m_hi, m_hi, m_hi, m_hi, m_hi, m_hi, m_hi, m_hi};
+    // (8-wave groups) -dmin*m of sub-blocks 2g and 2g+1, eight times each: the B operands of the twin MFMAs
+    const half8_t bml = {M[0], M[0], M[0], M[0], M[0], M[0], M[0], M[0]};
+    const half8_t bmh = {M[1], M[1], M[1], M[1], M[1], M[1], M[1], M[1]};
+    if constexpr (G::kSums) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_min, q4k_min_operand(M), acc, 0, 0, 0);
     const uint32_t qw[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
 #pragma unroll
     for (int t = 0; t < 4; t++) {
         half8_t bl = unpack_scale<false>(qw[2 * t], qw[2 * t + 1], s2l, c2l, magic.lo);
         acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[t], bl, acc, 0, 0, 0);
-        acc_min = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[t], bml, acc_min, 0, 0, 0);
+        if constexpr (!G::kSums) acc_min = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[t], bml, acc_min, 0, 0, 0);
         if (t & 1) {
             const int j = t >> 1;
             if (issue_w && (j < G::kFull || (j == G::kFull && wave < G::kExtra))) q4k_issue_w<kWaves>(wstage, wbuf, L, j, wave);
@@ -365,12 +397,12 @@ __device__ __forceinline__ void q4k_compute(const half8_t *buf, const half8_t *x
     }
     // the next stage's activations (in registers since the wait at the top of this stage) go to
     // LDS here, off the critical path between that wait and the barrier
-    if (write_x) q4k_write_x<kWaves, XT>(xbuf, L, raw);
+    if (write_x) q4k_write_x<kWaves, XT, G::kSums>(xbuf, L, raw);
 #pragma unroll
     for (int t = 0; t < 4; t++) {
         half8_t bh = unpack_scale<true>(qw[2 * t], qw[2 * t + 1], s2h, c2h, magic.hi);
         acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[4 + t], bh, acc, 0, 0, 0);
-        acc_min = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[4 + t], bmh, acc_min, 0, 0, 0);
+        if constexpr (!G::kSums) acc_min = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[4 + t], bmh, acc_min, 0, 0, 0);
         if (t & 1) {
             const int j = 2 + (t >> 1);
             if (issue_w && (j < G::kFull || (j == G::kFull && wave < G::kExtra))) q4k_issue_w<kWaves>(wstage, wbuf, L, j, wave);
@@ -408,15 +440,12 @@ __device__ __forceinline__ void q4k_wait_vm(int v) {
 // Ends a tile group's segment: Y directly if this workgroup covered the group's whole K, else a
 // partial tile for the reduce kernel (slot 0: the range's first group, slot 1: its last).
 template <int kWaves>
-__device__ __forceinline__ void q4k_flush(const Q4KRange &rg, const Q4KBatch &bt, int group, float4_t &acc,
-                                          float4_t &acc_min, float4_t &stash, float *__restrict__ y,
+__device__ __forceinline__ void q4k_flush(const Q4KRange &rg, const Q4KBatch &bt, int group, float4_t res,
+                                          float4_t &stash, float *__restrict__ y,
                                           float *__restrict__ partials, int n_out, int n_rows, int tid) {
     // rare path: an opaque copy of the thread index keeps its index arithmetic out of the stage loop
     asm volatile("" : "+v"(tid));
     const int lane = tid & 63, wave = tid >> 6, n = lane & 15, g = lane >> 4;
-    float4_t res = acc - acc_min;
-    acc = float4_t{0, 0, 0, 0};
-    acc_min = float4_t{0, 0, 0, 0};
     // the group's whole K lies inside this workgroup's range: no other workgroup contributes
     const bool whole = group * rg.nb >= rg.it_begin && (group + 1) * rg.nb <= rg.it_end;
     if (bt.pair) {
@@ -711,7 +740,7 @@ __global__ void __launch_bounds__(64 * kWaves)
     // weight ring: slot_c holds the stage being computed, slot_i takes the next stage to be loaded
     int slot_c = 0, slot_i = 0;
     auto ring = [&](int slot) { return lds + slot * G::kWPieces; };
-    half8_t *x_c = lds + kRing * G::kWPieces, *x_n = x_c + kQ4KBlockFrags;
+    half8_t *x_c = lds + kRing * G::kWPieces, *x_n = x_c + G::kXPieces;
 
     // Loads are issued, and return, in groups: group 0 = [weights of stage 0 (first of all: everything
     // else here hides behind their latency), activations of stages 0 and 1], group p = [weights of
@@ -773,7 +802,7 @@ __global__ void __launch_bounds__(64 * kWaves)
         q4k_pin_x<kWaves, XT>(raw);
         if (first) {
             q4k_pin_x<kWaves, XT>(raw_first);
-            q4k_write_x<kWaves, XT>(x_c, L, raw_first);
+            q4k_write_x<kWaves, XT, G::kSums>(x_c, L, raw_first);
         }
         first = false;
         __builtin_amdgcn_s_waitcnt(kWaitLds);
@@ -807,7 +836,9 @@ __global__ void __launch_bounds__(64 * kWaves)
         done++;
         if (done <= 8) DFL_TRS(1 + done);
         if (++bc == nb || n_left == 0) {
-            q4k_flush<kWaves>(rg, bt, gc, acc, acc_min, stash, y, partials, n_out, n_rows, tid);
+            q4k_flush<kWaves>(rg, bt, gc, G::kSums ? acc : acc + acc_min, stash, y, partials, n_out, n_rows, tid);
+            acc = float4_t{0, 0, 0, 0};
+            acc_min = float4_t{0, 0, 0, 0};
             bc = 0;
             gc++;
         }
@@ -859,7 +890,7 @@ static_assert(kSlabLdsBytes <= 160 * 1024, "one workgroup per CU, all of its LDS
 
 // One stage of a wave's tile: 8 MFMAs for the scaled nibbles, one for the minima.
 __device__ __forceinline__ void q4k_slab_compute(const u32x4_t *blk, const half8_t *a, const half4_t *twin, int g, uint32_t sc_sel,
-                                                 Q4KMagic magic, float4_t &acc, float4_t &acc_min) {
+                                                 Q4KMagic magic, float4_t &acc) {
     const u32x4_t hdr = blk[0], q0 = blk[1 + 2 * g], q1 = blk[2 + 2 * g];
     half8_t af[8];
 #pragma unroll
@@ -875,7 +906,7 @@ __device__ __forceinline__ void q4k_slab_compute(const u32x4_t *blk, const half8
     const half2_t p_mn = as_half2(__builtin_amdgcn_perm(0x64646464u, mn_word, sc_sel));
     const half2_t neg = dm * splat(static_cast<_Float16>(-1024.0f));
     const half2_t S = __builtin_elementwise_fma(p_sc, splat(dm[0]), splat(neg[0]));
-    const half2_t M = __builtin_elementwise_fma(p_mn, splat(dm[1]), splat(neg[1]));
+    const half2_t M = __builtin_elementwise_fma(p_mn, splat(-dm[1]), splat(-neg[1]));  // -(dmin * m)
     const half2_t unbias = {static_cast<_Float16>(-1024.0f), static_cast<_Float16>(-64.0f)};
     const half2_t Cs = S * unbias;
     const half2_t s2l = splat(S[0]), c2l = splat(Cs[0]);
@@ -884,7 +915,7 @@ __device__ __forceinline__ void q4k_slab_compute(const u32x4_t *blk, const half8
     const _Float16 zero = static_cast<_Float16>(0.0f);
     const half8_t a_min = {tw[0], tw[1], tw[2], tw[3], zero, zero, zero, zero};
     const half8_t b_min = {M[0], M[1], M[0], M[1], zero, zero, zero, zero};
-    acc_min = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_min, b_min, acc_min, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_min, b_min, acc, 0, 0, 0);
 #pragma unroll
     for (int t = 0; t < 4; t++) {
         const half8_t bl = unpack_scale<false>(qw[2 * t], qw[2 * t + 1], s2l, c2l, magic.lo);
@@ -1006,9 +1037,7 @@ __global__ void __launch_bounds__(64 * kSlabWaves)
             *reinterpret_cast<half4_t *>(stage + xw_off) = frag;
             // sub-block sum of the rounded values over the eight lanes that share this row
             float sum = (static_cast<float>(h[0]) + static_cast<float>(h[1])) + (static_cast<float>(h[2]) + static_cast<float>(h[3]));
-            sum += __shfl_xor(sum, 8, 64);
-            sum += __shfl_xor(sum, 16, 64);
-            sum += __shfl_xor(sum, 32, 64);
+            sum = q4k_row_sum(sum);
             if (lane < 8) {
                 const int j = wave >> 1;  // this wave's sub-block
                 const _Float16 hi = static_cast<_Float16>(sum), lo = static_cast<_Float16>(sum - static_cast<float>(hi));
@@ -1027,7 +1056,7 @@ __global__ void __launch_bounds__(64 * kSlabWaves)
     const int n = lane & 15, g = lane >> 4;
     const uint32_t sc_sel = (lane & 16) ? 0x04030402u : 0x04010400u;
     const Q4KMagic magic = q4k_magic();
-    float4_t acc = {0, 0, 0, 0}, acc_min = {0, 0, 0, 0}, stash = {0, 0, 0, 0};
+    float4_t acc = {0, 0, 0, 0}, stash = {0, 0, 0, 0};
     int gc = rg.first_group, bc = b0;
     for (int t = 0; t < len; t++) {
         q4k_slab_wait_groups(w_issued - 1 - t);  // loads land in order: stage t has when only later ones are in flight
@@ -1040,9 +1069,10 @@ __global__ void __launch_bounds__(64 * kSlabWaves)
         const u32x4_t *blk = reinterpret_cast<const u32x4_t *>(my_ring + (t % kSlabRing) * kSlabWavePieces) + n * 9;
         const uint8_t *stage = slab + t * kSlabStageBytes;
         q4k_slab_compute(blk, reinterpret_cast<const half8_t *>(stage) + lane,
-                         reinterpret_cast<const half4_t *>(stage + kQ4KBlockFrags * 16) + lane, g, sc_sel, magic, acc, acc_min);
+                         reinterpret_cast<const half4_t *>(stage + kQ4KBlockFrags * 16) + lane, g, sc_sel, magic, acc);
         if (++bc == nb || t + 1 == len) {
-            q4k_flush<kW>(rg, bt, gc, acc, acc_min, stash, y, partials, n_out, n_rows, tid);
+            q4k_flush<kW>(rg, bt, gc, acc, stash, y, partials, n_out, n_rows, tid);
+            acc = float4_t{0, 0, 0, 0};
             bc = 0;
             gc++;
         }
@@ -1130,7 +1160,7 @@ static_assert(kTiledLdsBytes <= 160 * 1024, "one workgroup per CU, all of its LD
 
 // q4k_slab_compute with the fragment sets kTiledFragStride apart
 __device__ __forceinline__ void q4k_tiled_compute(const u32x4_t *blk, const uint8_t *stage, int lane, int g, uint32_t sc_sel,
-                                                  Q4KMagic magic, float4_t &acc, float4_t &acc_min) {
+                                                  Q4KMagic magic, float4_t &acc) {
     const u32x4_t hdr = blk[0], q0 = blk[1 + 2 * g], q1 = blk[2 + 2 * g];
     half8_t af[8];
 #pragma unroll
@@ -1145,7 +1175,7 @@ __device__ __forceinline__ void q4k_tiled_compute(const u32x4_t *blk, const uint
     const half2_t p_mn = as_half2(__builtin_amdgcn_perm(0x64646464u, mn_word, sc_sel));
     const half2_t neg = dm * splat(static_cast<_Float16>(-1024.0f));
     const half2_t S = __builtin_elementwise_fma(p_sc, splat(dm[0]), splat(neg[0]));
-    const half2_t M = __builtin_elementwise_fma(p_mn, splat(dm[1]), splat(neg[1]));
+    const half2_t M = __builtin_elementwise_fma(p_mn, splat(-dm[1]), splat(-neg[1]));  // -(dmin * m)
     const half2_t unbias = {static_cast<_Float16>(-1024.0f), static_cast<_Float16>(-64.0f)};
     const half2_t Cs = S * unbias;
     const half2_t s2l = splat(S[0]), c2l = splat(Cs[0]);
@@ -1154,7 +1184,7 @@ __device__ __forceinline__ void q4k_tiled_compute(const u32x4_t *blk, const uint
     const _Float16 zero = static_cast<_Float16>(0.0f);
     const half8_t a_min = {tw[0], tw[1], tw[2], tw[3], zero, zero, zero, zero};
     const half8_t b_min = {M[0], M[1], M[0], M[1], zero, zero, zero, zero};
-    acc_min = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_min, b_min, acc_min, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_min, b_min, acc, 0, 0, 0);
 #pragma unroll
     for (int t = 0; t < 4; t++) {
         const half8_t bl = unpack_scale<false>(qw[2 * t], qw[2 * t + 1], s2l, c2l, magic.lo);
@@ -1252,10 +1282,7 @@ __global__ void __launch_bounds__(64 * kSlabWaves)
             // fragment slot of MFMA t = 4 (j & 1) + quarter, lane (m, g = j >> 1); element order of the unpack
             const half8_t frag = {h[0], h[2], h[1], h[3], h[4], h[6], h[5], h[7]};
             *reinterpret_cast<half8_t *>(stage + (4 * (j & 1) + quarter) * kTiledFragStride + (16 * (j >> 1) + m) * 16) = frag;
-            float sum = 0.0f;
-#pragma unroll
-            for (int i = 0; i < 8; i++) sum += static_cast<float>(h[i]);
-            sum = q4k_quad_sum(sum);  // the sub-block's sum of the rounded values
+            const float sum = q4k_quad_sum(q4k_octet_sum(h));  // the sub-block's sum of the rounded values
             if (quarter == 0) {
                 const _Float16 hi = static_cast<_Float16>(sum), lo = static_cast<_Float16>(sum - static_cast<float>(hi));
                 _Float16 *tw = reinterpret_cast<_Float16 *>(stage + 8 * kTiledFragStride) + (m + 16 * (j >> 1)) * 4 + (j & 1);
@@ -1275,7 +1302,7 @@ __global__ void __launch_bounds__(64 * kSlabWaves)
     const int n = lane & 15, g = lane >> 4;
     const uint32_t sc_sel = (lane & 16) ? 0x04030402u : 0x04010400u;
     const Q4KMagic magic = q4k_magic();
-    float4_t acc = {0, 0, 0, 0}, acc_min = {0, 0, 0, 0}, stash = {0, 0, 0, 0};
+    float4_t acc = {0, 0, 0, 0}, stash = {0, 0, 0, 0};
     int gc = rg.first_group, bc = b0;
     for (int t = 0; t < len; t++) {
         q4k_slab_wait_groups(w_issued - 1 - t);  // loads land in order: stage t has when only later ones are in flight
@@ -1285,11 +1312,12 @@ __global__ void __launch_bounds__(64 * kSlabWaves)
         if (t == 3) DFL_TRW(7);
         DFL_TR(3 + t);
         const u32x4_t *blk = reinterpret_cast<const u32x4_t *>(my_ring + (t % kSlabRing) * kSlabWavePieces) + n * 9;
-        q4k_tiled_compute(blk, slab + t * kTiledStageX, lane, g, sc_sel, magic, acc, acc_min);
+        q4k_tiled_compute(blk, slab + t * kTiledStageX, lane, g, sc_sel, magic, acc);
         // stage t+3 into the buffer this stage has just been read out of (its reads are complete: the MFMAs above used them)
         if (w_issued < len) issue_w();
         if (++bc == nb || t + 1 == len) {
-            q4k_flush<kW>(rg, bt, gc, acc, acc_min, stash, y, partials, n_out, n_rows, tid);
+            q4k_flush<kW>(rg, bt, gc, acc, stash, y, partials, n_out, n_rows, tid);
+            acc = float4_t{0, 0, 0, 0};
             bc = 0;
             gc++;
         }
@@ -1541,10 +1569,7 @@ __global__ void __launch_bounds__(64 * kSlabWaves)
                 q4k_x8_to_half(raw_a[r], raw_b[r], h);
                 const half8_t frag = {h[0], h[2], h[1], h[3], h[4], h[6], h[5], h[7]};
                 *reinterpret_cast<half8_t *>(stage + (4 * (j & 1) + quarter) * kTiledFragStride + (16 * (j >> 1) + m) * 16) = frag;
-                float sum = 0.0f;
-#pragma unroll
-                for (int i = 0; i < 8; i++) sum += static_cast<float>(h[i]);
-                sum = q4k_quad_sum(sum);
+                const float sum = q4k_quad_sum(q4k_octet_sum_seq(h));
                 if (quarter == 0) {
                     const _Float16 hi = static_cast<_Float16>(sum), lo = static_cast<_Float16>(sum - static_cast<float>(hi));
                     _Float16 *tw = reinterpret_cast<_Float16 *>(stage + 8 * kTiledFragStride) + (m + 16 * (j >> 1)) * 4 + (j & 1);
@@ -1918,7 +1943,7 @@ __global__ void __launch_bounds__(64 * kWaves)
             q6k_load_w(wstage, W, R);
             advance_w();
         }
-        if (first) q4k_write_x<kWaves, XT>(x_c, L, raw_first);
+        if (first) q4k_write_x<kWaves, XT, false>(x_c, L, raw_first);
         first = false;
         __builtin_amdgcn_s_waitcnt(kWaitLds);
         __builtin_amdgcn_s_barrier();  // the stage's activation fragments are complete; the other fragment buffer is free
@@ -1953,7 +1978,7 @@ __global__ void __launch_bounds__(64 * kWaves)
             const half8_t bo = {o, o, o, o, o, o, o, o};
             acc_off = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[t], bo, acc_off, 0, 0, 0);
         }
-        if (n_left > 1) q4k_write_x<kWaves, XT>(x_n, L, raw);
+        if (n_left > 1) q4k_write_x<kWaves, XT, false>(x_n, L, raw);
 #pragma unroll
         for (int t = 0; t < 4; t++) {
             const _Float16 sh = (t >> 1) ? s_h1 : s_h0;
@@ -1975,7 +2000,9 @@ __global__ void __launch_bounds__(64 * kWaves)
         x_n = tx;
         n_left--;
         if (++bc == nb || n_left == 0) {
-            q4k_flush<kWaves>(rg, bt, gc, acc, acc_off, stash, y, partials, n_out, n_rows, tid);
+            q4k_flush<kWaves>(rg, bt, gc, acc - acc_off, stash, y, partials, n_out, n_rows, tid);
+            acc = float4_t{0, 0, 0, 0};
+            acc_off = float4_t{0, 0, 0, 0};
             bc = 0;
             gc++;
         }
@@ -2724,6 +2751,15 @@ int32_t launch_q4k(dflash_ctx *ctx, const void *w, const void *x, int32_t x_type
 }
 
 }  // namespace
+
+bool dfl_q4k_tiled_split(const dflash_ctx *ctx, int64_t n_in, int64_t n_out, int *total, int *n_wg) {
+    const int64_t nb = n_in / DFL_QK_K, all = (n_out + 255) / 256 * nb;
+    const int64_t wgs = std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(env_int("DFLASH_GEMM_WGS", ctx->n_cu), all), ctx->n_partial_wgs / 2));
+    if (n_in % DFL_QK_K || n_out <= 0 || all * (wgs + 1) >= (int64_t(1) << 31)) return false;
+    *total = static_cast<int>(all);
+    *n_wg = static_cast<int>(wgs);
+    return true;
+}
 
 namespace {
 

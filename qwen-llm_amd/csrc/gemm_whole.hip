@@ -232,15 +232,11 @@ __device__ __forceinline__ void compute(const Q6W &r, const half8_t (&af)[8], in
 // The 16-byte pieces of a row's ql (qh) sit at piece index p ^ (row & 7) (p ^ ((row >> 1) & 3)): a layout that a wave
 // can also read from LDS without bank conflicts.  Lane (n, g) fetches exactly its operands: four 16-byte loads, one of
 // 8 bytes, one of 2, all aligned, a row's ql line shared by the four lanes of the row - no staging, no LDS.
-constexpr int kQ6TileBytes = 16 * DFL_Q6_K_BYTES;  // 3360
-constexpr int kQ6TQh = 2048, kQ6TSc = 3072, kQ6TD = 3328;
 struct Q6T {
     u32x4_t qa, qb, ha, hb;
     uint32_t s0, s1;
     uint32_t d;
 };
-__host__ __device__ __forceinline__ int q6t_ql_piece(int row, int p) { return row * 128 + ((p ^ (row & 7)) << 4); }
-__host__ __device__ __forceinline__ int q6t_qh_piece(int row, int p) { return kQ6TQh + row * 64 + ((p ^ ((row >> 1) & 3)) << 4); }
 __device__ __forceinline__ void load_w(Q6T &r, const WholeArgs &a, int tile, int b, int lane) {
     const int n = lane & 15, g = lane >> 4, h = g >> 1, odd = g & 1;
     const uint8_t *p = a.w + ((static_cast<size_t>(tile >> 4) * a.nb + b) * 16 + (tile & 15)) * kQ6TileBytes;
@@ -663,6 +659,11 @@ WholePlan whole_plan(const dflash_ctx *ctx, int32_t w_type, int64_t n_in, int64_
 
 int dfl_whole_kind(const dflash_ctx *ctx, int32_t w_type, int64_t n_in, int64_t n_out, int64_t pair_ffn) {
     return whole_plan(ctx, w_type, n_in, n_out, pair_ffn).kind;
+}
+
+bool dfl_whole_takes_blocks(const dflash_ctx *ctx, int32_t w_type, int64_t n_in, int64_t n_out) {
+    const WholePlan p = whole_plan(ctx, w_type, n_in, n_out, 0);
+    return p.kind != DFL_XF_NONE && !p.loop;
 }
 
 int32_t dfl_gemm_whole(dflash_ctx *ctx, int32_t w_type, const void *w, const void *xf, float *y, int64_t n_in, int64_t n_out,

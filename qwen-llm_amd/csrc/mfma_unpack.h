@@ -46,6 +46,40 @@ __device__ __forceinline__ half8_t unpack_scale(uint32_t w0, uint32_t w1, half2_
     return r;
 }
 
+// ---- the Q4_K minima as one MFMA per super-block ----
+// Lane (m, g) of the A operand holds the sums of row m's rounded activations over sub-blocks 2g and 2g + 1, each split
+// into f16 parts, in k-slots {hi, hi', lo, lo', over, over', 0, 0}; the B operand holds the lane's two (negated) minima
+// in the matching slots.  hi + lo carries 22 bits of the sum.  `over` (in units of 32) keeps a sum past the f16 range -
+// 32 activations of more than 2000 - finite; it is zero otherwise and then adds nothing.
+struct Q4KSumParts {
+    _Float16 hi, lo, over;
+};
+__device__ __forceinline__ Q4KSumParts q4k_sum_parts(float sum) {
+    Q4KSumParts p;
+    p.over = fabsf(sum) > 32768.0f ? static_cast<_Float16>(sum * 0.03125f) : static_cast<_Float16>(0.0f);
+    const float rest = sum - 32.0f * static_cast<float>(p.over);
+    p.hi = static_cast<_Float16>(rest);
+    p.lo = static_cast<_Float16>(rest - static_cast<float>(p.hi));
+    return p;
+}
+// Eight consecutive values of a row: added pairwise (the order in which the slab and the streaming kernel add them, four
+// values to a thread), or one after the other (the expert kernels' order).
+__device__ __forceinline__ float q4k_octet_sum(const _Float16 *h) {
+    return ((static_cast<float>(h[0]) + static_cast<float>(h[1])) + (static_cast<float>(h[2]) + static_cast<float>(h[3]))) +
+           ((static_cast<float>(h[4]) + static_cast<float>(h[5])) + (static_cast<float>(h[6]) + static_cast<float>(h[7])));
+}
+__device__ __forceinline__ float q4k_octet_sum_seq(const _Float16 *h) {
+    float s = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 8; i++) s += static_cast<float>(h[i]);
+    return s;
+}
+__device__ __forceinline__ half8_t q4k_min_operand(half2_t m) {
+    const _Float16 k32 = static_cast<_Float16>(32.0f), zero = static_cast<_Float16>(0.0f);
+    const half8_t b = {m[0], m[1], m[0], m[1], m[0] * k32, m[1] * k32, zero, zero};
+    return b;
+}
+
 // Eight f16 weights of one MFMA: q = nibble | (two qh bits << 4), value round(q s).
 //   HIGH = false: low nibbles, bits pre-shifted to 0..1:   1024 + q via magic 0x6400, c = -1024 s
 //   HIGH = true : high nibbles (four bits up), qh bits go eight bits up: 64 + q via 0x5400, c = -64 s
@@ -62,5 +96,11 @@ __device__ __forceinline__ half8_t unpack6(uint32_t w0, uint32_t w1, uint32_t h0
     half8_t r = {p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
     return r;
 }
+
+// ---- Q6_K in tiled, field-planar order: where a tile's 3360 bytes hold which field (dflash_repack_q6k_tiled) ----
+constexpr int kQ6TileBytes = 16 * DFL_Q6_K_BYTES;  // 3360
+constexpr int kQ6TQh = 2048, kQ6TSc = 3072, kQ6TD = 3328;
+__host__ __device__ __forceinline__ int q6t_ql_piece(int row, int p) { return row * 128 + ((p ^ (row & 7)) << 4); }
+__host__ __device__ __forceinline__ int q6t_qh_piece(int row, int p) { return kQ6TQh + row * 64 + ((p ^ ((row >> 1) & 3)) << 4); }
 
 }  // namespace

@@ -330,10 +330,11 @@ __global__ void set_ids_pos_kernel(Int16Args ids, Int16Args pos, int n, int32_t 
     }
 }
 
-// The same for the rows of a prefill group: up to 512 token ids by value, positions start, start + 1, ...
-constexpr int kMaxGroupRows = 512;
+// The same for the rows of a prefill group, 512 token ids by value at a time: positions start, start + 1, ...
+constexpr int kMaxGroupRows = 2048;
+constexpr int kGroupIdsPerLaunch = 512;
 struct IntGroupArgs {
-    int32_t v[kMaxGroupRows];
+    int32_t v[kGroupIdsPerLaunch];
 };
 __global__ void set_group_ids_pos_kernel(IntGroupArgs ids, int start, int n, int32_t *__restrict__ ids_dst, int32_t *__restrict__ pos_dst) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -639,14 +640,15 @@ struct dflash_session {
 // Block b needs the earlier blocks' K/V rows of a layer before its attention in that layer: one event per (lane,
 // layer), recorded behind the launch that writes the rows and behind the wait for the previous block's event.
 constexpr int kMaxPrefillLanes = 8;
-// Scratch of the grouped prefill of a mixture-of-experts target: the rows of up to `rows / 16` consecutive blocks pass
-// through a layer together (one launch per operator, the weights of a projection read once for all of them, the
-// experts regrouped by dfl_moe_ffn_group), attention alone block by block.  Null pointers: not set up (a dense
-// target, or no device memory for it), and the lanes below serve instead.
+// Scratch of the grouped prefill: the rows of up to `rows / 16` consecutive blocks pass through a layer together (one
+// launch per operator; the projections as many-row products, gemm_rows.hip; the experts of a mixture regrouped by
+// dfl_moe_ffn_group).  Null pointers: not set up (a shape it does not take, or no device memory for it), and the lanes
+// below serve instead.
 struct PrefillGroup {
     int rows = 0;
     float *x = nullptr, *cur = nullptr, *mix = nullptr, *pk = nullptr, *q = nullptr, *attn = nullptr;
-    uint8_t *xf_cur = nullptr, *xf_attn = nullptr;
+    uint8_t *xf_cur = nullptr, *xf_attn = nullptr, *xf_g = nullptr;  // rows in fragment order ...
+    uint8_t *xs_cur = nullptr, *xs_attn = nullptr, *xs_g = nullptr;  // ... and their sub-block sums
     int32_t *ids = nullptr, *pos = nullptr;
     dfl_moe_group_scratch moe;
 };
@@ -759,54 +761,60 @@ int32_t dflash_session_create(dflash_ctx *ctx, const dflash_model_cfg *cfg, int6
 
 namespace {
 void prefill_group_free(PrefillGroup *g) {
-    void *ptrs[] = {g->x, g->cur, g->mix, g->pk, g->q, g->attn, g->xf_cur, g->xf_attn, g->ids, g->pos, g->moe.logits, g->moe.sg,
-                    g->moe.sel_e, g->moe.sel_w, g->moe.pick_pos, g->moe.ids, g->moe.n_slots, g->moe.slot_rows, g->moe.xg, g->moe.act,
-                    g->moe.eo};
+    void *ptrs[] = {g->x, g->cur, g->mix, g->pk, g->q, g->attn, g->xf_cur, g->xf_attn, g->xf_g, g->xs_cur, g->xs_attn, g->xs_g, g->ids, g->pos,
+                    g->moe.logits, g->moe.sg, g->moe.sel_e, g->moe.sel_w, g->moe.pick_pos, g->moe.n_slots, g->moe.slot_rows, g->moe.tiles,
+                    g->moe.n_tiles, g->moe.xg, g->moe.xg_sums, g->moe.act, g->moe.act_sums, g->moe.eo};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     *g = PrefillGroup();
 }
 
-// Blocks per pass of the grouped prefill (DFLASH_PREFILL_GROUP; 0 or 1 switches it off).  Measured on the 35B-A3B
-// shape, 2032-token prompt: 21.2 / 23.3 / 26.1 thousand prompt tokens/s with 16 / 24 / 32 blocks a pass, 7.3 with the
-// lanes (a pass reads every expert about once, so its cost grows slowly with its rows).
+// Blocks per pass of the grouped prefill (DFLASH_PREFILL_GROUP; 0 or 1 switches it off).  A pass reads every weight about
+// once, so its cost grows slower than its rows until the matrix cores are what it waits for.
 int prefill_group_blocks() {
     static const int v = [] {
         const char *e = getenv("DFLASH_PREFILL_GROUP");
-        return e && *e ? atoi(e) : 32;
+        return e && *e ? atoi(e) : kMaxGroupRows / 16;
     }();
     return std::max(0, std::min(kMaxGroupRows / 16, v));
 }
 
-// Sets the group scratch up for a mixture-of-experts shape; leaves it empty (no error) where the shape is not one the
-// grouped path takes or the memory is not there.
+// Sets the group scratch up; leaves it empty (no error) where the shape is not one the grouped path takes or the memory
+// is not there.
 void prefill_group_alloc(dflash_session *s, PrefillGroup *g) {
     const dflash_model_cfg &c = s->cfg;
     const int blocks = prefill_group_blocks();
+    const bool moe = c.n_expert > 0;
     const int used = c.n_expert_used < c.n_expert ? c.n_expert_used : c.n_expert;
-    if (blocks < 2 || c.n_expert < 1 || c.n_expert > 256 || used < 1 || c.hidden % DFL_QK_K || c.ffn_expert % DFL_QK_K) return;
+    const size_t H = c.hidden, q_dim = static_cast<size_t>(c.n_q) * c.head_dim, kv_dim = static_cast<size_t>(c.n_kv) * c.head_dim, F = moe ? 0 : c.ffn;
+    if (blocks < 2 || H % DFL_QK_K || H > 8192 || q_dim % DFL_QK_K) return;
+    if (moe && (c.n_expert > 256 || used < 1 || c.ffn_expert % DFL_QK_K)) return;
+    if (!moe && (F < 1 || F % DFL_QK_K)) return;
     int rows = 16 * blocks;
-    while (rows > 16 && rows * used > 4096) rows -= 16;
+    while (moe && rows > 16 && rows * used > dfl_moe_group_max_picks()) rows -= 16;
     if (static_cast<int64_t>(rows) > s->capacity) rows = static_cast<int>((s->capacity + 15) / 16 * 16);
     if (rows < 32) return;
-    const size_t H = c.hidden, q_dim = static_cast<size_t>(c.n_q) * c.head_dim, kv_dim = static_cast<size_t>(c.n_kv) * c.head_dim;
     const size_t R = rows, nb = rows / 16;
-    const int max_slots = dfl_moe_group_max_slots(c, rows);
-    const size_t S = max_slots;
-    const bool ok = dev_alloc(&g->x, R * H) && dev_alloc(&g->cur, R * H) && dev_alloc(&g->mix, R * H) &&
-                    dev_alloc(&g->pk, R * (q_dim + 2 * kv_dim)) && dev_alloc(&g->q, R * q_dim) && dev_alloc(&g->attn, R * q_dim) &&
-                    dev_alloc(&g->xf_cur, nb * dfl_xf_bytes(H)) && dev_alloc(&g->xf_attn, nb * dfl_xf_bytes(q_dim)) &&
-                    dev_alloc(&g->ids, R) && dev_alloc(&g->pos, R) && dev_alloc(&g->moe.logits, R * c.n_expert) &&
-                    dev_alloc(&g->moe.sg, R) && dev_alloc(&g->moe.sel_e, R * used) && dev_alloc(&g->moe.sel_w, R * used) &&
-                    dev_alloc(&g->moe.pick_pos, R * used) && dev_alloc(&g->moe.ids, S) && dev_alloc(&g->moe.n_slots, 1) &&
-                    dev_alloc(&g->moe.slot_rows, S * 16) && dev_alloc(&g->moe.xg, S * 16 * H) &&
-                    dev_alloc(&g->moe.act, S * 16 * c.ffn_expert) && dev_alloc(&g->moe.eo, S * 16 * H);
+    bool ok = dev_alloc(&g->x, R * H) && dev_alloc(&g->cur, R * H) && dev_alloc(&g->mix, R * H) &&
+              dev_alloc(&g->pk, R * (q_dim + 2 * kv_dim)) && dev_alloc(&g->q, R * q_dim) && dev_alloc(&g->attn, R * q_dim) &&
+              dev_alloc(&g->xf_cur, nb * dfl_xf_bytes(H)) && dev_alloc(&g->xf_attn, nb * dfl_xf_bytes(q_dim)) &&
+              dev_alloc(&g->xs_cur, nb * dfl_xs_bytes(H)) && dev_alloc(&g->xs_attn, nb * dfl_xs_bytes(q_dim)) && dev_alloc(&g->ids, R) &&
+              dev_alloc(&g->pos, R);
+    if (ok && !moe) ok = dev_alloc(&g->xf_g, nb * dfl_xf_bytes(F)) && dev_alloc(&g->xs_g, nb * dfl_xs_bytes(F));
+    if (ok && moe) {
+        const size_t S = dfl_moe_group_max_slots(c, rows), E = c.n_expert, fe = c.ffn_expert;
+        ok = dev_alloc(&g->moe.logits, R * E) && dev_alloc(&g->moe.sg, R) && dev_alloc(&g->moe.sel_e, R * used) &&
+             dev_alloc(&g->moe.sel_w, R * used) && dev_alloc(&g->moe.pick_pos, R * used) && dev_alloc(&g->moe.n_slots, 1) &&
+             dev_alloc(&g->moe.slot_rows, S * 16) && dev_alloc(&g->moe.tiles, S * 4) && dev_alloc(&g->moe.n_tiles, 1) &&
+             dev_alloc(&g->moe.xg, S * dfl_xf_bytes(H)) && dev_alloc(&g->moe.xg_sums, S * dfl_xs_bytes(H)) &&
+             dev_alloc(&g->moe.act, S * dfl_xf_bytes(fe)) && dev_alloc(&g->moe.act_sums, S * dfl_xs_bytes(fe)) && dev_alloc(&g->moe.eo, S * 16 * H);
+        g->moe.max_slots = static_cast<int>(S);
+    }
     if (!ok) {
         (void)hipGetLastError();  // (an allocation that failed leaves its error behind)
         prefill_group_free(g);
         return;
     }
-    g->moe.max_slots = max_slots;
     g->rows = rows;
 }
 }  // namespace
@@ -1164,6 +1172,7 @@ void prefill_pipe_destroy_extras(PrefillPipe *p) {
 }
 
 int32_t prefill_pipe_create_lanes(dflash_ctx *ctx, dflash_session *s, PrefillPipe *p);
+int32_t prefill_lanes_create(dflash_ctx *ctx, dflash_session *s, PrefillPipe *p);
 
 // The extra lanes of the pipelined prefill.  If one of them cannot be made (device memory), what was made is taken down
 // again and the prefill runs with the owner's lane alone: slower, never failing for that reason.
@@ -1172,6 +1181,11 @@ int32_t prefill_pipe_create(dflash_ctx *ctx, dflash_session *s) {
     if (!p) return dfl_fail(ctx, DFLASH_ERR_HIP, "prefill_blocks: out of host memory");
     s->pipe = p;  // (whatever has been made so far is taken down with the session)
     prefill_group_alloc(s, &p->group);
+    if (p->group.rows) return DFLASH_OK;  // (the lanes only if a model comes along that the group does not take)
+    return prefill_lanes_create(ctx, s, p);
+}
+
+int32_t prefill_lanes_create(dflash_ctx *ctx, dflash_session *s, PrefillPipe *p) {
     if (prefill_pipe_create_lanes(ctx, s, p) != DFLASH_OK) {
         for (auto &v : p->kv_done) {
             for (hipEvent_t e : v)
@@ -1236,76 +1250,115 @@ int32_t prefill_pipe_create_lanes(dflash_ctx *ctx, dflash_session *s, PrefillPip
 int32_t dflash_prefill_prepare(dflash_ctx *ctx, dflash_session *s) {
     if (!ctx) return DFLASH_ERR_INVALID_INPUT;
     if (!s) return dfl_fail(ctx, DFLASH_ERR_INVALID_INPUT, "prefill_prepare: null session");
-    if (s->pipe) return s->pipe->ready ? DFLASH_OK : dfl_fail(ctx, DFLASH_ERR_STATE, "prefill_prepare: the extra lanes could not be set up earlier");
+    if (s->pipe)
+        return s->pipe->ready || s->pipe->group.rows ? DFLASH_OK
+                                                     : dfl_fail(ctx, DFLASH_ERR_STATE, "prefill_prepare: the extra lanes could not be set up earlier");
     return prefill_pipe_create(ctx, s);
 }
 
 namespace {
 
-// Whether every layer of the model is one the grouped prefill takes: q/k/v adjacent and, like the output projection,
-// a whole-K product over fragment-order rows; the experts as dfl_moe_ffn_group wants them.
+// The many-row plans of a layer's projections (kind DFL_XF_NONE: not taken).
+struct LayerRows {
+    dfl_rows_plan qkv = {}, wo = {}, gate_up = {}, down = {};
+};
+LayerRows layer_rows(const dflash_ctx *ctx, const dflash_model_cfg &c, const dflash_layer &L) {
+    const int64_t H = c.hidden, q_dim = static_cast<int64_t>(c.n_q) * c.head_dim, kv_dim = static_cast<int64_t>(c.n_kv) * c.head_dim;
+    LayerRows r;
+    if (adjacent(L.wq, q_dim, L.wk, H) && adjacent(L.wk, kv_dim, L.wv, H)) r.qkv = dfl_gemm_rows_plan(ctx, L.wq.type, H, q_dim + 2 * kv_dim, 0);
+    r.wo = dfl_gemm_rows_plan(ctx, L.wo.type, q_dim, H, 0);
+    if (c.n_expert == 0) {
+        if (adjacent(L.gate, c.ffn, L.up, H)) r.gate_up = dfl_gemm_rows_plan(ctx, L.gate.type, H, 2ll * c.ffn, c.ffn);
+        r.down = dfl_gemm_rows_plan(ctx, L.down.type, c.ffn, H, 0);
+    }
+    return r;
+}
+
+// Whether every layer of the model is one the grouped prefill takes: q/k/v adjacent, all projections many-row products
+// with the bits of the block path's; the experts as dfl_moe_ffn_group wants them.
 bool prefill_group_takes(const dflash_ctx *ctx, const dflash_model *model, const PrefillGroup &g) {
     const dflash_model_cfg &c = model->cfg;
-    if (!g.rows || c.n_expert < 1) return false;
-    const int64_t H = c.hidden, q_dim = static_cast<int64_t>(c.n_q) * c.head_dim, kv_dim = static_cast<int64_t>(c.n_kv) * c.head_dim;
+    if (!g.rows) return false;
     for (int il = 0; il < c.n_layers; il++) {
         const dflash_layer &L = model->layers[il];
-        const LayerXf k = layer_xf(ctx, L, true, H, q_dim, kv_dim, c.ffn, false);
-        if (k.qkv == DFL_XF_NONE || k.wo == DFL_XF_NONE || !dfl_moe_group_fits(ctx, c, L, g.rows)) return false;
+        const LayerRows r = layer_rows(ctx, c, L);
+        if (r.qkv.kind == DFL_XF_NONE || r.wo.kind == DFL_XF_NONE) return false;
+        if (c.n_expert ? !dfl_moe_group_fits(ctx, c, L, g.rows) : (r.gate_up.kind == DFL_XF_NONE || r.down.kind == DFL_XF_NONE)) return false;
     }
     return true;
 }
 
 // One group of n rows (positions start .. start + n - 1) through every layer, on `st`: K/V rows into the session's
 // cache, tapped residuals into hidden_capture.  A row gets the bits verify_enqueue gives it in its own 16-row block:
-// every operator here is that block's operator over more rows (or the block's own launch: attention).
+// every operator here is that block's operator over more rows.
 int32_t prefill_group_enqueue(dflash_ctx *ctx, const dflash_model *model, dflash_session *s, PrefillGroup &g, const int32_t *tokens,
                               int32_t n, int64_t start, const int32_t *tap_layers, int32_t n_taps, float *hidden_capture,
                               hipStream_t st) {
     const dflash_model_cfg &c = model->cfg;
     const int H = c.hidden, hd = c.head_dim;
+    const bool moe = c.n_expert > 0;
     const size_t q_dim = static_cast<size_t>(c.n_q) * hd, kv_dim = static_cast<size_t>(c.n_kv) * hd;
     const int64_t tot = static_cast<int64_t>(q_dim + 2 * kv_dim);
-    const size_t xf_h = dfl_xf_bytes(H), xf_q = dfl_xf_bytes(static_cast<int64_t>(q_dim));
-    IntGroupArgs ids_arg = {};
-    for (int i = 0; i < n; i++) ids_arg.v[i] = tokens[i];
-    set_group_ids_pos_kernel<<<(n + 255) / 256, 256, 0, st>>>(ids_arg, static_cast<int>(start), n, g.ids, g.pos);
+    const size_t xf_h = dfl_xf_bytes(H);
+    const int n_blocks = (n + 15) / 16;
+    for (int at = 0; at < n; at += kGroupIdsPerLaunch) {
+        const int m = std::min(kGroupIdsPerLaunch, n - at);
+        IntGroupArgs ids_arg = {};
+        for (int i = 0; i < m; i++) ids_arg.v[i] = tokens[at + i];
+        set_group_ids_pos_kernel<<<(m + 255) / 256, 256, 0, st>>>(ids_arg, static_cast<int>(start) + at, m, g.ids + at, g.pos + at);
+    }
     int32_t rc = embed_rows(ctx, model->token_embd, g.ids, n, H, g.x, st);
     if (rc) return rc;
     const float scale = 1.0f / sqrtf(static_cast<float>(hd));
     const size_t per_layer = static_cast<size_t>(s->capacity) * kv_dim;
-    auto qkv_kind = [&](int il) {
-        return il < c.n_layers ? layer_xf(ctx, model->layers[il], true, H, static_cast<int64_t>(q_dim), static_cast<int64_t>(kv_dim), c.ffn, false).qkv
-                               : DFL_XF_NONE;
+    // a many-row product of rows that are in fragment order, with their sub-block sums made first where its arithmetic wants them
+    auto product = [&](const dfl_rows_plan &p, const dflash_qtensor &w, const uint8_t *xf, uint8_t *xs, float *y, int64_t n_in, int64_t n_out) -> int32_t {
+        if (!p.twin)
+            if (const int32_t r = dfl_xf_sums(ctx, xf, n_in, n_blocks, xs, st)) return r;
+        return dfl_gemm_rows(ctx, p, w.type, w.data, xf, xs, y, n_in, n_out, n, 0, nullptr, nullptr, 0, st);
     };
-    for (int il = 0; il < c.n_layers; il++) {
+    const float *pending_resid = nullptr;  // a dense layer's FFN output still to be added to g.x
+    LayerRows rows = layer_rows(ctx, c, model->layers[0]), next_rows;
+    for (int il = 0; il < c.n_layers; il++, rows = next_rows) {
         const dflash_layer &L = model->layers[il];
         _Float16 *kc = s->k_cache + il * per_layer, *vtc = s->vt_cache + il * per_layer;
-        const LayerXf xk = layer_xf(ctx, L, true, H, static_cast<int64_t>(q_dim), static_cast<int64_t>(kv_dim), c.ffn, false);
-        if (il == 0)  // (later layers: the experts' last kernel has normalised their input)
-            rms_norm_kernel<<<n, 256, 0, st>>>(g.x, nullptr, L.attn_norm, g.cur, H, c.eps, nullptr, nullptr, g.xf_cur, xk.qkv, xf_h);
-        if ((rc = dfl_gemm_whole_blocks(ctx, L.wq.type, L.wq.data, g.xf_cur, g.pk, H, tot, n, 0, nullptr, DFL_XF_NONE, st))) return rc;
+        next_rows = il + 1 < c.n_layers ? layer_rows(ctx, c, model->layers[il + 1]) : LayerRows();
+        if (!moe || il == 0)  // (a mixture's later layers: the experts' last kernel has normalised their input)
+            rms_norm_kernel<<<n, 256, 0, st>>>(g.x, pending_resid, L.attn_norm, g.cur, H, c.eps, nullptr, nullptr, g.xf_cur, rows.qkv.kind, xf_h);
+        pending_resid = nullptr;
+        if ((rc = product(rows.qkv, L.wq, g.xf_cur, g.xs_cur, g.pk, H, tot))) return rc;
         qk_norm_rope_kernel<<<dim3(c.n_q + 2 * c.n_kv, n), 64, 0, st>>>(g.pk, tot, g.pk + q_dim, tot, g.q, nullptr, L.q_norm, L.k_norm, kc,
                                                                       g.pos, c.n_q, c.n_kv, hd, c.eps, c.rope_theta,
                                                                       g.pk + q_dim + kv_dim, tot, vtc, s->capacity);
+        bool tapped = false;
+        for (int t = 0; t < n_taps; t++) tapped = tapped || tap_layers[t] == il;
         // nothing of the last layer beyond its K/V rows is needed unless its residual is tapped (as in verify_enqueue)
-        if (il == c.n_layers - 1) {
-            bool tapped_last = false;
-            for (int t = 0; t < n_taps; t++) tapped_last = tapped_last || tap_layers[t] == il;
-            if (!tapped_last) break;
-        }
+        if (il == c.n_layers - 1 && !tapped) break;
         if ((rc = dfl_attn_blocks(ctx, g.q, DFLASH_TYPE_F32, kc, vtc, start, n, c.n_q, c.n_kv, hd, s->capacity, scale, g.attn, st, g.xf_attn,
-                                  xk.wo)))
+                                  rows.wo.kind)))
             return rc;
-        if ((rc = dfl_gemm_whole_blocks(ctx, L.wo.type, L.wo.data, g.xf_attn, g.mix, static_cast<int64_t>(q_dim), H, n, 0, nullptr,
-                                        DFL_XF_NONE, st)))
-            return rc;
-        const float *next_w = il + 1 < c.n_layers ? model->layers[il + 1].attn_norm : model->output_norm;
-        const int next_kind = qkv_kind(il + 1);
-        // x += mix, the experts' norm and the shared-expert gates: the block path's norm kernel over all the rows
-        rms_norm_kernel<<<n, 256, 0, st>>>(g.x, g.mix, L.post_norm, g.cur, H, c.eps, L.shexp_gate, g.moe.sg);
-        if ((rc = dfl_moe_ffn_group(ctx, c, L, g.x, g.cur, n, g.moe, next_w, next_kind ? g.xf_cur : nullptr, next_kind, xf_h, st)))
-            return rc;
+        if ((rc = product(rows.wo, L.wo, g.xf_attn, g.xs_attn, g.mix, static_cast<int64_t>(q_dim), H))) return rc;
+        if (moe) {
+            const float *next_w = il + 1 < c.n_layers ? model->layers[il + 1].attn_norm : model->output_norm;
+            // x += mix, the experts' norm and the shared-expert gates: the block path's norm kernel over all the rows
+            rms_norm_kernel<<<n, 256, 0, st>>>(g.x, g.mix, L.post_norm, g.cur, H, c.eps, L.shexp_gate, g.moe.sg);
+            if ((rc = dfl_moe_ffn_group(ctx, c, L, g.x, g.cur, n, g.moe, next_w, next_rows.qkv.kind ? g.xf_cur : nullptr, next_rows.qkv.kind, xf_h,
+                                        st)))
+                return rc;
+        } else {
+            rms_norm_kernel<<<n, 256, 0, st>>>(g.x, g.mix, L.post_norm, g.cur, H, c.eps, nullptr, nullptr, g.xf_cur, rows.gate_up.kind, xf_h);
+            if (!rows.gate_up.twin && (rc = dfl_xf_sums(ctx, g.xf_cur, H, n_blocks, g.xs_cur, st))) return rc;
+            // silu(gate) * up straight into fragment order, with the sums the down product wants
+            if ((rc = dfl_gemm_rows(ctx, rows.gate_up, L.gate.type, L.gate.data, g.xf_cur, g.xs_cur, nullptr, H, 2ll * c.ffn, n, c.ffn, g.xf_g,
+                                    rows.down.twin ? nullptr : g.xs_g, rows.down.kind, st)))
+                return rc;
+            if ((rc = dfl_gemm_rows(ctx, rows.down, L.down.type, L.down.data, g.xf_g, g.xs_g, g.mix, c.ffn, H, n, 0, nullptr, nullptr, 0, st)))
+                return rc;
+            if (tapped)  // (the residual is captured below; else the next norm adds it)
+                add_kernel<<<blocks_for(static_cast<size_t>(n) * H), 256, 0, st>>>(g.x, g.mix, static_cast<size_t>(n) * H);
+            else
+                pending_resid = g.mix;
+        }
         for (int t = 0; t < n_taps; t++)
             if (tap_layers[t] == il)
                 capture_kernel<<<dim3(blocks_for(H), n), 256, 0, st>>>(g.x, hidden_capture, H, n_taps, t);
@@ -1339,8 +1392,22 @@ int32_t dflash_prefill_blocks(dflash_ctx *ctx, const dflash_model *model, dflash
     int32_t rc = DFLASH_OK;
     if (!s->pipe && (rc = prefill_pipe_create(ctx, s))) return rc;
     PrefillPipe *p = s->pipe;
-    if (!p->ready) return dfl_fail(ctx, DFLASH_ERR_STATE, "prefill_blocks: the extra lanes could not be set up earlier");
-    if (n_tokens > 16 && start + n_tokens <= 0x7fffffffll && prefill_group_takes(ctx, model, p->group)) {
+    if (n_tokens <= 16) {  // a lone block: the verify's own launches, without its head
+        Int16Args ids_arg = {}, pos_arg = {};
+        for (int i = 0; i < n_tokens; i++) {
+            ids_arg.v[i] = tokens[i];
+            pos_arg.v[i] = static_cast<int32_t>(start + i);
+        }
+        hipStream_t st = static_cast<hipStream_t>(stream);
+        set_ids_pos_kernel<<<1, 64, 0, st>>>(ids_arg, pos_arg, n_tokens, s->ids, s->pos, nullptr, c.vocab);
+        if ((rc = verify_enqueue(ctx, model, s, n_tokens, start, tap_layers, n_taps, hidden_capture, s->logits, s->argmax, s->gap, st, false))) {
+            (void)hipStreamSynchronize(st);
+            return rc;
+        }
+        s->kv_n_pos = start + n_tokens;
+        return DFLASH_OK;
+    }
+    if (start + n_tokens <= 0x7fffffffll && prefill_group_takes(ctx, model, p->group)) {
         // rows of many blocks per pass (see PrefillGroup); the caller's stream alone
         const size_t cap_row = static_cast<size_t>(std::max(n_taps, 0)) * c.hidden;
         for (int32_t t0 = 0; t0 < n_tokens; t0 += p->group.rows) {
@@ -1355,6 +1422,7 @@ int32_t dflash_prefill_blocks(dflash_ctx *ctx, const dflash_model *model, dflash
         s->kv_n_pos = start + n_tokens;
         return DFLASH_OK;
     }
+    if (!p->ready && (rc = prefill_lanes_create(ctx, s, p))) return rc;
     const int n_lanes = p->n_lanes;
     hipStream_t lanes_st[kMaxPrefillLanes] = {static_cast<hipStream_t>(stream)};
     dflash_ctx *lanes_ctx[kMaxPrefillLanes] = {ctx};

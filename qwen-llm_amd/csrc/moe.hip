@@ -12,8 +12,10 @@
 // if there are none, so HBM traffic is the distinct experts of the block, not rows x k.
 #include "common.h"
 #include "device_quant.h"
+#include "mfma_unpack.h"
 #include "moe_route.h"
 
+#include <algorithm>
 #include <cstdlib>
 
 namespace {
@@ -465,18 +467,21 @@ __global__ void __launch_bounds__(1024)
 }
 
 // The slot list of a group of rows.  Expert e with c picks gets ceil(c / 16) consecutive slots, experts in ascending
-// order; behind them one slot per block of sixteen rows for the shared expert (id -1, rows 16 b .. 16 b + 15).
-//   ids[slot], *n_slots;  slot_rows[slot][16]: the rows whose activations the slot multiplies (unused places repeat
-//   row 0: computed, never read);  pick_pos[row][k] = 16 slot + place of the pick's output row.
+// order; behind them one slot per block of sixteen rows for the shared expert (rows 16 b .. 16 b + 15).
+//   *n_slots;  slot_rows[slot][16]: the rows whose activations the slot multiplies (unused places repeat
+//   row 0: computed, never read);  pick_pos[row][k] = 16 slot + place of the pick's output row;
+//   tiles[*n_tiles] = {expert (-1: the shared one), first slot, slots, 0}: runs of at most four slots of one expert, the
+//   row tiles of the expert products.
 // Places inside an expert's slots are handed out by an atomic counter, so they vary from run to run; no sum does.
-// One workgroup; n_rows * n_used <= 4096, n_expert <= 256.
-constexpr int kGroupPicksPerThread = 4;
+// One workgroup; n_rows * n_used <= 1024 kGroupPicksPerThread, n_expert <= 256.
+constexpr int kGroupPicksPerThread = 16;
+constexpr int kGroupTileSlots = 4;
 __global__ void __launch_bounds__(1024)
-    moe_group_slots_kernel(const int32_t *__restrict__ sel_e, int n_rows, int n_used, int n_expert, int32_t *__restrict__ ids,
-                           int32_t *__restrict__ n_slots, int32_t *__restrict__ slot_rows, int32_t *__restrict__ pick_pos,
-                           int max_slots) {
-    __shared__ int cnt[256], base[257];
-    const int tid = threadIdx.x;
+    moe_group_slots_kernel(const int32_t *__restrict__ sel_e, int n_rows, int n_used, int n_expert, int32_t *__restrict__ n_slots,
+                           int32_t *__restrict__ slot_rows, int32_t *__restrict__ pick_pos, int4 *__restrict__ tiles,
+                           int32_t *__restrict__ n_tiles, int max_slots) {
+    __shared__ int cnt[256], base[257], wave_s[4], wave_t[4];
+    const int tid = threadIdx.x, lane = tid & 63;
     if (tid < 256) cnt[tid] = 0;
     __syncthreads();
     const int n_picks = n_rows * n_used;
@@ -484,39 +489,56 @@ __global__ void __launch_bounds__(1024)
 #pragma unroll
     for (int j = 0; j < kGroupPicksPerThread; j++) {
         const int p = tid + 1024 * j;
-        my_e[j] = -1;
-        my_place[j] = 0;
-        if (p < n_picks) {
-            my_e[j] = min(max(sel_e[p], 0), n_expert - 1);
-            my_place[j] = atomicAdd(&cnt[my_e[j]], 1);
+        my_e[j] = p < n_picks ? min(max(sel_e[p], 0), n_expert - 1) : -1;
+    }
+#pragma unroll
+    for (int j = 0; j < kGroupPicksPerThread; j++) my_place[j] = my_e[j] >= 0 ? atomicAdd(&cnt[my_e[j]], 1) : 0;
+    __syncthreads();
+    // exclusive prefix sums over the experts of their slots and of their row tiles (four waves, then across them)
+    const int c = tid < n_expert ? cnt[tid] : 0, ns = (c + 15) >> 4, nt = (ns + kGroupTileSlots - 1) / kGroupTileSlots;
+    int ps = ns, pt = nt;
+    for (int off = 1; off < 64; off <<= 1) {
+        const int us = __shfl_up(ps, off, 64), ut = __shfl_up(pt, off, 64);
+        if (lane >= off) {
+            ps += us;
+            pt += ut;
         }
     }
+    if (tid < 256 && lane == 63) {
+        wave_s[tid >> 6] = ps;
+        wave_t[tid >> 6] = pt;
+    }
     __syncthreads();
+    int total = 0, total_t = 0;
+    for (int w = 0; w < 4; w++) {
+        if (w < (tid >> 6)) {
+            ps += wave_s[w];
+            pt += wave_t[w];
+        }
+        total += wave_s[w];
+        total_t += wave_t[w];
+    }
+    if (tid < n_expert) base[tid] = ps - ns;
+    const int n_blocks = (n_rows + 15) >> 4, shared_t = (n_blocks + kGroupTileSlots - 1) / kGroupTileSlots;
     if (tid == 0) {
-        int b = 0;
-        for (int e = 0; e < n_expert; e++) {
-            base[e] = b;
-            b += (cnt[e] + 15) >> 4;
-        }
-        base[n_expert] = b;
+        *n_slots = min(total + n_blocks, max_slots);  // (the host sizes max_slots for the worst case)
+        *n_tiles = total_t + shared_t;
     }
-    __syncthreads();
-    const int total = base[n_expert], n_blocks = (n_rows + 15) >> 4;
-    if (tid == 0) *n_slots = min(total + n_blocks, max_slots);  // (the host sizes max_slots for the worst case)
     if (tid < n_expert) {
-        const int c = cnt[tid], b = base[tid];
-        for (int t = 0; t < ((c + 15) >> 4); t++) ids[b + t] = tid;
+        const int b = ps - ns;
+        for (int t = 0; t < nt; t++)
+            tiles[pt - nt + t] = int4{tid, b + kGroupTileSlots * t, min(kGroupTileSlots, ns - kGroupTileSlots * t), 0};
         if (c & 15)
             for (int m = c & 15; m < 16; m++) slot_rows[(b + (c >> 4)) * 16 + m] = 0;
     }
-    for (int r = tid; r < 16 * n_blocks; r += 1024) {
-        slot_rows[total * 16 + r] = min(r, n_rows - 1);
-        if ((r & 15) == 0) ids[total + (r >> 4)] = -1;
-    }
+    for (int t = tid; t < shared_t; t += 1024)
+        tiles[total_t + t] = int4{-1, total + kGroupTileSlots * t, min(kGroupTileSlots, n_blocks - kGroupTileSlots * t), 0};
+    for (int r = tid; r < 16 * n_blocks; r += 1024) slot_rows[total * 16 + r] = min(r, n_rows - 1);
+    __syncthreads();
 #pragma unroll
     for (int j = 0; j < kGroupPicksPerThread; j++) {
-        const int p = tid + 1024 * j;
-        if (p < n_picks) {
+        if (my_e[j] >= 0) {
+            const int p = tid + 1024 * j;
             const int at = (base[my_e[j]] + (my_place[j] >> 4)) * 16 + (my_place[j] & 15);
             slot_rows[at] = p / n_used;
             pick_pos[p] = at;
@@ -524,21 +546,32 @@ __global__ void __launch_bounds__(1024)
     }
 }
 
-// xg[slot][place][:] = f16(cur[slot_rows[slot][place]][:]): what the expert kernel would round the row to as it loads it.
-__global__ void __launch_bounds__(256)
+// A slot's rows in fragment order (kind Q4K) with their sub-block sums, rounded to f16 as every few-row kernel rounds its
+// activations: one wave per (super-block, slot), lane (m, g) takes the 64 values of chunk g of the slot's row m.
+__global__ void __launch_bounds__(64)
     moe_group_gather_kernel(const float *__restrict__ cur, const int32_t *__restrict__ slot_rows, const int32_t *__restrict__ n_slots,
-                            int hidden, _Float16 *__restrict__ xg) {
-    typedef float f4 __attribute__((ext_vector_type(4)));
-    typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-    const int at = blockIdx.y;
-    if ((at >> 4) >= *n_slots) return;
-    const int i = 8 * (blockIdx.x * 256 + threadIdx.x);
-    if (i >= hidden) return;
-    const float *src = cur + static_cast<size_t>(slot_rows[at]) * hidden + i;
-    const f4 a = *reinterpret_cast<const f4 *>(src), b = *reinterpret_cast<const f4 *>(src + 4);
-    const h8 o = {static_cast<_Float16>(a[0]), static_cast<_Float16>(a[1]), static_cast<_Float16>(a[2]), static_cast<_Float16>(a[3]),
-                  static_cast<_Float16>(b[0]), static_cast<_Float16>(b[1]), static_cast<_Float16>(b[2]), static_cast<_Float16>(b[3])};
-    *reinterpret_cast<h8 *>(xg + static_cast<size_t>(at) * hidden + i) = o;
+                            int hidden, uint8_t *__restrict__ xg, uint8_t *__restrict__ sums) {
+    const int b = blockIdx.x, slot = blockIdx.y, lane = threadIdx.x, m = lane & 15, g = lane >> 4, nb = hidden >> 8;
+    if (slot >= *n_slots) return;
+    const float4_t *src = reinterpret_cast<const float4_t *>(cur + static_cast<size_t>(slot_rows[slot * 16 + m]) * hidden + 256 * b + 64 * g);
+    half8_t *dst = reinterpret_cast<half8_t *>(xg + (static_cast<size_t>(slot) * nb + b) * 8192) + lane;
+    float4_t v[16];
+#pragma unroll
+    for (int i = 0; i < 16; i++) v[i] = src[i];
+    float o[8];
+#pragma unroll
+    for (int t = 0; t < 8; t++) {
+        _Float16 h[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) h[i] = static_cast<_Float16>(v[2 * t + (i >> 2)][i & 3]);
+        const half8_t frag = {h[0], h[2], h[1], h[3], h[4], h[6], h[5], h[7]};
+        dst[t * 64] = frag;
+        o[t] = q4k_octet_sum_seq(h);
+    }
+    const Q4KSumParts s0 = q4k_sum_parts((o[0] + o[1]) + (o[2] + o[3])), s1 = q4k_sum_parts((o[4] + o[5]) + (o[6] + o[7]));
+    const _Float16 zero = static_cast<_Float16>(0.0f);
+    const half8_t r = {s0.hi, s1.hi, s0.lo, s1.lo, s0.over, s1.over, zero, zero};
+    reinterpret_cast<half8_t *>(sums + (static_cast<size_t>(slot) * nb + b) * 1024)[lane] = r;
 }
 
 }  // namespace
@@ -692,6 +725,8 @@ int32_t dfl_moe_ffn(dflash_ctx *ctx, const dflash_model_cfg &c, const dflash_lay
     return DFLASH_OK;
 }
 
+int dfl_moe_group_max_picks() { return 1024 * kGroupPicksPerThread; }
+
 int dfl_moe_group_max_slots(const dflash_model_cfg &c, int n_rows) {
     const int used = c.n_expert_used < c.n_expert ? c.n_expert_used : c.n_expert;
     const int picks = n_rows * used;
@@ -722,16 +757,17 @@ int32_t dfl_moe_ffn_group(dflash_ctx *ctx, const dflash_model_cfg &c, const dfla
     int32_t rc;
     if ((rc = dfl_router_rows(ctx, L.router.data, cur, s.logits, H, E, n_rows, st))) return rc;
     moe_group_route_kernel<<<(n_rows + 15) / 16, 1024, 0, st>>>(s.logits, n_rows, E, used, s.sel_e, s.sel_w);
-    moe_group_slots_kernel<<<1, 1024, 0, st>>>(s.sel_e, n_rows, used, E, s.ids, s.n_slots, s.slot_rows, s.pick_pos, max_slots);
-    moe_group_gather_kernel<<<dim3((H / 8 + 255) / 256, max_slots * 16), 256, 0, st>>>(cur, s.slot_rows, s.n_slots, H, s.xg);
+    moe_group_slots_kernel<<<1, 1024, 0, st>>>(s.sel_e, n_rows, used, E, s.n_slots, s.slot_rows, s.pick_pos, reinterpret_cast<int4 *>(s.tiles),
+                                             s.n_tiles, max_slots);
+    moe_group_gather_kernel<<<dim3(H / DFL_QK_K, max_slots), 64, 0, st>>>(cur, s.slot_rows, s.n_slots, H, s.xg, s.xg_sums);
     const size_t stride_in = dflash_q4k_tiled_bytes(H, fe), stride_dn = dflash_q4k_tiled_bytes(fe, H);
-    if ((rc = dfl_gemm_q4k_batched(ctx, L.gate_exps.data, stride_in, L.gate.data, s.ids, s.n_slots, max_slots, s.xg, DFLASH_TYPE_F16,
-                                   static_cast<size_t>(16) * H, s.act, DFLASH_TYPE_F16, static_cast<size_t>(16) * fe, H, fe, 16, 1,
-                                   L.up_exps.data, L.up.data, 1, st, nullptr)))
+    // most row tiles the list can have: one per kGroupTileSlots slots, and a short one per expert and for the shared one
+    const int max_tiles = std::min(max_slots, max_slots / kGroupTileSlots + E + 1);
+    if ((rc = dfl_gemm_rows_experts(ctx, L.gate_exps.data, L.gate.data, L.up_exps.data, L.up.data, stride_in, s.xg, s.xg_sums, s.tiles, s.n_tiles,
+                                    max_tiles, nullptr, H, fe, s.act, s.act_sums, st)))
         return rc;
-    if ((rc = dfl_gemm_q4k_batched(ctx, L.down_exps.data, stride_dn, L.down.data, s.ids, s.n_slots, max_slots, s.act, DFLASH_TYPE_F16,
-                                   static_cast<size_t>(16) * fe, s.eo, DFLASH_TYPE_F32, static_cast<size_t>(16) * H, fe, H, 16, 1, nullptr,
-                                   nullptr, 1, st, nullptr)))
+    if ((rc = dfl_gemm_rows_experts(ctx, L.down_exps.data, L.down.data, nullptr, nullptr, stride_dn, s.act, s.act_sums, s.tiles, s.n_tiles,
+                                    max_tiles, s.eo, fe, H, nullptr, nullptr, st)))
         return rc;
     moe_combine_norm_kernel<<<n_rows, 256, 0, st>>>(s.eo, s.pick_pos, s.sel_w, s.sg, nullptr, s.n_slots, used, H, x_resid, next_norm_w,
                                                     cur, c.eps, nullptr, next_xf, next_xf_kind, 1, next_xf_stride);

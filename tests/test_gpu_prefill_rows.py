@@ -1,0 +1,43 @@
+"""The grouped prefill's many-row products (csrc/gemm_rows.hip) against the block-by-block verify, whose own products
+are the oracle-checked ones: captured residuals bit for bit.
+
+The row counts are those where a launch changes its shape: two blocks (one of a single row); the whole-K kernel's last
+and the split's first count; tiles of every number of row blocks with a last tile that is not full; several rounds of
+the chip.  K and the column counts bring each kind of cut: 5120 (whole-K slices, twenty super-blocks), 17408 (stream-K
+ranges that differ from tile group to tile group), 1024 (fewer super-blocks than slices), Q6_K projections, experts
+with one to four blocks per tile."""
+import numpy as np
+import pytest
+import torch
+
+import qwen_llm_amd as dfl
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = {
+    "wide": (dfl.ModelConfig(n_layers=2, hidden=5120, n_q=32, n_kv=8, head_dim=128, ffn=17408, vocab=2048), dfl.synth.Q4_K),
+    "narrow": (dfl.ModelConfig(n_layers=2, hidden=1024, n_q=16, n_kv=8, head_dim=128, ffn=3072, vocab=2048), dfl.synth.Q4_K),
+    "experts": (dfl.ModelConfig(n_layers=2, hidden=2048, n_q=16, n_kv=2, head_dim=256, ffn=0, vocab=2048, n_expert=32, n_expert_used=4,
+                                ffn_expert=768, ffn_shared=768), dfl.synth.Q6_K),
+}
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = dfl.Context(0, workspace_bytes=256 << 20)
+    yield c
+    c.close()
+
+
+@pytest.mark.parametrize("rows", [17, 80, 97, 192, 200, 273, 530, 1001])
+@pytest.mark.parametrize("shape", sorted(SHAPES))
+def test_many_row_prefill_equals_block_by_block(ctx, shape, rows):
+    cfg, attn_type = SHAPES[shape]
+    model = dfl.TargetModel(ctx, cfg, dfl.synth_target_weights_device(cfg, 5, "cuda", attn_type=attn_type))
+    one, many = dfl.Session(ctx, model, rows + 16, [0, 1]), dfl.Session(ctx, model, rows + 16, [0, 1])
+    tokens = np.random.default_rng(rows).integers(0, cfg.vocab, rows).tolist()
+    got = many.prefill_blocks(tokens, 0)
+    want = torch.cat([one.encode_packed_verify_layer_major(tokens[i:i + 16], i, want_head=False).hidden_capture for i in range(0, rows, 16)])
+    assert torch.equal(got, want)
+    one.close()
+    many.close()
