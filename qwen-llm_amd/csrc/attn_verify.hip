@@ -67,9 +67,15 @@ __device__ __forceinline__ int attn_swz(int r) { return (r & 3) | ((r >> 1) & 4)
 // context length is only known on the device (a captured graph) can size its grid for the largest
 // context and let surplus workgroups leave.
 __host__ __device__ __forceinline__ int64_t attn_chunk(int64_t n_pos, int64_t want, int64_t min_chunk) {
-    int64_t chunk = (n_pos + want - 1) / want;
+    // (32-bit division where the positions fit: the 64-bit one is 150 instructions at the head of every workgroup)
+    int64_t chunk = n_pos + want <= 0x7fffffff ? static_cast<uint32_t>(n_pos + want - 1) / static_cast<uint32_t>(want) : (n_pos + want - 1) / want;
     chunk = (chunk + 31) / 32 * 32;
     return chunk < min_chunk ? min_chunk : chunk;
+}
+__device__ __forceinline__ int attn_splits(int64_t n_pos, int64_t want, int64_t min_chunk) {
+    const int64_t chunk = attn_chunk(n_pos, want, min_chunk);
+    return static_cast<int>(n_pos <= 0x7fffffff ? (static_cast<uint32_t>(n_pos) + static_cast<uint32_t>(chunk) - 1) / static_cast<uint32_t>(chunk)
+                                                : (n_pos + chunk - 1) / chunk);
 }
 
 // eight consecutive query values (16-byte aligned) as floats
@@ -367,7 +373,7 @@ namespace {
 __global__ void __launch_bounds__(256)
     attn_combine_kernel(const float *__restrict__ part_o, const float *__restrict__ part_ml, float *__restrict__ out,
                         int n_rows_total, int n_q, int hd, int64_t ctx_len, const int32_t *__restrict__ ctx_len_dev, int want,
-                        int min_chunk, void *__restrict__ out_xf, int out_xf_kind, int64_t part_slots, size_t xf_stride) {
+                        int min_chunk, void *__restrict__ out_xf, int out_xf_kind, int64_t part_slots, size_t xf_stride, int max_splits) {
     // blockIdx.z: which block of sixteen rows (see attn_split_kernel); rows past a short last block leave
     const int n_rows = min(16, n_rows_total - 16 * static_cast<int>(blockIdx.z));
     if (static_cast<int>(blockIdx.y) >= n_rows) return;
@@ -375,11 +381,6 @@ __global__ void __launch_bounds__(256)
     part_ml += static_cast<int64_t>(blockIdx.z) * part_slots * 2;
     out += static_cast<int64_t>(blockIdx.z) * 16 * n_q * hd;
     if (out_xf) out_xf = static_cast<uint8_t *>(out_xf) + blockIdx.z * xf_stride;
-    if (ctx_len_dev) ctx_len = *ctx_len_dev;
-    ctx_len += 16 * static_cast<int64_t>(blockIdx.z);
-    const int64_t n_pos = ctx_len + n_rows;
-    const int64_t chunk = attn_chunk(n_pos, want, min_chunk);
-    const int n_splits = static_cast<int>((n_pos + chunk - 1) / chunk);
     __shared__ float wgt[1024];          // 2^(m_s - m*) per split (n_splits <= 1024)
     __shared__ float red[8][256 + 4];    // partial outputs per split lane
     __shared__ float red_l[8];
@@ -391,8 +392,10 @@ __global__ void __launch_bounds__(256)
     float m_own[4];
 #pragma unroll
     for (int j = 0; j < 4; j++) {
+        m_own[j] = -INFINITY;
+        if (256 * j >= max_splits) continue;
         const int s = tid + 256 * j;
-        m_own[j] = s < n_splits ? part_ml[(slot0 + s * slot_stride) * 2] : -INFINITY;
+        m_own[j] = s < max_splits ? part_ml[(slot0 + s * slot_stride) * 2] : -INFINITY;
     }
     // The partial outputs of the first kPre rounds of splits are asked for right behind the maxima, before those are
     // waited for: their addresses do not depend on the weights, so the two trips to memory are in flight together
@@ -401,21 +404,24 @@ __global__ void __launch_bounds__(256)
     constexpr int kPre = 4;
     const int sl = tid >> 5, dl = tid & 31;  // split lane, dim lane
     const int n_vec = hd / 4;                // float4 per row: 16, 32 or 64
-    float4_t pre0[kPre], pre1[kPre];
-    float pre_l[kPre];
+    float4_t pre0[kPre] = {}, pre1[kPre] = {};
+    float pre_l[kPre] = {};
 #pragma unroll
     for (int i = 0; i < kPre; i++) {
-        const int s = sl + 8 * i;
-        pre0[i] = float4_t{0, 0, 0, 0};
-        pre1[i] = float4_t{0, 0, 0, 0};
-        pre_l[i] = 0.0f;
-        if (s < n_splits) {
-            const float4_t *po = reinterpret_cast<const float4_t *>(part_o + (slot0 + s * slot_stride) * hd);
-            if (dl < n_vec) pre0[i] = po[dl];
-            if (dl + 32 < n_vec) pre1[i] = po[dl + 32];
-            if (dl == 0) pre_l[i] = part_ml[(slot0 + s * slot_stride) * 2 + 1];
-        }
+        if (8 * i >= max_splits) continue;  // (uniform; inside a round, lanes past the last split re-read it)
+        const int64_t slot = slot0 + min(sl + 8 * i, max_splits - 1) * slot_stride;
+        const float4_t *po = reinterpret_cast<const float4_t *>(part_o + slot * hd);
+        pre0[i] = po[min(dl, n_vec - 1)];
+        if (n_vec > 32) pre1[i] = po[min(dl + 32, n_vec - 1)];
+        pre_l[i] = part_ml[slot * 2 + 1];
     }
+    // how many splits there are: the context length may have to be read first, and nothing above waits for it
+    if (ctx_len_dev) ctx_len = *ctx_len_dev;
+    ctx_len += 16 * static_cast<int64_t>(blockIdx.z);
+    const int n_splits = attn_splits(ctx_len + n_rows, want, min_chunk);
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+        if (tid + 256 * j >= n_splits) m_own[j] = -INFINITY;
     float m_loc = fmaxf(fmaxf(m_own[0], m_own[1]), fmaxf(m_own[2], m_own[3]));
     for (int off = 32; off > 0; off >>= 1) m_loc = fmaxf(m_loc, __shfl_xor(m_loc, off, 64));
     if ((tid & 63) == 0) red_l[tid >> 6] = m_loc;
@@ -728,7 +734,7 @@ static int32_t attn_rows(dflash_ctx *ctx, const void *q, int32_t q_type, const v
     if (rc) return rc;
     attn_combine_kernel<<<dim3(n_q, n_rows, n_blocks), 256, 0, st>>>(part_o, part_ml, out, n_rows_total, n_q, head_dim, ctx_len, ctx_len_dev,
                                                                     want, static_cast<int>(min_chunk), out_xf, out_xf_kind, part_slots,
-                                                                    dfl_xf_bytes(static_cast<int64_t>(n_q) * head_dim));
+                                                                    dfl_xf_bytes(static_cast<int64_t>(n_q) * head_dim), n_splits);
     DFL_HIP_CHECK(ctx, hipGetLastError());
     return DFLASH_OK;
 }

@@ -2252,7 +2252,7 @@ __global__ void __launch_bounds__(64 * kMaxSplit)
 // that precede it (rms_norm_kernel of the model followed by the kernel above, as one launch).  One workgroup per
 // (16 experts, block row): it normalises its row of x + add exactly as the norm kernel does (256 threads, the row in
 // registers), keeps the f16 copy in LDS as the one live row of the MFMA's X operand (the other fifteen are zeros: a
-// row's products do not depend on its neighbours) and multiplies it with its 16 staged weight rows.  The kernel
+// row's products do not depend on its neighbours) and multiplies it with its 16 weight rows.  The kernel
 // above gives a workgroup all 16 rows, 162 KB to take in where this one takes 50 KB, and a CU takes in only 20-30 KB
 // per microsecond: 16 x 8 small workgroups instead of 8 large ones, and no launch for the norm.  (Measured first
 // with the norm of all 16 rows inside each of the 8 workgroups, 290 KB each: slower than the two launches.)  The
@@ -2268,7 +2268,6 @@ __global__ void __launch_bounds__(64 * kMaxSplit)
                             int n_steps, size_t row_bytes) {
     typedef float f4 __attribute__((ext_vector_type(4)));
     typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-    __shared__ __attribute__((aligned(16))) uint8_t ws[16 * kQ8WRowStride];  // the raw weight rows, padded as above
     __shared__ half8_t xrow[4 * kQ8ChunkSteps];                              // [step][k-group]: the normalised row
     __shared__ float red[kMaxSplit][16];
     __shared__ float sq_part[4], dot_part[4];
@@ -2279,27 +2278,35 @@ __global__ void __launch_bounds__(64 * kMaxSplit)
     const bool first_tile = blockIdx.x == 0;
     const bool norm_wave = wave < 4;  // the norm is the work of 256 threads, as in rms_norm_kernel; the row's loads go out first
     DFL_TRR(0);
-    f4 v[2] = {f4{0, 0, 0, 0}, f4{0, 0, 0, 0}}, nw[2] = {f4{0, 0, 0, 0}, f4{0, 0, 0, 0}};
+    f4 v[2], av[2], nw[2], gw[2];
     if (norm_wave) {
         const float *xr = x + static_cast<size_t>(r) * hidden, *ar = add + static_cast<size_t>(r) * hidden;
 #pragma unroll
-        for (int j = 0; j < 2; j++) {
-            const int i = 4 * (tid + 256 * j);
-            if (i < hidden) {
-                v[j] = *reinterpret_cast<const f4 *>(xr + i) + *reinterpret_cast<const f4 *>(ar + i);
-                nw[j] = *reinterpret_cast<const f4 *>(norm_w + i);
-            }
+        for (int j = 0; j < 2; j++) {  // (unconditional loads, all in flight together; values past the row count as zeros)
+            const int i = min(4 * (tid + 256 * j), hidden - 4);
+            v[j] = *reinterpret_cast<const f4 *>(xr + i);
+            av[j] = *reinterpret_cast<const f4 *>(ar + i);
+            nw[j] = *reinterpret_cast<const f4 *>(norm_w + i);
+            if (first_tile) gw[j] = *reinterpret_cast<const f4 *>(gate_w + i);
         }
     }
-    const int wp_row = n_steps * DFL_Q8_0_BYTES / 16;
-    for (int p = tid; p < 16 * wp_row; p += 64 * kMaxSplit) {
-        const int wr = p / wp_row, c = p - wr * wp_row;
-        const int row = min(n0 + wr, n_out - 1);
-        *reinterpret_cast<u32x4_t *>(ws + wr * kQ8WRowStride + 16 * c) =
-            *reinterpret_cast<const u32x4_t *>(w + static_cast<size_t>(row) * row_bytes + 16 * c);
+    // this wave's steps of the product (at most four: hidden <= 2048), its lanes' weights straight from the rows: they
+    // arrive while the norm is computed, and nothing has to pass through LDS for them
+    const int s0 = n_steps * wave / kMaxSplit, s1 = n_steps * (wave + 1) / kMaxSplit;
+    constexpr int kSteps = kQ8ChunkSteps / kMaxSplit;
+    Raw8<DFLASH_TYPE_Q8_0> rw[kSteps];
+    {
+        const uint8_t *wrow = w + static_cast<size_t>(min(n0 + n, n_out - 1)) * row_bytes;
+#pragma unroll
+        for (int i = 0; i < kSteps; i++) rw[i] = load_raw8<DFLASH_TYPE_Q8_0>(wrow, static_cast<int64_t>(min(s0 + i, n_steps - 1)) * 32 + 8 * g);
     }
     if (norm_wave) {
         float s = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            v[j] += av[j];
+            if (4 * (tid + 256 * j) >= hidden) v[j] = f4{0, 0, 0, 0};
+        }
 #pragma unroll
         for (int j = 0; j < 2; j++)
             s += (v[j][0] * v[j][0] + v[j][1] * v[j][1]) + (v[j][2] * v[j][2] + v[j][3] * v[j][3]);
@@ -2322,8 +2329,7 @@ __global__ void __launch_bounds__(64 * kMaxSplit)
                 const f4 o = v[j] * scale * nw[j];
                 if (first_tile) {
                     *reinterpret_cast<f4 *>(cur + static_cast<size_t>(r) * hidden + i) = o;
-                    const f4 gw = *reinterpret_cast<const f4 *>(gate_w + i);
-                    dot += (o[0] * gw[0] + o[1] * gw[1]) + (o[2] * gw[2] + o[3] * gw[3]);
+                    dot += (o[0] * gw[j][0] + o[1] * gw[j][1]) + (o[2] * gw[j][2] + o[3] * gw[j][3]);
                 }
                 // values 8 c .. 8 c + 7 are piece c = 4 step + k-group; this thread's four are its lower or upper half
                 h4 *piece = reinterpret_cast<h4 *>(&xrow[i >> 3]);
@@ -2337,26 +2343,20 @@ __global__ void __launch_bounds__(64 * kMaxSplit)
         }
     }
     DFL_TRR(3);
-    __syncthreads();  // the row, the weight rows and the gate's partial sums are in LDS
+    __syncthreads();  // the row and the gate's partial sums are in LDS
     DFL_TRR(4);
     if (first_tile && tid == 0) {
         float d = 0.0f;
         for (int k = 0; k < 4; k++) d += dot_part[k];
         gate_out[r] = 1.0f / (1.0f + expf(-d));
     }
-    const uint8_t *rowp = ws + n * kQ8WRowStride;
     const half8_t zero = {0, 0, 0, 0, 0, 0, 0, 0};
-    const int s0 = n_steps * wave / kMaxSplit, s1 = n_steps * (wave + 1) / kMaxSplit;
     float4_t acc = {0, 0, 0, 0};
-    for (int st = s0; st < s1; st++) {
-        const uint8_t *blk = rowp + st * DFL_Q8_0_BYTES;  // 2-byte aligned
-        const uint16_t *q16 = reinterpret_cast<const uint16_t *>(blk + 2 + 8 * g);
-        Raw8<DFLASH_TYPE_Q8_0> rw;
-        rw.d = static_cast<float>(__builtin_bit_cast(_Float16, *reinterpret_cast<const uint16_t *>(blk)));
-        rw.q = static_cast<uint64_t>(q16[0]) | (static_cast<uint64_t>(q16[1]) << 16) | (static_cast<uint64_t>(q16[2]) << 32) |
-               (static_cast<uint64_t>(q16[3]) << 48);
-        const half8_t piece = xrow[4 * st + g];
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(n == (r & 15) ? piece : zero, convert_raw8<DFLASH_TYPE_Q8_0>(rw), acc, 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < kSteps; i++) {
+        if (s0 + i >= s1) break;
+        const half8_t piece = xrow[4 * (s0 + i) + g];
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(n == (r & 15) ? piece : zero, convert_raw8<DFLASH_TYPE_Q8_0>(rw[i]), acc, 0, 0, 0);
     }
     // the row rides in MFMA row r % 16 (any one would do: the other fifteen are zeros): lane group (r % 16) / 4, element r % 4
     const int ri = r & 3;

@@ -57,120 +57,127 @@ struct ConvResid {
     const float *base = nullptr;  // [2][kernel][n]
     int kernel_size = 0, group_size = 1;
 };
+bool norm_in_registers(int n) { return n >= 4 && n <= 8192 && n % 4 == 0; }
+// What bounds it: the one trip to memory, with sixteen workgroups on the chip.  So everything a thread will need - V
+// vectors of the row, of what is added, of the weights - is asked for at once and unconditionally (a vector past the row
+// re-reads its last one and counts as zeros; a load behind a branch waits for the branch in front of it): 6.9 -> 2.9 us
+// per launch inside a verify's graph for sixteen rows of 5120.  The sums keep one order whatever V: a thread's vectors in
+// turn, the lanes of a wave, the four waves.
+typedef float norm_f4 __attribute__((ext_vector_type(4)));
+template <int V, bool kConv>
 __global__ void __launch_bounds__(256) rms_norm_kernel(float *__restrict__ x, const float *__restrict__ add,
                                                        const float *__restrict__ w, float *__restrict__ y, int n,
                                                        float eps, const float *__restrict__ gate_w,
-                                                       float *__restrict__ gate_out, void *__restrict__ y_xf = nullptr,
-                                                       int y_xf_kind = 0, size_t xf_stride = 0, ConvResid conv = ConvResid()) {
-    typedef float f4 __attribute__((ext_vector_type(4)));
+                                                       float *__restrict__ gate_out, void *__restrict__ y_xf,
+                                                       int y_xf_kind, size_t xf_stride, ConvResid conv) {
+    typedef norm_f4 f4;
+    __shared__ float sh[4], sh_dot[4];
+    const int t = blockIdx.x, tid = threadIdx.x;
+    float *xr = x + static_cast<size_t>(t) * n;
+    float *yr = y + static_cast<size_t>(t) * n;
+    int at[V];
+    f4 v[V], a[V], wv[V], gw[V];
+#pragma unroll
+    for (int j = 0; j < V; j++) {
+        at[j] = min(4 * (tid + 256 * j), n - 4);
+        v[j] = *reinterpret_cast<const f4 *>(xr + at[j]);
+    }
+    if constexpr (kConv) {
+        // the residual term is the convolution: taps in order, fused multiply-adds (the host takes this path for
+        // group sizes that are multiples of four: one coefficient per vector and tap)
+        const int ks = conv.kernel_size, n_groups = n / conv.group_size;
+        const float *dyn_t = conv.dyn + (static_cast<size_t>(t) * 2 + 1) * ks * n_groups;
+        const float *base1 = conv.base + static_cast<size_t>(ks) * n;
+        int grp[V];
+#pragma unroll
+        for (int j = 0; j < V; j++) {
+            a[j] = f4{0, 0, 0, 0};
+            grp[j] = at[j] / conv.group_size;
+        }
+        for (int tap = 0; tap < ks && tap <= t; tap += 2) {
+            const bool two = tap + 1 < ks && tap + 1 <= t;  // (two taps' loads in flight together)
+            f4 b[2][V], src[2][V];
+            float dg[2][V];
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                const int tp = u && two ? tap + 1 : tap;
+#pragma unroll
+                for (int j = 0; j < V; j++) {
+                    b[u][j] = *reinterpret_cast<const f4 *>(base1 + static_cast<size_t>(tp) * n + at[j]);
+                    src[u][j] = *reinterpret_cast<const f4 *>(add + static_cast<size_t>(t - tp) * n + at[j]);
+                    dg[u][j] = dyn_t[static_cast<size_t>(tp) * n_groups + grp[j]];
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                if (u && !two) break;
+#pragma unroll
+                for (int j = 0; j < V; j++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) a[j][e] = __builtin_fmaf(b[u][j][e] + dg[u][j], src[u][j][e], a[j][e]);
+            }
+        }
+    } else if (add) {
+#pragma unroll
+        for (int j = 0; j < V; j++) a[j] = *reinterpret_cast<const f4 *>(add + static_cast<size_t>(t) * n + at[j]);
+    }
+#pragma unroll
+    for (int j = 0; j < V; j++) wv[j] = *reinterpret_cast<const f4 *>(w + at[j]);
+    if (gate_w) {
+#pragma unroll
+        for (int j = 0; j < V; j++) gw[j] = *reinterpret_cast<const f4 *>(gate_w + at[j]);
+    }
+    float s = 0.0f;
+#pragma unroll
+    for (int j = 0; j < V; j++) {
+        if (kConv || add) v[j] += a[j];
+        const bool in = 4 * (tid + 256 * j) < n;
+        if (!in) v[j] = f4{0, 0, 0, 0};
+        s += (v[j][0] * v[j][0] + v[j][1] * v[j][1]) + (v[j][2] * v[j][2] + v[j][3] * v[j][3]);
+    }
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+    if ((tid & 63) == 0) sh[tid >> 6] = s;
+    if (kConv || add) {
+#pragma unroll
+        for (int j = 0; j < V; j++)
+            if (4 * (tid + 256 * j) < n) *reinterpret_cast<f4 *>(xr + at[j]) = v[j];
+    }
+    __syncthreads();
+    s = ((sh[0] + sh[1]) + sh[2]) + sh[3];
+    const float scale = 1.0f / sqrtf(s / static_cast<float>(n) + eps);
+    float dot = 0.0f;
+#pragma unroll
+    for (int j = 0; j < V; j++) {
+        const int i = 4 * (tid + 256 * j);
+        if (i < n) {
+            const f4 o = v[j] * scale * wv[j];
+            *reinterpret_cast<f4 *>(yr + i) = o;
+            // (the host passes y_xf only for n a multiple of 256: whole waves are inside or outside the row)
+            // (more than sixteen rows: block b of sixteen at y_xf + b * xf_stride bytes)
+            if (y_xf)
+                dfl_xf_store_pair(static_cast<uint8_t *>(y_xf) + (t >> 4) * xf_stride, y_xf_kind, t & 15, i & ~7, o[0],
+                                  o[1], o[2], o[3]);
+            if (gate_w) dot += (o[0] * gw[j][0] + o[1] * gw[j][1]) + (o[2] * gw[j][2] + o[3] * gw[j][3]);
+        }
+    }
+    if (gate_w) {
+        for (int off = 32; off > 0; off >>= 1) dot += __shfl_xor(dot, off, 64);
+        if ((tid & 63) == 0) sh_dot[tid >> 6] = dot;
+        __syncthreads();
+        if (tid == 0) gate_out[t] = 1.0f / (1.0f + expf(-(((sh_dot[0] + sh_dot[1]) + sh_dot[2]) + sh_dot[3])));
+    }
+}
+
+// The same for any width, element by element (no fragment order: the host passes y_xf only where the kernel above runs).
+__global__ void __launch_bounds__(256) rms_norm_any_kernel(float *__restrict__ x, const float *__restrict__ add,
+                                                           const float *__restrict__ w, float *__restrict__ y, int n,
+                                                           float eps, const float *__restrict__ gate_w,
+                                                           float *__restrict__ gate_out) {
     __shared__ float sh[4];
     float *xr = x + static_cast<size_t>(blockIdx.x) * n;
     const float *ar = add ? add + static_cast<size_t>(blockIdx.x) * n : nullptr;
     float *yr = y + static_cast<size_t>(blockIdx.x) * n;
     const int tid = threadIdx.x;
-    if (conv.dyn && ar && n <= 8192 && n % 4 == 0) {
-        // (the same two passes as below; the residual term is the convolution)
-        constexpr int kVec = 8;
-        const int t = blockIdx.x, ks = conv.kernel_size, n_groups = n / conv.group_size;
-        const float *dyn_t = conv.dyn + (static_cast<size_t>(t) * 2 + 1) * ks * n_groups;
-        const float *base1 = conv.base + static_cast<size_t>(ks) * n;
-        f4 v[kVec];
-        float s = 0.0f;
-#pragma unroll
-        for (int j = 0; j < kVec; j++) {
-            const int i = 4 * (tid + 256 * j);
-            v[j] = f4{0, 0, 0, 0};
-            if (i < n) {
-                f4 acc = {0, 0, 0, 0};
-                // (the four channels' groups, once per vector: one division when the group size is a multiple of four)
-                int grp[4];
-                grp[0] = i / conv.group_size;
-                if (conv.group_size % 4 == 0) {
-                    grp[1] = grp[2] = grp[3] = grp[0];
-                } else {
-#pragma unroll
-                    for (int e = 1; e < 4; e++) grp[e] = (i + e) / conv.group_size;
-                }
-                for (int tap = 0; tap < ks && tap <= t; tap++) {
-                    const f4 b = *reinterpret_cast<const f4 *>(base1 + static_cast<size_t>(tap) * n + i);
-                    const f4 src = *reinterpret_cast<const f4 *>(add + static_cast<size_t>(t - tap) * n + i);
-                    const float *dg = dyn_t + static_cast<size_t>(tap) * n_groups;
-#pragma unroll
-                    for (int e = 0; e < 4; e++) acc[e] = __builtin_fmaf(b[e] + dg[grp[e]], src[e], acc[e]);
-                }
-                v[j] = *reinterpret_cast<const f4 *>(xr + i) + acc;
-                *reinterpret_cast<f4 *>(xr + i) = v[j];
-            }
-            s += (v[j][0] * v[j][0] + v[j][1] * v[j][1]) + (v[j][2] * v[j][2] + v[j][3] * v[j][3]);
-        }
-        s = block_sum(s, sh);
-        const float scale = 1.0f / sqrtf(s / static_cast<float>(n) + eps);
-#pragma unroll
-        for (int j = 0; j < kVec; j++) {
-            const int i = 4 * (tid + 256 * j);
-            if (i < n) {
-                const f4 o = v[j] * scale * *reinterpret_cast<const f4 *>(w + i);
-                *reinterpret_cast<f4 *>(yr + i) = o;
-                if (y_xf)
-                    dfl_xf_store_pair(static_cast<uint8_t *>(y_xf) + (blockIdx.x >> 4) * xf_stride, y_xf_kind, blockIdx.x & 15, i & ~7, o[0],
-                                      o[1], o[2], o[3]);
-            }
-        }
-        return;
-    }
-    if (n <= 8192 && n % 4 == 0) {
-        // (vectors past the row are zeros and add nothing: a row of up to 4096 values sums exactly as with four vectors)
-        constexpr int kVec = 8;
-        f4 v[kVec], wv[kVec];
-        float s = 0.0f;
-#pragma unroll
-        for (int j = 0; j < kVec; j++) {
-            const int i = 4 * (tid + 256 * j);
-            v[j] = f4{0, 0, 0, 0};
-            if (i < n) {
-                v[j] = *reinterpret_cast<const f4 *>(xr + i);
-                if (ar) v[j] += *reinterpret_cast<const f4 *>(ar + i);
-            }
-        }
-        // (the weights are asked for ahead of the sum's barrier, but behind the row: vector loads return in the order of
-        // their issue, and the row is what the sum waits for)
-#pragma unroll
-        for (int j = 0; j < kVec; j++) {
-            const int i = 4 * (tid + 256 * j);
-            wv[j] = i < n ? *reinterpret_cast<const f4 *>(w + i) : f4{0, 0, 0, 0};
-        }
-#pragma unroll
-        for (int j = 0; j < kVec; j++) {
-            const int i = 4 * (tid + 256 * j);
-            if (i < n && ar) *reinterpret_cast<f4 *>(xr + i) = v[j];
-            s += (v[j][0] * v[j][0] + v[j][1] * v[j][1]) + (v[j][2] * v[j][2] + v[j][3] * v[j][3]);
-        }
-        s = block_sum(s, sh);
-        const float scale = 1.0f / sqrtf(s / static_cast<float>(n) + eps);
-        float dot = 0.0f;
-#pragma unroll
-        for (int j = 0; j < kVec; j++) {
-            const int i = 4 * (tid + 256 * j);
-            if (i < n) {
-                const f4 o = v[j] * scale * wv[j];
-                *reinterpret_cast<f4 *>(yr + i) = o;
-                // (the host passes y_xf only for n a multiple of 256: whole waves are inside or outside the row)
-                // (more than sixteen rows: block b of sixteen at y_xf + b * xf_stride bytes)
-                if (y_xf)
-                    dfl_xf_store_pair(static_cast<uint8_t *>(y_xf) + (blockIdx.x >> 4) * xf_stride, y_xf_kind, blockIdx.x & 15, i & ~7, o[0],
-                                      o[1], o[2], o[3]);
-                if (gate_w) {
-                    const f4 gw = *reinterpret_cast<const f4 *>(gate_w + i);
-                    dot += (o[0] * gw[0] + o[1] * gw[1]) + (o[2] * gw[2] + o[3] * gw[3]);
-                }
-            }
-        }
-        if (gate_w) {
-            dot = block_sum(dot, sh);
-            if (tid == 0) gate_out[blockIdx.x] = 1.0f / (1.0f + expf(-dot));
-        }
-        return;
-    }
     float s = 0.0f;
     for (int i = tid; i < n; i += 256) {
         float v = xr[i];
@@ -194,6 +201,31 @@ __global__ void __launch_bounds__(256) rms_norm_kernel(float *__restrict__ x, co
     }
 }
 
+void rms_norm(int rows, hipStream_t st, float *x, const float *add, const float *w, float *y, int n, float eps, const float *gate_w,
+              float *gate_out, void *y_xf = nullptr, int y_xf_kind = 0, size_t xf_stride = 0, ConvResid conv = ConvResid()) {
+    if (!norm_in_registers(n)) {
+        rms_norm_any_kernel<<<rows, 256, 0, st>>>(x, add, w, y, n, eps, gate_w, gate_out);
+        return;
+    }
+#define DFL_NORM(V)                                                                                                          \
+    do {                                                                                                                     \
+        if (conv.dyn && add)                                                                                                 \
+            rms_norm_kernel<V, true><<<rows, 256, 0, st>>>(x, add, w, y, n, eps, gate_w, gate_out, y_xf, y_xf_kind, xf_stride, conv); \
+        else                                                                                                                 \
+            rms_norm_kernel<V, false><<<rows, 256, 0, st>>>(x, add, w, y, n, eps, gate_w, gate_out, y_xf, y_xf_kind, xf_stride, conv); \
+    } while (0)
+    switch ((n + 1023) / 1024) {
+        case 1: DFL_NORM(1); break;
+        case 2: DFL_NORM(2); break;
+        case 3: DFL_NORM(3); break;
+        case 4: DFL_NORM(4); break;
+        case 5: DFL_NORM(5); break;
+        case 6: DFL_NORM(6); break;
+        default: DFL_NORM(8); break;
+    }
+#undef DFL_NORM
+}
+
 // kernel_qk_rms_norm_rope_f32_packed_consecutive (attn.metal:137-196) + the f32 -> f16 KV scatter
 // (elementwise.metal:674-685).  One wave per (row, head): per-head RMSNorm (weight may be null),
 // NeoX RoPE over the full head (pairs (i, i + hd/2), angle = pos / theta^(2i/hd)).
@@ -201,87 +233,176 @@ __global__ void __launch_bounds__(256) rms_norm_kernel(float *__restrict__ x, co
 // as f16 into k_dst[pos][kv head][:] (k_dst == null: rewritten in place as f32 instead).
 // With vt_dst, n_kv more workgroups per row scatter the row's V heads, as f16, into column
 // pos[row] of the transposed cache [kv head][dim][capacity].
+// A lane's rotation pairs of one head: pair k is elements (i, i + HD/2), i = lane + 64 k (heads of 64: lanes 0..31).
+template <int HD>
+struct RopePairs {
+    static constexpr int N = HD <= 128 ? 1 : 2, kEl = HD / 64;  // pairs, elements per lane
+    float sn[N], cs[N];
+    __device__ __forceinline__ void angles(int lane, float theta, float pos) {
+#pragma unroll
+        for (int k = 0; k < N; k++) {
+            const int i = HD == 64 ? (lane & 31) : lane + 64 * k;
+            const float freq = pos / powf(theta, static_cast<float>(2 * i) / static_cast<float>(HD));
+            sincosf(freq, &sn[k], &cs[k]);
+        }
+    }
+};
+// ... and the head's values: element lane + 64 k in r[k], its norm weight in wr[k] (heads of 64: a lane also holds the
+// other element of its pair)
+template <int HD>
+struct RopeHead {
+    static constexpr int kEl = HD / 64;
+    float r[kEl], wr[kEl], r_far = 0.0f, w_far = 1.0f;
+    __device__ __forceinline__ void load(const float *v, const float *w, int lane) {
+#pragma unroll
+        for (int k = 0; k < kEl; k++) r[k] = v[lane + 64 * k];
+        if (HD == 64) r_far = v[lane ^ 32];
+#pragma unroll
+        for (int k = 0; k < kEl; k++) wr[k] = w ? w[lane + 64 * k] : 1.0f;
+        if (HD == 64) w_far = w ? w[lane ^ 32] : 1.0f;
+    }
+    // norm, weight (where there is one), rotation; put(i, value) for elements i and i + HD / 2 of every pair
+    template <typename Put>
+    __device__ __forceinline__ void finish(const RopePairs<HD> &t, bool weighted, int lane, float eps, Put put) const {
+        float s = r[0] * r[0];
+#pragma unroll
+        for (int k = 1; k < kEl; k++) s = __builtin_fmaf(r[k], r[k], s);
+        for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+        const float scale = 1.0f / sqrtf(s / static_cast<float>(HD) + eps);
+#pragma unroll
+        for (int k = 0; k < RopePairs<HD>::N; k++) {
+            constexpr int kFar = HD / 128;  // the partner's register, from k on
+            float a = r[k] * scale, b = (HD == 64 ? r_far : r[k + (HD == 64 ? 0 : kFar)]) * scale;
+            if (weighted) {
+                a *= wr[k];
+                b *= HD == 64 ? w_far : wr[k + (HD == 64 ? 0 : kFar)];
+            }
+            // (spelled out, so that the two kernels round alike; and a key's value is rounded to f32 before it is to f16)
+            float ra = __builtin_fmaf(a, t.cs[k], -(b * t.sn[k])), rb = __builtin_fmaf(b, t.cs[k], a * t.sn[k]);
+            asm volatile("" : "+v"(ra), "+v"(rb));
+            if (HD > 64 || lane < 32) put(lane + 64 * k, ra, rb);
+        }
+    }
+};
+
+// What bounds it: one trip to memory and the arithmetic of the angles (powf, sincosf), which wait for nothing but the
+// position: they run while the head's values are on their way.
+template <int HD>
 __global__ void __launch_bounds__(64)
     qk_norm_rope_kernel(const float *q_in, int64_t q_ld, const float *k_in, int64_t k_ld, float *q_out, float *k_out,
                         const float *__restrict__ q_w, const float *__restrict__ k_w, _Float16 *__restrict__ k_dst,
-                        const int32_t *__restrict__ pos, int n_q, int n_kv, int hd, float eps, float theta,
+                        const int32_t *__restrict__ pos, int n_q, int n_kv, float eps, float theta,
                         const float *__restrict__ v_src, int64_t v_ld, _Float16 *__restrict__ vt_dst, int64_t capacity) {
     const int row = blockIdx.y, head = blockIdx.x, lane = threadIdx.x;
     if (head >= n_q + n_kv) {
         const int vh = head - n_q - n_kv;
-        const float *src = v_src + static_cast<size_t>(row) * v_ld + static_cast<size_t>(vh) * hd;
-        _Float16 *dst = vt_dst + static_cast<size_t>(vh) * hd * capacity + pos[row];
-        for (int i = lane; i < hd; i += 64) dst[static_cast<size_t>(i) * capacity] = static_cast<_Float16>(src[i]);
+        const float *src = v_src + static_cast<size_t>(row) * v_ld + static_cast<size_t>(vh) * HD;
+        float r[HD / 64];
+#pragma unroll
+        for (int k = 0; k < HD / 64; k++) r[k] = src[lane + 64 * k];
+        _Float16 *dst = vt_dst + static_cast<size_t>(vh) * HD * capacity + pos[row];
+#pragma unroll
+        for (int k = 0; k < HD / 64; k++) dst[static_cast<size_t>(lane + 64 * k) * capacity] = static_cast<_Float16>(r[k]);
         return;
     }
     const bool is_q = head < n_q;
     // input rows may be slices of a wider matrix (row strides q_ld, k_ld); outputs are dense.  In
-    // place (q_out == q_in with a dense q_ld) is fine: a lane reads its two elements before it
-    // writes them.
-    const float *v = is_q ? q_in + static_cast<size_t>(row) * q_ld + static_cast<size_t>(head) * hd
-                          : k_in + static_cast<size_t>(row) * k_ld + static_cast<size_t>(head - n_q) * hd;
-    float *o = is_q ? q_out + (static_cast<size_t>(row) * n_q + head) * hd
-                    : (k_dst ? nullptr : k_out + (static_cast<size_t>(row) * n_kv + (head - n_q)) * hd);
+    // place (q_out == q_in with a dense q_ld) is fine: a wave reads its head before it writes it.
+    const float *v = is_q ? q_in + static_cast<size_t>(row) * q_ld + static_cast<size_t>(head) * HD
+                          : k_in + static_cast<size_t>(row) * k_ld + static_cast<size_t>(head - n_q) * HD;
+    float *o = is_q ? q_out + (static_cast<size_t>(row) * n_q + head) * HD
+                    : (k_dst ? nullptr : k_out + (static_cast<size_t>(row) * n_kv + (head - n_q)) * HD);
     const float *w = is_q ? q_w : k_w;
-    const int half = hd / 2;
-    // heads of 128 or 256: a lane's two or four elements stay in registers between the two passes (element lane + 64 k
-    // in r[k]; the partner of element i is i + half = r[k + half / 64]); same sums in the same order as the loops.
-    // The norm's weights and the position are asked for right behind them (vector loads return in the order of their
-    // issue: the elements, which the sum waits for, first), not after the sum: one trip to memory instead of two.
-    const bool in_regs = hd == 256 || hd == 128;
-    float r[4] = {0.0f, 0.0f, 0.0f, 0.0f}, wr[4] = {1.0f, 1.0f, 1.0f, 1.0f};
-    float s = 0.0f;
-    if (in_regs) {
-#pragma unroll
-        for (int k = 0; k < 4; k++)
-            if (lane + 64 * k < hd) r[k] = v[lane + 64 * k];
-        if (w) {
-#pragma unroll
-            for (int k = 0; k < 4; k++)
-                if (lane + 64 * k < hd) wr[k] = w[lane + 64 * k];
-        }
-    }
+    RopeHead<HD> h;
+    h.load(v, w, lane);
     const int32_t pos_row = pos[row];
-    if (in_regs) {
-#pragma unroll
-        for (int k = 0; k < 4; k++)
-            if (lane + 64 * k < hd) s += r[k] * r[k];
-    } else {
-        for (int i = lane; i < hd; i += 64) s += v[i] * v[i];
-    }
-    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-    const float scale = 1.0f / sqrtf(s / static_cast<float>(hd) + eps);
-    const float p = static_cast<float>(pos_row);
-    for (int i = lane, k = 0; i < half; i += 64, k++) {
-        float a, b;
-        if (in_regs) {
-            a = (k == 0 ? r[0] : r[1]) * scale;
-            b = (hd == 256 ? (k == 0 ? r[2] : r[3]) : r[1]) * scale;
-            if (w) {
-                a *= k == 0 ? wr[0] : wr[1];
-                b *= hd == 256 ? (k == 0 ? wr[2] : wr[3]) : wr[1];
-            }
-        } else {
-            a = v[i] * scale;
-            b = v[i + half] * scale;
-            if (w) {
-                a *= w[i];
-                b *= w[i + half];
-            }
-        }
-        const float freq = p / powf(theta, static_cast<float>(2 * i) / static_cast<float>(hd));
-        float sn, cs;
-        sincosf(freq, &sn, &cs);
-        const float ra = a * cs - b * sn, rb = a * sn + b * cs;
+    RopePairs<HD> t;
+    t.angles(lane, theta, static_cast<float>(pos_row));
+    _Float16 *dst = k_dst + (static_cast<size_t>(pos_row) * n_kv + (head - n_q)) * HD;
+    h.finish(t, w != nullptr, lane, eps, [&](int i, float ra, float rb) {
         if (o) {
             o[i] = ra;
-            o[i + half] = rb;
+            o[i + HD / 2] = rb;
         } else {
-            _Float16 *dst = k_dst + (static_cast<size_t>(pos_row) * n_kv + (head - n_q)) * hd;
             dst[i] = static_cast<_Float16>(ra);
-            dst[i + half] = static_cast<_Float16>(rb);
+            dst[i + HD / 2] = static_cast<_Float16>(rb);
         }
+    });
+}
+
+void qk_norm_rope(int hd, int heads, int rows, hipStream_t st, const float *q_in, int64_t q_ld, const float *k_in, int64_t k_ld, float *q_out,
+                  float *k_out, const float *q_w, const float *k_w, _Float16 *k_dst, const int32_t *pos, int n_q, int n_kv, float eps,
+                  float theta, const float *v_src, int64_t v_ld, _Float16 *vt_dst, int64_t capacity) {
+    const auto fn = hd == 64 ? qk_norm_rope_kernel<64> : hd == 128 ? qk_norm_rope_kernel<128> : qk_norm_rope_kernel<256>;
+    fn<<<dim3(heads, rows), 64, 0, st>>>(q_in, q_ld, k_in, k_ld, q_out, k_out, q_w, k_w, k_dst, pos, n_q, n_kv, eps, theta, v_src, v_ld,
+                                         vt_dst, capacity);
+}
+
+// The same for the rows of a prefill group, positions pos0 .. pos0 + n - 1, q | k | v side by side in pk: with this many
+// rows the angles' arithmetic is what there is most of, so a wave takes kRopeHeads heads of its row and computes them
+// once; and V goes through LDS, 32 rows of a head per workgroup, so that the transposed cache is written in runs of 32
+// positions (element by element before: 45 -> 21 us for 2048 rows of 16 + 2 + 2 heads of 256).
+constexpr int kRopeHeads = 6, kVRows = 32;
+template <int HD>
+__global__ void __launch_bounds__(256)
+    group_norm_rope_kernel(const float *__restrict__ pk, int64_t ld, float *__restrict__ q_out, const float *__restrict__ q_w,
+                           const float *__restrict__ k_w, _Float16 *__restrict__ k_dst, int64_t pos0, int n_rows, int n_q, int n_kv, float eps,
+                           float theta, _Float16 *__restrict__ vt_dst, int64_t capacity, int n_head_groups, int rope_blocks) {
+    __shared__ _Float16 tile[kVRows][HD + 2];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if (static_cast<int>(blockIdx.x) >= rope_blocks) {
+        const int b = blockIdx.x - rope_blocks, vh = b % n_kv, row0 = b / n_kv * kVRows, rows = min(kVRows, n_rows - row0);
+        const float *src = pk + static_cast<size_t>(row0) * ld + static_cast<size_t>(n_q + n_kv + vh) * HD;
+        constexpr int kPerRow = HD / 4;  // float4 per row
+#pragma unroll
+        for (int j = 0; j < kVRows * kPerRow / 256; j++) {
+            const int e = tid + 256 * j, r = e / kPerRow, c = e % kPerRow;
+            const norm_f4 f = *reinterpret_cast<const norm_f4 *>(src + static_cast<size_t>(min(r, rows - 1)) * ld + 4 * c);
+#pragma unroll
+            for (int i = 0; i < 4; i++) tile[r][4 * c + i] = static_cast<_Float16>(f[i]);
+        }
+        __syncthreads();
+        const int r = tid & (kVRows - 1);
+        _Float16 *dst = vt_dst + static_cast<size_t>(vh) * HD * capacity + pos0 + row0 + r;
+        if (r < rows)
+            for (int d = tid / kVRows; d < HD; d += 256 / kVRows) dst[static_cast<size_t>(d) * capacity] = tile[r][d];
+        return;
     }
+    const int row = blockIdx.x / n_head_groups * 4 + wave, head0 = blockIdx.x % n_head_groups * kRopeHeads;
+    if (row >= n_rows) return;
+    const int head1 = min(head0 + kRopeHeads, n_q + n_kv);
+    const int64_t pos = pos0 + row;
+    const float *v = pk + static_cast<size_t>(row) * ld;
+    auto weights = [&](int head) { return head < n_q ? q_w : k_w; };
+    RopeHead<HD> h;
+    h.load(v + static_cast<size_t>(head0) * HD, weights(head0), lane);
+    RopePairs<HD> t;
+    t.angles(lane, theta, static_cast<float>(static_cast<int32_t>(pos)));
+    for (int head = head0; head < head1; head++) {
+        RopeHead<HD> next;  // (the next head's values are on their way meanwhile)
+        const int ahead = min(head + 1, head1 - 1);
+        next.load(v + static_cast<size_t>(ahead) * HD, weights(ahead), lane);
+        float *o = q_out + (static_cast<size_t>(row) * n_q + head) * HD;
+        _Float16 *dst = k_dst + (static_cast<size_t>(pos) * n_kv + (head - n_q)) * HD;
+        h.finish(t, weights(head) != nullptr, lane, eps, [&](int i, float ra, float rb) {
+            if (head < n_q) {
+                o[i] = ra;
+                o[i + HD / 2] = rb;
+            } else {
+                dst[i] = static_cast<_Float16>(ra);
+                dst[i + HD / 2] = static_cast<_Float16>(rb);
+            }
+        });
+        h = next;
+    }
+}
+
+void group_norm_rope(int hd, hipStream_t st, const float *pk, int64_t ld, float *q_out, const float *q_w, const float *k_w, _Float16 *k_dst,
+                     int64_t pos0, int n_rows, int n_q, int n_kv, float eps, float theta, _Float16 *vt_dst, int64_t capacity) {
+    const auto fn = hd == 64 ? group_norm_rope_kernel<64> : hd == 128 ? group_norm_rope_kernel<128> : group_norm_rope_kernel<256>;
+    const int head_groups = (n_q + n_kv + kRopeHeads - 1) / kRopeHeads, rope_blocks = (n_rows + 3) / 4 * head_groups;
+    fn<<<rope_blocks + (n_rows + kVRows - 1) / kVRows * n_kv, 256, 0, st>>>(pk, ld, q_out, q_w, k_w, k_dst, pos0, n_rows, n_q, n_kv, eps, theta,
+                                                                             vt_dst, capacity, head_groups, rope_blocks);
 }
 
 // kernel_silu_mul_f32 (elementwise.metal:193): g = silu(g) * u
@@ -336,12 +457,9 @@ constexpr int kGroupIdsPerLaunch = 512;
 struct IntGroupArgs {
     int32_t v[kGroupIdsPerLaunch];
 };
-__global__ void set_group_ids_pos_kernel(IntGroupArgs ids, int start, int n, int32_t *__restrict__ ids_dst, int32_t *__restrict__ pos_dst) {
+__global__ void set_group_ids_kernel(IntGroupArgs ids, int n, int32_t *__restrict__ ids_dst) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) {
-        ids_dst[i] = ids.v[i];
-        pos_dst[i] = start + i;
-    }
+    if (i < n) ids_dst[i] = ids.v[i];
 }
 
 // kernel_add_inplace_f32 (elementwise.metal:89)
@@ -649,7 +767,7 @@ struct PrefillGroup {
     float *x = nullptr, *cur = nullptr, *mix = nullptr, *pk = nullptr, *q = nullptr, *attn = nullptr;
     uint8_t *xf_cur = nullptr, *xf_attn = nullptr, *xf_g = nullptr;  // rows in fragment order ...
     uint8_t *xs_cur = nullptr, *xs_attn = nullptr, *xs_g = nullptr;  // ... and their sub-block sums
-    int32_t *ids = nullptr, *pos = nullptr;
+    int32_t *ids = nullptr;
     dfl_moe_group_scratch moe;
 };
 struct PrefillPipe {
@@ -761,7 +879,7 @@ int32_t dflash_session_create(dflash_ctx *ctx, const dflash_model_cfg *cfg, int6
 
 namespace {
 void prefill_group_free(PrefillGroup *g) {
-    void *ptrs[] = {g->x, g->cur, g->mix, g->pk, g->q, g->attn, g->xf_cur, g->xf_attn, g->xf_g, g->xs_cur, g->xs_attn, g->xs_g, g->ids, g->pos,
+    void *ptrs[] = {g->x, g->cur, g->mix, g->pk, g->q, g->attn, g->xf_cur, g->xf_attn, g->xf_g, g->xs_cur, g->xs_attn, g->xs_g, g->ids,
                     g->moe.logits, g->moe.sg, g->moe.sel_e, g->moe.sel_w, g->moe.pick_pos, g->moe.n_slots, g->moe.slot_rows, g->moe.tiles,
                     g->moe.n_tiles, g->moe.xg, g->moe.xg_sums, g->moe.act, g->moe.act_sums, g->moe.eo};
     for (void *p : ptrs)
@@ -798,8 +916,7 @@ void prefill_group_alloc(dflash_session *s, PrefillGroup *g) {
     bool ok = dev_alloc(&g->x, R * H) && dev_alloc(&g->cur, R * H) && dev_alloc(&g->mix, R * H) &&
               dev_alloc(&g->pk, R * (q_dim + 2 * kv_dim)) && dev_alloc(&g->q, R * q_dim) && dev_alloc(&g->attn, R * q_dim) &&
               dev_alloc(&g->xf_cur, nb * dfl_xf_bytes(H)) && dev_alloc(&g->xf_attn, nb * dfl_xf_bytes(q_dim)) &&
-              dev_alloc(&g->xs_cur, nb * dfl_xs_bytes(H)) && dev_alloc(&g->xs_attn, nb * dfl_xs_bytes(q_dim)) && dev_alloc(&g->ids, R) &&
-              dev_alloc(&g->pos, R);
+              dev_alloc(&g->xs_cur, nb * dfl_xs_bytes(H)) && dev_alloc(&g->xs_attn, nb * dfl_xs_bytes(q_dim)) && dev_alloc(&g->ids, R);
     if (ok && !moe) ok = dev_alloc(&g->xf_g, nb * dfl_xf_bytes(F)) && dev_alloc(&g->xs_g, nb * dfl_xs_bytes(F));
     if (ok && moe) {
         const size_t S = dfl_moe_group_max_slots(c, rows), E = c.n_expert, fe = c.ffn_expert;
@@ -945,7 +1062,7 @@ int32_t verify_enqueue(dflash_ctx *ctx, const dflash_model *model, dflash_sessio
         const bool moe = c.n_expert > 0;
         const LayerXf xk = layer_kinds(il);
         if (!cur_ready)
-            rms_norm_kernel<<<n, 256, 0, st>>>(s->x, pending_resid, L.attn_norm, s->cur, H, c.eps, nullptr, nullptr,
+            rms_norm(n, st, s->x, pending_resid, L.attn_norm, s->cur, H, c.eps, nullptr, nullptr,
                                                xk.qkv ? s->xf_cur : nullptr, xk.qkv);
         pending_resid = nullptr;
         cur_ready = false;
@@ -953,9 +1070,8 @@ int32_t verify_enqueue(dflash_ctx *ctx, const dflash_model *model, dflash_sessio
         if ((rc = gemm_qkv(ctx, L.wq, L.wk, L.wv, s->cur, s->q, s->k, s->v, s->pk, true, &packed, H, q_dim, kv_dim, n, st, s->xf_cur, xk.qkv)))
             return rc;
         const int64_t tot = q_dim + 2 * kv_dim;
-        qk_norm_rope_kernel<<<dim3(c.n_q + 2 * c.n_kv, n), 64, 0, st>>>(
-            packed ? s->pk : s->q, packed ? tot : q_dim, packed ? s->pk + q_dim : s->k, packed ? tot : kv_dim, s->q, s->k, L.q_norm,
-            L.k_norm, kc, s->pos, c.n_q, c.n_kv, hd, c.eps, c.rope_theta, packed ? s->pk + q_dim + kv_dim : s->v,
+        qk_norm_rope(hd, c.n_q + 2 * c.n_kv, n, st, packed ? s->pk : s->q, packed ? tot : q_dim, packed ? s->pk + q_dim : s->k, packed ? tot : kv_dim, s->q, s->k, L.q_norm,
+            L.k_norm, kc, s->pos, c.n_q, c.n_kv, c.eps, c.rope_theta, packed ? s->pk + q_dim + kv_dim : s->v,
             packed ? tot : kv_dim, vtc, s->capacity);
         if (lane) {
             // This block's K/V rows of the layer are written; the earlier blocks' must be before the attention reads
@@ -986,7 +1102,7 @@ int32_t verify_enqueue(dflash_ctx *ctx, const dflash_model *model, dflash_sessio
         // s->mix together with the experts' sum)
         const bool norm_in_router = moe && dfl_moe_norm_fusable(ctx, c, L, n);
         if (!norm_in_router)
-            rms_norm_kernel<<<n, 256, 0, st>>>(s->x, s->mix, L.post_norm, s->cur, H, c.eps, moe ? L.shexp_gate : nullptr,
+            rms_norm(n, st, s->x, s->mix, L.post_norm, s->cur, H, c.eps, moe ? L.shexp_gate : nullptr,
                                                moe ? s->moe.sg : nullptr, xk.gate_up ? s->xf_cur : nullptr, xk.gate_up);
         if (moe) {
             const float *next_w = il + 1 < c.n_layers ? model->layers[il + 1].attn_norm : model->output_norm;
@@ -1019,7 +1135,7 @@ int32_t verify_enqueue(dflash_ctx *ctx, const dflash_model *model, dflash_sessio
     }
     if (want_head) {  // (not for a caller that asked for no output of it: a prefill block wants K/V and the taps only)
         if (!cur_ready)
-            rms_norm_kernel<<<n, 256, 0, st>>>(s->x, pending_resid, model->output_norm, s->cur, H, c.eps, nullptr, nullptr,
+            rms_norm(n, st, s->x, pending_resid, model->output_norm, s->cur, H, c.eps, nullptr, nullptr,
                                                head_kind ? s->xf_cur : nullptr, head_kind);
         if (head_kind)
             rc = dfl_gemm_whole(ctx, model->output.type, model->output.data, s->xf_cur, lg, H, c.vocab, n, 0, nullptr, DFL_XF_NONE, st);
@@ -1305,7 +1421,7 @@ int32_t prefill_group_enqueue(dflash_ctx *ctx, const dflash_model *model, dflash
         const int m = std::min(kGroupIdsPerLaunch, n - at);
         IntGroupArgs ids_arg = {};
         for (int i = 0; i < m; i++) ids_arg.v[i] = tokens[at + i];
-        set_group_ids_pos_kernel<<<(m + 255) / 256, 256, 0, st>>>(ids_arg, static_cast<int>(start) + at, m, g.ids + at, g.pos + at);
+        set_group_ids_kernel<<<(m + 255) / 256, 256, 0, st>>>(ids_arg, m, g.ids + at);
     }
     int32_t rc = embed_rows(ctx, model->token_embd, g.ids, n, H, g.x, st);
     if (rc) return rc;
@@ -1324,12 +1440,10 @@ int32_t prefill_group_enqueue(dflash_ctx *ctx, const dflash_model *model, dflash
         _Float16 *kc = s->k_cache + il * per_layer, *vtc = s->vt_cache + il * per_layer;
         next_rows = il + 1 < c.n_layers ? layer_rows(ctx, c, model->layers[il + 1]) : LayerRows();
         if (!moe || il == 0)  // (a mixture's later layers: the experts' last kernel has normalised their input)
-            rms_norm_kernel<<<n, 256, 0, st>>>(g.x, pending_resid, L.attn_norm, g.cur, H, c.eps, nullptr, nullptr, g.xf_cur, rows.qkv.kind, xf_h);
+            rms_norm(n, st, g.x, pending_resid, L.attn_norm, g.cur, H, c.eps, nullptr, nullptr, g.xf_cur, rows.qkv.kind, xf_h);
         pending_resid = nullptr;
         if ((rc = product(rows.qkv, L.wq, g.xf_cur, g.xs_cur, g.pk, H, tot))) return rc;
-        qk_norm_rope_kernel<<<dim3(c.n_q + 2 * c.n_kv, n), 64, 0, st>>>(g.pk, tot, g.pk + q_dim, tot, g.q, nullptr, L.q_norm, L.k_norm, kc,
-                                                                      g.pos, c.n_q, c.n_kv, hd, c.eps, c.rope_theta,
-                                                                      g.pk + q_dim + kv_dim, tot, vtc, s->capacity);
+        group_norm_rope(hd, st, g.pk, tot, g.q, L.q_norm, L.k_norm, kc, start, n, c.n_q, c.n_kv, c.eps, c.rope_theta, vtc, s->capacity);
         bool tapped = false;
         for (int t = 0; t < n_taps; t++) tapped = tapped || tap_layers[t] == il;
         // nothing of the last layer beyond its K/V rows is needed unless its residual is tapped (as in verify_enqueue)
@@ -1341,12 +1455,12 @@ int32_t prefill_group_enqueue(dflash_ctx *ctx, const dflash_model *model, dflash
         if (moe) {
             const float *next_w = il + 1 < c.n_layers ? model->layers[il + 1].attn_norm : model->output_norm;
             // x += mix, the experts' norm and the shared-expert gates: the block path's norm kernel over all the rows
-            rms_norm_kernel<<<n, 256, 0, st>>>(g.x, g.mix, L.post_norm, g.cur, H, c.eps, L.shexp_gate, g.moe.sg);
+            rms_norm(n, st, g.x, g.mix, L.post_norm, g.cur, H, c.eps, L.shexp_gate, g.moe.sg);
             if ((rc = dfl_moe_ffn_group(ctx, c, L, g.x, g.cur, n, g.moe, next_w, next_rows.qkv.kind ? g.xf_cur : nullptr, next_rows.qkv.kind, xf_h,
                                         st)))
                 return rc;
         } else {
-            rms_norm_kernel<<<n, 256, 0, st>>>(g.x, g.mix, L.post_norm, g.cur, H, c.eps, nullptr, nullptr, g.xf_cur, rows.gate_up.kind, xf_h);
+            rms_norm(n, st, g.x, g.mix, L.post_norm, g.cur, H, c.eps, nullptr, nullptr, g.xf_cur, rows.gate_up.kind, xf_h);
             if (!rows.gate_up.twin && (rc = dfl_xf_sums(ctx, g.xf_cur, H, n_blocks, g.xs_cur, st))) return rc;
             // silu(gate) * up straight into fragment order, with the sums the down product wants
             if ((rc = dfl_gemm_rows(ctx, rows.gate_up, L.gate.type, L.gate.data, g.xf_cur, g.xs_cur, nullptr, H, 2ll * c.ffn, n, c.ffn, g.xf_g,
@@ -1597,7 +1711,7 @@ int32_t draft_prepare(dflash_ctx *ctx, const dflash_draft_head *head, dflash_dra
     for (int64_t c0 = s->ctx_h_ready; c0 < s->ctx_len; c0 += 16) {
         const int m = static_cast<int>(std::min<int64_t>(16, s->ctx_len - c0));
         if ((rc = gemm(ctx, head->fc, s->ctx_raw + c0 * feat, s->tmp, feat, H, m, st))) return rc;
-        rms_norm_kernel<<<m, 256, 0, st>>>(s->tmp, nullptr, head->hidden_norm, s->ctx_h + c0 * H, H, c.eps, nullptr, nullptr);
+        rms_norm(m, st, s->tmp, nullptr, head->hidden_norm, s->ctx_h + c0 * H, H, c.eps, nullptr, nullptr);
     }
     // Every layer's K/V projection reads the same rows (ctx_h): when the layers' [wk; wv] pairs are Q4_K matrices
     // an equal distance apart (the loader put all layers' q/k/v in one allocation), they run as ONE batched GEMM,
@@ -1650,10 +1764,8 @@ int32_t draft_prepare(dflash_ctx *ctx, const dflash_draft_head *head, dflash_dra
                 if ((rc = gemm(ctx, L.wk, s->ctx_h + c0 * H, kc + c0 * kv_dim, H, kv_dim, m, st))) return rc;
                 if ((rc = gemm(ctx, L.wv, s->ctx_h + c0 * H, vc + c0 * kv_dim, H, kv_dim, m, st))) return rc;
             }
-            qk_norm_rope_kernel<<<dim3(c.n_kv, m), 64, 0, st>>>(nullptr, 0, kv_packed ? s->pk : kc + c0 * kv_dim,
-                                                               kv_packed ? 2 * kv_dim : kv_dim, nullptr, kc + c0 * kv_dim, nullptr,
-                                                               L.k_norm, nullptr, s->pos_ctx + c0, 0, c.n_kv, hd, c.eps,
-                                                               c.rope_theta, nullptr, 0, nullptr, 0);
+            qk_norm_rope(hd, c.n_kv, m, st, nullptr, 0, kv_packed ? s->pk : kc + c0 * kv_dim, kv_packed ? 2 * kv_dim : kv_dim, nullptr,
+                         kc + c0 * kv_dim, nullptr, L.k_norm, nullptr, s->pos_ctx + c0, 0, c.n_kv, c.eps, c.rope_theta, nullptr, 0, nullptr, 0);
             if (fast)
                 kv_to_f16_kernel<<<dim3(blocks_for(kv_dim), m), 256, 0, st>>>(
                     kc + c0 * kv_dim, kv_packed ? s->pk + kv_dim : vc + c0 * kv_dim, kv_packed ? 2 * kv_dim : kv_dim, k16, vt16,
@@ -1762,9 +1874,9 @@ int32_t draft_block_impl(dflash_ctx *ctx, const dflash_model *target, const dfla
 
     const float *pending_resid = nullptr;
     // DFlash-2: the side-1 convolution of a sublayer's output is what gets added to the residual; the norm kernel that
-    // adds it computes it on the way (rms_norm_kernel's ConvResid), unless the width is one that kernel keeps no row in
-    // registers for (then a launch of dflash2_conv_kernel comes first, as for the side-0 convolutions)
-    const bool conv_in_norm = conv && H <= 8192 && H % 4 == 0;
+    // adds it computes it on the way (rms_norm_kernel's ConvResid), unless the width or the group size is one that kernel is
+    // not made for (then a launch of dflash2_conv_kernel comes first, as for the side-0 convolutions)
+    const bool conv_in_norm = conv && norm_in_registers(H) && c.conv_group_size % 4 == 0;
     ConvResid pending_conv;
     for (int il = 0; il < c.n_layers; il++) {
         const dflash_draft_layer &L = head->layers[il];
@@ -1780,7 +1892,7 @@ int32_t draft_block_impl(dflash_ctx *ctx, const dflash_model *target, const dfla
         const int cp_attn = conv && fast ? dfl_whole_kind(ctx, L.conv_attn_proj.type, H, conv_dyn_dim, 0) : DFL_XF_NONE;
         const int cp_ffn = conv && fast ? dfl_whole_kind(ctx, L.conv_ffn_proj.type, H, conv_dyn_dim, 0) : DFL_XF_NONE;
         const int norm1_kind = conv ? cp_attn : xk.qkv;
-        rms_norm_kernel<<<N, 256, 0, st>>>(s->x, pending_resid, L.attn_norm, s->cur, H, c.eps, nullptr, nullptr,
+        rms_norm(N, st, s->x, pending_resid, L.attn_norm, s->cur, H, c.eps, nullptr, nullptr,
                                            norm1_kind ? s->xf_cur : nullptr, norm1_kind, 0, pending_conv);
         // DFlash-2 attention convolution (metal_dflash.rs:16210-16262): the dynamic coefficients come
         // from the normed input and serve both sides; q/k/v read the side-0 result
@@ -1802,9 +1914,8 @@ int32_t draft_block_impl(dflash_ctx *ctx, const dflash_model *target, const dfla
         if (fast) {
             // the block's own K (normed, rotated) and V go behind the context in the f16 mirror, written by the
             // same kernel (positions pos[i] = ctx_len + i on this path); one MFMA pass over context and block
-            qk_norm_rope_kernel<<<dim3(c.n_q + 2 * c.n_kv, N), 64, 0, st>>>(
-                packed ? s->pk : s->q, packed ? tot : q_dim, packed ? s->pk + q_dim : s->k, packed ? tot : kv_dim, s->q, s->k,
-                L.q_norm, L.k_norm, k16, s->pos, c.n_q, c.n_kv, hd, c.eps, c.rope_theta, packed ? s->pk + q_dim + kv_dim : s->v,
+            qk_norm_rope(hd, c.n_q + 2 * c.n_kv, N, st, packed ? s->pk : s->q, packed ? tot : q_dim, packed ? s->pk + q_dim : s->k, packed ? tot : kv_dim, s->q, s->k,
+                L.q_norm, L.k_norm, k16, s->pos, c.n_q, c.n_kv, c.eps, c.rope_theta, packed ? s->pk + q_dim + kv_dim : s->v,
                 packed ? tot : kv_dim, vt16, s->cap16);
             // (under capture the context length is pos[0], read on the device: the launches then serve every context
             // of the bucket; chunking, and so the result, is the same either way)
@@ -1814,9 +1925,8 @@ int32_t draft_block_impl(dflash_ctx *ctx, const dflash_model *target, const dfla
                                      xk.wo ? s->xf_attn : nullptr, xk.wo)))
                 return rc;
         } else {
-            qk_norm_rope_kernel<<<dim3(c.n_q + c.n_kv, N), 64, 0, st>>>(s->q, q_dim, s->k, kv_dim, s->q, s->k, L.q_norm, L.k_norm,
-                                                                     nullptr, s->pos, c.n_q, c.n_kv, hd, c.eps, c.rope_theta,
-                                                                     nullptr, 0, nullptr, 0);
+            qk_norm_rope(hd, c.n_q + c.n_kv, N, st, s->q, q_dim, s->k, kv_dim, s->q, s->k, L.q_norm, L.k_norm, nullptr, s->pos, c.n_q, c.n_kv,
+                         c.eps, c.rope_theta, nullptr, 0, nullptr, 0);
             draft_attn_kernel<<<dim3(c.n_q, N), 64, 0, st>>>(s->q, kc, vc, s->k, s->v, s->pos_ctx, static_cast<int>(s->ctx_len),
                                                             N, c.n_q, c.n_kv, hd, static_cast<int>(noise_start), c.causal,
                                                             L.is_swa ? static_cast<int>(c.swa_window) : 0, s->attn);
@@ -1839,7 +1949,7 @@ int32_t draft_block_impl(dflash_ctx *ctx, const dflash_model *target, const dfla
             resid = s->conv_buf;
         }
         const int norm2_kind = conv ? cp_ffn : xk.gate_up;
-        rms_norm_kernel<<<N, 256, 0, st>>>(s->x, resid, L.post_norm, s->cur, H, c.eps, nullptr, nullptr,
+        rms_norm(N, st, s->x, resid, L.post_norm, s->cur, H, c.eps, nullptr, nullptr,
                                            norm2_kind ? s->xf_cur : nullptr, norm2_kind, 0, resid_conv);
         const float *ffn_src = s->cur;
         if (conv) {  // the FFN pair (:16836-16885, 17003-17022)
@@ -1873,7 +1983,7 @@ int32_t draft_block_impl(dflash_ctx *ctx, const dflash_model *target, const dfla
         pending_resid = resid;  // residual 2: added by the norm that reads x next (same x + r, one launch fewer)
     }
     const int head_kind = dfl_whole_kind(ctx, target->output.type, H, V, 0);
-    rms_norm_kernel<<<N, 256, 0, st>>>(s->x, pending_resid, head->output_norm, s->cur, H, c.eps, nullptr, nullptr,
+    rms_norm(N, st, s->x, pending_resid, head->output_norm, s->cur, H, c.eps, nullptr, nullptr,
                                        head_kind ? s->xf_cur : nullptr, head_kind, 0, pending_conv);
     if (head_kind)
         rc = dfl_gemm_whole(ctx, target->output.type, target->output.data, s->xf_cur, lg, H, V, N, 0, nullptr, DFL_XF_NONE, st);

@@ -369,80 +369,101 @@ __global__ void moe_combine_slots_kernel(const float *__restrict__ eo, const int
 // attention norm or the output norm): y = x * rsqrt(mean(x^2) + eps) * norm_w.  One workgroup per
 // row, the row (hidden <= 4096, a multiple of 4) in registers; element sums and the sum of squares
 // are taken in the order of moe_combine_slots_kernel followed by the norm kernel.
+// What bounds it: two trips to memory (the picks, then their rows) and what one CU can take in, (n_used + 3) rows of
+// hidden values.  A thread asks for the rows of eight picks at once - unconditionally: past the last pick the last one
+// again, its product left out - where a loop over the picks waited for one row at a time; the picks themselves are scalar
+// loads (the same for the whole workgroup).  V: vectors of four values per thread.
+template <int V>
 __global__ void __launch_bounds__(256)
     moe_combine_norm_kernel(const float *__restrict__ eo, const int32_t *__restrict__ slot_of, const float *__restrict__ sel_w,
                             const float *__restrict__ sg, const float *__restrict__ shared, const int32_t *__restrict__ n_slots,
                             int n_used, int hidden, float *__restrict__ x, const float *__restrict__ norm_w,
                             float *__restrict__ y, float eps, const float *__restrict__ pre_add, void *__restrict__ y_xf,
-                            int y_xf_kind, int grouped = 0, size_t xf_stride = 0) {
+                            int y_xf_kind, int grouped, size_t xf_stride) {
     typedef float f4 __attribute__((ext_vector_type(4)));
     __shared__ float sh[4];
-    __shared__ float w_k[64];
-    __shared__ int32_t slot_k[64];  // row of eo that holds pick k of this row
     const int row = blockIdx.x, tid = threadIdx.x;
-    // Everything whose address depends on nothing this kernel reads is asked for first (the slot count, the gate, the
-    // residual row and the term to add to it), beside the picks: one trip to memory, then the picks' output rows.
-    const size_t n_slots_now = static_cast<size_t>(*n_slots);
-    const float gate = sg[row];
-    f4 v[4];
+    const size_t row_at = static_cast<size_t>(row) * hidden;
+    int at[V];
+    f4 v[V], pre[V], nw[V], shv[V], out[V];
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const int i = 4 * (tid + 256 * j);
-        v[j] = f4{0, 0, 0, 0};
-        if (i < hidden) {
-            v[j] = *reinterpret_cast<const f4 *>(x + static_cast<size_t>(row) * hidden + i);
-            // (a residual term the norm before this layer's experts left out: it goes in first, as it would have there)
-            if (pre_add) v[j] += *reinterpret_cast<const f4 *>(pre_add + static_cast<size_t>(row) * hidden + i);
-        }
-    }
+    for (int j = 0; j < V; j++) at[j] = min(4 * (tid + 256 * j), hidden - 4);
     // grouped (rows of several 16-row blocks, moe_group_slots_kernel): slot_of is the eo row of a pick itself, and the
     // shared expert's slots are the last gridDim.x / 16 (rounded up) of the list, one per block of rows
-    if (tid < n_used) {
-        w_k[tid] = sel_w[row * n_used + tid];
-        slot_k[tid] = grouped ? slot_of[row * n_used + tid] : slot_of[row * n_used + tid] * 16 + row;
-    }
-    __syncthreads();
+    const size_t n_slots_now = static_cast<size_t>(*n_slots);
+    const float gate = sg[row];
     const size_t last = grouped ? (n_slots_now - (gridDim.x + 15) / 16 + (row >> 4)) * 16 + (row & 15) : (n_slots_now - 1) * 16 + row;
+    const float *sh_row = shared ? shared + row_at : eo + last * hidden;
+#pragma unroll
+    for (int j = 0; j < V; j++) out[j] = f4{0, 0, 0, 0};
+    for (int k0 = 0; k0 < n_used; k0 += 8) {
+        const float *src[8];
+        float wk[8];
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            const int pick = row * n_used + min(k0 + k, n_used - 1);
+            wk[k] = sel_w[pick];
+            src[k] = eo + static_cast<size_t>(grouped ? slot_of[pick] : slot_of[pick] * 16 + row) * hidden;
+        }
+        f4 e[8][V];
+#pragma unroll
+        for (int k = 0; k < 8; k++)
+#pragma unroll
+            for (int j = 0; j < V; j++) e[k][j] = *reinterpret_cast<const f4 *>(src[k] + at[j]);
+        if (k0 == 0) {  // (what is needed after the picks, behind their rows in the order of issue)
+#pragma unroll
+            for (int j = 0; j < V; j++) {
+                shv[j] = *reinterpret_cast<const f4 *>(sh_row + at[j]);
+                v[j] = *reinterpret_cast<const f4 *>(x + row_at + at[j]);
+                if (pre_add) pre[j] = *reinterpret_cast<const f4 *>(pre_add + row_at + at[j]);
+                nw[j] = *reinterpret_cast<const f4 *>(norm_w + at[j]);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            if (k0 + k < n_used) {
+#pragma unroll
+                for (int j = 0; j < V; j++) out[j] += wk[k] * e[k][j];
+            }
+        }
+    }
     float s = 0.0f;
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const int i = 4 * (tid + 256 * j);
-        if (i < hidden) {
-            f4 out = {0, 0, 0, 0};
-            for (int k = 0; k < n_used; k++)
-                out += w_k[k] * *reinterpret_cast<const f4 *>(eo + static_cast<size_t>(slot_k[k]) * hidden + i);
-            const f4 shv = shared ? *reinterpret_cast<const f4 *>(shared + static_cast<size_t>(row) * hidden + i)
-                                  : *reinterpret_cast<const f4 *>(eo + last * hidden + i);
-            out += gate * shv;
-            v[j] += out;
-            *reinterpret_cast<f4 *>(x + static_cast<size_t>(row) * hidden + i) = v[j];
-        }
+    for (int j = 0; j < V; j++) {
+        // (a residual term the norm before this layer's experts left out: it goes in first, as it would have there)
+        if (pre_add) v[j] += pre[j];
+        out[j] += gate * shv[j];
+        v[j] += out[j];
+        if (4 * (tid + 256 * j) >= hidden) v[j] = f4{0, 0, 0, 0};
         s += (v[j][0] * v[j][0] + v[j][1] * v[j][1]) + (v[j][2] * v[j][2] + v[j][3] * v[j][3]);
-    }
-    // (the next norm's weights are asked for here, behind the picks' rows in the order of issue - loads return in that
-    // order, and these come from further away than the rows the sum is waiting for - and ahead of the barrier)
-    f4 nw[4];
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const int i = 4 * (tid + 256 * j);
-        nw[j] = i < hidden ? *reinterpret_cast<const f4 *>(norm_w + i) : f4{0, 0, 0, 0};
     }
     for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
     if ((tid & 63) == 0) sh[tid >> 6] = s;
+#pragma unroll
+    for (int j = 0; j < V; j++)
+        if (4 * (tid + 256 * j) < hidden) *reinterpret_cast<f4 *>(x + row_at + at[j]) = v[j];
     __syncthreads();
     s = ((sh[0] + sh[1]) + sh[2]) + sh[3];
     const float scale = 1.0f / sqrtf(s / static_cast<float>(hidden) + eps);
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
+    for (int j = 0; j < V; j++) {
         const int i = 4 * (tid + 256 * j);
         if (i < hidden) {
             const f4 o = v[j] * scale * nw[j];
-            *reinterpret_cast<f4 *>(y + static_cast<size_t>(row) * hidden + i) = o;
+            *reinterpret_cast<f4 *>(y + row_at + i) = o;
             // (hidden a multiple of 256 here: whole waves are inside or outside the row)
             if (y_xf)
                 dfl_xf_store_pair(static_cast<uint8_t *>(y_xf) + (row >> 4) * xf_stride, y_xf_kind, row & 15, i & ~7, o[0], o[1], o[2], o[3]);
         }
     }
+}
+
+void moe_combine_norm(int rows, hipStream_t st, const float *eo, const int32_t *slot_of, const float *sel_w, const float *sg, const float *shared,
+                      const int32_t *n_slots, int n_used, int hidden, float *x, const float *norm_w, float *y, float eps, const float *pre_add,
+                      void *y_xf, int y_xf_kind, int grouped = 0, size_t xf_stride = 0) {
+    const auto fn = hidden <= 1024 ? moe_combine_norm_kernel<1> : hidden <= 2048 ? moe_combine_norm_kernel<2> : moe_combine_norm_kernel<4>;
+    fn<<<rows, 256, 0, st>>>(eo, slot_of, sel_w, sg, shared, n_slots, n_used, hidden, x, norm_w, y, eps, pre_add, y_xf, y_xf_kind, grouped,
+                             xf_stride);
 }
 
 // ---- rows of several 16-row blocks through one pass over the experts (prefill) ----
@@ -711,7 +732,7 @@ int32_t dfl_moe_ffn(dflash_ctx *ctx, const dflash_model_cfg &c, const dflash_lay
         if ((rc = dfl_gemm_fewrow_checked(ctx, L.down.type, L.down.data, s.g, DFLASH_TYPE_F32, s.shared, fs, H, n, st))) return rc;
     }
     if (batched && next_norm_w && next_cur && next_done && H <= 4096 && H % 4 == 0) {
-        moe_combine_norm_kernel<<<n, 256, 0, st>>>(s.eo, s.slot_of, s.sel_w, s.sg, folded_shared ? nullptr : s.shared, s.n_distinct,
+        moe_combine_norm(n, st, s.eo, s.slot_of, s.sel_w, s.sg, folded_shared ? nullptr : s.shared, s.n_distinct,
                                                    used, H, x_resid, next_norm_w, next_cur, c.eps, pre_add,
                                                    H % DFL_QK_K == 0 ? next_xf : nullptr, next_xf_kind);
         *next_done = true;
@@ -769,7 +790,7 @@ int32_t dfl_moe_ffn_group(dflash_ctx *ctx, const dflash_model_cfg &c, const dfla
     if ((rc = dfl_gemm_rows_experts(ctx, L.down_exps.data, L.down.data, nullptr, nullptr, stride_dn, s.act, s.act_sums, s.tiles, s.n_tiles,
                                     max_tiles, s.eo, fe, H, nullptr, nullptr, st)))
         return rc;
-    moe_combine_norm_kernel<<<n_rows, 256, 0, st>>>(s.eo, s.pick_pos, s.sel_w, s.sg, nullptr, s.n_slots, used, H, x_resid, next_norm_w,
+    moe_combine_norm(n_rows, st, s.eo, s.pick_pos, s.sel_w, s.sg, nullptr, s.n_slots, used, H, x_resid, next_norm_w,
                                                     cur, c.eps, nullptr, next_xf, next_xf_kind, 1, next_xf_stride);
     DFL_HIP_CHECK(ctx, hipGetLastError());
     return DFLASH_OK;
