@@ -26,8 +26,12 @@ FLAGS = [
 # the compiler does not know their destination registers are still being filled).  If register pressure makes the
 # compiler spill, it can save such a register to scratch BEFORE its data has arrived and restore the stale value
 # later: silently wrong activations or weights.  The build therefore refuses any of them that uses scratch at all.
-NO_SCRATCH_KERNELS = ("gemm_q4k_stream_kernel", "gemm_q4k_slab_kernel", "gemm_q4k_tiled_kernel", "gemm_q4k_experts_kernel",
-                      "gemm_q6k_stream_kernel")
+NO_SCRATCH_BY_FILE = {
+    "gemm_fewrow.hip": ("gemm_q4k_stream_kernel", "gemm_q4k_slab_kernel", "gemm_q4k_tiled_kernel", "gemm_q4k_experts_kernel",
+                        "gemm_q6k_stream_kernel"),
+    "attn_verify.hip": ("attn_split_kernel",),
+}
+NO_SCRATCH_KERNELS = tuple(k for kernels in NO_SCRATCH_BY_FILE.values() for k in kernels)
 # Inspected exceptions, by mangled-name fragment -> spilled VGPRs: none at present.  An entry belongs here only after
 # the generated code has been read and every spill store found to precede the kernel's first asm load; any other
 # count than the recorded one fails the build, so that the code is read again when it changes.
@@ -109,7 +113,7 @@ def build(verbose: bool = False) -> str:
             sys.stderr.write(f"hipcc failed for {src}:\n{out}\n")
             continue
         # (the guarded kernels all live in gemm_fewrow.hip: only there is their absence from the remarks a failure)
-        bad = check_no_scratch(raw, NO_SCRATCH_KERNELS if os.path.basename(src) == "gemm_fewrow.hip" else ())
+        bad = check_no_scratch(raw, NO_SCRATCH_BY_FILE.get(os.path.basename(src), ()))
         if bad:
             failed = True
             sys.stderr.write(f"{src}: kernels with loads in flight must not use scratch:\n  " + "\n  ".join(bad) + "\n")

@@ -46,10 +46,10 @@ __device__ __forceinline__ float xor_lane(float v, int mask) {
 typedef const __attribute__((address_space(1))) void *gptr_t;
 typedef __attribute__((address_space(3))) void *lptr_t;
 
-constexpr int kAttnBufs = 3;  // LDS ring: stages in flight + the one being consumed (a fourth buffer measured the same)
+constexpr int kAttnBufs = 4;  // LDS ring: two stages in flight, the one whose scores are computed, the one whose values are read
 
-// s_waitcnt vmcnt(n) with the other counters left alone (gfx9 encoding)
-constexpr int attn_vmcnt(int n) { return ((n & 0xF) | ((n & 0x30) << 10)) | 0x0F70; }
+// s_waitcnt vmcnt(n) lgkmcnt(0) (gfx9 encoding)
+constexpr int attn_vmcnt(int n) { return ((n & 0xF) | ((n & 0x30) << 10)) | 0x0070; }
 
 // bank swizzle of the K tile: 16-byte chunk j of key row r sits at chunk j ^ swz(r), so that the
 // eight key rows one MFMA operand read touches at a time land in eight different bank groups
@@ -58,10 +58,8 @@ __device__ __forceinline__ int attn_swz(int r) { return (r & 3) | ((r >> 1) & 4)
 // One workgroup = one KV head x one contiguous chunk of keys; wave w = query head w of the GQA
 // group.  Stage = 32 keys: the K tile [32 keys][HD] and the V^T tile [HD dims][32 keys] are copied
 // global -> LDS with direct-to-LDS loads into a ring of kAttnBufs buffers, so the whole group
-// shares one copy and the loads of the next stages are in flight while this one is consumed.
-// MAXW = most waves a workgroup may have; it sets the register budget.  HPW = query heads per wave:
-// with two, every K and V^T fragment read from LDS feeds two MFMAs (half the LDS traffic per head,
-// and two independent dependency chains per wave).
+// shares one copy and the loads of the next stages are in flight while one is consumed.
+// MAXW = most waves a workgroup may have; it sets the register budget.
 // Keys per KV split for n_pos visible positions: an even share of `want` splits, rounded up to
 // whole 32-key stages, at least min_chunk.  Host and kernels use the same rule, so a launch whose
 // context length is only known on the device (a captured graph) can size its grid for the largest
@@ -78,19 +76,38 @@ __device__ __forceinline__ int attn_splits(int64_t n_pos, int64_t want, int64_t 
                                                 : (n_pos + chunk - 1) / chunk);
 }
 
-// eight consecutive query values (16-byte aligned) as floats
-__device__ __forceinline__ void attn_load8(const float *p, float v[8]) {
-    const float4_t a = *reinterpret_cast<const float4_t *>(p), b = *reinterpret_cast<const float4_t *>(p + 4);
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        v[i] = a[i];
-        v[4 + i] = b[i];
+// Eight consecutive query values (16-byte aligned): asked for ahead of everything else and read behind the first stages'
+// requests.  Asm loads with a wait of the kernel's own: the compiler, which cannot know how many stage loads follow
+// them, would wait for those as well.  (The build refuses this kernel if it uses scratch: see build.py.)
+template <typename TQ>
+struct AttnQ8;
+template <>
+struct AttnQ8<float> {
+    float4_t a, b;
+    template <int OFF>
+    __device__ __forceinline__ void load(const float *p) {
+        asm volatile("global_load_dwordx4 %0, %1, off offset:%2" : "=v"(a) : "v"(p), "n"(OFF * 4) : "memory");
+        asm volatile("global_load_dwordx4 %0, %1, off offset:%2" : "=v"(b) : "v"(p), "n"(OFF * 4 + 16) : "memory");
     }
-}
-__device__ __forceinline__ void attn_load8(const _Float16 *p, float v[8]) {
-    const half8_t a = *reinterpret_cast<const half8_t *>(p);
-#pragma unroll
-    for (int i = 0; i < 8; i++) v[i] = static_cast<float>(a[i]);
+    __device__ __forceinline__ void arrived() { asm volatile("" : "+v"(a), "+v"(b)); }
+    __device__ __forceinline__ float get(int i) const { return i < 4 ? a[i] : b[i - 4]; }
+};
+template <>
+struct AttnQ8<_Float16> {
+    half8_t a;
+    template <int OFF>
+    __device__ __forceinline__ void load(const _Float16 *p) {
+        asm volatile("global_load_dwordx4 %0, %1, off offset:%2" : "=v"(a) : "v"(p), "n"(OFF * 2) : "memory");
+    }
+    __device__ __forceinline__ void arrived() { asm volatile("" : "+v"(a)); }
+    __device__ __forceinline__ float get(int i) const { return static_cast<float>(a[i]); }
+};
+template <int S, int KS, typename TQ>
+__device__ __forceinline__ void attn_load_q(AttnQ8<TQ> *v, const TQ *p) {
+    if constexpr (S < KS) {
+        v[S].template load<32 * S>(p);
+        attn_load_q<S + 1, KS>(v, p);
+    }
 }
 
 #ifdef DFLASH_TRACE
@@ -107,7 +124,27 @@ __device__ unsigned long long *g_attn_trace = nullptr;  // [n_wg][16]
     } while (0)
 #endif
 
-template <int HD, typename TQ, int MAXW, int HPW>
+// s_waitcnt vmcnt(n), lgkmcnt(0) for a wave-uniform n: at most n loads into LDS still on their way, and this wave's LDS
+// reads done (the barrier that follows hands what they read to the next loads)
+__device__ __forceinline__ void attn_wait(int n) {
+    switch (n) {
+#define DFL_W(N) case N: __builtin_amdgcn_s_waitcnt(attn_vmcnt(N)); break
+        DFL_W(1); DFL_W(2); DFL_W(3); DFL_W(4); DFL_W(5); DFL_W(6); DFL_W(7); DFL_W(8); DFL_W(10); DFL_W(11); DFL_W(12);
+        DFL_W(14); DFL_W(15); DFL_W(16); DFL_W(18); DFL_W(21); DFL_W(22); DFL_W(24); DFL_W(32); DFL_W(33); DFL_W(48);
+#undef DFL_W
+        case 64: case 96: __builtin_amdgcn_s_waitcnt(attn_vmcnt(63)); break;
+        default: __builtin_amdgcn_s_waitcnt(attn_vmcnt(0)); break;
+    }
+}
+
+// MAXL: most loads a wave issues per stage (2 HD / 16 / waves, rounded up to a power of two).
+// What bounds it is a stage's chain, not its bytes: loads landed, barrier, K fragments, two chains of MFMAs, the
+// maximum over the row's lanes, the exponentials, the second product.  So the scores of stage t + 1 are computed ahead
+// of the softmax of stage t (the matrix cores work under the exponentials), V fragments are asked for ahead of
+// them, the maximum crosses the lanes without LDS, the last stage's special cases stand outside of the others' code, and
+// a load's address is made of one lane part and one uniform part: 16 rows x 100 k keys, 48 / 8 heads of 128, with the
+// merge: 110 -> 99 us (4.1 TB/s of keys and values; a copy reaches 5.07).
+template <int HD, typename TQ, int MAXW, int MAXL>
 __global__ void __launch_bounds__(64 * MAXW)
     attn_split_kernel(const TQ *__restrict__ q, const _Float16 *__restrict__ k_cache,
                       const _Float16 *__restrict__ vt_cache, float *__restrict__ part_o, float *__restrict__ part_ml,
@@ -125,6 +162,7 @@ __global__ void __launch_bounds__(64 * MAXW)
     constexpr int CH = HD / 8;        // 16-byte chunks per key row
     constexpr int kKPieces = 32 * CH; // pieces of the K tile; the V^T tile has as many
     constexpr int kWaveLoads = 2 * kKPieces / 64;
+    static_assert(HD < 256 || MAXW == 8, "sixteen waves leave a wave 128 registers");
     extern __shared__ half8_t lds[];  // kAttnBufs x (K tile, V^T tile)
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -135,7 +173,12 @@ __global__ void __launch_bounds__(64 * MAXW)
     // blockIdx.x = split + split_stride * (part of the GQA group this workgroup serves); split_stride is a multiple
     // of 8, so the workgroups that read one chunk of keys are dispatched to the same XCD and share its L2 copy
     const int split = blockIdx.x % split_stride;
-    const int head0 = kvh * group + ((blockIdx.x / split_stride) * n_waves + wave) * HPW;  // this wave serves heads head0 .. head0 + HPW - 1
+    const int head = kvh * group + (blockIdx.x / split_stride) * n_waves + wave;  // this wave's query head
+    // Q^T fragments: lane (row n, g) holds Q[n][head][32 s + 8 g ..+8]
+    // (rows at or past n_rows repeat the last row: they are never stored)
+    AttnQ8<TQ> q_raw[KS];
+    const TQ *qrow = q + (static_cast<int64_t>(min(n, n_rows - 1)) * n_q + head) * HD + 8 * g;
+    attn_load_q<0, KS>(q_raw, qrow);
     if (ctx_len_dev) ctx_len = *ctx_len_dev;
     ctx_len += 16 * static_cast<int64_t>(blockIdx.z);
     const int64_t n_pos = ctx_len + n_rows;
@@ -148,211 +191,184 @@ __global__ void __launch_bounds__(64 * MAXW)
     const int per_wave = (kWaveLoads + n_waves - 1) / n_waves;  // loads each wave issues per stage
     ATT_TR(0);
 
-    const uint8_t *kbytes = reinterpret_cast<const uint8_t *>(k_cache + static_cast<int64_t>(kvh) * HD);
-    const uint8_t *vbytes = reinterpret_cast<const uint8_t *>(vt_cache + static_cast<int64_t>(kvh) * HD * vt_stride);
     // Stage `st` (keys c0 + 32 st ..) into ring buffer st % kAttnBufs: wave-load qd covers LDS pieces
     // 64 qd ..; this wave takes qd = j n_waves + wave, and loads past the end repeat earlier ones
     // (same bytes to the same place) so that every wave issues per_wave loads.  Key rows at or past
     // n_pos are never dereferenced: the last stage of the cache re-reads row n_pos - 1 instead (its
     // scores are masked and its V columns zeroed below).
-    auto issue_stage = [&](int st) {
-        const int64_t key0 = c0 + 32ll * st;
-        half8_t *buf = lds + (st % kAttnBufs) * (2 * kKPieces);
-        for (int j = 0; j < per_wave; j++) {
-            const int qd = (j * n_waves + wave) % kWaveLoads;  // uniform
-            const int p = qd * 64 + lane;
+    const uint8_t *ksrc = reinterpret_cast<const uint8_t *>(k_cache + static_cast<int64_t>(kvh) * HD) + c0 * kv_dim * 2;
+    const uint8_t *vsrc = reinterpret_cast<const uint8_t *>(vt_cache + static_cast<int64_t>(kvh) * HD * vt_stride) + c0 * 2;
+    // A wave-load is 64 / CH key rows or sixteen dims of V^T: the first row is the uniform part of its address, and the
+    // lane's part is the same for every load but for the swizzle, whose bits of the first row are one more xor.
+    constexpr int kRowsPerLoad = 64 / CH;
+    const int sub = lane / CH;
+    const uint32_t k_row = static_cast<uint32_t>(sub) * static_cast<uint32_t>(kv_dim) * 2, k_chunk = ((lane % CH) ^ attn_swz(sub)) * 16;
+    const uint32_t v_off = static_cast<uint32_t>(lane >> 2) * static_cast<uint32_t>(vt_stride) * 2 + 16 * (lane & 3);
+    int issued = 0;
+    auto issue_stage = [&]() {
+        half8_t *buf = lds + (issued % kAttnBufs) * (2 * kKPieces);
+        const int rows_left = static_cast<int>(min(n_pos - c0 - 32ll * issued, static_cast<int64_t>(32)));
+        int qd = wave;
+        if constexpr (MAXL > 8) asm volatile("" : "+s"(qd));  // (so many addresses are made anew per stage, not kept in registers)
+#pragma unroll
+        for (int j = 0; j < MAXL; j++) {
+            if (j >= per_wave) break;
+            if (qd >= kWaveLoads) qd -= kWaveLoads;
             const uint8_t *src;
             if (qd * 64 < kKPieces) {
-                const int r = p / CH, jc = (p % CH) ^ attn_swz(r);
-                const int64_t key = min(key0 + r, n_pos - 1);
-                src = kbytes + key * kv_dim * 2 + jc * 16;
+                const int row0 = qd * kRowsPerLoad;
+                uint32_t o = k_row + (k_chunk ^ static_cast<uint32_t>(attn_swz(row0) * 16));
+                if (rows_left < 32) o -= static_cast<uint32_t>(max(row0 + sub - (rows_left - 1), 0)) * static_cast<uint32_t>(kv_dim) * 2;
+                src = ksrc + static_cast<int64_t>(row0) * kv_dim * 2 + static_cast<int32_t>(o);
             } else {
-                const int pv = p - kKPieces;
-                src = vbytes + ((static_cast<int64_t>(pv >> 2) * vt_stride + key0 + 8 * (pv & 3)) * 2);
+                src = vsrc + static_cast<int64_t>((qd * 64 - kKPieces) >> 2) * vt_stride * 2 + v_off;
             }
             __builtin_amdgcn_global_load_lds((gptr_t)(src), (lptr_t)(buf + qd * 64), 16, 0, 0);
+            qd += n_waves;
         }
+        ksrc += 64 * kv_dim;
+        vsrc += 64;
+        issued++;
     };
 
     // prologue: kAttnBufs - 1 stages in flight
-    int issued = 0;
 #pragma unroll
-    for (int st = 0; st < kAttnBufs - 1; st++) {
-        if (issued < n_steps) {
-            issue_stage(issued);
-            issued++;
-        }
-    }
+    for (int st = 0; st < kAttnBufs - 1; st++)
+        if (issued < n_steps) issue_stage();
 
     ATT_TR(1);
-    // Q^T fragments: lane (row n, g) holds Q[n][head][32 s + 8 g ..+8] * scale * log2(e)
-    // (rows at or past n_rows repeat the last row: they are never stored)
-    half8_t qf[HPW][KS];
+    half8_t qf[KS];  // Q^T, times scale * log2(e)
     {
         const float mult = scale * kLog2e;
-        const int nq = min(n, n_rows - 1);
+        attn_wait(per_wave * issued);
 #pragma unroll
-        for (int h = 0; h < HPW; h++) {
-            const TQ *qrow = q + (static_cast<int64_t>(nq) * n_q + head0 + h) * HD + 8 * g;
+        for (int s = 0; s < KS; s++) {
+            q_raw[s].arrived();
 #pragma unroll
-            for (int s = 0; s < KS; s++) {
-                float v[8];
-                attn_load8(qrow + 32 * s, v);
-#pragma unroll
-                for (int i = 0; i < 8; i++) qf[h][s][i] = static_cast<_Float16>(v[i] * mult);
-            }
+            for (int i = 0; i < 8; i++) qf[s][i] = static_cast<_Float16>(q_raw[s].get(i) * mult);
         }
     }
 
     ATT_TR(2);
-    float4_t acc[HPW][DT];
+    float4_t acc[DT];
 #pragma unroll
-    for (int h = 0; h < HPW; h++)
-#pragma unroll
-        for (int t = 0; t < DT; t++) acc[h][t] = float4_t{0, 0, 0, 0};
-    float m_run[HPW], l_run[HPW];  // running maximum of row n (base-2 logits, shared by its four lanes); this lane's share of the row sum
-#pragma unroll
-    for (int h = 0; h < HPW; h++) {
-        m_run[h] = -INFINITY;
-        l_run[h] = 0.0f;
-    }
+    for (int t = 0; t < DT; t++) acc[t] = float4_t{0, 0, 0, 0};
+    float m_run = -INFINITY, l_run = 0.0f;  // running maximum of row n (base-2 logits, shared by its four lanes); this lane's share of the row sum
     // visible keys of row n, relative to c0: [lo, hi].  Block-causal: everything up to the row's own
     // position; full_block (drafter, non-causal): the whole block; a window keeps |distance| < window.
-    const int64_t row_pos = ctx_len + n;
-    int64_t hi64 = full_block ? n_pos - 1 : row_pos;
-    int64_t lo64 = 0;
-    if (window > 0) {
-        lo64 = row_pos - window + 1;
-        hi64 = min(hi64, row_pos + window - 1);
-    }
-    hi64 = min(hi64, c1 - 1);
-    const int row_hi = static_cast<int>(max(min(hi64 - c0, static_cast<int64_t>(0x3fffffff)), static_cast<int64_t>(-1)));
-    const int row_lo = static_cast<int>(max(min(lo64 - c0, static_cast<int64_t>(0x3fffffff)), static_cast<int64_t>(0)));
-    // steps whose 32 keys are visible to every row need no masking: [all_lo, all_hi] in keys
-    int all_hi = row_hi, all_lo = row_lo;
-#pragma unroll
-    for (int off = 1; off < 16; off <<= 1) {
-        all_hi = min(all_hi, __shfl_xor(all_hi, off, 64));
-        all_lo = max(all_lo, __shfl_xor(all_lo, off, 64));
-    }
-    all_hi = __builtin_amdgcn_readfirstlane(all_hi);
-    all_lo = __builtin_amdgcn_readfirstlane(all_lo);
+    auto row_range = [&](int row, int &lo, int &hi) {
+        const int64_t row_pos = ctx_len + row;
+        int64_t hi64 = full_block ? n_pos - 1 : row_pos;
+        int64_t lo64 = 0;
+        if (window > 0) {
+            lo64 = row_pos - window + 1;
+            hi64 = min(hi64, row_pos + window - 1);
+        }
+        hi64 = min(hi64, c1 - 1);
+        hi = static_cast<int>(max(min(hi64 - c0, static_cast<int64_t>(0x3fffffff)), static_cast<int64_t>(-1)));
+        lo = static_cast<int>(max(min(lo64 - c0, static_cast<int64_t>(0x3fffffff)), static_cast<int64_t>(0)));
+    };
+    int row_lo, row_hi, all_lo, all_hi, unused;
+    row_range(n, row_lo, row_hi);
+    // steps whose 32 keys are visible to every row need no masking: [all_lo, all_hi] in keys (both bounds grow with the row)
+    row_range(0, unused, all_hi);
+    row_range(15, all_lo, unused);
 
     const int rk0 = 8 * (n >> 2) + (n & 3);  // key row of S^T tile 0 this lane's A operand reads
-    for (int st = 0; st < n_steps; st++) {
-        if (issued - st - 1 >= kAttnBufs - 2) {
-            // the loads of the kAttnBufs - 2 younger stages may still be in flight
-            switch (per_wave * (kAttnBufs - 2)) {
-                case 1: __builtin_amdgcn_s_waitcnt(attn_vmcnt(1)); break;
-                case 2: __builtin_amdgcn_s_waitcnt(attn_vmcnt(2)); break;
-                case 3: __builtin_amdgcn_s_waitcnt(attn_vmcnt(3)); break;
-                case 4: __builtin_amdgcn_s_waitcnt(attn_vmcnt(4)); break;
-                case 5: __builtin_amdgcn_s_waitcnt(attn_vmcnt(5)); break;
-                case 6: __builtin_amdgcn_s_waitcnt(attn_vmcnt(6)); break;
-                case 8: __builtin_amdgcn_s_waitcnt(attn_vmcnt(8)); break;
-                case 10: __builtin_amdgcn_s_waitcnt(attn_vmcnt(10)); break;
-                case 12: __builtin_amdgcn_s_waitcnt(attn_vmcnt(12)); break;
-                case 16: __builtin_amdgcn_s_waitcnt(attn_vmcnt(16)); break;
-                case 32: __builtin_amdgcn_s_waitcnt(attn_vmcnt(32)); break;
-                default: __builtin_amdgcn_s_waitcnt(attn_vmcnt(0)); break;
-            }
-        } else {
-            __builtin_amdgcn_s_waitcnt(attn_vmcnt(0));
-        }
-        __builtin_amdgcn_s_barrier();  // stage st is in LDS for everyone; buffer (st - 1) % kAttnBufs is free
-        if (issued < n_steps) {
-            issue_stage(issued);
-            issued++;
-        }
+    auto scores = [&](int st, float4_t (&sc)[2]) {
         const half8_t *kt = lds + (st % kAttnBufs) * (2 * kKPieces);
-        const half8_t *vt = kt + kKPieces;
-        const int key0 = 32 * st;  // relative to c0
-
-        float4_t sc[HPW][2];
 #pragma unroll
         for (int T = 0; T < 2; T++) {
-            const int r = rk0 + 4 * T;
-            const int sw = attn_swz(r);
+            const int r = rk0 + 4 * T, sw = attn_swz(r);
+            sc[T] = float4_t{0, 0, 0, 0};
 #pragma unroll
-            for (int h = 0; h < HPW; h++) sc[h][T] = float4_t{0, 0, 0, 0};
-#pragma unroll
-            for (int s = 0; s < KS; s++) {
-                const half8_t kf = kt[r * CH + ((4 * s + g) ^ sw)];
-#pragma unroll
-                for (int h = 0; h < HPW; h++) sc[h][T] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, qf[h][s], sc[h][T], 0, 0, 0);
-            }
+            for (int s = 0; s < KS; s++) sc[T] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kt[r * CH + ((4 * s + g) ^ sw)], qf[s], sc[T], 0, 0, 0);
         }
+    };
+    // stage `st` is in LDS for everyone; every wave is done with stage st - 2
+    auto landed = [&](int st) {
+        attn_wait(per_wave * (issued - 1 - st));
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    float4_t sc[2], sc_next[2];
+    landed(0);
+    scores(0, sc);
+    for (int st = 0; st < n_steps; st++) {
+        const half8_t *vt = lds + (st % kAttnBufs) * (2 * kKPieces) + kKPieces;
+        const int key0 = 32 * st;  // relative to c0
+        if (st + 1 < n_steps) {
+            landed(st + 1);
+            if (issued < n_steps) issue_stage();  // into the buffer of stage st - 1
+            scores(st + 1, sc_next);
+        }
+        half8_t vf[DT];
+#pragma unroll
+        for (int t = 0; t < DT; t++) vf[t] = vt[(16 * t + n) * 4 + g];
         const bool masked = !(key0 >= all_lo && key0 + 31 <= all_hi);  // uniform: some key of this step is hidden from some row
-        half8_t pf[HPW];
+        float p[8];
 #pragma unroll
-        for (int h = 0; h < HPW; h++) {
-            float p[8];
-#pragma unroll
-            for (int i = 0; i < 8; i++) p[i] = (i < 4) ? sc[h][0][i] : sc[h][1][i - 4];
-            if (masked) {
-#pragma unroll
-                for (int i = 0; i < 8; i++) {
-                    const int key = key0 + 8 * g + i;
-                    p[i] = (key >= row_lo && key <= row_hi) ? p[i] : -INFINITY;
-                }
-            }
-            float mx = fmaxf(fmaxf(fmaxf(p[0], p[1]), fmaxf(p[2], p[3])), fmaxf(fmaxf(p[4], p[5]), fmaxf(p[6], p[7])));
-            mx = fmaxf(mx, xor_lane(mx, 16));
-            mx = fmaxf(mx, xor_lane(mx, 32));
-            const float m_new = fmaxf(m_run[h], mx);
-            // all keys of this step masked for this row and nothing seen before: keep the state
-            const float m_safe = (m_new == -INFINITY) ? 0.0f : m_new;
-            const float alpha = __builtin_amdgcn_exp2f(m_run[h] - m_safe);  // 0 when m_run = -inf
-            float psum = 0.0f;
+        for (int i = 0; i < 8; i++) p[i] = (i < 4) ? sc[0][i] : sc[1][i - 4];
+        if (masked) {
 #pragma unroll
             for (int i = 0; i < 8; i++) {
-                p[i] = __builtin_amdgcn_exp2f(p[i] - m_safe);
-                psum += p[i];
+                const int key = key0 + 8 * g + i;
+                p[i] = (key >= row_lo && key <= row_hi) ? p[i] : -INFINITY;
             }
-            l_run[h] = l_run[h] * alpha + psum;
-            if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {
-#pragma unroll
-                for (int t = 0; t < DT; t++) acc[h][t] *= alpha;
-            }
-            m_run[h] = m_new;
-#pragma unroll
-            for (int i = 0; i < 8; i++) pf[h][i] = static_cast<_Float16>(p[i]);
         }
+        float mx = fmaxf(fmaxf(fmaxf(p[0], p[1]), fmaxf(p[2], p[3])), fmaxf(fmaxf(p[4], p[5]), fmaxf(p[6], p[7])));
+        mx = dfl_max_far(mx);
+        const float m_new = fmaxf(m_run, mx);
+        // all keys of this step masked for this row and nothing seen before: keep the state
+        const float m_safe = (m_new == -INFINITY) ? 0.0f : m_new;
+        const float alpha = __builtin_amdgcn_exp2f(m_run - m_safe);  // 0 when m_run = -inf
+        float psum = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            p[i] = __builtin_amdgcn_exp2f(p[i] - m_safe);
+            psum += p[i];
+        }
+        l_run = __builtin_fmaf(l_run, alpha, psum);
+        if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {
+#pragma unroll
+            for (int t = 0; t < DT; t++) acc[t] *= alpha;
+        }
+        m_run = m_new;
+        half8_t pf;
+#pragma unroll
+        for (int i = 0; i < 8; i++) pf[i] = static_cast<_Float16>(p[i]);
         // O^T tile t (dims 16 t ..): A = V^T[dim 16 t + n][keys key0 + 8 g ..+8].  Columns at or past
         // n_pos hold whatever the cache held before (possibly NaN patterns; 0 * NaN would poison
         // the accumulator): zero them in the last stage of the cache
-        const int64_t vkey = c0 + key0 + 8 * g;
-        const bool tail = c0 + key0 + 32 > n_pos;
+        if (c0 + key0 + 32 > n_pos) {
+            const int vkeys = static_cast<int>(n_pos - (c0 + key0)) - 8 * g;  // this lane's columns ahead of n_pos
 #pragma unroll
-        for (int t = 0; t < DT; t++) {
-            half8_t vf = vt[(16 * t + n) * 4 + g];
-            if (tail) {
+            for (int t = 0; t < DT; t++)
 #pragma unroll
                 for (int i = 0; i < 8; i++)
-                    if (vkey + i >= n_pos) vf[i] = static_cast<_Float16>(0.0f);
-            }
-#pragma unroll
-            for (int h = 0; h < HPW; h++) acc[h][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, pf[h], acc[h][t], 0, 0, 0);
+                    if (i >= vkeys) vf[t][i] = static_cast<_Float16>(0.0f);
         }
+#pragma unroll
+        for (int t = 0; t < DT; t++) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf[t], pf, acc[t], 0, 0, 0);
+        sc[0] = sc_next[0];
+        sc[1] = sc_next[1];
         if (st < 8) ATT_TR(3 + st);
     }
     ATT_TR(12);
 
     // row sums over the four lanes of a row; partials: O^T tile t, lane (row n, g) holds dims 16 t + 4 g + i
+    float l = l_run;
+    l += xor_lane(l, 16);
+    l += xor_lane(l, 32);
+    if (n < n_rows) {
+        const int64_t slot = (static_cast<int64_t>(split) * n_q + head) * 16 + n;
+        float *po = part_o + slot * HD;
 #pragma unroll
-    for (int h = 0; h < HPW; h++) {
-        float l = l_run[h];
-        l += xor_lane(l, 16);
-        l += xor_lane(l, 32);
-        if (n < n_rows) {
-            const int64_t slot = (static_cast<int64_t>(split) * n_q + head0 + h) * 16 + n;
-            float *po = part_o + slot * HD;
-#pragma unroll
-            for (int t = 0; t < DT; t++) *reinterpret_cast<float4_t *>(po + 16 * t + 4 * g) = acc[h][t];
-            if (g == 0) {
-                part_ml[slot * 2] = m_run[h];
-                part_ml[slot * 2 + 1] = l;
-            }
+        for (int t = 0; t < DT; t++) *reinterpret_cast<float4_t *>(po + 16 * t + 4 * g) = acc[t];
+        if (g == 0) {
+            part_ml[slot * 2] = m_run;
+            part_ml[slot * 2 + 1] = l;
         }
     }
     ATT_TR(13);
@@ -478,6 +494,76 @@ __global__ void __launch_bounds__(256)
     }
 }
 
+// The same for at most 48 splits, with the same sums in the same order (a split lane's every eighth split, then the eight
+// in turn).  What bounds it is its chain: a trip to memory for the maxima and the partial outputs, which are in flight
+// together, the maximum over the splits, the sums.  Here lane s of every wave keeps split s's maximum and sum, so that the
+// weights need no LDS and no barrier (a wave shuffles them to where they are used), and the only barrier stands between
+// the split lanes' sums and their total: 5.1 -> 3.6 us inside a verify's graph (24 splits, 32 heads of 128, 16 rows).
+// A wave's 64 lanes cover 64 / (HD / 4) split lanes, four dims per lane.
+template <int HD>
+__global__ void __launch_bounds__(HD == 64 ? 128 : 256)
+    attn_combine_few_kernel(const float *__restrict__ part_o, const float *__restrict__ part_ml, float *__restrict__ out, int n_rows_total,
+                            int n_q, int64_t ctx_len, const int32_t *__restrict__ ctx_len_dev, int want, int min_chunk,
+                            void *__restrict__ out_xf, int out_xf_kind, int64_t part_slots, size_t xf_stride, int max_splits) {
+    constexpr int kLanes = HD / 4, kPerWave = 64 / kLanes, kWaves = HD == 64 ? 2 : 4, kSteps = 8 / (kPerWave * kWaves);
+    const int n_rows = min(16, n_rows_total - 16 * static_cast<int>(blockIdx.z));
+    if (static_cast<int>(blockIdx.y) >= n_rows) return;
+    const int head = blockIdx.x, row = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    __shared__ __attribute__((aligned(16))) float red[8][HD + 4];
+    __shared__ float red_l[8];
+    const int64_t slot_stride = static_cast<int64_t>(n_q) * 16;
+    const float2 *ml = reinterpret_cast<const float2 *>(part_ml) + static_cast<int64_t>(blockIdx.z) * part_slots + head * 16 + row;
+    const float *po = part_o + (static_cast<int64_t>(blockIdx.z) * part_slots + head * 16 + row) * HD + 4 * (lane % kLanes);
+    const float2 own = ml[min(lane, max_splits - 1) * slot_stride];
+    float4_t o[kSteps][6];
+#pragma unroll
+    for (int j = 0; j < kSteps; j++)
+#pragma unroll
+        for (int i = 0; i < 6; i++) {
+            if (8 * i >= max_splits) continue;  // (uniform; a lane past the last split re-reads it)
+            const int s = min(wave * kPerWave + lane / kLanes + j * kPerWave * kWaves + 8 * i, max_splits - 1);
+            o[j][i] = *reinterpret_cast<const float4_t *>(po + s * slot_stride * HD);
+        }
+    if (ctx_len_dev) ctx_len = *ctx_len_dev;
+    const int n_splits = attn_splits(ctx_len + 16 * static_cast<int64_t>(blockIdx.z) + n_rows, want, min_chunk);
+    float m_star = lane < n_splits ? own.x : -INFINITY;
+    const float m_own = m_star;
+    m_star = dfl_wave_max(m_star);
+    const float wgt = m_own == -INFINITY ? 0.0f : exp2f(m_own - m_star);
+#pragma unroll
+    for (int j = 0; j < kSteps; j++) {
+        const int sl = wave * kPerWave + lane / kLanes + j * kPerWave * kWaves;
+        float4_t acc = {0, 0, 0, 0};
+        float l = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 6; i++) {
+            if (8 * i >= max_splits) continue;
+            const int s = sl + 8 * i;
+            const float w = __shfl(wgt, s, 64), ls = __shfl(own.y, s, 64);
+            if (s < n_splits) {
+                acc += w * o[j][i];
+                l = __builtin_fmaf(w, ls, l);
+            }
+        }
+        *reinterpret_cast<float4_t *>(&red[sl][4 * (lane % kLanes)]) = acc;
+        if (lane % kLanes == 0) red_l[sl] = l;
+    }
+    __syncthreads();
+    float lsum = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 8; k++) lsum += red_l[k];
+    if (tid < kLanes) {
+        const int d = 4 * tid;
+        float4_t v = {0, 0, 0, 0};
+#pragma unroll
+        for (int k = 0; k < 8; k++) v += *reinterpret_cast<const float4_t *>(&red[k][d]);
+        v /= lsum;
+        *reinterpret_cast<float4_t *>(out + ((static_cast<int64_t>(blockIdx.z) * 16 + row) * n_q + head) * HD + d) = v;
+        if (out_xf)
+            dfl_xf_store_pair(static_cast<uint8_t *>(out_xf) + blockIdx.z * xf_stride, out_xf_kind, row, head * HD + (d & ~7), v[0], v[1], v[2], v[3]);
+    }
+}
+
 // V [pos][n_kv][hd] -> V^T [n_kv][hd][stride]; one workgroup per (32 positions, kv head)
 __global__ void __launch_bounds__(256) transpose_v_kernel(const _Float16 *__restrict__ v, _Float16 *__restrict__ vt,
                                                           int64_t n_pos, int n_kv, int hd, int64_t stride) {
@@ -503,21 +589,33 @@ int32_t launch_split(dflash_ctx *ctx, dim3 grid, int threads, hipStream_t st, co
                   int64_t vt_stride, int want, int min_chunk, float scale, int full_block, int64_t window, int split_stride,
                   int64_t part_slots) {
     const size_t lds = static_cast<size_t>(kAttnBufs) * 2 * (32 * HD / 8) * sizeof(half8_t);
-#define DFL_ATTN_LAUNCH(MAXW, HPW)                                                                                  \
+    constexpr int kWaveLoads = 2 * 32 * (HD / 8) / 64;
+    const int n_waves = threads / 64, per_wave = (kWaveLoads + n_waves - 1) / n_waves;
+#define DFL_ATTN_LAUNCH(MAXW, MAXL)                                                                                 \
     do {                                                                                                            \
-        if (const int32_t rc_ = dfl_raise_lds_limit(ctx, reinterpret_cast<const void *>(attn_split_kernel<HD, TQ, MAXW, HPW>), lds)) \
+        if (const int32_t rc_ = dfl_raise_lds_limit(ctx, reinterpret_cast<const void *>(attn_split_kernel<HD, TQ, MAXW, MAXL>), lds)) \
             return rc_;                                                                                             \
-        attn_split_kernel<HD, TQ, MAXW, HPW><<<grid, threads / HPW, lds, st>>>(static_cast<const TQ *>(q), k, vt, po, pml, \
-                                                                              ctx_len, ctx_len_dev, n_rows, n_q, n_kv, \
-                                                                              vt_stride, want, min_chunk, scale,    \
-                                                                              full_block, window, split_stride, part_slots); \
+        attn_split_kernel<HD, TQ, MAXW, MAXL><<<grid, threads, lds, st>>>(static_cast<const TQ *>(q), k, vt, po, pml, \
+                                                                         ctx_len, ctx_len_dev, n_rows, n_q, n_kv, \
+                                                                         vt_stride, want, min_chunk, scale,    \
+                                                                         full_block, window, split_stride, part_slots); \
     } while (0)
-    // one head per wave: two (HPW = 2) halve the LDS reads per head but measured slower on MI355X
+    // one head per wave: two halve the LDS reads per head but measured slower on MI355X
     // (fewer waves to hide the per-stage dependency chain)
-    if (threads <= 512)
-        DFL_ATTN_LAUNCH(8, 1);
+    if constexpr (HD < 256) {
+        if (threads > 512) {
+            DFL_ATTN_LAUNCH(16, 4);
+            return DFLASH_OK;
+        }
+    }
+    if (per_wave <= 4)
+        DFL_ATTN_LAUNCH(8, 4);
+    else if (per_wave <= 8)
+        DFL_ATTN_LAUNCH(8, 8);
+    else if (per_wave <= 16)
+        DFL_ATTN_LAUNCH(8, 16);
     else
-        DFL_ATTN_LAUNCH(16, 1);
+        DFL_ATTN_LAUNCH(8, 32);
 #undef DFL_ATTN_LAUNCH
     return DFLASH_OK;
 }
@@ -626,7 +724,7 @@ static int32_t attn_rows(dflash_ctx *ctx, const void *q, int32_t q_type, const v
     // tiles (16 rows x its heads x head_dim floats) are then as many bytes as the keys and values it read.  Half a
     // workgroup per CU there (16 q / 2 kv heads of 256, 40-layer verify: 5.25 -> 4.79 ms at 16 k of context with chunks
     // of 256 keys instead of 128, 6.21 -> 5.80 ms at 32 k with 512; a quarter measured slower again).
-    const size_t ring_bytes = static_cast<size_t>(kAttnBufs) * 2 * 32 * head_dim * sizeof(_Float16);
+    const size_t ring_bytes = static_cast<size_t>(3) * 2 * 32 * head_dim * sizeof(_Float16);  // (three buffers' worth: what the figures here were taken with)
     int per_cu_x2 = bucket >= 16384 ? (2 * ring_bytes <= static_cast<size_t>(ctx->lds_bytes) ? 4 : 1) : 2;
     int64_t min_chunk = bucket >= 8192 ? 128 : 64;
     // A workgroup serves hw heads of a GQA group (one wave each).  What a workgroup moves is its chunk of K and V,
@@ -666,6 +764,13 @@ static int32_t attn_rows(dflash_ctx *ctx, const void *q, int32_t q_type, const v
     if (n_blocks > 1) {
         hw = group;
         n_parts = 1;
+    }
+    // heads of 256: eight waves at most (registers); again the split of the keys stays
+    while (head_dim == 256 && hw > 8) {
+        int d = hw - 1;
+        while (group % d) d--;
+        hw = d;
+        n_parts = group / hw;
     }
     // most splits any context up to n_pos can have
     auto splits_for = [&](int64_t np) {
@@ -732,6 +837,15 @@ static int32_t attn_rows(dflash_ctx *ctx, const void *q, int32_t q_type, const v
 #undef DFL_ATTN
     }
     if (rc) return rc;
+    // (more splits than that and the shuffles of the weights cost more than the barriers they replace)
+    if (n_splits <= 48) {
+        const auto fn = head_dim == 64 ? attn_combine_few_kernel<64> : head_dim == 128 ? attn_combine_few_kernel<128> : attn_combine_few_kernel<256>;
+        fn<<<dim3(n_q, n_rows, n_blocks), head_dim == 64 ? 128 : 256, 0, st>>>(part_o, part_ml, out, n_rows_total, n_q, ctx_len, ctx_len_dev, want,
+                                                                              static_cast<int>(min_chunk), out_xf, out_xf_kind, part_slots,
+                                                                              dfl_xf_bytes(static_cast<int64_t>(n_q) * head_dim), n_splits);
+        DFL_HIP_CHECK(ctx, hipGetLastError());
+        return DFLASH_OK;
+    }
     attn_combine_kernel<<<dim3(n_q, n_rows, n_blocks), 256, 0, st>>>(part_o, part_ml, out, n_rows_total, n_q, head_dim, ctx_len, ctx_len_dev,
                                                                     want, static_cast<int>(min_chunk), out_xf, out_xf_kind, part_slots,
                                                                     dfl_xf_bytes(static_cast<int64_t>(n_q) * head_dim), n_splits);

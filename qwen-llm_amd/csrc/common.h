@@ -169,6 +169,49 @@ __device__ static inline void dfl_xf_store(void *xf, int kind, int m, int k0, fl
                      static_cast<_Float16>(v4), static_cast<_Float16>(v6), static_cast<_Float16>(v5), static_cast<_Float16>(v7)};
     *reinterpret_cast<h8 *>(static_cast<uint8_t *>(xf) + dfl_xf_slot(kind, m, k0)) = frag;
 }
+// Reductions over a wave without LDS (a shuffle is a trip through it, and six in a row stand in the middle of most small
+// kernels): the lane 32 or 16 away by v_permlane32/16_swap, the nearer ones by DPP moves.  The tree is that of
+// `for (off = 32; off; off >>= 1) v += __shfl_xor(v, off)`, lane for lane, so a sum has that loop's bits.
+// (The swaps as asm: through the builtins the compiler used one of the two results twice.  Both want two wait states
+// behind the write of their operands.)
+template <int CTRL>
+__device__ static inline float dfl_dpp(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
+}
+__device__ static inline void dfl_swap16(float &a, float &b) { asm("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b)); }
+__device__ static inline void dfl_swap32(float &a, float &b) { asm("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(a), "+v"(b)); }
+__device__ static inline float dfl_xor4(float v) {  // the value of the lane 4 away: banks 0 and 2 of a row from above, 1 and 3 from below
+    const int up = __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x104, 0xF, 0x5, false);
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(up, __builtin_bit_cast(int, v), 0x114, 0xF, 0xA, false));
+}
+__device__ static inline float dfl_wave_sum(float v) {
+    float a = v, b = v;
+    dfl_swap32(a, b);
+    v = a + b;
+    a = v, b = v;
+    dfl_swap16(a, b);
+    v = a + b;
+    v += dfl_dpp<0x128>(v);  // row_ror:8
+    v += dfl_xor4(v);
+    v += dfl_dpp<0x4E>(v);   // quad_perm [2,3,0,1]
+    v += dfl_dpp<0xB1>(v);   // quad_perm [1,0,3,2]
+    return v;
+}
+__device__ static inline float dfl_max_far(float v) {  // maximum over the four lanes 16 apart, in each of them
+    float a = v, b = v;
+    dfl_swap32(a, b);
+    v = fmaxf(a, b);
+    a = v, b = v;
+    dfl_swap16(a, b);
+    return fmaxf(a, b);
+}
+__device__ static inline float dfl_wave_max(float v) {
+    v = dfl_max_far(v);
+    v = fmaxf(v, dfl_dpp<0x128>(v));
+    v = fmaxf(v, dfl_xor4(v));
+    v = fmaxf(v, dfl_dpp<0x4E>(v));
+    return fmaxf(v, dfl_dpp<0xB1>(v));
+}
 // Lanes (2 p, 2 p + 1) of a wave hold values i .. i + 3 and i + 4 .. i + 7 of row m (i a multiple of 8 on the even lane):
 // the even lane stores the octet.  Every lane of the wave must call it.
 __device__ static inline void dfl_xf_store_pair(void *xf, int kind, int m, int i, float a, float b, float c, float d) {

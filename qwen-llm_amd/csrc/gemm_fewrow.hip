@@ -2310,7 +2310,7 @@ __global__ void __launch_bounds__(64 * kMaxSplit)
 #pragma unroll
         for (int j = 0; j < 2; j++)
             s += (v[j][0] * v[j][0] + v[j][1] * v[j][1]) + (v[j][2] * v[j][2] + v[j][3] * v[j][3]);
-        for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+        s = dfl_wave_sum(s);
         if (lane == 0) sq_part[wave] = s;
     }
     DFL_TRR(1);
@@ -2338,7 +2338,7 @@ __global__ void __launch_bounds__(64 * kMaxSplit)
             }
         }
         if (first_tile) {  // (the same for the whole workgroup)
-            for (int off = 32; off > 0; off >>= 1) dot += __shfl_xor(dot, off, 64);
+            dot = dfl_wave_sum(dot);
             if (lane == 0) dot_part[wave] = dot;
         }
     }
@@ -2559,7 +2559,7 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
     for (int m = 0; m < 16; m++) {
         float v = acc[m];
-        for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+        v = dfl_wave_sum(v);
         if (lane == 0 && m < n_rows) y[static_cast<size_t>(m) * n_out + row] = v;
     }
 }

@@ -31,7 +31,7 @@ __global__ void get_rows_kernel(int type, const uint8_t *__restrict__ table, siz
 }
 
 __device__ float block_sum(float v, float *sh) {
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    v = dfl_wave_sum(v);
     __syncthreads();
     if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
     __syncthreads();
@@ -135,7 +135,7 @@ __global__ void __launch_bounds__(256) rms_norm_kernel(float *__restrict__ x, co
         if (!in) v[j] = f4{0, 0, 0, 0};
         s += (v[j][0] * v[j][0] + v[j][1] * v[j][1]) + (v[j][2] * v[j][2] + v[j][3] * v[j][3]);
     }
-    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+    s = dfl_wave_sum(s);
     if ((tid & 63) == 0) sh[tid >> 6] = s;
     if (kConv || add) {
 #pragma unroll
@@ -161,7 +161,7 @@ __global__ void __launch_bounds__(256) rms_norm_kernel(float *__restrict__ x, co
         }
     }
     if (gate_w) {
-        for (int off = 32; off > 0; off >>= 1) dot += __shfl_xor(dot, off, 64);
+        dot = dfl_wave_sum(dot);
         if ((tid & 63) == 0) sh_dot[tid >> 6] = dot;
         __syncthreads();
         if (tid == 0) gate_out[t] = 1.0f / (1.0f + expf(-(((sh_dot[0] + sh_dot[1]) + sh_dot[2]) + sh_dot[3])));
@@ -267,7 +267,7 @@ struct RopeHead {
         float s = r[0] * r[0];
 #pragma unroll
         for (int k = 1; k < kEl; k++) s = __builtin_fmaf(r[k], r[k], s);
-        for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+        s = dfl_wave_sum(s);
         const float scale = 1.0f / sqrtf(s / static_cast<float>(HD) + eps);
 #pragma unroll
         for (int k = 0; k < RopePairs<HD>::N; k++) {
@@ -502,7 +502,7 @@ __global__ void __launch_bounds__(64)
                                         : v_noise + static_cast<size_t>(kk - ctx_len) * kv_dim) + kvh * hd + lane * per;
         float s = 0.0f;
         for (int i = 0; i < per; i++) s += qv[i] * kr[i];
-        for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+        s = dfl_wave_sum(s);
         s *= scale;
         const float m_new = fmaxf(m, s);
         const float alpha = expf(m - m_new), p = expf(s - m_new);
@@ -557,7 +557,7 @@ __global__ void __launch_bounds__(64)
     const int half = hd / 2;
     float s = 0.0f;
     for (int i = lane; i < hd; i += 64) s += v[i] * v[i];
-    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+    s = dfl_wave_sum(s);
     const float scale = 1.0f / sqrtf(s / static_cast<float>(hd) + eps);
     const float p = static_cast<float>(pos[col]);
     for (int i = lane; i < half; i += 64) {

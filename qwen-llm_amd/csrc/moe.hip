@@ -99,7 +99,7 @@ __global__ void __launch_bounds__(1024)
         } else {
             for (int i = lane; i < hidden; i += 64) dot += xr[i] * shexp_gate[i];
         }
-        for (int off = 32; off > 0; off >>= 1) dot += __shfl_xor(dot, off, 64);
+        dot = dfl_wave_sum(dot);
         if (shexp_gate && lane == 0) sg[row] = 1.0f / (1.0f + expf(-dot));
 
         float mx = -INFINITY;
@@ -121,7 +121,7 @@ __global__ void __launch_bounds__(1024)
             pr[e] = ex;
             sum += ex;
         }
-        for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
+        sum = dfl_wave_sum(sum);
         const float inv = 1.0f / sum;
         for (int e = lane; e < n_expert; e += 64) pr[e] *= inv;
     }
@@ -225,7 +225,7 @@ __global__ void __launch_bounds__(1024)
         } else {
             for (int i = lane; i < hidden; i += 64) dot += xr[i] * shexp_gate[i];
         }
-        for (int off = 32; off > 0; off >>= 1) dot += __shfl_xor(dot, off, 64);
+        dot = dfl_wave_sum(dot);
         if (shexp_gate && lane == 0) sg[row] = 1.0f / (1.0f + expf(-dot));
 
         const dfl_route::RowPicks pk = dfl_route::route_row(lg, n_expert, n_used, lane);
@@ -437,7 +437,7 @@ __global__ void __launch_bounds__(256)
         if (4 * (tid + 256 * j) >= hidden) v[j] = f4{0, 0, 0, 0};
         s += (v[j][0] * v[j][0] + v[j][1] * v[j][1]) + (v[j][2] * v[j][2] + v[j][3] * v[j][3]);
     }
-    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+    s = dfl_wave_sum(s);
     if ((tid & 63) == 0) sh[tid >> 6] = s;
 #pragma unroll
     for (int j = 0; j < V; j++)
