@@ -161,29 +161,6 @@ __device__ __forceinline__ uint64_t wave_sort_u64(uint64_t v) {
     return v;
 }
 
-// Minimum of a key over the wave, in every lane: data-parallel-primitive moves within rows of 16 lanes (shift right
-// by 1, 2, 4, 8: lane 15 of a row then holds the row's minimum), then lane 15 of rows 0 and 2 into rows 1 and 3, then
-// lane 31 into rows 2 and 3; lane 63 has the result.  Lanes without a source read the identity.  No LDS round trips.
-__device__ __forceinline__ uint64_t wave_min_u64(uint64_t v) {
-#define DFL_MIN_STEP(ctrl, row_mask)                                                                                     \
-    do {                                                                                                                 \
-        const unsigned lo = __builtin_amdgcn_update_dpp(0xffffffffu, static_cast<unsigned>(v), ctrl, row_mask, 0xf, false);       \
-        const unsigned hi = __builtin_amdgcn_update_dpp(0xffffffffu, static_cast<unsigned>(v >> 32), ctrl, row_mask, 0xf, false); \
-        const uint64_t o = (static_cast<uint64_t>(hi) << 32) | lo;                                                       \
-        v = o < v ? o : v;                                                                                               \
-    } while (0)
-    DFL_MIN_STEP(0x111, 0xf);  // row_shr:1
-    DFL_MIN_STEP(0x112, 0xf);  // row_shr:2
-    DFL_MIN_STEP(0x114, 0xf);  // row_shr:4
-    DFL_MIN_STEP(0x118, 0xf);  // row_shr:8
-    DFL_MIN_STEP(0x142, 0xa);  // row_bcast:15 into rows 1 and 3
-    DFL_MIN_STEP(0x143, 0xc);  // row_bcast:31 into rows 2 and 3
-#undef DFL_MIN_STEP
-    const unsigned lo = __builtin_amdgcn_readlane(static_cast<unsigned>(v), 63);
-    const unsigned hi = __builtin_amdgcn_readlane(static_cast<unsigned>(v >> 32), 63);
-    return (static_cast<uint64_t>(hi) << 32) | lo;
-}
-
 // The k smallest keys, in order, of n_lists <= 64 ascending lists of k keys each (list l at base + l * stride; missing
 // keys are kNoKey, at the end), by ONE wave: lane l holds the head of list l, a step takes the minimum of the heads
 // and advances the list it came from (keys are distinct).  Returns the k-th; with `out`, out[0 .. k) gets them all.
@@ -547,7 +524,7 @@ struct DecideArgs {
     const double *tile_sums;
     int32_t n_tiles;
     float temperature, draft_temperature;
-    // wide candidate sets (effective top-k above kMaxK): row r's kept candidates are the first n_keep sorted keys
+    // wide candidate sets (effective top-k above kMaxK): row r's kept candidates are the first n_keep ordered keys
     // / weights at r * wide_stride of these arrays instead of the arrays inside RowDist; null otherwise
     const uint64_t *wide_keys;
     const double *wide_w;
@@ -562,16 +539,6 @@ struct DistView {
     __device__ int32_t token(int i) const { return keys ? static_cast<int32_t>(keys[i] & kWideTokenMask) : rd->tokens[i]; }
     __device__ double weight(int i) const { return w ? w[i] : rd->weights[i]; }
 };
-
-// first candidate whose running sum exceeds x, else the last (sampling.rs:1587-1596)
-__device__ int pick_index_view(const DistView &v, int n, double x) {
-    double cumulative = 0.0;
-    for (int i = 0; i < n; i++) {
-        cumulative += v.weight(i);
-        if (x < cumulative) return i;
-    }
-    return n - 1;
-}
 
 __device__ bool in_list(const int32_t *ids, int n, int32_t v) {
     for (int i = 0; i < n; i++)
@@ -602,19 +569,23 @@ __device__ RowOutcome decide_row(const DecideArgs &a, const RowDist *rows, int r
     const int n_drafts = a.n_tokens - 1;
     const bool greedy = a.temperature == 0.0f;
     const RowDist &rd = rows[row];
-    const DistView dv = {&rd, a.wide_keys ? a.wide_keys + row * a.wide_stride : nullptr,
-                         a.wide_w ? a.wide_w + row * a.wide_stride : nullptr};
     int draws = greedy ? 0 : row;
     const int draws0 = draws;
+    // the target token that draw `row` falls on (wide sets: the row's chain has walked its order with that draw)
+    auto target_token = [&]() {
+        if (a.wide_keys) {
+            draws++;
+            return rd.pick;
+        }
+        return rd.tokens[greedy ? 0 : pick_index(rd.weights, rd.n_keep, a.uniforms[draws++] * rd.total)];
+    };
     if (row == n_drafts) {  // bonus = sample(last reached row)
         if (rd.err) {
             o.err = rd.err;
             o.err_index = rd.err_index;
             return o;
         }
-        int idx = 0;
-        if (!greedy) idx = pick_index_view(dv, rd.n_keep, a.uniforms[draws++] * rd.total);
-        o.token = dv.token(idx);
+        o.token = target_token();
         o.draws = draws - draws0;
         return o;
     }
@@ -625,9 +596,7 @@ __device__ RowOutcome decide_row(const DecideArgs &a, const RowDist *rows, int r
             o.err_index = rd.err_index;
             return o;
         }
-        int idx = 0;
-        if (!greedy) idx = pick_index_view(dv, rd.n_keep, a.uniforms[draws++] * rd.total);
-        o.token = dv.token(idx);
+        o.token = target_token();
         o.acc = o.token == draft;
         o.draws = draws - draws0;
         return o;
@@ -676,8 +645,11 @@ __device__ RowOutcome decide_row(const DecideArgs &a, const RowDist *rows, int r
     }
     if (o.err) return o;
     double tp = -0.0;
-    for (int i = 0; i < rd.n_keep; i++)
-        if (dv.token(i) == draft) tp += dv.weight(i);
+    if (a.wide_keys)
+        tp = rd.draft_weight;
+    else
+        for (int i = 0; i < rd.n_keep; i++)
+            if (rd.tokens[i] == draft) tp += rd.weights[i];
     const double target_probability = tp / rd.total;
     const double proposal_probability = prop_tok_w / prop_total;
     const double acceptance = fmin(target_probability / proposal_probability, 1.0);
@@ -1134,7 +1106,7 @@ int32_t dflash_accept_prefix(dflash_ctx *ctx, const int32_t *verified, int32_t n
     }
     const dflash_sampling_config &sc = sampler->cfg;
     int64_t k_eff = (sc.temperature == 0.0f) ? 1 : ((sc.top_k == 0 || static_cast<int64_t>(sc.top_k) >= vocab) ? vocab : static_cast<int64_t>(sc.top_k));
-    const bool wide = k_eff > kMaxK;  // top_k = 0 or a large top_k: full order by radix sort (accept_wide.hip)
+    const bool wide = k_eff > kMaxK;  // top_k = 0 or a large top_k: accept_wide.hip
     const int n_chunks = static_cast<int>((vocab + kSelChunk - 1) / kSelChunk);
     if (!wide && n_chunks * k_eff > 2 * kSelThreads)
         return dfl_fail(ctx, DFLASH_ERR_UNSUPPORTED, "accept_prefix: vocabulary %lld x top_k %lld too large", static_cast<long long>(vocab), static_cast<long long>(k_eff));
@@ -1182,7 +1154,12 @@ int32_t dflash_accept_prefix(dflash_ctx *ctx, const int32_t *verified, int32_t n
         const uint64_t *wide_keys = nullptr;
         const double *wide_w = nullptr;
         if (wide) {
-            if (const int32_t rc_ = dfl_accept_wide_rows(ctx, target_logits, n_tokens, vocab, vocab, cfg, rows, &off, &wide_keys, &wide_w, st))
+            WideWalk walk = {};
+            walk.n_tokens = n_tokens;
+            for (int i = 0; i < n_tokens; i++) walk.verified[i] = verified[i];
+            for (int i = 0; i <= n_tokens; i++) walk.uniforms[i] = a.uniforms[i];
+            if (const int32_t rc_ = dfl_accept_wide_rows(ctx, target_logits, n_tokens, vocab, vocab, cfg, walk, rows, &off, &wide_keys, &wide_w,
+                                                         &a.wide_stride, st))
                 return rc_;
             if (dense) select_chunk_kernel<<<dim3(n_chunks, n_drafts), kSelThreads, 0, st>>>(draft_logits, vocab, vocab, 1, dchunks, false);
         } else if (dense) {
@@ -1202,7 +1179,6 @@ int32_t dflash_accept_prefix(dflash_ctx *ctx, const int32_t *verified, int32_t n
         }
         a.wide_keys = wide_keys;
         a.wide_w = wide_w;
-        a.wide_stride = vocab;
         a.n_tokens = n_tokens;
         a.n_stop = n_stop;
         a.mode = mode;

@@ -5,7 +5,12 @@
 // the (descending logit bits, token) keys; top_k < len: the top_k smallest keys, sorted), chain
 // sampling.rs:1541-1615.
 //
-// All rows of the block are ordered by ONE device-wide radix sort: a key is
+// Two ways.  A set of at most kPickMax candidates (the chat preset's 200) is selected, not sorted: a workgroup per
+// 8192 tokens finds its own k smallest keys, a workgroup per row the k smallest of those, ranks them by counting and
+// runs the chain with a candidate per thread.  Two launches that read the logits once, each bound
+// by its chain of barriers and LDS round trips (the logits take 2 us): 16 rows x 151936 tokens, k = 200: 11.2 + 12.9 us
+// where the sort, its 17 clears and its chain take 316; the whole call 334 -> 44.5 us.
+// Anything larger (the whole vocabulary) is ordered by ONE device-wide radix sort: a key is
 //   row << 60 | descending_logit_bits << 28 | token          (token < 2^28, row < 16)
 // and ascending key order is (row, descending logit in f32 total order, ascending token id): row r's
 // candidates end up, best first, at [r * vocab, (r + 1) * vocab).  All 64 bits are sorted (tokens are
@@ -20,6 +25,7 @@
 #include "common.h"
 #include "sampler_chain.h"
 
+#include <algorithm>
 #include <cstring>
 
 #include <rocprim/device/device_radix_sort.hpp>
@@ -50,6 +56,295 @@ __global__ void __launch_bounds__(256)
                             (static_cast<uint64_t>(desc_bits(__float_as_uint(v))) << kWideTokenBits) | static_cast<uint64_t>(i);
 }
 
+// ------------------------------------------------------------------------------------------
+// selection of up to kPickMax candidates
+// ------------------------------------------------------------------------------------------
+constexpr int kPickThreads = 512;
+constexpr int kPickChunk = 8192;  // tokens per workgroup: 16 rows of 151936 are 304 workgroups, one round of two per CU
+constexpr int kPickMax = 1024;    // threads of the row kernel: a candidate each
+constexpr int kPickSlots = 16 * kPickMax;  // chunk winners of a row that its workgroup holds in registers
+constexpr uint64_t kNoKeyW = ~0ull;  // (a NaN's logit bits: no key has them)
+
+template <int THREADS>
+struct KthShared {
+    int hist[3][256];
+    uint64_t lo[THREADS / 64], hi[THREADS / 64];
+    int n[THREADS / 64];
+};
+
+// A bound B <= limit such that exactly k of the workgroup's keys are <= B; limit if no more than k are <= limit.
+// Digit by digit from the first bit in which the keys differ (they share row, sign and most of the exponent: a digit
+// above it would put every key on one counter), and no further than until a digit's counts end at k.  Keys are
+// distinct, so the last digit ends there at the latest.  One barrier per digit: every wave adds up the counters by
+// itself, and of three sets of counters one is counted in, one may still be read, one is cleared for the next digit.
+template <int PER, int THREADS>
+__device__ uint64_t block_kth(const uint64_t (&key)[PER], uint64_t limit, int k, KthShared<THREADS> &sh) {
+    constexpr int kWaves = THREADS / 64;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    uint64_t lo = kNoKeyW, hi = 0;
+    int n = 0;
+#pragma unroll
+    for (int j = 0; j < PER; j++) {
+        const bool in = key[j] <= limit;
+        lo = in && key[j] < lo ? key[j] : lo;
+        hi = in && key[j] > hi ? key[j] : hi;
+        n += __popcll(__builtin_amdgcn_ballot_w64(in));
+    }
+    lo = wave_min_u64(lo);
+    hi = ~wave_min_u64(~hi);
+    if (lane == 0) {
+        sh.lo[wave] = lo;
+        sh.hi[wave] = hi;
+        sh.n[wave] = n;
+    }
+    if (tid < 256) sh.hist[0][tid] = 0;
+    __syncthreads();
+    lo = wave_min_u64(lane < kWaves ? sh.lo[lane] : kNoKeyW);
+    hi = ~wave_min_u64(lane < kWaves ? ~sh.hi[lane] : kNoKeyW);
+    n = __builtin_amdgcn_readlane(wave_scan_i32(lane < kWaves ? sh.n[lane] : 0), 63);
+    if (n <= k) return limit;
+    int shift = 64 - __clzll(static_cast<long long>(lo ^ hi));  // (n > k >= 1 distinct keys; at most 60, they share the row)
+    uint64_t prefix = lo >> shift;
+    for (int set = 0;; set = set == 2 ? 0 : set + 1) {
+        const int digit = shift > 8 ? shift - 8 : 0, mask = (1 << (shift - digit)) - 1;
+#pragma unroll
+        for (int j = 0; j < PER; j++)
+            if (key[j] <= limit && (key[j] >> shift) == prefix) atomicAdd(&sh.hist[set][static_cast<int>(key[j] >> digit) & mask], 1);
+        if (tid < 256) sh.hist[set == 2 ? 0 : set + 1][tid] = 0;
+        __syncthreads();
+        const int4 c = *reinterpret_cast<const int4 *>(&sh.hist[set][4 * lane]);
+        const int upto = wave_scan_i32(c.x + c.y + c.z + c.w);
+        int below = upto - (c.x + c.y + c.z + c.w), bin = 4 * lane, count = c.x;
+        const bool here = below < k && k <= upto;  // in one lane
+        if (below + count < k) below += count, bin++, count = c.y;
+        if (bin == 4 * lane + 1 && below + count < k) below += count, bin++, count = c.z;
+        if (bin == 4 * lane + 2 && below + count < k) below += count, bin++, count = c.w;
+        const int from = __builtin_ctzll(__builtin_amdgcn_ballot_w64(here));
+        k -= __builtin_amdgcn_readlane(below, from);
+        prefix = (prefix << (shift - digit)) | static_cast<uint64_t>(__builtin_amdgcn_readlane(bin, from));
+        shift = digit;
+        if (__builtin_amdgcn_readlane(count, from) == k) return (prefix << shift) | ((uint64_t(1) << shift) - 1);
+    }
+}
+
+template <int PER>
+__device__ __forceinline__ uint64_t thread_best(const uint64_t (&key)[PER]) {
+    uint64_t best = kNoKeyW;
+#pragma unroll
+    for (int j = 0; j < PER; j++) best = key[j] < best ? key[j] : best;
+    return best;
+}
+
+// The workgroup's keys <= bound to the slots [0, cap) of out, in no order, as far as they fit; *cnt (0 before) becomes
+// their number.  A wave asks for its slots with one addition.
+template <int PER>
+__device__ void compact_keys(const uint64_t (&key)[PER], uint64_t bound, uint64_t *out, int cap, int *cnt) {
+    const int lane = threadIdx.x & 63;
+    int n = 0;
+#pragma unroll
+    for (int j = 0; j < PER; j++) n += __popcll(__builtin_amdgcn_ballot_w64(key[j] <= bound));
+    if (n == 0) return;
+    int at = 0;
+    if (lane == 0) at = atomicAdd(cnt, n);
+    at = __builtin_amdgcn_readfirstlane(at);
+#pragma unroll
+    for (int j = 0; j < PER; j++) {
+        const uint64_t m = __builtin_amdgcn_ballot_w64(key[j] <= bound);
+        const int slot = at + __popcll(m & ((uint64_t(1) << lane) - 1));
+        if (key[j] <= bound && slot < cap) out[slot] = key[j];
+        at += __popcll(m);
+    }
+}
+
+// A chunk's winners, the k best keys and at most cap >= k, in no order, at out[(row * n_chunks + chunk) * cap], filled up
+// with kNoKeyW; the chunk's lowest NaN token.  The k-th best of the per-thread bests bounds every winner, and what is
+// below it usually fits the slots (k = 200: about 250 keys); only where it does not, the k best of all are looked for.
+__global__ void __launch_bounds__(kPickThreads)
+    pick_chunk_kernel(const float *__restrict__ logits, int64_t vocab, int64_t stride, int k, int cap, uint64_t *__restrict__ out,
+                      int32_t *__restrict__ nan_first) {
+    constexpr int kPer = kPickChunk / kPickThreads;
+    __shared__ KthShared<kPickThreads> sh;
+    __shared__ int cnt[2], nan_sh;
+    const int row = blockIdx.y, tid = threadIdx.x;
+    const float *x = logits + row * stride;
+    const int64_t base = static_cast<int64_t>(blockIdx.x) * kPickChunk + tid;
+    float v[kPer];
+#pragma unroll
+    for (int j = 0; j < kPer; j++) v[j] = x[base + j * kPickThreads < vocab ? base + j * kPickThreads : vocab - 1];
+    if (tid == 0) {
+        cnt[0] = cnt[1] = 0;
+        nan_sh = kNoNanW;
+    }
+    __syncthreads();
+    uint64_t key[kPer];
+#pragma unroll
+    for (int j = 0; j < kPer; j++) {
+        const int64_t i = base + j * kPickThreads;
+        const bool nan = v[j] != v[j];
+        if (i < vocab && nan) atomicMin(&nan_sh, static_cast<int32_t>(i));
+        key[j] = i < vocab && !nan ? (static_cast<uint64_t>(row) << 60) |
+                                         (static_cast<uint64_t>(desc_bits(__float_as_uint(v[j]))) << kWideTokenBits) | static_cast<uint64_t>(i)
+                                   : kNoKeyW;
+    }
+    const uint64_t best[1] = {thread_best(key)};
+    uint64_t bound = block_kth<1>(best, kNoKeyW - 1, k, sh);
+    const int64_t at = static_cast<int64_t>(row) * gridDim.x + blockIdx.x;
+    uint64_t *o = out + at * cap;
+    compact_keys(key, bound, o, cap, &cnt[0]);
+    __syncthreads();
+    int n = cnt[0];
+    if (n > cap) {
+        bound = block_kth<kPer>(key, bound, k, sh);
+        compact_keys(key, bound, o, cap, &cnt[1]);
+        n = k;
+    }
+    for (int i = n + tid; i < cap; i += kPickThreads) o[i] = kNoKeyW;
+    if (tid == 0) nan_first[at] = nan_sh;
+}
+
+// One row: the k best of its chunks' winners (n_chunks * cap <= PER * kPickMax slots), ranked by counting, then
+// wide_chain_kernel's chain with a candidate per thread.  The kept candidates go to keys_out / weights [row * k ..].
+template <int PER>
+__global__ void __launch_bounds__(kPickMax)
+    pick_row_kernel(const uint64_t *__restrict__ chunk_keys, const int32_t *__restrict__ chunk_nan, int n_chunks, int cap, ChainCfg cfg,
+                    WideWalk walk, RowDist *__restrict__ rows, uint64_t *__restrict__ keys_out, double *__restrict__ weights) {
+    constexpr int kFold = 16;  // additions per round of the sum
+    __shared__ KthShared<kPickMax> sh;
+    __shared__ uint64_t cand[kPickMax], sorted[kPickMax];
+    __shared__ alignas(16) double w_sh[kPickMax + kFold], upto[kPickMax];
+    __shared__ int rank_sh[kPickMax];
+    __shared__ int cnt[2], nan_sh;
+    const int row = blockIdx.x, tid = threadIdx.x, k = cfg.k, n_in = n_chunks * cap;
+    RowDist *d = rows + row;
+    uint64_t key[PER];
+#pragma unroll
+    for (int j = 0; j < PER; j++) {
+        const int i = j * kPickMax + tid;
+        const uint64_t got = chunk_keys[static_cast<int64_t>(row) * n_in + (i < n_in ? i : 0)];
+        key[j] = i < n_in ? got : kNoKeyW;
+    }
+    const int nan = tid < n_chunks ? chunk_nan[row * n_chunks + tid] : kNoNanW;  // (n_chunks <= kPickSlots / k < kPickMax)
+    rank_sh[tid] = 0;
+    if (tid == 0) {
+        cnt[0] = cnt[1] = 0;
+        nan_sh = kNoNanW;
+    }
+    __syncthreads();
+    if (nan != kNoNanW) atomicMin(&nan_sh, nan);
+    const uint64_t best[1] = {thread_best(key)};
+    uint64_t bound = block_kth<1>(best, kNoKeyW - 1, k, sh);  // (its barriers are behind the minimum)
+    auto finish = [&](int32_t err, int64_t err_index, int n_keep, double total, int32_t pick, double draft_weight) {
+        if (tid == 0) {
+            d->n_keep = n_keep;
+            d->err = err;
+            d->err_index = err_index;
+            d->total = total;
+            d->pick = pick;
+            d->draft_weight = draft_weight;
+            d->d_err = 0;
+            d->d_err_index = -1;
+        }
+    };
+    if (nan_sh != kNoNanW) return finish(DFLASH_ERR_NAN_LOGIT, nan_sh, 0, 0.0, 0, -0.0);
+    compact_keys(key, bound, cand, kPickMax, &cnt[0]);
+    __syncthreads();
+    int n = cnt[0];
+    if (n > kPickMax) {
+        bound = block_kth<PER>(key, bound, k, sh);
+        compact_keys(key, bound, cand, kPickMax, &cnt[1]);
+        __syncthreads();
+        n = cnt[1];
+    }
+    {
+        // candidate i = tid % n counts the candidates below it in slice tid / n of the list
+        const int slices = kPickMax / n, i = tid % n, sl = tid / n;
+        if (sl < slices) {
+            const int per = (n + slices - 1) / slices, j0 = sl * per, j1 = min(n, j0 + per);
+            const uint64_t x = cand[i];
+            int c = 0;
+#pragma unroll 8
+            for (int j = j0; j < j1; j++) c += cand[j] < x;
+            if (c) atomicAdd(&rank_sh[i], c);
+        }
+    }
+    __syncthreads();
+    if (tid < n && rank_sh[tid] < k) sorted[rank_sh[tid]] = cand[tid];
+    __syncthreads();
+    n = min(n, k);
+    const uint64_t mine = tid < n ? sorted[tid] : 0;
+    const double l = tid < n ? static_cast<double>(wide_key_logit(mine)) : 0.0, l0 = static_cast<double>(wide_key_logit(sorted[0]));
+    int len = n;
+    if (cfg.min_p > 0.0f && isfinite(l0)) len = __syncthreads_count(tid < len && l >= l0 + cfg.ln_min_p);  // a prefix of the order
+    if (len == 0) return finish(DFLASH_ERR_NO_CANDIDATES, -1, 0, 0.0, 0, -0.0);
+    double w = 0.0;
+    if (l0 == INFINITY) {
+        len = __syncthreads_count(tid < len && l == INFINITY);
+        w = tid < len ? 1.0 : 0.0;
+    } else {
+        const double temperature = static_cast<double>(cfg.temperature), max_logit = l0 / temperature;
+        if (max_logit == -INFINITY) return finish(DFLASH_ERR_NO_CANDIDATES, -1, 0, 0.0, 0, -0.0);
+        if (tid < len) w = exp(l / temperature - max_logit);
+        if (__syncthreads_or(!isfinite(w))) return finish(DFLASH_ERR_NO_CANDIDATES, -1, 0, 0.0, 0, -0.0);
+    }
+    w_sh[tid] = w;
+    if (tid < len) {
+        keys_out[static_cast<int64_t>(row) * k + tid] = mine;
+        weights[static_cast<int64_t>(row) * k + tid] = w;
+    }
+    __syncthreads();
+    if (tid >= 64) return;
+    // Every sum of the chain is a prefix of one: the weights added in order, one after the other (from +0 or -0 is the
+    // same, no weight is below +0), a round's elements asked for ahead of the round before it.
+    {
+        double acc = 0.0, r[kFold];
+#pragma unroll
+        for (int j = 0; j < kFold; j++) r[j] = w_sh[j];
+        for (int base = 0; base < len; base += kFold) {
+            double next[kFold];
+#pragma unroll
+            for (int j = 0; j < kFold; j++) next[j] = w_sh[base + kFold + j];
+#pragma unroll
+            for (int j = 0; j < kFold; j++) {
+                acc += r[j];
+                r[j] = acc;
+            }
+            if (tid == 0) {
+#pragma unroll
+                for (int j = 0; j < kFold; j++) upto[base + j] = r[j];
+            }
+#pragma unroll
+            for (int j = 0; j < kFold; j++) r[j] = next[j];
+        }
+    }
+    __builtin_amdgcn_s_waitcnt(0);
+    __builtin_amdgcn_wave_barrier();
+    auto first = [&](auto reached) {  // the first of [0, len) whose running sum does, or len - 1
+        for (int base = 0; base < len; base += 64) {
+            const uint64_t m = __builtin_amdgcn_ballot_w64(base + tid < len && reached(upto[base + tid < len ? base + tid : 0]));
+            if (m) return base + static_cast<int>(__builtin_ctzll(m));
+        }
+        return len - 1;
+    };
+    if (cfg.top_p < 1.0f) {
+        const double target = upto[len - 1] * static_cast<double>(cfg.top_p);
+        len = first([&](double s) { return s >= target; }) + 1;
+    }
+    const double total = upto[len - 1];
+    if (!(isfinite(total) && total > 0.0)) return finish(DFLASH_ERR_NO_CANDIDATES, -1, 0, 0.0, 0, -0.0);
+    const double drawn = walk.uniforms[row] * total;
+    const int at = first([&](double s) { return drawn < s; });
+    double draft_weight = -0.0;
+    for (int base = 0; base < len; base += 64) {  // (tokens are distinct: at most one is the draft)
+        const uint64_t m = __builtin_amdgcn_ballot_w64(base + tid < len && row + 1 < walk.n_tokens &&
+                                                       static_cast<int32_t>(sorted[base + tid] & kWideTokenMask) == walk.verified[row + 1]);
+        if (m) draft_weight = w_sh[base + __builtin_ctzll(m)];
+    }
+    finish(0, -1, len, total, static_cast<int32_t>(sorted[at] & kWideTokenMask), draft_weight);
+}
+
+// ------------------------------------------------------------------------------------------
+// the full order
+// ------------------------------------------------------------------------------------------
 __global__ void wide_init_kernel(int32_t *nan_first, int n) {
     if (static_cast<int>(threadIdx.x) < n) nan_first[threadIdx.x] = kNoNanW;
 }
@@ -66,9 +361,9 @@ __device__ int64_t block_sum_i64(int64_t v, int64_t *sh) {
 }
 
 // The reference's `acc = start; for w in weights[..n] { acc += w }` by thread 0, weights staged through LDS.
-// With stop_at >= 0 the fold stops after the first element that brings the sum to >= stop_at (top-p); *count is
-// the number of elements added.  Returns the sum (to every thread).
-__device__ double sequential_fold(const double *__restrict__ w, int64_t n, double start, bool use_stop, double stop_at,
+// With use_stop the fold stops after the first element that brings the sum to >= stop_at (top-p; strict: above it, the
+// categorical pick); *count is the number of elements added.  Returns the sum (to every thread).
+__device__ double sequential_fold(const double *__restrict__ w, int64_t n, double start, bool use_stop, bool strict, double stop_at,
                                   int64_t *count, double *tile, double *bcast, int64_t *bcast_n, int *done) {
     if (threadIdx.x == 0) {
         *bcast = start;
@@ -85,7 +380,7 @@ __device__ double sequential_fold(const double *__restrict__ w, int64_t n, doubl
             int i = 0;
             for (; i < m; i++) {
                 acc += tile[i];
-                if (use_stop && acc >= stop_at) {
+                if (use_stop && (strict ? stop_at < acc : acc >= stop_at)) {
                     i++;
                     *done = 1;
                     break;
@@ -105,8 +400,8 @@ __device__ double sequential_fold(const double *__restrict__ w, int64_t n, doubl
 
 // sampling.rs:1541-1615 on the ordered candidates of one row; weights[row * vocab + i] receives candidate i's weight
 __global__ void __launch_bounds__(kWideThreads)
-    wide_chain_kernel(const uint64_t *__restrict__ keys_sorted, int64_t vocab, ChainCfg cfg, const int32_t *__restrict__ nan_first,
-                      RowDist *__restrict__ rows, double *__restrict__ weights) {
+    wide_chain_kernel(const uint64_t *__restrict__ keys_sorted, int64_t vocab, ChainCfg cfg, WideWalk walk,
+                      const int32_t *__restrict__ nan_first, RowDist *__restrict__ rows, double *__restrict__ weights) {
     __shared__ double tile[kWideTile];
     __shared__ int64_t red[kWideThreads / 64];
     __shared__ double bcast;
@@ -124,6 +419,8 @@ __global__ void __launch_bounds__(kWideThreads)
             d->total = total;
             d->d_err = 0;
             d->d_err_index = -1;
+            d->pick = 0;
+            d->draft_weight = -0.0;
         }
     };
     if (nan_first[row] != kNoNanW) return finish(DFLASH_ERR_NAN_LOGIT, nan_first[row], 0, 0.0);
@@ -159,23 +456,59 @@ __global__ void __launch_bounds__(kWideThreads)
     }
     __syncthreads();  // the weights are read back by other threads below
     if (cfg.top_p < 1.0f) {
-        const double total = sequential_fold(w, len, -0.0, false, 0.0, nullptr, tile, &bcast, &bcast_n, &done);
+        const double total = sequential_fold(w, len, -0.0, false, false, 0.0, nullptr, tile, &bcast, &bcast_n, &done);
         const double target = total * static_cast<double>(cfg.top_p);
         int64_t keep = 0;
-        sequential_fold(w, len, 0.0, true, target, &keep, tile, &bcast, &bcast_n, &done);
+        sequential_fold(w, len, 0.0, true, false, target, &keep, tile, &bcast, &bcast_n, &done);
         len = keep < 1 ? 1 : keep;
     }
-    const double total_weight = sequential_fold(w, len, -0.0, false, 0.0, nullptr, tile, &bcast, &bcast_n, &done);
+    const double total_weight = sequential_fold(w, len, -0.0, false, false, 0.0, nullptr, tile, &bcast, &bcast_n, &done);
     if (!(isfinite(total_weight) && total_weight > 0.0)) return finish(DFLASH_ERR_NO_CANDIDATES, -1, 0, 0.0);
+    // what the decision takes from the row's order: the token its draw falls on, and the weight of its draft
+    int64_t upto = 0;
+    const double drawn = walk.uniforms[row] * total_weight;
+    const double sum = sequential_fold(w, len, 0.0, true, true, drawn, &upto, tile, &bcast, &bcast_n, &done);
     finish(0, -1, len, total_weight);
+    __syncthreads();  // (thread 0 has cleared the draft's weight)
+    if (tid == 0) d->pick = static_cast<int32_t>(keys[(drawn < sum ? upto : len) - 1] & kWideTokenMask);
+    if (row + 1 < walk.n_tokens)  // (tokens are distinct: at most one is the draft)
+        for (int64_t i = tid; i < len; i += kWideThreads)
+            if (static_cast<int32_t>(keys[i] & kWideTokenMask) == walk.verified[row + 1]) d->draft_weight = w[i];
 }
 
 }  // namespace
 
 int32_t dfl_accept_wide_rows(dflash_ctx *ctx, const float *logits, int32_t n_rows, int64_t vocab, int64_t stride, const ChainCfg &cfg,
-                             RowDist *rows, size_t *ws_off, const uint64_t **keys_out, const double **weights_out, hipStream_t st) {
+                             const WideWalk &walk, RowDist *rows, size_t *ws_off, const uint64_t **keys_out, const double **weights_out,
+                             int64_t *out_stride, hipStream_t st) {
     if (n_rows > 16 || vocab >= (int64_t(1) << kWideTokenBits))
         return dfl_fail(ctx, DFLASH_ERR_UNSUPPORTED, "accept_prefix: wide top-k needs <= 16 rows and a vocabulary below 2^28");
+    // Selection where a thread can hold each candidate and a workgroup the winners of all of a row's chunks (k <= 862 at
+    // 151936 tokens); the sort is the only one that has no such bound.
+    const int64_t n_chunks = (vocab + kPickChunk - 1) / kPickChunk;
+    if (cfg.k <= kPickMax && n_chunks * cfg.k <= kPickSlots) {
+        const int cap = static_cast<int>(std::min<int64_t>(2 * cfg.k, kPickSlots / n_chunks));
+        const size_t slots = static_cast<size_t>(n_chunks) * cap, kept = static_cast<size_t>(n_rows) * cfg.k;
+        uint64_t *winners = dfl_ws_take<uint64_t>(ctx, ws_off, n_rows * slots * sizeof(uint64_t));
+        int32_t *nans = dfl_ws_take<int32_t>(ctx, ws_off, n_rows * n_chunks * sizeof(int32_t));
+        uint64_t *keys = dfl_ws_take<uint64_t>(ctx, ws_off, kept * sizeof(uint64_t));
+        double *weights = dfl_ws_take<double>(ctx, ws_off, kept * sizeof(double));
+        if (!winners || !nans || !keys || !weights)
+            return dfl_fail(ctx, DFLASH_ERR_WORKSPACE,
+                            "accept_prefix: top_k %lld over a vocabulary of %lld needs about %zu KB of context workspace",
+                            static_cast<long long>(cfg.k), static_cast<long long>(vocab), (n_rows * slots + 2 * kept) * 8 >> 10);
+        const int nc = static_cast<int>(n_chunks);
+        pick_chunk_kernel<<<dim3(nc, n_rows), kPickThreads, 0, st>>>(logits, vocab, stride, cfg.k, cap, winners, nans);
+        if (slots <= 8 * kPickMax)
+            pick_row_kernel<8><<<n_rows, kPickMax, 0, st>>>(winners, nans, nc, cap, cfg, walk, rows, keys, weights);
+        else
+            pick_row_kernel<16><<<n_rows, kPickMax, 0, st>>>(winners, nans, nc, cap, cfg, walk, rows, keys, weights);
+        DFL_HIP_CHECK(ctx, hipGetLastError());
+        *keys_out = keys;
+        *weights_out = weights;
+        *out_stride = cfg.k;
+        return DFLASH_OK;
+    }
     const size_t n = static_cast<size_t>(n_rows) * static_cast<size_t>(vocab);
     uint64_t *keys_a = dfl_ws_take<uint64_t>(ctx, ws_off, n * sizeof(uint64_t));
     uint64_t *keys_b = dfl_ws_take<uint64_t>(ctx, ws_off, n * sizeof(uint64_t));
@@ -192,9 +525,10 @@ int32_t dfl_accept_wide_rows(dflash_ctx *ctx, const float *logits, int32_t n_row
     wide_init_kernel<<<1, 64, 0, st>>>(nan_first, n_rows);
     wide_keys_kernel<<<dim3(static_cast<unsigned>((vocab + 255) / 256), n_rows), 256, 0, st>>>(logits, vocab, stride, keys_a, nan_first);
     DFL_HIP_CHECK(ctx, rocprim::radix_sort_keys(tmp, tmp_bytes, keys_a, keys_b, n, 0, 64, st, false));
-    wide_chain_kernel<<<n_rows, kWideThreads, 0, st>>>(keys_b, vocab, cfg, nan_first, rows, weights);
+    wide_chain_kernel<<<n_rows, kWideThreads, 0, st>>>(keys_b, vocab, cfg, walk, nan_first, rows, weights);
     DFL_HIP_CHECK(ctx, hipGetLastError());
     *keys_out = keys_b;
     *weights_out = weights;
+    *out_stride = vocab;
     return DFLASH_OK;
 }

@@ -26,10 +26,10 @@ struct RowDist {
     double weights[kMaxK];
     // dense proposal side
     int32_t d_err;
-    int32_t d_pad;
+    int32_t pick;  // wide sets: the token the row's draw falls on
     int64_t d_err_index;
     double d_max_scaled;  // f64(max draft logit) / T
-    double d_total;       // P
+    double draft_weight;  // wide sets: weight of the row's draft among the kept candidates, -0 if it is not one
 };
 
 struct ChainCfg {
@@ -57,6 +57,42 @@ __device__ __forceinline__ float key_logit(uint64_t key) {
     return __uint_as_float(bits);
 }
 __device__ __forceinline__ int32_t key_token(uint64_t key) { return static_cast<int32_t>(static_cast<uint32_t>(key)); }
+
+// Minimum of a key over the wave, in every lane: data-parallel-primitive moves within rows of 16 lanes (shift right
+// by 1, 2, 4, 8: lane 15 of a row then holds the row's minimum), then lane 15 of rows 0 and 2 into rows 1 and 3, then
+// lane 31 into rows 2 and 3; lane 63 has the result.  Lanes without a source read the identity.  No LDS round trips.
+__device__ __forceinline__ uint64_t wave_min_u64(uint64_t v) {
+#define DFL_MIN_STEP(ctrl, row_mask)                                                                                     \
+    do {                                                                                                                 \
+        const unsigned lo = __builtin_amdgcn_update_dpp(0xffffffffu, static_cast<unsigned>(v), ctrl, row_mask, 0xf, false);       \
+        const unsigned hi = __builtin_amdgcn_update_dpp(0xffffffffu, static_cast<unsigned>(v >> 32), ctrl, row_mask, 0xf, false); \
+        const uint64_t o = (static_cast<uint64_t>(hi) << 32) | lo;                                                       \
+        v = o < v ? o : v;                                                                                               \
+    } while (0)
+    DFL_MIN_STEP(0x111, 0xf);  // row_shr:1
+    DFL_MIN_STEP(0x112, 0xf);  // row_shr:2
+    DFL_MIN_STEP(0x114, 0xf);  // row_shr:4
+    DFL_MIN_STEP(0x118, 0xf);  // row_shr:8
+    DFL_MIN_STEP(0x142, 0xa);  // row_bcast:15 into rows 1 and 3
+    DFL_MIN_STEP(0x143, 0xc);  // row_bcast:31 into rows 2 and 3
+#undef DFL_MIN_STEP
+    const unsigned lo = __builtin_amdgcn_readlane(static_cast<unsigned>(v), 63);
+    const unsigned hi = __builtin_amdgcn_readlane(static_cast<unsigned>(v >> 32), 63);
+    return (static_cast<uint64_t>(hi) << 32) | lo;
+}
+
+// Inclusive sum over the wave's lanes, by the same moves.
+__device__ __forceinline__ int wave_scan_i32(int v) {
+#define DFL_SUM_STEP(ctrl, row_mask) v += __builtin_amdgcn_update_dpp(0, v, ctrl, row_mask, 0xf, false)
+    DFL_SUM_STEP(0x111, 0xf);
+    DFL_SUM_STEP(0x112, 0xf);
+    DFL_SUM_STEP(0x114, 0xf);
+    DFL_SUM_STEP(0x118, 0xf);
+    DFL_SUM_STEP(0x142, 0xa);
+    DFL_SUM_STEP(0x143, 0xc);
+#undef DFL_SUM_STEP
+    return v;
+}
 
 // sampling.rs:1541-1615 on the ordered candidates of one row (keys ascending = best first)
 // Work arrays of the chain (kMaxK entries each): a caller that runs the chain on one thread of a workgroup

@@ -459,6 +459,27 @@ def test_wide_top_k_edge_rows(ctx, oracle):
             assert_same(oracle, *r)
 
 
+@pytest.mark.parametrize("vocab,top_k", [(66, 65), (1024, 1024), (1025, 1024), (8192, 1023), (8193, 200), (16385, 1024), (32769, 819), (32769, 820),
+                                         (131073, 963), (131073, 964), (9000, 1025)])
+def test_wide_selection_at_its_edges(ctx, oracle, vocab, top_k):
+    """Candidate sets around the selection's limits (1024 candidates, 4096 and 16384 chunk winners per row, chunks of
+    8192 tokens) over logits with many ties, mixed signs, infinities and rows with fewer finite logits than top_k."""
+    rng = np.random.default_rng(vocab * 31 + top_k)
+    n = 4
+    for trial in range(3):
+        tl = np.round(rng.standard_normal((n, vocab)) * 3.0, 0 if trial == 1 else 2).astype(np.float32)
+        if trial == 2:
+            tl[0, 50:] = -np.inf
+            tl[1] = -np.abs(tl[1]) - 1.0
+            tl[2] = 0.25
+        drafts = [int(np.argmax(tl[r])) for r in range(n - 1)]
+        props = [(d, [(d, 0.75), ((d + 1) % vocab, 0.25)]) for d in drafts]
+        for p in (None, props):
+            r = both(ctx, oracle, [1] + drafts, tl, vocab, p, 100, [], temperature=0.8, top_k=top_k, top_p=0.97 if trial else 1.0,
+                     min_p=0.0, seed=trial)
+            assert_same(oracle, *r)
+
+
 def test_qwen_chat_preset_full_vocabulary(ctx, oracle):
     """The reference's default chat sampler (temperature 0.7, top_k 200, min_p 0.05) at vocabulary 151936, block 16, both
     random streams, coupled to drafts sampled from the vocabulary-wide draft distribution and to deterministic drafts."""
