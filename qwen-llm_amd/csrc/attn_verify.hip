@@ -144,25 +144,40 @@ __device__ __forceinline__ void attn_wait(int n) {
 // them, the maximum crosses the lanes without LDS, the last stage's special cases stand outside of the others' code, and
 // a load's address is made of one lane part and one uniform part: 16 rows x 100 k keys, 48 / 8 heads of 128, with the
 // merge: 110 -> 99 us (4.1 TB/s of keys and values; a copy reaches 5.07).
-template <int HD, typename TQ, int MAXW, int MAXL>
-__global__ void __launch_bounds__(64 * MAXW)
-    attn_split_kernel(const TQ *__restrict__ q, const _Float16 *__restrict__ k_cache,
-                      const _Float16 *__restrict__ vt_cache, float *__restrict__ part_o, float *__restrict__ part_ml,
-                      int64_t ctx_len, const int32_t *__restrict__ ctx_len_dev, int n_rows_total, int n_q, int n_kv,
-                      int64_t vt_stride, int want, int min_chunk, float scale, int full_block, int64_t window,
-                      int split_stride, int64_t part_slots) {
-    // blockIdx.z: which block of sixteen query rows (a prefill group hands over many: block b's rows follow block
+// Splits are merged in order: what came before times `old`, plus the next one's result times `next`.
+struct AttnMerge {
+    float m, old, next;
+    __device__ __forceinline__ AttnMerge(float m_before, float m_next) {
+        m = fmaxf(m_before, m_next);
+        old = m_before == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_before - m);
+        next = m_next == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_next - m);
+    }
+    __device__ __forceinline__ float add(float before, float v) const { return __builtin_fmaf(next, v, old * before); }
+};
+
+// MERGE: the workgroup takes all of its rows' keys, split by split, and merges the splits as it goes (see
+// attn_rows_kernel); else one split, whose partial result it writes.
+template <int HD, typename TQ, int MAXW, int MAXL, bool MERGE>
+__device__ __forceinline__ void attn_body(const TQ *__restrict__ q, const _Float16 *__restrict__ k_cache,
+                                          const _Float16 *__restrict__ vt_cache, float *__restrict__ part_o, float *__restrict__ part_ml,
+                                          int64_t ctx_len, const int32_t *__restrict__ ctx_len_dev, int n_rows_total, int n_q, int n_kv,
+                                          int64_t vt_stride, int want, int min_chunk, float scale, int full_block, int64_t window,
+                                          int split_stride, int64_t part_slots, int block, float *__restrict__ out, void *__restrict__ out_xf,
+                                          int out_xf_kind, size_t xf_stride) {
+    // block: which block of sixteen query rows (a prefill group hands over many: block b's rows follow block
     // b - 1's in q and in the cache, its partial tiles sit part_slots slots further on)
-    const int n_rows = min(16, n_rows_total - 16 * static_cast<int>(blockIdx.z));
-    q += static_cast<int64_t>(blockIdx.z) * 16 * n_q * HD;
-    part_o += static_cast<int64_t>(blockIdx.z) * part_slots * HD;
-    part_ml += static_cast<int64_t>(blockIdx.z) * part_slots * 2;
+    const int n_rows = min(16, n_rows_total - 16 * block);
+    q += static_cast<int64_t>(block) * 16 * n_q * HD;
+    if constexpr (!MERGE) {
+        part_o += static_cast<int64_t>(block) * part_slots * HD;
+        part_ml += static_cast<int64_t>(block) * part_slots * 2;
+    }
     constexpr int KS = HD / 32;       // k-steps of the score product
     constexpr int DT = HD / 16;       // 16-dim tiles of the output
     constexpr int CH = HD / 8;        // 16-byte chunks per key row
     constexpr int kKPieces = 32 * CH; // pieces of the K tile; the V^T tile has as many
     constexpr int kWaveLoads = 2 * kKPieces / 64;
-    static_assert(HD < 256 || MAXW == 8, "sixteen waves leave a wave 128 registers");
+    static_assert(HD < 256 || MAXW <= 8, "sixteen waves leave a wave 128 registers");
     extern __shared__ half8_t lds[];  // kAttnBufs x (K tile, V^T tile)
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -172,20 +187,20 @@ __global__ void __launch_bounds__(64 * MAXW)
     const int kvh = blockIdx.y;
     // blockIdx.x = split + split_stride * (part of the GQA group this workgroup serves); split_stride is a multiple
     // of 8, so the workgroups that read one chunk of keys are dispatched to the same XCD and share its L2 copy
-    const int split = blockIdx.x % split_stride;
-    const int head = kvh * group + (blockIdx.x / split_stride) * n_waves + wave;  // this wave's query head
+    const int split = MERGE ? 0 : blockIdx.x % split_stride;
+    const int head = kvh * group + (MERGE ? blockIdx.x : blockIdx.x / split_stride) * n_waves + wave;  // this wave's query head
     // Q^T fragments: lane (row n, g) holds Q[n][head][32 s + 8 g ..+8]
     // (rows at or past n_rows repeat the last row: they are never stored)
     AttnQ8<TQ> q_raw[KS];
     const TQ *qrow = q + (static_cast<int64_t>(min(n, n_rows - 1)) * n_q + head) * HD + 8 * g;
     attn_load_q<0, KS>(q_raw, qrow);
     if (ctx_len_dev) ctx_len = *ctx_len_dev;
-    ctx_len += 16 * static_cast<int64_t>(blockIdx.z);
+    ctx_len += 16 * static_cast<int64_t>(block);
     const int64_t n_pos = ctx_len + n_rows;
     const int64_t chunk = attn_chunk(n_pos, want, min_chunk);
-    if (split * chunk >= n_pos) return;  // the grid is sized for the longest context
-    const int64_t c0 = split * chunk;
-    const int64_t c1 = min(n_pos, c0 + chunk);
+    if (!MERGE && split * chunk >= n_pos) return;  // the grid is sized for the longest context
+    const int64_t c0 = MERGE ? 0 : split * chunk;
+    const int64_t c1 = MERGE ? n_pos : min(n_pos, c0 + chunk);
     const int n_steps = static_cast<int>((c1 - c0 + 31) / 32);
     const int64_t kv_dim = static_cast<int64_t>(n_kv) * HD;
     const int per_wave = (kWaveLoads + n_waves - 1) / n_waves;  // loads each wave issues per stage
@@ -292,6 +307,15 @@ __global__ void __launch_bounds__(64 * MAXW)
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
     };
+    // MERGE: what the splits so far come to; the split at hand ends ahead of stage split_end
+    float4_t tot[MERGE ? DT : 1];
+    float m_tot = -INFINITY, l_tot = 0.0f;
+    const int chunk_steps = static_cast<int>(min(chunk / 32, static_cast<int64_t>(0x3fffffff)));
+    int split_end = chunk_steps;
+    bool split_begins = true;
+    if constexpr (MERGE)
+#pragma unroll
+        for (int t = 0; t < DT; t++) tot[t] = float4_t{0, 0, 0, 0};
     float4_t sc[2], sc_next[2];
     landed(0);
     scores(0, sc);
@@ -330,7 +354,7 @@ __global__ void __launch_bounds__(64 * MAXW)
             psum += p[i];
         }
         l_run = __builtin_fmaf(l_run, alpha, psum);
-        if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {
+        if (!(MERGE && split_begins) && __builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {
 #pragma unroll
             for (int t = 0; t < DT; t++) acc[t] *= alpha;
         }
@@ -349,14 +373,67 @@ __global__ void __launch_bounds__(64 * MAXW)
                 for (int i = 0; i < 8; i++)
                     if (i >= vkeys) vf[t][i] = static_cast<_Float16>(0.0f);
         }
+        if (MERGE && split_begins) {  // (as from an accumulator of zeros)
 #pragma unroll
-        for (int t = 0; t < DT; t++) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf[t], pf, acc[t], 0, 0, 0);
+            for (int t = 0; t < DT; t++) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf[t], pf, float4_t{0, 0, 0, 0}, 0, 0, 0);
+        } else {
+#pragma unroll
+            for (int t = 0; t < DT; t++) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf[t], pf, acc[t], 0, 0, 0);
+        }
+        if constexpr (MERGE) {
+            split_begins = st + 1 == split_end || st + 1 == n_steps;
+            if (split_begins) {
+                float l = l_run;
+                l += xor_lane(l, 16);
+                l += xor_lane(l, 32);
+                const AttnMerge w(m_tot, m_run);
+                l_tot = w.add(l_tot, l);
+                if (__builtin_amdgcn_ballot_w64(w.old != 1.0f) != 0) {
+#pragma unroll
+                    for (int t = 0; t < DT; t++) tot[t] *= w.old;
+                }
+#pragma unroll
+                for (int t = 0; t < DT; t++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++) tot[t][i] = __builtin_fmaf(w.next, acc[t][i], tot[t][i]);
+                m_tot = w.m;
+                m_run = -INFINITY;
+                l_run = 0.0f;
+                split_end += chunk_steps;
+            }
+        }
         sc[0] = sc_next[0];
         sc[1] = sc_next[1];
         if (st < 8) ATT_TR(3 + st);
     }
     ATT_TR(12);
 
+    if constexpr (MERGE) {
+        float *o = out + ((static_cast<int64_t>(block) * 16 + n) * n_q + head) * HD;
+#pragma unroll
+        for (int t = 0; t < DT; t++) {
+            tot[t] /= l_tot;
+            if (n < n_rows) *reinterpret_cast<float4_t *>(o + 16 * t + 4 * g) = tot[t];
+        }
+        if (out_xf) {
+            out_xf = static_cast<uint8_t *>(out_xf) + block * xf_stride;
+            // a lane has four dims of an octet, the lane 16 away the other four: even lane rows take tile t's, odd ones tile t + 1's
+#pragma unroll
+            for (int t = 0; t < DT; t += 2) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    float lo = tot[t][i], hi = tot[t + 1][i];
+                    dfl_swap16(lo, hi);
+                    tot[t][i] = lo;
+                    tot[t + 1][i] = hi;
+                }
+                const float4_t a = tot[t], b = tot[t + 1];
+                if (n < n_rows)
+                    dfl_xf_store(out_xf, out_xf_kind, n, head * HD + 16 * (t + (g & 1)) + 8 * (g >> 1), a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]);
+            }
+        }
+        return;
+    }
     // row sums over the four lanes of a row; partials: O^T tile t, lane (row n, g) holds dims 16 t + 4 g + i
     float l = l_run;
     l += xor_lane(l, 16);
@@ -372,6 +449,43 @@ __global__ void __launch_bounds__(64 * MAXW)
         }
     }
     ATT_TR(13);
+}
+
+template <int HD, typename TQ, int MAXW, int MAXL>
+__global__ void __launch_bounds__(64 * MAXW)
+    attn_split_kernel(const TQ *__restrict__ q, const _Float16 *__restrict__ k_cache,
+                      const _Float16 *__restrict__ vt_cache, float *__restrict__ part_o, float *__restrict__ part_ml,
+                      int64_t ctx_len, const int32_t *__restrict__ ctx_len_dev, int n_rows_total, int n_q, int n_kv,
+                      int64_t vt_stride, int want, int min_chunk, float scale, int full_block, int64_t window,
+                      int split_stride, int64_t part_slots) {
+    attn_body<HD, TQ, MAXW, MAXL, false>(q, k_cache, vt_cache, part_o, part_ml, ctx_len, ctx_len_dev, n_rows_total, n_q, n_kv, vt_stride, want,
+                                         min_chunk, scale, full_block, window, split_stride, part_slots, blockIdx.z, nullptr, nullptr, 0, 0);
+}
+
+// Many blocks of rows at once, a prompt's prefill: the blocks are enough workgroups, so one takes all of its block's keys
+// and the partial results never leave its registers.  The splits stay (a block's own policy: want and min_chunk of the
+// run of blocks it belongs to) as the points where the running result is merged, in the order and with the
+// arithmetic of attn_combine_ordered_kernel: the same bits as the block on its own.  Blocks of one launch differ in their
+// keys: the longest go first.  Bound by a stage's chain, as the split kernel (1.3 us a stage with two workgroups on a CU):
+// 1000 rows of 32 / 8 heads of 128, the first to the last: 153 us as splits and their merges, 42 us here.  (Two blocks per
+// workgroup, sharing its keys and values: 50 us; the bytes are not what bounds it.)
+constexpr int kAttnRuns = 16;
+struct AttnRuns {
+    int n, first[kAttnRuns], want[kAttnRuns], min_chunk[kAttnRuns];
+};
+template <int HD, int MAXL>
+__global__ void __launch_bounds__(512)
+    attn_rows_kernel(const float *__restrict__ q, const _Float16 *__restrict__ k_cache, const _Float16 *__restrict__ vt_cache, int64_t ctx_len,
+                     int n_rows_total, int n_q, int n_kv, int64_t vt_stride, AttnRuns runs, float scale, float *__restrict__ out,
+                     void *__restrict__ out_xf, int out_xf_kind, size_t xf_stride) {
+    const int block = gridDim.z - 1 - blockIdx.z;
+    int want = runs.want[0], min_chunk = runs.min_chunk[0];
+    for (int r = 1; r < runs.n && runs.first[r] <= block; r++) {
+        want = runs.want[r];
+        min_chunk = runs.min_chunk[r];
+    }
+    attn_body<HD, float, 8, MAXL, true>(q, k_cache, vt_cache, nullptr, nullptr, ctx_len, nullptr, n_rows_total, n_q, n_kv, vt_stride, want, min_chunk,
+                                        scale, 0, 0, 1, 0, block, out, out_xf, out_xf_kind, xf_stride);
 }
 
 #ifdef DFLASH_TRACE
@@ -564,6 +678,66 @@ __global__ void __launch_bounds__(HD == 64 ? 128 : 256)
     }
 }
 
+// The partial results merged one after the other, as attn_rows_kernel does (which blocks take this: see attn_policy).  What bounds it is its chain: a trip to memory for the maxima and the partial outputs, which
+// are in flight together, then the merges.  Lane s of every wave keeps split s's maximum and sum and computes its two factors
+// (the maximum of the splits before it is a scan over the lanes); a thread adds up one dim, with the factors read from the lane
+// they are in: no LDS, no barrier.
+constexpr int kOrderedSplits = 32;
+template <int HD>
+__global__ void __launch_bounds__(HD)
+    attn_combine_ordered_kernel(const float *__restrict__ part_o, const float *__restrict__ part_ml, float *__restrict__ out, int n_rows_total,
+                            int n_q, int64_t ctx_len, const int32_t *__restrict__ ctx_len_dev, int want, int min_chunk,
+                            void *__restrict__ out_xf, int out_xf_kind, int64_t part_slots, size_t xf_stride, int max_splits) {
+    const int n_rows = min(16, n_rows_total - 16 * static_cast<int>(blockIdx.z));
+    if (static_cast<int>(blockIdx.y) >= n_rows) return;
+    const int head = blockIdx.x, row = blockIdx.y, d = threadIdx.x, lane = d & 63;
+    const int64_t slot_stride = static_cast<int64_t>(n_q) * 16;
+    const float2 *ml = reinterpret_cast<const float2 *>(part_ml) + static_cast<int64_t>(blockIdx.z) * part_slots + head * 16 + row;
+    const float *po = part_o + (static_cast<int64_t>(blockIdx.z) * part_slots + head * 16 + row) * HD + d;
+    const float2 own = ml[min(lane, max_splits - 1) * slot_stride];
+    float o[kOrderedSplits];
+#pragma unroll
+    for (int s = 0; s < kOrderedSplits; s++) {
+        if ((s & ~7) >= max_splits) continue;  // (uniform; past the last split it is read again)
+        o[s] = po[min(s, max_splits - 1) * slot_stride * HD];
+    }
+    if (ctx_len_dev) ctx_len = *ctx_len_dev;
+    const int n_splits = attn_splits(ctx_len + 16 * static_cast<int64_t>(blockIdx.z) + n_rows, want, min_chunk);
+    const float m = lane < n_splits ? own.x : -INFINITY;
+    const int none = __builtin_bit_cast(int, -INFINITY);
+    float upto = m;
+#define DFL_MAX_STEP(ctrl, row_mask) \
+    upto = fmaxf(upto, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(none, __builtin_bit_cast(int, upto), ctrl, row_mask, 0xf, false)))
+    DFL_MAX_STEP(0x111, 0xf);  // row_shr:1, 2, 4, 8
+    DFL_MAX_STEP(0x112, 0xf);
+    DFL_MAX_STEP(0x114, 0xf);
+    DFL_MAX_STEP(0x118, 0xf);
+    DFL_MAX_STEP(0x142, 0xa);  // row_bcast:15 into rows 1 and 3
+    DFL_MAX_STEP(0x143, 0xc);  // row_bcast:31 into rows 2 and 3
+#undef DFL_MAX_STEP
+    const float before = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(none, __builtin_bit_cast(int, upto), 0x138, 0xf, 0xf, false));  // wave_shr:1
+    const AttnMerge w(before, m);
+    auto at = [](float v, int s) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), s)); };
+    float acc = 0.0f, l = 0.0f;
+#pragma unroll
+    for (int s = 0; s < kOrderedSplits; s++) {
+        if ((s & ~7) >= max_splits) continue;
+        if (s < n_splits) {
+            const float old = at(w.old, s), next = at(w.next, s);
+            acc = __builtin_fmaf(next, o[s], old * acc);
+            l = __builtin_fmaf(next, at(own.y, s), old * l);
+        }
+    }
+    const float v = acc / l;
+    out[((static_cast<int64_t>(blockIdx.z) * 16 + row) * n_q + head) * HD + d] = v;
+    if (out_xf) {
+        // eight consecutive dims sit in eight consecutive lanes of a row of sixteen
+        const float e[8] = {v, dfl_dpp<0x101>(v), dfl_dpp<0x102>(v), dfl_dpp<0x103>(v), dfl_dpp<0x104>(v), dfl_dpp<0x105>(v), dfl_dpp<0x106>(v), dfl_dpp<0x107>(v)};
+        if ((d & 7) == 0)
+            dfl_xf_store(static_cast<uint8_t *>(out_xf) + blockIdx.z * xf_stride, out_xf_kind, row, head * HD + d, e[0], e[1], e[2], e[3], e[4], e[5], e[6], e[7]);
+    }
+}
+
 // V [pos][n_kv][hd] -> V^T [n_kv][hd][stride]; one workgroup per (32 positions, kv head)
 __global__ void __launch_bounds__(256) transpose_v_kernel(const _Float16 *__restrict__ v, _Float16 *__restrict__ vt,
                                                           int64_t n_pos, int n_kv, int hd, int64_t stride) {
@@ -620,6 +794,20 @@ int32_t launch_split(dflash_ctx *ctx, dim3 grid, int threads, hipStream_t st, co
     return DFLASH_OK;
 }
 
+template <int HD>
+int32_t launch_rows(dflash_ctx *ctx, dim3 grid, int n_waves, hipStream_t st, const float *q, const _Float16 *k, const _Float16 *vt, int64_t ctx_len,
+                    int n_rows, int n_q, int n_kv, int64_t vt_stride, const AttnRuns &runs, float scale, float *out, void *out_xf, int out_xf_kind) {
+    const size_t lds = static_cast<size_t>(kAttnBufs) * 2 * (32 * HD / 8) * sizeof(half8_t);
+    constexpr int kWaveLoads = 2 * 32 * (HD / 8) / 64;
+    const int per_wave = (kWaveLoads + n_waves - 1) / n_waves;
+    const auto fn = per_wave <= 4 ? attn_rows_kernel<HD, 4> : per_wave <= 8 ? attn_rows_kernel<HD, 8> : attn_rows_kernel<HD, 16>;
+    if (const int32_t rc_ = dfl_raise_lds_limit(ctx, reinterpret_cast<const void *>(fn), lds)) return rc_;
+    fn<<<grid, 64 * n_waves, lds, st>>>(q, k, vt, ctx_len, n_rows, n_q, n_kv, vt_stride, runs, scale, out, out_xf, out_xf_kind,
+                                       dfl_xf_bytes(static_cast<int64_t>(n_q) * HD));
+    DFL_HIP_CHECK(ctx, hipGetLastError());
+    return DFLASH_OK;
+}
+
 }  // namespace
 
 extern "C" int32_t dflash_attn_verify_block(dflash_ctx *ctx, const void *q, int32_t q_type, const void *k_cache,
@@ -647,42 +835,10 @@ int32_t dfl_attn_block(dflash_ctx *ctx, const void *q, int32_t q_type, const voi
                      full_block, window, ctx_len_dev, out_xf, out_xf_kind, nullptr);
 }
 
-int32_t dfl_attn_blocks(dflash_ctx *ctx, const void *q, int32_t q_type, const void *k_cache, const void *vt_cache, int64_t ctx_len,
-                        int32_t n_rows_total, int32_t n_q, int32_t n_kv, int32_t head_dim, int64_t kv_capacity, float scale,
-                        float *out, dflash_stream_t stream, void *out_xf, int out_xf_kind) {
-    if (!ctx) return DFLASH_ERR_INVALID_INPUT;
-    if (n_rows_total < 1) return dfl_fail(ctx, DFLASH_ERR_BAD_SHAPE, "attn_verify: %d rows", n_rows_total);
-    const size_t q_block = static_cast<size_t>(16) * n_q * head_dim;
-    const size_t xf_block = dfl_xf_bytes(static_cast<int64_t>(n_q) * head_dim);
-    const size_t q_el = q_type == DFLASH_TYPE_F16 ? 2 : 4;
-    int32_t done = 0;
-    const int32_t n_blocks = (n_rows_total + 15) / 16;
-    while (done < n_blocks) {
-        // a run: the blocks from `done` on that share its bucket (the split policy is a function of the bucket)
-        const int64_t len0 = ctx_len + 16ll * done;
-        const int64_t bucket = dfl_attn_bucket(len0 + std::min(16, n_rows_total - 16 * done));
-        int32_t run = 1;
-        while (done + run < n_blocks &&
-               dfl_attn_bucket(ctx_len + 16ll * (done + run) + std::min(16, n_rows_total - 16 * (done + run))) == bucket)
-            run++;
-        const int32_t rows = std::min(n_rows_total - 16 * done, 16 * run);
-        int32_t taken = 0;
-        const int32_t rc = attn_rows(ctx, static_cast<const uint8_t *>(q) + done * q_block * q_el, q_type, k_cache, vt_cache, 1, len0, rows,
-                                     n_q, n_kv, head_dim, kv_capacity, scale, out + done * q_block, stream, 0, 0, nullptr,
-                                     out_xf ? static_cast<uint8_t *>(out_xf) + done * xf_block : nullptr, out_xf_kind, &taken);
-        if (rc) return rc;
-        done += taken;
-    }
-    return DFLASH_OK;
-}
-
-static int32_t attn_rows(dflash_ctx *ctx, const void *q, int32_t q_type, const void *k_cache, const void *v_cache,
-                         int32_t v_layout, int64_t ctx_len, int32_t n_rows_total, int32_t n_q, int32_t n_kv, int32_t head_dim,
-                         int64_t kv_capacity, float scale, float *out, dflash_stream_t stream, int32_t full_block,
-                         int64_t window, const int32_t *ctx_len_dev, void *out_xf, int out_xf_kind, int32_t *blocks_done) {
-    int32_t n_blocks = (n_rows_total + 15) / 16;
-    const int32_t n_rows = std::min(16, n_rows_total);  // rows of the first block: what the split policy looks at
-    if (n_blocks > 1 && (v_layout != 1 || ctx_len_dev))
+static int32_t attn_check(dflash_ctx *ctx, const void *q, int32_t q_type, const void *k_cache, const void *v_cache, int32_t v_layout,
+                          int64_t ctx_len, int32_t n_rows_total, int32_t n_q, int32_t n_kv, int32_t head_dim, int64_t kv_capacity,
+                          const float *out, const int32_t *ctx_len_dev, const void *out_xf, int out_xf_kind) {
+    if (n_rows_total > 16 && (v_layout != 1 || ctx_len_dev))
         return dfl_fail(ctx, DFLASH_ERR_UNSUPPORTED, "attn_verify: several blocks need the transposed V cache and a host-side context length");
     if (out_xf && ((n_q * head_dim) % DFL_QK_K || reinterpret_cast<uintptr_t>(out_xf) % 16 ||
                    (out_xf_kind != DFL_XF_Q4K && out_xf_kind != DFL_XF_Q6K)))
@@ -706,15 +862,17 @@ static int32_t attn_rows(dflash_ctx *ctx, const void *q, int32_t q_type, const v
     if (reinterpret_cast<uintptr_t>(q) % 16 || reinterpret_cast<uintptr_t>(k_cache) % 16 ||
         reinterpret_cast<uintptr_t>(v_cache) % 16 || reinterpret_cast<uintptr_t>(out) % 16)
         return dfl_fail(ctx, DFLASH_ERR_ALIGNMENT, "attn_verify: Q, K, V and the output must be 16-byte aligned");
+    return DFLASH_OK;
+}
 
-    hipStream_t st = static_cast<hipStream_t>(stream);
-    const int group = n_q / n_kv;
-    // with ctx_len_dev the context length is read on the device: everything sized here is then sized for the
-    // largest context of the bucket
-    const int64_t bucket = dfl_attn_bucket(ctx_len + n_rows);
-    // (several blocks: sized for the last one, which sees the most keys)
-    int64_t n_pos = ctx_len_dev ? std::min<int64_t>(kv_capacity, 2 * bucket - 1) : ctx_len + n_rows_total;
-
+// How a block's keys are split and its heads shared out, by the bucket of its context length alone.
+struct AttnPolicy {
+    int want;           // splits asked for
+    int64_t min_chunk;  // keys per split at least
+    int hw;             // heads per workgroup, a single block
+    bool ordered;       // the splits' results are merged in order (attn_combine_ordered_kernel, attn_rows_kernel)
+};
+static AttnPolicy attn_policy(const dflash_ctx *ctx, int64_t bucket, int n_kv, int group, int head_dim) {
     // KV splits: enough workgroups to cover the chip once or twice, chunks a multiple of 32 keys and at least
     // min_chunk keys long (a split costs a partial tile per head and row).  The policy is a function of the
     // bucket alone.
@@ -748,7 +906,7 @@ static int32_t attn_rows(dflash_ctx *ctx, const void *q, int32_t q_type, const v
     if (env_hw > 0 && group % env_hw == 0) hw = env_hw;
     if (per_cu_x2 < 1) per_cu_x2 = 1;
     if (min_chunk < 32) min_chunk = 32;
-    int n_parts = group / hw;  // workgroups per (chunk, KV head)
+    const int n_parts = group / hw;
     int want = static_cast<int>(std::max<int64_t>(
         1, (static_cast<int64_t>(per_cu_x2) * ctx->n_cu + 2 * n_kv * n_parts - 1) / (2 * n_kv * n_parts)));
     // (one workgroup per CU at most: beyond half the chip the chunks stay at 512 to 1024 keys - at 64 k of context 256
@@ -757,6 +915,102 @@ static int32_t attn_rows(dflash_ctx *ctx, const void *q, int32_t q_type, const v
     // (at most 256 splits, which two workgroups per CU would ask for as well: the partial tiles' share of the workspace stays what it was)
     if (per_cu_x2 == 1)
         want = std::max<int>(want, static_cast<int>(std::min<int64_t>(256, bucket / (env_long_chunk >= 32 ? env_long_chunk : 512))));
+    // In order where a prefill's workgroup can then keep a merge in registers beside the split at hand (heads of 256 are
+    // two accumulators of 64 a lane, the queries' 32 and the values' 64: one wave per SIMD) and where the merge is no slower
+    // for a block alone (16 rows of 32 heads of 128 inside a graph: 17 to 32 splits 4.6 -> 4.2 us; 64 splits, 16 rows x
+    // 100 k keys, 101.3 -> 102.7 us with the attention).  By the most splits any context of the bucket can have, not the
+    // launch's: the bits must not depend on it.
+    const int64_t max_splits = std::min<int64_t>(want, (2 * bucket - 1 + min_chunk - 1) / min_chunk);
+    return {want, min_chunk, hw, head_dim < 256 && max_splits <= kOrderedSplits};
+}
+
+int32_t dfl_attn_blocks(dflash_ctx *ctx, const void *q, int32_t q_type, const void *k_cache, const void *vt_cache, int64_t ctx_len,
+                        int32_t n_rows_total, int32_t n_q, int32_t n_kv, int32_t head_dim, int64_t kv_capacity, float scale,
+                        float *out, dflash_stream_t stream, void *out_xf, int out_xf_kind) {
+    if (!ctx) return DFLASH_ERR_INVALID_INPUT;
+    if (n_rows_total < 1) return dfl_fail(ctx, DFLASH_ERR_BAD_SHAPE, "attn_verify: %d rows", n_rows_total);
+    const size_t q_block = static_cast<size_t>(16) * n_q * head_dim;
+    const size_t xf_block = dfl_xf_bytes(static_cast<int64_t>(n_q) * head_dim);
+    const size_t q_el = q_type == DFLASH_TYPE_F16 ? 2 : 4;
+    int32_t done = 0;
+    const int32_t n_blocks = (n_rows_total + 15) / 16;
+    if (const int32_t rc_ = attn_check(ctx, q, q_type, k_cache, vt_cache, 1, ctx_len, n_rows_total, n_q, n_kv, head_dim, kv_capacity, out, nullptr,
+                                       out_xf, out_xf_kind))
+        return rc_;
+    const int group = n_q / n_kv;
+    auto bucket_of = [&](int32_t b) { return dfl_attn_bucket(ctx_len + 16ll * b + std::min(16, n_rows_total - 16 * b)); };
+    {
+        // The leading blocks whose splits are merged in order: one launch without partial results, if they are enough
+        // workgroups for it.  A workgroup of it takes its stages one after the other, 1 us each: n_steps of them for the last
+        // block.  The splits spread them over the chip, but a partial result goes out and comes back every two of them, and
+        // there are two launches: 8 us and 1.25 us per stage of a CU's share.  (Six layers of 16 / 8 heads of 128, behind 1900
+        // positions: 512 rows 1178 -> 1035 us this way, 256 rows 782 -> 897; behind none 739 -> 631 and 543 -> 512.)
+        AttnRuns runs = {};
+        int32_t taken = 0;
+        for (int64_t last = -1; taken < n_blocks && q_type == DFLASH_TYPE_F32; taken++) {
+            const int64_t bucket = bucket_of(taken);
+            if (bucket == last) continue;
+            const AttnPolicy p = attn_policy(ctx, bucket, n_kv, group, head_dim);
+            if (!p.ordered || runs.n == kAttnRuns) break;
+            last = bucket;
+            runs.first[runs.n] = taken;
+            runs.want[runs.n] = p.want;
+            runs.min_chunk[runs.n++] = static_cast<int>(p.min_chunk);
+        }
+        int hw = std::min(group, 8);
+        while (group % hw) hw--;
+        const int32_t rows = std::min(n_rows_total, 16 * taken);
+        const int64_t wgs = static_cast<int64_t>(taken) * n_kv * (group / hw), n_steps = (ctx_len + rows + 31) / 32;
+        const int64_t stages = wgs * (ctx_len + rows / 2) / 32;
+        if (taken > 1 && 4 * n_steps * ctx->n_cu <= 32 * ctx->n_cu + 5 * stages) {
+            hipStream_t st = static_cast<hipStream_t>(stream);
+            dfl_timed timer(ctx, st, DFL_T_ATTN);
+            const auto launch = head_dim == 64 ? launch_rows<64> : launch_rows<128>;
+            if (const int32_t rc_ = launch(ctx, dim3(group / hw, n_kv, taken), hw, st, static_cast<const float *>(q), static_cast<const _Float16 *>(k_cache),
+                                           static_cast<const _Float16 *>(vt_cache), ctx_len, rows, n_q, n_kv, kv_capacity, runs, scale, out, out_xf,
+                                           out_xf_kind))
+                return rc_;
+            done = taken;
+        }
+    }
+    while (done < n_blocks) {
+        // a run: the blocks from `done` on that share its bucket (the split policy is a function of the bucket)
+        const int64_t len0 = ctx_len + 16ll * done;
+        int32_t run = 1;
+        while (done + run < n_blocks && bucket_of(done + run) == bucket_of(done)) run++;
+        const int32_t rows = std::min(n_rows_total - 16 * done, 16 * run);
+        int32_t taken = 0;
+        const int32_t rc = attn_rows(ctx, static_cast<const uint8_t *>(q) + done * q_block * q_el, q_type, k_cache, vt_cache, 1, len0, rows,
+                                     n_q, n_kv, head_dim, kv_capacity, scale, out + done * q_block, stream, 0, 0, nullptr,
+                                     out_xf ? static_cast<uint8_t *>(out_xf) + done * xf_block : nullptr, out_xf_kind, &taken);
+        if (rc) return rc;
+        done += taken;
+    }
+    return DFLASH_OK;
+}
+
+static int32_t attn_rows(dflash_ctx *ctx, const void *q, int32_t q_type, const void *k_cache, const void *v_cache,
+                         int32_t v_layout, int64_t ctx_len, int32_t n_rows_total, int32_t n_q, int32_t n_kv, int32_t head_dim,
+                         int64_t kv_capacity, float scale, float *out, dflash_stream_t stream, int32_t full_block,
+                         int64_t window, const int32_t *ctx_len_dev, void *out_xf, int out_xf_kind, int32_t *blocks_done) {
+    int32_t n_blocks = (n_rows_total + 15) / 16;
+    const int32_t n_rows = std::min(16, n_rows_total);  // rows of the first block: what the split policy looks at
+    if (const int32_t rc_ = attn_check(ctx, q, q_type, k_cache, v_cache, v_layout, ctx_len, n_rows_total, n_q, n_kv, head_dim, kv_capacity, out,
+                                       ctx_len_dev, out_xf, out_xf_kind))
+        return rc_;
+
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    const int group = n_q / n_kv;
+    // with ctx_len_dev the context length is read on the device: everything sized here is then sized for the
+    // largest context of the bucket
+    const int64_t bucket = dfl_attn_bucket(ctx_len + n_rows);
+    // (several blocks: sized for the last one, which sees the most keys)
+    int64_t n_pos = ctx_len_dev ? std::min<int64_t>(kv_capacity, 2 * bucket - 1) : ctx_len + n_rows_total;
+
+    const AttnPolicy policy = attn_policy(ctx, bucket, n_kv, group, head_dim);
+    const int want = policy.want;
+    const int64_t min_chunk = policy.min_chunk;
+    int hw = policy.hw, n_parts = group / hw;  // workgroups per (chunk, KV head)
     // Several blocks in one launch cover the chip between them: a workgroup then serves the whole GQA group, so a chunk
     // of keys is staged once instead of group / hw times (a workgroup's LDS ring leaves no room for a second one on
     // its CU, whatever its size).  The split of the keys (want, min_chunk) stays the single block's, and a head is one
@@ -837,6 +1091,14 @@ static int32_t attn_rows(dflash_ctx *ctx, const void *q, int32_t q_type, const v
 #undef DFL_ATTN
     }
     if (rc) return rc;
+    if (policy.ordered) {
+        const auto fn = head_dim == 64 ? attn_combine_ordered_kernel<64> : attn_combine_ordered_kernel<128>;
+        fn<<<dim3(n_q, n_rows, n_blocks), head_dim, 0, st>>>(part_o, part_ml, out, n_rows_total, n_q, ctx_len, ctx_len_dev, want,
+                                                            static_cast<int>(min_chunk), out_xf, out_xf_kind, part_slots,
+                                                            dfl_xf_bytes(static_cast<int64_t>(n_q) * head_dim), n_splits);
+        DFL_HIP_CHECK(ctx, hipGetLastError());
+        return DFLASH_OK;
+    }
     // (more splits than that and the shuffles of the weights cost more than the barriers they replace)
     if (n_splits <= 48) {
         const auto fn = head_dim == 64 ? attn_combine_few_kernel<64> : head_dim == 128 ? attn_combine_few_kernel<128> : attn_combine_few_kernel<256>;
