@@ -20,6 +20,8 @@ SHAPES = {
     "experts": (dfl.ModelConfig(n_layers=2, hidden=2048, n_q=16, n_kv=2, head_dim=256, ffn=0, vocab=2048, n_expert=32, n_expert_used=4,
                                 ffn_expert=768, ffn_shared=768), dfl.synth.Q6_K),
 }
+SHAPES["heads64"] = (dfl.ModelConfig(n_layers=2, hidden=1024, n_q=24, n_kv=2, head_dim=64, ffn=3072, vocab=2048), dfl.synth.Q4_K)
+SHAPES["heads256x5"] = (dfl.ModelConfig(n_layers=2, hidden=1280, n_q=5, n_kv=1, head_dim=256, ffn=3072, vocab=2048), dfl.synth.Q4_K)
 
 
 @pytest.fixture(scope="module")
@@ -30,7 +32,7 @@ def ctx():
 
 
 @pytest.mark.parametrize("rows", [17, 80, 97, 192, 200, 273, 530, 1001])
-@pytest.mark.parametrize("shape", sorted(SHAPES))
+@pytest.mark.parametrize("shape", ["experts", "narrow", "wide"])
 def test_many_row_prefill_equals_block_by_block(ctx, shape, rows):
     cfg, attn_type = SHAPES[shape]
     model = dfl.TargetModel(ctx, cfg, dfl.synth_target_weights_device(cfg, 5, "cuda", attn_type=attn_type))
@@ -38,6 +40,26 @@ def test_many_row_prefill_equals_block_by_block(ctx, shape, rows):
     tokens = np.random.default_rng(rows).integers(0, cfg.vocab, rows).tolist()
     got = many.prefill_blocks(tokens, 0)
     want = torch.cat([one.encode_packed_verify_layer_major(tokens[i:i + 16], i, want_head=False).hidden_capture for i in range(0, rows, 16)])
+    assert torch.equal(got, want)
+    one.close()
+    many.close()
+
+
+@pytest.mark.parametrize("head,rows", [(7, 40), (245, 33), (480, 400), (1000, 530), (1000, 1100)])
+@pytest.mark.parametrize("shape", ["narrow", "experts", "heads64", "heads256x5"])
+def test_continued_prefill_equals_block_by_block(ctx, shape, head, rows):
+    """Behind a context, where the attention takes the keys of many blocks split by split in one workgroup or leaves
+    them to several (by how many workgroups there are), across buckets of context lengths, with a last split and a
+    last stage that are not full, a first position off the stages' raster, and groups of 2, 5, 8 and 12 heads."""
+    cfg, attn_type = SHAPES[shape]
+    model = dfl.TargetModel(ctx, cfg, dfl.synth_target_weights_device(cfg, 5, "cuda", attn_type=attn_type))
+    one, many = dfl.Session(ctx, model, head + rows + 16, [0, 1]), dfl.Session(ctx, model, head + rows + 16, [0, 1])
+    tokens = np.random.default_rng(rows).integers(0, cfg.vocab, head + rows).tolist()
+    for s in (one, many):
+        for i in range(0, head, 16):
+            s.encode_packed_verify_layer_major(tokens[i:min(i + 16, head)], i, want_head=False)
+    got = many.prefill_blocks(tokens[head:], head)
+    want = torch.cat([one.encode_packed_verify_layer_major(tokens[i:i + 16], i, want_head=False).hidden_capture for i in range(head, head + rows, 16)])
     assert torch.equal(got, want)
     one.close()
     many.close()
