@@ -22,6 +22,7 @@
 //    together with the draft rows' tile sums, the decision (written straight to pinned host memory).
 #include "common.h"
 #include "sampler_chain.h"
+#include "accept_select.h"
 #include "accept_wide.h"
 
 #include <cmath>
@@ -36,28 +37,7 @@ constexpr int kChunk = 8192;       // tokens per workgroup of the argmax / top-2
 constexpr int kSelChunk = 16384;
 constexpr int kSelThreads = 1024;  // 8 tokens per thread
 constexpr int kMaxRows = 16;
-constexpr uint64_t kNoKey = ~0ull;
 constexpr int kNoNan = 0x7fffffff;
-
-// Ascending bitonic sort of n (power of two, <= 2 * blockDim.x) keys in LDS.
-__device__ void bitonic_sort(uint64_t *keys, int n) {
-    for (int size = 2; size <= n; size <<= 1) {
-        for (int stride = size >> 1; stride > 0; stride >>= 1) {
-            __syncthreads();
-            for (int i = threadIdx.x; i < n / 2; i += blockDim.x) {
-                int lo = 2 * i - (i & (stride - 1));  // index with the `stride` bit clear
-                int hi = lo + stride;
-                bool up = (lo & size) == 0;
-                uint64_t a = keys[lo], b = keys[hi];
-                if ((a > b) == up) {
-                    keys[lo] = b;
-                    keys[hi] = a;
-                }
-            }
-        }
-    }
-    __syncthreads();
-}
 
 // ------------------------------------------------------------------------------------------
 // argmax_top2: IEEE comparisons, lowest index on ties, second value counts duplicates
@@ -143,50 +123,6 @@ __device__ uint64_t block_min_u64(uint64_t v, uint64_t *sh) {
     return r;
 }
 
-// Ascending sort of one key per lane over the wave (bitonic network of 21 compare-exchange steps between lanes: no
-// LDS arrays, no barriers).
-__device__ __forceinline__ uint64_t wave_sort_u64(uint64_t v) {
-    const int lane = threadIdx.x & 63;
-#pragma unroll
-    for (int size = 2; size <= 64; size <<= 1) {
-#pragma unroll
-        for (int stride = size >> 1; stride > 0; stride >>= 1) {
-            const uint32_t lo = __shfl_xor(static_cast<uint32_t>(v), stride, 64), hi = __shfl_xor(static_cast<uint32_t>(v >> 32), stride, 64);
-            const uint64_t o = (static_cast<uint64_t>(hi) << 32) | lo;
-            const bool lower = (lane & stride) == 0, ascending = (lane & size) == 0;
-            const uint64_t mn = v < o ? v : o, mx = v < o ? o : v;
-            v = (lower == ascending) ? mn : mx;
-        }
-    }
-    return v;
-}
-
-// The k smallest keys, in order, of n_lists <= 64 ascending lists of k keys each (list l at base + l * stride; missing
-// keys are kNoKey, at the end), by ONE wave: lane l holds the head of list l, a step takes the minimum of the heads
-// and advances the list it came from (keys are distinct).  Returns the k-th; with `out`, out[0 .. k) gets them all.
-// (Measured in the selection kernel, k = 20: 3.3 us; every published key searching the sixteen lists instead, spread
-// over all 1024 threads, 5.7 us: the waves of a workgroup share four instruction issuers, and the index arithmetic
-// of 5120 searches costs more than twenty dependent steps of one wave.)
-__device__ __forceinline__ uint64_t wave_merge_lists(const uint64_t *base, int n_lists, int stride, int k, uint64_t *out) {
-    const int lane = threadIdx.x & 63;
-    const bool own = lane < n_lists;
-    const uint64_t *list = base + (own ? lane : 0) * stride;
-    int pos = 0;
-    uint64_t head = own ? list[0] : kNoKey;
-    uint64_t next = (own && k > 1) ? list[1] : kNoKey;  // fetched one step ahead of its use
-    uint64_t m = kNoKey;
-    for (int step = 0; step < k; step++) {
-        m = wave_min_u64(head);
-        if (out && lane == 0) out[step] = m;
-        if (own && head == m && m != kNoKey) {
-            head = next;
-            pos++;
-            next = pos + 1 < k ? list[pos + 1] : kNoKey;
-        }
-    }
-    return m;
-}
-
 // below[j] = number of keys below x[j] in the ascending list of 1 <= n <= kMaxK keys at base + off[j], four binary
 // searches in lockstep: a probe is an LDS read the next one depends on, and a thread that runs its searches one
 // after the other spends its time waiting for them.  step0 = the largest power of two <= n.
@@ -209,19 +145,18 @@ __device__ __forceinline__ void count_below4(const uint64_t *base, const int (&o
 
 // K == 1 fast path is the greedy / draft-max case: only the minimum key is needed.
 //
-// K > 1, without a sort over the workgroup (a bitonic network in LDS is one workgroup barrier per step, 91 steps
-// here): every wave sorts its 64 per-thread bests between its lanes and publishes the first k; the k-th best of all
-// 1024 per-thread bests (it bounds every winner of the chunk) is the k-th key of the merge of the sixteen published
-// lists, which wave 0 runs; the at most 16 k elements at or below that bound are then ranked by counting the
-// candidates below each, and a candidate of rank r < k is output r.  Keys are distinct (the token id is in the low
-// bits), so ranks are too.
+// K > 1, without a sort: the k-th best of the 1024 per-thread bests bounds every winner of the chunk (block_kth); the at
+// most 16 k elements at or below that bound are then ranked by counting the candidates below each, and a candidate of
+// rank r < k is output r.  Keys are distinct (the token id is in the low bits), so ranks are too.  (The bound by sorting
+// every wave's bests between its lanes and merging the sixteen lists was 21 rounds of shuffles through LDS and k
+// dependent steps: 16.8 -> 14.6 us for 31 rows of 151936, k = 20 on 16 of them.)
 __device__ __forceinline__ void select_chunk_body(const float *__restrict__ logits, int64_t vocab, int64_t stride, int k,
                                                   ChunkOut *__restrict__ out, bool nan_is_candidate, int row) {
-    __shared__ uint64_t sk[kSelThreads];  // k == 1: scratch of the minimum; else [16 waves][kMaxK] published bests
-    __shared__ uint64_t cand[(kSelChunk / kSelThreads) * kMaxK];
+    constexpr int kMaxCand = (kSelChunk / kSelThreads) * kMaxK;
+    __shared__ uint64_t cand[kMaxCand];
     __shared__ uint64_t outk[kMaxK];
-    __shared__ uint64_t tau_sh;
-    __shared__ int rank_sh[kSelThreads];  // [16 waves][kMaxK] published bests, then the candidates (at most as many)
+    __shared__ KthShared<kSelThreads> kth;
+    __shared__ int rank_sh[kMaxCand];
     __shared__ int cnt;
     __shared__ int nan_sh;
     const int chunk = blockIdx.x, tid = threadIdx.x;
@@ -253,33 +188,18 @@ __device__ __forceinline__ void select_chunk_body(const float *__restrict__ logi
     if (nan_first != kNoNan) atomicMin(&nan_sh, nan_first);
     ChunkOut *o = out + (row * gridDim.x + chunk);
     if (k == 1) {
-        uint64_t m = block_min_u64(best, sk);
+        uint64_t m = block_min_u64(best, outk);
         if (tid == 0) {
             o->keys[0] = m;
             o->nan_first = nan_sh;
         }
         return;
     }
-    // k-th best of the per-thread bests bounds every winner of the chunk
-    const int lane = tid & 63, wave = tid >> 6;
-    const uint64_t sorted = wave_sort_u64(best);
-    if (lane < k) sk[wave * kMaxK + lane] = sorted;
     if (tid < kMaxK) outk[tid] = kNoKey;
     rank_sh[tid] = 0;
-    __syncthreads();
-    // the k-th best of the sixteen published lists: wave 0 merges them (fewer than k keys in all: kNoKey, and every
-    // key of the chunk is a candidate)
-    if (wave == 0) {
-        const uint64_t kth = wave_merge_lists(sk, kSelThreads / 64, kMaxK, k, nullptr);
-        if (lane == 0) tau_sh = kth;
-    }
-    __syncthreads();
-    const uint64_t tau = tau_sh;
-    if (best <= tau && best != kNoKey) {
-#pragma unroll
-        for (int j = 0; j < kSelChunk / kSelThreads; j++)
-            if (keys[j] <= tau && keys[j] != kNoKey) cand[atomicAdd(&cnt, 1)] = keys[j];
-    }
+    const uint64_t mine[1] = {best};
+    const uint64_t bound = block_kth<1>(mine, kNoKey - 1, k, kth);
+    compact_keys(keys, bound, cand, kMaxCand, &cnt);
     __syncthreads();
     const int n_cand = cnt;  // <= 16 k <= kSelThreads
     if (n_cand > 0) {
@@ -446,13 +366,25 @@ __global__ void __launch_bounds__(kSelThreads)
 __global__ void __launch_bounds__(kSelThreads)
     top16_merge_kernel(const ChunkOut *__restrict__ chunks, int n_chunks, int32_t *__restrict__ ids,
                        float *__restrict__ vals) {
-    __shared__ uint64_t sk[2 * kSelThreads];
+    __shared__ uint64_t lists[2 * kSelThreads], sk[16];
     const int row = blockIdx.x, tid = threadIdx.x;
-    const int n_in = n_chunks * 16;
-    int n_sort = 16;
-    while (n_sort < n_in) n_sort <<= 1;
-    for (int i = tid; i < n_sort; i += kSelThreads) sk[i] = i < n_in ? chunks[row * n_chunks + i / 16].keys[i % 16] : kNoKey;
-    bitonic_sort(sk, n_sort);
+    const int n_in = n_chunks * 16;  // <= 2048, checked on the host
+    for (int i = tid; i < n_in; i += kSelThreads) lists[i] = chunks[row * n_chunks + i / 16].keys[i % 16];
+    if (tid < 16) sk[tid] = kNoKey;
+    __syncthreads();
+    // a key's rank by counting the keys below it, sixteen lanes a key: a chunk's list each, sixteen chunks a round
+    for (int i0 = 0; i0 < n_in; i0 += kSelThreads / 16) {
+        const int i = i0 + (tid >> 4);
+        const uint64_t key = i < n_in ? lists[i] : 0;
+        int below = 0;
+        for (int c = tid & 15; c < n_chunks; c += 16) {
+#pragma unroll
+            for (int j = 0; j < 16; j++) below += lists[16 * c + j] < key;
+        }
+        for (int off = 8; off > 0; off >>= 1) below += __shfl_xor(below, off, 64);
+        if (i < n_in && (tid & 15) == 0 && key != kNoKey && below < 16) sk[below] = key;
+    }
+    __syncthreads();
     if (tid < 16) {
         uint64_t key = sk[tid];
         ids[row * 16 + tid] = key == kNoKey ? -1 : key_token(key);
@@ -726,13 +658,17 @@ __device__ void residual_pick(const DecideArgs &a, const RowDist *rows, int row,
 
 // Thread r evaluates row r (all rows at once); thread 0 then walks the outcomes in order exactly as the serial
 // loop of accept.rs:147-183 does: rows behind the first rejection, stop or error are never looked at.
-__global__ void __launch_bounds__(64) decide_kernel(DecideArgs a, dflash_accept_decision *__restrict__ out) {
+// What it spends its time on is the way to its data and its own code: a single wave made sixty requests of tile sums,
+// each with its own branch, out of 16 KB of instructions that nothing has fetched before.  Eight waves ask for
+// everything in eight requests each; the first one decides (16.3 -> 10.2 us for a 16-row block with dense proposals).
+constexpr int kDecThreads = 512;
+__global__ void __launch_bounds__(kDecThreads) decide_kernel(DecideArgs a, dflash_accept_decision *__restrict__ out) {
     constexpr int kStage = 256;  // tile sums per row and round
     __shared__ double p_total[kMaxRows];
     __shared__ RowOutcome outcome[kMaxRows + 1];
     // the rows' distributions are walked element by element: they are copied to LDS once, coalesced
     __shared__ RowDist rows_sh[kMaxRows];
-    __shared__ double staged[kMaxRows][kStage];
+    __shared__ double staged[kMaxRows][kStage + 1];  // (a row per lane is read: the lanes' banks differ)
     __shared__ float draft_tok_logit[kMaxRows];
     __shared__ float resid_logit[kMaxRows][kMaxK];
     static_assert(sizeof(RowDist) % 8 == 0, "copied as double words");
@@ -743,47 +679,40 @@ __global__ void __launch_bounds__(64) decide_kernel(DecideArgs a, dflash_accept_
     // trip: everything whose address is known is requested before anything is waited for (the first round of tile
     // sums, each draft row's logit of its own draft token, the rows), the candidates' draft logits as soon as the
     // rows are there, and the arithmetic runs on LDS copies.
-    double tsum[kMaxRows - 1][kStage / 64];
+    constexpr int kPerRow = kDecThreads / kStage;  // rows a round of requests covers
+    auto tile_sum = [&](int r, int t) { return r < n_drafts && t < a.n_tiles ? a.tile_sums[r * a.n_tiles + t] : 0.0; };
+    double tsum[kMaxRows / kPerRow];
     float my_logit = 0.0f;
     if (dense) {
 #pragma unroll
-        for (int r = 0; r < kMaxRows - 1; r++)
-#pragma unroll
-            for (int u = 0; u < kStage / 64; u++) {
-                const int t = u * 64 + tid;
-                tsum[r][u] = (r < n_drafts && t < a.n_tiles) ? a.tile_sums[r * a.n_tiles + t] : 0.0;
-            }
+        for (int j = 0; j < kMaxRows / kPerRow; j++) tsum[j] = tile_sum(kPerRow * j + tid / kStage, tid % kStage);
         if (tid < n_drafts) my_logit = a.draft[tid * a.draft_stride + a.verified[tid + 1]];
     }
     {
         const uint64_t *src = reinterpret_cast<const uint64_t *>(a.rows);
         uint64_t *dst = reinterpret_cast<uint64_t *>(rows_sh);
         const int n_words = a.n_tokens * static_cast<int>(sizeof(RowDist) / 8);
-        for (int base = 0; base < n_words; base += 64 * 8) {
-            uint64_t v[8];
+        constexpr int kRounds = (kMaxRows * static_cast<int>(sizeof(RowDist) / 8) + kDecThreads - 1) / kDecThreads;
+        uint64_t v[kRounds];
 #pragma unroll
-            for (int u = 0; u < 8; u++) v[u] = base + u * 64 + tid < n_words ? src[base + u * 64 + tid] : 0;
+        for (int u = 0; u < kRounds; u++) v[u] = src[min(u * kDecThreads + tid, n_words - 1)];
 #pragma unroll
-            for (int u = 0; u < 8; u++)
-                if (base + u * 64 + tid < n_words) dst[base + u * 64 + tid] = v[u];
-        }
+        for (int u = 0; u < kRounds; u++)
+            if (u * kDecThreads + tid < n_words) dst[u * kDecThreads + tid] = v[u];
     }
     if (dense) {
 #pragma unroll
-        for (int r = 0; r < kMaxRows - 1; r++)
-#pragma unroll
-            for (int u = 0; u < kStage / 64; u++) staged[r][u * 64 + tid] = tsum[r][u];
+        for (int j = 0; j < kMaxRows / kPerRow; j++) staged[kPerRow * j + tid / kStage][tid % kStage] = tsum[j];
         if (tid < n_drafts) draft_tok_logit[tid] = my_logit;
     }
     __syncthreads();
     const bool prefetched = dense && !a.wide_keys;
     if (prefetched) {
-        float v[kMaxRows - 1];
 #pragma unroll
-        for (int r = 0; r < kMaxRows - 1; r++)
-            v[r] = (r < n_drafts && tid < rows_sh[r].n_keep) ? a.draft[r * a.draft_stride + rows_sh[r].tokens[tid]] : 0.0f;
-#pragma unroll
-        for (int r = 0; r < kMaxRows - 1; r++) resid_logit[r][tid] = v[r];
+        for (int j = 0; j < kMaxRows / (kDecThreads / 64); j++) {
+            const int r = kDecThreads / 64 * j + (tid >> 6), i = tid & 63;
+            resid_logit[r][i] = (r < n_drafts && i < rows_sh[r].n_keep) ? a.draft[r * a.draft_stride + rows_sh[r].tokens[i]] : 0.0f;
+        }
     }
     if (dense) {
         // P = sequential sum of a row's tile sums, in tile order, by thread r from the LDS copies
@@ -791,16 +720,19 @@ __global__ void __launch_bounds__(64) decide_kernel(DecideArgs a, dflash_accept_
         for (int t0 = 0; t0 < a.n_tiles; t0 += kStage) {
             if (t0 > 0) {  // further rounds (vocabularies above 262144 tokens)
                 __syncthreads();
-                for (int r = 0; r < n_drafts; r++)
-                    for (int u = 0; u < kStage / 64; u++) {
-                        const int t = t0 + u * 64 + tid;
-                        staged[r][u * 64 + tid] = t < a.n_tiles ? a.tile_sums[r * a.n_tiles + t] : 0.0;
-                    }
+                for (int r = tid / kStage; r < n_drafts; r += kPerRow) staged[r][tid % kStage] = tile_sum(r, t0 + tid % kStage);
                 __syncthreads();
             }
             if (tid < n_drafts) {
+                // (sixteen read ahead of their additions; past the last tile is +0, which changes no sum of exponentials)
                 const int n = min(kStage, a.n_tiles - t0);
-                for (int i = 0; i < n; i++) P += staged[tid][i];
+                for (int i = 0; i < n; i += 16) {
+                    double v[16];
+#pragma unroll
+                    for (int j = 0; j < 16; j++) v[j] = staged[tid][i + j];
+#pragma unroll
+                    for (int j = 0; j < 16; j++) P += v[j];
+                }
             }
         }
         if (tid < n_drafts) p_total[tid] = P;
@@ -808,7 +740,8 @@ __global__ void __launch_bounds__(64) decide_kernel(DecideArgs a, dflash_accept_
     __syncthreads();
     if (tid <= n_drafts) outcome[tid] = decide_row(a, rows_sh, tid, p_total, draft_tok_logit);
     __syncthreads();
-    // The walk, by every lane alike (the workgroup is one wave; everything it reads is uniform): at the row it stops
+    if (tid >= 64) return;
+    // The walk, by every lane alike (one wave; everything it reads is uniform): at the row it stops
     // at, a rejected draft's correction token is drawn by the whole wave.  The decision is put together in LDS and
     // leaves as one coalesced store: `out` may be host memory, where every separate store is a transaction over the
     // bus.
@@ -866,11 +799,12 @@ __global__ void __launch_bounds__(64) decide_kernel(DecideArgs a, dflash_accept_
             d.draws_used = draws;
         }
     }
-    __syncthreads();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
     {
         const uint32_t *src = reinterpret_cast<const uint32_t *>(&d_sh);
         uint32_t *dst = reinterpret_cast<uint32_t *>(out);
-        for (int i = threadIdx.x; i < static_cast<int>(sizeof(dflash_accept_decision) / 4); i += blockDim.x) dst[i] = src[i];
+        for (int i = threadIdx.x; i < static_cast<int>(sizeof(dflash_accept_decision) / 4); i += 64) dst[i] = src[i];
     }
 }
 
@@ -1199,7 +1133,7 @@ int32_t dflash_accept_prefix(dflash_ctx *ctx, const int32_t *verified, int32_t n
         void *pinned_dev = nullptr;
         const bool direct = ctx->pinned && hipHostGetDevicePointer(&pinned_dev, ctx->pinned, 0) == hipSuccess && pinned_dev;
         if (!direct) (void)hipGetLastError();
-        decide_kernel<<<1, 64, 0, st>>>(a, direct ? static_cast<dflash_accept_decision *>(pinned_dev) : d_out);
+        decide_kernel<<<1, kDecThreads, 0, st>>>(a, direct ? static_cast<dflash_accept_decision *>(pinned_dev) : d_out);
         DFL_HIP_CHECK(ctx, hipGetLastError());
         if (!direct) DFL_HIP_CHECK(ctx, hipMemcpyAsync(ctx->pinned, d_out, sizeof(*out), hipMemcpyDeviceToHost, st));
     }

@@ -1,0 +1,102 @@
+// Selection of the k best of a workgroup's ordering keys without sorting them: shared by the chunk selections of
+// accept.hip (k <= 64) and accept_wide.hip (k <= 1024).
+#pragma once
+
+#include "sampler_chain.h"
+
+namespace {
+
+constexpr uint64_t kNoKey = ~0ull;  // no key: a NaN's logit bits above the largest token
+
+template <int THREADS>
+struct KthShared {
+    int hist[3][256];
+    uint64_t lo[THREADS / 64], hi[THREADS / 64];
+    int n[THREADS / 64];
+};
+
+// A bound B <= limit such that exactly k of the workgroup's keys are <= B; limit if no more than k are <= limit.
+// Digit by digit from the first bit in which the keys differ (most share sign and most of the exponent: a digit
+// above it would put every key on one counter), and no further than until a digit's counts end at k.  Keys are
+// distinct, so the last digit ends there at the latest.  One barrier per digit: every wave adds up the counters by
+// itself, and of three sets of counters one is counted in, one may still be read, one is cleared for the next digit.
+template <int PER, int THREADS>
+__device__ uint64_t block_kth(const uint64_t (&key)[PER], uint64_t limit, int k, KthShared<THREADS> &sh) {
+    constexpr int kWaves = THREADS / 64;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    uint64_t lo = kNoKey, hi = 0;
+    int n = 0;
+#pragma unroll
+    for (int j = 0; j < PER; j++) {
+        const bool in = key[j] <= limit;
+        lo = in && key[j] < lo ? key[j] : lo;
+        hi = in && key[j] > hi ? key[j] : hi;
+        n += __popcll(__builtin_amdgcn_ballot_w64(in));
+    }
+    lo = wave_min_u64(lo);
+    hi = ~wave_min_u64(~hi);
+    if (lane == 0) {
+        sh.lo[wave] = lo;
+        sh.hi[wave] = hi;
+        sh.n[wave] = n;
+    }
+    if (tid < 256) sh.hist[0][tid] = 0;
+    __syncthreads();
+    lo = wave_min_u64(lane < kWaves ? sh.lo[lane] : kNoKey);
+    hi = ~wave_min_u64(lane < kWaves ? ~sh.hi[lane] : kNoKey);
+    n = __builtin_amdgcn_readlane(wave_scan_i32(lane < kWaves ? sh.n[lane] : 0), 63);
+    if (n <= k) return limit;
+    int shift = 64 - __clzll(static_cast<long long>(lo ^ hi));  // 1 .. 64: n > k >= 1 distinct keys
+    uint64_t prefix = (lo >> 1) >> (shift - 1);
+    for (int set = 0;; set = set == 2 ? 0 : set + 1) {
+        const int digit = shift > 8 ? shift - 8 : 0, mask = (1 << (shift - digit)) - 1;
+#pragma unroll
+        for (int j = 0; j < PER; j++)
+            if (key[j] <= limit && ((key[j] >> 1) >> (shift - 1)) == prefix) atomicAdd(&sh.hist[set][static_cast<int>(key[j] >> digit) & mask], 1);
+        if (tid < 256) sh.hist[set == 2 ? 0 : set + 1][tid] = 0;
+        __syncthreads();
+        const int4 c = *reinterpret_cast<const int4 *>(&sh.hist[set][4 * lane]);
+        const int upto = wave_scan_i32(c.x + c.y + c.z + c.w);
+        int below = upto - (c.x + c.y + c.z + c.w), bin = 4 * lane, count = c.x;
+        const bool here = below < k && k <= upto;  // in one lane
+        if (below + count < k) below += count, bin++, count = c.y;
+        if (bin == 4 * lane + 1 && below + count < k) below += count, bin++, count = c.z;
+        if (bin == 4 * lane + 2 && below + count < k) below += count, bin++, count = c.w;
+        const int from = __builtin_ctzll(__builtin_amdgcn_ballot_w64(here));
+        k -= __builtin_amdgcn_readlane(below, from);
+        prefix = (prefix << (shift - digit)) | static_cast<uint64_t>(__builtin_amdgcn_readlane(bin, from));
+        shift = digit;
+        if (__builtin_amdgcn_readlane(count, from) == k) return (prefix << shift) | ((uint64_t(1) << shift) - 1);
+    }
+}
+
+template <int PER>
+__device__ __forceinline__ uint64_t thread_best(const uint64_t (&key)[PER]) {
+    uint64_t best = kNoKey;
+#pragma unroll
+    for (int j = 0; j < PER; j++) best = key[j] < best ? key[j] : best;
+    return best;
+}
+
+// The workgroup's keys <= bound to the slots [0, cap) of out, in no order, as far as they fit; *cnt (0 before) becomes
+// their number.  A wave asks for its slots with one addition.
+template <int PER>
+__device__ void compact_keys(const uint64_t (&key)[PER], uint64_t bound, uint64_t *out, int cap, int *cnt) {
+    const int lane = threadIdx.x & 63;
+    int n = 0;
+#pragma unroll
+    for (int j = 0; j < PER; j++) n += __popcll(__builtin_amdgcn_ballot_w64(key[j] <= bound));
+    if (n == 0) return;
+    int at = 0;
+    if (lane == 0) at = atomicAdd(cnt, n);
+    at = __builtin_amdgcn_readfirstlane(at);
+#pragma unroll
+    for (int j = 0; j < PER; j++) {
+        const uint64_t m = __builtin_amdgcn_ballot_w64(key[j] <= bound);
+        const int slot = at + __popcll(m & ((uint64_t(1) << lane) - 1));
+        if (key[j] <= bound && slot < cap) out[slot] = key[j];
+        at += __popcll(m);
+    }
+}
+
+}  // namespace

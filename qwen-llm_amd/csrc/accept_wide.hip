@@ -30,6 +30,7 @@
 
 #include <rocprim/device/device_radix_sort.hpp>
 
+#include "accept_select.h"
 #include "accept_wide.h"
 
 namespace {
@@ -63,101 +64,9 @@ constexpr int kPickThreads = 512;
 constexpr int kPickChunk = 8192;  // tokens per workgroup: 16 rows of 151936 are 304 workgroups, one round of two per CU
 constexpr int kPickMax = 1024;    // threads of the row kernel: a candidate each
 constexpr int kPickSlots = 16 * kPickMax;  // chunk winners of a row that its workgroup holds in registers
-constexpr uint64_t kNoKeyW = ~0ull;  // (a NaN's logit bits: no key has them)
-
-template <int THREADS>
-struct KthShared {
-    int hist[3][256];
-    uint64_t lo[THREADS / 64], hi[THREADS / 64];
-    int n[THREADS / 64];
-};
-
-// A bound B <= limit such that exactly k of the workgroup's keys are <= B; limit if no more than k are <= limit.
-// Digit by digit from the first bit in which the keys differ (they share row, sign and most of the exponent: a digit
-// above it would put every key on one counter), and no further than until a digit's counts end at k.  Keys are
-// distinct, so the last digit ends there at the latest.  One barrier per digit: every wave adds up the counters by
-// itself, and of three sets of counters one is counted in, one may still be read, one is cleared for the next digit.
-template <int PER, int THREADS>
-__device__ uint64_t block_kth(const uint64_t (&key)[PER], uint64_t limit, int k, KthShared<THREADS> &sh) {
-    constexpr int kWaves = THREADS / 64;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    uint64_t lo = kNoKeyW, hi = 0;
-    int n = 0;
-#pragma unroll
-    for (int j = 0; j < PER; j++) {
-        const bool in = key[j] <= limit;
-        lo = in && key[j] < lo ? key[j] : lo;
-        hi = in && key[j] > hi ? key[j] : hi;
-        n += __popcll(__builtin_amdgcn_ballot_w64(in));
-    }
-    lo = wave_min_u64(lo);
-    hi = ~wave_min_u64(~hi);
-    if (lane == 0) {
-        sh.lo[wave] = lo;
-        sh.hi[wave] = hi;
-        sh.n[wave] = n;
-    }
-    if (tid < 256) sh.hist[0][tid] = 0;
-    __syncthreads();
-    lo = wave_min_u64(lane < kWaves ? sh.lo[lane] : kNoKeyW);
-    hi = ~wave_min_u64(lane < kWaves ? ~sh.hi[lane] : kNoKeyW);
-    n = __builtin_amdgcn_readlane(wave_scan_i32(lane < kWaves ? sh.n[lane] : 0), 63);
-    if (n <= k) return limit;
-    int shift = 64 - __clzll(static_cast<long long>(lo ^ hi));  // (n > k >= 1 distinct keys; at most 60, they share the row)
-    uint64_t prefix = lo >> shift;
-    for (int set = 0;; set = set == 2 ? 0 : set + 1) {
-        const int digit = shift > 8 ? shift - 8 : 0, mask = (1 << (shift - digit)) - 1;
-#pragma unroll
-        for (int j = 0; j < PER; j++)
-            if (key[j] <= limit && (key[j] >> shift) == prefix) atomicAdd(&sh.hist[set][static_cast<int>(key[j] >> digit) & mask], 1);
-        if (tid < 256) sh.hist[set == 2 ? 0 : set + 1][tid] = 0;
-        __syncthreads();
-        const int4 c = *reinterpret_cast<const int4 *>(&sh.hist[set][4 * lane]);
-        const int upto = wave_scan_i32(c.x + c.y + c.z + c.w);
-        int below = upto - (c.x + c.y + c.z + c.w), bin = 4 * lane, count = c.x;
-        const bool here = below < k && k <= upto;  // in one lane
-        if (below + count < k) below += count, bin++, count = c.y;
-        if (bin == 4 * lane + 1 && below + count < k) below += count, bin++, count = c.z;
-        if (bin == 4 * lane + 2 && below + count < k) below += count, bin++, count = c.w;
-        const int from = __builtin_ctzll(__builtin_amdgcn_ballot_w64(here));
-        k -= __builtin_amdgcn_readlane(below, from);
-        prefix = (prefix << (shift - digit)) | static_cast<uint64_t>(__builtin_amdgcn_readlane(bin, from));
-        shift = digit;
-        if (__builtin_amdgcn_readlane(count, from) == k) return (prefix << shift) | ((uint64_t(1) << shift) - 1);
-    }
-}
-
-template <int PER>
-__device__ __forceinline__ uint64_t thread_best(const uint64_t (&key)[PER]) {
-    uint64_t best = kNoKeyW;
-#pragma unroll
-    for (int j = 0; j < PER; j++) best = key[j] < best ? key[j] : best;
-    return best;
-}
-
-// The workgroup's keys <= bound to the slots [0, cap) of out, in no order, as far as they fit; *cnt (0 before) becomes
-// their number.  A wave asks for its slots with one addition.
-template <int PER>
-__device__ void compact_keys(const uint64_t (&key)[PER], uint64_t bound, uint64_t *out, int cap, int *cnt) {
-    const int lane = threadIdx.x & 63;
-    int n = 0;
-#pragma unroll
-    for (int j = 0; j < PER; j++) n += __popcll(__builtin_amdgcn_ballot_w64(key[j] <= bound));
-    if (n == 0) return;
-    int at = 0;
-    if (lane == 0) at = atomicAdd(cnt, n);
-    at = __builtin_amdgcn_readfirstlane(at);
-#pragma unroll
-    for (int j = 0; j < PER; j++) {
-        const uint64_t m = __builtin_amdgcn_ballot_w64(key[j] <= bound);
-        const int slot = at + __popcll(m & ((uint64_t(1) << lane) - 1));
-        if (key[j] <= bound && slot < cap) out[slot] = key[j];
-        at += __popcll(m);
-    }
-}
 
 // A chunk's winners, the k best keys and at most cap >= k, in no order, at out[(row * n_chunks + chunk) * cap], filled up
-// with kNoKeyW; the chunk's lowest NaN token.  The k-th best of the per-thread bests bounds every winner, and what is
+// with kNoKey; the chunk's lowest NaN token.  The k-th best of the per-thread bests bounds every winner, and what is
 // below it usually fits the slots (k = 200: about 250 keys); only where it does not, the k best of all are looked for.
 __global__ void __launch_bounds__(kPickThreads)
     pick_chunk_kernel(const float *__restrict__ logits, int64_t vocab, int64_t stride, int k, int cap, uint64_t *__restrict__ out,
@@ -184,10 +93,10 @@ __global__ void __launch_bounds__(kPickThreads)
         if (i < vocab && nan) atomicMin(&nan_sh, static_cast<int32_t>(i));
         key[j] = i < vocab && !nan ? (static_cast<uint64_t>(row) << 60) |
                                          (static_cast<uint64_t>(desc_bits(__float_as_uint(v[j]))) << kWideTokenBits) | static_cast<uint64_t>(i)
-                                   : kNoKeyW;
+                                   : kNoKey;
     }
     const uint64_t best[1] = {thread_best(key)};
-    uint64_t bound = block_kth<1>(best, kNoKeyW - 1, k, sh);
+    uint64_t bound = block_kth<1>(best, kNoKey - 1, k, sh);
     const int64_t at = static_cast<int64_t>(row) * gridDim.x + blockIdx.x;
     uint64_t *o = out + at * cap;
     compact_keys(key, bound, o, cap, &cnt[0]);
@@ -198,7 +107,7 @@ __global__ void __launch_bounds__(kPickThreads)
         compact_keys(key, bound, o, cap, &cnt[1]);
         n = k;
     }
-    for (int i = n + tid; i < cap; i += kPickThreads) o[i] = kNoKeyW;
+    for (int i = n + tid; i < cap; i += kPickThreads) o[i] = kNoKey;
     if (tid == 0) nan_first[at] = nan_sh;
 }
 
@@ -221,7 +130,7 @@ __global__ void __launch_bounds__(kPickMax)
     for (int j = 0; j < PER; j++) {
         const int i = j * kPickMax + tid;
         const uint64_t got = chunk_keys[static_cast<int64_t>(row) * n_in + (i < n_in ? i : 0)];
-        key[j] = i < n_in ? got : kNoKeyW;
+        key[j] = i < n_in ? got : kNoKey;
     }
     const int nan = tid < n_chunks ? chunk_nan[row * n_chunks + tid] : kNoNanW;  // (n_chunks <= kPickSlots / k < kPickMax)
     rank_sh[tid] = 0;
@@ -232,7 +141,7 @@ __global__ void __launch_bounds__(kPickMax)
     __syncthreads();
     if (nan != kNoNanW) atomicMin(&nan_sh, nan);
     const uint64_t best[1] = {thread_best(key)};
-    uint64_t bound = block_kth<1>(best, kNoKeyW - 1, k, sh);  // (its barriers are behind the minimum)
+    uint64_t bound = block_kth<1>(best, kNoKey - 1, k, sh);  // (its barriers are behind the minimum)
     auto finish = [&](int32_t err, int64_t err_index, int n_keep, double total, int32_t pick, double draft_weight) {
         if (tid == 0) {
             d->n_keep = n_keep;
