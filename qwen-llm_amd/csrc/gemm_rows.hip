@@ -17,7 +17,7 @@
 // Measured for 2032 rows (four blocks per pass through the 16-row kernels before): 5120 -> 2 x 17408 with SwiGLU 795 us
 // (0.92 PFLOP/s; 30 us per block before), 17408 -> 5120 428 us (0.85), 5120 -> 6144 226 us and 4096 -> 5120 175 us (0.57
 // and 0.49: their twin MFMAs, which the block path's bits ask for, are as many again); a 64-layer prompt of 1000 rows
-// 72.6 ms against 292.
+// 72.6 ms against 292 (65 with the attention's splits merged in registers).
 // The experts' tiles (a list, mostly one to four row blocks) take workgroups of half the columns, two of them on a CU:
 // each waits for its own weights while the other computes (2 - 4 % of a prompt of 33 - 130 rows).
 //
