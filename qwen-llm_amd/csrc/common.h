@@ -365,7 +365,8 @@ int32_t dfl_attn_block(dflash_ctx *ctx, const void *q, int32_t q_type, const voi
 // dfl_attn_block would run it alone at its own context length (ctx_len + 16 b): the same split of the keys, so the same
 // bits.  The leading blocks whose splits are merged in order go out as one launch that needs no workspace where they are
 // enough workgroups for it; else blocks whose context lengths fall in the same bucket go out as one launch pair (as many
-// of them as the workspace holds partial tiles for).
+// of them as the workspace holds partial tiles for).  Transposed V cache; block b's rows at q + 16 b rows, out likewise,
+// out_xf + b * dfl_xf_bytes(n_q * head_dim).  The K/V rows of all the blocks are in the cache already.
 int32_t dfl_attn_blocks(dflash_ctx *ctx, const void *q, int32_t q_type, const void *k_cache, const void *vt_cache, int64_t ctx_len,
                         int32_t n_rows_total, int32_t n_q, int32_t n_kv, int32_t head_dim, int64_t kv_capacity, float scale,
                         float *out, dflash_stream_t stream, void *out_xf, int out_xf_kind);
