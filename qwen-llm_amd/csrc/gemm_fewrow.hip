@@ -437,6 +437,20 @@ __device__ __forceinline__ void q4k_wait_vm(int v) {
     }
 }
 
+// The same where v is at most ten (a ring of three stages, three loads each, and a refill's activations): a shorter search.
+__device__ __forceinline__ void q4k_wait_vm_few(int v) {
+    switch (v) {
+#define DFL_VM(n)                                      \
+    case n:                                            \
+        __builtin_amdgcn_s_waitcnt(q4k_vmcnt(n));      \
+        break;
+        DFL_VM(1) DFL_VM(2) DFL_VM(3) DFL_VM(4) DFL_VM(5) DFL_VM(6) DFL_VM(7) DFL_VM(8) DFL_VM(9) DFL_VM(10)
+#undef DFL_VM
+    default:
+        __builtin_amdgcn_s_waitcnt(q4k_vmcnt(0));
+    }
+}
+
 // Ends a tile group's segment: Y directly if this workgroup covered the group's whole K, else a
 // partial tile for the reduce kernel (slot 0: the range's first group, slot 1: its last).
 template <int kWaves>
@@ -889,13 +903,8 @@ constexpr size_t kSlabLdsBytes = static_cast<size_t>(kSlabStages) * kSlabStageBy
 static_assert(kSlabLdsBytes <= 160 * 1024, "one workgroup per CU, all of its LDS");
 
 // One stage of a wave's tile: 8 MFMAs for the scaled nibbles, one for the minima.
-__device__ __forceinline__ void q4k_slab_compute(const u32x4_t *blk, const half8_t *a, const half4_t *twin, int g, uint32_t sc_sel,
-                                                 Q4KMagic magic, float4_t &acc) {
-    const u32x4_t hdr = blk[0], q0 = blk[1 + 2 * g], q1 = blk[2 + 2 * g];
-    half8_t af[8];
-#pragma unroll
-    for (int t = 0; t < 8; t++) af[t] = a[t * 64];
-    const half4_t tw = *twin;
+__device__ __forceinline__ void q4k_stage(u32x4_t hdr, u32x4_t q0, u32x4_t q1, const half8_t *af, half8_t a_min, int g, uint32_t sc_sel,
+                                          Q4KMagic magic, float4_t &acc, bool over) {
     // scales and minima of sub-blocks 2g and 2g+1 (see q4k_compute)
     const uint32_t upper = 0u - static_cast<uint32_t>(g >> 1);
     const uint32_t sc_lo = hdr.y & 0x3F3F3F3Fu, sc_hi = (hdr.w & 0x0F0F0F0Fu) | ((hdr.y >> 2) & 0x30303030u);
@@ -913,9 +922,8 @@ __device__ __forceinline__ void q4k_slab_compute(const u32x4_t *blk, const half8
     const half2_t s2h = splat(S[1]), c2h = splat(Cs[1]);
     const uint32_t qw[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
     const _Float16 zero = static_cast<_Float16>(0.0f);
-    const half8_t a_min = {tw[0], tw[1], tw[2], tw[3], zero, zero, zero, zero};
-    const half8_t b_min = {M[0], M[1], M[0], M[1], zero, zero, zero, zero};
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_min, b_min, acc, 0, 0, 0);
+    const half8_t b_two = {M[0], M[1], M[0], M[1], zero, zero, zero, zero};  // (no `over` parts in a_min)
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_min, over ? q4k_min_operand(M) : b_two, acc, 0, 0, 0);
 #pragma unroll
     for (int t = 0; t < 4; t++) {
         const half8_t bl = unpack_scale<false>(qw[2 * t], qw[2 * t + 1], s2l, c2l, magic.lo);
@@ -926,6 +934,67 @@ __device__ __forceinline__ void q4k_slab_compute(const u32x4_t *blk, const half8
         const half8_t bh = unpack_scale<true>(qw[2 * t], qw[2 * t + 1], s2h, c2h, magic.hi);
         acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[4 + t], bh, acc, 0, 0, 0);
     }
+}
+
+__device__ __forceinline__ void q4k_slab_compute(const u32x4_t *blk, const half8_t *a, const half4_t *twin, int g, uint32_t sc_sel,
+                                                 Q4KMagic magic, float4_t &acc) {
+    const u32x4_t hdr = blk[0], q0 = blk[1 + 2 * g], q1 = blk[2 + 2 * g];
+    half8_t af[8];
+#pragma unroll
+    for (int t = 0; t < 8; t++) af[t] = a[t * 64];
+    const half4_t tw = *twin;
+    const _Float16 zero = static_cast<_Float16>(0.0f);
+    const half8_t a_min = {tw[0], tw[1], tw[2], tw[3], zero, zero, zero, zero};
+    q4k_stage(hdr, q0, q1, af, a_min, g, sc_sel, magic, acc, false);
+}
+
+// ---- a tile again, for sums past the f16 range (mfma_unpack.h, Q4KSumParts) ----
+// The kernels that keep two parts of a sub-block's sum ask at the end of a tile whether a NaN came out (of such a sum, or
+// of what the caller passed in: then it comes out again), which costs a lightly loaded wave nothing that can be measured.
+// All parts in LDS, or a flag per slab, cost the expert kernel 0.5 us a launch (decode step of 40 layers 2.70 -> 2.75 ms).
+__device__ __forceinline__ bool q4k_any_nan(float4_t v) {
+    const float s = (v[0] + v[1]) + (v[2] + v[3]);
+    return __ballot(s != s) != 0;
+}
+__device__ __forceinline__ void q4k_octet_to_half(const float *p, _Float16 *h) {
+    const float4_t a = *reinterpret_cast<const float4_t *>(p), b = *reinterpret_cast<const float4_t *>(p + 4);
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        h[i] = static_cast<_Float16>(a[i]);
+        h[4 + i] = static_cast<_Float16>(b[i]);
+    }
+}
+__device__ __forceinline__ void q4k_octet_to_half(const _Float16 *p, _Float16 *h) {  // (8-byte aligned)
+    const half4_t a = *reinterpret_cast<const half4_t *>(p), b = *reinterpret_cast<const half4_t *>(p + 4);
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        h[i] = a[i];
+        h[4 + i] = b[i];
+    }
+}
+// The product over `len` super-blocks straight from memory: the lane's weight row at `w`, w_step bytes from one super-block
+// to the next, and its row of X.  Sums in the order of the kernel that asks (kSeq: q4k_octet_sum_seq).
+template <typename XT, bool kSeq>
+__device__ __forceinline__ float4_t q4k_again(const uint8_t *w, size_t w_step, const XT *x, int len, int g, uint32_t sc_sel, Q4KMagic magic) {
+    float4_t acc = {0, 0, 0, 0};
+    x += 64 * g;
+#pragma nounroll
+    for (int b = 0; b < len; b++, w += w_step, x += DFL_QK_K) {
+        const u32x4_t *blk = reinterpret_cast<const u32x4_t *>(w);
+        half8_t af[8];
+        float o[8];
+#pragma unroll
+        for (int t = 0; t < 8; t++) {
+            _Float16 h[8];
+            q4k_octet_to_half(x + 8 * t, h);
+            const half8_t frag = {h[0], h[2], h[1], h[3], h[4], h[6], h[5], h[7]};
+            af[t] = frag;
+            o[t] = kSeq ? q4k_octet_sum_seq(h) : q4k_octet_sum(h);
+        }
+        const half8_t a_min = q4k_sum_operand((o[0] + o[1]) + (o[2] + o[3]), (o[4] + o[5]) + (o[6] + o[7]));
+        q4k_stage(blk[0], blk[1 + 2 * g], blk[2 + 2 * g], af, a_min, g, sc_sel, magic, acc, true);
+    }
+    return acc;
 }
 
 // s_waitcnt vmcnt(3 n): at most n load groups (three instructions each) still in flight, n uniform
@@ -1057,7 +1126,7 @@ __global__ void __launch_bounds__(64 * kSlabWaves)
     const uint32_t sc_sel = (lane & 16) ? 0x04030402u : 0x04010400u;
     const Q4KMagic magic = q4k_magic();
     float4_t acc = {0, 0, 0, 0}, stash = {0, 0, 0, 0};
-    int gc = rg.first_group, bc = b0;
+    int gc = rg.first_group, bc = b0, bs = b0;  // group, super-block, first super-block of the group's part here
     for (int t = 0; t < len; t++) {
         q4k_slab_wait_groups(w_issued - 1 - t);  // loads land in order: stage t has when only later ones are in flight
         if (t == 0) DFL_TRW(4);
@@ -1071,9 +1140,14 @@ __global__ void __launch_bounds__(64 * kSlabWaves)
         q4k_slab_compute(blk, reinterpret_cast<const half8_t *>(stage) + lane,
                          reinterpret_cast<const half4_t *>(stage + kQ4KBlockFrags * 16) + lane, g, sc_sel, magic, acc);
         if (++bc == nb || t + 1 == len) {
+            if (__builtin_expect(q4k_any_nan(acc), 0)) {
+                const int row = min((gc * kW + wave) * 16 + n, n_out - 1);
+                acc = q4k_again<XT, false>(w + static_cast<size_t>(row) * row_bytes + static_cast<size_t>(bs) * DFL_Q4_K_BYTES, DFL_Q4_K_BYTES,
+                                           x + static_cast<size_t>(min(n, n_rows - 1)) * n_in + bs * DFL_QK_K, bc - bs, g, sc_sel, magic);
+            }
             q4k_flush<kW>(rg, bt, gc, acc, stash, y, partials, n_out, n_rows, tid);
             acc = float4_t{0, 0, 0, 0};
-            bc = 0;
+            bc = bs = 0;
             gc++;
         }
     }
@@ -1166,35 +1240,9 @@ __device__ __forceinline__ void q4k_tiled_compute(const u32x4_t *blk, const uint
 #pragma unroll
     for (int t = 0; t < 8; t++) af[t] = *reinterpret_cast<const half8_t *>(stage + t * kTiledFragStride + lane * 16);
     const half4_t tw = *reinterpret_cast<const half4_t *>(stage + 8 * kTiledFragStride + lane * 8);
-    const uint32_t upper = 0u - static_cast<uint32_t>(g >> 1);
-    const uint32_t sc_lo = hdr.y & 0x3F3F3F3Fu, sc_hi = (hdr.w & 0x0F0F0F0Fu) | ((hdr.y >> 2) & 0x30303030u);
-    const uint32_t mn_lo = hdr.z & 0x3F3F3F3Fu, mn_hi = ((hdr.w >> 4) & 0x0F0F0F0Fu) | ((hdr.z >> 2) & 0x30303030u);
-    const uint32_t sc_word = (sc_hi & upper) | (sc_lo & ~upper), mn_word = (mn_hi & upper) | (mn_lo & ~upper);
-    const half2_t dm = __builtin_bit_cast(half2_t, hdr.x);
-    const half2_t p_sc = as_half2(__builtin_amdgcn_perm(0x64646464u, sc_word, sc_sel));
-    const half2_t p_mn = as_half2(__builtin_amdgcn_perm(0x64646464u, mn_word, sc_sel));
-    const half2_t neg = dm * splat(static_cast<_Float16>(-1024.0f));
-    const half2_t S = __builtin_elementwise_fma(p_sc, splat(dm[0]), splat(neg[0]));
-    const half2_t M = __builtin_elementwise_fma(p_mn, splat(-dm[1]), splat(-neg[1]));  // -(dmin * m)
-    const half2_t unbias = {static_cast<_Float16>(-1024.0f), static_cast<_Float16>(-64.0f)};
-    const half2_t Cs = S * unbias;
-    const half2_t s2l = splat(S[0]), c2l = splat(Cs[0]);
-    const half2_t s2h = splat(S[1]), c2h = splat(Cs[1]);
-    const uint32_t qw[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
     const _Float16 zero = static_cast<_Float16>(0.0f);
     const half8_t a_min = {tw[0], tw[1], tw[2], tw[3], zero, zero, zero, zero};
-    const half8_t b_min = {M[0], M[1], M[0], M[1], zero, zero, zero, zero};
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_min, b_min, acc, 0, 0, 0);
-#pragma unroll
-    for (int t = 0; t < 4; t++) {
-        const half8_t bl = unpack_scale<false>(qw[2 * t], qw[2 * t + 1], s2l, c2l, magic.lo);
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[t], bl, acc, 0, 0, 0);
-    }
-#pragma unroll
-    for (int t = 0; t < 4; t++) {
-        const half8_t bh = unpack_scale<true>(qw[2 * t], qw[2 * t + 1], s2h, c2h, magic.hi);
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[4 + t], bh, acc, 0, 0, 0);
-    }
+    q4k_stage(hdr, q0, q1, af, a_min, g, sc_sel, magic, acc, false);
 }
 
 // The tiled kernel.  Same work split, flush and reduction as the slab kernel.  Order of the prologue: the
@@ -1303,7 +1351,7 @@ __global__ void __launch_bounds__(64 * kSlabWaves)
     const uint32_t sc_sel = (lane & 16) ? 0x04030402u : 0x04010400u;
     const Q4KMagic magic = q4k_magic();
     float4_t acc = {0, 0, 0, 0}, stash = {0, 0, 0, 0};
-    int gc = rg.first_group, bc = b0;
+    int gc = rg.first_group, bc = b0, bs = b0;  // group, super-block, first super-block of the group's part here
     for (int t = 0; t < len; t++) {
         q4k_slab_wait_groups(w_issued - 1 - t);  // loads land in order: stage t has when only later ones are in flight
         if (t == 0) DFL_TRW(4);
@@ -1316,9 +1364,13 @@ __global__ void __launch_bounds__(64 * kSlabWaves)
         // stage t+3 into the buffer this stage has just been read out of (its reads are complete: the MFMAs above used them)
         if (w_issued < len) issue_w();
         if (++bc == nb || t + 1 == len) {
+            if (__builtin_expect(q4k_any_nan(acc), 0))
+                acc = q4k_again<XT, false>(w + (static_cast<size_t>(gc) * nb + bs) * kTiledStageBytes + wave * kTiledTileBytes + n * DFL_Q4_K_BYTES,
+                                           kTiledStageBytes, x + static_cast<size_t>(min(n, n_rows - 1)) * n_in + bs * DFL_QK_K, bc - bs, g,
+                                           sc_sel, magic);
             q4k_flush<kW>(rg, bt, gc, acc, stash, y, partials, n_out, n_rows, tid);
             acc = float4_t{0, 0, 0, 0};
-            bc = 0;
+            bc = bs = 0;
             gc++;
         }
     }
@@ -1403,6 +1455,7 @@ __global__ void __launch_bounds__(64 * kSlabWaves)
     constexpr int kW = kSlabWaves;
     constexpr int kItems = kExpChunk * 8 / kW;  // activation items (eight values of one row) per thread and refill: 2
     constexpr int kXInstr = kItems * Q4KX8<XT>::kLoads;
+    static_assert(3 * (kSlabRing - 1) + kXInstr <= 10 && 3 * kSlabRing <= 10, "q4k_wait_vm_few");
     extern __shared__ half8_t lds[];
     uint8_t *slab = reinterpret_cast<uint8_t *>(lds);                              // [kExpChunk][kTiledStageX]
     half8_t *ring = reinterpret_cast<half8_t *>(slab + kExpChunk * kTiledStageX);  // [wave][kSlabRing][144]
@@ -1629,7 +1682,7 @@ __global__ void __launch_bounds__(64 * kSlabWaves)
     for (int t = 0; t < 2; t++)
         if (it_valid) issue();
     DFL_TRE(2);
-    q4k_wait_vm(3 * w_issued);  // the activations are older than every weight load
+    q4k_wait_vm_few(3 * w_issued);  // the activations are older than every weight load
     convert(0);
     __builtin_amdgcn_s_waitcnt(kWaitLds);
     __builtin_amdgcn_s_barrier();
@@ -1640,6 +1693,25 @@ __global__ void __launch_bounds__(64 * kSlabWaves)
     const int n = lane & 15, g = lane >> 4;
     const uint32_t sc_sel = (lane & 16) ? 0x04030402u : 0x04010400u;
     const Q4KMagic magic = q4k_magic();
+    auto put = [&](int slot, int tile, float4_t res, const float4_t &up) {  // the unit's results; whether there is a NaN among them
+        if (bt.pair) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) res[i] = res[i] / (1.0f + expf(-res[i])) * up[i];  // silu(gate) * up
+        }
+        // (rare path: an opaque copy of the lane index keeps its address arithmetic out of the stage loop's registers)
+        int ol = lane;
+        asm volatile("" : "+v"(ol));
+        const int on = ol & 15, og = ol >> 4;
+        YT *yo = y + static_cast<size_t>(slot) * bt.y_stride;
+        const int orow = tile * 16 + on;
+        if (orow < n_out) {
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                if (4 * og + i < n_rows) yo[static_cast<size_t>(4 * og + i) * n_out + orow] = static_cast<YT>(res[i]);
+        }
+        return q4k_any_nan(res);
+    };
+    bool again = false;
     for (int r = 0; r < n_rounds; r++) {
         int slot = 0, tile = 0;
         const bool active = unit_of(r, slot, tile);
@@ -1648,7 +1720,7 @@ __global__ void __launch_bounds__(64 * kSlabWaves)
         for (int c = 0; c < n_chunks; c++) {
             if (xslot != slab_slot || c != slab_chunk) {
                 __builtin_amdgcn_s_barrier();  // every wave has read what it needed of the old slab
-                if (x_pending) q4k_wait_vm(3 * min(w_issued - x_pos, w_issued - w_done));
+                if (x_pending) q4k_wait_vm_few(3 * min(w_issued - x_pos, w_issued - w_done));
                 x_pending = false;
                 convert(c);
                 __builtin_amdgcn_s_waitcnt(kWaitLds);
@@ -1678,7 +1750,7 @@ __global__ void __launch_bounds__(64 * kSlabWaves)
                 for (int s = 0; s < clen; s++) {
                     // stage w_done has landed when only younger loads are in flight
                     const bool x_younger = x_pending && x_pos > w_done;
-                    q4k_wait_vm(3 * (w_issued - 1 - w_done) + (x_younger ? kXInstr : 0));
+                    q4k_wait_vm_few(3 * (w_issued - 1 - w_done) + (x_younger ? kXInstr : 0));
                     if (!x_younger) x_pending = false;
                     if (w_done == 0) DFL_TRE(4);
                     const u32x4_t *blk = reinterpret_cast<const u32x4_t *>(my_ring + ring_c * kSlabWavePieces) + n * 9;
@@ -1700,23 +1772,25 @@ __global__ void __launch_bounds__(64 * kSlabWaves)
             __builtin_amdgcn_s_barrier();
             if (active && wave < kW / 2) acc1 = *xchg;
         }
-        if (active && !(hsplit && wave >= kW / 2)) {
-            float4_t res = acc0;
-            if (bt.pair) {
-#pragma unroll
-                for (int i = 0; i < 4; i++) res[i] = res[i] / (1.0f + expf(-res[i])) * acc1[i];  // silu(gate) * up
+        if (active && !(hsplit && wave >= kW / 2)) again |= put(slot, tile, acc0, acc1);
+    }
+    if (__builtin_expect(again, 0)) {  // (all of the wave's units: the others get the bits they have)
+        int al = lane;                 // (opaque copy, as above)
+        asm volatile("" : "+v"(al));
+        const int an = al & 15;
+#pragma nounroll
+        for (int r = 0; r < n_rounds; r++) {
+            int slot = 0, tile = 0;
+            if (!unit_of(r, slot, tile)) continue;
+            const XT *xrow = x + static_cast<size_t>(xslot_of(r)) * bt.x_stride + static_cast<size_t>(min(an, n_rows - 1)) * n_in;
+            float4_t acc[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+#pragma nounroll
+            for (int h = 0; h < halves; h++) {
+                const float4_t v = q4k_again<XT, true>(tile_base(slot, tile, h) + an * DFL_Q4_K_BYTES, kTiledStageBytes, xrow, nb, al >> 4,
+                                                       (al & 16) ? 0x04030402u : 0x04010400u, q4k_magic());
+                if (h) acc[1] = v; else acc[0] = v;
             }
-            // (rare path: an opaque copy of the lane index keeps its address arithmetic out of the stage loop's registers)
-            int ol = lane;
-            asm volatile("" : "+v"(ol));
-            const int on = ol & 15, og = ol >> 4;
-            YT *yo = y + static_cast<size_t>(slot) * bt.y_stride;
-            const int orow = tile * 16 + on;
-            if (orow < n_out) {
-#pragma unroll
-                for (int i = 0; i < 4; i++)
-                    if (4 * og + i < n_rows) yo[static_cast<size_t>(4 * og + i) * n_out + orow] = static_cast<YT>(res[i]);
-            }
+            put(slot, tile, acc[0], acc[1]);
         }
     }
     DFL_TRE(6);

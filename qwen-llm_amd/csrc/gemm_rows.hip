@@ -506,9 +506,7 @@ __global__ void __launch_bounds__(64) xf_sums_kernel(const uint8_t *__restrict__
         const _Float16 h[8] = {f[0], f[2], f[1], f[3], f[4], f[6], f[5], f[7]};
         o[t] = q4k_octet_sum(h);
     }
-    const Q4KSumParts s0 = q4k_sum_parts((o[0] + o[1]) + (o[2] + o[3])), s1 = q4k_sum_parts((o[4] + o[5]) + (o[6] + o[7]));
-    const _Float16 zero = static_cast<_Float16>(0.0f);
-    const half8_t r = {s0.hi, s1.hi, s0.lo, s1.lo, s0.over, s1.over, zero, zero};
+    const half8_t r = q4k_sum_operand((o[0] + o[1]) + (o[2] + o[3]), (o[4] + o[5]) + (o[6] + o[7]));
     reinterpret_cast<half8_t *>(xs + (static_cast<size_t>(blk) * nb + b) * 1024)[lane] = r;
 }
 

@@ -49,14 +49,16 @@ __device__ __forceinline__ half8_t unpack_scale(uint32_t w0, uint32_t w1, half2_
 // ---- the Q4_K minima as one MFMA per super-block ----
 // Lane (m, g) of the A operand holds the sums of row m's rounded activations over sub-blocks 2g and 2g + 1, each split
 // into f16 parts, in k-slots {hi, hi', lo, lo', over, over', 0, 0}; the B operand holds the lane's two (negated) minima
-// in the matching slots.  hi + lo carries 22 bits of the sum.  `over` (in units of 32) keeps a sum past the f16 range -
-// 32 activations of more than 2000 - finite; it is zero otherwise and then adds nothing.
+// in the matching slots.  hi + lo carries 22 bits of the sum.  `over` (in units of 32) keeps a sum that would round past
+// the largest f16 - 32 activations of about 2000 - finite; it is zero otherwise and then adds nothing.  The slab, tiled
+// and expert kernels hold hi and lo alone (LDS, and the chain of a lightly loaded wave): such a sum is infinite there,
+// its row's results come out NaN, and the wave computes its tile again with all three parts (q4k_again, gemm_fewrow.hip).
 struct Q4KSumParts {
     _Float16 hi, lo, over;
 };
 __device__ __forceinline__ Q4KSumParts q4k_sum_parts(float sum) {
     Q4KSumParts p;
-    p.over = fabsf(sum) > 32768.0f ? static_cast<_Float16>(sum * 0.03125f) : static_cast<_Float16>(0.0f);
+    p.over = fabsf(sum) >= 65520.0f ? static_cast<_Float16>(sum * 0.03125f) : static_cast<_Float16>(0.0f);
     const float rest = sum - 32.0f * static_cast<float>(p.over);
     p.hi = static_cast<_Float16>(rest);
     p.lo = static_cast<_Float16>(rest - static_cast<float>(p.hi));
@@ -73,6 +75,13 @@ __device__ __forceinline__ float q4k_octet_sum_seq(const _Float16 *h) {
 #pragma unroll
     for (int i = 0; i < 8; i++) s += static_cast<float>(h[i]);
     return s;
+}
+// A lane's A operand from the sums of its two sub-blocks.
+__device__ __forceinline__ half8_t q4k_sum_operand(float sum0, float sum1) {
+    const Q4KSumParts s0 = q4k_sum_parts(sum0), s1 = q4k_sum_parts(sum1);
+    const _Float16 zero = static_cast<_Float16>(0.0f);
+    const half8_t a = {s0.hi, s1.hi, s0.lo, s1.lo, s0.over, s1.over, zero, zero};
+    return a;
 }
 __device__ __forceinline__ half8_t q4k_min_operand(half2_t m) {
     const _Float16 k32 = static_cast<_Float16>(32.0f), zero = static_cast<_Float16>(0.0f);

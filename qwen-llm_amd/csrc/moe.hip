@@ -589,9 +589,7 @@ __global__ void __launch_bounds__(64)
         dst[t * 64] = frag;
         o[t] = q4k_octet_sum_seq(h);
     }
-    const Q4KSumParts s0 = q4k_sum_parts((o[0] + o[1]) + (o[2] + o[3])), s1 = q4k_sum_parts((o[4] + o[5]) + (o[6] + o[7]));
-    const _Float16 zero = static_cast<_Float16>(0.0f);
-    const half8_t r = {s0.hi, s1.hi, s0.lo, s1.lo, s0.over, s1.over, zero, zero};
+    const half8_t r = q4k_sum_operand((o[0] + o[1]) + (o[2] + o[3]), (o[4] + o[5]) + (o[6] + o[7]));
     reinterpret_cast<half8_t *>(sums + (static_cast<size_t>(slot) * nb + b) * 1024)[lane] = r;
 }
 

@@ -226,6 +226,30 @@ def test_gemm_q4k_tiled_order_is_bit_identical(ctx, n_in, n_out, n_rows, x_dtype
     assert torch.isnan(buf[:guard]).all() and torch.isnan(buf[-guard:]).all()
 
 
+@pytest.mark.parametrize("n_in,n_out", [(256, 16), (1280, 1000), (5120, 6144), (17408, 512), (2048, 50000)])
+@pytest.mark.parametrize("x_dtype", [np.float32, np.float16])
+def test_gemm_q4k_sums_past_f16(ctx, oracle, n_in, n_out, x_dtype, canaries):
+    """Rows whose sub-block sums lie on both sides of 65520, where a sum no longer rounds to an f16, and at the most that
+    f16 activations can reach (32 x 60000), beside ordinary rows: the slab, the tiled and the streaming kernel (2048 ->
+    50000) against the f64 product, row order and tiled order bit for bit, and an ordinary row with the bits it has alone."""
+    import torch
+    rng = np.random.default_rng(n_in + n_out)
+    w = dfl.synth.random_blocks(dfl.synth.Q4_K, n_out * n_in // 256, n_in + n_out)
+    level = np.array([0.0, 1000.0, 1024.0, -2030.0, 2046.0, -2060.0, 2500.0, 9000.0, -30000.0, 60000.0, 0.0])
+    x = (rng.standard_normal((len(level), n_in)) * np.maximum(np.abs(level[:, None]) * 0.01, 1.0) + level[:, None]).astype(x_dtype)
+    wd, xd = dev(w), dev(x)
+    y = gemm_fast(ctx, wd, dfl.TYPE_Q4_K, xd, n_in, n_out)
+    yt = ctx.gemm_fewrow(ctx.repack_q4k_tiled(wd, n_in, n_out), dfl.TYPE_Q4_K_TILED, xd, n_in, n_out)
+    assert torch.isfinite(y).all()
+    assert torch.equal(y.view(torch.int32), yt.view(torch.int32))
+    alone = gemm_fast(ctx, wd, dfl.TYPE_Q4_K, xd[:1].contiguous(), n_in, n_out)
+    assert torch.equal(y[:1].view(torch.int32), alone.view(torch.int32))
+    cols = rng.permutation(n_out)[:1000]
+    ref = f64_reference(oracle, dfl.synth.Q4_K, w.reshape(n_out, -1)[cols], x.astype(np.float32), n_in, len(cols))
+    for r in range(len(level)):
+        check_gemm(y[r:r + 1, cols].cpu().numpy(), ref[r:r + 1], f"{n_in}x{n_out} row around {level[r]}")
+
+
 def test_q4k_tiled_repack_layout(ctx):
     """Block (row r, super-block b) of the row-order matrix sits at [r // 256][b][r % 256] of the tiled one; rows
     past n_out are zero blocks."""

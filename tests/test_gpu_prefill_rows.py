@@ -63,3 +63,37 @@ def test_continued_prefill_equals_block_by_block(ctx, shape, head, rows):
     assert torch.equal(got, want)
     one.close()
     many.close()
+
+
+def _rescale(mat, factor):
+    blocks = mat[1].view(-1, dfl.synth.BLOCK_BYTES[dfl.synth.Q4_K])
+    blocks[:, :4] = (blocks[:, :4].contiguous().view(torch.float16) * factor).view(torch.uint8)
+
+
+@pytest.mark.parametrize("where", ["gate_up", "down"])
+@pytest.mark.parametrize("shape,expert_wgs", [("experts", 256), ("experts", 40), ("narrow", 256), ("wide", 256)])
+def test_prefill_equals_block_by_block_with_sums_past_f16(ctx, monkeypatch, shape, expert_wgs, where):
+    """Activations whose sub-block sums pass the largest f16, with every activation itself inside: in the normed rows
+    (gains of 4000: the sums of 32 are about +-23000) or in the SwiGLU rows (gate = up: 32 values of one sign, some 2000
+    each).  The expert launches with gate and up of a tile on two waves (256 workgroups) and in rounds on one (40)."""
+    monkeypatch.setenv("DFLASH_MOE_WGS", str(expert_wgs))
+    cfg, attn_type = SHAPES[shape]
+    w = dfl.synth_target_weights_device(cfg, 5, "cuda", attn_type=attn_type)
+    for L in w["layers"]:
+        L["post_norm"] = L["post_norm"] * (4000.0 if where == "gate_up" else 47.0)
+        for gate, up in (("gate", "up"),) + ((("gate_exps", "up_exps"),) if cfg.n_expert else ()):
+            if where == "gate_up":
+                _rescale(L[gate], 1 / 400)
+                _rescale(L[up], 1 / 400)
+            else:
+                L[up] = (L[gate][0], L[gate][1].clone())
+    model = dfl.TargetModel(ctx, cfg, w)
+    rows = 97
+    one, many = dfl.Session(ctx, model, rows + 16, [0, 1]), dfl.Session(ctx, model, rows + 16, [0, 1])
+    tokens = np.random.default_rng(rows).integers(0, cfg.vocab, rows).tolist()
+    got = many.prefill_blocks(tokens, 0)
+    want = torch.cat([one.encode_packed_verify_layer_major(tokens[i:i + 16], i, want_head=False).hidden_capture for i in range(0, rows, 16)])
+    assert torch.isfinite(got).all() and torch.isfinite(want).all()
+    assert torch.equal(got, want)
+    one.close()
+    many.close()
