@@ -20,6 +20,8 @@ SHAPES = {
     "experts": (dfl.ModelConfig(n_layers=2, hidden=2048, n_q=16, n_kv=2, head_dim=256, ffn=0, vocab=2048, n_expert=32, n_expert_used=4,
                                 ffn_expert=768, ffn_shared=768), dfl.synth.Q6_K),
 }
+SHAPES["experts128"] = (dfl.ModelConfig(n_layers=2, hidden=2048, n_q=16, n_kv=2, head_dim=256, ffn=0, vocab=2048, n_expert=128, n_expert_used=8,
+                                        ffn_expert=768, ffn_shared=768), dfl.synth.Q6_K)
 SHAPES["heads64"] = (dfl.ModelConfig(n_layers=2, hidden=1024, n_q=24, n_kv=2, head_dim=64, ffn=3072, vocab=2048), dfl.synth.Q4_K)
 SHAPES["heads256x5"] = (dfl.ModelConfig(n_layers=2, hidden=1280, n_q=5, n_kv=1, head_dim=256, ffn=3072, vocab=2048), dfl.synth.Q4_K)
 
@@ -71,12 +73,11 @@ def _rescale(mat, factor):
 
 
 @pytest.mark.parametrize("where", ["gate_up", "down"])
-@pytest.mark.parametrize("shape,expert_wgs", [("experts", 256), ("experts", 40), ("narrow", 256), ("wide", 256)])
-def test_prefill_equals_block_by_block_with_sums_past_f16(ctx, monkeypatch, shape, expert_wgs, where):
+@pytest.mark.parametrize("shape", ["experts", "experts128", "narrow", "wide"])
+def test_prefill_equals_block_by_block_with_sums_past_f16(ctx, shape, where):
     """Activations whose sub-block sums pass the largest f16, with every activation itself inside: in the normed rows
     (gains of 4000: the sums of 32 are about +-23000) or in the SwiGLU rows (gate = up: 32 values of one sign, some 2000
-    each).  The expert launches with gate and up of a tile on two waves (256 workgroups) and in rounds on one (40)."""
-    monkeypatch.setenv("DFLASH_MOE_WGS", str(expert_wgs))
+    each).  A block of 16 picks some 28 of 32 experts, gate and up of a tile on two waves, or 80 of 128, both on one."""
     cfg, attn_type = SHAPES[shape]
     w = dfl.synth_target_weights_device(cfg, 5, "cuda", attn_type=attn_type)
     for L in w["layers"]:
