@@ -2677,21 +2677,19 @@ int32_t launch_q4k(dflash_ctx *ctx, const void *w, const void *x, int32_t x_type
                                                                                            no, nb, n_rows, bt, upm, by_upm, max_slots, early_ids); \
     } while (0)
         if (bt.route_logits) {
-            if (x_type != DFLASH_TYPE_F32 || per_slot_x || bt.route_experts > 256 || bt.route_experts < 1 || bt.route_used < 1 ||
+            if (x_type != DFLASH_TYPE_F32 || per_slot_x || !bt.y_f16 || bt.route_experts > 256 || bt.route_experts < 1 || bt.route_used < 1 ||
                 bt.route_used > 64 || bt.route_used > bt.route_experts || max_slots + 0 > kExpRouteIds - 1)
-                return dfl_fail(ctx, DFLASH_ERR_UNSUPPORTED, "gemm_q4k_batched: routing inside the launch needs f32 shared activations and at most 256 experts");
-            if (bt.y_f16)
-                DFL_LAUNCH_EXPERTS(float, _Float16, true);
-            else
-                DFL_LAUNCH_EXPERTS(float, float, true);
-        } else if (x_type == DFLASH_TYPE_F32 && !bt.y_f16)
+                return dfl_fail(ctx, DFLASH_ERR_UNSUPPORTED, "gemm_q4k_batched: routing inside the launch needs f32 shared activations, f16 output and at most 256 experts");
+            DFL_LAUNCH_EXPERTS(float, _Float16, true);
+        } else if (x_type == DFLASH_TYPE_F32 && !bt.y_f16) {
             DFL_LAUNCH_EXPERTS(float, float, false);
-        else if (x_type == DFLASH_TYPE_F32)
+        } else if (x_type == DFLASH_TYPE_F32) {
             DFL_LAUNCH_EXPERTS(float, _Float16, false);
-        else if (!bt.y_f16)
+        } else if (!bt.y_f16) {
             DFL_LAUNCH_EXPERTS(_Float16, float, false);
-        else
-            DFL_LAUNCH_EXPERTS(_Float16, _Float16, false);
+        } else {
+            return dfl_fail(ctx, DFLASH_ERR_UNSUPPORTED, "gemm_q4k_batched: f16 output needs f32 activations");
+        }
 #undef DFL_LAUNCH_EXPERTS
         DFL_HIP_CHECK(ctx, hipGetLastError());
         return DFLASH_OK;
