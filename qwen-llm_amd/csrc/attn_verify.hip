@@ -940,29 +940,37 @@ int32_t dfl_attn_blocks(dflash_ctx *ctx, const void *q, int32_t q_type, const vo
     const int group = n_q / n_kv;
     auto bucket_of = [&](int32_t b) { return dfl_attn_bucket(ctx_len + 16ll * b + std::min(16, n_rows_total - 16 * b)); };
     {
-        // The leading blocks whose splits are merged in order: one launch without partial results, if they are enough
-        // workgroups for it.  A workgroup of it takes its stages one after the other, 1 us each: n_steps of them for the last
-        // block.  The splits spread them over the chip, but a partial result goes out and comes back every two of them, and
-        // there are two launches: 8 us and 1.25 us per stage of a CU's share.  (Six layers of 16 / 8 heads of 128, behind 1900
-        // positions: 512 rows 1178 -> 1035 us this way, 256 rows 782 -> 897; behind none 739 -> 631 and 543 -> 512.)
+        // The leading blocks whose splits are merged in order: one launch without partial results, or the splits and their
+        // merges.  A workgroup of the one launch takes its stages one after the other, about 1.15 us each: n_steps of them for
+        // the last block.  The splits spread them over the chip, but they are two launches for every run of blocks that
+        // shares a policy (11 us), and a partial tile (16 rows of a head, 8 KB at 128 dims) goes out and comes back; besides,
+        // a stage of a workgroup.  Both sides in us, by least squares over 111 pairs of measured sides: 16 / 8, 32 / 8, 48 / 8
+        // and 20 / 4 heads of 128, 32 / 4 of 64, 33 - 1024 rows behind 0 - 3900 positions (one layer, splits against one
+        // launch: 32 / 8 heads 143 : 46 us for 1024 rows behind none, 87 : 78 for 256 behind 1900, 56 : 134 for 128 behind
+        // 3900; 32 / 4 of 64 80 : 36, 55 : 66, 32 : 115).  The better side, or within 6 % of it, in all but one (1.24).
         AttnRuns runs = {};
         int32_t taken = 0;
+        int64_t partials = 0;  // partial tiles of 128 dims
         for (int64_t last = -1; taken < n_blocks && q_type == DFLASH_TYPE_F32; taken++) {
-            const int64_t bucket = bucket_of(taken);
-            if (bucket == last) continue;
-            const AttnPolicy p = attn_policy(ctx, bucket, n_kv, group, head_dim);
-            if (!p.ordered || runs.n == kAttnRuns) break;
-            last = bucket;
-            runs.first[runs.n] = taken;
-            runs.want[runs.n] = p.want;
-            runs.min_chunk[runs.n++] = static_cast<int>(p.min_chunk);
+            const int64_t n_pos = ctx_len + std::min(16 * (taken + 1), n_rows_total), bucket = dfl_attn_bucket(n_pos);
+            if (bucket != last) {
+                const AttnPolicy p = attn_policy(ctx, bucket, n_kv, group, head_dim);
+                if (!p.ordered || runs.n == kAttnRuns) break;
+                last = bucket;
+                runs.first[runs.n] = taken;
+                runs.want[runs.n] = p.want;
+                runs.min_chunk[runs.n++] = static_cast<int>(p.min_chunk);
+            }
+            const int64_t chunk = attn_chunk(n_pos, runs.want[runs.n - 1], runs.min_chunk[runs.n - 1]);
+            partials += (n_pos + chunk - 1) / chunk * n_q * head_dim / 128;
         }
         int hw = std::min(group, 8);
         while (group % hw) hw--;
         const int32_t rows = std::min(n_rows_total, 16 * taken);
         const int64_t wgs = static_cast<int64_t>(taken) * n_kv * (group / hw), n_steps = (ctx_len + rows + 31) / 32;
         const int64_t stages = wgs * (ctx_len + rows / 2) / 32;
-        if (taken > 1 && 4 * n_steps * ctx->n_cu <= 32 * ctx->n_cu + 5 * stages) {
+        const double one_launch = 5.5 + 1.15 * n_steps, as_splits = 11.0 * runs.n + (0.5 * stages + 1.1 * partials) / ctx->n_cu;
+        if (taken > 1 && one_launch <= as_splits) {
             hipStream_t st = static_cast<hipStream_t>(stream);
             dfl_timed timer(ctx, st, DFL_T_ATTN);
             const auto launch = head_dim == 64 ? launch_rows<64> : launch_rows<128>;

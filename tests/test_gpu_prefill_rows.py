@@ -23,6 +23,7 @@ SHAPES = {
 SHAPES["experts128"] = (dfl.ModelConfig(n_layers=2, hidden=2048, n_q=16, n_kv=2, head_dim=256, ffn=0, vocab=2048, n_expert=128, n_expert_used=8,
                                         ffn_expert=768, ffn_shared=768), dfl.synth.Q6_K)
 SHAPES["heads64"] = (dfl.ModelConfig(n_layers=2, hidden=1024, n_q=24, n_kv=2, head_dim=64, ffn=3072, vocab=2048), dfl.synth.Q4_K)
+SHAPES["heads64x12"] = (dfl.ModelConfig(n_layers=2, hidden=1024, n_q=48, n_kv=4, head_dim=64, ffn=3072, vocab=2048), dfl.synth.Q4_K)
 SHAPES["heads256x5"] = (dfl.ModelConfig(n_layers=2, hidden=1280, n_q=5, n_kv=1, head_dim=256, ffn=3072, vocab=2048), dfl.synth.Q4_K)
 
 
@@ -48,7 +49,7 @@ def test_many_row_prefill_equals_block_by_block(ctx, shape, rows):
 
 
 @pytest.mark.parametrize("head,rows", [(7, 40), (245, 33), (480, 400), (1000, 530), (1000, 1100)])
-@pytest.mark.parametrize("shape", ["narrow", "experts", "heads64", "heads256x5"])
+@pytest.mark.parametrize("shape", ["narrow", "experts", "heads64", "heads64x12", "heads256x5"])
 def test_continued_prefill_equals_block_by_block(ctx, shape, head, rows):
     """Behind a context, where the attention takes the keys of many blocks split by split in one workgroup or leaves
     them to several (by how many workgroups there are), across buckets of context lengths, with a last split and a
