@@ -234,7 +234,8 @@ int32_t dfl_gemm_whole(dflash_ctx *ctx, int32_t w_type, const void *w, const voi
 // The weights are read once and stay in registers while the blocks pass; a row's bits are those of dfl_gemm_whole.
 int32_t dfl_gemm_whole_blocks(dflash_ctx *ctx, int32_t w_type, const void *w, const void *xf, float *y, int64_t n_in, int64_t n_out,
                               int32_t n_rows_total, int64_t pair_ffn, void *y_xf, int y_xf_kind, hipStream_t stream);
-bool dfl_whole_takes_blocks(const dflash_ctx *ctx, int32_t w_type, int64_t n_in, int64_t n_out);  // (the looping variant takes one)
+// Whether a wave has one super-block of one tile, whose unpacked weights it then keeps from block to block.
+bool dfl_whole_holds_weights(const dflash_ctx *ctx, int32_t w_type, int64_t n_in, int64_t n_out);
 
 // ---- many rows at once (gemm_rows.hip): the products of a prompt's prefill ----
 // Every row gets the bits the 16-row kernels give it in its own block: dfl_gemm_rows_plan says which of their

@@ -636,12 +636,19 @@ int32_t dfl_gemm_rows(dflash_ctx *ctx, const dfl_rows_plan &p, int32_t w_type, c
     const int ranges = p.by_group ? std::max(1, static_cast<int>(static_cast<int64_t>(a.nb) * a.n_cut / a.total)) : a.n_cut;
     const int most_ranges = p.by_group ? static_cast<int>((static_cast<int64_t>(a.nb) * a.n_cut + a.total - 1) / a.total) + 1 : a.n_cut;
     if (2 * tiles <= ctx->n_cu && ranges > 1) {
-        // The whole-K kernel does the few blocks of a short prompt in one launch, one block after the other past weights it
-        // holds in registers: better than a split with its reduction (two launches) up to about 190 rows of a Q6_K matrix
-        // (2048 -> 5120: 7.7 against 7.1 + 4.9 us for two blocks, 16.7 against 16.1 + 5.4 for eight), 80 of a Q4_K one of
-        // eight super-blocks; Q4_K matrices of more (5120 -> 6144) are the faster split from the second block on.
-        const int whole_most = w_type == DFLASH_TYPE_Q6_K_TILED ? 12 : a.nb <= 8 ? 5 : 0;
-        if (p.twin && a.n_blocks <= whole_most && dfl_whole_takes_blocks(ctx, w_type, n_in, n_out))
+        // The whole-K kernel does the few blocks of a short prompt in one launch, one block after the other: 1.5 us each past
+        // weights it holds unpacked, 4 to 10 us each where a wave has two tiles or two super-blocks and unpacks them again.
+        // The split with its reduction costs 9 to 18 us and then the less per block the smaller the matrix.  Crossing points,
+        // Q4_K and Q6_K alike (whole : split in us, 2 / 4 / 12 blocks, Q4_K):
+        //   held    2048 -> 5120  7.9 : 11.7  10.7 : 16.1  21.9 : 23.3     4096 -> 4096  8.3 : 15.6  11.4 : 19.2  24.4 : 32.9
+        //           2560 -> 2560  6.3 : 11.5   8.0 : 12.5  17.1 : 17.8     4096 -> 2048  8.2 : 13.0  11.0 : 15.0  22.8 : 22.4
+        //           1024 -> 4096  6.6 :  9.2   9.4 : 10.2  21.2 : 17.0     2048 -> 1024  6.3 :  9.5   9.2 :  9.8  20.6 : 11.6
+        //   not     4096 -> 6144 22.1 : 17.9  29.6 : 22.9  (Q6_K 32.5 : 19.5  50.5 : 27.8)
+        //           4096 -> 5120 20.4 : 18.9  27.8 : 20.1  (Q6_K 32.1 : 21.8  49.0 : 24.1), 5120 -> 6144 52.6 : 18.1  69.3 : 23.5
+        // so: twelve blocks for matrices of 80 super-blocks x column tiles or more, four for smaller ones, none where the
+        // weights are not held.
+        const int whole_most = a.nb * a.n_ct >= 80 ? 12 : 4;
+        if (p.twin && a.n_blocks <= whole_most && dfl_whole_holds_weights(ctx, w_type, n_in, n_out))
             return dfl_gemm_whole_blocks(ctx, w_type, w, xf, y, n_in, n_out, n_rows, 0, nullptr, 0, st);
         a.n_split = std::min<int>(ranges, static_cast<int>(ctx->n_cu / tiles));
         size_t off = 0;

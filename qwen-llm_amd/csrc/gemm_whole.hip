@@ -661,9 +661,9 @@ int dfl_whole_kind(const dflash_ctx *ctx, int32_t w_type, int64_t n_in, int64_t 
     return whole_plan(ctx, w_type, n_in, n_out, pair_ffn).kind;
 }
 
-bool dfl_whole_takes_blocks(const dflash_ctx *ctx, int32_t w_type, int64_t n_in, int64_t n_out) {
+bool dfl_whole_holds_weights(const dflash_ctx *ctx, int32_t w_type, int64_t n_in, int64_t n_out) {
     const WholePlan p = whole_plan(ctx, w_type, n_in, n_out, 0);
-    return p.kind != DFL_XF_NONE && !p.loop;
+    return p.kind != DFL_XF_NONE && !p.loop && p.R == 1 && n_in / DFL_QK_K <= p.ksplit;
 }
 
 int32_t dfl_gemm_whole(dflash_ctx *ctx, int32_t w_type, const void *w, const void *xf, float *y, int64_t n_in, int64_t n_out,

@@ -2,8 +2,8 @@
 are the oracle-checked ones: captured residuals bit for bit.
 
 The row counts are those where a launch changes its shape: two blocks (one of a single row); the whole-K kernel's last
-and the split's first count; tiles of every number of row blocks with a last tile that is not full; several rounds of
-the chip.  K and the column counts bring each kind of cut: 5120 (whole-K slices, twenty super-blocks), 17408 (stream-K
+and the split's first count (64 | 80 rows narrow, 192 | 200 experts); tiles of every number of row blocks with a last
+tile that is not full; several rounds of the chip.  K and the column counts bring each kind of cut: 5120 (whole-K slices, twenty super-blocks), 17408 (stream-K
 ranges that differ from tile group to tile group), 1024 (fewer super-blocks than slices), Q6_K projections, experts
 with one to four blocks per tile."""
 import numpy as np
@@ -22,6 +22,9 @@ SHAPES = {
 }
 SHAPES["experts128"] = (dfl.ModelConfig(n_layers=2, hidden=2048, n_q=16, n_kv=2, head_dim=256, ffn=0, vocab=2048, n_expert=128, n_expert_used=8,
                                         ffn_expert=768, ffn_shared=768), dfl.synth.Q6_K)
+# (Q6_K projections whose weights the whole-K kernel does not hold, two tiles of a super-block or two super-blocks a wave)
+SHAPES["q6k4096"] = (dfl.ModelConfig(n_layers=2, hidden=4096, n_q=32, n_kv=8, head_dim=128, ffn=3072, vocab=2048), dfl.synth.Q6_K)
+SHAPES["q6k5120"] = (dfl.ModelConfig(n_layers=2, hidden=5120, n_q=32, n_kv=8, head_dim=128, ffn=3072, vocab=2048), dfl.synth.Q6_K)
 SHAPES["heads64"] = (dfl.ModelConfig(n_layers=2, hidden=1024, n_q=24, n_kv=2, head_dim=64, ffn=3072, vocab=2048), dfl.synth.Q4_K)
 SHAPES["heads64x12"] = (dfl.ModelConfig(n_layers=2, hidden=1024, n_q=48, n_kv=4, head_dim=64, ffn=3072, vocab=2048), dfl.synth.Q4_K)
 SHAPES["heads256x5"] = (dfl.ModelConfig(n_layers=2, hidden=1280, n_q=5, n_kv=1, head_dim=256, ffn=3072, vocab=2048), dfl.synth.Q4_K)
@@ -34,8 +37,8 @@ def ctx():
     c.close()
 
 
-@pytest.mark.parametrize("rows", [17, 80, 97, 192, 200, 273, 530, 1001])
-@pytest.mark.parametrize("shape", ["experts", "narrow", "wide"])
+@pytest.mark.parametrize("rows", [17, 64, 80, 97, 192, 200, 273, 530, 1001])
+@pytest.mark.parametrize("shape", ["experts", "narrow", "wide", "q6k4096", "q6k5120"])
 def test_many_row_prefill_equals_block_by_block(ctx, shape, rows):
     cfg, attn_type = SHAPES[shape]
     model = dfl.TargetModel(ctx, cfg, dfl.synth_target_weights_device(cfg, 5, "cuda", attn_type=attn_type))
