@@ -112,7 +112,7 @@ def build(verbose: bool = False) -> str:
             failed = True
             sys.stderr.write(f"hipcc failed for {src}:\n{out}\n")
             continue
-        # (the guarded kernels all live in gemm_fewrow.hip: only there is their absence from the remarks a failure)
+        # (a guarded kernel's absence from the remarks is a failure in the file it lives in)
         bad = check_no_scratch(raw, NO_SCRATCH_BY_FILE.get(os.path.basename(src), ()))
         if bad:
             failed = True

@@ -55,11 +55,6 @@ constexpr int attn_vmcnt(int n) { return ((n & 0xF) | ((n & 0x30) << 10)) | 0x00
 // eight key rows one MFMA operand read touches at a time land in eight different bank groups
 __device__ __forceinline__ int attn_swz(int r) { return (r & 3) | ((r >> 1) & 4); }
 
-// One workgroup = one KV head x one contiguous chunk of keys; wave w = query head w of the GQA
-// group.  Stage = 32 keys: the K tile [32 keys][HD] and the V^T tile [HD dims][32 keys] are copied
-// global -> LDS with direct-to-LDS loads into a ring of kAttnBufs buffers, so the whole group
-// shares one copy and the loads of the next stages are in flight while one is consumed.
-// MAXW = most waves a workgroup may have; it sets the register budget.
 // Keys per KV split for n_pos visible positions: an even share of `want` splits, rounded up to
 // whole 32-key stages, at least min_chunk.  Host and kernels use the same rule, so a launch whose
 // context length is only known on the device (a captured graph) can size its grid for the largest
@@ -137,13 +132,6 @@ __device__ __forceinline__ void attn_wait(int n) {
     }
 }
 
-// MAXL: most loads a wave issues per stage (2 HD / 16 / waves, rounded up to a power of two).
-// What bounds it is a stage's chain, not its bytes: loads landed, barrier, K fragments, two chains of MFMAs, the
-// maximum over the row's lanes, the exponentials, the second product.  So the scores of stage t + 1 are computed ahead
-// of the softmax of stage t (the matrix cores work under the exponentials), V fragments are asked for ahead of
-// them, the maximum crosses the lanes without LDS, the last stage's special cases stand outside of the others' code, and
-// a load's address is made of one lane part and one uniform part: 16 rows x 100 k keys, 48 / 8 heads of 128, with the
-// merge: 110 -> 99 us (4.1 TB/s of keys and values; a copy reaches 5.07).
 // Splits are merged in order: what came before times `old`, plus the next one's result times `next`.
 struct AttnMerge {
     float m, old, next;
@@ -155,6 +143,18 @@ struct AttnMerge {
     __device__ __forceinline__ float add(float before, float v) const { return __builtin_fmaf(next, v, old * before); }
 };
 
+// One workgroup = one KV head x one contiguous chunk of keys; wave w = query head w of the GQA
+// group.  Stage = 32 keys: the K tile [32 keys][HD] and the V^T tile [HD dims][32 keys] are copied
+// global -> LDS with direct-to-LDS loads into a ring of kAttnBufs buffers, so the whole group
+// shares one copy and the loads of the next stages are in flight while one is consumed.
+// MAXW = most waves a workgroup may have; it sets the register budget.
+// MAXL: most loads a wave issues per stage (2 HD / 16 / waves, rounded up to a power of two).
+// What bounds it is a stage's chain, not its bytes: loads landed, barrier, K fragments, two chains of MFMAs, the
+// maximum over the row's lanes, the exponentials, the second product.  So the scores of stage t + 1 are computed ahead
+// of the softmax of stage t (the matrix cores work under the exponentials), V fragments are asked for ahead of
+// them, the maximum crosses the lanes without LDS, the last stage's special cases stand outside of the others' code, and
+// a load's address is made of one lane part and one uniform part: 16 rows x 100 k keys, 48 / 8 heads of 128, with the
+// merge: 105.9 -> 98.3 us, both trees in turn (4.2 TB/s of keys and values; a copy reaches 5.03).
 // MERGE: the workgroup takes all of its rows' keys, split by split, and merges the splits as it goes (see
 // attn_rows_kernel); else one split, whose partial result it writes.
 template <int HD, typename TQ, int MAXW, int MAXL, bool MERGE>
@@ -678,8 +678,9 @@ __global__ void __launch_bounds__(HD == 64 ? 128 : 256)
     }
 }
 
-// The partial results merged one after the other, as attn_rows_kernel does (which blocks take this: see attn_policy).  What bounds it is its chain: a trip to memory for the maxima and the partial outputs, which
-// are in flight together, then the merges.  Lane s of every wave keeps split s's maximum and sum and computes its two factors
+// The partial results merged one after the other, as attn_rows_kernel does (which blocks take this: see attn_policy).
+// What bounds it is its chain: a trip to memory for the maxima and the partial outputs, which are in flight together,
+// then the merges.  Lane s of every wave keeps split s's maximum and sum and computes its two factors
 // (the maximum of the splits before it is a scan over the lanes); a thread adds up one dim, with the factors read from the lane
 // they are in: no LDS, no barrier.
 constexpr int kOrderedSplits = 32;
@@ -878,11 +879,12 @@ static AttnPolicy attn_policy(const dflash_ctx *ctx, int64_t bucket, int n_kv, i
     // bucket alone.
     // Workgroups per CU the split aims at, in halves.  Short contexts: one (fewer splits, fewer partial tiles to merge).
     // Long contexts: two where two workgroups' LDS rings fit a CU side by side (heads of 64 or 128); with heads of 256 a
-    // ring is 96 KB, a CU holds one workgroup, and a second round of them only halves the chunk: a workgroup's partial
+    // ring is 128 KB, a CU holds one workgroup, and a second round of them only halves the chunk: a workgroup's partial
     // tiles (16 rows x its heads x head_dim floats) are then as many bytes as the keys and values it read.  Half a
     // workgroup per CU there (16 q / 2 kv heads of 256, 40-layer verify: 5.25 -> 4.79 ms at 16 k of context with chunks
-    // of 256 keys instead of 128, 6.21 -> 5.80 ms at 32 k with 512; a quarter measured slower again).
-    const size_t ring_bytes = static_cast<size_t>(3) * 2 * 32 * head_dim * sizeof(_Float16);  // (three buffers' worth: what the figures here were taken with)
+    // of 256 keys instead of 128, 6.21 -> 5.80 ms at 32 k with 512; a quarter measured slower again.  Taken with rings of
+    // three buffers, 96 KB, which share a CU as little.)
+    const size_t ring_bytes = static_cast<size_t>(kAttnBufs) * 2 * 32 * head_dim * sizeof(_Float16);
     int per_cu_x2 = bucket >= 16384 ? (2 * ring_bytes <= static_cast<size_t>(ctx->lds_bytes) ? 4 : 1) : 2;
     int64_t min_chunk = bucket >= 8192 ? 128 : 64;
     // A workgroup serves hw heads of a GQA group (one wave each).  What a workgroup moves is its chunk of K and V,

@@ -226,13 +226,6 @@ void rms_norm(int rows, hipStream_t st, float *x, const float *add, const float 
 #undef DFL_NORM
 }
 
-// kernel_qk_rms_norm_rope_f32_packed_consecutive (attn.metal:137-196) + the f32 -> f16 KV scatter
-// (elementwise.metal:674-685).  One wave per (row, head): per-head RMSNorm (weight may be null),
-// NeoX RoPE over the full head (pairs (i, i + hd/2), angle = pos / theta^(2i/hd)).
-// Heads [0, n_q) are queries (rewritten in place, f32); heads [n_q, n_q+n_kv) are keys, written
-// as f16 into k_dst[pos][kv head][:] (k_dst == null: rewritten in place as f32 instead).
-// With vt_dst, n_kv more workgroups per row scatter the row's V heads, as f16, into column
-// pos[row] of the transposed cache [kv head][dim][capacity].
 // A lane's rotation pairs of one head: pair k is elements (i, i + HD/2), i = lane + 64 k (heads of 64: lanes 0..31).
 template <int HD>
 struct RopePairs {
@@ -285,6 +278,13 @@ struct RopeHead {
     }
 };
 
+// kernel_qk_rms_norm_rope_f32_packed_consecutive (attn.metal:137-196) + the f32 -> f16 KV scatter
+// (elementwise.metal:674-685).  One wave per (row, head): per-head RMSNorm (weight may be null),
+// NeoX RoPE over the full head (pairs (i, i + hd/2), angle = pos / theta^(2i/hd)).
+// Heads [0, n_q) are queries (rewritten in place, f32); heads [n_q, n_q+n_kv) are keys, written
+// as f16 into k_dst[pos][kv head][:] (k_dst == null: rewritten in place as f32 instead).
+// With vt_dst, n_kv more workgroups per row scatter the row's V heads, as f16, into column
+// pos[row] of the transposed cache [kv head][dim][capacity].
 // What bounds it: one trip to memory and the arithmetic of the angles (powf, sincosf), which wait for nothing but the
 // position: they run while the head's values are on their way.
 template <int HD>
