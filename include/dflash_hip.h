@@ -463,7 +463,9 @@ int32_t dflash_restore(dflash_ctx *ctx, dflash_session *session, int64_t start_p
  * is made on the first call that needs it.  Results equal those of the same blocks through dflash_verify_block bit for bit.  Guards
  * as dflash_verify_block; on an error kv_n_pos is unchanged. */
 /* Makes the group buffers - or, for a shape that has none, the extra streams, scratch sets and contexts - of dflash_prefill_blocks
- * ahead of its first call (which makes them otherwise): the allocations then stay out of the first prompt's latency.  No counterpart in the reference. */
+ * ahead of its first call (which makes them otherwise): the allocations then stay out of the first prompt's latency.  A
+ * target whose shape has group buffers and whose tensors are in row order makes its lanes in the first call all the same:
+ * a session does not know its target's tensors.  No counterpart in the reference. */
 int32_t dflash_prefill_prepare(dflash_ctx *ctx, dflash_session *session);
 int32_t dflash_prefill_blocks(dflash_ctx *ctx, const dflash_model *model, dflash_session *session,
                               const int32_t *tokens_host, int32_t n_tokens, int64_t start_position,

@@ -905,7 +905,8 @@ void prefill_group_alloc(dflash_session *s, PrefillGroup *g) {
     const bool moe = c.n_expert > 0;
     const int used = c.n_expert_used < c.n_expert ? c.n_expert_used : c.n_expert;
     const size_t H = c.hidden, q_dim = static_cast<size_t>(c.n_q) * c.head_dim, kv_dim = static_cast<size_t>(c.n_kv) * c.head_dim, F = moe ? 0 : c.ffn;
-    if (blocks < 2 || H % DFL_QK_K || H > 8192 || q_dim % DFL_QK_K) return;
+    // (heads whose K or V rows are not whole tile groups cannot lie side by side in the tiled order: see prefill_group_takes)
+    if (blocks < 2 || H % DFL_QK_K || H > 8192 || q_dim % DFL_QK_K || kv_dim % DFL_QK_K) return;
     if (moe && (c.n_expert > 256 || used < 1 || c.ffn_expert % DFL_QK_K)) return;
     if (!moe && (F < 1 || F % DFL_QK_K)) return;
     int rows = 16 * blocks;

@@ -102,3 +102,21 @@ def test_prefill_equals_block_by_block_with_sums_past_f16(ctx, shape, where):
     assert torch.equal(got, want)
     one.close()
     many.close()
+
+
+@pytest.mark.parametrize("shape", ["narrow", "experts", "heads64"])
+def test_a_prepared_session_allocates_nothing_for_its_first_prompt(ctx, shape):
+    """dflash_prefill_prepare makes what the first prompt needs: a group's buffers, or the lanes of a shape (heads64: K and
+    V rows of half a tile group) that the grouped pass cannot take."""
+    cfg, attn_type = SHAPES[shape]
+    model = dfl.TargetModel(ctx, cfg, dfl.synth_target_weights_device(cfg, 5, "cuda", attn_type=attn_type))
+    for i in range(2):  # (the first session has the runtime load the kernels, which takes memory of its own)
+        sess = dfl.Session(ctx, model, 160, [0, 1])
+        sess.prepare_prefill()
+        torch.cuda.synchronize()
+        free = torch.cuda.mem_get_info()[0]
+        sess.prefill_blocks(list(range(130)), 0, want_hidden=False)
+        torch.cuda.synchronize()
+        taken = free - torch.cuda.mem_get_info()[0]
+        sess.close()
+    assert taken == 0
