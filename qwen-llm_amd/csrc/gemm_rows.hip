@@ -3,21 +3,27 @@
 // Same contraction as encode_mat_mat_dispatch_dflash_verify (metal_forward/dispatch.rs:365-378).
 //
 // What bounds it.  With sixteen rows a weight is unpacked for one MFMA and the kernel streams weights; here a weight
-// unpacked once serves up to 128 rows, and the matrix cores are what there is most of to do.  A workgroup of eight waves
-// computes 16 RB rows x 256 columns (a SwiGLU pair: 128 gate and the 128 up columns that go with them); a wave, 16 RB rows
-// x 32 columns:
-//   * per super-block of K the activations of its row blocks (8 KB each) and the raw quant blocks of its 16-row weight
-//     tiles are copied into LDS with direct-to-LDS loads, both as they lie in memory (contiguous pieces), the weights a
-//     super-block ahead, the activations half a super-block;
+// unpacked once serves up to 128 rows, and the matrix cores are what there is most of to do: a wave's 2 MFMAs per
+// fragment, with the fragment's LDS read and its share of the unpacking (4 vector instructions), run at 1.5 PFLOP/s where
+// nothing else stands in the way (random operands, clock held down to 1.6 GHz by the power they draw; the MFMAs alone 2.0).
+// A workgroup of eight waves computes 16 RB rows x 256 columns (a SwiGLU pair: 128 gate and the 128 up columns that go with
+// them); a wave, 16 RB rows x 32 columns:
+//   * the activations of its row blocks (half a super-block at a time, three halves in LDS) and the raw quant blocks of its
+//     own two 16-row weight tiles (one super-block) are copied into LDS with direct-to-LDS loads, both as they lie in memory
+//     (contiguous pieces: weights loaded straight into registers touch eighteen lines a load and cost 10 %), the activations
+//     one to two halves ahead, the weights one super-block;
+//   * the copies stand one by one between the products, and an LDS read six products ahead of its own: a wave that issues a
+//     super-block's copies together stands still until the memory pipeline has taken them;
 //   * no two waves unpack the same weights (with the waves two by four, which halves the LDS reads, the unpacking on the
 //     vector ALU took as long as the products); an activation fragment read from LDS feeds two products;
 //   * the weights stay quantised up to the registers: a matrix is read from memory once and from L2 once per row tile, at
 //     4.5 or 6.6 bits a weight instead of 16.
 // Workgroups that share weights are dispatched to one XCD (rows_linear), so that a matrix passes through one L2.
-// Measured for 2032 rows (four blocks per pass through the 16-row kernels before): 5120 -> 2 x 17408 with SwiGLU 795 us
-// (0.92 PFLOP/s; 30 us per block before), 17408 -> 5120 428 us (0.85), 5120 -> 6144 226 us and 4096 -> 5120 175 us (0.57
-// and 0.49: their twin MFMAs, which the block path's bits ask for, are as many again); a 64-layer prompt of 1000 rows
-// 72.6 ms against 292 (65 with the attention's splits merged in registers).
+// Measured for 1000 rows, before (a whole super-block's copies behind a barrier, the compiler's waits: every LDS read waited
+// for ahead of its two products) and now, six layers of a prompt: 5120 -> 2 x 17408 with SwiGLU 429 -> 364 us (0.98
+// PFLOP/s, matrix cores busy for 57 % of the cycles, 42 % before), 17408 -> 5120 233 -> 193 us (0.92), 5120 -> 6144 and 4096 ->
+// 5120 together 240 -> 210 us (0.50: their twin MFMAs, which the block path's bits ask for, are as many again); 2048 rows:
+// 2048 -> 5120 and 4096 -> 2048 in Q6_K together 220 -> 186 us.  A 64-layer prompt of 1000 rows 64.7 -> 59.7 ms.
 // The experts' tiles (a list, mostly one to four row blocks) take workgroups of half the columns, two of them on a CU:
 // each waits for its own weights while the other computes (2 - 4 % of a prompt of 33 - 130 rows).
 //
@@ -91,16 +97,58 @@ __device__ __forceinline__ half8_t splat8(_Float16 v) {
     return r;
 }
 
-// One tile's raw weights of one super-block in a lane's registers; operand<H>(t) is that of MFMA 4 H + t.
+template <int I, int N, typename F>
+__device__ __forceinline__ void static_for(F &&f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>());
+        static_for<I + 1, N>(f);
+    }
+}
+
+// Reads from LDS and the waits for them are asm: the compiler cannot tell LDS reads from the direct-to-LDS loads in flight and
+// waits for every read it has issued (lgkmcnt(0)) ahead of each product.  (The build refuses this kernel if it spills: see build.py.)
+typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+template <typename T, int OFF>
+__device__ __forceinline__ T lds_read(uint32_t at) {
+    T v;
+    if constexpr (sizeof(T) == 16)
+        asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(at), "n"(OFF));
+    else if constexpr (sizeof(T) == 8)
+        asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(v) : "v"(at), "n"(OFF));
+    else
+        asm volatile("ds_read_u16 %0, %1 offset:%2" : "=v"(v) : "v"(at), "n"(OFF));
+    return v;
+}
+// v has arrived, with at most LATER of the reads issued behind it still under way
+template <int LATER>
+__device__ __forceinline__ void lds_arrived(half8_t &v) {
+    asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(v) : "n"(LATER < 15 ? LATER : 15));
+}
+// this wave's loads into LDS but for the last N are done
+template <int N>
+__device__ __forceinline__ void copies_done() {
+    __builtin_amdgcn_s_waitcnt((N & 0xF) | ((N & 0x30) << 10) | 0x0F70);  // vmcnt(N)
+    asm volatile("" ::: "memory");
+}
+
+// One tile's weights of one super-block in a lane's registers: read asks LDS for the lane's quant bytes (kReads reads, there
+// behind arrived), scales makes of them what operand<H>(t), the operand of MFMA 4 H + t, needs besides.
 struct TileQ4 {
-    static constexpr int kBytes = 16 * DFL_Q4_K_BYTES;
-    u32x4_t q0, q1;
+    static constexpr int kBytes = 16 * DFL_Q4_K_BYTES, kReads = 3;
+    struct At {
+        uint32_t hdr, q;
+        __device__ __forceinline__ At(uint32_t tile, int n, int g) : hdr(tile + n * DFL_Q4_K_BYTES), q(hdr + 32 * g) {}
+    };
+    u32x4_t hdr, q0, q1;
     half2_t S, Cs, m;
-    __device__ __forceinline__ void load(const uint8_t *tile, int n, int g, uint32_t sc_sel, bool negate_min) {
-        const u32x4_t *blk = reinterpret_cast<const u32x4_t *>(tile) + n * 9;
-        const u32x4_t hdr = blk[0];
-        q0 = blk[1 + 2 * g];
-        q1 = blk[2 + 2 * g];
+    template <int OFF>
+    __device__ __forceinline__ void read(const At &at) {
+        hdr = lds_read<u32x4_t, OFF>(at.hdr);
+        q0 = lds_read<u32x4_t, OFF + 16>(at.q);
+        q1 = lds_read<u32x4_t, OFF + 32>(at.q);
+    }
+    __device__ __forceinline__ void arrived() { asm volatile("" : "+v"(hdr), "+v"(q0), "+v"(q1)); }
+    __device__ __forceinline__ void scales(int g, uint32_t sc_sel, bool negate_min) {
         const uint32_t upper = 0u - static_cast<uint32_t>(g >> 1);
         const uint32_t sc_lo = hdr.y & 0x3F3F3F3Fu, sc_hi = (hdr.w & 0x0F0F0F0Fu) | ((hdr.y >> 2) & 0x30303030u);
         const uint32_t mn_lo = hdr.z & 0x3F3F3F3Fu, mn_hi = ((hdr.w >> 4) & 0x0F0F0F0Fu) | ((hdr.z >> 2) & 0x30303030u);
@@ -123,21 +171,35 @@ struct TileQ4 {
     __device__ __forceinline__ half8_t twin(int) const {
         return splat8(m[H]);
     }
+    __device__ __forceinline__ half8_t minima() const { return q4k_min_operand(m); }
 };
 
 struct TileQ6 {
-    static constexpr int kBytes = kQ6TileBytes;
+    static constexpr int kBytes = kQ6TileBytes, kReads = 6;
+    struct At {
+        uint32_t ql, ql1, qh, qh1, sc, d;
+        __device__ __forceinline__ At(uint32_t tile, int n, int g)
+            : ql(tile + q6t_ql_piece(n, 2 * g)), ql1(tile + q6t_ql_piece(n, 2 * g + 1)), qh(tile + q6t_qh_piece(n, g & 2)),
+              qh1(tile + q6t_qh_piece(n, (g & 2) + 1)), sc(tile + kQ6TSc + n * 16 + 4 * (g & 2)), d(tile + kQ6TD + n * 2) {}
+    };
     u32x4_t qa, qb, ha, hb;
+    u32x2_t sc;
+    uint32_t d16;
     _Float16 s[4];
     int odd2;
-    __device__ __forceinline__ void load(const uint8_t *tile, int n, int g, uint32_t, bool) {
-        const int h = g >> 1, odd = g & 1;
-        qa = *reinterpret_cast<const u32x4_t *>(tile + q6t_ql_piece(n, 4 * h + 2 * odd));
-        qb = *reinterpret_cast<const u32x4_t *>(tile + q6t_ql_piece(n, 4 * h + 2 * odd + 1));
-        ha = *reinterpret_cast<const u32x4_t *>(tile + q6t_qh_piece(n, 2 * h));
-        hb = *reinterpret_cast<const u32x4_t *>(tile + q6t_qh_piece(n, 2 * h + 1));
-        const uint2 sc = *reinterpret_cast<const uint2 *>(tile + kQ6TSc + n * 16 + 8 * h);
-        const float d = __half2float(__ushort_as_half(*reinterpret_cast<const uint16_t *>(tile + kQ6TD + n * 2)));
+    template <int OFF>
+    __device__ __forceinline__ void read(const At &at) {
+        qa = lds_read<u32x4_t, OFF>(at.ql);
+        qb = lds_read<u32x4_t, OFF>(at.ql1);
+        ha = lds_read<u32x4_t, OFF>(at.qh);
+        hb = lds_read<u32x4_t, OFF>(at.qh1);
+        sc = lds_read<u32x2_t, OFF>(at.sc);
+        d16 = lds_read<uint32_t, OFF>(at.d);
+    }
+    __device__ __forceinline__ void arrived() { asm volatile("" : "+v"(qa), "+v"(qb), "+v"(ha), "+v"(hb), "+v"(sc), "+v"(d16)); }
+    __device__ __forceinline__ void scales(int g, uint32_t, bool) {
+        const int odd = g & 1;
+        const float d = __half2float(__ushort_as_half(static_cast<uint16_t>(d16)));
 #pragma unroll
         for (int j = 0; j < 2; j++) {
             s[j] = static_cast<_Float16>(d * static_cast<float>(static_cast<int8_t>(sc.x >> (16 * odd + 8 * j))));
@@ -158,7 +220,16 @@ struct TileQ6 {
     __device__ __forceinline__ half8_t twin(int t) const {
         return splat8(s[2 * H + (t >> 1)] * static_cast<_Float16>(32.0f));
     }
+    __device__ __forceinline__ half8_t minima() const { return splat8(static_cast<_Float16>(0.0f)); }
 };
+
+// this wave's reads from LDS are done, and everybody has come this far
+__device__ __forceinline__ void landed_for_all() {
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
 
 // Dispatch index -> linear tile index: the hardware deals consecutive workgroups to the eight XCDs in turn, so dispatch
 // indices i, i + 8, i + 16, ... share an L2; they get consecutive tiles.  Returns -1 past the end.
@@ -169,18 +240,25 @@ __device__ __forceinline__ int rows_linear(int dispatch, int count) {
 
 enum { kEpiY = 0, kEpiSwiglu = 1, kEpiSplit = 2 };
 
+// LDS of a tile: three halves of a super-block of its activations (4 KB per row block), two super-blocks of their sub-block
+// sums where the minima go by them, one of every wave's weights.
+template <typename Tile, bool kTwin, int RB, int W>
+struct RowsLds {
+    static constexpr int kHalf = RB * 4096, kSums = kTwin ? 0 : RB * 1024, kW = 2 * Tile::kBytes;
+    static constexpr int sums = 3 * kHalf, w = sums + 2 * kSums, total = w + W * kW;
+};
+
 // kTwin: the minima / offsets through a twin MFMA per activation fragment into a second accumulator (the whole-K
 // kernel's arithmetic); else one MFMA per super-block over the sub-block sums (the streaming and expert kernels').
 // kCut: K is cut somewhere.  RB: 16-row blocks of the tile.
 template <typename Tile, bool kTwin, bool kCut, int RB, int kEpi, bool kList>
-__global__ void __launch_bounds__(64 * (kList ? kListWaves : kRowsWaves)) gemm_rows_kernel(RowsArgs a) {
+__global__ void __launch_bounds__(64 * (kList ? kListWaves : kRowsWaves), 2) gemm_rows_kernel(RowsArgs a) {
     constexpr int W = kList ? kListWaves : kRowsWaves;  // waves, 32 columns each
     constexpr bool kPair = kEpi == kEpiSwiglu, kSplit = kEpi == kEpiSplit, kTotal = kCut && !kSplit;
     constexpr int NSEG = kPair ? 2 : 1, kSegTiles = 2 * W / NSEG;
-    constexpr int kABytes = RB * 4096, kWSeg = kSegTiles * Tile::kBytes, kWBytes = NSEG * kWSeg, kSBytes = kTwin ? 0 : RB * 1024;
-    static_assert(2 * (kABytes + kWBytes + kSBytes) <= 160 * 1024, "one workgroup per CU, all of its LDS");
+    typedef RowsLds<Tile, kTwin, RB, W> Lds;
+    static_assert((kList ? 2 : 1) * Lds::total <= 160 * 1024, "a CU's LDS");
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-    uint8_t *const lds_w = lds + 2 * kABytes, *const lds_s = lds_w + 2 * kWBytes;
     const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
@@ -235,61 +313,26 @@ __global__ void __launch_bounds__(64 * (kList ? kListWaves : kRowsWaves)) gemm_r
 
     // ---- copies into LDS; a wave-load is 64 lanes x 16 bytes, consecutive in memory and in LDS ----
     auto copy = [&](const uint8_t *src, uint8_t *dst) {
-        __builtin_amdgcn_global_load_lds((gptr_t)(src + lane * 16), (lptr_t)(dst), 16, 0, 0);
+        __builtin_amdgcn_global_load_lds((gptr_t)(src + static_cast<uint32_t>(lane * 16)), (lptr_t)(dst), 16, 0, 0);
     };
-    auto issue_x = [&](int b, int h) {  // half h of super-block b: 4 KB per row block (blocks past the end repeat the last one)
-        uint8_t *dst = lds + h * kABytes;
-#pragma unroll
-        for (int j = 0; j < (RB * 4 + W - 1) / W; j++) {
-            const int p = wave + W * j, blk = min(p >> 2, blocks_left - 1);
-            if (RB * 4 % W == 0 || p < RB * 4)
-                copy(xf0 + blk * xf_stride + static_cast<size_t>(b) * 8192 + h * 4096 + (p & 3) * 1024, dst + p * 1024);
-        }
+    // A wave makes the same number of copies in every half of a super-block (where the pieces do not come out even, some copy
+    // what another copies too), so that a constant says how many may still be under way.
+    auto copy_x = [&](auto rows, int half, int slot, int j) {  // half-super-block `half` of `rows` row blocks, this wave's piece j
+        constexpr int R = decltype(rows)::value;
+        const int p = min(wave + W * j, R * 4 - 1), blk = min(p >> 2, blocks_left - 1);  // (blocks past the end repeat the last one)
+        copy(xf0 + blk * xf_stride + static_cast<size_t>(half) * 4096 + (p & 3) * 1024, lds + slot * Lds::kHalf + p * 1024);
     };
-    constexpr int kFull = kWSeg / 1024, kRest = (kWSeg % 1024) / 16;  // whole wave-loads of a segment, lanes of its last one
-    auto issue_w = [&](int b) {
-        uint8_t *dst = lds_w + (b & 1) * kWBytes;
-#pragma unroll
-        for (int s = 0; s < NSEG; s++) {
-            const uint8_t *src = wbase[s] + static_cast<size_t>(b) * 16 * Tile::kBytes;
-#pragma unroll
-            for (int j = 0; j < (kFull + W - 1) / W; j++) {
-                const int p = ((wave + W / 2 * s) & (W - 1)) + W * j;
-                if (p < kFull) copy(src + p * 1024, dst + s * kWSeg + p * 1024);
-            }
-            if (kRest > 0 && wave == W - 1 - s && lane < kRest) copy(src + kFull * 1024, dst + s * kWSeg + kFull * 1024);
-        }
-        if constexpr (!kTwin) {
-            static_assert(RB <= W, "a wave copies one block's sums");
-            if (wave < RB) {
-                const int blk = min(wave, blocks_left - 1);
-                copy(xs0 + blk * xs_stride + static_cast<size_t>(b) * 1024, lds_s + (b & 1) * kSBytes + wave * 1024);
-            }
-        }
+    auto copy_s = [&](auto rows, int b) {
+        constexpr int R = decltype(rows)::value;
+        static_assert(RB <= W, "a wave copies one block's sums");
+        const int blk = min(wave, R - 1);
+        copy(xs0 + min(blk, blocks_left - 1) * xs_stride + static_cast<size_t>(b) * 1024, lds + Lds::sums + (b & 1) * Lds::kSums + blk * 1024);
     };
-    // how many copies issue_w makes in this wave: what may still be in flight when the activations issued before it are needed
-    int w_copies = 0;
-#pragma unroll
-    for (int s = 0; s < NSEG; s++) {
-        const int v = (wave + W / 2 * s) & (W - 1);
-        w_copies += (kFull - v + W - 1) / W + (kRest > 0 && wave == W - 1 - s ? 1 : 0);
-    }
-    if (!kTwin && wave < RB) w_copies++;
-    auto landed = [&](bool weights_in_flight) {  // this wave's copies are in LDS, then everybody's
-        if (!weights_in_flight) {
-            __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0), and its LDS reads (lgkmcnt(0)) before others overwrite what they read
-        } else {
-            switch (w_copies) {  // vmcnt(w_copies), lgkmcnt(0)
-                case 4: __builtin_amdgcn_s_waitcnt(0x0074); break;
-                case 5: __builtin_amdgcn_s_waitcnt(0x0075); break;
-                case 6: __builtin_amdgcn_s_waitcnt(0x0076); break;
-                case 7: __builtin_amdgcn_s_waitcnt(0x0077); break;
-                default: __builtin_amdgcn_s_waitcnt(0x0070); break;
-            }
-        }
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
+    // (a wave-load less than a whole one starts early enough to be one)
+    constexpr int kWRun = kPair ? Tile::kBytes : 2 * Tile::kBytes, kWLoads = (kWRun + 1023) / 1024, kWCopies = NSEG * kWLoads;
+    auto copy_w = [&](int b, int i) {
+        const int s = i / kWLoads, at = min(i % kWLoads * 1024, kWRun - 1024);
+        copy(wbase[s] + static_cast<size_t>(b) * 16 * Tile::kBytes + wave * kWRun + at, lds + Lds::w + wave * Lds::kW + s * Tile::kBytes + at);
     };
 
     const uint32_t sc_sel = (lane & 16) ? 0x04030402u : 0x04010400u;
@@ -307,44 +350,34 @@ __global__ void __launch_bounds__(64 * (kList ? kListWaves : kRowsWaves)) gemm_r
 #pragma unroll
     for (int s = 0; s < NSEG; s++) first[s] = true;
 
-    // A tile with fewer than RB row blocks (an expert's few rows, a prompt's tail) computes those alone, behind uniform
-    // branches that the full tile's code does not have.
     const int live = min(blocks_left, RB);
     Tile tile[2];
-    auto compute = [&](auto half, auto partial, int b) {
-        constexpr int H = decltype(half)::value;
-        constexpr bool kPart = decltype(partial)::value != 0;
-        if constexpr (H == 0) {
-            const uint8_t *wt = lds_w + (b & 1) * kWBytes;
-#pragma unroll
-            for (int j = 0; j < 2; j++) tile[j].load(wt + (kPair ? j * kWSeg + wave * Tile::kBytes : (2 * wave + j) * Tile::kBytes), n, g, sc_sel, !kTwin);
-            if constexpr (!kTwin) {
-                const half8_t *sm = reinterpret_cast<const half8_t *>(lds_s + (b & 1) * kSBytes) + lane;
-                const half8_t m0 = q4k_min_operand(tile[0].m), m1 = q4k_min_operand(tile[1].m);
-#pragma unroll
-                for (int r = 0; r < RB; r++) {
-                    if (kPart && r >= live) break;
-                    const half8_t am = sm[r * 64];
-                    acc[r][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(am, m0, acc[r][0], 0, 0, 0);
-                    acc[r][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(am, m1, acc[r][1], 0, 0, 0);
-                }
-            }
+    const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lptr_t)lds));
+    const typename Tile::At w_at(lds0 + Lds::w + wave * Lds::kW, n, g);
+    // The products of a super-block stand in the order step (the minima, then MFMA 0 to 7 of a tile), row block.  A product's
+    // fragment is read kRing products ahead, the weights of a step are unpacked under the products of the one before, and the
+    // copies stand between the products (a wave that issues many at once waits at the issue and computes nothing meanwhile).
+    // A barrier says that a half has landed for everybody and that everybody has read the one before it; it comes
+    // when the ring still holds kTail fragments, whose products then cover the first reads of the new half.  So what runs
+    // from one such barrier to the same one a super-block later begins with the last kTail products of the super-block before.
+    auto product = [&](auto row, const half8_t &x, const half8_t (&o)[4]) {
+        constexpr int r = decltype(row)::value, z = kTwin ? r : 0;
+        acc[r][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, o[0], acc[r][0], 0, 0, 0);
+        acc[r][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, o[1], acc[r][1], 0, 0, 0);
+        if constexpr (kTwin) {
+            sub[z][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, o[2], sub[z][0], 0, 0, 0);
+            sub[z][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, o[3], sub[z][1], 0, 0, 0);
         }
-        const half8_t *xa = reinterpret_cast<const half8_t *>(lds + H * kABytes) + lane;
+    };
+    auto operands = [&](auto st, half8_t (&o)[4]) {  // the weights of a step, and their twins
+        constexpr int step = decltype(st)::value - (kTwin ? 0 : 1);
 #pragma unroll
-        for (int t = 0; t < 4; t++) {
-            const half8_t b0 = tile[0].template operand<H>(t, magic), b1 = tile[1].template operand<H>(t, magic);
-#pragma unroll
-            for (int r = 0; r < RB; r++) {
-                if (kPart && r >= live) break;
-                const half8_t af = xa[r * 256 + t * 64];
-                acc[r][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af, b0, acc[r][0], 0, 0, 0);
-                acc[r][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af, b1, acc[r][1], 0, 0, 0);
-                if constexpr (kTwin) {
-                    constexpr int z = kTwin ? 1 : 0;
-                    sub[z * r][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af, tile[0].template twin<H>(t), sub[z * r][0], 0, 0, 0);
-                    sub[z * r][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af, tile[1].template twin<H>(t), sub[z * r][1], 0, 0, 0);
-                }
+        for (int j = 0; j < 2; j++) {
+            if constexpr (step < 0) {
+                o[j] = tile[j].minima();
+            } else {
+                o[j] = tile[j].template operand<step / 4>(step % 4, magic);
+                if (kTwin) o[2 + j] = tile[j].template twin<step / 4>(step % 4);
             }
         }
     };
@@ -352,7 +385,7 @@ __global__ void __launch_bounds__(64 * (kList ? kListWaves : kRowsWaves)) gemm_r
         if constexpr (kTwin) return acc[r][j] - sub[kTwin ? r : 0][j];
         return acc[r][j];
     };
-    auto store_y = [&](float *y, int r, int j, float4_t v) {
+    auto store_y = [&](float *y, int r, int j, float4_t v) __attribute__((always_inline)) {
         if (r >= live) return;
         const int64_t row0 = static_cast<int64_t>(block0 + r) * 16 + 4 * g;
         const int col = (tile0[0] + 2 * wave + j) * 16 + n;
@@ -362,7 +395,7 @@ __global__ void __launch_bounds__(64 * (kList ? kListWaves : kRowsWaves)) gemm_r
                 if (kList || kSplit || row0 + i < a.n_rows) y[(row0 + i) * a.n_out + col] = v[i];
         }
     };
-    auto fold = [&](int s) {  // the range that ends here joins the total of segment s (kSplit: goes to memory by itself)
+    auto fold = [&](int s) __attribute__((always_inline)) {  // the range that ends here joins the total of segment s (kSplit: goes to memory by itself)
         float *py = kSplit ? a.y + static_cast<size_t>(cut[0].wg - cut[0].first) * a.n_blocks * 16 * a.n_out : nullptr;
 #pragma unroll
         for (int r = 0; r < RB; r++)
@@ -382,37 +415,183 @@ __global__ void __launch_bounds__(64 * (kList ? kListWaves : kRowsWaves)) gemm_r
         first[s] = false;
     };
 
-    auto walk_k = [&](auto partial) {
-        for (int b = b_begin; b < b_end; b++) {
-            landed(false);
-            issue_x(b, 1);
-            const bool more = b + 1 < b_end;
-            if (more) issue_w(b + 1);
-            compute(std::integral_constant<int, 0>(), partial, b);
-            landed(more);
-            if (more) issue_x(b + 1, 0);
-            compute(std::integral_constant<int, 1>(), partial, b);
-            if constexpr (kCut) {
+    auto walk_k = [&](auto rows) __attribute__((always_inline)) {
+        constexpr int R = decltype(rows)::value, kFirst = kTwin ? 0 : 1, kSteps = 8 + kFirst, N = kSteps * R, kMid = (4 + kFirst) * R;
+        constexpr int kRing = kTwin ? 4 : R == 1 || R == 3 ? 3 : R == 5 || R == 7 ? R : 6;  // (divides N: a fragment's place is its product's index)
+        constexpr int kTail = kRing - kRing / 2, kTail0 = (N - kTail) / R, kTailSteps = kSteps - kTail0;
+        constexpr int kX = (R * 4 + W - 1) / W, kEarly = kWCopies + kX, kLate = kFirst + kX;  // copies in the first part and in the second
+        constexpr int kSwitch = kMid - kTail, kEnd = N - kTail;  // the barriers stand ahead of these products
+        // The next weights are read ahead of this one: into the registers of the present ones where all of those are unpacked by
+        // then (the last step's are while the step before it begins), else into others.
+        constexpr bool kInPlace = R > 2;
+        constexpr int kReadW = kInPlace && kEnd - 1 - kRing < (kSteps - 2) * R ? (kSteps - 2) * R : kEnd - 1 - kRing;
+        static_assert(N % kRing == 0 && kReadW >= kSwitch && kReadW < kEnd, "shape of the pipeline");
+        half8_t ring[kRing], tail[kTailSteps][4];
+        // fragments asked for ahead of the wait of product i
+        struct Reads {
+            static constexpr int upto(int i) { return i < kSwitch ? (i + kRing < kMid ? i + kRing : kMid) : i + kRing < N ? i + kRing : N; }
+            static constexpr int later(int i) {
+                return upto(i) - i - 1 + (i >= kReadW && i < upto(kReadW) ? 2 * Tile::kReads : 0);
+            }
+        };
+        auto body = [&](int b, int ahead, int slot) __attribute__((always_inline)) {
+            const int slot1 = slot == 2 ? 0 : slot + 1, slot2 = slot1 == 2 ? 0 : slot1 + 1;
+            const uint32_t at_s = lds0 + Lds::sums + (b & 1) * Lds::kSums + lane * 16;
+            const uint32_t at0 = lds0 + slot * Lds::kHalf + lane * 16, at1 = lds0 + slot1 * Lds::kHalf + lane * 16;
+            auto read = [&](auto i) {
+                constexpr int I = decltype(i)::value, step = I / R - kFirst, r = I % R;
+                if constexpr (step < 0)
+                    ring[I % kRing] = lds_read<half8_t, r * 1024>(at_s);
+                else if constexpr (step < 4)
+                    ring[I % kRing] = lds_read<half8_t, r * 4096 + step * 1024>(at0);
+                else
+                    ring[I % kRing] = lds_read<half8_t, r * 4096 + (step - 4) * 1024>(at1);
+            };
+            // first part: the next super-block's weights, then its first half's activations; second: its sums and its second half's
+            auto copies = [&](auto i) {
+                constexpr int I = decltype(i)::value;
+                if constexpr (I < kSwitch) {
+                    constexpr int at = I + kTail;
+                    static_for<at * kEarly / kMid, (at + 1) * kEarly / kMid>([&](auto c) {
+                        constexpr int C = decltype(c)::value;
+                        if constexpr (C < kWCopies)
+                            copy_w(ahead, C);
+                        else
+                            copy_x(rows, 2 * ahead, slot2, C - kWCopies);
+                    });
+                } else {
+                    constexpr int at = I - kSwitch;
+                    static_for<at * kLate / (N - kMid), (at + 1) * kLate / (N - kMid)>([&](auto c) {
+                        constexpr int C = decltype(c)::value;
+                        if constexpr (C < kFirst)
+                            copy_s(rows, ahead);
+                        else
+                            copy_x(rows, 2 * ahead + 1, slot, C - kFirst);
+                    });
+                }
+            };
+            half8_t op[4], op_next[4];
+            Tile next[2];
+            static_for<0, kTail>([&](auto t) {  // what is left of the super-block before
+                constexpr int I = decltype(t)::value - kTail, P = N + I;
+                static_for<(I == -kTail ? 0 : Reads::upto(I - 1)), Reads::upto(I)>(read);
+                copies(std::integral_constant<int, I>());
+                product(std::integral_constant<int, P % R>(), ring[P % kRing], tail[P / R - kTail0]);
+                if constexpr (I == -kTail) {
 #pragma unroll
-                for (int s = 0; s < NSEG; s++) {
-                    if constexpr (kSplit) {  // (the range's own number is needed before it moves on)
-                        if (b + 1 == cut[s].next || !more) {
+                    for (int j = 0; j < 2; j++) tile[j].scales(g, sc_sel, !kTwin);
+                    operands(std::integral_constant<int, 0>(), op);
+                }
+            });
+            if constexpr (kCut) {
+                // (no register waits for LDS where the code branches: the compiler may copy one there)
+                __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+#pragma unroll
+                for (int i = 0; i < kRing; i++) asm volatile("" : "+v"(ring[i]));
+                if (b > b_begin) {
+#pragma unroll
+                    for (int s = 0; s < NSEG; s++) {
+                        if constexpr (kSplit) {  // (the range's own number is needed before it moves on)
+                            if (b == cut[s].next) {
+                                fold(s);
+                                (void)cut[s].at(b, a);
+                            }
+                        } else if (cut[s].at(b, a)) {
                             fold(s);
-                            if (more) (void)cut[s].at(b + 1, a);
                         }
-                    } else if (more && cut[s].at(b + 1, a)) {
-                        fold(s);
                     }
                 }
             }
+            static_for<0, kEnd>([&](auto i) {
+                constexpr int I = decltype(i)::value, step = I / R, r = I % R;
+                if constexpr (r == 0 && step + 1 < kSteps && !(kInPlace && I > kReadW)) operands(std::integral_constant<int, step + 1>(), op_next);
+                if constexpr (I == kSwitch) {  // the second half is in LDS for everybody, and everybody has read the first
+                    copies_done<kEarly>();
+                    landed_for_all();
+                }
+                static_for<Reads::upto(I - 1), Reads::upto(I)>(read);
+                if constexpr (I == kReadW) {  // (the weights were the first copies of this super-block)
+                    copies_done<kX + (I - kSwitch) * kLate / (N - kMid)>();
+                    if constexpr (kInPlace) {
+                        static_for<kTail0, kSteps>([&](auto st) { operands(st, tail[decltype(st)::value - kTail0]); });
+#pragma unroll
+                        for (int q = 0; q < kTailSteps; q++)
+#pragma unroll
+                            for (int j = 0; j < (kTwin ? 4 : 2); j++) asm volatile("" : "+v"(tail[q][j]));
+                    }
+                    (kInPlace ? tile : next)[0].template read<0>(w_at);
+                    (kInPlace ? tile : next)[1].template read<Tile::kBytes>(w_at);
+                }
+                copies(i);
+                lds_arrived<Reads::later(I)>(ring[I % kRing]);
+                if constexpr (kInPlace && step >= kTail0 && I >= kReadW)
+                    product(std::integral_constant<int, r>(), ring[I % kRing], tail[step - kTail0]);
+                else
+                    product(std::integral_constant<int, r>(), ring[I % kRing], op);
+                if constexpr (r == R - 1) {
+#pragma unroll
+                    for (int j = 0; j < 4; j++) op[j] = op_next[j];
+                }
+            });
+            if constexpr (!kInPlace) static_for<kTail0, kSteps>([&](auto st) { operands(st, tail[decltype(st)::value - kTail0]); });
+            copies_done<kX>();  // all but the second half's activations
+            landed_for_all();
+#pragma unroll
+            for (int i = 0; i < kRing; i++) asm volatile("" : "+v"(ring[i]));
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                (kInPlace ? tile : next)[j].arrived();
+                if (!kInPlace) tile[j] = next[j];
+            }
+        };
+#pragma unroll
+        for (int i = 0; i < kWCopies; i++) copy_w(b_begin, i);
+        if constexpr (!kTwin) copy_s(rows, b_begin);
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+            for (int j = 0; j < kX; j++) copy_x(rows, 2 * b_begin + h, h, j);
+        copies_done<0>();
+        tile[0].template read<0>(w_at);
+        tile[1].template read<Tile::kBytes>(w_at);
+        landed_for_all();
+        tile[0].arrived();
+        tile[1].arrived();
+        const half8_t none = splat8(static_cast<_Float16>(0.0f));  // (nothing is left of the super-block before the first)
+#pragma unroll
+        for (int i = 0; i < kRing; i++) ring[i] = none;
+#pragma unroll
+        for (int i = 0; i < kTailSteps; i++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) tail[i][j] = none;
+        int slot = 0;
+        for (int b = b_begin; b < b_end; b++) {
+            body(b, min(b + 1, b_end - 1), slot);  // (the last one copies itself again, to where nobody reads any more)
+            slot = slot == 0 ? 2 : slot - 1;
         }
+        static_for<N - kTail, N>([&](auto i) {
+            constexpr int P = decltype(i)::value;
+            product(std::integral_constant<int, P % R>(), ring[P % kRing], tail[P / R - kTail0]);
+        });
+        if constexpr (kSplit) fold(0);
+        copies_done<0>();  // (the epilogue has other uses for LDS, and the next workgroup too)
     };
-    issue_x(b_begin, 0);
-    issue_w(b_begin);
-    if (blocks_left >= RB)
-        walk_k(std::integral_constant<int, 0>());
-    else
-        walk_k(std::integral_constant<int, 1>());
+    // An expert's few rows are computed alone, by code of their own; a tail of no more than half the tile's blocks as half a tile.
+    if constexpr (kList) {
+        switch (live) {
+            case 1: walk_k(std::integral_constant<int, 1>()); break;
+            case 2: walk_k(std::integral_constant<int, 2>()); break;
+            case 3: walk_k(std::integral_constant<int, 3>()); break;
+            default: walk_k(std::integral_constant<int, RB>()); break;
+        }
+        static_assert(!kList || RB == 4, "a list's tiles");
+    } else {
+        constexpr int kHalf = RB > 2 ? (RB + 1) / 2 : RB;
+        if (live <= kHalf)
+            walk_k(std::integral_constant<int, kHalf>());
+        else if constexpr (kHalf < RB)
+            walk_k(std::integral_constant<int, RB>());
+    }
     if constexpr (kSplit) return;
     if constexpr (kTotal) {
 #pragma unroll
@@ -510,11 +689,6 @@ __global__ void __launch_bounds__(64) xf_sums_kernel(const uint8_t *__restrict__
     reinterpret_cast<half8_t *>(xs + (static_cast<size_t>(blk) * nb + b) * 1024)[lane] = r;
 }
 
-template <typename Tile, bool kTwin, int RB, int W>
-constexpr size_t rows_lds() {
-    return 2 * (static_cast<size_t>(RB) * 4096 + static_cast<size_t>(2 * W) * Tile::kBytes + (kTwin ? 0 : static_cast<size_t>(RB) * 1024));
-}
-
 }  // namespace
 
 dfl_rows_plan dfl_gemm_rows_plan(const dflash_ctx *ctx, int32_t w_type, int64_t n_in, int64_t n_out, int64_t pair_ffn) {
@@ -555,7 +729,7 @@ template <typename Tile, bool kTwin, bool kCut, int RB, int kEpi, bool kList>
 int32_t rows_launch(dflash_ctx *ctx, const RowsArgs &a, int64_t tiles, hipStream_t st) {
     const auto fn = gemm_rows_kernel<Tile, kTwin, kCut, RB, kEpi, kList>;
     constexpr int W = kList ? kListWaves : kRowsWaves;
-    const size_t lds = rows_lds<Tile, kTwin, RB, W>();
+    const size_t lds = RowsLds<Tile, kTwin, RB, W>::total;
     if (const int32_t rc = dfl_raise_lds_limit(ctx, reinterpret_cast<const void *>(fn), lds)) return rc;
     if (tiles < 1 || tiles > 0x0fffffff) return dfl_fail(ctx, DFLASH_ERR_BAD_SHAPE, "gemm_rows: %lld tiles", static_cast<long long>(tiles));
     dfl_timed timer(ctx, st, DFL_T_GEMM);

@@ -51,6 +51,13 @@ def test_many_row_prefill_equals_block_by_block(ctx, shape, rows):
     many.close()
 
 
+@pytest.mark.parametrize("rows", [33, 49, 113, 129, 161, 225, 305, 369, 481])
+@pytest.mark.parametrize("shape", ["experts", "narrow", "wide", "q6k4096"])
+def test_last_row_tiles_of_every_fill_equal_block_by_block(ctx, shape, rows):
+    """3 to 31 blocks: last row tiles of up to half their blocks (computed as half a tile), of more, and of a single row."""
+    test_many_row_prefill_equals_block_by_block(ctx, shape, rows)
+
+
 @pytest.mark.parametrize("head,rows", [(7, 40), (245, 33), (480, 400), (1000, 530), (1000, 1100)])
 @pytest.mark.parametrize("shape", ["narrow", "experts", "heads64", "heads64x12", "heads256x5"])
 def test_continued_prefill_equals_block_by_block(ctx, shape, head, rows):
