@@ -12,7 +12,7 @@
 //    (the block's rows are exactly the 16-wide side of v_mfma_f32_16x16x32_f16).
 //  * K and V stream HBM -> LDS once per workgroup in stages of 32 keys (direct-to-LDS loads into a
 //    ring of buffers, the next stages in flight while one is consumed), so the group's heads share
-//    one copy; the K tile is bank-swizzled on the way in so that MFMA operand reads are conflict-free.
+//    one copy; both tiles are bank-swizzled on the way in so that MFMA operand reads are conflict-free.
 //  * scores are computed transposed, S^T = K . Q^T: K rows are the A operand, Q^T stays in
 //    registers for the whole kernel (pre-multiplied by scale*log2(e), rounded to f16 as the
 //    reference's decode kernel does, attn_v4.metal:20-31).  The result leaves every lane holding
@@ -51,9 +51,15 @@ constexpr int kAttnBufs = 4;  // LDS ring: two stages in flight, the one whose s
 // s_waitcnt vmcnt(n) lgkmcnt(0) (gfx9 encoding)
 constexpr int attn_vmcnt(int n) { return ((n & 0xF) | ((n & 0x30) << 10)) | 0x0070; }
 
-// bank swizzle of the K tile: 16-byte chunk j of key row r sits at chunk j ^ swz(r), so that the
-// eight key rows one MFMA operand read touches at a time land in eight different bank groups
-__device__ __forceinline__ int attn_swz(int r) { return (r & 3) | ((r >> 1) & 4); }
+// LDS reads sixteen lanes of 16 bytes a clock (64 banks of 4 bytes) when they fall into sixteen different sixteenths of 256
+// bytes.  K: 16-byte chunk j of key row r sits at chunk j ^ swz(r): the sixteen lanes of an MFMA operand read rows 8 (n >> 2) +
+// (n & 3) at the same j, whole multiples of 256 bytes apart from heads of 128 on (sixteen values; heads of 64 have eight
+// chunks a row, two rows to 256 bytes, and eight values do).  V^T: chunk g of dim d sits at g ^ ((d >> 1) & 3): the lanes read
+// sixteen dims, 64 bytes apart, at the same g.  Measured, reads of this pattern: 222 bytes a clock and CU (124 with eight values
+// for K and V as it comes; contiguous lanes 217).
+template <int CH>
+__device__ __forceinline__ int attn_swz(int r) { return (r & 3) | ((r >> 1) & (CH >= 16 ? 12 : 4)); }
+__device__ __forceinline__ int attn_swz_v(int d) { return (d >> 1) & 3; }
 
 // Keys per KV split for n_pos visible positions: an even share of `want` splits, rounded up to
 // whole 32-key stages, at least min_chunk.  Host and kernels use the same rule, so a launch whose
@@ -217,8 +223,8 @@ __device__ __forceinline__ void attn_body(const TQ *__restrict__ q, const _Float
     // lane's part is the same for every load but for the swizzle, whose bits of the first row are one more xor.
     constexpr int kRowsPerLoad = 64 / CH;
     const int sub = lane / CH;
-    const uint32_t k_row = static_cast<uint32_t>(sub) * static_cast<uint32_t>(kv_dim) * 2, k_chunk = ((lane % CH) ^ attn_swz(sub)) * 16;
-    const uint32_t v_off = static_cast<uint32_t>(lane >> 2) * static_cast<uint32_t>(vt_stride) * 2 + 16 * (lane & 3);
+    const uint32_t k_row = static_cast<uint32_t>(sub) * static_cast<uint32_t>(kv_dim) * 2, k_chunk = ((lane % CH) ^ attn_swz<CH>(sub)) * 16;
+    const uint32_t v_off = static_cast<uint32_t>(lane >> 2) * static_cast<uint32_t>(vt_stride) * 2 + 16 * ((lane & 3) ^ attn_swz_v(lane >> 2));
     int issued = 0;
     auto issue_stage = [&]() {
         half8_t *buf = lds + (issued % kAttnBufs) * (2 * kKPieces);
@@ -232,7 +238,7 @@ __device__ __forceinline__ void attn_body(const TQ *__restrict__ q, const _Float
             const uint8_t *src;
             if (qd * 64 < kKPieces) {
                 const int row0 = qd * kRowsPerLoad;
-                uint32_t o = k_row + (k_chunk ^ static_cast<uint32_t>(attn_swz(row0) * 16));
+                uint32_t o = k_row + (k_chunk ^ static_cast<uint32_t>(attn_swz<CH>(row0) * 16));
                 if (rows_left < 32) o -= static_cast<uint32_t>(max(row0 + sub - (rows_left - 1), 0)) * static_cast<uint32_t>(kv_dim) * 2;
                 src = ksrc + static_cast<int64_t>(row0) * kv_dim * 2 + static_cast<int32_t>(o);
             } else {
@@ -294,7 +300,7 @@ __device__ __forceinline__ void attn_body(const TQ *__restrict__ q, const _Float
         const half8_t *kt = lds + (st % kAttnBufs) * (2 * kKPieces);
 #pragma unroll
         for (int T = 0; T < 2; T++) {
-            const int r = rk0 + 4 * T, sw = attn_swz(r);
+            const int r = rk0 + 4 * T, sw = attn_swz<CH>(r);
             sc[T] = float4_t{0, 0, 0, 0};
 #pragma unroll
             for (int s = 0; s < KS; s++) sc[T] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kt[r * CH + ((4 * s + g) ^ sw)], qf[s], sc[T], 0, 0, 0);
@@ -329,7 +335,7 @@ __device__ __forceinline__ void attn_body(const TQ *__restrict__ q, const _Float
         }
         half8_t vf[DT];
 #pragma unroll
-        for (int t = 0; t < DT; t++) vf[t] = vt[(16 * t + n) * 4 + g];
+        for (int t = 0; t < DT; t++) vf[t] = vt[(16 * t + n) * 4 + (g ^ attn_swz_v(n))];
         const bool masked = !(key0 >= all_lo && key0 + 31 <= all_hi);  // uniform: some key of this step is hidden from some row
         float p[8];
 #pragma unroll
