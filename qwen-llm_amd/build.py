@@ -29,7 +29,7 @@ FLAGS = [
 NO_SCRATCH_BY_FILE = {
     "gemm_fewrow.hip": ("gemm_q4k_stream_kernel", "gemm_q4k_slab_kernel", "gemm_q4k_tiled_kernel", "gemm_q4k_experts_kernel",
                         "gemm_q6k_stream_kernel"),
-    "attn_verify.hip": ("attn_split_kernel", "attn_rows_kernel"),
+    "attn_verify.hip": ("attn_split_kernel", "attn_rows_kernel", "attn_rows_pair_kernel"),
     "gemm_rows.hip": ("gemm_rows_kernel",),
 }
 NO_SCRATCH_KERNELS = tuple(k for kernels in NO_SCRATCH_BY_FILE.values() for k in kernels)

@@ -25,6 +25,7 @@
 //    skipped while no row's maximum moves, and stages every row sees in full skip the mask.
 //  * each workgroup writes (m, l, O) partials; a second small kernel merges the splits.
 #include "common.h"
+#include "lds_read.h"
 
 #include <cmath>
 #include <algorithm>
@@ -148,6 +149,24 @@ struct AttnMerge {
     }
     __device__ __forceinline__ float add(float before, float v) const { return __builtin_fmaf(next, v, old * before); }
 };
+
+// A lane's dims 16 t + 4 g + i of row n, as f16 in fragment order: it has four dims of an octet, the lane 16 away the other
+// four; even lane rows take tile t's octets, odd ones tile t + 1's.
+template <int DT>
+__device__ __forceinline__ void attn_store_xf(float4_t (&tot)[DT], void *out_xf, int kind, int n, int g, int dim0, bool live) {
+#pragma unroll
+    for (int t = 0; t < DT; t += 2) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            float lo = tot[t][i], hi = tot[t + 1][i];
+            dfl_swap16(lo, hi);
+            tot[t][i] = lo;
+            tot[t + 1][i] = hi;
+        }
+        const float4_t a = tot[t], b = tot[t + 1];
+        if (live) dfl_xf_store(out_xf, kind, n, dim0 + 16 * (t + (g & 1)) + 8 * (g >> 1), a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]);
+    }
+}
 
 // One workgroup = one KV head x one contiguous chunk of keys; wave w = query head w of the GQA
 // group.  Stage = 32 keys: the K tile [32 keys][HD] and the V^T tile [HD dims][32 keys] are copied
@@ -423,20 +442,7 @@ __device__ __forceinline__ void attn_body(const TQ *__restrict__ q, const _Float
         }
         if (out_xf) {
             out_xf = static_cast<uint8_t *>(out_xf) + block * xf_stride;
-            // a lane has four dims of an octet, the lane 16 away the other four: even lane rows take tile t's, odd ones tile t + 1's
-#pragma unroll
-            for (int t = 0; t < DT; t += 2) {
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    float lo = tot[t][i], hi = tot[t + 1][i];
-                    dfl_swap16(lo, hi);
-                    tot[t][i] = lo;
-                    tot[t + 1][i] = hi;
-                }
-                const float4_t a = tot[t], b = tot[t + 1];
-                if (n < n_rows)
-                    dfl_xf_store(out_xf, out_xf_kind, n, head * HD + 16 * (t + (g & 1)) + 8 * (g >> 1), a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]);
-            }
+            attn_store_xf<DT>(tot, out_xf, out_xf_kind, n, g, head * HD, n < n_rows);
         }
         return;
     }
@@ -492,6 +498,274 @@ __global__ void __launch_bounds__(512)
     }
     attn_body<HD, float, 8, MAXL, true>(q, k_cache, vt_cache, nullptr, nullptr, ctx_len, nullptr, n_rows_total, n_q, n_kv, vt_stride, want, min_chunk,
                                         scale, 0, 0, 1, 0, block, out, out_xf, out_xf_kind, xf_stride);
+}
+
+// The same for heads of 256, whose splits are merged by attn_combine_few_kernel: every eighth split after the other, times
+// 2^(m_s - m*), then the eight sums in turn.  That order asks for the maximum m* over all splits ahead of the first sum: the keys
+// are walked twice, the first time for the scores' maxima alone, the second time split by split in the merge's order.
+// Splits are of 64 keys, two stages (the host's rule): both stages' probabilities are there before the first value is
+// multiplied, so that a tile of 16 dims goes through its two products, the rescale between them and the merge in four
+// registers, and beside the queries a lane keeps one sum.
+// LDS: three 64-key tiles of K for the first walk; for the second two splits of K and V, the first of them behind the
+// three tiles (it is asked for while the first walk ends), the other in the place of two of them.
+// What bounds it: a wave's products (96 MFMAs a split) and vector work (270 instructions) stand mostly one behind the other, 3.4 us
+// a split with eight waves, 2.6 with four; without the loads 7 % less.  Computing the next split's scores under this
+// one's softmax: 151 -> 160 us (registers).  2048 rows of 16 / 2 heads: 425 us as splits (286 MB of partial results out
+// and as many back), 151 here; 300 rows 36 -> 26 us.
+constexpr int kPairSplit = 64, kPairKeys = 32 * 1024, kPairLds = 5 * kPairKeys;
+__global__ void __launch_bounds__(512)
+    attn_rows_pair_kernel(const float *__restrict__ q, const _Float16 *__restrict__ k_cache, const _Float16 *__restrict__ vt_cache, int64_t ctx_len,
+                          int n_rows_total, int n_q, int n_kv, int64_t vt_stride, float scale, float *__restrict__ out, void *__restrict__ out_xf,
+                          int out_xf_kind, size_t xf_stride) {
+    constexpr int HD = 256, KS = HD / 32, DT = HD / 16, CH = HD / 8;
+    extern __shared__ half8_t lds[];
+    const int block = gridDim.z - 1 - blockIdx.z;  // (the longest first)
+    const int n_rows = min(16, n_rows_total - 16 * block);
+    ctx_len += 16 * static_cast<int64_t>(block);
+    const int n_pos = static_cast<int>(ctx_len) + n_rows;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n_waves = blockDim.x >> 6;
+    const int n = lane & 15, g = lane >> 4;
+    const int kvh = blockIdx.y, head = kvh * (n_q / n_kv) + blockIdx.x * n_waves + wave;
+    const int n_splits = (n_pos + kPairSplit - 1) / kPairSplit;
+    const int64_t kv_dim = static_cast<int64_t>(n_kv) * HD;
+    const uint8_t *const k_base = reinterpret_cast<const uint8_t *>(k_cache + static_cast<int64_t>(kvh) * HD);
+    const uint8_t *const v_base = reinterpret_cast<const uint8_t *>(vt_cache + static_cast<int64_t>(kvh) * HD * vt_stride);
+    const uint32_t v_lane = static_cast<uint32_t>(lane >> 2) * static_cast<uint32_t>(vt_stride) * 2 + 16 * ((lane & 3) ^ attn_swz_v(lane >> 2));
+
+    // A wave-load is 1 KB: two key rows, or 16 dims of 32 values.  32 of them are a split's keys, as many again its values; a
+    // wave takes every n_waves-th, and where they do not come out even some load what another loads too.  With eight or
+    // four waves the loads of a whole split differ by uniform strides and uniform bits of the swizzle.
+    const uint32_t k_lane = static_cast<uint32_t>(2 * wave + (lane >> 5)) * static_cast<uint32_t>(kv_dim * 2) +
+                            (((lane & 31) ^ attn_swz<CH>(2 * wave + (lane >> 5))) << 4);
+    auto load = [&](int split, bool values, uint8_t *dst) {
+        const int total = values ? 64 : 32, c0 = split * kPairSplit, last = n_pos - 1 - c0;
+        auto whole = [&](auto waves) {
+            constexpr int NW = decltype(waves)::value;
+            const uint8_t *k = k_base + c0 * kv_dim * 2, *v = v_base + static_cast<int64_t>(16 * wave) * vt_stride * 2 + 2 * static_cast<int64_t>(c0);
+            uint8_t *to = dst + wave * 1024;
+#pragma unroll
+            for (int j = 0; j < 32 / NW; j++, to += NW * 1024)
+                __builtin_amdgcn_global_load_lds((gptr_t)(k + j * 4 * NW * kv_dim + (k_lane ^ static_cast<uint32_t>(attn_swz<CH>(2 * NW * j & 31) << 4))), (lptr_t)(to),
+                                                 16, 0, 0);
+            if (values) {
+#pragma unroll
+                for (int j = 0; j < 32 / NW; j++, to += NW * 1024)
+                    __builtin_amdgcn_global_load_lds((gptr_t)(v + (NW * j & 15) * 32 * vt_stride + (NW * j >> 4) * 64 + v_lane), (lptr_t)(to), 16, 0, 0);
+            }
+        };
+        if (n_waves == 8 && last >= kPairSplit - 1) return whole(std::integral_constant<int, 8>());
+        if (n_waves == 4 && last >= kPairSplit - 1) return whole(std::integral_constant<int, 4>());
+        for (int i = wave; i < (total + n_waves - 1) / n_waves * n_waves; i += n_waves) {
+            const int p = i < total ? i : i - total;
+            const uint8_t *src;
+            if (p < 32) {  // (rows past the last position are never dereferenced: the last one again, its scores are masked)
+                const int row = 2 * p + (lane >> 5);
+                src = k_base + c0 * kv_dim * 2 + static_cast<uint32_t>(min(row, last)) * static_cast<uint32_t>(kv_dim * 2) + (((lane & 31) ^ attn_swz<CH>(row & 31)) << 4);
+            } else {  // (nor is a second stage past the last position: the first one again, its values are zeroed)
+                const int stage = (p - 32) >> 4, key = c0 + (32 * stage <= last ? 32 * stage : 0);
+                src = v_base + static_cast<int64_t>((p & 15) * 16) * vt_stride * 2 + 2 * static_cast<int64_t>(key) + v_lane;
+            }
+            __builtin_amdgcn_global_load_lds((gptr_t)(src), (lptr_t)(dst + p * 1024), 16, 0, 0);
+        }
+    };
+    const int per_keys = (32 + n_waves - 1) / n_waves, per_split = (64 + n_waves - 1) / n_waves;
+    auto landed = [&](int later) {
+        attn_wait(later);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    uint8_t *const lds_b = reinterpret_cast<uint8_t *>(lds);
+
+    half8_t qf[KS];
+    {
+        const float mult = scale * kLog2e;
+        const float *qrow = q + (static_cast<int64_t>(block) * 16 + min(n, n_rows - 1)) * n_q * HD + static_cast<int64_t>(head) * HD + 8 * g;
+        AttnQ8<float> raw[KS];
+        load(0, false, lds_b);
+        if (n_splits > 1)
+            load(1, false, lds_b + kPairKeys);
+        else
+            load(0, true, lds_b + 3 * kPairKeys);
+        attn_load_q<0, KS>(raw, qrow);  // (behind the branches: no asm load is under way where the code branches)
+        attn_wait(0);
+#pragma unroll
+        for (int s = 0; s < KS; s++) {
+            raw[s].arrived();
+#pragma unroll
+            for (int i = 0; i < 8; i++) qf[s][i] = static_cast<_Float16>(raw[s].get(i) * mult);
+        }
+    }
+    // A split's fragments, in the order of their use: K rows of step s of the four score tiles T (4 s + T), then V^T of the
+    // two stages of the sixteen tiles of dims (32 + 2 t + st).  Each is read kRing uses ahead, the first of V under the softmax.
+    // (K's swizzle permutes a lane's steps four by four: four addresses, the rest is in the offset.)
+    constexpr int kRing = 8;
+    const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lptr_t)lds));
+    const uint32_t k_at = lds0 + (8 * (n >> 2) + (n & 3)) * (CH * 16) + (g ^ (n & 3)) * 16, v_at = lds0 + kPairKeys + (4 * n + (g ^ attn_swz_v(n))) * 16;
+    const uint32_t k_step[4] = {k_at + (n >> 2) * 64, k_at + ((n >> 2) ^ 1) * 64, k_at + ((n >> 2) ^ 2) * 64, k_at + ((n >> 2) ^ 3) * 64};
+    half8_t ring[kRing];
+    auto read = [&](auto i, uint32_t buf) {
+        constexpr int I = decltype(i)::value;
+        if constexpr (I < 4 * KS)
+            ring[I % kRing] = lds_read<half8_t, (32 * (I >> 1 & 1) + 4 * (I & 1)) * CH * 16 + (I >> 4) * 256>(k_step[I >> 2 & 3] + buf);
+        else
+            ring[I % kRing] = lds_read<half8_t, ((I - 4 * KS) >> 1) * 1024 + (I & 1) * 16384>(v_at + buf);
+    };
+    // The scores of a split's two stages, base-2 logits: p[8 st + i] of key 32 st + 8 g + i.  masked: some are hidden from some row.
+    auto scores = [&](auto masked, auto with_values, int split, uint32_t buf, float (&p)[16]) {
+        constexpr int N = decltype(with_values)::value ? 4 * KS + 2 * DT : 4 * KS;
+        float4_t sc[4];
+        static_for<0, kRing>([&](auto i) { read(i, buf); });
+        static_for<0, 4 * KS>([&](auto i) {
+            constexpr int I = decltype(i)::value, T = I & 3, left = N - 1 - I;
+            lds_arrived<(left < kRing - 1 ? left : kRing - 1)>(ring[I % kRing]);
+            sc[T] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ring[I % kRing], qf[I >> 2], I < 4 ? float4_t{0, 0, 0, 0} : sc[T], 0, 0, 0);
+            if constexpr (I + kRing < N) read(std::integral_constant<int, I + kRing>(), buf);
+        });
+        const int seen = static_cast<int>(ctx_len) + n - split * kPairSplit - 8 * g;
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            p[i] = sc[2 * (i >> 3) + ((i >> 2) & 1)][i & 3];
+            if (decltype(masked)::value && 32 * (i >> 3) + (i & 7) > seen) p[i] = -INFINITY;
+        }
+    };
+    // (a split that ends behind the block's first row is the only kind that hides a key from a row)
+    auto edge = [&](int split) { return (split + 1) * kPairSplit - 1 > static_cast<int>(ctx_len); };
+
+    // first walk: the maximum over every key a row sees
+    float m_star = -INFINITY;
+    for (int split = 0, buf = 0; split < n_splits; split++) {
+        landed(split + 1 < n_splits ? per_keys : per_split);
+        uint8_t *const free_buf = lds_b + (buf == 0 ? 2 : buf - 1) * kPairKeys;
+        if (split + 2 < n_splits)
+            load(split + 2, false, free_buf);
+        else if (split + 2 == n_splits)
+            load(0, true, lds_b + 3 * kPairKeys);
+        auto maxima = [&](auto masked) {
+            float p[16];
+            scores(masked, std::false_type(), split, buf * kPairKeys, p);
+#pragma unroll
+            for (int i = 0; i < 16; i++) m_star = fmaxf(m_star, p[i]);
+        };
+        if (edge(split))
+            maxima(std::true_type());
+        else
+            maxima(std::false_type());
+        buf = buf == 2 ? 0 : buf + 1;
+    }
+    m_star = dfl_max_far(m_star);
+
+    // second walk.  Up to eight splits are an eighth each: `sum` is the total.  Else it is an eighth's sum, and the total waits in
+    // the block's output rows of this head, seven times there and back (the registers do not hold both): lane by lane, a
+    // kilobyte a row, where all sixteen rows are there, else where it belongs.
+    float *const o = out + ((static_cast<int64_t>(block) * 16 + n) * n_q + head) * HD + 4 * g;
+    const bool live = n < n_rows, held = live || n_rows == 16;
+    float *const wait_at = n_rows == 16 ? out + (static_cast<int64_t>(block) * 16 * n_q + head) * HD + 4 * lane : o;
+    const int64_t wait_step = n_rows == 16 ? static_cast<int64_t>(n_q) * HD : 16;
+    float4_t sum[DT];
+#pragma unroll
+    for (int t = 0; t < DT; t++) sum[t] = float4_t{0, 0, 0, 0};
+    float l_sum = 0.0f, l_tot = 0.0f;
+    const bool few = n_splits <= 8;
+    for (int split = 0, at = 0; at < n_splits; at++) {
+        const bool ends = split + 8 >= n_splits;  // the last of this one's eighth
+        const int next = ends ? (split & 7) + 1 : split + 8;
+        landed(0);
+        const uint32_t buf = at & 1 ? 0 : 3 * kPairKeys;
+        if (at + 1 < n_splits) load(next, true, lds_b + (at & 1 ? 3 * kPairKeys : 0));
+        auto merge = [&](auto masked, auto of_few) {
+            constexpr bool kFew = decltype(of_few)::value;
+            float p[16];
+            scores(masked, std::true_type(), split, buf, p);
+            // the two stages: running maximum, rescale of the first stage by the second's, row sum
+            float mx[2];
+#pragma unroll
+            for (int st = 0; st < 2; st++) {
+                const float *v = p + 8 * st;
+                mx[st] = dfl_max_far(fmaxf(fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3])), fmaxf(fmaxf(v[4], v[5]), fmaxf(v[6], v[7]))));
+            }
+            const float m1 = mx[0], m2 = fmaxf(m1, mx[1]);
+            const float safe[2] = {m1 == -INFINITY ? 0.0f : m1, m2 == -INFINITY ? 0.0f : m2};
+            const float alpha = __builtin_amdgcn_exp2f(m1 - safe[1]);
+            half8_t pf[2];
+            float ps[2] = {0.0f, 0.0f};
+#pragma unroll
+            for (int st = 0; st < 2; st++)
+#pragma unroll
+                for (int i = 0; i < 8; i++) {
+                    const float e = __builtin_amdgcn_exp2f(p[8 * st + i] - safe[st]);
+                    ps[st] += e;
+                    pf[st][i] = static_cast<_Float16>(e);
+                }
+            // (over the row's four lanes: the lane 16 away, then the pair 32 away)
+            float l = __builtin_fmaf(ps[0], alpha, ps[1]), l2 = l;
+            dfl_swap16(l, l2);
+            l += l2;
+            l2 = l;
+            dfl_swap32(l, l2);
+            l += l2;
+            const float w = m2 == -INFINITY ? 0.0f : exp2f(m2 - m_star);
+            l_sum = kFew ? l_sum + __builtin_fmaf(w, l, 0.0f) : __builtin_fmaf(w, l, l_sum);
+            const int left = n_pos - split * kPairSplit - 8 * g;  // this lane's columns ahead of n_pos
+            float4_t a[DT];
+            static_for<4 * KS, 4 * KS + 2 * DT>([&](auto i) {
+                constexpr int I = decltype(i)::value, t = (I - 4 * KS) >> 1, st = I & 1, later = 4 * KS + 2 * DT - 1 - I;
+                half8_t &v = ring[I % kRing];
+                lds_arrived<(later < kRing - 1 ? later : kRing - 1)>(v);
+                if constexpr (decltype(masked)::value) {  // (what the cache holds past n_pos may be NaN patterns)
+#pragma unroll
+                    for (int k = 0; k < 8; k++)
+                        if (32 * st + k >= left) v[k] = static_cast<_Float16>(0.0f);
+                }
+                if constexpr (st == 0) {
+                    a[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(v, pf[0], float4_t{0, 0, 0, 0}, 0, 0, 0);
+                    a[t] *= alpha;
+                } else {
+                    a[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(v, pf[1], a[t], 0, 0, 0);
+#pragma unroll
+                    for (int k = 0; k < 4; k++) sum[t][k] = kFew ? sum[t][k] + __builtin_fmaf(w, a[t][k], 0.0f) : __builtin_fmaf(w, a[t][k], sum[t][k]);
+                }
+                if constexpr (I + kRing < 4 * KS + 2 * DT) read(std::integral_constant<int, I + kRing>(), buf);
+            });
+        };
+        if (few && edge(split))
+            merge(std::true_type(), std::true_type());
+        else if (few)
+            merge(std::false_type(), std::true_type());
+        else if (edge(split))
+            merge(std::true_type(), std::false_type());
+        else
+            merge(std::false_type(), std::false_type());
+        if (ends && !few) {
+            l_tot += l_sum;
+            float *at_row = wait_at;  // (opaque: sixteen addresses kept across the walk would not fit)
+            asm volatile("" : "+v"(at_row));
+            if (held && (split & 7) != 0) {
+                float4_t v[DT];
+                const float *p = at_row;
+#pragma unroll
+                for (int t = 0; t < DT; t++, p += wait_step) v[t] = *reinterpret_cast<const float4_t *>(p);
+#pragma unroll
+                for (int t = 0; t < DT; t++) sum[t] = v[t] + sum[t];
+            }
+            if ((split & 7) != 7) {
+                l_sum = 0.0f;
+#pragma unroll
+                for (int t = 0; t < DT; t++, at_row += wait_step) {
+                    if (held) *reinterpret_cast<float4_t *>(at_row) = sum[t];
+                    sum[t] = float4_t{0, 0, 0, 0};
+                }
+            }
+        }
+        split = next;
+    }
+    if (few) l_tot = l_sum;
+#pragma unroll
+    for (int t = 0; t < DT; t++) {
+        sum[t] /= l_tot;
+        if (live) *reinterpret_cast<float4_t *>(o + 16 * t) = sum[t];
+    }
+    if (out_xf) attn_store_xf<DT>(sum, static_cast<uint8_t *>(out_xf) + block * xf_stride, out_xf_kind, n, g, head * HD, live);
 }
 
 #ifdef DFLASH_TRACE
@@ -814,6 +1088,14 @@ int32_t launch_rows(dflash_ctx *ctx, dim3 grid, int n_waves, hipStream_t st, con
     DFL_HIP_CHECK(ctx, hipGetLastError());
     return DFLASH_OK;
 }
+int32_t launch_rows_pair(dflash_ctx *ctx, dim3 grid, int n_waves, hipStream_t st, const float *q, const _Float16 *k, const _Float16 *vt, int64_t ctx_len,
+                         int n_rows, int n_q, int n_kv, int64_t vt_stride, float scale, float *out, void *out_xf, int out_xf_kind) {
+    if (const int32_t rc_ = dfl_raise_lds_limit(ctx, reinterpret_cast<const void *>(attn_rows_pair_kernel), kPairLds)) return rc_;
+    attn_rows_pair_kernel<<<grid, 64 * n_waves, kPairLds, st>>>(q, k, vt, ctx_len, n_rows, n_q, n_kv, vt_stride, scale, out, out_xf, out_xf_kind,
+                                                                dfl_xf_bytes(static_cast<int64_t>(n_q) * 256));
+    DFL_HIP_CHECK(ctx, hipGetLastError());
+    return DFLASH_OK;
+}
 
 }  // namespace
 
@@ -963,26 +1245,42 @@ int32_t dfl_attn_blocks(dflash_ctx *ctx, const void *q, int32_t q_type, const vo
             const int64_t n_pos = ctx_len + std::min(16 * (taken + 1), n_rows_total), bucket = dfl_attn_bucket(n_pos);
             if (bucket != last) {
                 const AttnPolicy p = attn_policy(ctx, bucket, n_kv, group, head_dim);
-                if (!p.ordered || runs.n == kAttnRuns) break;
+                if ((!p.ordered && head_dim != 256) || runs.n == kAttnRuns) break;
                 last = bucket;
                 runs.first[runs.n] = taken;
                 runs.want[runs.n] = p.want;
                 runs.min_chunk[runs.n++] = static_cast<int>(p.min_chunk);
             }
             const int64_t chunk = attn_chunk(n_pos, runs.want[runs.n - 1], runs.min_chunk[runs.n - 1]);
+            if (head_dim == 256 && (chunk != kPairSplit || n_pos > 0x3fffffff)) break;
             partials += (n_pos + chunk - 1) / chunk * n_q * head_dim / 128;
         }
         int hw = std::min(group, 8);
         while (group % hw) hw--;
         const int32_t rows = std::min(n_rows_total, 16 * taken);
+        // heads of 256, half the waves on a workgroup's splits where those workgroups still fit the chip side by side: 2.6 us a
+        // split instead of 3.4 (16 / 2 heads, 1024 rows 85 -> 67 us; 2048 rows, twice the chip's CUs, 157 : 154)
+        if (head_dim == 256 && hw == 8 && static_cast<int64_t>(taken) * n_kv * (group / 4) <= ctx->n_cu) hw = 4;
         const int64_t wgs = static_cast<int64_t>(taken) * n_kv * (group / hw), n_steps = (ctx_len + rows + 31) / 32;
         const int64_t stages = wgs * (ctx_len + rows / 2) / 32;
-        const double one_launch = 5.5 + 1.15 * n_steps, as_splits = 11.0 * runs.n + (0.5 * stages + 1.1 * partials) / ctx->n_cu;
+        const double as_splits = (head_dim == 256 ? 18.0 : 11.0) * runs.n + (0.5 * stages + 1.1 * partials) / ctx->n_cu;
+        double one_launch = 5.5 + 1.15 * n_steps;
+        // Heads of 256 walk the keys twice: 16 us and 2.6, 3.4 or (workgroups of neither four nor eight heads) 4.2 us for a split of
+        // two stages, 8 us more where the total goes out and back; the two launches of a run 18 us.  Both sides in us, the last layer's worth of 95 measured
+        // pairs (splits : one launch): 16 / 2 heads 452 : 154 for 2048 rows behind none, 60 : 36 for 512, 155 : 111 for 512 behind
+        // 1520, 71 : 98 for 256 behind 1520, 38 : 149 for 64 behind 3040; 8 / 1 heads 74 : 107 and 161 : 129 for 512 and 1024
+        // behind 1520; 32 / 4 heads 43 : 25 for 256 behind none; 5 / 1 heads 191 : 193 for 2048 behind none.
+        if (head_dim == 256)
+            one_launch = (n_steps > 16 ? 24.0 : 16.0) + (hw == 4 ? 2.6 : hw == 8 ? 3.4 : 4.2) * std::max(0.5 * n_steps, 0.65 * stages / ctx->n_cu);
         if (taken > 1 && one_launch <= as_splits) {
             hipStream_t st = static_cast<hipStream_t>(stream);
             dfl_timed timer(ctx, st, DFL_T_ATTN);
-            const auto launch = head_dim == 64 ? launch_rows<64> : launch_rows<128>;
-            if (const int32_t rc_ = launch(ctx, dim3(group / hw, n_kv, taken), hw, st, static_cast<const float *>(q), static_cast<const _Float16 *>(k_cache),
+            if (head_dim == 256) {
+                if (const int32_t rc_ = launch_rows_pair(ctx, dim3(group / hw, n_kv, taken), hw, st, static_cast<const float *>(q),
+                                                         static_cast<const _Float16 *>(k_cache), static_cast<const _Float16 *>(vt_cache), ctx_len, rows, n_q,
+                                                         n_kv, kv_capacity, scale, out, out_xf, out_xf_kind))
+                    return rc_;
+            } else if (const int32_t rc_ = (head_dim == 64 ? launch_rows<64> : launch_rows<128>)(ctx, dim3(group / hw, n_kv, taken), hw, st, static_cast<const float *>(q), static_cast<const _Float16 *>(k_cache),
                                            static_cast<const _Float16 *>(vt_cache), ctx_len, rows, n_q, n_kv, kv_capacity, runs, scale, out, out_xf,
                                            out_xf_kind))
                 return rc_;

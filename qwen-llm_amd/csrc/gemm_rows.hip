@@ -34,6 +34,7 @@
 // partial tiles are added in.  That order is also what a split of K over workgroups has to keep: each range between two
 // cuts goes to memory on its own and rows_reduce_kernel adds them up (kSplit; few rows against a narrow matrix).
 #include "common.h"
+#include "lds_read.h"
 #include "mfma_unpack.h"
 
 #include <algorithm>
@@ -97,33 +98,8 @@ __device__ __forceinline__ half8_t splat8(_Float16 v) {
     return r;
 }
 
-template <int I, int N, typename F>
-__device__ __forceinline__ void static_for(F &&f) {
-    if constexpr (I < N) {
-        f(std::integral_constant<int, I>());
-        static_for<I + 1, N>(f);
-    }
-}
-
-// Reads from LDS and the waits for them are asm: the compiler cannot tell LDS reads from the direct-to-LDS loads in flight and
-// waits for every read it has issued (lgkmcnt(0)) ahead of each product.  (The build refuses this kernel if it spills: see build.py.)
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
-template <typename T, int OFF>
-__device__ __forceinline__ T lds_read(uint32_t at) {
-    T v;
-    if constexpr (sizeof(T) == 16)
-        asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(at), "n"(OFF));
-    else if constexpr (sizeof(T) == 8)
-        asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(v) : "v"(at), "n"(OFF));
-    else
-        asm volatile("ds_read_u16 %0, %1 offset:%2" : "=v"(v) : "v"(at), "n"(OFF));
-    return v;
-}
-// v has arrived, with at most LATER of the reads issued behind it still under way
-template <int LATER>
-__device__ __forceinline__ void lds_arrived(half8_t &v) {
-    asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(v) : "n"(LATER < 15 ? LATER : 15));
-}
+
 // this wave's loads into LDS but for the last N are done
 template <int N>
 __device__ __forceinline__ void copies_done() {

@@ -29,6 +29,9 @@ SHAPES["heads64"] = (dfl.ModelConfig(n_layers=2, hidden=1024, n_q=24, n_kv=2, he
 SHAPES["heads64x12"] = (dfl.ModelConfig(n_layers=2, hidden=1024, n_q=48, n_kv=4, head_dim=64, ffn=3072, vocab=2048), dfl.synth.Q4_K)
 SHAPES["heads256x5"] = (dfl.ModelConfig(n_layers=2, hidden=1280, n_q=5, n_kv=1, head_dim=256, ffn=3072, vocab=2048), dfl.synth.Q4_K)
 
+SHAPES["heads256x1"] = (dfl.ModelConfig(n_layers=2, hidden=1024, n_q=4, n_kv=4, head_dim=256, ffn=3072, vocab=2048), dfl.synth.Q4_K)
+SHAPES["heads256x12"] = (dfl.ModelConfig(n_layers=2, hidden=1024, n_q=12, n_kv=1, head_dim=256, ffn=3072, vocab=2048), dfl.synth.Q4_K)
+
 
 @pytest.fixture(scope="module")
 def ctx():
@@ -76,6 +79,14 @@ def test_continued_prefill_equals_block_by_block(ctx, shape, head, rows):
     assert torch.equal(got, want)
     one.close()
     many.close()
+
+
+@pytest.mark.parametrize("head,rows", [(0, 2033), (64, 1500), (0, 513), (480, 70), (37, 600)])
+@pytest.mark.parametrize("shape", ["experts", "heads256x1", "heads256x5", "heads256x12"])
+def test_heads_of_256_equal_block_by_block(ctx, shape, head, rows):
+    """Keys walked twice in one workgroup against splits and their merge: one, four, five, six and eight waves, up to eight
+    splits (the total in registers) and more (in the output rows, also where the last block is short), a last split of one stage and of two."""
+    test_continued_prefill_equals_block_by_block(ctx, shape, head, rows)
 
 
 def _rescale(mat, factor):
