@@ -1263,15 +1263,15 @@ int32_t dfl_attn_blocks(dflash_ctx *ctx, const void *q, int32_t q_type, const vo
         if (head_dim == 256 && hw == 8 && static_cast<int64_t>(taken) * n_kv * (group / 4) <= ctx->n_cu) hw = 4;
         const int64_t wgs = static_cast<int64_t>(taken) * n_kv * (group / hw), n_steps = (ctx_len + rows + 31) / 32;
         const int64_t stages = wgs * (ctx_len + rows / 2) / 32;
-        const double as_splits = (head_dim == 256 ? 18.0 : 11.0) * runs.n + (0.5 * stages + 1.1 * partials) / ctx->n_cu;
+        const double as_splits = (head_dim == 256 ? 20.0 : 11.0) * runs.n + (0.5 * stages + 1.1 * partials) / ctx->n_cu;
         double one_launch = 5.5 + 1.15 * n_steps;
-        // Heads of 256 walk the keys twice: 16 us and 2.6, 3.4 or (workgroups of neither four nor eight heads) 4.2 us for a split of
-        // two stages, 8 us more where the total goes out and back; the two launches of a run 18 us.  Both sides in us, the last layer's worth of 95 measured
+        // Heads of 256 walk the keys twice: 14 us and 2.6, 3.4 or (workgroups of neither four nor eight heads) 4.2 us for a split of
+        // two stages, 8 us more where the total goes out and back; the two launches of a run 20 us.  Both sides in us, the last layer's worth of 95 measured
         // pairs (splits : one launch): 16 / 2 heads 452 : 154 for 2048 rows behind none, 60 : 36 for 512, 155 : 111 for 512 behind
         // 1520, 71 : 98 for 256 behind 1520, 38 : 149 for 64 behind 3040; 8 / 1 heads 74 : 107 and 161 : 129 for 512 and 1024
         // behind 1520; 32 / 4 heads 43 : 25 for 256 behind none; 5 / 1 heads 191 : 193 for 2048 behind none.
         if (head_dim == 256)
-            one_launch = (n_steps > 16 ? 24.0 : 16.0) + (hw == 4 ? 2.6 : hw == 8 ? 3.4 : 4.2) * std::max(0.5 * n_steps, 0.65 * stages / ctx->n_cu);
+            one_launch = (n_steps > 16 ? 22.0 : 14.0) + (hw == 4 ? 2.6 : hw == 8 ? 3.4 : 4.2) * std::max(0.5 * n_steps, 0.65 * stages / ctx->n_cu);
         if (taken > 1 && one_launch <= as_splits) {
             hipStream_t st = static_cast<hipStream_t>(stream);
             dfl_timed timer(ctx, st, DFL_T_ATTN);
