@@ -256,10 +256,10 @@ int32_t dfl_xf_sums(dflash_ctx *ctx, const void *xf, int64_t n_in, int32_t n_blo
 int32_t dfl_gemm_rows(dflash_ctx *ctx, const dfl_rows_plan &plan, int32_t w_type, const void *w, const void *xf, const void *xs, float *y,
                       int64_t n_in, int64_t n_out, int32_t n_rows, int64_t pair_ffn, void *y_xf, void *y_xs, int y_kind, hipStream_t stream);
 // The experts' products over row tiles listed on the device, tiles[i] = {expert (-1: the extra matrix), first block,
-// blocks (1..4), -}: the arithmetic of gemm_q4k_experts_kernel.  w_up != null: silu(x . w^T) * (x . w_up^T) to y_xf / y_xs.
+// blocks (1..tile_blocks, which is 4 or 8), -}: the arithmetic of gemm_q4k_experts_kernel.  w_up != null: silu(x . w^T) * (x . w_up^T) to y_xf / y_xs.
 int32_t dfl_gemm_rows_experts(dflash_ctx *ctx, const void *w, const void *w_extra, const void *w_up, const void *w_up_extra, size_t w_stride,
-                              const void *xf, const void *xs, const int32_t *tiles, const int32_t *n_tiles, int32_t max_tiles, float *y,
-                              int64_t n_in, int64_t n_out, void *y_xf, void *y_xs, hipStream_t stream);
+                              const void *xf, const void *xs, const int32_t *tiles, const int32_t *n_tiles, int32_t max_tiles,
+                              int32_t tile_blocks, float *y, int64_t n_in, int64_t n_out, void *y_xf, void *y_xs, hipStream_t stream);
 // How dfl_gemm_fewrow_checked splits a Q4_K matrix in tiled order: workgroup i of n_wg takes stages
 // [total i / n_wg, total (i + 1) / n_wg) of the (256-row tile group x super-block) space; false where it does not take it.
 bool dfl_q4k_tiled_split(const dflash_ctx *ctx, int64_t n_in, int64_t n_out, int *total, int *n_wg);

@@ -24,8 +24,9 @@
 // PFLOP/s, matrix cores busy for 57 % of the cycles, 42 % before), 17408 -> 5120 233 -> 193 us (0.92), 5120 -> 6144 and 4096 ->
 // 5120 together 240 -> 210 us (0.50: their twin MFMAs, which the block path's bits ask for, are as many again); 2048 rows:
 // 2048 -> 5120 and 4096 -> 2048 in Q6_K together 220 -> 186 us.  A 64-layer prompt of 1000 rows 64.7 -> 59.7 ms.
-// The experts' tiles (a list, mostly one to four row blocks) take workgroups of half the columns, two of them on a CU:
-// each waits for its own weights while the other computes (2 - 4 % of a prompt of 33 - 130 rows).
+// The experts' tiles (a list) take workgroups of half the columns and up to four row blocks, two of them on a CU, each
+// waiting for its own weights while the other computes, or, where an expert has rows enough, of all columns and up to eight blocks
+// (the rule and both sides' figures stand in dfl_moe_ffn_group).
 //
 // Bits.  Every row of Y has the bits that the 16-row kernels give it in its own block.  The arithmetic of a
 // super-block is theirs (the same unpacking, the same v_mfma_f32_16x16x32_f16 sequence into the same accumulator); K is
@@ -45,7 +46,7 @@ namespace {
 typedef const __attribute__((address_space(1))) void *gptr_t;
 typedef __attribute__((address_space(3))) void *lptr_t;
 
-constexpr int kRowsWaves = 8, kListWaves = 4;
+constexpr int kRowsWaves = 8;
 
 struct RowsArgs {
     const uint8_t *w[2];       // matrix of column segment 0 and 1 (a list: the stacks' first matrices)
@@ -227,13 +228,13 @@ struct RowsLds {
 // kTwin: the minima / offsets through a twin MFMA per activation fragment into a second accumulator (the whole-K
 // kernel's arithmetic); else one MFMA per super-block over the sub-block sums (the streaming and expert kernels').
 // kCut: K is cut somewhere.  RB: 16-row blocks of the tile.
-template <typename Tile, bool kTwin, bool kCut, int RB, int kEpi, bool kList>
-__global__ void __launch_bounds__(64 * (kList ? kListWaves : kRowsWaves), 2) gemm_rows_kernel(RowsArgs a) {
-    constexpr int W = kList ? kListWaves : kRowsWaves;  // waves, 32 columns each
+template <typename Tile, bool kTwin, bool kCut, int RB, int kEpi, int kList>
+__global__ void __launch_bounds__(64 * (kList ? kList : kRowsWaves), 2) gemm_rows_kernel(RowsArgs a) {
+    constexpr int W = kList ? kList : kRowsWaves;  // waves, 32 columns each
     constexpr bool kPair = kEpi == kEpiSwiglu, kSplit = kEpi == kEpiSplit, kTotal = kCut && !kSplit;
     constexpr int NSEG = kPair ? 2 : 1, kSegTiles = 2 * W / NSEG;
     typedef RowsLds<Tile, kTwin, RB, W> Lds;
-    static_assert((kList ? 2 : 1) * Lds::total <= 160 * 1024, "a CU's LDS");
+    static_assert(8 / W * Lds::total <= 160 * 1024, "a CU's LDS");
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -558,9 +559,21 @@ __global__ void __launch_bounds__(64 * (kList ? kListWaves : kRowsWaves), 2) gem
             case 1: walk_k(std::integral_constant<int, 1>()); break;
             case 2: walk_k(std::integral_constant<int, 2>()); break;
             case 3: walk_k(std::integral_constant<int, 3>()); break;
-            default: walk_k(std::integral_constant<int, RB>()); break;
+            default:
+                if constexpr (RB > 4) {
+                    switch (live) {
+                        case 4: walk_k(std::integral_constant<int, 4>()); break;
+                        case 5: walk_k(std::integral_constant<int, 5>()); break;
+                        case 6: walk_k(std::integral_constant<int, 6>()); break;
+                        case 7: walk_k(std::integral_constant<int, 7>()); break;
+                        default: walk_k(std::integral_constant<int, RB>()); break;
+                    }
+                } else {
+                    walk_k(std::integral_constant<int, RB>());
+                }
+                break;
         }
-        static_assert(!kList || RB == 4, "a list's tiles");
+        static_assert(!kList || RB == kList, "a list's tiles");
     } else {
         constexpr int kHalf = RB > 2 ? (RB + 1) / 2 : RB;
         if (live <= kHalf)
@@ -701,10 +714,10 @@ int32_t dfl_xf_sums(dflash_ctx *ctx, const void *xf, int64_t n_in, int32_t n_blo
 }
 
 namespace {
-template <typename Tile, bool kTwin, bool kCut, int RB, int kEpi, bool kList>
+template <typename Tile, bool kTwin, bool kCut, int RB, int kEpi, int kList>
 int32_t rows_launch(dflash_ctx *ctx, const RowsArgs &a, int64_t tiles, hipStream_t st) {
     const auto fn = gemm_rows_kernel<Tile, kTwin, kCut, RB, kEpi, kList>;
-    constexpr int W = kList ? kListWaves : kRowsWaves;
+    constexpr int W = kList ? kList : kRowsWaves;
     const size_t lds = RowsLds<Tile, kTwin, RB, W>::total;
     if (const int32_t rc = dfl_raise_lds_limit(ctx, reinterpret_cast<const void *>(fn), lds)) return rc;
     if (tiles < 1 || tiles > 0x0fffffff) return dfl_fail(ctx, DFLASH_ERR_BAD_SHAPE, "gemm_rows: %lld tiles", static_cast<long long>(tiles));
@@ -733,17 +746,17 @@ int rows_pick_rb(const dflash_ctx *ctx, int n_blocks, int n_ct, int most) {
 template <typename Tile, bool kTwin, int kEpi>
 int32_t rows_dispatch(dflash_ctx *ctx, const RowsArgs &a, int rb, int64_t tiles, hipStream_t st) {
     switch (rb) {
-        case 2: return rows_launch<Tile, kTwin, true, 2, kEpi, false>(ctx, a, tiles, st);
-        case 3: return rows_launch<Tile, kTwin, true, 3, kEpi, false>(ctx, a, tiles, st);
-        case 4: return rows_launch<Tile, kTwin, true, 4, kEpi, false>(ctx, a, tiles, st);
+        case 2: return rows_launch<Tile, kTwin, true, 2, kEpi, 0>(ctx, a, tiles, st);
+        case 3: return rows_launch<Tile, kTwin, true, 3, kEpi, 0>(ctx, a, tiles, st);
+        case 4: return rows_launch<Tile, kTwin, true, 4, kEpi, 0>(ctx, a, tiles, st);
         default: break;
     }
     if constexpr (!kTwin) {
         switch (rb) {
-            case 5: return rows_launch<Tile, kTwin, true, 5, kEpi, false>(ctx, a, tiles, st);
-            case 6: return rows_launch<Tile, kTwin, true, 6, kEpi, false>(ctx, a, tiles, st);
-            case 7: return rows_launch<Tile, kTwin, true, 7, kEpi, false>(ctx, a, tiles, st);
-            case 8: return rows_launch<Tile, kTwin, true, 8, kEpi, false>(ctx, a, tiles, st);
+            case 5: return rows_launch<Tile, kTwin, true, 5, kEpi, 0>(ctx, a, tiles, st);
+            case 6: return rows_launch<Tile, kTwin, true, 6, kEpi, 0>(ctx, a, tiles, st);
+            case 7: return rows_launch<Tile, kTwin, true, 7, kEpi, 0>(ctx, a, tiles, st);
+            case 8: return rows_launch<Tile, kTwin, true, 8, kEpi, 0>(ctx, a, tiles, st);
             default: break;
         }
     }
@@ -820,10 +833,10 @@ int32_t dfl_gemm_rows(dflash_ctx *ctx, const dfl_rows_plan &p, int32_t w_type, c
 }
 
 int32_t dfl_gemm_rows_experts(dflash_ctx *ctx, const void *w, const void *w_extra, const void *w_up, const void *w_up_extra, size_t w_stride,
-                              const void *xf, const void *xs, const int32_t *tiles, const int32_t *n_tiles, int32_t max_tiles, float *y,
-                              int64_t n_in, int64_t n_out, void *y_xf, void *y_xs, hipStream_t st) {
+                              const void *xf, const void *xs, const int32_t *tiles, const int32_t *n_tiles, int32_t max_tiles,
+                              int32_t tile_blocks, float *y, int64_t n_in, int64_t n_out, void *y_xf, void *y_xs, hipStream_t st) {
     if (!w || !w_extra || !xf || !xs || !tiles || !n_tiles || max_tiles < 1 || n_in <= 0 || n_in % DFL_QK_K || n_out <= 0 || n_out % DFL_QK_K ||
-        (w_up ? (!w_up_extra || !y_xf || !y_xs) : !y) || ctx->lds_bytes < 160 * 1024)
+        (w_up ? (!w_up_extra || !y_xf || !y_xs) : !y) || (tile_blocks != 4 && tile_blocks != 8) || ctx->lds_bytes < 160 * 1024)
         return dfl_fail(ctx, DFLASH_ERR_UNSUPPORTED, "gemm_rows_experts: shape not taken or null operand");
     RowsArgs a = {};
     a.w[0] = static_cast<const uint8_t *>(w);
@@ -842,8 +855,9 @@ int32_t dfl_gemm_rows_experts(dflash_ctx *ctx, const void *w, const void *w_extr
     a.y_xs = static_cast<uint8_t *>(y_xs);
     a.y_kind = DFL_XF_Q4K;
     a.nb_out = static_cast<int>(n_out / DFL_QK_K);
-    a.n_ct = static_cast<int>(n_out / ((w_up ? 16 : 32) * kListWaves));
+    a.n_ct = static_cast<int>(n_out / ((w_up ? 16 : 32) * tile_blocks));  // (as many waves as a tile has row blocks at most)
     const int64_t tiles_max = static_cast<int64_t>(max_tiles) * a.n_ct;
-    return w_up ? rows_launch<TileQ4, false, false, 4, kEpiSwiglu, true>(ctx, a, tiles_max, st)
-                : rows_launch<TileQ4, false, false, 4, kEpiY, true>(ctx, a, tiles_max, st);
+    if (tile_blocks == 8)
+        return w_up ? rows_launch<TileQ4, false, false, 8, kEpiSwiglu, 8>(ctx, a, tiles_max, st) : rows_launch<TileQ4, false, false, 8, kEpiY, 8>(ctx, a, tiles_max, st);
+    return w_up ? rows_launch<TileQ4, false, false, 4, kEpiSwiglu, 4>(ctx, a, tiles_max, st) : rows_launch<TileQ4, false, false, 4, kEpiY, 4>(ctx, a, tiles_max, st);
 }

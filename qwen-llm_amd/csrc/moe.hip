@@ -491,16 +491,15 @@ __global__ void __launch_bounds__(1024)
 // order; behind them one slot per block of sixteen rows for the shared expert (rows 16 b .. 16 b + 15).
 //   *n_slots;  slot_rows[slot][16]: the rows whose activations the slot multiplies (unused places repeat
 //   row 0: computed, never read);  pick_pos[row][k] = 16 slot + place of the pick's output row;
-//   tiles[*n_tiles] = {expert (-1: the shared one), first slot, slots, 0}: runs of at most four slots of one expert, the
-//   row tiles of the expert products.
+//   tiles[*n_tiles] = {expert (-1: the shared one), first slot, slots, 0}: an expert's slots in runs of at most tile_slots, as
+//   even as they come (a tile of one slot unpacks its weights for that one alone), the row tiles of the expert products.
 // Places inside an expert's slots are handed out by an atomic counter, so they vary from run to run; no sum does.
 // One workgroup; n_rows * n_used <= 1024 kGroupPicksPerThread, n_expert <= 256.
 constexpr int kGroupPicksPerThread = 16;
-constexpr int kGroupTileSlots = 4;
 __global__ void __launch_bounds__(1024)
     moe_group_slots_kernel(const int32_t *__restrict__ sel_e, int n_rows, int n_used, int n_expert, int32_t *__restrict__ n_slots,
                            int32_t *__restrict__ slot_rows, int32_t *__restrict__ pick_pos, int4 *__restrict__ tiles,
-                           int32_t *__restrict__ n_tiles, int max_slots) {
+                           int32_t *__restrict__ n_tiles, int max_slots, int tile_slots) {
     __shared__ int cnt[256], base[257], wave_s[4], wave_t[4];
     const int tid = threadIdx.x, lane = tid & 63;
     if (tid < 256) cnt[tid] = 0;
@@ -516,7 +515,7 @@ __global__ void __launch_bounds__(1024)
     for (int j = 0; j < kGroupPicksPerThread; j++) my_place[j] = my_e[j] >= 0 ? atomicAdd(&cnt[my_e[j]], 1) : 0;
     __syncthreads();
     // exclusive prefix sums over the experts of their slots and of their row tiles (four waves, then across them)
-    const int c = tid < n_expert ? cnt[tid] : 0, ns = (c + 15) >> 4, nt = (ns + kGroupTileSlots - 1) / kGroupTileSlots;
+    const int c = tid < n_expert ? cnt[tid] : 0, ns = (c + 15) >> 4, nt = (ns + tile_slots - 1) / tile_slots;
     int ps = ns, pt = nt;
     for (int off = 1; off < 64; off <<= 1) {
         const int us = __shfl_up(ps, off, 64), ut = __shfl_up(pt, off, 64);
@@ -540,20 +539,24 @@ __global__ void __launch_bounds__(1024)
         total_t += wave_t[w];
     }
     if (tid < n_expert) base[tid] = ps - ns;
-    const int n_blocks = (n_rows + 15) >> 4, shared_t = (n_blocks + kGroupTileSlots - 1) / kGroupTileSlots;
+    const int n_blocks = (n_rows + 15) >> 4, shared_t = (n_blocks + tile_slots - 1) / tile_slots;
     if (tid == 0) {
         *n_slots = min(total + n_blocks, max_slots);  // (the host sizes max_slots for the worst case)
         *n_tiles = total_t + shared_t;
     }
     if (tid < n_expert) {
         const int b = ps - ns;
-        for (int t = 0; t < nt; t++)
-            tiles[pt - nt + t] = int4{tid, b + kGroupTileSlots * t, min(kGroupTileSlots, ns - kGroupTileSlots * t), 0};
+        for (int t = 0; t < nt; t++) {
+            const int first = ns * t / nt;
+            tiles[pt - nt + t] = int4{tid, b + first, ns * (t + 1) / nt - first, 0};
+        }
         if (c & 15)
             for (int m = c & 15; m < 16; m++) slot_rows[(b + (c >> 4)) * 16 + m] = 0;
     }
-    for (int t = tid; t < shared_t; t += 1024)
-        tiles[total_t + t] = int4{-1, total + kGroupTileSlots * t, min(kGroupTileSlots, n_blocks - kGroupTileSlots * t), 0};
+    for (int t = tid; t < shared_t; t += 1024) {
+        const int first = n_blocks * t / shared_t;
+        tiles[total_t + t] = int4{-1, total + first, n_blocks * (t + 1) / shared_t - first, 0};
+    }
     for (int r = tid; r < 16 * n_blocks; r += 1024) slot_rows[total * 16 + r] = min(r, n_rows - 1);
     __syncthreads();
 #pragma unroll
@@ -776,17 +779,21 @@ int32_t dfl_moe_ffn_group(dflash_ctx *ctx, const dflash_model_cfg &c, const dfla
     int32_t rc;
     if ((rc = dfl_router_rows(ctx, L.router.data, cur, s.logits, H, E, n_rows, st))) return rc;
     moe_group_route_kernel<<<(n_rows + 15) / 16, 1024, 0, st>>>(s.logits, n_rows, E, used, s.sel_e, s.sel_w);
+    // Row tiles of eight blocks (a workgroup of eight waves fills a CU) take in half the weights and fewer activations for a
+    // product, those of four (two workgroups on a CU) hide each other's waits and leave less of a tile empty.  128 experts top-8, gate
+    // and up + down in us, 4 : 8: 98 rows an expert (1500 tokens) 220 : 208, 128 rows 281 : 256; 62 rows 164 : 180, 25 rows 116 : 139.
+    const int tile_slots = n_rows * used >= 80 * E ? 8 : 4;
     moe_group_slots_kernel<<<1, 1024, 0, st>>>(s.sel_e, n_rows, used, E, s.n_slots, s.slot_rows, s.pick_pos, reinterpret_cast<int4 *>(s.tiles),
-                                             s.n_tiles, max_slots);
+                                             s.n_tiles, max_slots, tile_slots);
     moe_group_gather_kernel<<<dim3(H / DFL_QK_K, max_slots), 64, 0, st>>>(cur, s.slot_rows, s.n_slots, H, s.xg, s.xg_sums);
     const size_t stride_in = dflash_q4k_tiled_bytes(H, fe), stride_dn = dflash_q4k_tiled_bytes(fe, H);
-    // most row tiles the list can have: one per kGroupTileSlots slots, and a short one per expert and for the shared one
-    const int max_tiles = std::min(max_slots, max_slots / kGroupTileSlots + E + 1);
+    // most row tiles the list can have: one per tile_slots slots, and a short one per expert and for the shared one
+    const int max_tiles = std::min(max_slots, max_slots / tile_slots + E + 1);
     if ((rc = dfl_gemm_rows_experts(ctx, L.gate_exps.data, L.gate.data, L.up_exps.data, L.up.data, stride_in, s.xg, s.xg_sums, s.tiles, s.n_tiles,
-                                    max_tiles, nullptr, H, fe, s.act, s.act_sums, st)))
+                                    max_tiles, tile_slots, nullptr, H, fe, s.act, s.act_sums, st)))
         return rc;
     if ((rc = dfl_gemm_rows_experts(ctx, L.down_exps.data, L.down.data, nullptr, nullptr, stride_dn, s.act, s.act_sums, s.tiles, s.n_tiles,
-                                    max_tiles, s.eo, fe, H, nullptr, nullptr, st)))
+                                    max_tiles, tile_slots, s.eo, fe, H, nullptr, nullptr, st)))
         return rc;
     moe_combine_norm(n_rows, st, s.eo, s.pick_pos, s.sel_w, s.sg, nullptr, s.n_slots, used, H, x_resid, next_norm_w,
                                                     cur, c.eps, nullptr, next_xf, next_xf_kind, 1, next_xf_stride);
