@@ -228,12 +228,15 @@ __device__ static inline void dfl_xf_store_pair(void *xf, int kind, int m, int i
 // and / or as XF of kind y_xf_kind in y_xf (may be null), the activations of the down projection that follows.
 int dfl_whole_kind(const dflash_ctx *ctx, int32_t w_type, int64_t n_in, int64_t n_out, int64_t pair_ffn);
 int32_t dfl_gemm_whole(dflash_ctx *ctx, int32_t w_type, const void *w, const void *xf, float *y, int64_t n_in, int64_t n_out,
-                       int32_t n_rows, int64_t pair_ffn, void *y_xf, int y_xf_kind, hipStream_t stream);
+                       int32_t n_rows, int64_t pair_ffn, void *y_xf, int y_xf_kind, hipStream_t stream, bool by_sums = false);
+// by_sums: where dfl_whole_by_sums says so, minima through the activations' sub-block sums, as dfl_gemm_rows has them (a target's
+// layers); else through twin products (a drafter's, and the public operator).
+static inline bool dfl_whole_by_sums(int32_t w_type, int64_t n_in) { return w_type == DFLASH_TYPE_Q4_K_TILED && n_in >= 16 * DFL_QK_K; }
 // The same for n_rows_total rows, sixteen to a block (the last one may be shorter): block i's rows are in XF order at
 // xf + i * dfl_xf_bytes(n_in), its result at y + i * 16 * n_out (pair mode: 16 * pair_ffn; y_xf + i * dfl_xf_bytes(pair_ffn)).
 // The weights are read once and stay in registers while the blocks pass; a row's bits are those of dfl_gemm_whole.
 int32_t dfl_gemm_whole_blocks(dflash_ctx *ctx, int32_t w_type, const void *w, const void *xf, float *y, int64_t n_in, int64_t n_out,
-                              int32_t n_rows_total, int64_t pair_ffn, void *y_xf, int y_xf_kind, hipStream_t stream);
+                              int32_t n_rows_total, int64_t pair_ffn, void *y_xf, int y_xf_kind, hipStream_t stream, bool by_sums = false);
 // Whether a wave has one super-block of one tile, whose unpacked weights it then keeps from block to block.
 bool dfl_whole_holds_weights(const dflash_ctx *ctx, int32_t w_type, int64_t n_in, int64_t n_out);
 
@@ -242,18 +245,19 @@ bool dfl_whole_holds_weights(const dflash_ctx *ctx, int32_t w_type, int64_t n_in
 // arithmetics the matrix takes there and where K is cut.  kind == DFL_XF_NONE: not taken (only the tiled orders are).
 struct dfl_rows_plan {
     int kind;      // fragment order the activations must be in
-    int twin;      // whole-K kernel's arithmetic (no sub-block sums needed)
+    int whole;     // the 16-row kernel is the whole-K kernel (K is cut at its slices)
+    int sums;      // the activations' sub-block sums are needed (else: twin products)
     int total, n_cut, by_group;
 };
 dfl_rows_plan dfl_gemm_rows_plan(const dflash_ctx *ctx, int32_t w_type, int64_t n_in, int64_t n_out, int64_t pair_ffn);
-// Sub-block sums of n_blocks blocks of rows in fragment order (kind Q4K), for the plans without `twin`:
+// Sub-block sums of n_blocks blocks of rows in fragment order (kind Q4K), for the plans with `sums`:
 // dfl_xs_bytes(n_in) bytes per block.
 static inline size_t dfl_xs_bytes(int64_t n_in) { return static_cast<size_t>(n_in / 256) * 1024; }
 int32_t dfl_xf_sums(dflash_ctx *ctx, const void *xf, int64_t n_in, int32_t n_blocks, void *xs, hipStream_t stream);
 // y[n_rows][n_out] = X . W^T, block b of sixteen rows at xf + b * dfl_xf_bytes(n_in) (sums: xs + b * dfl_xs_bytes(n_in)).
 // pair_ffn > 0: W is a fused gate | up matrix and silu(gate) * up goes to y_xf in fragment order y_kind (and its sub-block
-// sums to y_xs unless null) instead.
-int32_t dfl_gemm_rows(dflash_ctx *ctx, const dfl_rows_plan &plan, int32_t w_type, const void *w, const void *xf, const void *xs, float *y,
+// sums to y_xs unless null) instead.  make_sums: xs is to be computed first, where the plan needs it.
+int32_t dfl_gemm_rows(dflash_ctx *ctx, const dfl_rows_plan &plan, int32_t w_type, const void *w, const void *xf, void *xs, bool make_sums, float *y,
                       int64_t n_in, int64_t n_out, int32_t n_rows, int64_t pair_ffn, void *y_xf, void *y_xs, int y_kind, hipStream_t stream);
 // The experts' products over row tiles listed on the device, tiles[i] = {expert (-1: the extra matrix), first block,
 // blocks (1..tile_blocks, which is 4 or 8), -}: the arithmetic of gemm_q4k_experts_kernel.  w_up != null: silu(x . w^T) * (x . w_up^T) to y_xf / y_xs.

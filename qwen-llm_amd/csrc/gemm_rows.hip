@@ -21,9 +21,9 @@
 // Workgroups that share weights are dispatched to one XCD (rows_linear), so that a matrix passes through one L2.
 // Measured for 1000 rows, before (a whole super-block's copies behind a barrier, the compiler's waits: every LDS read waited
 // for ahead of its two products) and now, six layers of a prompt: 5120 -> 2 x 17408 with SwiGLU 429 -> 364 us (0.98
-// PFLOP/s, matrix cores busy for 57 % of the cycles, 42 % before), 17408 -> 5120 233 -> 193 us (0.92), 5120 -> 6144 and 4096 ->
-// 5120 together 240 -> 210 us (0.50: their twin MFMAs, which the block path's bits ask for, are as many again); 2048 rows:
-// 2048 -> 5120 and 4096 -> 2048 in Q6_K together 220 -> 186 us.  A 64-layer prompt of 1000 rows 64.7 -> 59.7 ms.
+// PFLOP/s, matrix cores busy for 57 % of the cycles, 42 % before), 17408 -> 5120 233 -> 193 us (0.92), 5120 -> 6144 105 -> 76 us
+// (0.82; the 105 with a twin MFMA for every product, which the block path's bits then asked for); 2048 rows: 2048 -> 5120 and
+// 4096 -> 2048 in Q6_K, still with twins, together 220 -> 186 us.  A 64-layer prompt of 1000 rows 64.7 -> 59.7 ms, 53.5 without the twins.
 // The experts' tiles (a list) take workgroups of half the columns and up to four row blocks, two of them on a CU, each
 // waiting for its own weights while the other computes, or, where an expert has rows enough, of all columns and up to eight blocks
 // (the rule and both sides' figures stand in dfl_moe_ffn_group).
@@ -197,7 +197,7 @@ struct TileQ6 {
     __device__ __forceinline__ half8_t twin(int t) const {
         return splat8(s[2 * H + (t >> 1)] * static_cast<_Float16>(32.0f));
     }
-    __device__ __forceinline__ half8_t minima() const { return splat8(static_cast<_Float16>(0.0f)); }
+    __device__ __forceinline__ half8_t minima() const { return splat8(static_cast<_Float16>(0.0f)); }  // (named, never asked for)
 };
 
 // this wave's reads from LDS are done, and everybody has come this far
@@ -225,8 +225,8 @@ struct RowsLds {
     static constexpr int sums = 3 * kHalf, w = sums + 2 * kSums, total = w + W * kW;
 };
 
-// kTwin: the minima / offsets through a twin MFMA per activation fragment into a second accumulator (the whole-K
-// kernel's arithmetic); else one MFMA per super-block over the sub-block sums (the streaming and expert kernels').
+// kTwin: the minima / offsets through a twin MFMA per activation fragment into a second accumulator (the whole-K kernel's
+// arithmetic for Q6_K and short K); else one MFMA per super-block over the sub-block sums.
 // kCut: K is cut somewhere.  RB: 16-row blocks of the tile.
 template <typename Tile, bool kTwin, bool kCut, int RB, int kEpi, int kList>
 __global__ void __launch_bounds__(64 * (kList ? kList : kRowsWaves), 2) gemm_rows_kernel(RowsArgs a) {
@@ -354,7 +354,7 @@ __global__ void __launch_bounds__(64 * (kList ? kList : kRowsWaves), 2) gemm_row
                 o[j] = tile[j].minima();
             } else {
                 o[j] = tile[j].template operand<step / 4>(step % 4, magic);
-                if (kTwin) o[2 + j] = tile[j].template twin<step / 4>(step % 4);
+                if constexpr (kTwin) o[2 + j] = tile[j].template twin<step / 4>(step % 4);
             }
         }
     };
@@ -528,7 +528,7 @@ __global__ void __launch_bounds__(64 * (kList ? kList : kRowsWaves), 2) gemm_row
         for (int h = 0; h < 2; h++)
 #pragma unroll
             for (int j = 0; j < kX; j++) copy_x(rows, 2 * b_begin + h, h, j);
-        copies_done<0>();
+        copies_done<kX>();  // (all but the second half)
         tile[0].template read<0>(w_at);
         tile[1].template read<Tile::kBytes>(w_at);
         landed_for_all();
@@ -690,7 +690,8 @@ dfl_rows_plan dfl_gemm_rows_plan(const dflash_ctx *ctx, int32_t w_type, int64_t 
     const int kind = dfl_whole_kind(ctx, w_type, n_in, n_out, pair_ffn);
     if (kind != DFL_XF_NONE) {
         p.kind = kind;
-        p.twin = 1;
+        p.whole = 1;
+        p.sums = dfl_whole_by_sums(w_type, n_in);
         p.total = nb;
         p.n_cut = nb < 16 ? nb : 16;  // the whole-K kernel's slices
         return p;
@@ -699,6 +700,7 @@ dfl_rows_plan dfl_gemm_rows_plan(const dflash_ctx *ctx, int32_t w_type, int64_t 
     int total = 0, n_wg = 0;
     if (!dfl_q4k_tiled_split(ctx, n_in, n_out, &total, &n_wg)) return p;
     p.kind = DFL_XF_Q4K;
+    p.sums = 1;
     p.total = total;
     p.n_cut = n_wg;
     p.by_group = 1;
@@ -764,9 +766,9 @@ int32_t rows_dispatch(dflash_ctx *ctx, const RowsArgs &a, int rb, int64_t tiles,
 }
 }  // namespace
 
-int32_t dfl_gemm_rows(dflash_ctx *ctx, const dfl_rows_plan &p, int32_t w_type, const void *w, const void *xf, const void *xs, float *y,
+int32_t dfl_gemm_rows(dflash_ctx *ctx, const dfl_rows_plan &p, int32_t w_type, const void *w, const void *xf, void *xs, bool make_sums, float *y,
                       int64_t n_in, int64_t n_out, int32_t n_rows, int64_t pair_ffn, void *y_xf, void *y_xs, int y_kind, hipStream_t st) {
-    if (p.kind == DFL_XF_NONE || !w || !xf || n_rows < 1 || (!p.twin && !xs) || (pair_ffn ? !y_xf : !y))
+    if (p.kind == DFL_XF_NONE || !w || !xf || n_rows < 1 || (p.sums && !xs) || (pair_ffn ? !y_xf : !y))
         return dfl_fail(ctx, DFLASH_ERR_UNSUPPORTED, "gemm_rows: shape not taken or null operand");
     if (reinterpret_cast<uintptr_t>(w) % 16 || reinterpret_cast<uintptr_t>(xf) % 16 || reinterpret_cast<uintptr_t>(xs) % 16 ||
         reinterpret_cast<uintptr_t>(y_xf) % 16 || reinterpret_cast<uintptr_t>(y_xs) % 16)
@@ -789,11 +791,16 @@ int32_t dfl_gemm_rows(dflash_ctx *ctx, const dfl_rows_plan &p, int32_t w_type, c
     a.y_kind = y_kind;
     a.nb_out = static_cast<int>(pair_ffn / DFL_QK_K);
     a.n_ct = static_cast<int>(pair_ffn ? pair_ffn / 128 : (n_out + 255) / 256);
-    const int most = p.twin ? 4 : 8;
-    int rb = rows_pick_rb(ctx, a.n_blocks, a.n_ct, most);
+    const bool q6 = w_type == DFLASH_TYPE_Q6_K_TILED;
+    const int most = p.sums ? 8 : 4;  // (a twin product's second accumulators)
+    const int rb = rows_pick_rb(ctx, a.n_blocks, a.n_ct, most);
     a.n_rt = (a.n_blocks + rb - 1) / rb;
     int64_t tiles = static_cast<int64_t>(a.n_ct) * a.n_rt;
-    if (pair_ffn) return p.twin ? rows_dispatch<TileQ4, true, kEpiSwiglu>(ctx, a, rb, tiles, st) : rows_dispatch<TileQ4, false, kEpiSwiglu>(ctx, a, rb, tiles, st);
+    auto sums = [&]() -> int32_t { return p.sums && make_sums ? dfl_xf_sums(ctx, xf, n_in, a.n_blocks, xs, st) : DFLASH_OK; };
+    if (pair_ffn) {
+        if (const int32_t rc = sums()) return rc;
+        return p.sums ? rows_dispatch<TileQ4, false, kEpiSwiglu>(ctx, a, rb, tiles, st) : rows_dispatch<TileQ4, true, kEpiSwiglu>(ctx, a, rb, tiles, st);
+    }
     // Tiles for less than half the chip: K is shared by several workgroups, each range between two cuts on its own (as
     // many as there are at least in every tile group), where the workspace holds the partial products.
     const int ranges = p.by_group ? std::max(1, static_cast<int>(static_cast<int64_t>(a.nb) * a.n_cut / a.total)) : a.n_cut;
@@ -811,25 +818,29 @@ int32_t dfl_gemm_rows(dflash_ctx *ctx, const dfl_rows_plan &p, int32_t w_type, c
         // so: twelve blocks for matrices of 80 super-blocks x column tiles or more, four for smaller ones, none where the
         // weights are not held.
         const int whole_most = a.nb * a.n_ct >= 80 ? 12 : 4;
-        if (p.twin && a.n_blocks <= whole_most && dfl_whole_holds_weights(ctx, w_type, n_in, n_out))
-            return dfl_gemm_whole_blocks(ctx, w_type, w, xf, y, n_in, n_out, n_rows, 0, nullptr, 0, st);
+        if (p.whole && a.n_blocks <= whole_most && dfl_whole_holds_weights(ctx, w_type, n_in, n_out))
+            return dfl_gemm_whole_blocks(ctx, w_type, w, xf, y, n_in, n_out, n_rows, 0, nullptr, 0, st, true);
         a.n_split = std::min<int>(ranges, static_cast<int>(ctx->n_cu / tiles));
         size_t off = 0;
         float *part = dfl_ws_take<float>(ctx, &off, static_cast<size_t>(most_ranges) * a.n_blocks * 16 * n_out * sizeof(float));
         if (part && a.n_split > 1) {
             a.y = part;
             tiles *= a.n_split;
-            const int32_t rc = w_type == DFLASH_TYPE_Q6_K_TILED ? rows_dispatch<TileQ6, true, kEpiSplit>(ctx, a, rb, tiles, st)
-                               : p.twin                         ? rows_dispatch<TileQ4, true, kEpiSplit>(ctx, a, rb, tiles, st)
-                                                                : rows_dispatch<TileQ4, false, kEpiSplit>(ctx, a, rb, tiles, st);
+            int32_t rc = sums();
+            if (!rc)
+                rc = q6       ? rows_dispatch<TileQ6, true, kEpiSplit>(ctx, a, rb, tiles, st)
+                     : p.sums ? rows_dispatch<TileQ4, false, kEpiSplit>(ctx, a, rb, tiles, st)
+                              : rows_dispatch<TileQ4, true, kEpiSplit>(ctx, a, rb, tiles, st);
             if (rc) return rc;
             rows_reduce_kernel<<<dim3(static_cast<unsigned>((n_out + 1023) / 1024), n_rows), 256, 0, st>>>(a, part, y);
             DFL_HIP_CHECK(ctx, hipGetLastError());
             return DFLASH_OK;
         }
     }
-    if (w_type == DFLASH_TYPE_Q6_K_TILED) return rows_dispatch<TileQ6, true, kEpiY>(ctx, a, rb, tiles, st);
-    return p.twin ? rows_dispatch<TileQ4, true, kEpiY>(ctx, a, rb, tiles, st) : rows_dispatch<TileQ4, false, kEpiY>(ctx, a, rb, tiles, st);
+    if (const int32_t rc = sums()) return rc;
+    return q6       ? rows_dispatch<TileQ6, true, kEpiY>(ctx, a, rb, tiles, st)
+           : p.sums ? rows_dispatch<TileQ4, false, kEpiY>(ctx, a, rb, tiles, st)
+                    : rows_dispatch<TileQ4, true, kEpiY>(ctx, a, rb, tiles, st);
 }
 
 int32_t dfl_gemm_rows_experts(dflash_ctx *ctx, const void *w, const void *w_extra, const void *w_up, const void *w_up_extra, size_t w_stride,

@@ -19,7 +19,11 @@
 //
 // Arithmetic: that of the streaming kernels (exact f16 integers from the quant bits, one packed fma with
 // s = d * scale, f32 accumulation on v_mfma_f32_16x16x32_f16; the Q4_K minima and the Q6_K offset through a twin MFMA
-// of the same activation fragment into a second accumulator that is subtracted at the end).
+// of the same activation fragment into a second accumulator that is subtracted at the end).  Where a target's Q4_K matrix
+// has 16 super-blocks of K or more (Q4S) the minima go by one MFMA over the activations' sub-block sums ahead of the
+// eight: the same MFMAs are what a prompt's many-row product is made of (gemm_rows.hip, whose rows have this kernel's bits),
+// and twins are half of them there.  The sums cost a wave 90 vector instructions a stage (4096 -> 5120 and 5120 -> 6144 9.1 -> 9.4 us a
+// launch); matrices of short K, where a launch is 4 us and a prompt's product as short, keep the twins.
 #include "common.h"
 #include "mfma_unpack.h"
 
@@ -98,6 +102,26 @@ __device__ __forceinline__ void compute(const Q4W &r, const half8_t (&af)[8], in
     }
 }
 
+// The minima by the sums of the activations (the A operand of gemm_rows.hip's xf_sums_kernel, bit for bit): a lane's eight
+// fragments are eight octets of its row, the first four one sub-block and the last four the next.
+struct Q4S : Q4W {};
+// h0 + h1 and h2 + h3 of a fragment's half (dwords (h0, h2) and (h1, h3)), each one rounding to f32
+__device__ __forceinline__ float pair_sums(uint32_t a, uint32_t b) {
+    float lo, hi;
+    asm("v_fma_mix_f32 %0, %1, 1.0, %2 op_sel_hi:[1,0,1]" : "=v"(lo) : "v"(a), "v"(b));
+    asm("v_fma_mix_f32 %0, %1, 1.0, %2 op_sel:[1,0,1] op_sel_hi:[1,0,1]" : "=v"(hi) : "v"(a), "v"(b));
+    return lo + hi;
+}
+__device__ __forceinline__ half8_t sum_operand(const half8_t (&af)[8]) {
+    float o[8];
+#pragma unroll
+    for (int t = 0; t < 8; t++) {
+        const u32x4_t f = __builtin_bit_cast(u32x4_t, af[t]);
+        o[t] = pair_sums(f.x, f.y) + pair_sums(f.z, f.w);
+    }
+    return q4k_sum_operand((o[0] + o[1]) + (o[2] + o[3]), (o[4] + o[5]) + (o[6] + o[7]));
+}
+
 // The same in two steps, for a launch that multiplies many row blocks with one set of weights: the B operands of a
 // super-block's eight MFMAs once (unpack), then only the MFMAs per row block (mma), in compute()'s order.
 struct Q4F {
@@ -138,6 +162,20 @@ __device__ __forceinline__ void mma(const Q4F &f, const half8_t (&af)[8], float4
         acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[t], f.b[t], acc, 0, 0, 0);
         acc_sub = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[t], t < 4 ? bml : bmh, acc_sub, 0, 0, 0);
     }
+}
+
+struct Q4SF : Q4F {};
+__device__ __forceinline__ void mma(const Q4SF &f, const half8_t (&af)[8], float4_t &acc, float4_t &) {
+    const half2_t m = {-f.m_lo, -f.m_hi};
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(sum_operand(af), q4k_min_operand(m), acc, 0, 0, 0);
+#pragma unroll
+    for (int t = 0; t < 8; t++) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[t], f.b[t], acc, 0, 0, 0);
+}
+__device__ __forceinline__ void compute(const Q4S &r, const half8_t (&af)[8], int lane, uint8_t *area, uint32_t sc_sel, Q4KMagic magic,
+                                        float4_t &acc, float4_t &acc_sub) {
+    Q4SF f;
+    unpack(r, lane, area, sc_sel, magic, f);
+    mma(f, af, acc, acc_sub);
 }
 
 // ---- Q6_K, GGUF row order: 210-byte blocks (ql[128], qh[64], scales[16], d), rows 2-byte aligned ----
@@ -312,6 +350,10 @@ struct FragsOf;
 template <>
 struct FragsOf<Q4W> {
     typedef Q4F type;
+};
+template <>
+struct FragsOf<Q4S> {
+    typedef Q4SF type;
 };
 template <>
 struct FragsOf<Q6W> {
@@ -667,12 +709,12 @@ bool dfl_whole_holds_weights(const dflash_ctx *ctx, int32_t w_type, int64_t n_in
 }
 
 int32_t dfl_gemm_whole(dflash_ctx *ctx, int32_t w_type, const void *w, const void *xf, float *y, int64_t n_in, int64_t n_out,
-                       int32_t n_rows, int64_t pair_ffn, void *y_xf, int y_xf_kind, hipStream_t st) {
-    return dfl_gemm_whole_blocks(ctx, w_type, w, xf, y, n_in, n_out, n_rows, pair_ffn, y_xf, y_xf_kind, st);
+                       int32_t n_rows, int64_t pair_ffn, void *y_xf, int y_xf_kind, hipStream_t st, bool by_sums) {
+    return dfl_gemm_whole_blocks(ctx, w_type, w, xf, y, n_in, n_out, n_rows, pair_ffn, y_xf, y_xf_kind, st, by_sums);
 }
 
 int32_t dfl_gemm_whole_blocks(dflash_ctx *ctx, int32_t w_type, const void *w, const void *xf, float *y, int64_t n_in, int64_t n_out,
-                              int32_t n_rows_total, int64_t pair_ffn, void *y_xf, int y_xf_kind, hipStream_t st) {
+                              int32_t n_rows_total, int64_t pair_ffn, void *y_xf, int y_xf_kind, hipStream_t st, bool by_sums) {
     const int32_t n_blocks = (n_rows_total + 15) / 16;
     const int32_t n_rows = n_rows_total - 16 * (n_blocks - 1);  // rows of the last block
     if (n_rows_total < 1 || n_blocks > 4096) return dfl_fail(ctx, DFLASH_ERR_BAD_SHAPE, "gemm_whole: %d rows", n_rows_total);
@@ -728,9 +770,13 @@ int32_t dfl_gemm_whole_blocks(dflash_ctx *ctx, int32_t w_type, const void *w, co
         DFL_HIP_CHECK(ctx, hipGetLastError());
         return DFLASH_OK;
     }
+    by_sums = by_sums && dfl_whole_by_sums(w_type, n_in);
     const int multi = n_blocks > 1 ? (a.nb > p.ksplit ? 2 : 1) : 0;
+    if (multi && by_sums && (p.R != 1 || multi != 1))
+        return dfl_fail(ctx, DFLASH_ERR_UNSUPPORTED, "gemm_whole: several blocks by sums only past weights a wave holds");
 #define DFL_WHOLE_PICK(WT, RR) (multi == 0 ? gemm_whole_kernel<WT, RR, 0> : multi == 1 ? gemm_whole_kernel<WT, RR, 1> : gemm_whole_kernel<WT, RR, 2>)
-    const kernel_t fn = p.kind == DFL_XF_Q4K ? (p.R == 2 ? DFL_WHOLE_PICK(Q4W, 2) : DFL_WHOLE_PICK(Q4W, 1))
+    const kernel_t fn = p.kind == DFL_XF_Q4K && by_sums ? (p.R == 2 ? gemm_whole_kernel<Q4S, 2, 0> : multi ? gemm_whole_kernel<Q4S, 1, 1> : gemm_whole_kernel<Q4S, 1, 0>)
+                        : p.kind == DFL_XF_Q4K          ? (p.R == 2 ? DFL_WHOLE_PICK(Q4W, 2) : DFL_WHOLE_PICK(Q4W, 1))
                         : q6_tiled           ? (p.R == 2 ? DFL_WHOLE_PICK(Q6T, 2) : DFL_WHOLE_PICK(Q6T, 1))
                                              : (p.R == 2 ? DFL_WHOLE_PICK(Q6W, 2) : DFL_WHOLE_PICK(Q6W, 1));
 #undef DFL_WHOLE_PICK

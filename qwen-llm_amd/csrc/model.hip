@@ -8,6 +8,7 @@
 // kernels/rope.metal:96-121, kernels/elementwise.metal:89, 193, 674-685, 727-900.
 #include "common.h"
 #include "device_quant.h"
+#include "mfma_unpack.h"
 
 #include <algorithm>
 #include <array>
@@ -69,7 +70,7 @@ __global__ void __launch_bounds__(256) rms_norm_kernel(float *__restrict__ x, co
                                                        const float *__restrict__ w, float *__restrict__ y, int n,
                                                        float eps, const float *__restrict__ gate_w,
                                                        float *__restrict__ gate_out, void *__restrict__ y_xf,
-                                                       int y_xf_kind, size_t xf_stride, ConvResid conv) {
+                                                       int y_xf_kind, size_t xf_stride, ConvResid conv, void *__restrict__ y_xs) {
     typedef norm_f4 f4;
     __shared__ float sh[4], sh_dot[4];
     const int t = blockIdx.x, tid = threadIdx.x;
@@ -157,6 +158,29 @@ __global__ void __launch_bounds__(256) rms_norm_kernel(float *__restrict__ x, co
             if (y_xf)
                 dfl_xf_store_pair(static_cast<uint8_t *>(y_xf) + (t >> 4) * xf_stride, y_xf_kind, t & 15, i & ~7, o[0],
                                   o[1], o[2], o[3]);
+            if (y_xs) {
+                // the sums of the sub-blocks of 32 rounded values (eight lanes), as xf_sums_kernel adds and stores them
+                _Float16 h[4];
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    float e = o[k];
+                    asm volatile("" : "+v"(e));  // (rounded to f32 first, as what is stored: the product is not fused into the conversion)
+                    h[k] = static_cast<_Float16>(e);
+                }
+                float sub = (static_cast<float>(h[0]) + static_cast<float>(h[1])) + (static_cast<float>(h[2]) + static_cast<float>(h[3]));
+                sub += dfl_dpp<0xB1>(sub);
+                sub += dfl_dpp<0x4E>(sub);
+                sub += dfl_xor4(sub);
+                if ((tid & 7) == 0) {
+                    const int jj = (i >> 5) & 7;
+                    _Float16 *to = static_cast<_Float16 *>(y_xs) + (static_cast<size_t>(t >> 4) * (n >> 8) + (i >> 8)) * 512 + ((t & 15) + 16 * (jj >> 1)) * 8 + (jj & 1);
+                    const Q4KSumParts parts = q4k_sum_parts(sub);
+                    to[0] = parts.hi;
+                    to[2] = parts.lo;
+                    to[4] = parts.over;
+                    to[6] = static_cast<_Float16>(0.0f);
+                }
+            }
             if (gate_w) dot += (o[0] * gw[j][0] + o[1] * gw[j][1]) + (o[2] * gw[j][2] + o[3] * gw[j][3]);
         }
     }
@@ -202,7 +226,7 @@ __global__ void __launch_bounds__(256) rms_norm_any_kernel(float *__restrict__ x
 }
 
 void rms_norm(int rows, hipStream_t st, float *x, const float *add, const float *w, float *y, int n, float eps, const float *gate_w,
-              float *gate_out, void *y_xf = nullptr, int y_xf_kind = 0, size_t xf_stride = 0, ConvResid conv = ConvResid()) {
+              float *gate_out, void *y_xf = nullptr, int y_xf_kind = 0, size_t xf_stride = 0, ConvResid conv = ConvResid(), void *y_xs = nullptr) {
     if (!norm_in_registers(n)) {
         rms_norm_any_kernel<<<rows, 256, 0, st>>>(x, add, w, y, n, eps, gate_w, gate_out);
         return;
@@ -210,9 +234,9 @@ void rms_norm(int rows, hipStream_t st, float *x, const float *add, const float 
 #define DFL_NORM(V)                                                                                                          \
     do {                                                                                                                     \
         if (conv.dyn && add)                                                                                                 \
-            rms_norm_kernel<V, true><<<rows, 256, 0, st>>>(x, add, w, y, n, eps, gate_w, gate_out, y_xf, y_xf_kind, xf_stride, conv); \
+            rms_norm_kernel<V, true><<<rows, 256, 0, st>>>(x, add, w, y, n, eps, gate_w, gate_out, y_xf, y_xf_kind, xf_stride, conv, y_xs); \
         else                                                                                                                 \
-            rms_norm_kernel<V, false><<<rows, 256, 0, st>>>(x, add, w, y, n, eps, gate_w, gate_out, y_xf, y_xf_kind, xf_stride, conv); \
+            rms_norm_kernel<V, false><<<rows, 256, 0, st>>>(x, add, w, y, n, eps, gate_w, gate_out, y_xf, y_xf_kind, xf_stride, conv, y_xs); \
     } while (0)
     switch ((n + 1023) / 1024) {
         case 1: DFL_NORM(1); break;
@@ -671,10 +695,10 @@ LayerXf layer_xf(const dflash_ctx *ctx, const LayerT &L, bool packed_qkv_allowed
 // layer_xf: implies adjacent weights): the rows are in x_xf in fragment order and the whole-K kernel takes them.
 int32_t gemm_qkv(dflash_ctx *ctx, const dflash_qtensor &wq, const dflash_qtensor &wk, const dflash_qtensor &wv, const float *x,
                  float *q, float *k, float *v, float *pk, bool allow_packed, bool *packed, int64_t n_in, int64_t q_dim,
-                 int64_t kv_dim, int n, hipStream_t st, const void *x_xf = nullptr, int xf_kind = DFL_XF_NONE) {
+                 int64_t kv_dim, int n, hipStream_t st, const void *x_xf = nullptr, int xf_kind = DFL_XF_NONE, bool by_sums = false) {
     *packed = allow_packed && pk && adjacent(wq, q_dim, wk, n_in) && adjacent(wk, kv_dim, wv, n_in);
     if (*packed && xf_kind != DFL_XF_NONE && x_xf)
-        return dfl_gemm_whole(ctx, wq.type, wq.data, x_xf, pk, n_in, q_dim + 2 * kv_dim, n, 0, nullptr, DFL_XF_NONE, st);
+        return dfl_gemm_whole(ctx, wq.type, wq.data, x_xf, pk, n_in, q_dim + 2 * kv_dim, n, 0, nullptr, DFL_XF_NONE, st, by_sums);
     if (*packed) return gemm(ctx, wq, x, pk, n_in, q_dim + 2 * kv_dim, n, st);
     if (wq.type == DFLASH_TYPE_Q6_K && wk.type == DFLASH_TYPE_Q6_K && wv.type == DFLASH_TYPE_Q6_K && n_in % DFL_QK_K == 0) {
         const void *w[3] = {wq.data, wk.data, wv.data};
@@ -693,11 +717,11 @@ int32_t gemm_qkv(dflash_ctx *ctx, const dflash_qtensor &wq, const dflash_qtensor
 // activation in its epilogue; g_xf / g_xf_kind: the result also goes there in the order the down projection reads.
 int32_t gemm_gate_up(dflash_ctx *ctx, const dflash_qtensor &gate, const dflash_qtensor &up, const float *x, float *g, float *u,
                      float *pk, int64_t n_in, int64_t ffn, int n, hipStream_t st, const void *x_xf = nullptr,
-                     int xf_kind = DFL_XF_NONE, void *g_xf = nullptr, int g_xf_kind = DFL_XF_NONE) {
+                     int xf_kind = DFL_XF_NONE, void *g_xf = nullptr, int g_xf_kind = DFL_XF_NONE, bool by_sums = false) {
     int32_t rc;
     if (xf_kind != DFL_XF_NONE && x_xf)
         return dfl_gemm_whole(ctx, gate.type, gate.data, x_xf, g, n_in, 2 * ffn, n, ffn, g_xf_kind != DFL_XF_NONE ? g_xf : nullptr,
-                              g_xf_kind, st);
+                              g_xf_kind, st, by_sums);
     if (pk && adjacent(gate, ffn, up, n_in)) {
         // (a product split over K applies the activation in its reduction: one launch less)
         ctx->swiglu_out = ffn % 16 == 0 ? g : nullptr;
@@ -1068,7 +1092,7 @@ int32_t verify_enqueue(dflash_ctx *ctx, const dflash_model *model, dflash_sessio
         pending_resid = nullptr;
         cur_ready = false;
         bool packed;
-        if ((rc = gemm_qkv(ctx, L.wq, L.wk, L.wv, s->cur, s->q, s->k, s->v, s->pk, true, &packed, H, q_dim, kv_dim, n, st, s->xf_cur, xk.qkv)))
+        if ((rc = gemm_qkv(ctx, L.wq, L.wk, L.wv, s->cur, s->q, s->k, s->v, s->pk, true, &packed, H, q_dim, kv_dim, n, st, s->xf_cur, xk.qkv, true)))
             return rc;
         const int64_t tot = q_dim + 2 * kv_dim;
         qk_norm_rope(hd, c.n_q + 2 * c.n_kv, n, st, packed ? s->pk : s->q, packed ? tot : q_dim, packed ? s->pk + q_dim : s->k, packed ? tot : kv_dim, s->q, s->k, L.q_norm,
@@ -1094,7 +1118,7 @@ int32_t verify_enqueue(dflash_ctx *ctx, const dflash_model *model, dflash_sessio
                                  s->attn, st, 0, 0, ctx->capturing ? s->pos : nullptr, xk.wo ? s->xf_attn : nullptr, xk.wo)))
             return rc;
         if (xk.wo)
-            rc = dfl_gemm_whole(ctx, L.wo.type, L.wo.data, s->xf_attn, s->mix, static_cast<int64_t>(q_dim), H, n, 0, nullptr, DFL_XF_NONE, st);
+            rc = dfl_gemm_whole(ctx, L.wo.type, L.wo.data, s->xf_attn, s->mix, static_cast<int64_t>(q_dim), H, n, 0, nullptr, DFL_XF_NONE, st, true);
         else
             rc = gemm(ctx, L.wo, s->attn, s->mix, q_dim, H, n, st);
         if (rc) return rc;
@@ -1115,10 +1139,10 @@ int32_t verify_enqueue(dflash_ctx *ctx, const dflash_model *model, dflash_sessio
         } else {
             // the down projection reads fragment-order rows only where the gate/up launch can write them
             const int down_kind = xk.gate_up ? xk.down : DFL_XF_NONE;
-            if ((rc = gemm_gate_up(ctx, L.gate, L.up, s->cur, s->g, s->u, s->pk, H, c.ffn, n, st, s->xf_cur, xk.gate_up, s->xf_g, down_kind)))
+            if ((rc = gemm_gate_up(ctx, L.gate, L.up, s->cur, s->g, s->u, s->pk, H, c.ffn, n, st, s->xf_cur, xk.gate_up, s->xf_g, down_kind, true)))
                 return rc;
             if (down_kind)
-                rc = dfl_gemm_whole(ctx, L.down.type, L.down.data, s->xf_g, s->mix, c.ffn, H, n, 0, nullptr, DFL_XF_NONE, st);
+                rc = dfl_gemm_whole(ctx, L.down.type, L.down.data, s->xf_g, s->mix, c.ffn, H, n, 0, nullptr, DFL_XF_NONE, st, true);
             else
                 rc = gemm(ctx, L.down, s->g, s->mix, c.ffn, H, n, st);
             if (rc) return rc;
@@ -1417,7 +1441,6 @@ int32_t prefill_group_enqueue(dflash_ctx *ctx, const dflash_model *model, dflash
     const size_t q_dim = static_cast<size_t>(c.n_q) * hd, kv_dim = static_cast<size_t>(c.n_kv) * hd;
     const int64_t tot = static_cast<int64_t>(q_dim + 2 * kv_dim);
     const size_t xf_h = dfl_xf_bytes(H);
-    const int n_blocks = (n + 15) / 16;
     for (int at = 0; at < n; at += kGroupIdsPerLaunch) {
         const int m = std::min(kGroupIdsPerLaunch, n - at);
         IntGroupArgs ids_arg = {};
@@ -1428,11 +1451,10 @@ int32_t prefill_group_enqueue(dflash_ctx *ctx, const dflash_model *model, dflash
     if (rc) return rc;
     const float scale = 1.0f / sqrtf(static_cast<float>(hd));
     const size_t per_layer = static_cast<size_t>(s->capacity) * kv_dim;
-    // a many-row product of rows that are in fragment order, with their sub-block sums made first where its arithmetic wants them
-    auto product = [&](const dfl_rows_plan &p, const dflash_qtensor &w, const uint8_t *xf, uint8_t *xs, float *y, int64_t n_in, int64_t n_out) -> int32_t {
-        if (!p.twin)
-            if (const int32_t r = dfl_xf_sums(ctx, xf, n_in, n_blocks, xs, st)) return r;
-        return dfl_gemm_rows(ctx, p, w.type, w.data, xf, xs, y, n_in, n_out, n, 0, nullptr, nullptr, 0, st);
+    // a many-row product of rows that are in fragment order (make_sums: no kernel before has left their sub-block sums)
+    auto product = [&](const dfl_rows_plan &p, const dflash_qtensor &w, const uint8_t *xf, uint8_t *xs, bool make_sums, float *y, int64_t n_in,
+                       int64_t n_out) -> int32_t {
+        return dfl_gemm_rows(ctx, p, w.type, w.data, xf, xs, make_sums, y, n_in, n_out, n, 0, nullptr, nullptr, 0, st);
     };
     const float *pending_resid = nullptr;  // a dense layer's FFN output still to be added to g.x
     LayerRows rows = layer_rows(ctx, c, model->layers[0]), next_rows;
@@ -1441,9 +1463,10 @@ int32_t prefill_group_enqueue(dflash_ctx *ctx, const dflash_model *model, dflash
         _Float16 *kc = s->k_cache + il * per_layer, *vtc = s->vt_cache + il * per_layer;
         next_rows = il + 1 < c.n_layers ? layer_rows(ctx, c, model->layers[il + 1]) : LayerRows();
         if (!moe || il == 0)  // (a mixture's later layers: the experts' last kernel has normalised their input)
-            rms_norm(n, st, g.x, pending_resid, L.attn_norm, g.cur, H, c.eps, nullptr, nullptr, g.xf_cur, rows.qkv.kind, xf_h);
+            rms_norm(n, st, g.x, pending_resid, L.attn_norm, g.cur, H, c.eps, nullptr, nullptr, g.xf_cur, rows.qkv.kind, xf_h, ConvResid(),
+                     rows.qkv.sums ? g.xs_cur : nullptr);
         pending_resid = nullptr;
-        if ((rc = product(rows.qkv, L.wq, g.xf_cur, g.xs_cur, g.pk, H, tot))) return rc;
+        if ((rc = product(rows.qkv, L.wq, g.xf_cur, g.xs_cur, moe && il, g.pk, H, tot))) return rc;
         group_norm_rope(hd, st, g.pk, tot, g.q, L.q_norm, L.k_norm, kc, start, n, c.n_q, c.n_kv, c.eps, c.rope_theta, vtc, s->capacity);
         bool tapped = false;
         for (int t = 0; t < n_taps; t++) tapped = tapped || tap_layers[t] == il;
@@ -1452,7 +1475,7 @@ int32_t prefill_group_enqueue(dflash_ctx *ctx, const dflash_model *model, dflash
         if ((rc = dfl_attn_blocks(ctx, g.q, DFLASH_TYPE_F32, kc, vtc, start, n, c.n_q, c.n_kv, hd, s->capacity, scale, g.attn, st, g.xf_attn,
                                   rows.wo.kind)))
             return rc;
-        if ((rc = product(rows.wo, L.wo, g.xf_attn, g.xs_attn, g.mix, static_cast<int64_t>(q_dim), H))) return rc;
+        if ((rc = product(rows.wo, L.wo, g.xf_attn, g.xs_attn, true, g.mix, static_cast<int64_t>(q_dim), H))) return rc;
         if (moe) {
             const float *next_w = il + 1 < c.n_layers ? model->layers[il + 1].attn_norm : model->output_norm;
             // x += mix, the experts' norm and the shared-expert gates: the block path's norm kernel over all the rows
@@ -1461,13 +1484,13 @@ int32_t prefill_group_enqueue(dflash_ctx *ctx, const dflash_model *model, dflash
                                         st)))
                 return rc;
         } else {
-            rms_norm(n, st, g.x, g.mix, L.post_norm, g.cur, H, c.eps, nullptr, nullptr, g.xf_cur, rows.gate_up.kind, xf_h);
-            if (!rows.gate_up.twin && (rc = dfl_xf_sums(ctx, g.xf_cur, H, n_blocks, g.xs_cur, st))) return rc;
+            rms_norm(n, st, g.x, g.mix, L.post_norm, g.cur, H, c.eps, nullptr, nullptr, g.xf_cur, rows.gate_up.kind, xf_h, ConvResid(),
+                     rows.gate_up.sums ? g.xs_cur : nullptr);
             // silu(gate) * up straight into fragment order, with the sums the down product wants
-            if ((rc = dfl_gemm_rows(ctx, rows.gate_up, L.gate.type, L.gate.data, g.xf_cur, g.xs_cur, nullptr, H, 2ll * c.ffn, n, c.ffn, g.xf_g,
-                                    rows.down.twin ? nullptr : g.xs_g, rows.down.kind, st)))
+            if ((rc = dfl_gemm_rows(ctx, rows.gate_up, L.gate.type, L.gate.data, g.xf_cur, g.xs_cur, false, nullptr, H, 2ll * c.ffn, n, c.ffn, g.xf_g,
+                                    rows.down.sums ? g.xs_g : nullptr, rows.down.kind, st)))
                 return rc;
-            if ((rc = dfl_gemm_rows(ctx, rows.down, L.down.type, L.down.data, g.xf_g, g.xs_g, g.mix, c.ffn, H, n, 0, nullptr, nullptr, 0, st)))
+            if ((rc = dfl_gemm_rows(ctx, rows.down, L.down.type, L.down.data, g.xf_g, g.xs_g, false, g.mix, c.ffn, H, n, 0, nullptr, nullptr, 0, st)))
                 return rc;
             if (tapped)  // (the residual is captured below; else the next norm adds it)
                 add_kernel<<<blocks_for(static_cast<size_t>(n) * H), 256, 0, st>>>(g.x, g.mix, static_cast<size_t>(n) * H);

@@ -30,6 +30,7 @@ SHAPES["heads64x12"] = (dfl.ModelConfig(n_layers=2, hidden=1024, n_q=48, n_kv=4,
 SHAPES["heads256x5"] = (dfl.ModelConfig(n_layers=2, hidden=1280, n_q=5, n_kv=1, head_dim=256, ffn=3072, vocab=2048), dfl.synth.Q4_K)
 
 SHAPES["heads256x1"] = (dfl.ModelConfig(n_layers=2, hidden=1024, n_q=4, n_kv=4, head_dim=256, ffn=3072, vocab=2048), dfl.synth.Q4_K)
+SHAPES["held4096"] = (dfl.ModelConfig(n_layers=2, hidden=4096, n_q=16, n_kv=4, head_dim=128, ffn=3072, vocab=2048), dfl.synth.Q4_K)
 SHAPES["heads256x12"] = (dfl.ModelConfig(n_layers=2, hidden=1024, n_q=12, n_kv=1, head_dim=256, ffn=3072, vocab=2048), dfl.synth.Q4_K)
 
 
@@ -112,6 +113,30 @@ def test_prefill_equals_block_by_block_with_sums_past_f16(ctx, shape, where):
                 L[up] = (L[gate][0], L[gate][1].clone())
     model = dfl.TargetModel(ctx, cfg, w)
     rows = 97
+    one, many = dfl.Session(ctx, model, rows + 16, [0, 1]), dfl.Session(ctx, model, rows + 16, [0, 1])
+    tokens = np.random.default_rng(rows).integers(0, cfg.vocab, rows).tolist()
+    got = many.prefill_blocks(tokens, 0)
+    want = torch.cat([one.encode_packed_verify_layer_major(tokens[i:i + 16], i, want_head=False).hidden_capture for i in range(0, rows, 16)])
+    assert torch.isfinite(got).all() and torch.isfinite(want).all()
+    assert torch.equal(got, want)
+    one.close()
+    many.close()
+
+
+@pytest.mark.parametrize("gain", [1.0, 4000.0])
+@pytest.mark.parametrize("rows", [17, 64, 97, 128, 192, 200])
+@pytest.mark.parametrize("shape", ["held4096", "wide"])
+def test_projections_with_minima_by_sums_equal_block_by_block(ctx, shape, rows, gain):
+    """Q4_K projections of 16 and 20 super-blocks, whose minima go by the sub-block sums on both paths (the whole-K kernel's
+    own and the norm kernel's): blocks past held weights up to the last such count and the first of the split, with a
+    last block that is not full, and with sums past the largest f16 (gains of 4000)."""
+    cfg, attn_type = SHAPES[shape]
+    w = dfl.synth_target_weights_device(cfg, 5, "cuda", attn_type=attn_type)
+    for L in w["layers"]:
+        L["attn_norm"] = L["attn_norm"] * gain
+        for name in ("wq", "wk", "wv"):
+            _rescale(L[name], min(1.0, 10 / gain))
+    model = dfl.TargetModel(ctx, cfg, w)
     one, many = dfl.Session(ctx, model, rows + 16, [0, 1]), dfl.Session(ctx, model, rows + 16, [0, 1])
     tokens = np.random.default_rng(rows).integers(0, cfg.vocab, rows).tolist()
     got = many.prefill_blocks(tokens, 0)
