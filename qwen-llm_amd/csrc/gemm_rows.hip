@@ -745,6 +745,26 @@ int rows_pick_rb(const dflash_ctx *ctx, int n_blocks, int n_ct, int most) {
     return rb;
 }
 
+// The same where the workgroups of a tile share K: what larger tiles leave idle goes to more shares, so the cost is that
+// of the longest share, and the weights are read by fewer row tiles.  The tile by whole rounds (2 blocks) : this one.  Q4_K,
+// 100 rows, 5120 -> 6144, 4096 -> 5120 and 17408 -> 5120 on average 28.1 : 23.8 us (6 and 3 blocks); 200 rows, 4096 -> 5120 26.5 :
+// 23.2 (4).  Q6_K, 300 rows, 4096 -> 2048 27.4 : 20.2 (4).
+int rows_pick_split_rb(const dflash_ctx *ctx, int n_blocks, int n_ct, int most, int ranges) {
+    int rb = 2;
+    int64_t best = -1;
+    for (int r = most; r >= 2; r--) {
+        const int64_t tiles = static_cast<int64_t>(n_ct) * ((n_blocks + r - 1) / r);
+        const int64_t n_split = std::min<int64_t>(ranges, ctx->n_cu / tiles);
+        if (n_split < 2) continue;
+        const int64_t cost = (ranges + n_split - 1) / n_split * (4 * r + 5);
+        if (best < 0 || cost < best) {
+            best = cost;
+            rb = r;
+        }
+    }
+    return rb;
+}
+
 template <typename Tile, bool kTwin, int kEpi>
 int32_t rows_dispatch(dflash_ctx *ctx, const RowsArgs &a, int rb, int64_t tiles, hipStream_t st) {
     switch (rb) {
@@ -793,7 +813,7 @@ int32_t dfl_gemm_rows(dflash_ctx *ctx, const dfl_rows_plan &p, int32_t w_type, c
     a.n_ct = static_cast<int>(pair_ffn ? pair_ffn / 128 : (n_out + 255) / 256);
     const bool q6 = w_type == DFLASH_TYPE_Q6_K_TILED;
     const int most = p.sums ? 8 : 4;  // (a twin product's second accumulators)
-    const int rb = rows_pick_rb(ctx, a.n_blocks, a.n_ct, most);
+    int rb = rows_pick_rb(ctx, a.n_blocks, a.n_ct, most);
     a.n_rt = (a.n_blocks + rb - 1) / rb;
     int64_t tiles = static_cast<int64_t>(a.n_ct) * a.n_rt;
     auto sums = [&]() -> int32_t { return p.sums && make_sums ? dfl_xf_sums(ctx, xf, n_in, a.n_blocks, xs, st) : DFLASH_OK; };
@@ -820,10 +840,13 @@ int32_t dfl_gemm_rows(dflash_ctx *ctx, const dfl_rows_plan &p, int32_t w_type, c
         const int whole_most = a.nb * a.n_ct >= 80 ? 12 : 4;
         if (p.whole && a.n_blocks <= whole_most && dfl_whole_holds_weights(ctx, w_type, n_in, n_out))
             return dfl_gemm_whole_blocks(ctx, w_type, w, xf, y, n_in, n_out, n_rows, 0, nullptr, 0, st, true);
-        a.n_split = std::min<int>(ranges, static_cast<int>(ctx->n_cu / tiles));
         size_t off = 0;
         float *part = dfl_ws_take<float>(ctx, &off, static_cast<size_t>(most_ranges) * a.n_blocks * 16 * n_out * sizeof(float));
-        if (part && a.n_split > 1) {
+        if (part) {
+            rb = rows_pick_split_rb(ctx, a.n_blocks, a.n_ct, most, ranges);
+            a.n_rt = (a.n_blocks + rb - 1) / rb;
+            tiles = static_cast<int64_t>(a.n_ct) * a.n_rt;
+            a.n_split = std::min<int>(ranges, static_cast<int>(ctx->n_cu / tiles));
             a.y = part;
             tiles *= a.n_split;
             int32_t rc = sums();
