@@ -835,6 +835,8 @@ int32_t dfl_gemm_rows(dflash_ctx *ctx, const dfl_rows_plan &p, int32_t w_type, c
         //           1024 -> 4096  6.6 :  9.2   9.4 : 10.2  21.2 : 17.0     2048 -> 1024  6.3 :  9.5   9.2 :  9.8  20.6 : 11.6
         //   not     4096 -> 6144 22.1 : 17.9  29.6 : 22.9  (Q6_K 32.5 : 19.5  50.5 : 27.8)
         //           4096 -> 5120 20.4 : 18.9  27.8 : 20.1  (Q6_K 32.1 : 21.8  49.0 : 24.1), 5120 -> 6144 52.6 : 18.1  69.3 : 23.5
+        // (the split of that table with tiles of two blocks; with the tiles it has now, 2048 -> 5120 and 4096 -> 2048 in Q6_K on
+        // average, 7 / 9 / 12 blocks: 13.7 : 18.2, 17.2 : 19.7, 22.2 : 22.7, the same line)
         // so: twelve blocks for matrices of 80 super-blocks x column tiles or more, four for smaller ones, none where the
         // weights are not held.
         const int whole_most = a.nb * a.n_ct >= 80 ? 12 : 4;
