@@ -230,8 +230,9 @@ int dfl_whole_kind(const dflash_ctx *ctx, int32_t w_type, int64_t n_in, int64_t 
 int32_t dfl_gemm_whole(dflash_ctx *ctx, int32_t w_type, const void *w, const void *xf, float *y, int64_t n_in, int64_t n_out,
                        int32_t n_rows, int64_t pair_ffn, void *y_xf, int y_xf_kind, hipStream_t stream, bool by_sums = false);
 // by_sums: where dfl_whole_by_sums says so, minima through the activations' sub-block sums, as dfl_gemm_rows has them (a target's
-// layers); else through twin products (a drafter's, and the public operator).
-static inline bool dfl_whole_by_sums(int32_t w_type, int64_t n_in) { return w_type == DFLASH_TYPE_Q4_K_TILED && n_in >= 16 * DFL_QK_K; }
+// layers); else through twin products (a drafter's, and the public operator).  It says so for a Q4_K matrix of 16 super-blocks of K
+// or more whose tiles are one round of the chip (the looping kernel has twins alone).
+bool dfl_whole_by_sums(const dflash_ctx *ctx, int32_t w_type, int64_t n_in, int64_t n_out, int64_t pair_ffn);
 // The same for n_rows_total rows, sixteen to a block (the last one may be shorter): block i's rows are in XF order at
 // xf + i * dfl_xf_bytes(n_in), its result at y + i * 16 * n_out (pair mode: 16 * pair_ffn; y_xf + i * dfl_xf_bytes(pair_ffn)).
 // The weights are read once and stay in registers while the blocks pass; a row's bits are those of dfl_gemm_whole.

@@ -691,7 +691,7 @@ dfl_rows_plan dfl_gemm_rows_plan(const dflash_ctx *ctx, int32_t w_type, int64_t 
     if (kind != DFL_XF_NONE) {
         p.kind = kind;
         p.whole = 1;
-        p.sums = dfl_whole_by_sums(w_type, n_in);
+        p.sums = dfl_whole_by_sums(ctx, w_type, n_in, n_out, pair_ffn);
         p.total = nb;
         p.n_cut = nb < 16 ? nb : 16;  // the whole-K kernel's slices
         return p;

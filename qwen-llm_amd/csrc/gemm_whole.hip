@@ -20,7 +20,7 @@
 // Arithmetic: that of the streaming kernels (exact f16 integers from the quant bits, one packed fma with
 // s = d * scale, f32 accumulation on v_mfma_f32_16x16x32_f16; the Q4_K minima and the Q6_K offset through a twin MFMA
 // of the same activation fragment into a second accumulator that is subtracted at the end).  Where a target's Q4_K matrix
-// has 16 super-blocks of K or more (Q4S) the minima go by one MFMA over the activations' sub-block sums ahead of the
+// has 16 super-blocks of K or more and one round of tiles (Q4S; dfl_whole_by_sums) the minima go by one MFMA over the activations' sub-block sums ahead of the
 // eight: the same MFMAs are what a prompt's many-row product is made of (gemm_rows.hip, whose rows have this kernel's bits),
 // and twins are half of them there.  The sums cost a wave 90 vector instructions a stage (4096 -> 5120 and 5120 -> 6144 9.1 -> 9.4 us a
 // launch); matrices of short K, where a launch is 4 us and a prompt's product as short, keep the twins.
@@ -511,7 +511,7 @@ __global__ void __launch_bounds__(1024) gemm_whole_kernel(WholeArgs a) {
 // the same super-block in every unit, so its eight activation fragments are loaded ONCE and stay in registers; the
 // weights of the next unit travel while the current one is unpacked and multiplied; the slices' partial tiles meet
 // in one of two LDS buffers in turn (one barrier per unit: a buffer is rewritten two units later, behind the barrier
-// of the unit in between).  Same sums, in the same order, as gemm_whole_kernel.
+// of the unit in between).  Same sums, in the same order, as gemm_whole_kernel with twin products.
 template <typename W>
 __global__ void __launch_bounds__(1024) gemm_whole_loop_kernel(WholeArgs a) {
     extern __shared__ float4_t red[];  // [2][16 waves][64]; Q6_K in row order: then a staging area per wave
@@ -703,6 +703,12 @@ int dfl_whole_kind(const dflash_ctx *ctx, int32_t w_type, int64_t n_in, int64_t 
     return whole_plan(ctx, w_type, n_in, n_out, pair_ffn).kind;
 }
 
+bool dfl_whole_by_sums(const dflash_ctx *ctx, int32_t w_type, int64_t n_in, int64_t n_out, int64_t pair_ffn) {
+    if (w_type != DFLASH_TYPE_Q4_K_TILED || n_in < 16 * DFL_QK_K) return false;
+    const WholePlan p = whole_plan(ctx, w_type, n_in, n_out, pair_ffn);
+    return p.kind != DFL_XF_NONE && !p.loop;
+}
+
 bool dfl_whole_holds_weights(const dflash_ctx *ctx, int32_t w_type, int64_t n_in, int64_t n_out) {
     const WholePlan p = whole_plan(ctx, w_type, n_in, n_out, 0);
     return p.kind != DFL_XF_NONE && !p.loop && p.R == 1 && n_in / DFL_QK_K <= p.ksplit;
@@ -770,7 +776,7 @@ int32_t dfl_gemm_whole_blocks(dflash_ctx *ctx, int32_t w_type, const void *w, co
         DFL_HIP_CHECK(ctx, hipGetLastError());
         return DFLASH_OK;
     }
-    by_sums = by_sums && dfl_whole_by_sums(w_type, n_in);
+    by_sums = by_sums && dfl_whole_by_sums(ctx, w_type, n_in, n_out, pair_ffn);
     const int multi = n_blocks > 1 ? (a.nb > p.ksplit ? 2 : 1) : 0;
     if (multi && by_sums && (p.R != 1 || multi != 1))
         return dfl_fail(ctx, DFLASH_ERR_UNSUPPORTED, "gemm_whole: several blocks by sums only past weights a wave holds");

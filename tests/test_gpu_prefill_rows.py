@@ -31,6 +31,8 @@ SHAPES["heads256x5"] = (dfl.ModelConfig(n_layers=2, hidden=1280, n_q=5, n_kv=1, 
 
 SHAPES["heads256x1"] = (dfl.ModelConfig(n_layers=2, hidden=1024, n_q=4, n_kv=4, head_dim=256, ffn=3072, vocab=2048), dfl.synth.Q4_K)
 SHAPES["held4096"] = (dfl.ModelConfig(n_layers=2, hidden=4096, n_q=16, n_kv=4, head_dim=128, ffn=3072, vocab=2048), dfl.synth.Q4_K)
+# (q|k|v of 16 super-blocks and 9216 columns: more tiles than one round of 256 CUs, the looping whole-K kernel)
+SHAPES["loop4096"] = (dfl.ModelConfig(n_layers=2, hidden=4096, n_q=64, n_kv=4, head_dim=128, ffn=3072, vocab=2048), dfl.synth.Q4_K)
 SHAPES["heads256x12"] = (dfl.ModelConfig(n_layers=2, hidden=1024, n_q=12, n_kv=1, head_dim=256, ffn=3072, vocab=2048), dfl.synth.Q4_K)
 
 
@@ -125,10 +127,10 @@ def test_prefill_equals_block_by_block_with_sums_past_f16(ctx, shape, where):
 
 @pytest.mark.parametrize("gain", [1.0, 4000.0])
 @pytest.mark.parametrize("rows", [17, 64, 97, 128, 192, 200])
-@pytest.mark.parametrize("shape", ["held4096", "wide"])
+@pytest.mark.parametrize("shape", ["held4096", "wide", "loop4096"])
 def test_projections_with_minima_by_sums_equal_block_by_block(ctx, shape, rows, gain):
     """Q4_K projections of 16 and 20 super-blocks, whose minima go by the sub-block sums on both paths (the whole-K kernel's
-    own and the norm kernel's): blocks past held weights up to the last such count and the first of the split, with a
+    own and the norm kernel's) where the block's product is one round of the chip, by twin products on both where it loops: blocks past held weights up to the last such count and the first of the split, with a
     last block that is not full, and with sums past the largest f16 (gains of 4000)."""
     cfg, attn_type = SHAPES[shape]
     w = dfl.synth_target_weights_device(cfg, 5, "cuda", attn_type=attn_type)
