@@ -244,13 +244,15 @@ bool dfl_whole_holds_weights(const dflash_ctx *ctx, int32_t w_type, int64_t n_in
 // ---- many rows at once (gemm_rows.hip): the products of a prompt's prefill ----
 // Every row gets the bits the 16-row kernels give it in its own block: dfl_gemm_rows_plan says which of their
 // arithmetics the matrix takes there and where K is cut.  kind == DFL_XF_NONE: not taken (only the tiled orders are).
+// row_major: the block's rows reach this matrix in row order, so that its 16-row kernel is the streaming one whatever its
+// shape (Q4_K; a tiled Q6_K matrix has no such kernel).
 struct dfl_rows_plan {
     int kind;      // fragment order the activations must be in
     int whole;     // the 16-row kernel is the whole-K kernel (K is cut at its slices)
     int sums;      // the activations' sub-block sums are needed (else: twin products)
     int total, n_cut, by_group;
 };
-dfl_rows_plan dfl_gemm_rows_plan(const dflash_ctx *ctx, int32_t w_type, int64_t n_in, int64_t n_out, int64_t pair_ffn);
+dfl_rows_plan dfl_gemm_rows_plan(const dflash_ctx *ctx, int32_t w_type, int64_t n_in, int64_t n_out, int64_t pair_ffn, bool row_major = false);
 // Sub-block sums of n_blocks blocks of rows in fragment order (kind Q4K), for the plans with `sums`:
 // dfl_xs_bytes(n_in) bytes per block.
 static inline size_t dfl_xs_bytes(int64_t n_in) { return static_cast<size_t>(n_in / 256) * 1024; }

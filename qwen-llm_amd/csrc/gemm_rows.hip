@@ -680,14 +680,14 @@ __global__ void __launch_bounds__(64) xf_sums_kernel(const uint8_t *__restrict__
 
 }  // namespace
 
-dfl_rows_plan dfl_gemm_rows_plan(const dflash_ctx *ctx, int32_t w_type, int64_t n_in, int64_t n_out, int64_t pair_ffn) {
+dfl_rows_plan dfl_gemm_rows_plan(const dflash_ctx *ctx, int32_t w_type, int64_t n_in, int64_t n_out, int64_t pair_ffn, bool row_major) {
     dfl_rows_plan p = {};
     if (w_type != DFLASH_TYPE_Q4_K_TILED && w_type != DFLASH_TYPE_Q6_K_TILED) return p;
     if (n_in <= 0 || n_in % DFL_QK_K || n_out <= 0 || n_out >= (1 << 24) || n_in >= (1 << 24)) return p;
     if (pair_ffn && (n_out != 2 * pair_ffn || pair_ffn % DFL_QK_K || w_type != DFLASH_TYPE_Q4_K_TILED)) return p;
     if (ctx->lds_bytes < 160 * 1024) return p;
     const int nb = static_cast<int>(n_in / DFL_QK_K);
-    const int kind = dfl_whole_kind(ctx, w_type, n_in, n_out, pair_ffn);
+    const int kind = row_major && w_type == DFLASH_TYPE_Q4_K_TILED ? DFL_XF_NONE : dfl_whole_kind(ctx, w_type, n_in, n_out, pair_ffn);
     if (kind != DFL_XF_NONE) {
         p.kind = kind;
         p.whole = 1;

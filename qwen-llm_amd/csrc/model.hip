@@ -1410,7 +1410,8 @@ LayerRows layer_rows(const dflash_ctx *ctx, const dflash_model_cfg &c, const dfl
     r.wo = dfl_gemm_rows_plan(ctx, L.wo.type, q_dim, H, 0);
     if (c.n_expert == 0) {
         if (adjacent(L.gate, c.ffn, L.up, H)) r.gate_up = dfl_gemm_rows_plan(ctx, L.gate.type, H, 2ll * c.ffn, c.ffn);
-        r.down = dfl_gemm_rows_plan(ctx, L.down.type, c.ffn, H, 0);
+        // (verify_enqueue: down reads fragment order only behind a gate | up that is a whole-K product)
+        r.down = dfl_gemm_rows_plan(ctx, L.down.type, c.ffn, H, 0, !r.gate_up.whole);
     }
     return r;
 }

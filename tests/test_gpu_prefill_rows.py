@@ -31,6 +31,10 @@ SHAPES["heads256x5"] = (dfl.ModelConfig(n_layers=2, hidden=1280, n_q=5, n_kv=1, 
 
 SHAPES["heads256x1"] = (dfl.ModelConfig(n_layers=2, hidden=1024, n_q=4, n_kv=4, head_dim=256, ffn=3072, vocab=2048), dfl.synth.Q4_K)
 SHAPES["held4096"] = (dfl.ModelConfig(n_layers=2, hidden=4096, n_q=16, n_kv=4, head_dim=128, ffn=3072, vocab=2048), dfl.synth.Q4_K)
+# (gate|up of more tiles than one round, behind it a down projection that by its own shape the whole-K kernel would take: K of
+# 27 super-blocks, and of 17, the fewest, with 9 of gate|up)
+SHAPES["ffn6912"] = (dfl.ModelConfig(n_layers=2, hidden=2560, n_q=16, n_kv=4, head_dim=128, ffn=6912, vocab=2048), dfl.synth.Q4_K)
+SHAPES["ffn4352"] = (dfl.ModelConfig(n_layers=2, hidden=2304, n_q=16, n_kv=4, head_dim=128, ffn=4352, vocab=2048), dfl.synth.Q4_K)
 # (q|k|v of 16 super-blocks and 9216 columns: more tiles than one round of 256 CUs, the looping whole-K kernel)
 SHAPES["loop4096"] = (dfl.ModelConfig(n_layers=2, hidden=4096, n_q=64, n_kv=4, head_dim=128, ffn=3072, vocab=2048), dfl.synth.Q4_K)
 SHAPES["heads256x12"] = (dfl.ModelConfig(n_layers=2, hidden=1024, n_q=12, n_kv=1, head_dim=256, ffn=3072, vocab=2048), dfl.synth.Q4_K)
@@ -61,6 +65,13 @@ def test_many_row_prefill_equals_block_by_block(ctx, shape, rows):
 @pytest.mark.parametrize("shape", ["experts", "narrow", "wide", "q6k4096"])
 def test_last_row_tiles_of_every_fill_equal_block_by_block(ctx, shape, rows):
     """3 to 31 blocks: last row tiles of up to half their blocks (computed as half a tile), of more, and of a single row."""
+    test_many_row_prefill_equals_block_by_block(ctx, shape, rows)
+
+
+@pytest.mark.parametrize("rows", [17, 64, 200, 530])
+@pytest.mark.parametrize("shape", ["ffn4352", "ffn6912"])
+def test_down_behind_a_streamed_gate_up_equals_block_by_block(ctx, shape, rows):
+    """The block path's down product streams there, although the matrix alone would be a whole-K product: K is cut elsewhere."""
     test_many_row_prefill_equals_block_by_block(ctx, shape, rows)
 
 
