@@ -1,7 +1,8 @@
 // Reads from LDS with hand-counted waits, for kernels that have direct-to-LDS loads under way: the compiler cannot tell the
 // two apart and waits for every read it has issued (lgkmcnt(0)) ahead of each use.  A register is not touched between its
 // read and lds_arrived, which the compiler does not know: no such read may be under way where the code branches (it may copy
-// one there), and the build refuses these kernels if they spill (build.py).
+// one there).  The build refuses these kernels if they spill (build.py), and if their generated code touches such a register
+// ahead of its wait (inflight.py).
 #pragma once
 
 #include "common.h"
