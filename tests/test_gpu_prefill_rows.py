@@ -6,6 +6,10 @@ and the split's first count (64 | 80 rows narrow, 192 | 200 experts); tiles of e
 tile that is not full; several rounds of the chip.  K and the column counts bring each kind of cut: 5120 (whole-K slices, twenty super-blocks), 17408 (stream-K
 ranges that differ from tile group to tile group), 1024 (fewer super-blocks than slices), Q6_K projections, experts
 with one to four blocks per tile."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 import torch
@@ -37,6 +41,9 @@ SHAPES["ffn6912"] = (dfl.ModelConfig(n_layers=2, hidden=2560, n_q=16, n_kv=4, he
 SHAPES["ffn4352"] = (dfl.ModelConfig(n_layers=2, hidden=2304, n_q=16, n_kv=4, head_dim=128, ffn=4352, vocab=2048), dfl.synth.Q4_K)
 # (q|k|v of 16 super-blocks and 9216 columns: more tiles than one round of 256 CUs, the looping whole-K kernel)
 SHAPES["loop4096"] = (dfl.ModelConfig(n_layers=2, hidden=4096, n_q=64, n_kv=4, head_dim=128, ffn=3072, vocab=2048), dfl.synth.Q4_K)
+# (a mixture's projections in Q4_K: wo of 16 super-blocks, by sums that no kernel ahead of it has left)
+SHAPES["experts_q4k"] = (dfl.ModelConfig(n_layers=3, hidden=2048, n_q=16, n_kv=2, head_dim=256, ffn=0, vocab=2048, n_expert=32, n_expert_used=4,
+                                         ffn_expert=768, ffn_shared=768), dfl.synth.Q4_K)
 SHAPES["heads256x12"] = (dfl.ModelConfig(n_layers=2, hidden=1024, n_q=12, n_kv=1, head_dim=256, ffn=3072, vocab=2048), dfl.synth.Q4_K)
 
 
@@ -158,6 +165,34 @@ def test_projections_with_minima_by_sums_equal_block_by_block(ctx, shape, rows, 
     assert torch.equal(got, want)
     one.close()
     many.close()
+
+
+@pytest.mark.parametrize("rows", [17, 192, 200, 530])
+def test_a_mixture_with_q4k_projections_equals_block_by_block(ctx, rows):
+    """Its output projection's minima go by sums made ahead of the product: past held weights up to their last count, and split."""
+    test_many_row_prefill_equals_block_by_block(ctx, "experts_q4k", rows)
+
+
+_STREAMED_PROBE = r"""
+import sys
+sys.path.insert(0, "tests")
+import qwen_llm_amd as dfl
+import test_gpu_prefill_rows as t
+ctx = dfl.Context(0, workspace_bytes=256 << 20)
+for rows in (40, 530):
+    t.test_many_row_prefill_equals_block_by_block(ctx, "experts_q4k", rows)
+print("equal")
+"""
+
+
+def test_a_mixture_whose_projections_stream_equals_block_by_block():
+    """Without the whole-K kernels every Q4_K projection goes by sums: the first layer's q|k|v by the norm kernel's, the later
+    ones', which the experts' last kernel has normalised, by sums made ahead of the product.  (The switch is read once per
+    process.)"""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    env = dict(os.environ, PYTHONPATH=root + os.pathsep + os.environ.get("PYTHONPATH", ""), DFLASH_GEMM_WHOLE="0")
+    r = subprocess.run([sys.executable, "-c", _STREAMED_PROBE], env=env, cwd=root, capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0 and r.stdout.split()[-1] == "equal", r.stderr[-2000:]
 
 
 @pytest.mark.parametrize("shape", ["narrow", "experts", "heads64"])
