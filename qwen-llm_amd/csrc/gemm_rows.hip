@@ -554,6 +554,8 @@ __global__ void __launch_bounds__(64 * (kList ? kList : kRowsWaves), 2) gemm_row
         copies_done<0>();  // (the epilogue has other uses for LDS, and the next workgroup too)
     };
     // An expert's few rows are computed alone, by code of their own; a tail of no more than half the tile's blocks as half a tile.
+    // What the instances of a list earn against 1, 2, 4 and 8 alone (a layer of a mixture's prompt, 128 experts top-8, rows,
+    // that : this): 2048 697 : 673 us, 1500 550 : 536, 600 300 : 295; 32 top-4, 1000 rows 320 : 314.
     if constexpr (kList) {
         switch (live) {
             case 1: walk_k(std::integral_constant<int, 1>()); break;

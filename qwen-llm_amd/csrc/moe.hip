@@ -780,9 +780,17 @@ int32_t dfl_moe_ffn_group(dflash_ctx *ctx, const dflash_model_cfg &c, const dfla
     if ((rc = dfl_router_rows(ctx, L.router.data, cur, s.logits, H, E, n_rows, st))) return rc;
     moe_group_route_kernel<<<(n_rows + 15) / 16, 1024, 0, st>>>(s.logits, n_rows, E, used, s.sel_e, s.sel_w);
     // Row tiles of eight blocks (a workgroup of eight waves fills a CU) take in half the weights and fewer activations for a
-    // product, those of four (two workgroups on a CU) hide each other's waits and leave less of a tile empty.  128 experts top-8, gate
-    // and up + down in us, 4 : 8: 98 rows an expert (1500 tokens) 220 : 208, 128 rows 281 : 256; 62 rows 164 : 180, 25 rows 116 : 139.
-    const int tile_slots = n_rows * used >= 80 * E ? 8 : 4;
+    // product, those of four (two workgroups on a CU) hide each other's waits, leave less of a tile empty and make more
+    // workgroups.  Eight where an expert has 85 rows on average and the experts alone are two rounds of the chip in the
+    // narrower product.  A layer in us, 4 : 8 (hidden 2048; 94 pairs over 14 mixtures of 8 to 256 experts; the better side, or
+    // within 7 us of it, in all but two, 9 and 11 us):
+    //   two rounds, 80 / 90 / 100 / 128 rows an expert: 128 experts top-8 FFN 768 482 : 481, 519 : 514, 563 : 550, 693 : 677;
+    //               64 top-6 of 1536 388 : 390, 410 : 402, 467 : 454, 552 : 543 (50 rows 287 : 308)
+    //   fewer, 80 / 100 / 130 / 200 rows: 8 top-2 of 3584 183 : 197, 209 : 216, 254 : 256, 332 : 325; 32 top-4 of 2048 296 : 307,
+    //               340 : 338, 422 : 419, 565 : 554; 64 top-8 of 512 249 : 262, 293 : 300, 367 : 370, 482 : 485; 48 top-4 of 1024 323 : 320,
+    //               385 : 385, 468 : 468, 575 : 590
+    const int narrow_ct = std::min(fe / 128, H / 256);  // column tiles of the narrower product, gate and up or down
+    const int tile_slots = n_rows * used >= 85 * E && E * narrow_ct >= 2 * ctx->n_cu ? 8 : 4;
     moe_group_slots_kernel<<<1, 1024, 0, st>>>(s.sel_e, n_rows, used, E, s.n_slots, s.slot_rows, s.pick_pos, reinterpret_cast<int4 *>(s.tiles),
                                              s.n_tiles, max_slots, tile_slots);
     moe_group_gather_kernel<<<dim3(H / DFL_QK_K, max_slots), 64, 0, st>>>(cur, s.slot_rows, s.n_slots, H, s.xg, s.xg_sums);

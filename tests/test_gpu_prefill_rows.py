@@ -167,6 +167,12 @@ def test_projections_with_minima_by_sums_equal_block_by_block(ctx, shape, rows, 
     many.close()
 
 
+@pytest.mark.parametrize("rows", [1344, 1361, 1777, 2033])
+def test_expert_tiles_of_eight_blocks_equal_block_by_block(ctx, rows):
+    """128 experts of 84 rows on average (the last count with tiles of four blocks), 85, 111 and 127 (tiles of five to eight)."""
+    test_many_row_prefill_equals_block_by_block(ctx, "experts128", rows)
+
+
 @pytest.mark.parametrize("rows", [17, 192, 200, 530])
 def test_a_mixture_with_q4k_projections_equals_block_by_block(ctx, rows):
     """Its output projection's minima go by sums made ahead of the product: past held weights up to their last count, and split."""
