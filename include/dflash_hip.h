@@ -207,10 +207,12 @@ const char *dflash_gemm_fewrow_noalloc_error(void);
  *   dflash_gemm_fewrow_xf_kind: the XF kind (DFLASH_XF_Q4K / DFLASH_XF_Q6K) this (type, shape) reads, or
  *     DFLASH_XF_NONE where it is not taken: w_type must be DFLASH_TYPE_Q4_K_TILED, DFLASH_TYPE_Q6_K_TILED or
  *     DFLASH_TYPE_Q6_K | DFLASH_TYPE_RANGE_CHECKED (these kernels scale in f16: a range-checked tensor only), n_in at most 8192, and
- *     the matrix at most one round of the chip (about 320 workgroups of 16 or 32 rows).
+ *     the matrix at most one round of the chip (a workgroup of 16 or 32 rows on every CU) or, with n_in at most 4096, any number.
  *   dflash_pack_xf: row-major x[n_rows][n_in] (f32 or f16) -> xf, rounding to f16 as every few-row kernel does.
  *   dflash_gemm_fewrow_xf: Y[n_rows][n_out] = X . W^T; same guards as dflash_gemm_fewrow; DFLASH_ERR_UNSUPPORTED
  *     where the kind is DFLASH_XF_NONE.  A (row, column) result depends on that activation row and weight row only.
+ *     More than sixteen rows (a matrix of one round of the chip only): blocks of sixteen, the last one may be shorter,
+ *     block i in fragment order at xf + i * dflash_xf_bytes(n_in).
  * All enqueue-only. */
 enum { DFLASH_XF_NONE = 0, DFLASH_XF_Q4K = 1, DFLASH_XF_Q6K = 2 };
 size_t dflash_xf_bytes(int64_t n_in);

@@ -235,7 +235,8 @@ int32_t dfl_gemm_whole(dflash_ctx *ctx, int32_t w_type, const void *w, const voi
 bool dfl_whole_by_sums(const dflash_ctx *ctx, int32_t w_type, int64_t n_in, int64_t n_out, int64_t pair_ffn);
 // The same for n_rows_total rows, sixteen to a block (the last one may be shorter): block i's rows are in XF order at
 // xf + i * dfl_xf_bytes(n_in), its result at y + i * 16 * n_out (pair mode: 16 * pair_ffn; y_xf + i * dfl_xf_bytes(pair_ffn)).
-// The weights are read once and stay in registers while the blocks pass; a row's bits are those of dfl_gemm_whole.
+// The weights are read once and stay in registers while the blocks pass; a row's bits are those of dfl_gemm_whole.  A looping
+// plan takes one block; by sums, several only where dfl_whole_holds_weights says so (else DFLASH_ERR_UNSUPPORTED).
 int32_t dfl_gemm_whole_blocks(dflash_ctx *ctx, int32_t w_type, const void *w, const void *xf, float *y, int64_t n_in, int64_t n_out,
                               int32_t n_rows_total, int64_t pair_ffn, void *y_xf, int y_xf_kind, hipStream_t stream, bool by_sums = false);
 // Whether a wave has one super-block of one tile, whose unpacked weights it then keeps from block to block.

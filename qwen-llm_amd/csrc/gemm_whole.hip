@@ -372,7 +372,8 @@ __device__ __forceinline__ void load_xf(half8_t (&af)[8], const uint8_t *xf, int
 
 // W: Q4W or Q6W.  R: tiles per wave and stage (they share the stage's activation fragments).
 // kMulti: several 16-row blocks per launch (a.n_blocks): 1 = every wave has one stage (K of at most 16 super-blocks), 2 = one or
-// two; the single-block instances (0) keep the registers of a kernel without the loop.
+// two; the single-block instances (0) keep the registers of a kernel without the loop.  (A prefill takes 1 with R = 1 in the tiled
+// orders, whose weights a wave holds; the others serve dflash_gemm_fewrow_xf.)
 template <typename W, int R, int kMulti>
 __global__ void __launch_bounds__(1024) gemm_whole_kernel(WholeArgs a) {
     // [16 waves][R] partial tiles; Q6_K: then a staging area per wave
@@ -906,7 +907,8 @@ extern "C" int32_t dflash_gemm_fewrow_xf(dflash_ctx *ctx, int32_t w_type, const 
                           : w_type == DFLASH_TYPE_Q6_K_TILED ? dflash_q6k_tiled_bytes(n_in, n_out)
                                                              : dflash_row_bytes(w_type, n_in) * n_out;
         const size_t yb = static_cast<size_t>(n_rows > 0 ? n_rows : 1) * n_out * sizeof(float);
-        if (dfl_ranges_overlap(y, yb, xf, dfl_xf_bytes(n_in)) || dfl_ranges_overlap(y, yb, w, wb))
+        const size_t xb = static_cast<size_t>(n_rows > 16 ? (n_rows + 15) / 16 : 1) * dfl_xf_bytes(n_in);
+        if (dfl_ranges_overlap(y, yb, xf, xb) || dfl_ranges_overlap(y, yb, w, wb))
             return dfl_fail(ctx, DFLASH_ERR_ALIAS, "gemm_fewrow_xf: y aliases an input");
     }
     return dfl_gemm_whole(ctx, w_type, w, xf, y, n_in, n_out, n_rows, 0, nullptr, DFL_XF_NONE, static_cast<hipStream_t>(stream));

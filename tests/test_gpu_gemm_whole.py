@@ -163,6 +163,29 @@ def test_rows_are_independent(ctx):
             assert np.array_equal(y1[0].view(np.uint32), y[r].view(np.uint32))
 
 
+@pytest.mark.parametrize("qtype,tiled", [(dfl.synth.Q4_K, True), (dfl.synth.Q6_K, True), (dfl.synth.Q6_K, False)])
+@pytest.mark.parametrize("n_in,n_out", [(2048, 1000), (4096, 5120), (6144, 2048), (5120, 6144)])
+def test_several_blocks_in_a_call_equal_block_by_block(ctx, canaries, qtype, tiled, n_in, n_out):
+    """More than sixteen rows, their blocks' fragment orders one behind the other: one and two stages per wave, one and two
+    tiles, a last block that is not full."""
+    import torch
+
+    w, w_type, _, _ = upload(ctx, qtype, n_in, n_out, seed=n_in + 7)
+    if qtype == dfl.synth.Q6_K and tiled:
+        w, w_type = ctx.repack_q6k_tiled(w, n_in, n_out), dfl.TYPE_Q6_K_TILED
+    kind = ctx.xf_kind(w_type, n_in, n_out)
+    x = dev(np.random.default_rng(37).standard_normal((37, n_in)).astype(np.float32))
+    blocks = [ctx.pack_xf(x[i:i + 16].contiguous(), kind) for i in (0, 16, 32)]
+    got = ctx.gemm_fewrow_xf(w, w_type, torch.cat(blocks), 37, n_in, n_out)
+    want = torch.cat([ctx.gemm_fewrow_xf(w, w_type, b, n, n_in, n_out) for b, n in zip(blocks, (16, 16, 5))])
+    canaries.check()
+    assert torch.equal(got, want)
+    xf = torch.zeros(3 * blocks[0].numel() + 37 * n_out * 4, dtype=torch.uint8, device="cuda")
+    with pytest.raises(dfl.DFlashError) as e:  # the result over the third block of rows
+        ctx.gemm_fewrow_xf(w, w_type, xf, 37, n_in, n_out, y=xf[2 * blocks[0].numel():])
+    assert e.value.kind == "Alias"
+
+
 def test_shapes_outside_the_path_are_declined(ctx):
     import torch
 
