@@ -72,7 +72,7 @@ __host__ __device__ __forceinline__ int64_t attn_chunk(int64_t n_pos, int64_t wa
     chunk = (chunk + 31) / 32 * 32;
     return chunk < min_chunk ? min_chunk : chunk;
 }
-__device__ __forceinline__ int attn_splits(int64_t n_pos, int64_t want, int64_t min_chunk) {
+__host__ __device__ __forceinline__ int attn_splits(int64_t n_pos, int64_t want, int64_t min_chunk) {
     const int64_t chunk = attn_chunk(n_pos, want, min_chunk);
     return static_cast<int>(n_pos <= 0x7fffffff ? (static_cast<uint32_t>(n_pos) + static_cast<uint32_t>(chunk) - 1) / static_cast<uint32_t>(chunk)
                                                 : (n_pos + chunk - 1) / chunk);
@@ -1318,7 +1318,6 @@ static int32_t attn_rows(dflash_ctx *ctx, const void *q, int32_t q_type, const v
     // with ctx_len_dev the context length is read on the device: everything sized here is then sized for the
     // largest context of the bucket
     const int64_t bucket = dfl_attn_bucket(ctx_len + n_rows);
-    // (several blocks: sized for the last one, which sees the most keys)
     int64_t n_pos = ctx_len_dev ? std::min<int64_t>(kv_capacity, 2 * bucket - 1) : ctx_len + n_rows_total;
 
     const AttnPolicy policy = attn_policy(ctx, bucket, n_kv, group, head_dim);
@@ -1340,12 +1339,16 @@ static int32_t attn_rows(dflash_ctx *ctx, const void *q, int32_t q_type, const v
         hw = d;
         n_parts = group / hw;
     }
-    // most splits any context up to n_pos can have
-    auto splits_for = [&](int64_t np) {
-        return ctx_len_dev ? static_cast<int>(std::min<int64_t>(want, (np + min_chunk - 1) / min_chunk))
-                           : static_cast<int>((np + attn_chunk(np, want, min_chunk) - 1) / attn_chunk(np, want, min_chunk));
+    // The most splits that any of the blocks has, or, with ctx_len_dev, that any context up to n_pos can have.  Not always the
+    // last block's: where a split's share of the keys passes a whole stage, all splits grow by one and there are fewer of them
+    // (6 splits asked for: 384 keys are 6 of 64, 385 are 5 of 96).
+    auto splits_for = [&](int32_t blocks) {
+        if (ctx_len_dev) return static_cast<int>(std::min<int64_t>(want, (n_pos + min_chunk - 1) / min_chunk));
+        int most = 1;
+        for (int32_t b = 0; b < blocks; b++) most = std::max(most, attn_splits(ctx_len + std::min(16 * (b + 1), n_rows_total), want, min_chunk));
+        return most;
     };
-    int n_splits = splits_for(n_pos);
+    int n_splits = splits_for(n_blocks);
     // several blocks: as many as the workspace has room for partial tiles of (the caller comes back for the rest)
     const size_t slot_bytes = static_cast<size_t>(n_q) * 16 * (head_dim + 2) * sizeof(float);
     if (n_blocks > 1) {
@@ -1354,7 +1357,7 @@ static int32_t attn_rows(dflash_ctx *ctx, const void *q, int32_t q_type, const v
             n_blocks--;
             n_rows_total = 16 * n_blocks;
             n_pos = ctx_len + n_rows_total;
-            n_splits = splits_for(n_pos);
+            n_splits = splits_for(n_blocks);
         }
     }
     if (blocks_done) *blocks_done = n_blocks;

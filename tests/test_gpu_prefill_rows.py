@@ -110,6 +110,13 @@ def test_heads_of_256_equal_block_by_block(ctx, shape, head, rows):
     test_continued_prefill_equals_block_by_block(ctx, shape, head, rows)
 
 
+@pytest.mark.parametrize("shape,head,rows", [("heads64x12", 249, 165), ("narrow", 2980, 150), ("heads256x12", 1350, 100)])
+def test_prefill_over_a_change_of_the_splits_length_equals_block_by_block(ctx, shape, head, rows):
+    """Blocks of one split launch whose last has fewer splits than the ones ahead of it: the keys of a split pass a whole stage at
+    384 (6 splits asked for), 3072 (32) and 1408 (22) positions, and from there on splits are longer and fewer."""
+    test_continued_prefill_equals_block_by_block(ctx, shape, head, rows)
+
+
 def _rescale(mat, factor):
     blocks = mat[1].view(-1, dfl.synth.BLOCK_BYTES[dfl.synth.Q4_K])
     blocks[:, :4] = (blocks[:, :4].contiguous().view(torch.float16) * factor).view(torch.uint8)
