@@ -242,6 +242,12 @@ int32_t dfl_gemm_whole_blocks(dflash_ctx *ctx, int32_t w_type, const void *w, co
 // Whether a wave has one super-block of one tile, whose unpacked weights it then keeps from block to block.
 bool dfl_whole_holds_weights(const dflash_ctx *ctx, int32_t w_type, int64_t n_in, int64_t n_out);
 
+// The whole-K kernel on rows in row order (f32 or f16), for the public operator: y[n_rows][n_out] = x . w^T in one launch, for Q4_K in either
+// order and Q6_K in row order; the same bits for both orders.
+bool dfl_gemm_direct_takes(const dflash_ctx *ctx, int32_t w_type, int64_t n_in, int64_t n_out);
+int32_t dfl_gemm_direct(dflash_ctx *ctx, int32_t w_type, const void *w, const void *x, int32_t x_type, float *y, int64_t n_in, int64_t n_out,
+                        int32_t n_rows, hipStream_t stream);
+
 // ---- many rows at once (gemm_rows.hip): the products of a prompt's prefill ----
 // Every row gets the bits the 16-row kernels give it in its own block: dfl_gemm_rows_plan says which of their
 // arithmetics the matrix takes there and where K is cut.  kind == DFL_XF_NONE: not taken (only the tiled orders are).

@@ -2998,7 +2998,7 @@ int32_t dfl_gemm_q4k_batched(dflash_ctx *ctx, const void *w_stack, size_t w_stri
 
 namespace {
 int32_t gemm_fewrow_impl(dflash_ctx *ctx, int32_t w_type, const void *w, const void *x, int32_t x_type, float *y, int64_t n_in,
-                         int64_t n_out, int32_t n_rows, dflash_stream_t stream);
+                         int64_t n_out, int32_t n_rows, dflash_stream_t stream, bool direct);
 }
 
 extern "C" size_t dflash_q4k_tiled_bytes(int64_t n_in, int64_t n_out) {
@@ -3033,18 +3033,18 @@ extern "C" int32_t dflash_repack_q4k_tiled(dflash_ctx *ctx, const void *w, void 
 extern "C" int32_t dflash_gemm_fewrow(dflash_ctx *ctx, int32_t w_type, const void *w, const void *x, int32_t x_type,
                                       float *y, int64_t n_in, int64_t n_out, int32_t n_rows, dflash_stream_t stream) {
     if (!ctx) return DFLASH_ERR_INVALID_INPUT;
-    return gemm_fewrow_impl(ctx, w_type, w, x, x_type, y, n_in, n_out, n_rows, stream);
+    return gemm_fewrow_impl(ctx, w_type, w, x, x_type, y, n_in, n_out, n_rows, stream, true);
 }
 
 int32_t dfl_gemm_fewrow_checked(dflash_ctx *ctx, int32_t w_type, const void *w, const void *x, int32_t x_type, float *y,
                                 int64_t n_in, int64_t n_out, int32_t n_rows, dflash_stream_t stream) {
-    return gemm_fewrow_impl(ctx, w_type | DFLASH_TYPE_RANGE_CHECKED, w, x, x_type, y, n_in, n_out, n_rows, stream);
+    return gemm_fewrow_impl(ctx, w_type | DFLASH_TYPE_RANGE_CHECKED, w, x, x_type, y, n_in, n_out, n_rows, stream, false);
 }
 
 namespace {
 
 int32_t gemm_fewrow_impl(dflash_ctx *ctx, int32_t w_type, const void *w, const void *x, int32_t x_type, float *y, int64_t n_in,
-                         int64_t n_out, int32_t n_rows, dflash_stream_t stream) {
+                         int64_t n_out, int32_t n_rows, dflash_stream_t stream, bool direct) {
     if (!w || !x || !y) return dfl_fail(ctx, DFLASH_ERR_INVALID_INPUT, "gemm_fewrow: null pointer");
     if (n_rows < 1 || n_rows > 16)
         return dfl_fail(ctx, DFLASH_ERR_BAD_SHAPE, "gemm_fewrow: n_rows %d outside 1..16", n_rows);
@@ -3097,7 +3097,11 @@ int32_t gemm_fewrow_impl(dflash_ctx *ctx, int32_t w_type, const void *w, const v
     } else if (w_type == DFLASH_TYPE_Q4_K) {
         if (tiled && reinterpret_cast<uintptr_t>(w) % 128)
             return dfl_fail(ctx, DFLASH_ERR_ALIGNMENT, "gemm_fewrow: tiled Q4_K weights must be 128-byte aligned");
+        if (direct && dfl_gemm_direct_takes(ctx, w_type, n_in, n_out))
+            return dfl_gemm_direct(ctx, tiled ? DFLASH_TYPE_Q4_K_TILED : DFLASH_TYPE_Q4_K, w, x, x_type, y, n_in, n_out, n_rows, st);
         return launch_q4k(ctx, w, x, x_type, y, n_in, n_out, n_rows, st, nullptr, 1, tiled);
+    } else if (w_type == DFLASH_TYPE_Q6_K && direct && env_int("DFLASH_Q6K_STREAM", 1) && dfl_gemm_direct_takes(ctx, w_type, n_in, n_out)) {
+        return dfl_gemm_direct(ctx, w_type, w, x, x_type, y, n_in, n_out, n_rows, st);
     } else if (w_type == DFLASH_TYPE_Q6_K && env_int("DFLASH_Q6K_STREAM", 1)) {
         const int32_t rc = launch_q6k_stream(ctx, w, x, x_type, y, n_in, n_out, n_rows, st);
         if (rc) return rc;
@@ -3241,7 +3245,7 @@ extern "C" int32_t dflash_gemm_fewrow_noalloc(int32_t w_type, const void *w, con
     if (!w || !x || !y)
         rc = dfl_fail(&local, DFLASH_ERR_INVALID_INPUT, "gemm_fewrow_noalloc: null pointer");
     else
-        rc = gemm_fewrow_impl(&local, w_type, w, x, x_type, y, n_in, n_out, n_rows, stream);
+        rc = gemm_fewrow_impl(&local, w_type, w, x, x_type, y, n_in, n_out, n_rows, stream, true);
     memcpy(dev.lds_attr_fn, local.lds_attr_fn, sizeof(dev.lds_attr_fn));
     memcpy(dev.lds_attr_bytes, local.lds_attr_bytes, sizeof(dev.lds_attr_bytes));
     dev.n_lds_attr = local.n_lds_attr;

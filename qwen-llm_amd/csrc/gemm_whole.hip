@@ -29,6 +29,7 @@
 
 #include <algorithm>
 #include <cstdlib>
+#include <type_traits>
 
 namespace {
 
@@ -61,6 +62,15 @@ __device__ __forceinline__ void load_w(Q4W &r, const WholeArgs &a, int tile, int
     const int n = lane & 15, g = lane >> 4;
     const uint8_t *p = a.w + ((static_cast<size_t>(tile >> 4) * a.nb + b) * 16 + (tile & 15)) * (16 * DFL_Q4_K_BYTES) +
                        n * DFL_Q4_K_BYTES;
+    r.hdr = *reinterpret_cast<const u32x4_t *>(p);
+    r.q0 = *reinterpret_cast<const u32x4_t *>(p + 16 + 32 * g);
+    r.q1 = *reinterpret_cast<const u32x4_t *>(p + 32 + 32 * g);
+}
+// The same blocks in GGUF row order (the rows of a tile a row stride apart): the same operands, so the same products.
+struct Q4R : Q4W {};
+__device__ __forceinline__ void load_w(Q4R &r, const WholeArgs &a, int tile, int b, int lane) {
+    const int row = min(tile * 16 + (lane & 15), a.n_out - 1), g = lane >> 4;  // rows past the matrix re-read its last row; never stored
+    const uint8_t *p = a.w + static_cast<size_t>(row) * a.row_bytes + static_cast<size_t>(b) * DFL_Q4_K_BYTES;
     r.hdr = *reinterpret_cast<const u32x4_t *>(p);
     r.q0 = *reinterpret_cast<const u32x4_t *>(p + 16 + 32 * g);
     r.q1 = *reinterpret_cast<const u32x4_t *>(p + 32 + 32 * g);
@@ -352,6 +362,10 @@ struct FragsOf<Q4W> {
     typedef Q4F type;
 };
 template <>
+struct FragsOf<Q4R> {
+    typedef Q4F type;
+};
+template <>
 struct FragsOf<Q4S> {
     typedef Q4SF type;
 };
@@ -370,11 +384,78 @@ __device__ __forceinline__ void load_xf(half8_t (&af)[8], const uint8_t *xf, int
     for (int t = 0; t < 8; t++) af[t] = p[t * 64];
 }
 
+// Where a wave's activation fragments come from: a buffer in fragment order (XfSrc), or the caller's rows, f32 or f16 in row order
+// (RowSrc).  Rows come in row-contiguous loads and go through a wave-private LDS area to the fragments' places, rounded as
+// pack_xf_kernel rounds them, so the products have the bits of a pack followed by the fragment-order launch.  (Each lane
+// loading its own octets instead touches 64 cache lines a load: 16 f32 rows, 2048 -> 5120, 9.8 us against 5.9.)  Rows the call does
+// not have stay what the area held: a row of the product depends on its own activation row only, and they are not stored.
+struct XfSrc {};
+template <typename XT>
+struct RowSrc {};
+constexpr int kRowAreaBytes = 16 * DFL_QK_K * 2;  // sixteen rows of a super-block in f16; row m's 16-byte slot o sits at o ^ m
+typedef u32x4_t u32x4_row_t __attribute__((aligned(8)));
+template <typename W>
+__device__ __forceinline__ void load_act(XfSrc, half8_t (&af)[8], const WholeArgs &, const uint8_t *xf, int b, int lane, uint8_t *) {
+    load_xf(af, xf, b, lane);
+}
+template <typename W, typename XT>
+__device__ __forceinline__ void load_act(RowSrc<XT>, half8_t (&af)[8], const WholeArgs &a, const uint8_t *x, int b, int lane, uint8_t *area) {
+    const XT *xb = reinterpret_cast<const XT *>(x) + b * DFL_QK_K;
+    const size_t stride = static_cast<size_t>(a.nb) * DFL_QK_K;
+    if constexpr (sizeof(XT) == 4) {
+        float4_t raw[16];
+#pragma unroll
+        for (int m = 0; m < 16; m++)
+            if (m < a.n_rows) raw[m] = *reinterpret_cast<const float4_t *>(xb + m * stride + 4 * lane);
+#pragma unroll
+        for (int m = 0; m < 16; m++)
+            if (m < a.n_rows) {
+                const half4_t h = {static_cast<_Float16>(raw[m][0]), static_cast<_Float16>(raw[m][2]), static_cast<_Float16>(raw[m][1]),
+                                   static_cast<_Float16>(raw[m][3])};
+                *reinterpret_cast<half4_t *>(area + m * 512 + (((lane >> 1) ^ m) * 16 + (lane & 1) * 8)) = h;
+            }
+    } else {
+        u32x4_t raw[8];
+        const int odd = lane >> 5, o = lane & 31;
+#pragma unroll
+        for (int p = 0; p < 8; p++)
+            if (2 * p < a.n_rows) raw[p] = *reinterpret_cast<const u32x4_row_t *>(xb + min(2 * p + odd, a.n_rows - 1) * stride + 8 * o);
+#pragma unroll
+        for (int p = 0; p < 8; p++)
+            if (2 * p < a.n_rows) {
+                const int m = 2 * p + odd;
+                const u32x4_t r = raw[p];  // element order 0 2 1 3 4 6 5 7
+                *reinterpret_cast<u32x4_t *>(area + m * 512 + (o ^ m) * 16) =
+                    u32x4_t{__builtin_amdgcn_perm(r.y, r.x, 0x05040100u), __builtin_amdgcn_perm(r.y, r.x, 0x07060302u),
+                            __builtin_amdgcn_perm(r.w, r.z, 0x05040100u), __builtin_amdgcn_perm(r.w, r.z, 0x07060302u)};
+            }
+    }
+    __builtin_amdgcn_wave_barrier();
+    constexpr bool q6 = std::is_same<typename FragsOf<W>::type, Q6F>::value;
+    const int m = lane & 15, g = lane >> 4;
+    // (octets of a lane: common.h, "XF")
+#pragma unroll
+    for (int t = 0; t < 8; t++) {
+        const int o = q6 ? 16 * (g >> 1) + 8 * (t >> 2) + 4 * (g & 1) + (t & 3) : 8 * g + t;
+        af[t] = *reinterpret_cast<const half8_t *>(area + m * 512 + (o ^ m) * 16);
+    }
+    __builtin_amdgcn_wave_barrier();  // (a wave's LDS accesses run in order: what comes next may overwrite the area)
+}
+template <typename X>
+struct AreaBytes {
+    static constexpr int value = kQ6AreaBytes;
+};
+template <typename XT>
+struct AreaBytes<RowSrc<XT>> {
+    static constexpr int value = kRowAreaBytes;  // (a Q6_K tile's stage passes through it behind the activations)
+};
+static_assert(kRowAreaBytes >= kQ6AreaBytes, "one area for both");
+
 // W: Q4W or Q6W.  R: tiles per wave and stage (they share the stage's activation fragments).
 // kMulti: several 16-row blocks per launch (a.n_blocks): 1 = every wave has one stage (K of at most 16 super-blocks), 2 = one or
 // two; the single-block instances (0) keep the registers of a kernel without the loop.  (A prefill takes 1 with R = 1 in the tiled
 // orders, whose weights a wave holds; the others serve dflash_gemm_fewrow_xf.)
-template <typename W, int R, int kMulti>
+template <typename W, int R, int kMulti, typename X = XfSrc>
 __global__ void __launch_bounds__(1024) gemm_whole_kernel(WholeArgs a) {
     // [16 waves][R] partial tiles; Q6_K: then a staging area per wave
     extern __shared__ float4_t red[];
@@ -393,7 +474,7 @@ __global__ void __launch_bounds__(1024) gemm_whole_kernel(WholeArgs a) {
     float4_t acc[R], acc_sub[R];
     const uint32_t sc_sel = (lane & 16) ? 0x04030402u : 0x04010400u;
     const Q4KMagic magic = q4k_magic();
-    uint8_t *area = reinterpret_cast<uint8_t *>(red + 16 * R * 64) + wave * kQ6AreaBytes;
+    uint8_t *area = reinterpret_cast<uint8_t *>(red + 16 * R * 64) + wave * AreaBytes<X>::value;
     // (every load in flight together where the registers hold them; else one tile at a time)
     constexpr bool kEarly = sizeof(W) * R <= 96;
     W w0[kEarly ? R : 1], w1[kEarly ? R : 1];
@@ -408,7 +489,7 @@ __global__ void __launch_bounds__(1024) gemm_whole_kernel(WholeArgs a) {
     }
     const int n_blocks = kMulti ? a.n_blocks : 1;
     half8_t af[8];
-    if (kEarly && active) load_xf(af, a.xf, b0, lane);
+    if (kEarly && active) load_act<W>(X(), af, a, a.xf, b0, lane, area);
     // many row blocks, one tile per wave: the B operands are unpacked once and stay in registers in place of the raw weights
     constexpr bool kFrags = kMulti != 0 && kEarly && R == 1;
     typename FragsOf<W>::type f0, f1;
@@ -425,24 +506,24 @@ __global__ void __launch_bounds__(1024) gemm_whole_kernel(WholeArgs a) {
             if constexpr (kFrags) {
                 mma(f0, af, acc[0], acc_sub[0]);
                 if (two) {
-                    load_xf(af, xf, b0 + 1, lane);
+                    load_act<W>(X(), af, a, xf, b0 + 1, lane, area);
                     mma(f1, af, acc[0], acc_sub[0]);
                 }
-                if (blk + 1 < n_blocks) load_xf(af, xf + a.xf_stride, b0, lane);
+                if (blk + 1 < n_blocks) load_act<W>(X(), af, a, xf + a.xf_stride, b0, lane, area);
             } else if constexpr (kEarly) {
                 // (af holds this block's first stage: loaded above, or behind the previous block's products)
 #pragma unroll
                 for (int r = 0; r < R; r++) compute(w0[r], af, lane, area, sc_sel, magic, acc[r], acc_sub[r]);
                 if (two) {
-                    load_xf(af, xf, b0 + 1, lane);
+                    load_act<W>(X(), af, a, xf, b0 + 1, lane, area);
 #pragma unroll
                     for (int r = 0; r < R; r++) compute(w1[r], af, lane, area, sc_sel, magic, acc[r], acc_sub[r]);
                 }
                 // the next block's fragments travel while this block's partial tiles are summed and written
-                if (kMulti != 0 && blk + 1 < n_blocks) load_xf(af, xf + a.xf_stride, b0, lane);
+                if (kMulti != 0 && blk + 1 < n_blocks) load_act<W>(X(), af, a, xf + a.xf_stride, b0, lane, area);
             } else {
                 for (int b = b0; b < b1; b++) {
-                    load_xf(af, xf, b, lane);
+                    load_act<W>(X(), af, a, xf, b, lane, area);
 #pragma unroll
                     for (int r = 0; r < R; r++) {
                         W w;
@@ -793,6 +874,79 @@ int32_t dfl_gemm_whole_blocks(dflash_ctx *ctx, int32_t w_type, const void *w, co
     dfl_timed timer(ctx, st, DFL_T_GEMM);
     fn<<<p.n_wg, threads, lds, st>>>(a);
     DFL_HIP_CHECK(ctx, hipGetLastError());
+    return DFLASH_OK;
+}
+
+// ---- the public operator on rows in row order ----
+namespace {
+// One launch in place of the streaming kernel and its reduction, where the tiles are one round of the chip, in the smallest
+// workgroups that hold them so.  The line depends on the matrix alone, not on its order, the rows or their type, so neither do the
+// bits.  us of the GPU per call, streaming : direct, 1 row f32 / 16 rows f16 / 16 rows f32:
+//   one tile per wave   Q6_K 2048 -> 512   7.3 : 4.2   7.9 : 4.9   7.9 : 5.4    tiled Q4_K 4096 -> 4096  8.4 : 4.4   9.7 : 5.5   9.7 : 6.1
+//                       Q6_K 6144 -> 2048 10.0 : 8.1  11.1 :10.3  11.1 :11.1    Q4_K in row order 6144 -> 2048  8.9 : 6.5  10.0 : 8.2   9.9 : 9.2
+//     beyond 24 super-blocks  Q6_K 8192 -> 1024   9.9 : 8.8  10.7 :11.0  10.8 :12.4 (two stages a wave, each with its rows to bring in)
+//   two tiles per wave  tiled Q4_K 4096 -> 5120  8.9 : 5.8  10.1 : 7.1  10.2 : 7.7    in row order  9.1 : 6.6  10.8 : 8.0  10.8 : 8.9
+//     beyond 16 super-blocks  5120 -> 5120  8.7 : 8.3  10.1 :10.2  10.2 :10.7    Q6_K, 4096 -> 5120  11.5 :13.4 (its registers spill)
+WholePlan rows_direct_plan(const dflash_ctx *ctx, int32_t w_type, int64_t n_in, int64_t n_out) {
+    WholePlan p = {DFL_XF_NONE, 0, 0, 0, 0, 0, false};
+    const int kind = w_type == DFLASH_TYPE_Q6_K ? DFL_XF_Q6K : (w_type == DFLASH_TYPE_Q4_K || w_type == DFLASH_TYPE_Q4_K_TILED) ? DFL_XF_Q4K : DFL_XF_NONE;
+    const int nb = static_cast<int>(n_in / DFL_QK_K);
+    if (kind == DFL_XF_NONE || n_in % DFL_QK_K || nb < 1 || nb > 24 || n_out < 1 || n_out >= (1 << 24)) return p;
+    const int ksplit = nb < 16 ? nb : 16, tiles = static_cast<int>((n_out + 15) / 16);
+    for (int R = 1; R <= (kind == DFL_XF_Q4K && nb <= 16 ? 2 : 1); R++)
+        for (int tl = 1; tl <= 16 / ksplit; tl++) {
+            const int units = (tiles + R - 1) / R, n_wg = (units + tl - 1) / tl;
+            if (n_wg > ctx->n_cu) continue;
+            p = {kind, ksplit, tl, R, units, n_wg, false};
+            // (lines of LDS: the partial tiles and a wave's rows)
+            if (static_cast<size_t>(16) * R * 64 * sizeof(float4_t) + static_cast<size_t>(ksplit) * tl * kRowAreaBytes > ctx->lds_bytes) p.kind = DFL_XF_NONE;
+            return p;
+        }
+    return p;
+}
+template <typename W, typename XT>
+const void *rows_direct_fn(int R) {
+    if constexpr (!std::is_same<W, Q6W>::value)
+        if (R == 2) return reinterpret_cast<const void *>(gemm_whole_kernel<W, 2, 0, RowSrc<XT>>);
+    return reinterpret_cast<const void *>(gemm_whole_kernel<W, 1, 0, RowSrc<XT>>);
+}
+}  // namespace
+
+bool dfl_gemm_direct_takes(const dflash_ctx *ctx, int32_t w_type, int64_t n_in, int64_t n_out) {
+    return rows_direct_plan(ctx, w_type, n_in, n_out).kind != DFL_XF_NONE;
+}
+
+int32_t dfl_gemm_direct(dflash_ctx *ctx, int32_t w_type, const void *w, const void *x, int32_t x_type, float *y, int64_t n_in, int64_t n_out,
+                        int32_t n_rows, hipStream_t st) {
+    const WholePlan p = rows_direct_plan(ctx, w_type, n_in, n_out);
+    if (p.kind == DFL_XF_NONE || n_rows < 1 || n_rows > 16)
+        return dfl_fail(ctx, DFLASH_ERR_UNSUPPORTED, "gemm_direct: type %d, %lld -> %lld not taken", w_type, static_cast<long long>(n_in),
+                        static_cast<long long>(n_out));
+    if (reinterpret_cast<uintptr_t>(x) % (x_type == DFLASH_TYPE_F32 ? 16 : 8))
+        return dfl_fail(ctx, DFLASH_ERR_ALIGNMENT, "gemm_fewrow: activations must be 16-byte (f32) / 8-byte (f16) aligned");
+    const bool q6 = w_type == DFLASH_TYPE_Q6_K, f32 = x_type == DFLASH_TYPE_F32;
+    WholeArgs a = {};
+    a.w = static_cast<const uint8_t *>(w);
+    a.xf = static_cast<const uint8_t *>(x);
+    a.y = y;
+    a.n_out = static_cast<int>(n_out);
+    a.nb = static_cast<int>(n_in / DFL_QK_K);
+    a.n_rows = n_rows;
+    a.ksplit = p.ksplit;
+    a.tl = p.tl;
+    a.n_units = p.n_units;
+    a.row_bytes = static_cast<uint32_t>(a.nb) * (q6 ? DFL_Q6_K_BYTES : DFL_Q4_K_BYTES);
+    a.n_blocks = 1;
+    a.rows_last = n_rows;
+    const size_t lds = static_cast<size_t>(16) * p.R * 64 * sizeof(float4_t) + static_cast<size_t>(p.ksplit) * p.tl * kRowAreaBytes;
+    const void *fn = q6 ? (f32 ? rows_direct_fn<Q6W, float>(p.R) : rows_direct_fn<Q6W, _Float16>(p.R))
+                     : w_type == DFLASH_TYPE_Q4_K_TILED ? (f32 ? rows_direct_fn<Q4W, float>(p.R) : rows_direct_fn<Q4W, _Float16>(p.R))
+                                                        : (f32 ? rows_direct_fn<Q4R, float>(p.R) : rows_direct_fn<Q4R, _Float16>(p.R));
+    if (lds > 48 * 1024)
+        if (const int32_t rc = dfl_raise_lds_limit(ctx, fn, lds)) return rc;
+    dfl_timed timer(ctx, st, DFL_T_GEMM);
+    void *args[] = {&a};
+    DFL_HIP_CHECK(ctx, hipLaunchKernel(fn, dim3(p.n_wg), dim3(64 * p.ksplit * p.tl), args, lds, st));
     return DFLASH_OK;
 }
 

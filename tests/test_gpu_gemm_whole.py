@@ -204,3 +204,39 @@ def test_shapes_outside_the_path_are_declined(ctx):
     with pytest.raises(dfl.DFlashError) as e:
         ctx.pack_xf(torch.zeros((16, 300), device="cuda"), dfl.XF_Q4K)
     assert e.value.kind == "BadShape"
+
+
+# one super-block and one tile; a last tile and a last super-block slice that are ragged; both sides of one round of tiles at
+# one tile a wave, of two tiles a wave (Q4_K), and of the widest K taken (24 super-blocks; 16 for two tiles)
+DIRECT_SHAPES = [(256, 5), (2048, 512), (1280, 4097), (4096, 4096), (4096, 4097), (4096, 8192), (4096, 8193), (4352, 130), (6144, 2047), (6400, 64)]
+
+
+@pytest.mark.parametrize("qtype", [dfl.synth.Q4_K, dfl.synth.Q6_K])
+@pytest.mark.parametrize("n_in,n_out", DIRECT_SHAPES)
+@pytest.mark.parametrize("rows,x_dtype", [(1, "f32"), (2, "f16"), (15, "f32"), (16, "f16")])
+def test_rows_in_row_order_give_the_bits_of_packed_rows(ctx, oracle, canaries, qtype, n_in, n_out, rows, x_dtype):
+    """The public operator on small matrices is one launch that brings the caller's rows in itself: the bits of pack_xf +
+    gemm_fewrow_xf on the same operands (where both run, the same products in the same order), f16 rows at an 8-byte
+    boundary included, and the same bits for either order of the weights and for a row alone."""
+    import torch
+
+    w, w_type, blocks, w_rows = upload(ctx, qtype, n_in, n_out, seed=n_in + n_out)
+    tag = ctx.checked_type(qtype, w_rows)
+    x = dev(np.random.default_rng(rows).standard_normal((rows, n_in)).astype(np.float32))
+    if x_dtype == "f16":
+        x = torch.cat([torch.zeros(4, device="cuda", dtype=torch.float16), x.half().flatten()])[4:].view(rows, n_in)
+        assert x.data_ptr() % 16 == 8
+    y = ctx.gemm_fewrow(w_rows, tag, x, n_in, n_out)
+    canaries.check()
+    assert torch.equal(ctx.gemm_fewrow(w, w_type, x, n_in, n_out).view(torch.int32), y.view(torch.int32))
+    alone = x[rows - 1:].clone()
+    assert torch.equal(ctx.gemm_fewrow(w_rows, tag, alone, n_in, n_out).view(torch.int32), y[rows - 1:].view(torch.int32))
+    tiles = (n_out + 15) // 16
+    one_round = 256 * (16 // min(n_in // 256, 16))
+    if n_in <= 6144 and (tiles <= one_round or (qtype == dfl.synth.Q4_K and n_in <= 4096 and tiles <= 2 * one_round)):
+        xf = ctx.pack_xf(x, ctx.xf_kind(w_type, n_in, n_out))
+        assert torch.equal(ctx.gemm_fewrow_xf(w, w_type, xf, rows, n_in, n_out).view(torch.int32), y.view(torch.int32))
+    cols = np.unique(np.concatenate([np.arange(min(n_out, 40)), np.arange(max(0, n_out - 40), n_out)]))
+    wf = oracle.dequant(qtype, np.ascontiguousarray(blocks[cols]), len(cols) * n_in).reshape(len(cols), n_in).astype(np.float64)
+    ref = x.half().cpu().numpy().astype(np.float64) @ wf.T
+    check(y[:, torch.from_numpy(cols).cuda()].cpu().numpy(), ref, f"{n_in}->{n_out} x{rows}")
