@@ -27,6 +27,8 @@
 #include "common.h"
 #include "mfma_unpack.h"
 
+#include <hip/hip_ext.h>
+
 #include <algorithm>
 #include <cstdlib>
 #include <type_traits>
@@ -398,39 +400,52 @@ template <typename W>
 __device__ __forceinline__ void load_act(XfSrc, half8_t (&af)[8], const WholeArgs &, const uint8_t *xf, int b, int lane, uint8_t *) {
     load_xf(af, xf, b, lane);
 }
-template <typename W, typename XT>
-__device__ __forceinline__ void load_act(RowSrc<XT>, half8_t (&af)[8], const WholeArgs &a, const uint8_t *x, int b, int lane, uint8_t *area) {
-    const XT *xb = reinterpret_cast<const XT *>(x) + b * DFL_QK_K;
-    const size_t stride = static_cast<size_t>(a.nb) * DFL_QK_K;
-    if constexpr (sizeof(XT) == 4) {
-        float4_t raw[16];
+// One super-block of the rows, row-contiguous: f32 a row a load, f16 two rows a load.
+template <typename XT>
+struct RowsRaw {
+    static constexpr int kLoads = 16 * sizeof(XT) / 4, kRowsPerLoad = 16 / kLoads;
+    u32x4_t v[kLoads];
+};
+template <typename XT>
+__device__ __forceinline__ void rows_load(RowsRaw<XT> &r, const XT *xb, size_t stride, int n_rows, int lane) {
 #pragma unroll
-        for (int m = 0; m < 16; m++)
-            if (m < a.n_rows) raw[m] = *reinterpret_cast<const float4_t *>(xb + m * stride + 4 * lane);
+    for (int i = 0; i < RowsRaw<XT>::kLoads; i++)
+        if (i * RowsRaw<XT>::kRowsPerLoad < n_rows) {
+            if constexpr (sizeof(XT) == 4)
+                r.v[i] = *reinterpret_cast<const u32x4_t *>(xb + i * stride + 4 * lane);
+            else
+                r.v[i] = *reinterpret_cast<const u32x4_row_t *>(xb + min(2 * i + (lane >> 5), n_rows - 1) * stride + 8 * (lane & 31));
+        }
+}
+// Rows 16 / kParts * part .. as f16 into the area, row m (from the part's first) at 512 m, its 16-byte slot o at o ^ m, a slot's eight values in
+// fragment order (0 2 1 3 4 6 5 7).
+template <typename XT, int kParts>
+__device__ __forceinline__ void rows_to_lds(const RowsRaw<XT> &r, int part, int n_rows, int lane, uint8_t *area) {
+    constexpr int kPer = RowsRaw<XT>::kLoads / kParts;
 #pragma unroll
-        for (int m = 0; m < 16; m++)
-            if (m < a.n_rows) {
-                const half4_t h = {static_cast<_Float16>(raw[m][0]), static_cast<_Float16>(raw[m][2]), static_cast<_Float16>(raw[m][1]),
-                                   static_cast<_Float16>(raw[m][3])};
-                *reinterpret_cast<half4_t *>(area + m * 512 + (((lane >> 1) ^ m) * 16 + (lane & 1) * 8)) = h;
-            }
-    } else {
-        u32x4_t raw[8];
-        const int odd = lane >> 5, o = lane & 31;
-#pragma unroll
-        for (int p = 0; p < 8; p++)
-            if (2 * p < a.n_rows) raw[p] = *reinterpret_cast<const u32x4_row_t *>(xb + min(2 * p + odd, a.n_rows - 1) * stride + 8 * o);
-#pragma unroll
-        for (int p = 0; p < 8; p++)
-            if (2 * p < a.n_rows) {
-                const int m = 2 * p + odd;
-                const u32x4_t r = raw[p];  // element order 0 2 1 3 4 6 5 7
+    for (int j = 0; j < kPer; j++) {
+        const int i = part * kPer + j;
+        if (i * RowsRaw<XT>::kRowsPerLoad < n_rows) {
+            const u32x4_t v = r.v[i];
+            if constexpr (sizeof(XT) == 4) {
+                const float4_t f = __builtin_bit_cast(float4_t, v);
+                *reinterpret_cast<half4_t *>(area + j * 512 + ((lane >> 1) ^ j) * 16 + (lane & 1) * 8) =
+                    half4_t{static_cast<_Float16>(f[0]), static_cast<_Float16>(f[2]), static_cast<_Float16>(f[1]), static_cast<_Float16>(f[3])};
+            } else {
+                const int m = 2 * j + (lane >> 5), o = lane & 31;
                 *reinterpret_cast<u32x4_t *>(area + m * 512 + (o ^ m) * 16) =
-                    u32x4_t{__builtin_amdgcn_perm(r.y, r.x, 0x05040100u), __builtin_amdgcn_perm(r.y, r.x, 0x07060302u),
-                            __builtin_amdgcn_perm(r.w, r.z, 0x05040100u), __builtin_amdgcn_perm(r.w, r.z, 0x07060302u)};
+                    u32x4_t{__builtin_amdgcn_perm(v.y, v.x, 0x05040100u), __builtin_amdgcn_perm(v.y, v.x, 0x07060302u),
+                            __builtin_amdgcn_perm(v.w, v.z, 0x05040100u), __builtin_amdgcn_perm(v.w, v.z, 0x07060302u)};
             }
+        }
     }
     __builtin_amdgcn_wave_barrier();
+}
+template <typename W, typename XT>
+__device__ __forceinline__ void load_act(RowSrc<XT>, half8_t (&af)[8], const WholeArgs &a, const uint8_t *x, int b, int lane, uint8_t *area) {
+    RowsRaw<XT> raw;
+    rows_load(raw, reinterpret_cast<const XT *>(x) + b * DFL_QK_K, static_cast<size_t>(a.nb) * DFL_QK_K, a.n_rows, lane);
+    rows_to_lds<XT, 1>(raw, 0, a.n_rows, lane, area);
     constexpr bool q6 = std::is_same<typename FragsOf<W>::type, Q6F>::value;
     const int m = lane & 15, g = lane >> 4;
     // (octets of a lane: common.h, "XF")
@@ -715,6 +730,176 @@ __global__ void __launch_bounds__(1024) gemm_q6t_loop_kernel(WholeArgs a) {
     }
 }
 
+// The public operator on a Q4_K matrix of many rounds of tiles, K of at most 32 super-blocks, rows in row order: one workgroup per
+// CU walks units of one tile, its waves share K.  A wave keeps the fragments and the sub-block sums of its one or two
+// super-blocks in registers for every tile, so a tile costs it nothing but weights, which it streams through a private
+// ring of LDS slots (a slot: one super-block of the tile, 144 pieces of 16 bytes, three direct-to-LDS loads); the slices' partial tiles
+// meet in one of two LDS buffers in turn, one barrier per tile, a different wave adding each time.  No partial tiles in memory, no second launch.
+// What bounds it: the stream of the weights (46 KB a tile of K = 5120 at 5.3 - 5.6 TB/s over the chip) behind a start of 4 us, in which every
+// CU takes in all of the rows; where the tiles are a few rounds, the last one, for which only some CUs have a tile.
+// us a call, weights cold, streaming kernel and reduction : this one, 1 row f32 / 16 rows f16 / 16 rows f32:
+//   tiled Q4_K  5120 -> 17408 17.9 :17.0 20.2 :17.2 20.5 :19.4   2560 -> 16384 12.2 : 9.2 13.3 :10.2 13.4 :10.8   2048 -> 40000 17.0 :13.0 20.3 :14.4 20.3 :15.9
+//   row order   5120 -> 17408 18.1 :17.7 19.8 :18.2 19.9 :20.3   2560 -> 16384 12.6 : 9.4 14.4 :10.1 14.4 :11.3   2048 -> 40000 17.0 :13.5 19.2 :15.1 19.2 :16.6
+// (no stage ahead of the rows, or four: 18.3 and 18.5 for 16 f16 rows, 5120 -> 17408).
+// `landed` is an s_waitcnt vmcnt of the loads behind: they return in order, and a Y store among them only makes it stricter.
+constexpr int kWideSlot = 16 * DFL_Q4_K_BYTES;  // 2304 bytes
+constexpr int kWideSlots = 6;                        // at most (the counts below)
+__device__ __forceinline__ void wide_wait(int ahead) {  // at most `ahead` stages (three loads each) still under way, ahead uniform
+    if (ahead <= 0)
+        __builtin_amdgcn_s_waitcnt(kVmcnt0);
+    else if (ahead == 1)
+        __builtin_amdgcn_s_waitcnt(0x0F70 | 3);
+    else if (ahead == 2)
+        __builtin_amdgcn_s_waitcnt(0x0F70 | 6);
+    else if (ahead == 3)
+        __builtin_amdgcn_s_waitcnt(0x0F70 | 9);
+    else if (ahead == 4)
+        __builtin_amdgcn_s_waitcnt(0x0F70 | 12);
+    else
+        __builtin_amdgcn_s_waitcnt(0x0F70 | 15);
+}
+// The fragments of one super-block out of its rows: in one go through 8 KB of LDS, or eight rows at a time through 4 KB.
+template <typename XT, int kParts>
+__device__ __forceinline__ void wide_fragments(half8_t (&af)[8], const RowsRaw<XT> &raw, int n_rows, int lane, uint8_t *area) {
+    const int g = lane >> 4;
+#pragma unroll
+    for (int part = 0; part < kParts; part++) {
+        rows_to_lds<XT, kParts>(raw, part, n_rows, lane, area);
+        const int m = lane & (16 / kParts - 1);
+        half8_t v[8];
+#pragma unroll
+        for (int t = 0; t < 8; t++) v[t] = *reinterpret_cast<const half8_t *>(area + m * 512 + ((8 * g + t) ^ m) * 16);
+#pragma unroll
+        for (int t = 0; t < 8; t++) {
+            asm volatile("" : "+v"(v[t]));  // (read by every lane: a select, not a branch around each read)
+            af[t] = kParts == 1 || ((lane & 15) >> 3) == part ? v[t] : af[t];
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+// kLen: super-blocks a wave has at most (two: at most twelve waves, whose registers hold both).
+template <typename XT, bool kTiled, int kLen, int kSlots>
+__global__ void __launch_bounds__(kLen == 2 ? 768 : 1024) gemm_q4k_wide_kernel(WholeArgs a) {
+    extern __shared__ float4_t red[];  // [2][waves][64], then the rings [wave][kSlots][kWideSlot]
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), waves = a.ksplit * a.tl;
+    const int tlane = wave / a.ksplit, kslice = wave - tlane * a.ksplit;
+    const int n = lane & 15, g = lane >> 4;
+    const int b0 = a.nb * kslice / a.ksplit, len = a.nb * (kslice + 1) / a.ksplit - b0;  // one or two super-blocks (host)
+    const int n_tiles = (a.n_out + 15) >> 4, stride = static_cast<int>(gridDim.x) * a.tl;
+    const int first = static_cast<int>(blockIdx.x) * a.tl, unit0 = first + tlane;
+    const int units = unit0 < n_tiles ? (n_tiles - 1 - unit0) / stride + 1 : 0;  // of this wave
+    const int rounds = (n_tiles - 1 - first) / stride + 1;                       // of the workgroup (its first tile lane has the most)
+    const int n_stages = units * len;
+    uint8_t *ring = reinterpret_cast<uint8_t *>(red + 2 * waves * 64) + static_cast<size_t>(wave) * (kSlots * kWideSlot);
+    // the next stage to issue: super-block b0 + i_b of tile i_tile, into slot i_slot
+    int issued = 0, i_b = 0, i_tile = unit0, i_slot = 0;
+    int r0 = 0, r1 = 0, r2 = 0, p0 = 0, p1 = 0, p2 = 0;  // row order: the lane's three pieces of a stage, rows and bytes in them
+    if constexpr (!kTiled) {
+        r0 = lane / 9, p0 = 16 * (lane - 9 * r0);
+        r1 = (lane + 64) / 9, p1 = 16 * (lane + 64 - 9 * r1);
+        r2 = (lane + 128) / 9, p2 = 16 * (lane + 128 - 9 * r2);  // (lanes past 15 issue nothing)
+    }
+    auto issue = [&]() {
+        uint8_t *dst = ring + i_slot * kWideSlot;
+        const int tile = min(i_tile, n_tiles - 1);  // (past the last: one of the first stages, which go out whatever there is; not read)
+        if constexpr (kTiled) {
+            const uint8_t *src = a.w + ((static_cast<size_t>(tile >> 4) * a.nb + b0 + i_b) * 16 + (tile & 15)) * kWideSlot + lane * 16;
+            __builtin_amdgcn_global_load_lds((gptr_t)(src), (lptr_t)(dst), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds((gptr_t)(src + 1024), (lptr_t)(dst + 1024), 16, 0, 0);
+            if (lane < 16) __builtin_amdgcn_global_load_lds((gptr_t)(src + 2048), (lptr_t)(dst + 2048), 16, 0, 0);
+        } else {
+            // (rows past the matrix re-read its last row; never stored)
+            const uint8_t *src = a.w + static_cast<size_t>(b0 + i_b) * DFL_Q4_K_BYTES;
+            const int t = tile * 16, last = a.n_out - 1;
+            __builtin_amdgcn_global_load_lds((gptr_t)(src + static_cast<size_t>(min(t + r0, last)) * a.row_bytes + p0), (lptr_t)(dst), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds((gptr_t)(src + static_cast<size_t>(min(t + r1, last)) * a.row_bytes + p1), (lptr_t)(dst + 1024), 16, 0, 0);
+            if (lane < 16)
+                __builtin_amdgcn_global_load_lds((gptr_t)(src + static_cast<size_t>(min(t + r2, last)) * a.row_bytes + p2), (lptr_t)(dst + 2048), 16, 0, 0);
+        }
+        issued++;
+        if (++i_slot == kSlots) i_slot = 0;
+        if (++i_b == len) {
+            i_b = 0;
+            i_tile += stride;
+        }
+    };
+    // The rows first (they come from L2), behind them the first stages, as many as leave the rows' way through LDS alone; the others
+    // once the fragments stand.
+    constexpr int kAreaSlots = kLen == 2 ? 4 : 2;  // 8 KB, or 4 KB where there are three slots to a wave
+    half8_t af0[8] = {}, af1[kLen == 2 ? 8 : 1] = {}, am0, am1;
+    {
+        uint8_t *area = ring + (kSlots - kAreaSlots) * kWideSlot;
+        static_assert(kAreaSlots * kWideSlot >= 16 * 512 / (kLen == 2 ? 1 : 2), "the rows' area");
+        const XT *xb = reinterpret_cast<const XT *>(a.xf) + static_cast<size_t>(b0) * DFL_QK_K;
+        const size_t xs = static_cast<size_t>(a.nb) * DFL_QK_K;
+        RowsRaw<XT> raw0, raw1;
+        rows_load(raw0, xb, xs, a.n_rows, lane);
+        if constexpr (kLen == 2)
+            if (len > 1) rows_load(raw1, xb + DFL_QK_K, xs, a.n_rows, lane);
+        // (a fixed number of stages without a branch: the compiler then waits for the rows alone, not for what is behind them)
+        issue();
+        if constexpr (kSlots - kAreaSlots > 1) issue();
+        wide_fragments<XT, kLen == 2 ? 1 : 2>(af0, raw0, a.n_rows, lane, area);
+        if constexpr (kLen == 2) {
+            if (len > 1) {
+                wide_fragments<XT, 1>(af1, raw1, a.n_rows, lane, area);
+            }
+            am1 = sum_operand(af1);
+        }
+        am0 = sum_operand(af0);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // (the area's last reads are done: its slots may be loaded into)
+    while (issued < n_stages && issued < kSlots) issue();
+
+    const uint32_t sc_sel = (lane & 16) ? 0x04030402u : 0x04010400u;
+    const Q4KMagic magic = q4k_magic();
+    int done = 0, slot = 0;
+    float4_t acc;
+    auto stage = [&](const half8_t (&af)[8], const half8_t &am) {
+        wide_wait(issued - done - 1);
+        const u32x4_t *p = reinterpret_cast<const u32x4_t *>(ring + slot * kWideSlot) + n * 9;
+        Q4S w;
+        w.hdr = p[0];
+        w.q0 = p[1 + 2 * g];
+        w.q1 = p[2 + 2 * g];
+        Q4SF f;
+        unpack(w, lane, nullptr, sc_sel, magic, f);
+        const half2_t mn = {-f.m_lo, -f.m_hi};
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(am, q4k_min_operand(mn), acc, 0, 0, 0);
+#pragma unroll
+        for (int t = 0; t < 8; t++) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[t], f.b[t], acc, 0, 0, 0);
+        done++;
+        if (++slot == kSlots) slot = 0;
+        if (issued < n_stages) issue();  // (into the slot just read: its operands are in registers)
+    };
+    for (int it = 0; it < rounds; it++) {
+        const int unit = unit0 + it * stride;
+        acc = float4_t{0, 0, 0, 0};
+        if (it < units) {
+            stage(af0, am0);
+            if constexpr (kLen == 2)
+                if (len > 1) stage(af1, am1);
+        }
+        float4_t *buf = red + (it & 1) * (waves * 64);
+        buf[wave * 64 + lane] = acc;
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        // the slices take turns at the sum (a buffer is rewritten two rounds later, behind the barrier of the round between)
+        if (kslice == it % a.ksplit && it < units) {
+            const float4_t *part = buf + tlane * a.ksplit * 64 + lane;
+            float4_t sum = part[0];
+            for (int s = 1; s < a.ksplit; s++) sum += part[s * 64];
+            const int col = unit * 16 + n;
+            if (col < a.n_out) {
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    if (4 * g + i < a.n_rows) a.y[static_cast<size_t>(4 * g + i) * a.n_out + col] = sum[i];
+            }
+        }
+    }
+    if (issued > n_stages) __builtin_amdgcn_s_waitcnt(kVmcnt0);  // (nothing is under way into LDS when the wave ends)
+}
+
 // Row-major activations -> XF: one thread per (row, eight consecutive values).
 template <typename XT>
 __global__ void __launch_bounds__(256) pack_xf_kernel(const XT *__restrict__ x, int n_rows, int n_in, int kind, uint8_t *__restrict__ xf) {
@@ -904,6 +1089,25 @@ WholePlan rows_direct_plan(const dflash_ctx *ctx, int32_t w_type, int64_t n_in, 
         }
     return p;
 }
+// The looping kernel's: K shared by one or two super-blocks a wave, as many waves as the ring leaves room for.
+struct WidePlan {
+    int ksplit, tl, slots, n_wg;
+};
+WidePlan rows_wide_plan(const dflash_ctx *ctx, int32_t w_type, int64_t n_in, int64_t n_out) {
+    WidePlan p = {0, 0, 0, 0};
+    const int nb = static_cast<int>(n_in / DFL_QK_K);
+    if ((w_type != DFLASH_TYPE_Q4_K && w_type != DFLASH_TYPE_Q4_K_TILED) || n_in % DFL_QK_K || nb < 1 || nb > 24 || n_out < 1 || n_out >= (1 << 24)) return p;
+    const int tiles = static_cast<int>((n_out + 15) / 16);
+    // (two super-blocks a wave take in the rows in 2 us more: from three rounds on; 5120 -> 6144, 16 rows f32, tiled 11.5 :12.1)
+    if (nb > 16 && tiles < 3 * ctx->n_cu) return p;
+    const int ksplit = nb > 16 ? (nb + 1) / 2 : nb, tl = 16 / ksplit > 0 && nb <= 16 ? 16 / ksplit : 1, waves = ksplit * tl;
+    const size_t red = static_cast<size_t>(2) * waves * 64 * sizeof(float4_t);
+    if (red >= ctx->lds_bytes) return p;
+    const int slots = std::min<int>(kWideSlots, static_cast<int>((ctx->lds_bytes - red) / (static_cast<size_t>(waves) * kWideSlot)));
+    if (slots < (nb > 16 ? 5 : 3)) return p;
+    p = {ksplit, tl, slots == 5 && nb <= 16 ? 4 : slots, std::min((tiles + tl - 1) / tl, ctx->n_cu)};
+    return p;
+}
 template <typename W, typename XT>
 const void *rows_direct_fn(int R) {
     if constexpr (!std::is_same<W, Q6W>::value)
@@ -913,13 +1117,14 @@ const void *rows_direct_fn(int R) {
 }  // namespace
 
 bool dfl_gemm_direct_takes(const dflash_ctx *ctx, int32_t w_type, int64_t n_in, int64_t n_out) {
-    return rows_direct_plan(ctx, w_type, n_in, n_out).kind != DFL_XF_NONE;
+    return rows_direct_plan(ctx, w_type, n_in, n_out).kind != DFL_XF_NONE || rows_wide_plan(ctx, w_type, n_in, n_out).ksplit;
 }
 
 int32_t dfl_gemm_direct(dflash_ctx *ctx, int32_t w_type, const void *w, const void *x, int32_t x_type, float *y, int64_t n_in, int64_t n_out,
                         int32_t n_rows, hipStream_t st) {
     const WholePlan p = rows_direct_plan(ctx, w_type, n_in, n_out);
-    if (p.kind == DFL_XF_NONE || n_rows < 1 || n_rows > 16)
+    const WidePlan wp = rows_wide_plan(ctx, w_type, n_in, n_out);
+    if ((p.kind == DFL_XF_NONE && !wp.ksplit) || n_rows < 1 || n_rows > 16)
         return dfl_fail(ctx, DFLASH_ERR_UNSUPPORTED, "gemm_direct: type %d, %lld -> %lld not taken", w_type, static_cast<long long>(n_in),
                         static_cast<long long>(n_out));
     if (reinterpret_cast<uintptr_t>(x) % (x_type == DFLASH_TYPE_F32 ? 16 : 8))
@@ -938,6 +1143,27 @@ int32_t dfl_gemm_direct(dflash_ctx *ctx, int32_t w_type, const void *w, const vo
     a.row_bytes = static_cast<uint32_t>(a.nb) * (q6 ? DFL_Q6_K_BYTES : DFL_Q4_K_BYTES);
     a.n_blocks = 1;
     a.rows_last = n_rows;
+    if (p.kind == DFL_XF_NONE) {
+        a.ksplit = wp.ksplit;
+        a.tl = wp.tl;
+        const int waves = wp.ksplit * wp.tl;
+        const bool tiled = w_type == DFLASH_TYPE_Q4_K_TILED;
+        const size_t wlds = static_cast<size_t>(2) * waves * 64 * sizeof(float4_t) + static_cast<size_t>(waves) * wp.slots * kWideSlot;
+        const bool two = a.nb > 16;
+#define DFL_WIDE_PICK(XT, LEN, SLOTS) (tiled ? (kernel_t)gemm_q4k_wide_kernel<XT, true, LEN, SLOTS> : (kernel_t)gemm_q4k_wide_kernel<XT, false, LEN, SLOTS>)
+#define DFL_WIDE_PICK4(XT) (two ? (wp.slots == 6 ? DFL_WIDE_PICK(XT, 2, 6) : DFL_WIDE_PICK(XT, 2, 5)) \
+                                : (wp.slots == 6 ? DFL_WIDE_PICK(XT, 1, 6) : wp.slots == 4 ? DFL_WIDE_PICK(XT, 1, 4) : DFL_WIDE_PICK(XT, 1, 3)))
+        typedef void (*kernel_t)(WholeArgs);
+        const void *wfn = reinterpret_cast<const void *>(f32 ? DFL_WIDE_PICK4(float) : DFL_WIDE_PICK4(_Float16));
+#undef DFL_WIDE_PICK4
+#undef DFL_WIDE_PICK
+        if (const int32_t rc = dfl_raise_lds_limit(ctx, wfn, wlds)) return rc;
+        dfl_timed timer(ctx, st, DFL_T_GEMM);
+        const dfl_stamp sp(ctx, DFL_T_KERNEL_Q4K_TILED);
+        void *wargs[] = {&a};
+        DFL_HIP_CHECK(ctx, hipExtLaunchKernel(wfn, dim3(wp.n_wg), dim3(64 * waves), wargs, wlds, st, sp.start, sp.stop, 0));
+        return DFLASH_OK;
+    }
     const size_t lds = static_cast<size_t>(16) * p.R * 64 * sizeof(float4_t) + static_cast<size_t>(p.ksplit) * p.tl * kRowAreaBytes;
     const void *fn = q6 ? (f32 ? rows_direct_fn<Q6W, float>(p.R) : rows_direct_fn<Q6W, _Float16>(p.R))
                      : w_type == DFLASH_TYPE_Q4_K_TILED ? (f32 ? rows_direct_fn<Q4W, float>(p.R) : rows_direct_fn<Q4W, _Float16>(p.R))

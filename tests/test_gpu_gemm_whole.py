@@ -240,3 +240,36 @@ def test_rows_in_row_order_give_the_bits_of_packed_rows(ctx, oracle, canaries, q
     wf = oracle.dequant(qtype, np.ascontiguousarray(blocks[cols]), len(cols) * n_in).reshape(len(cols), n_in).astype(np.float64)
     ref = x.half().cpu().numpy().astype(np.float64) @ wf.T
     check(y[:, torch.from_numpy(cols).cuda()].cpu().numpy(), ref, f"{n_in}->{n_out} x{rows}")
+
+
+# many rounds of tiles: K of one super-block (sixteen tiles a workgroup), of one and two super-blocks a wave, an odd split of K
+# (17: nine waves, one of them with one super-block), the widest (24); a ragged last tile, a last round that few workgroups have
+WIDE_SHAPES = [(256, 140001), (768, 45000), (1024, 33000), (2048, 16400), (2560, 8200), (4096, 8193), (4352, 12300), (5120, 17408), (6144, 12289)]
+
+
+@pytest.mark.parametrize("n_in,n_out", WIDE_SHAPES)
+@pytest.mark.parametrize("rows,x_dtype", [(1, "f32"), (7, "f16"), (9, "f32"), (16, "f16"), (16, "f32")])
+def test_rows_in_row_order_against_many_rounds_of_tiles(ctx, oracle, canaries, n_in, n_out, rows, x_dtype):
+    """The looping product of the public operator: against the f64 product on columns of every round, the same bits for either
+    order of the weights and for a row alone, twice in a row, rows whose sub-block sums pass the f16 range included."""
+    import torch
+
+    blocks = dfl.synth.random_blocks(dfl.synth.Q4_K, n_out * n_in // 256, seed=n_in + n_out).reshape(n_out, -1)
+    w_rows = dev(blocks)
+    tag = ctx.checked_type(dfl.synth.Q4_K, w_rows)
+    wt = ctx.repack_q4k_tiled(w_rows, n_in, n_out)
+    x = np.random.default_rng(rows).standard_normal((rows, n_in)).astype(np.float32)
+    x[rows // 2] += 2500.0
+    xd = dev(x.astype(np.float16 if x_dtype == "f16" else np.float32))
+    y = ctx.gemm_fewrow(w_rows, tag, xd, n_in, n_out)
+    canaries.check()
+    for other in (ctx.gemm_fewrow(wt, dfl.TYPE_Q4_K_TILED, xd, n_in, n_out), ctx.gemm_fewrow(w_rows, tag, xd, n_in, n_out)):
+        assert torch.equal(other.view(torch.int32), y.view(torch.int32))
+    alone = ctx.gemm_fewrow(wt, dfl.TYPE_Q4_K_TILED, xd[rows - 1:].clone(), n_in, n_out)
+    assert torch.equal(alone.view(torch.int32), y[rows - 1:].view(torch.int32))
+    cols = np.unique(np.concatenate([np.arange(16), np.random.default_rng(n_out).integers(0, n_out, 500), np.arange(n_out - 20, n_out)]))
+    wf = oracle.dequant(dfl.synth.Q4_K, np.ascontiguousarray(blocks[cols]), len(cols) * n_in).reshape(len(cols), n_in).astype(np.float64)
+    ref = x.astype(np.float16).astype(np.float64) @ wf.T
+    got = y[:, torch.from_numpy(cols).cuda()].cpu().numpy()
+    for r in range(rows):
+        check(got[r:r + 1], ref[r:r + 1], f"{n_in}->{n_out} row {r}")
