@@ -47,7 +47,7 @@ struct WholeArgs {
     int ksplit;  // K slices per unit; waves per workgroup = ksplit * tl
     int tl;      // units per workgroup
     int n_units; // plain: ceil(tiles / R) units of R consecutive tiles; pair: ffn / 16 units of (gate tile, up tile)
-    int pair_off;  // pair mode: tiles between a gate tile and its up tile; 0 = plain
+    int pair_off;  // pair mode: tiles between a gate tile and its up tile; 0 = plain.  (The looping kernels: workgroups of the launch.)
     uint32_t row_bytes;  // Q6_K (GGUF row order): bytes per weight row
     // several 16-row blocks against the same weights (a prefill): block i reads xf + i * xf_stride bytes and writes
     // y + i * y_stride floats (y_xf + i * y_xf_stride bytes); the last block has rows_last rows, the others 16
@@ -55,6 +55,34 @@ struct WholeArgs {
     uint32_t xf_stride, y_xf_stride;
     size_t y_stride;
 };
+// As kernel parameters: what a wave needs for its first loads as words of their own, fourteen at most, which arrive in its
+// scalar registers (a parameter that is a structure has to be loaded, a trip of 0.5 us to memory the host has just written,
+// and a division by ksplit is some forty instructions, ahead of the first weight); the rest behind them.
+// TAILNEW
+struct WholeTail {
+    uint8_t *y_xf;
+    int y_xf_kind, n_blocks, rows_last;
+    uint32_t xf_stride, y_xf_stride;
+    size_t y_stride;
+};
+#define DFL_WHOLE_PARAMS                                                                                                             \
+    const uint8_t *w, const uint8_t *xf, float *y, uint32_t split, uint32_t by_ksplit, int nb, int n_out, int n_units, int pair_off, \
+        uint32_t row_bytes, WholeTail tail
+#define DFL_WHOLE_ARGS                                                                                                                        \
+    WholeArgs {                                                                                                                               \
+        w, xf, y, tail.y_xf, tail.y_xf_kind, n_out, nb, static_cast<int>(split >> 16), static_cast<int>(split & 255), static_cast<int>(split >> 8 & 255), \
+            n_units, pair_off, row_bytes, tail.n_blocks, tail.rows_last, tail.xf_stride, tail.y_xf_stride, tail.y_stride                      \
+    }
+typedef void (*whole_kernel_t)(DFL_WHOLE_PARAMS);
+// by_ksplit = ceil(65536 / ksplit): x / ksplit for 0 <= x <= 512 (a wave's index, a super-block's index times a slice's)
+__device__ __forceinline__ int whole_div(int x, uint32_t by_ksplit) { return static_cast<int>(static_cast<uint32_t>(x) * by_ksplit >> 16); }
+void whole_launch(whole_kernel_t fn, int grid, int threads, size_t lds, hipStream_t st, const WholeArgs &a, hipEvent_t start = nullptr,
+                  hipEvent_t stop = nullptr) {
+    const WholeTail tail = {a.y_xf, a.y_xf_kind, a.n_blocks, a.rows_last, a.xf_stride, a.y_xf_stride, a.y_stride};
+    const uint32_t split = static_cast<uint32_t>(a.ksplit | a.tl << 8 | a.n_rows << 16), by_ksplit = (65536u + a.ksplit - 1) / a.ksplit;
+    hipExtLaunchKernelGGL(fn, dim3(grid), dim3(threads), lds, st, start, stop, 0, a.w, a.xf, a.y, split, by_ksplit, a.nb, a.n_out, a.n_units, a.pair_off,
+                          a.row_bytes, tail);
+}
 
 // ---- Q4_K, tiled order: [tile group of 256 rows][super-block][tile][row][144-byte block] ----
 struct Q4W {
@@ -471,16 +499,17 @@ static_assert(kRowAreaBytes >= kQ6AreaBytes, "one area for both");
 // two; the single-block instances (0) keep the registers of a kernel without the loop.  (A prefill takes 1 with R = 1 in the tiled
 // orders, whose weights a wave holds; the others serve dflash_gemm_fewrow_xf.)
 template <typename W, int R, int kMulti, typename X = XfSrc>
-__global__ void __launch_bounds__(1024) gemm_whole_kernel(WholeArgs a) {
+__global__ void __launch_bounds__(1024) gemm_whole_kernel(DFL_WHOLE_PARAMS) {
+    const WholeArgs a = DFL_WHOLE_ARGS;
     // [16 waves][R] partial tiles; Q6_K: then a staging area per wave
     extern __shared__ float4_t red[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int tlane = wave / a.ksplit, kslice = wave - tlane * a.ksplit;
+    const int tlane = whole_div(wave, by_ksplit), kslice = wave - tlane * a.ksplit;
     const int unit = blockIdx.x * a.tl + tlane;
     const bool active = unit < a.n_units;
     const int n = lane & 15, g = lane >> 4;
-    const int b0 = a.nb * kslice / a.ksplit, b1 = a.nb * (kslice + 1) / a.ksplit;  // one or two stages (host)
+    const int b0 = whole_div(a.nb * kslice, by_ksplit), b1 = whole_div(a.nb * (kslice + 1), by_ksplit);  // one or two stages (host)
     const bool two = kMulti != 1 && b1 - b0 > 1;
     const int n_tiles = (a.n_out + 15) >> 4;
     int tile[R];
@@ -610,16 +639,17 @@ __global__ void __launch_bounds__(1024) gemm_whole_kernel(WholeArgs a) {
 // in one of two LDS buffers in turn (one barrier per unit: a buffer is rewritten two units later, behind the barrier
 // of the unit in between).  Same sums, in the same order, as gemm_whole_kernel with twin products.
 template <typename W>
-__global__ void __launch_bounds__(1024) gemm_whole_loop_kernel(WholeArgs a) {
+__global__ void __launch_bounds__(1024) gemm_whole_loop_kernel(DFL_WHOLE_PARAMS) {
+    const WholeArgs a = DFL_WHOLE_ARGS;
     extern __shared__ float4_t red[];  // [2][16 waves][64]; Q6_K in row order: then a staging area per wave
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int tlane = wave / a.ksplit, kslice = wave - tlane * a.ksplit;
+    const int tlane = whole_div(wave, by_ksplit), kslice = wave - tlane * a.ksplit;
     const int n = lane & 15, g = lane >> 4;
-    const int b0 = a.nb * kslice / a.ksplit;  // one stage per wave (host: nb <= 16, so ksplit == nb and every slice is one super-block)
-    const bool has_stage = a.nb * (kslice + 1) / a.ksplit > b0;
+    const int b0 = whole_div(a.nb * kslice, by_ksplit);  // one stage per wave (host: nb <= 16, so ksplit == nb and every slice is one super-block)
+    const bool has_stage = whole_div(a.nb * (kslice + 1), by_ksplit) > b0;
     const int n_tiles = (a.n_out + 15) >> 4;
-    const int stride = static_cast<int>(gridDim.x) * a.tl;
+    const int stride = a.pair_off * a.tl;
     const uint32_t sc_sel = (lane & 16) ? 0x04030402u : 0x04010400u;
     const Q4KMagic magic = q4k_magic();
     uint8_t *area = reinterpret_cast<uint8_t *>(red + 2 * 16 * 64) + wave * kQ6AreaBytes;
@@ -664,15 +694,16 @@ typedef __attribute__((address_space(3))) void *lptr_t;
 constexpr int kQ6RingDepth = 2;
 constexpr int kVmcnt4 = (4 & 0xF) | 0x0F70, kVmcnt0 = 0x0F70;  // s_waitcnt vmcnt(n), the other counters left alone (gfx9 encoding)
 constexpr size_t kQ6LoopLds = static_cast<size_t>(2) * 16 * 64 * sizeof(float4_t) + static_cast<size_t>(16) * kQ6RingDepth * kQ6TileBytes;
-__global__ void __launch_bounds__(1024) gemm_q6t_loop_kernel(WholeArgs a) {
+__global__ void __launch_bounds__(1024) gemm_q6t_loop_kernel(DFL_WHOLE_PARAMS) {
+    const WholeArgs a = DFL_WHOLE_ARGS;
     extern __shared__ float4_t red[];  // [2][16 waves][64], then the rings [16 waves][kQ6RingDepth][3360 bytes]
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int tlane = wave / a.ksplit, kslice = wave - tlane * a.ksplit;
+    const int tlane = whole_div(wave, by_ksplit), kslice = wave - tlane * a.ksplit;
     const int n = lane & 15, g = lane >> 4, h = g >> 1, odd = g & 1;
     const int b0 = kslice;  // (host: nb <= 16, so ksplit == nb and every slice is one super-block)
     const int n_tiles = (a.n_out + 15) >> 4;
-    const int stride = static_cast<int>(gridDim.x) * a.tl;
+    const int stride = a.pair_off * a.tl;
     const Q4KMagic magic = q4k_magic();
     uint8_t *ring = reinterpret_cast<uint8_t *>(red + 2 * 16 * 64) + static_cast<size_t>(wave) * (kQ6RingDepth * kQ6TileBytes);
     auto issue = [&](int unit, int slot) {  // the unit's 210 pieces into ring buffer `slot`
@@ -779,14 +810,15 @@ __device__ __forceinline__ void wide_fragments(half8_t (&af)[8], const RowsRaw<X
 }
 // kLen: super-blocks a wave has at most (two: at most twelve waves, whose registers hold both).
 template <typename XT, bool kTiled, int kLen, int kSlots>
-__global__ void __launch_bounds__(kLen == 2 ? 768 : 1024) gemm_q4k_wide_kernel(WholeArgs a) {
+__global__ void __launch_bounds__(kLen == 2 ? 768 : 1024) gemm_q4k_wide_kernel(DFL_WHOLE_PARAMS) {
+    const WholeArgs a = DFL_WHOLE_ARGS;
     extern __shared__ float4_t red[];  // [2][waves][64], then the rings [wave][kSlots][kWideSlot]
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), waves = a.ksplit * a.tl;
-    const int tlane = wave / a.ksplit, kslice = wave - tlane * a.ksplit;
+    const int tlane = whole_div(wave, by_ksplit), kslice = wave - tlane * a.ksplit;
     const int n = lane & 15, g = lane >> 4;
-    const int b0 = a.nb * kslice / a.ksplit, len = a.nb * (kslice + 1) / a.ksplit - b0;  // one or two super-blocks (host)
-    const int n_tiles = (a.n_out + 15) >> 4, stride = static_cast<int>(gridDim.x) * a.tl;
+    const int b0 = whole_div(a.nb * kslice, by_ksplit), len = whole_div(a.nb * (kslice + 1), by_ksplit) - b0;  // one or two super-blocks (host)
+    const int n_tiles = (a.n_out + 15) >> 4, stride = a.pair_off * a.tl;
     const int first = static_cast<int>(blockIdx.x) * a.tl, unit0 = first + tlane;
     const int units = unit0 < n_tiles ? (n_tiles - 1 - unit0) / stride + 1 : 0;  // of this wave
     const int rounds = (n_tiles - 1 - first) / stride + 1;                       // of the workgroup (its first tile lane has the most)
@@ -1024,11 +1056,10 @@ int32_t dfl_gemm_whole_blocks(dflash_ctx *ctx, int32_t w_type, const void *w, co
     const int threads = 64 * p.ksplit * p.tl;
     const size_t red_bytes = static_cast<size_t>(16) * p.R * 64 * sizeof(float4_t);
     const size_t lds = red_bytes + ((p.kind == DFL_XF_Q6K && !q6_tiled) ? static_cast<size_t>(16) * kQ6AreaBytes : 0);
-    typedef void (*kernel_t)(WholeArgs);
     if (p.loop) {
         if (n_blocks > 1) return dfl_fail(ctx, DFLASH_ERR_UNSUPPORTED, "gemm_whole: a matrix of %d tiles takes one block of rows per call", p.n_units);
         const bool q6_ring = q6_tiled && kQ6LoopLds <= ctx->lds_bytes && env_int("DFLASH_Q6T_RING", 1);
-        const kernel_t lf = p.kind == DFL_XF_Q4K ? gemm_whole_loop_kernel<Q4W>
+        const whole_kernel_t lf = p.kind == DFL_XF_Q4K ? gemm_whole_loop_kernel<Q4W>
                             : q6_ring            ? gemm_q6t_loop_kernel
                             : q6_tiled           ? gemm_whole_loop_kernel<Q6T>
                                                  : gemm_whole_loop_kernel<Q6W>;
@@ -1039,7 +1070,8 @@ int32_t dfl_gemm_whole_blocks(dflash_ctx *ctx, int32_t w_type, const void *w, co
         if (llds > 48 * 1024)
             if (const int32_t rc = dfl_raise_lds_limit(ctx, reinterpret_cast<const void *>(lf), llds)) return rc;
         dfl_timed timer(ctx, st, DFL_T_GEMM);
-        lf<<<p.n_wg, 64 * p.ksplit * p.tl, llds, st>>>(a);
+        a.pair_off = p.n_wg;
+        whole_launch(lf, p.n_wg, 64 * p.ksplit * p.tl, llds, st, a);
         DFL_HIP_CHECK(ctx, hipGetLastError());
         return DFLASH_OK;
     }
@@ -1048,7 +1080,7 @@ int32_t dfl_gemm_whole_blocks(dflash_ctx *ctx, int32_t w_type, const void *w, co
     if (multi && by_sums && (p.R != 1 || multi != 1))
         return dfl_fail(ctx, DFLASH_ERR_UNSUPPORTED, "gemm_whole: several blocks by sums only past weights a wave holds");
 #define DFL_WHOLE_PICK(WT, RR) (multi == 0 ? gemm_whole_kernel<WT, RR, 0> : multi == 1 ? gemm_whole_kernel<WT, RR, 1> : gemm_whole_kernel<WT, RR, 2>)
-    const kernel_t fn = p.kind == DFL_XF_Q4K && by_sums ? (p.R == 2 ? gemm_whole_kernel<Q4S, 2, 0> : multi ? gemm_whole_kernel<Q4S, 1, 1> : gemm_whole_kernel<Q4S, 1, 0>)
+    const whole_kernel_t fn = p.kind == DFL_XF_Q4K && by_sums ? (p.R == 2 ? gemm_whole_kernel<Q4S, 2, 0> : multi ? gemm_whole_kernel<Q4S, 1, 1> : gemm_whole_kernel<Q4S, 1, 0>)
                         : p.kind == DFL_XF_Q4K          ? (p.R == 2 ? DFL_WHOLE_PICK(Q4W, 2) : DFL_WHOLE_PICK(Q4W, 1))
                         : q6_tiled           ? (p.R == 2 ? DFL_WHOLE_PICK(Q6T, 2) : DFL_WHOLE_PICK(Q6T, 1))
                                              : (p.R == 2 ? DFL_WHOLE_PICK(Q6W, 2) : DFL_WHOLE_PICK(Q6W, 1));
@@ -1057,7 +1089,7 @@ int32_t dfl_gemm_whole_blocks(dflash_ctx *ctx, int32_t w_type, const void *w, co
     if (lds > 48 * 1024)
         if (const int32_t rc = dfl_raise_lds_limit(ctx, reinterpret_cast<const void *>(fn), lds)) return rc;
     dfl_timed timer(ctx, st, DFL_T_GEMM);
-    fn<<<p.n_wg, threads, lds, st>>>(a);
+    whole_launch(fn, p.n_wg, threads, lds, st, a);
     DFL_HIP_CHECK(ctx, hipGetLastError());
     return DFLASH_OK;
 }
@@ -1109,10 +1141,10 @@ WidePlan rows_wide_plan(const dflash_ctx *ctx, int32_t w_type, int64_t n_in, int
     return p;
 }
 template <typename W, typename XT>
-const void *rows_direct_fn(int R) {
+whole_kernel_t rows_direct_fn(int R) {
     if constexpr (!std::is_same<W, Q6W>::value)
-        if (R == 2) return reinterpret_cast<const void *>(gemm_whole_kernel<W, 2, 0, RowSrc<XT>>);
-    return reinterpret_cast<const void *>(gemm_whole_kernel<W, 1, 0, RowSrc<XT>>);
+        if (R == 2) return gemm_whole_kernel<W, 2, 0, RowSrc<XT>>;
+    return gemm_whole_kernel<W, 1, 0, RowSrc<XT>>;
 }
 }  // namespace
 
@@ -1150,29 +1182,29 @@ int32_t dfl_gemm_direct(dflash_ctx *ctx, int32_t w_type, const void *w, const vo
         const bool tiled = w_type == DFLASH_TYPE_Q4_K_TILED;
         const size_t wlds = static_cast<size_t>(2) * waves * 64 * sizeof(float4_t) + static_cast<size_t>(waves) * wp.slots * kWideSlot;
         const bool two = a.nb > 16;
-#define DFL_WIDE_PICK(XT, LEN, SLOTS) (tiled ? (kernel_t)gemm_q4k_wide_kernel<XT, true, LEN, SLOTS> : (kernel_t)gemm_q4k_wide_kernel<XT, false, LEN, SLOTS>)
+#define DFL_WIDE_PICK(XT, LEN, SLOTS) (tiled ? gemm_q4k_wide_kernel<XT, true, LEN, SLOTS> : gemm_q4k_wide_kernel<XT, false, LEN, SLOTS>)
 #define DFL_WIDE_PICK4(XT) (two ? (wp.slots == 6 ? DFL_WIDE_PICK(XT, 2, 6) : DFL_WIDE_PICK(XT, 2, 5)) \
                                 : (wp.slots == 6 ? DFL_WIDE_PICK(XT, 1, 6) : wp.slots == 4 ? DFL_WIDE_PICK(XT, 1, 4) : DFL_WIDE_PICK(XT, 1, 3)))
-        typedef void (*kernel_t)(WholeArgs);
-        const void *wfn = reinterpret_cast<const void *>(f32 ? DFL_WIDE_PICK4(float) : DFL_WIDE_PICK4(_Float16));
+        const whole_kernel_t wfn = f32 ? DFL_WIDE_PICK4(float) : DFL_WIDE_PICK4(_Float16);
 #undef DFL_WIDE_PICK4
 #undef DFL_WIDE_PICK
-        if (const int32_t rc = dfl_raise_lds_limit(ctx, wfn, wlds)) return rc;
+        if (const int32_t rc = dfl_raise_lds_limit(ctx, reinterpret_cast<const void *>(wfn), wlds)) return rc;
         dfl_timed timer(ctx, st, DFL_T_GEMM);
         const dfl_stamp sp(ctx, DFL_T_KERNEL_Q4K_TILED);
-        void *wargs[] = {&a};
-        DFL_HIP_CHECK(ctx, hipExtLaunchKernel(wfn, dim3(wp.n_wg), dim3(64 * waves), wargs, wlds, st, sp.start, sp.stop, 0));
+        a.pair_off = wp.n_wg;
+        whole_launch(wfn, wp.n_wg, 64 * waves, wlds, st, a, sp.start, sp.stop);
+        DFL_HIP_CHECK(ctx, hipGetLastError());
         return DFLASH_OK;
     }
     const size_t lds = static_cast<size_t>(16) * p.R * 64 * sizeof(float4_t) + static_cast<size_t>(p.ksplit) * p.tl * kRowAreaBytes;
-    const void *fn = q6 ? (f32 ? rows_direct_fn<Q6W, float>(p.R) : rows_direct_fn<Q6W, _Float16>(p.R))
+    const whole_kernel_t fn = q6 ? (f32 ? rows_direct_fn<Q6W, float>(p.R) : rows_direct_fn<Q6W, _Float16>(p.R))
                      : w_type == DFLASH_TYPE_Q4_K_TILED ? (f32 ? rows_direct_fn<Q4W, float>(p.R) : rows_direct_fn<Q4W, _Float16>(p.R))
                                                         : (f32 ? rows_direct_fn<Q4R, float>(p.R) : rows_direct_fn<Q4R, _Float16>(p.R));
     if (lds > 48 * 1024)
-        if (const int32_t rc = dfl_raise_lds_limit(ctx, fn, lds)) return rc;
+        if (const int32_t rc = dfl_raise_lds_limit(ctx, reinterpret_cast<const void *>(fn), lds)) return rc;
     dfl_timed timer(ctx, st, DFL_T_GEMM);
-    void *args[] = {&a};
-    DFL_HIP_CHECK(ctx, hipLaunchKernel(fn, dim3(p.n_wg), dim3(64 * p.ksplit * p.tl), args, lds, st));
+    whole_launch(fn, p.n_wg, 64 * p.ksplit * p.tl, lds, st, a);
+    DFL_HIP_CHECK(ctx, hipGetLastError());
     return DFLASH_OK;
 }
 
