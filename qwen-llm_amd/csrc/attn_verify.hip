@@ -185,18 +185,15 @@ __device__ __forceinline__ void attn_store_xf(float4_t (&tot)[DT], void *out_xf,
 template <int HD, typename TQ, int MAXW, int MAXL, bool MERGE>
 __device__ __forceinline__ void attn_body(const TQ *__restrict__ q, const _Float16 *__restrict__ k_cache,
                                           const _Float16 *__restrict__ vt_cache, float *__restrict__ part_o, float *__restrict__ part_ml,
-                                          int64_t ctx_len, const int32_t *__restrict__ ctx_len_dev, int n_rows_total, int n_q, int n_kv,
+                                          int64_t ctx_len, const int32_t *__restrict__ ctx_len_dev, int n_rows_total, int n_kv, int group, int n_waves,
                                           int64_t vt_stride, int want, int min_chunk, float scale, int full_block, int64_t window,
                                           int split_stride, int64_t part_slots, int block, float *__restrict__ out, void *__restrict__ out_xf,
                                           int out_xf_kind, size_t xf_stride) {
+    const int n_q = n_kv * group;
     // block: which block of sixteen query rows (a prefill group hands over many: block b's rows follow block
     // b - 1's in q and in the cache, its partial tiles sit part_slots slots further on)
     const int n_rows = min(16, n_rows_total - 16 * block);
     q += static_cast<int64_t>(block) * 16 * n_q * HD;
-    if constexpr (!MERGE) {
-        part_o += static_cast<int64_t>(block) * part_slots * HD;
-        part_ml += static_cast<int64_t>(block) * part_slots * 2;
-    }
     constexpr int KS = HD / 32;       // k-steps of the score product
     constexpr int DT = HD / 16;       // 16-dim tiles of the output
     constexpr int CH = HD / 8;        // 16-byte chunks per key row
@@ -206,9 +203,7 @@ __device__ __forceinline__ void attn_body(const TQ *__restrict__ q, const _Float
     extern __shared__ half8_t lds[];  // kAttnBufs x (K tile, V^T tile)
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int n_waves = blockDim.x >> 6;
     const int n = lane & 15, g = lane >> 4;
-    const int group = n_q / n_kv;
     const int kvh = blockIdx.y;
     // blockIdx.x = split + split_stride * (part of the GQA group this workgroup serves); split_stride is a multiple
     // of 8, so the workgroups that read one chunk of keys are dispatched to the same XCD and share its L2 copy
@@ -219,10 +214,10 @@ __device__ __forceinline__ void attn_body(const TQ *__restrict__ q, const _Float
     AttnQ8<TQ> q_raw[KS];
     const TQ *qrow = q + (static_cast<int64_t>(min(n, n_rows - 1)) * n_q + head) * HD + 8 * g;
     attn_load_q<0, KS>(q_raw, qrow);
-    if (ctx_len_dev) ctx_len = *ctx_len_dev;
+    if (ctx_len < 0) ctx_len = *ctx_len_dev;
     ctx_len += 16 * static_cast<int64_t>(block);
     const int64_t n_pos = ctx_len + n_rows;
-    const int64_t chunk = attn_chunk(n_pos, want, min_chunk);
+    const int64_t chunk = want ? attn_chunk(n_pos, want, min_chunk) : min_chunk;
     if (!MERGE && split * chunk >= n_pos) return;  // the grid is sized for the longest context
     const int64_t c0 = MERGE ? 0 : split * chunk;
     const int64_t c1 = MERGE ? n_pos : min(n_pos, c0 + chunk);
@@ -275,6 +270,13 @@ __device__ __forceinline__ void attn_body(const TQ *__restrict__ q, const _Float
 #pragma unroll
     for (int st = 0; st < kAttnBufs - 1; st++)
         if (issued < n_steps) issue_stage();
+    if constexpr (!MERGE) {
+        dfl_have(scale, full_block, window, part_o, part_ml);
+        if (block) {
+            part_o += static_cast<int64_t>(block) * part_slots * HD;
+            part_ml += static_cast<int64_t>(block) * part_slots * 2;
+        }
+    }
 
     ATT_TR(1);
     half8_t qf[KS];  // Q^T, times scale * log2(e)
@@ -465,13 +467,15 @@ __device__ __forceinline__ void attn_body(const TQ *__restrict__ q, const _Float
 
 template <int HD, typename TQ, int MAXW, int MAXL>
 __global__ void __launch_bounds__(64 * MAXW)
-    attn_split_kernel(const TQ *__restrict__ q, const _Float16 *__restrict__ k_cache,
-                      const _Float16 *__restrict__ vt_cache, float *__restrict__ part_o, float *__restrict__ part_ml,
-                      int64_t ctx_len, const int32_t *__restrict__ ctx_len_dev, int n_rows_total, int n_q, int n_kv,
-                      int64_t vt_stride, int want, int min_chunk, float scale, int full_block, int64_t window,
-                      int split_stride, int64_t part_slots) {
-    attn_body<HD, TQ, MAXW, MAXL, false>(q, k_cache, vt_cache, part_o, part_ml, ctx_len, ctx_len_dev, n_rows_total, n_q, n_kv, vt_stride, want,
-                                         min_chunk, scale, full_block, window, split_stride, part_slots, blockIdx.z, nullptr, nullptr, 0, 0);
+    attn_split_kernel(const TQ *__restrict__ q, const _Float16 *__restrict__ k_cache, const _Float16 *__restrict__ vt_cache, int64_t ctx_len,
+                      int64_t vt_stride, uint32_t heads, uint32_t split_waves, int n_rows_total, int min_chunk, int want, float scale,
+                      float *__restrict__ part_o, float *__restrict__ part_ml, int full_block, int64_t window, int64_t part_slots,
+                      const int32_t *__restrict__ ctx_len_dev) {
+    // The arguments in the order of their use: the first fourteen words, which the first loads need, come preloaded with the wave.
+    // heads = KV heads | group << 20, split_waves = split_stride | waves << 24; ctx_len < 0: it is in device memory; want == 0: min_chunk is the chunk.
+    attn_body<HD, TQ, MAXW, MAXL, false>(q, k_cache, vt_cache, part_o, part_ml, ctx_len, ctx_len_dev, n_rows_total, heads & 0xfffff, heads >> 20,
+                                         split_waves >> 24, vt_stride, want, min_chunk, scale, full_block, window, split_waves & 0xffffff, part_slots,
+                                         blockIdx.z, nullptr, nullptr, 0, 0);
 }
 
 // Many blocks of rows at once, a prompt's prefill: the blocks are enough workgroups, so one takes all of its block's keys
@@ -496,7 +500,7 @@ __global__ void __launch_bounds__(512)
         want = runs.want[r];
         min_chunk = runs.min_chunk[r];
     }
-    attn_body<HD, float, 8, MAXL, true>(q, k_cache, vt_cache, nullptr, nullptr, ctx_len, nullptr, n_rows_total, n_q, n_kv, vt_stride, want, min_chunk,
+    attn_body<HD, float, 8, MAXL, true>(q, k_cache, vt_cache, nullptr, nullptr, ctx_len, nullptr, n_rows_total, n_kv, n_q / n_kv, blockDim.x >> 6, vt_stride, want, min_chunk,
                                         scale, 0, 0, 1, 0, block, out, out_xf, out_xf_kind, xf_stride);
 }
 
@@ -896,9 +900,10 @@ __global__ void __launch_bounds__(256)
 // A wave's 64 lanes cover 64 / (HD / 4) split lanes, four dims per lane.
 template <int HD>
 __global__ void __launch_bounds__(HD == 64 ? 128 : 256)
-    attn_combine_few_kernel(const float *__restrict__ part_o, const float *__restrict__ part_ml, float *__restrict__ out, int n_rows_total,
-                            int n_q, int64_t ctx_len, const int32_t *__restrict__ ctx_len_dev, int want, int min_chunk,
-                            void *__restrict__ out_xf, int out_xf_kind, int64_t part_slots, size_t xf_stride, int max_splits) {
+    attn_combine_few_kernel(const float *__restrict__ part_o, const float *__restrict__ part_ml, int64_t ctx_len, int n_q, int n_rows_total, int max_splits,
+                            int min_chunk, int want, float *__restrict__ out, void *__restrict__ out_xf, int out_xf_kind, int64_t part_slots,
+                            size_t xf_stride, const int32_t *__restrict__ ctx_len_dev) {
+    // (the arguments in the order of their use and with attn_split_kernel's conventions, but want == 0: min_chunk is the number of splits)
     constexpr int kLanes = HD / 4, kPerWave = 64 / kLanes, kWaves = HD == 64 ? 2 : 4, kSteps = 8 / (kPerWave * kWaves);
     const int n_rows = min(16, n_rows_total - 16 * static_cast<int>(blockIdx.z));
     if (static_cast<int>(blockIdx.y) >= n_rows) return;
@@ -906,8 +911,9 @@ __global__ void __launch_bounds__(HD == 64 ? 128 : 256)
     __shared__ __attribute__((aligned(16))) float red[8][HD + 4];
     __shared__ float red_l[8];
     const int64_t slot_stride = static_cast<int64_t>(n_q) * 16;
-    const float2 *ml = reinterpret_cast<const float2 *>(part_ml) + static_cast<int64_t>(blockIdx.z) * part_slots + head * 16 + row;
-    const float *po = part_o + (static_cast<int64_t>(blockIdx.z) * part_slots + head * 16 + row) * HD + 4 * (lane % kLanes);
+    const int64_t slot0 = (blockIdx.z ? static_cast<int64_t>(blockIdx.z) * part_slots : 0) + head * 16 + row;
+    const float2 *ml = reinterpret_cast<const float2 *>(part_ml) + slot0;
+    const float *po = part_o + slot0 * HD + 4 * (lane % kLanes);
     const float2 own = ml[min(lane, max_splits - 1) * slot_stride];
     float4_t o[kSteps][6];
 #pragma unroll
@@ -918,8 +924,9 @@ __global__ void __launch_bounds__(HD == 64 ? 128 : 256)
             const int s = min(wave * kPerWave + lane / kLanes + j * kPerWave * kWaves + 8 * i, max_splits - 1);
             o[j][i] = *reinterpret_cast<const float4_t *>(po + s * slot_stride * HD);
         }
-    if (ctx_len_dev) ctx_len = *ctx_len_dev;
-    const int n_splits = attn_splits(ctx_len + 16 * static_cast<int64_t>(blockIdx.z) + n_rows, want, min_chunk);
+    dfl_have(out, out_xf, out_xf_kind, xf_stride);
+    if (ctx_len < 0) ctx_len = *ctx_len_dev;
+    const int n_splits = want ? attn_splits(ctx_len + 16 * static_cast<int64_t>(blockIdx.z) + n_rows, want, min_chunk) : min_chunk;
     float m_star = lane < n_splits ? own.x : -INFINITY;
     const float m_own = m_star;
     m_star = dfl_wave_max(m_star);
@@ -966,15 +973,17 @@ __global__ void __launch_bounds__(HD == 64 ? 128 : 256)
 constexpr int kOrderedSplits = 32;
 template <int HD>
 __global__ void __launch_bounds__(HD)
-    attn_combine_ordered_kernel(const float *__restrict__ part_o, const float *__restrict__ part_ml, float *__restrict__ out, int n_rows_total,
-                            int n_q, int64_t ctx_len, const int32_t *__restrict__ ctx_len_dev, int want, int min_chunk,
-                            void *__restrict__ out_xf, int out_xf_kind, int64_t part_slots, size_t xf_stride, int max_splits) {
+    attn_combine_ordered_kernel(const float *__restrict__ part_o, const float *__restrict__ part_ml, int64_t ctx_len, int n_q, int n_rows_total,
+                                int max_splits, int min_chunk, int want, float *__restrict__ out, void *__restrict__ out_xf, int out_xf_kind,
+                                int64_t part_slots, size_t xf_stride, const int32_t *__restrict__ ctx_len_dev) {
+    // (the arguments as attn_combine_few_kernel's)
     const int n_rows = min(16, n_rows_total - 16 * static_cast<int>(blockIdx.z));
     if (static_cast<int>(blockIdx.y) >= n_rows) return;
     const int head = blockIdx.x, row = blockIdx.y, d = threadIdx.x, lane = d & 63;
     const int64_t slot_stride = static_cast<int64_t>(n_q) * 16;
-    const float2 *ml = reinterpret_cast<const float2 *>(part_ml) + static_cast<int64_t>(blockIdx.z) * part_slots + head * 16 + row;
-    const float *po = part_o + (static_cast<int64_t>(blockIdx.z) * part_slots + head * 16 + row) * HD + d;
+    const int64_t slot0 = (blockIdx.z ? static_cast<int64_t>(blockIdx.z) * part_slots : 0) + head * 16 + row;
+    const float2 *ml = reinterpret_cast<const float2 *>(part_ml) + slot0;
+    const float *po = part_o + slot0 * HD + d;
     const float2 own = ml[min(lane, max_splits - 1) * slot_stride];
     float o[kOrderedSplits];
 #pragma unroll
@@ -982,8 +991,9 @@ __global__ void __launch_bounds__(HD)
         if ((s & ~7) >= max_splits) continue;  // (uniform; past the last split it is read again)
         o[s] = po[min(s, max_splits - 1) * slot_stride * HD];
     }
-    if (ctx_len_dev) ctx_len = *ctx_len_dev;
-    const int n_splits = attn_splits(ctx_len + 16 * static_cast<int64_t>(blockIdx.z) + n_rows, want, min_chunk);
+    dfl_have(out, out_xf, out_xf_kind, xf_stride);
+    if (ctx_len < 0) ctx_len = *ctx_len_dev;
+    const int n_splits = want ? attn_splits(ctx_len + 16 * static_cast<int64_t>(blockIdx.z) + n_rows, want, min_chunk) : min_chunk;
     const float m = lane < n_splits ? own.x : -INFINITY;
     const int none = __builtin_bit_cast(int, -INFINITY);
     float upto = m;
@@ -1046,14 +1056,21 @@ int32_t launch_split(dflash_ctx *ctx, dim3 grid, int threads, hipStream_t st, co
     const size_t lds = static_cast<size_t>(kAttnBufs) * 2 * (32 * HD / 8) * sizeof(half8_t);
     constexpr int kWaveLoads = 2 * 32 * (HD / 8) / 64;
     const int n_waves = threads / 64, per_wave = (kWaveLoads + n_waves - 1) / n_waves;
+    const uint32_t heads = static_cast<uint32_t>(n_kv) | static_cast<uint32_t>(n_q / n_kv) << 20;  // (a group is at most 16)
+    const uint32_t split_waves = static_cast<uint32_t>(split_stride) | static_cast<uint32_t>(n_waves) << 24;
+    // a single block whose context length is known here: its chunk is, too
+    const int64_t chunk = attn_chunk(ctx_len + n_rows, want, min_chunk);
+    if (n_rows <= 16 && !ctx_len_dev && chunk <= 0x7fffffff) {
+        want = 0;
+        min_chunk = static_cast<int>(chunk);
+    }
 #define DFL_ATTN_LAUNCH(MAXW, MAXL)                                                                                 \
     do {                                                                                                            \
         if (const int32_t rc_ = dfl_raise_lds_limit(ctx, reinterpret_cast<const void *>(attn_split_kernel<HD, TQ, MAXW, MAXL>), lds)) \
             return rc_;                                                                                             \
-        attn_split_kernel<HD, TQ, MAXW, MAXL><<<grid, threads, lds, st>>>(static_cast<const TQ *>(q), k, vt, po, pml, \
-                                                                         ctx_len, ctx_len_dev, n_rows, n_q, n_kv, \
-                                                                         vt_stride, want, min_chunk, scale,    \
-                                                                         full_block, window, split_stride, part_slots); \
+        attn_split_kernel<HD, TQ, MAXW, MAXL><<<grid, threads, lds, st>>>(static_cast<const TQ *>(q), k, vt, ctx_len_dev ? -1 : ctx_len, vt_stride, \
+                                                                         heads, split_waves, n_rows, min_chunk, want, scale, po, pml, \
+                                                                         full_block, window, part_slots, ctx_len_dev); \
     } while (0)
     // one head per wave: two halve the LDS reads per head but measured slower on MI355X
     // (fewer waves to hide the per-stage dependency chain)
@@ -1408,20 +1425,22 @@ static int32_t attn_rows(dflash_ctx *ctx, const void *q, int32_t q_type, const v
 #undef DFL_ATTN
     }
     if (rc) return rc;
+    const bool known = n_blocks == 1 && !ctx_len_dev;  // (the number of splits: the one block's)
     if (policy.ordered) {
         const auto fn = head_dim == 64 ? attn_combine_ordered_kernel<64> : attn_combine_ordered_kernel<128>;
-        fn<<<dim3(n_q, n_rows, n_blocks), head_dim, 0, st>>>(part_o, part_ml, out, n_rows_total, n_q, ctx_len, ctx_len_dev, want,
-                                                            static_cast<int>(min_chunk), out_xf, out_xf_kind, part_slots,
-                                                            dfl_xf_bytes(static_cast<int64_t>(n_q) * head_dim), n_splits);
+        fn<<<dim3(n_q, n_rows, n_blocks), head_dim, 0, st>>>(part_o, part_ml, ctx_len_dev ? -1 : ctx_len, n_q, n_rows_total, n_splits, known ? n_splits : static_cast<int>(min_chunk),
+                                                            known ? 0 : want, out, out_xf, out_xf_kind, part_slots,
+                                                            dfl_xf_bytes(static_cast<int64_t>(n_q) * head_dim), ctx_len_dev);
         DFL_HIP_CHECK(ctx, hipGetLastError());
         return DFLASH_OK;
     }
     // (more splits than that and the shuffles of the weights cost more than the barriers they replace)
     if (n_splits <= 48) {
         const auto fn = head_dim == 64 ? attn_combine_few_kernel<64> : head_dim == 128 ? attn_combine_few_kernel<128> : attn_combine_few_kernel<256>;
-        fn<<<dim3(n_q, n_rows, n_blocks), head_dim == 64 ? 128 : 256, 0, st>>>(part_o, part_ml, out, n_rows_total, n_q, ctx_len, ctx_len_dev, want,
-                                                                              static_cast<int>(min_chunk), out_xf, out_xf_kind, part_slots,
-                                                                              dfl_xf_bytes(static_cast<int64_t>(n_q) * head_dim), n_splits);
+        fn<<<dim3(n_q, n_rows, n_blocks), head_dim == 64 ? 128 : 256, 0, st>>>(part_o, part_ml, ctx_len_dev ? -1 : ctx_len, n_q, n_rows_total, n_splits,
+                                                                              known ? n_splits : static_cast<int>(min_chunk), known ? 0 : want, out, out_xf,
+                                                                              out_xf_kind, part_slots, dfl_xf_bytes(static_cast<int64_t>(n_q) * head_dim),
+                                                                              ctx_len_dev);
         DFL_HIP_CHECK(ctx, hipGetLastError());
         return DFLASH_OK;
     }

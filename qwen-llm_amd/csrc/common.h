@@ -169,6 +169,16 @@ __device__ static inline void dfl_xf_store(void *xf, int kind, int m, int k0, fl
                      static_cast<_Float16>(v4), static_cast<_Float16>(v6), static_cast<_Float16>(v5), static_cast<_Float16>(v7)};
     *reinterpret_cast<h8 *>(static_cast<uint8_t *>(xf) + dfl_xf_slot(kind, m, k0)) = frag;
 }
+// A kernel's arguments beyond the first fourteen words are loaded where they are first used, 0.3 us of a wave that waits for
+// nothing else at that place.  This asks for them here, behind a kernel's first loads, under which they arrive.
+template <typename T>
+__device__ static __forceinline__ void dfl_have_one(T v) {
+    asm volatile("" ::"s"(v));
+}
+template <typename... T>
+__device__ static __forceinline__ void dfl_have(T... v) {
+    (dfl_have_one(v), ...);
+}
 // Reductions over a wave without LDS (a shuffle is a trip through it, and six in a row stand in the middle of most small
 // kernels): the lane 32 or 16 away by v_permlane32/16_swap, the nearer ones by DPP moves.  The tree is that of
 // `for (off = 32; off; off >>= 1) v += __shfl_xor(v, off)`, lane for lane, so a sum has that loop's bits.

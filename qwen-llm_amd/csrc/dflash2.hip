@@ -17,23 +17,28 @@ namespace {
 // y[t][c] = sum_tap (base[side][tap][c] + dyn[t][side][tap][c / group_size]) * x[t - tap][c]; rows
 // before the block count as zeros; taps accumulate in order with a fused multiply-add, as the
 // reference kernel does.  One thread per element.
+// What bounds it: one trip to memory.  So the index arithmetic has no divisions (by_group: ceil(2^32 / group_size), or 0 where that
+// is not exact for every channel), two taps' values travel together, and what the first loads need comes preloaded with the wave.
 __global__ void __launch_bounds__(256)
-    dflash2_conv_kernel(const float *__restrict__ x, const float *__restrict__ dyn, const float *__restrict__ base,
-                        float *__restrict__ y, int n_tokens, int h, int kernel_size, int group_size, int side,
-                        void *__restrict__ y_xf, int y_xf_kind) {
-    const int64_t gid = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (gid >= static_cast<int64_t>(n_tokens) * h) return;
-    const int t = static_cast<int>(gid / h), c = static_cast<int>(gid % h);
-    const int n_groups = h / group_size, g = c / group_size;
-    const size_t dyn_row = static_cast<size_t>(t) * 2 * kernel_size * n_groups + static_cast<size_t>(side) * kernel_size * n_groups;
-    const size_t base_side = static_cast<size_t>(side) * kernel_size * h;
+    dflash2_conv_kernel(const float *__restrict__ x, const float *__restrict__ dyn, const float *__restrict__ base, int h, int kernel_size,
+                        int n_groups, uint32_t by_group, int side, int group_size, float *__restrict__ y, void *__restrict__ y_xf, int y_xf_kind) {
+    const int t = blockIdx.x, c = blockIdx.y * 256 + threadIdx.x;
+    if (c >= h) return;
+    const int g = by_group ? static_cast<int>(__umulhi(c, by_group)) : c / group_size;
+    const float *dyn_t = dyn + (static_cast<size_t>(t) * 2 + side) * kernel_size * n_groups + g;
+    const float *base_c = base + static_cast<size_t>(side) * kernel_size * h + c, *x_c = x + c;
     float acc = 0.0f;
-    for (int tap = 0; tap < kernel_size && tap <= t; tap++) {
-        const float b = base[base_side + static_cast<size_t>(tap) * h + c];
-        const float d = dyn[dyn_row + static_cast<size_t>(tap) * n_groups + g];
-        acc = __builtin_fmaf(b + d, x[static_cast<size_t>(t - tap) * h + c], acc);
+    for (int tap = 0; tap < kernel_size && tap <= t; tap += 2) {
+        const bool two = tap + 1 < kernel_size && tap + 1 <= t;
+        const int tp = two ? tap + 1 : tap;
+        const float b0 = base_c[static_cast<size_t>(tap) * h], b1 = base_c[static_cast<size_t>(tp) * h];
+        const float d0 = dyn_t[static_cast<size_t>(tap) * n_groups], d1 = dyn_t[static_cast<size_t>(tp) * n_groups];
+        const float x0 = x_c[static_cast<size_t>(t - tap) * h], x1 = x_c[static_cast<size_t>(t - tp) * h];
+        if (tap == 0) dfl_have(y, y_xf, y_xf_kind);
+        acc = __builtin_fmaf(b0 + d0, x0, acc);
+        if (two) acc = __builtin_fmaf(b1 + d1, x1, acc);
     }
-    y[gid] = acc;
+    y[static_cast<size_t>(t) * h + c] = acc;
     if (y_xf) {
         // (h a multiple of 256: the grid has no ragged end and eight consecutive lanes hold eight consecutive channels of a row)
         float v[8];
@@ -342,9 +347,11 @@ int32_t dfl_dflash2_conv(dflash_ctx *ctx, const float *x, const float *dyn, cons
     const size_t bytes = static_cast<size_t>(n_tokens) * h * sizeof(float);
     if (dfl_ranges_overlap(y, bytes, x, bytes))
         return dfl_fail(ctx, DFLASH_ERR_ALIAS, "dflash2_conv: y aliases x (taps read neighbouring rows)");
-    const int64_t total = static_cast<int64_t>(n_tokens) * h;
-    dflash2_conv_kernel<<<static_cast<unsigned>((total + 255) / 256), 256, 0, static_cast<hipStream_t>(stream)>>>(
-        x, dyn, base, y, n_tokens, h, kernel_size, group_size, side, y_xf, y_xf_kind);
+    // c * ceil(2^32 / g) >> 32 is c / g while c * g stays below 2^32
+    const uint32_t by_group = group_size > 1 && static_cast<int64_t>(h) * group_size < (1ll << 32)
+                                  ? static_cast<uint32_t>(((1ull << 32) + group_size - 1) / group_size) : 0;
+    dflash2_conv_kernel<<<dim3(n_tokens, (h + 255) / 256), 256, 0, static_cast<hipStream_t>(stream)>>>(
+        x, dyn, base, h, kernel_size, h / group_size, by_group, side, group_size, y, y_xf, y_xf_kind);
     DFL_HIP_CHECK(ctx, hipGetLastError());
     return DFLASH_OK;
 }

@@ -2337,9 +2337,8 @@ __global__ void __launch_bounds__(64 * kMaxSplit)
 // chunk: hidden <= 2048.
 __global__ void __launch_bounds__(64 * kMaxSplit)
     q8_0_norm_router_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x, const float *__restrict__ add,
-                            const float *__restrict__ norm_w, const float *__restrict__ gate_w, float eps,
-                            float *__restrict__ cur, float *__restrict__ gate_out, float *__restrict__ y, int n_out,
-                            int n_steps, size_t row_bytes) {
+                            const float *__restrict__ norm_w, const float *__restrict__ gate_w, int n_out, int n_steps, float eps,
+                            float *__restrict__ cur, float *__restrict__ gate_out, float *__restrict__ y) {
     typedef float f4 __attribute__((ext_vector_type(4)));
     typedef _Float16 h4 __attribute__((ext_vector_type(4)));
     __shared__ half8_t xrow[4 * kQ8ChunkSteps];                              // [step][k-group]: the normalised row
@@ -2370,10 +2369,11 @@ __global__ void __launch_bounds__(64 * kMaxSplit)
     constexpr int kSteps = kQ8ChunkSteps / kMaxSplit;
     Raw8<DFLASH_TYPE_Q8_0> rw[kSteps];
     {
-        const uint8_t *wrow = w + static_cast<size_t>(min(n0 + n, n_out - 1)) * row_bytes;
+        const uint8_t *wrow = w + static_cast<size_t>(min(n0 + n, n_out - 1)) * (n_steps * DFL_Q8_0_BYTES);
 #pragma unroll
         for (int i = 0; i < kSteps; i++) rw[i] = load_raw8<DFLASH_TYPE_Q8_0>(wrow, static_cast<int64_t>(min(s0 + i, n_steps - 1)) * 32 + 8 * g);
     }
+    dfl_have(cur, gate_out, y);
     if (norm_wave) {
         float s = 0.0f;
 #pragma unroll
@@ -2922,9 +2922,8 @@ int32_t dfl_router_norm(dflash_ctx *ctx, const void *router_w, const float *x, c
     const int n_steps = static_cast<int>(hidden / DFL_QK8_0);
     const int tiles = (n_expert + 15) / 16;
     dfl_timed timer(ctx, st, DFL_T_GEMM);
-    q8_0_norm_router_kernel<<<dim3(tiles, n_rows), 64 * kMaxSplit, 0, st>>>(static_cast<const uint8_t *>(router_w), x, add, norm_w, gate_w, eps, cur,
-                                                                 gate_out, logits, n_expert, n_steps,
-                                                                 static_cast<size_t>(n_steps) * DFL_Q8_0_BYTES);
+    q8_0_norm_router_kernel<<<dim3(tiles, n_rows), 64 * kMaxSplit, 0, st>>>(static_cast<const uint8_t *>(router_w), x, add, norm_w, gate_w, n_expert,
+                                                                 n_steps, eps, cur, gate_out, logits);
     DFL_HIP_CHECK(ctx, hipGetLastError());
     return DFLASH_OK;
 }

@@ -58,7 +58,7 @@ struct WholeArgs {
 // As kernel parameters: what a wave needs for its first loads as words of their own, fourteen at most, which arrive in its
 // scalar registers (a parameter that is a structure has to be loaded, a trip of 0.5 us to memory the host has just written,
 // and a division by ksplit is some forty instructions, ahead of the first weight); the rest behind them.
-// TAILNEW
+// (a step of 40 layers, 80 such launches: 2689 -> 2664 us)
 struct WholeTail {
     uint8_t *y_xf;
     int y_xf_kind, n_blocks, rows_last;

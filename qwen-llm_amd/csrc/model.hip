@@ -65,12 +65,13 @@ bool norm_in_registers(int n) { return n >= 4 && n <= 8192 && n % 4 == 0; }
 // per launch inside a verify's graph for sixteen rows of 5120.  The sums keep one order whatever V: a thread's vectors in
 // turn, the lanes of a wave, the four waves.
 typedef float norm_f4 __attribute__((ext_vector_type(4)));
+// (The arguments in the order of their use: what the row's loads need comes preloaded with the wave.)
 template <int V, bool kConv>
-__global__ void __launch_bounds__(256) rms_norm_kernel(float *__restrict__ x, const float *__restrict__ add,
-                                                       const float *__restrict__ w, float *__restrict__ y, int n,
-                                                       float eps, const float *__restrict__ gate_w,
-                                                       float *__restrict__ gate_out, void *__restrict__ y_xf,
-                                                       int y_xf_kind, size_t xf_stride, ConvResid conv, void *__restrict__ y_xs) {
+__global__ void __launch_bounds__(256) rms_norm_kernel(float *__restrict__ x, const float *__restrict__ add, const float *__restrict__ w, int n,
+                                                       int conv_ks, const float *__restrict__ conv_dyn, const float *__restrict__ conv_base,
+                                                       int conv_groups, uint32_t by_group, float *__restrict__ y, float eps,
+                                                       const float *__restrict__ gate_w, float *__restrict__ gate_out, void *__restrict__ y_xf,
+                                                       int y_xf_kind, size_t xf_stride, void *__restrict__ y_xs) {
     typedef norm_f4 f4;
     __shared__ float sh[4], sh_dot[4];
     const int t = blockIdx.x, tid = threadIdx.x;
@@ -86,14 +87,14 @@ __global__ void __launch_bounds__(256) rms_norm_kernel(float *__restrict__ x, co
     if constexpr (kConv) {
         // the residual term is the convolution: taps in order, fused multiply-adds (the host takes this path for
         // group sizes that are multiples of four: one coefficient per vector and tap)
-        const int ks = conv.kernel_size, n_groups = n / conv.group_size;
-        const float *dyn_t = conv.dyn + (static_cast<size_t>(t) * 2 + 1) * ks * n_groups;
-        const float *base1 = conv.base + static_cast<size_t>(ks) * n;
+        const int ks = conv_ks, n_groups = conv_groups;
+        const float *dyn_t = conv_dyn + (static_cast<size_t>(t) * 2 + 1) * ks * n_groups;
+        const float *base1 = conv_base + static_cast<size_t>(ks) * n;
         int grp[V];
 #pragma unroll
         for (int j = 0; j < V; j++) {
             a[j] = f4{0, 0, 0, 0};
-            grp[j] = at[j] / conv.group_size;
+            grp[j] = static_cast<int>(__umulhi(at[j], by_group));  // at[j] / group_size
         }
         for (int tap = 0; tap < ks && tap <= t; tap += 2) {
             const bool two = tap + 1 < ks && tap + 1 <= t;  // (two taps' loads in flight together)
@@ -128,6 +129,7 @@ __global__ void __launch_bounds__(256) rms_norm_kernel(float *__restrict__ x, co
 #pragma unroll
         for (int j = 0; j < V; j++) gw[j] = *reinterpret_cast<const f4 *>(gate_w + at[j]);
     }
+    dfl_have(y, eps, gate_out, y_xf, y_xf_kind, xf_stride, y_xs);
     float s = 0.0f;
 #pragma unroll
     for (int j = 0; j < V; j++) {
@@ -231,12 +233,14 @@ void rms_norm(int rows, hipStream_t st, float *x, const float *add, const float 
         rms_norm_any_kernel<<<rows, 256, 0, st>>>(x, add, w, y, n, eps, gate_w, gate_out);
         return;
     }
+    // (ceil(2^32 / group_size): exact quotients for the values of a row of at most 8192; groups of four or more)
+    const uint32_t by_group = conv.group_size > 1 ? static_cast<uint32_t>(((1ull << 32) + conv.group_size - 1) / conv.group_size) : 0;
+    const int groups = n / std::max(conv.group_size, 1);
 #define DFL_NORM(V)                                                                                                          \
     do {                                                                                                                     \
-        if (conv.dyn && add)                                                                                                 \
-            rms_norm_kernel<V, true><<<rows, 256, 0, st>>>(x, add, w, y, n, eps, gate_w, gate_out, y_xf, y_xf_kind, xf_stride, conv, y_xs); \
-        else                                                                                                                 \
-            rms_norm_kernel<V, false><<<rows, 256, 0, st>>>(x, add, w, y, n, eps, gate_w, gate_out, y_xf, y_xf_kind, xf_stride, conv, y_xs); \
+        const auto fn = conv.dyn && add ? rms_norm_kernel<V, true> : rms_norm_kernel<V, false>;                              \
+        fn<<<rows, 256, 0, st>>>(x, add, w, n, conv.kernel_size, conv.dyn, conv.base, groups, by_group, y, eps, gate_w, gate_out, y_xf, y_xf_kind, \
+                                 xf_stride, y_xs);                                                                           \
     } while (0)
     switch ((n + 1023) / 1024) {
         case 1: DFL_NORM(1); break;
@@ -310,13 +314,12 @@ struct RopeHead {
 // With vt_dst, n_kv more workgroups per row scatter the row's V heads, as f16, into column
 // pos[row] of the transposed cache [kv head][dim][capacity].
 // What bounds it: one trip to memory and the arithmetic of the angles (powf, sincosf), which wait for nothing but the
-// position: they run while the head's values are on their way.
+// position: they run while the head's values are on their way.  (The arguments in the order of their use, as the norm's.)
 template <int HD>
 __global__ void __launch_bounds__(64)
-    qk_norm_rope_kernel(const float *q_in, int64_t q_ld, const float *k_in, int64_t k_ld, float *q_out, float *k_out,
-                        const float *__restrict__ q_w, const float *__restrict__ k_w, _Float16 *__restrict__ k_dst,
-                        const int32_t *__restrict__ pos, int n_q, int n_kv, float eps, float theta,
-                        const float *__restrict__ v_src, int64_t v_ld, _Float16 *__restrict__ vt_dst, int64_t capacity) {
+    qk_norm_rope_kernel(const float *q_in, const float *k_in, const float *__restrict__ v_src, const int32_t *__restrict__ pos, int q_ld, int k_ld,
+                        int v_ld, int n_q, int n_kv, float theta, float *q_out, float *k_out, const float *__restrict__ q_w,
+                        const float *__restrict__ k_w, _Float16 *__restrict__ k_dst, _Float16 *__restrict__ vt_dst, int64_t capacity, float eps) {
     const int row = blockIdx.y, head = blockIdx.x, lane = threadIdx.x;
     if (head >= n_q + n_kv) {
         const int vh = head - n_q - n_kv;
@@ -324,6 +327,7 @@ __global__ void __launch_bounds__(64)
         float r[HD / 64];
 #pragma unroll
         for (int k = 0; k < HD / 64; k++) r[k] = src[lane + 64 * k];
+        dfl_have(vt_dst, capacity);
         _Float16 *dst = vt_dst + static_cast<size_t>(vh) * HD * capacity + pos[row];
 #pragma unroll
         for (int k = 0; k < HD / 64; k++) dst[static_cast<size_t>(lane + 64 * k) * capacity] = static_cast<_Float16>(r[k]);
@@ -340,6 +344,7 @@ __global__ void __launch_bounds__(64)
     RopeHead<HD> h;
     h.load(v, w, lane);
     const int32_t pos_row = pos[row];
+    dfl_have(q_out, k_out, k_dst, eps);
     RopePairs<HD> t;
     t.angles(lane, theta, static_cast<float>(pos_row));
     _Float16 *dst = k_dst + (static_cast<size_t>(pos_row) * n_kv + (head - n_q)) * HD;
@@ -354,12 +359,12 @@ __global__ void __launch_bounds__(64)
     });
 }
 
-void qk_norm_rope(int hd, int heads, int rows, hipStream_t st, const float *q_in, int64_t q_ld, const float *k_in, int64_t k_ld, float *q_out,
+void qk_norm_rope(int hd, int heads, int rows, hipStream_t st, const float *q_in, int q_ld, const float *k_in, int k_ld, float *q_out,
                   float *k_out, const float *q_w, const float *k_w, _Float16 *k_dst, const int32_t *pos, int n_q, int n_kv, float eps,
-                  float theta, const float *v_src, int64_t v_ld, _Float16 *vt_dst, int64_t capacity) {
+                  float theta, const float *v_src, int v_ld, _Float16 *vt_dst, int64_t capacity) {
     const auto fn = hd == 64 ? qk_norm_rope_kernel<64> : hd == 128 ? qk_norm_rope_kernel<128> : qk_norm_rope_kernel<256>;
-    fn<<<dim3(heads, rows), 64, 0, st>>>(q_in, q_ld, k_in, k_ld, q_out, k_out, q_w, k_w, k_dst, pos, n_q, n_kv, eps, theta, v_src, v_ld,
-                                         vt_dst, capacity);
+    fn<<<dim3(heads, rows), 64, 0, st>>>(q_in, k_in, v_src, pos, q_ld, k_ld, v_ld, n_q, n_kv, theta, q_out, k_out, q_w, k_w, k_dst, vt_dst, capacity,
+                                         eps);
 }
 
 // The same for the rows of a prefill group, positions pos0 .. pos0 + n - 1, q | k | v side by side in pk: with this many

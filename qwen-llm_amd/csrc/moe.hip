@@ -373,13 +373,13 @@ __global__ void moe_combine_slots_kernel(const float *__restrict__ eo, const int
 // hidden values.  A thread asks for the rows of eight picks at once - unconditionally: past the last pick the last one
 // again, its product left out - where a loop over the picks waited for one row at a time; the picks themselves are scalar
 // loads (the same for the whole workgroup).  V: vectors of four values per thread.
-template <int V>
+template <int V, bool grouped>
 __global__ void __launch_bounds__(256)
     moe_combine_norm_kernel(const float *__restrict__ eo, const int32_t *__restrict__ slot_of, const float *__restrict__ sel_w,
                             const float *__restrict__ sg, const float *__restrict__ shared, const int32_t *__restrict__ n_slots,
                             int n_used, int hidden, float *__restrict__ x, const float *__restrict__ norm_w,
                             float *__restrict__ y, float eps, const float *__restrict__ pre_add, void *__restrict__ y_xf,
-                            int y_xf_kind, int grouped, size_t xf_stride) {
+                            int y_xf_kind, size_t xf_stride) {
     typedef float f4 __attribute__((ext_vector_type(4)));
     __shared__ float sh[4];
     const int row = blockIdx.x, tid = threadIdx.x;
@@ -418,6 +418,7 @@ __global__ void __launch_bounds__(256)
                 if (pre_add) pre[j] = *reinterpret_cast<const f4 *>(pre_add + row_at + at[j]);
                 nw[j] = *reinterpret_cast<const f4 *>(norm_w + at[j]);
             }
+            dfl_have(y, eps, y_xf, y_xf_kind, xf_stride);
         }
 #pragma unroll
         for (int k = 0; k < 8; k++) {
@@ -460,10 +461,11 @@ __global__ void __launch_bounds__(256)
 
 void moe_combine_norm(int rows, hipStream_t st, const float *eo, const int32_t *slot_of, const float *sel_w, const float *sg, const float *shared,
                       const int32_t *n_slots, int n_used, int hidden, float *x, const float *norm_w, float *y, float eps, const float *pre_add,
-                      void *y_xf, int y_xf_kind, int grouped = 0, size_t xf_stride = 0) {
-    const auto fn = hidden <= 1024 ? moe_combine_norm_kernel<1> : hidden <= 2048 ? moe_combine_norm_kernel<2> : moe_combine_norm_kernel<4>;
-    fn<<<rows, 256, 0, st>>>(eo, slot_of, sel_w, sg, shared, n_slots, n_used, hidden, x, norm_w, y, eps, pre_add, y_xf, y_xf_kind, grouped,
-                             xf_stride);
+                      void *y_xf, int y_xf_kind, bool grouped = false, size_t xf_stride = 0) {
+#define DFL_COMBINE(V) (grouped ? moe_combine_norm_kernel<V, true> : moe_combine_norm_kernel<V, false>)
+    const auto fn = hidden <= 1024 ? DFL_COMBINE(1) : hidden <= 2048 ? DFL_COMBINE(2) : DFL_COMBINE(4);
+#undef DFL_COMBINE
+    fn<<<rows, 256, 0, st>>>(eo, slot_of, sel_w, sg, shared, n_slots, n_used, hidden, x, norm_w, y, eps, pre_add, y_xf, y_xf_kind, xf_stride);
 }
 
 // ---- rows of several 16-row blocks through one pass over the experts (prefill) ----
@@ -804,7 +806,7 @@ int32_t dfl_moe_ffn_group(dflash_ctx *ctx, const dflash_model_cfg &c, const dfla
                                     max_tiles, tile_slots, s.eo, fe, H, nullptr, nullptr, st)))
         return rc;
     moe_combine_norm(n_rows, st, s.eo, s.pick_pos, s.sel_w, s.sg, nullptr, s.n_slots, used, H, x_resid, next_norm_w,
-                                                    cur, c.eps, nullptr, next_xf, next_xf_kind, 1, next_xf_stride);
+                                                    cur, c.eps, nullptr, next_xf, next_xf_kind, true, next_xf_stride);
     DFL_HIP_CHECK(ctx, hipGetLastError());
     return DFLASH_OK;
 }
