@@ -145,10 +145,18 @@ inline Q4KDiv q4k_make_div(uint32_t d) {
     return {static_cast<uint32_t>((1ull << (31 + L)) / d + 1), L - 1};
 }
 
+// A launch's split of its flattened iterations: `total` of them (tile groups x nb super-blocks) over n_wg workgroups.
+// (All of this index arithmetic fits 32 bits: the host checks total * (n_wg + 1) < 2^31.)
+struct Q4KSplit {
+    int nb, total, n_wg;
+    Q4KDiv by_total, by_wg;
+};
+inline Q4KSplit q4k_make_split(int nb, int total, int n_wg) {
+    return {nb, total, n_wg, q4k_make_div(static_cast<uint32_t>(total)), q4k_make_div(static_cast<uint32_t>(n_wg))};
+}
 // index of the workgroup whose range contains flattened iteration `it`
-// (all of this index arithmetic fits 32 bits: the host checks total * n_wg < 2^31)
-__device__ __forceinline__ int q4k_wg_of(int it, int total, int n_wg) {
-    return static_cast<int>((static_cast<uint32_t>(it + 1) * n_wg + total - 1) / static_cast<uint32_t>(total)) - 1;
+__device__ __forceinline__ int q4k_wg_of(int it, const Q4KSplit &sp) {
+    return static_cast<int>(q4k_div(static_cast<uint32_t>(it + 1) * sp.n_wg + sp.total - 1, sp.by_total)) - 1;
 }
 
 struct Q4KRange {
@@ -453,7 +461,7 @@ __device__ __forceinline__ void q4k_wait_vm_few(int v) {
 
 // Ends a tile group's segment: Y directly if this workgroup covered the group's whole K, else a
 // partial tile for the reduce kernel (slot 0: the range's first group, slot 1: its last).
-template <int kWaves>
+template <int kWaves, bool kBatch>
 __device__ __forceinline__ void q4k_flush(const Q4KRange &rg, const Q4KBatch &bt, int group, float4_t res,
                                           float4_t &stash, float *__restrict__ y,
                                           float *__restrict__ partials, int n_out, int n_rows, int tid) {
@@ -462,7 +470,7 @@ __device__ __forceinline__ void q4k_flush(const Q4KRange &rg, const Q4KBatch &bt
     const int lane = tid & 63, wave = tid >> 6, n = lane & 15, g = lane >> 4;
     // the group's whole K lies inside this workgroup's range: no other workgroup contributes
     const bool whole = group * rg.nb >= rg.it_begin && (group + 1) * rg.nb <= rg.it_end;
-    if (bt.pair) {
+    if (kBatch && bt.pair) {
         if ((group & 1) == 0) {  // gate half: keep the tile for the up half that follows
             stash = res;
             return;
@@ -471,8 +479,12 @@ __device__ __forceinline__ void q4k_flush(const Q4KRange &rg, const Q4KBatch &bt
         for (int i = 0; i < 4; i++) res[i] = stash[i] / (1.0f + expf(-stash[i])) * res[i];  // silu(gate) * up
         group >>= 1;
     }
-    const int slot_j = bt.ids ? static_cast<int>(q4k_div(group, bt.by_gpm)) : 0, lg = group - slot_j * bt.groups_per_mat;
-    y += static_cast<size_t>(slot_j) * bt.y_stride;
+    int lg = group;
+    if (kBatch) {
+        const int slot_j = static_cast<int>(q4k_div(group, bt.by_gpm));
+        lg -= slot_j * bt.groups_per_mat;
+        y += static_cast<size_t>(slot_j) * bt.y_stride;
+    }
     const int orow = (lg * kWaves + wave) * 16 + n;
     if (whole) {
         if (orow < n_out) {
@@ -503,23 +515,58 @@ __device__ __forceinline__ void q4k_flush(const Q4KRange &rg, const Q4KBatch &bt
 // with its 320 waves, 11.7 instead of 5.4 + 3.9 for the latter with its 16 workgroups (a CU takes in only
 // 20-30 KB per microsecond, so a narrow kernel that reads 8-16 times the data loses more than the launch it
 // saves); a 40-layer verify took 4.77 ms instead of 4.70 ms with the first alone.)
-// Element e = 16 m + n of output tile (group, wave) of a split group: the sum of its partial tiles in workgroup order.
+// What bounds it: the trip to memory for the partial tiles, written on other XCDs, behind the index arithmetic that says which they
+// are.  So the quotients are multiplications by what the host prepares, the workgroup-uniform part stays in scalar registers,
+// and sixteen contributors' tiles are asked for together (four at a time were a trip each: a group of K = 17408 has fourteen).
+// The partial tiles of an output tile (group, wave) of a split group: element e = 16 m + n of the first one at p[e], of the `left`
+// others at p[at_j * stride + e], in workgroup order.
+struct Q4KParts {
+    const float *p, *rest;
+    size_t stride;  // floats per workgroup
+    int left;
+};
 template <int kWaves>
-__device__ __forceinline__ float q4k_partial_sum(const float *__restrict__ partials, int group, int wave, int e, int nb, int total,
-                                                 int n_wg, int wg_first, int wg_last) {
+__device__ __forceinline__ Q4KParts q4k_parts(const float *__restrict__ partials, int group, int wave, const Q4KSplit &sp, int wg_first, int wg_last) {
     // a contributor's partial sits in slot 0 if its range starts inside this group (true for all
     // but possibly the first contributor), else in slot 1
-    const int first_begin = static_cast<int>(static_cast<uint32_t>(total) * wg_first / n_wg);
-    const int first_slot = first_begin >= group * nb ? 0 : 1;
-    const size_t stride = static_cast<size_t>(2) * kWaves * 256;  // floats per workgroup
-    const float *p = partials + static_cast<size_t>(wave) * 256 + e;
-    float sum = p[wg_first * stride + static_cast<size_t>(first_slot) * kWaves * 256];
-    int wg = wg_first + 1;
-    for (; wg + 3 <= wg_last; wg += 4) {
-        const float a0 = p[wg * stride], a1 = p[(wg + 1) * stride], a2 = p[(wg + 2) * stride], a3 = p[(wg + 3) * stride];
-        sum = (((sum + a0) + a1) + a2) + a3;
+    const int first_begin = static_cast<int>(q4k_div(static_cast<uint32_t>(sp.total) * wg_first, sp.by_wg));
+    const int first_slot = first_begin >= group * sp.nb ? 0 : 1;
+    Q4KParts t;
+    t.stride = static_cast<size_t>(2) * kWaves * 256;
+    t.rest = partials + wg_first * t.stride + wave * 256;
+    t.p = t.rest + first_slot * kWaves * 256;
+    t.left = wg_last - wg_first;
+    return t;
+}
+// the next kN contributors (unconditional loads, all in flight together: past the last it is read again) ...
+template <int kN>
+__device__ __forceinline__ void q4k_parts_load(const Q4KParts &t, int e, float (&a)[kN]) {
+#pragma unroll
+    for (int j = 0; j < kN; j++) a[j] = t.rest[min(j + 1, t.left) * t.stride + e];
+}
+// ... added in order
+template <int kN>
+__device__ __forceinline__ float q4k_parts_add(const Q4KParts &t, const float (&a)[kN], float sum) {
+#pragma unroll
+    for (int j = 0; j < kN; j++) sum = j < t.left ? sum + a[j] : sum;
+    return sum;
+}
+__device__ __forceinline__ float q4k_partial_sum(Q4KParts t, int e) {
+    float sum = t.p[e];
+    for (; t.left > 8; t.left -= 16, t.rest += 16 * t.stride) {
+        float a[16];
+        q4k_parts_load<16>(t, e, a);
+        sum = q4k_parts_add<16>(t, a, sum);
     }
-    for (; wg <= wg_last; wg++) sum += p[wg * stride];
+    if (t.left > 4) {
+        float a[8];
+        q4k_parts_load<8>(t, e, a);
+        sum = q4k_parts_add<8>(t, a, sum);
+    } else if (t.left > 0) {
+        float a[4];
+        q4k_parts_load<4>(t, e, a);
+        sum = q4k_parts_add<4>(t, a, sum);
+    }
     return sum;
 }
 
@@ -529,39 +576,62 @@ __device__ __forceinline__ float q4k_partial_sum(const float *__restrict__ parti
 // streaming kernel stored in y.  One launch instead of the reduction and the activation kernel; same bits.
 template <int kWaves>
 __global__ void __launch_bounds__(256)
-    q4k_reduce_swiglu_kernel(const float *__restrict__ partials, const float *__restrict__ y, float *__restrict__ out, int ffn, int nb,
-                             int n_rows, int n_groups, int n_wg) {
+    q4k_reduce_swiglu_kernel(const float *__restrict__ partials, int nb, int total, int n_wg, uint32_t total_mul, uint32_t total_shift, uint32_t wg_mul,
+                             uint32_t wg_shift, int n_rows, int ffn, const float *__restrict__ y, float *__restrict__ out) {
     const int e = threadIdx.x, m = e >> 4, n = e & 15;
-    const int col = blockIdx.x * 16 + n;
-    if (m >= n_rows || col >= ffn) return;
-    const int total = n_groups * nb, n_out = 2 * ffn;
-    auto value = [&](int c) {
-        const int tile = c >> 4, group = tile / kWaves, wave = tile - group * kWaves;
-        const int wg_first = q4k_wg_of(group * nb, total, n_wg), wg_last = q4k_wg_of((group + 1) * nb - 1, total, n_wg);
-        if (wg_first == wg_last) return y[static_cast<size_t>(m) * n_out + c];
-        return q4k_partial_sum<kWaves>(partials, group, wave, e, nb, total, n_wg, wg_first, wg_last);
-    };
-    const float g = value(col), u = value(col + ffn);  // (ffn is a multiple of 16: the same n in both tiles)
-    out[static_cast<size_t>(m) * ffn + col] = g / (1.0f + expf(-g)) * u;
+    const int col = blockIdx.x * 16 + n;  // (ffn is a multiple of 16: the same n in both tiles)
+    if (m >= n_rows) return;
+    const Q4KSplit sp = {nb, total, n_wg, {total_mul, total_shift}, {wg_mul, wg_shift}};
+    Q4KParts t[2];
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const int tile = blockIdx.x + (i ? ffn >> 4 : 0), group = tile / kWaves;
+        t[i] = q4k_parts<kWaves>(partials, group, tile - group * kWaves, sp, q4k_wg_of(group * nb, sp), q4k_wg_of((group + 1) * nb - 1, sp));
+    }
+    float v[2];
+    if (t[0].left > 0 && t[1].left > 0 && t[0].left <= 4 && t[1].left <= 4) {  // (a few contributors each: all of them in flight together)
+        float a[4], b[4];
+        v[0] = t[0].p[e], v[1] = t[1].p[e];
+        q4k_parts_load<4>(t[0], e, a);
+        q4k_parts_load<4>(t[1], e, b);
+        v[0] = q4k_parts_add<4>(t[0], a, v[0]);
+        v[1] = q4k_parts_add<4>(t[1], b, v[1]);
+    } else {
+#pragma unroll
+        for (int i = 0; i < 2; i++) v[i] = t[i].left ? q4k_partial_sum(t[i], e) : y[static_cast<size_t>(m) * (2 * ffn) + col + (i ? ffn : 0)];
+    }
+    out[static_cast<size_t>(m) * ffn + col] = v[0] / (1.0f + expf(-v[0])) * v[1];
 }
 
-template <int kWaves>
+// kBatch: the tile groups of the matrices that a device-side list names (their number with them).
+template <int kWaves, bool kBatch>
 __global__ void __launch_bounds__(256)
-    q4k_reduce_kernel(const float *__restrict__ partials, float *__restrict__ y, int n_out, int nb, int n_rows,
-                      int n_groups, int n_wg, Q4KBatch bt) {
+    q4k_reduce_kernel(const float *__restrict__ partials, int nb, int total, int n_wg, uint32_t total_mul, uint32_t total_shift, uint32_t wg_mul,
+                             uint32_t wg_shift, int n_rows, int n_out,
+                      float *__restrict__ y, Q4KBatch bt) {
     const int group = blockIdx.x / kWaves, wave = blockIdx.x % kWaves;
-    if (bt.ids) n_groups = bt.groups_per_mat * *bt.n_slots;
-    if (group >= n_groups) return;
-    const int total = n_groups * nb;
-    const int wg_first = q4k_wg_of(group * nb, total, n_wg);
-    const int wg_last = q4k_wg_of((group + 1) * nb - 1, total, n_wg);
-    if (wg_first == wg_last) return;
     const int e = threadIdx.x, m = e >> 4, n = e & 15;
-    const int slot_j = group / bt.groups_per_mat, lg = group - slot_j * bt.groups_per_mat;
-    y += static_cast<size_t>(slot_j) * bt.y_stride;
+    Q4KSplit sp = {nb, total, n_wg, {total_mul, total_shift}, {wg_mul, wg_shift}};
+    int wg_first, wg_last;
+    if constexpr (kBatch) {
+        const int n_groups = bt.groups_per_mat * *bt.n_slots;
+        if (group >= n_groups) return;
+        sp.total = n_groups * nb;
+        auto wg_of = [&](int it) { return static_cast<int>((static_cast<uint32_t>(it + 1) * n_wg + sp.total - 1) / static_cast<uint32_t>(sp.total)) - 1; };
+        wg_first = wg_of(group * nb), wg_last = wg_of((group + 1) * nb - 1);
+    } else {
+        wg_first = q4k_wg_of(group * nb, sp), wg_last = q4k_wg_of((group + 1) * nb - 1, sp);
+    }
+    if (wg_first == wg_last) return;
+    int lg = group;
+    if constexpr (kBatch) {
+        const int slot_j = group / bt.groups_per_mat;
+        lg -= slot_j * bt.groups_per_mat;
+        y += static_cast<size_t>(slot_j) * bt.y_stride;
+    }
     const int orow = (lg * kWaves + wave) * 16 + n;
     if (m >= n_rows || orow >= n_out) return;
-    y[static_cast<size_t>(m) * n_out + orow] = q4k_partial_sum<kWaves>(partials, group, wave, e, nb, total, n_wg, wg_first, wg_last);
+    y[static_cast<size_t>(m) * n_out + orow] = q4k_partial_sum(q4k_parts<kWaves>(partials, group, wave, sp, wg_first, wg_last), e);
 }
 
 // Cache-policy bits of the direct-to-LDS weight loads of the tiled and the expert kernel (0: the default policy).
@@ -632,10 +702,14 @@ __device__ unsigned long long *g_trace2 = nullptr;  // [n_wg][16 waves][4]: cycl
     } while (0)
 #endif
 
-template <int kWaves, typename XT>
+// The arguments in the order of their use: the first fourteen words come preloaded with the wave.  kBatch: the matrices of bt's list.
+template <int kWaves, typename XT, bool kBatch>
 __global__ void __launch_bounds__(64 * kWaves)
-    gemm_q4k_stream_kernel(const uint8_t *__restrict__ w, const XT *__restrict__ x, float *__restrict__ y,
-                           float *__restrict__ partials, int n_out, int nb, int n_rows, int n_groups, Q4KBatch bt, int tiled) {
+    gemm_q4k_stream_kernel(const uint8_t *__restrict__ w, const XT *__restrict__ x, int nb, int n_rows, int n_groups, int n_wg, uint32_t wg_mul,
+                           uint32_t wg_shift, uint32_t nb_mul, uint32_t nb_shift, int n_out, int tiled, float *__restrict__ y,
+                           float *__restrict__ partials, Q4KBatch bt) {
+    const Q4KDiv by_wg = {wg_mul, wg_shift}, by_nb = {nb_mul, nb_shift};
+    const bool pair = kBatch && bt.pair;
     using G = Q4KGeom<kWaves>;
     extern __shared__ half8_t lds[];  // kLdsPieces
 
@@ -644,23 +718,23 @@ __global__ void __launch_bounds__(64 * kWaves)
     DFL_TRS(0);
     Q4KRange rg;
     rg.nb = nb;
-    rg.n_wg = gridDim.x;
-    const int vshift = bt.pair ? 1 : 0;  // virtual groups per real group, as a shift
-    const int n_slots = bt.ids ? *bt.n_slots : 1;
-    if (bt.ids) n_groups = (bt.groups_per_mat * n_slots) << vshift;  // how many matrices take part is decided on the device
+    rg.n_wg = n_wg;
+    const int vshift = pair ? 1 : 0;  // virtual groups per real group, as a shift
+    const int n_slots = kBatch ? *bt.n_slots : 1;
+    if (kBatch) n_groups = (bt.groups_per_mat * n_slots) << vshift;  // how many matrices take part is decided on the device
     rg.total = n_groups * nb;
     rg.wg = q4k_range_index(blockIdx.x, rg.n_wg);
-    if (bt.whole_groups) {
+    if (kBatch && bt.whole_groups) {
         // cut between real groups (pair mode: between pairs of virtual groups)
         const uint32_t units = static_cast<uint32_t>(n_groups) >> vshift;
-        rg.it_begin = (static_cast<int>(q4k_div(units * rg.wg, bt.by_wg)) << vshift) * nb;
-        rg.it_end = (static_cast<int>(q4k_div(units * (rg.wg + 1), bt.by_wg)) << vshift) * nb;
+        rg.it_begin = (static_cast<int>(q4k_div(units * rg.wg, by_wg)) << vshift) * nb;
+        rg.it_end = (static_cast<int>(q4k_div(units * (rg.wg + 1), by_wg)) << vshift) * nb;
     } else {
-        rg.it_begin = static_cast<int>(q4k_div(static_cast<uint32_t>(rg.total) * rg.wg, bt.by_wg));
-        rg.it_end = static_cast<int>(q4k_div(static_cast<uint32_t>(rg.total) * (rg.wg + 1), bt.by_wg));
+        rg.it_begin = static_cast<int>(q4k_div(static_cast<uint32_t>(rg.total) * rg.wg, by_wg));
+        rg.it_end = static_cast<int>(q4k_div(static_cast<uint32_t>(rg.total) * (rg.wg + 1), by_wg));
     }
     if (rg.it_begin >= rg.it_end) return;  // more workgroups than work
-    rg.first_group = static_cast<int>(q4k_div(rg.it_begin, bt.by_nb));
+    rg.first_group = static_cast<int>(q4k_div(rg.it_begin, by_nb));
     const int b0 = rg.it_begin - rg.first_group * nb;
     const uint32_t row_bytes = static_cast<uint32_t>(nb) * DFL_Q4_K_BYTES;
     const uint32_t n_in = static_cast<uint32_t>(nb) * DFL_QK_K;
@@ -690,8 +764,8 @@ __global__ void __launch_bounds__(64 * kWaves)
     auto group_w = [&](int group) {
         const uint8_t *mat = w;
         int lg = group;
-        if (bt.ids) {
-            const bool up = bt.pair && (group & 1);
+        if (kBatch) {
+            const bool up = pair && (group & 1);
             const int g = group >> vshift;
             const int j = static_cast<int>(q4k_div(g, bt.by_gpm));
             lg = g - j * bt.groups_per_mat;
@@ -704,12 +778,12 @@ __global__ void __launch_bounds__(64 * kWaves)
         return q4k_uniform(mat + static_cast<size_t>(lg) * group_bytes);
     };
     auto group_x = [&](int group) {
-        if (!bt.ids) return xbytes;
+        if (!kBatch) return xbytes;
         return xbytes + static_cast<size_t>(q4k_div(group >> vshift, bt.by_gpm)) * bt.x_stride * sizeof(XT);
     };
     auto group_local = [&](int group) {
         group >>= vshift;
-        return bt.ids ? group - static_cast<int>(q4k_div(group, bt.by_gpm)) * bt.groups_per_mat : group;
+        return kBatch ? group - static_cast<int>(q4k_div(group, bt.by_gpm)) * bt.groups_per_mat : group;
     };
     DFL_TRS(10);
     Q4KLane<kWaves> L;
@@ -723,7 +797,7 @@ __global__ void __launch_bounds__(64 * kWaves)
     int bw = b0, gw = rg.first_group, w_left = rg.it_end - rg.it_begin;
     const uint8_t *xblock = group_x(rg.first_group) + static_cast<size_t>(b0) * kXBlockBytes;
     int bx = b0, gx = rg.first_group, x_left = w_left;
-    const bool ragged = bt.groups_per_mat * G::kRows > n_out;  // a matrix's last group has fewer rows
+    const bool ragged = (kBatch ? bt.groups_per_mat : n_groups) * G::kRows > n_out;  // a matrix's last group has fewer rows
     auto advance_w = [&]() {
         wstage += tiled ? kTiledStageBytes : DFL_Q4_K_BYTES;
         w_left--;
@@ -850,7 +924,7 @@ __global__ void __launch_bounds__(64 * kWaves)
         done++;
         if (done <= 8) DFL_TRS(1 + done);
         if (++bc == nb || n_left == 0) {
-            q4k_flush<kWaves>(rg, bt, gc, G::kSums ? acc : acc + acc_min, stash, y, partials, n_out, n_rows, tid);
+            q4k_flush<kWaves, kBatch>(rg, bt, gc, G::kSums ? acc : acc + acc_min, stash, y, partials, n_out, n_rows, tid);
             acc = float4_t{0, 0, 0, 0};
             acc_min = float4_t{0, 0, 0, 0};
             bc = 0;
@@ -1145,7 +1219,7 @@ __global__ void __launch_bounds__(64 * kSlabWaves)
                 acc = q4k_again<XT, false>(w + static_cast<size_t>(row) * row_bytes + static_cast<size_t>(bs) * DFL_Q4_K_BYTES, DFL_Q4_K_BYTES,
                                            x + static_cast<size_t>(min(n, n_rows - 1)) * n_in + bs * DFL_QK_K, bc - bs, g, sc_sel, magic);
             }
-            q4k_flush<kW>(rg, bt, gc, acc, stash, y, partials, n_out, n_rows, tid);
+            q4k_flush<kW, false>(rg, bt, gc, acc, stash, y, partials, n_out, n_rows, tid);
             acc = float4_t{0, 0, 0, 0};
             bc = bs = 0;
             gc++;
@@ -1245,13 +1319,15 @@ __device__ __forceinline__ void q4k_tiled_compute(const u32x4_t *blk, const uint
     q4k_stage(hdr, q0, q1, af, a_min, g, sc_sel, magic, acc, false);
 }
 
-// The tiled kernel.  Same work split, flush and reduction as the slab kernel.  Order of the prologue: the
+// The tiled kernel (arguments as the streaming kernel's).  Same work split, flush and reduction as the slab kernel.  Order of the prologue: the
 // activation loads alone, then (once they are back and converted) the first three weight stages into the wave's
 // ring; see the measurements at the issue points.
 template <typename XT>
 __global__ void __launch_bounds__(64 * kSlabWaves)
-    gemm_q4k_tiled_kernel(const uint8_t *__restrict__ w, const XT *__restrict__ x, float *__restrict__ y,
-                          float *__restrict__ partials, int n_out, int nb, int n_rows, int n_groups, Q4KBatch bt, int kPre) {
+    gemm_q4k_tiled_kernel(const uint8_t *__restrict__ w, const XT *__restrict__ x, int nb, int n_rows, int n_groups, int n_wg, uint32_t wg_mul,
+                          uint32_t wg_shift, uint32_t nb_mul, uint32_t nb_shift, int kPre, int n_out, float *__restrict__ y, float *__restrict__ partials) {
+    const Q4KBatch bt = {};
+    const Q4KDiv by_wg = {wg_mul, wg_shift}, by_nb = {nb_mul, nb_shift};
     constexpr int kW = kSlabWaves;
     extern __shared__ half8_t lds[];
     uint8_t *slab = reinterpret_cast<uint8_t *>(lds);                                // [kSlabStages][kTiledStageX]
@@ -1260,15 +1336,15 @@ __global__ void __launch_bounds__(64 * kSlabWaves)
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     Q4KRange rg;
     rg.nb = nb;
-    rg.n_wg = gridDim.x;
+    rg.n_wg = n_wg;
     rg.total = n_groups * nb;
     rg.wg = q4k_range_index(blockIdx.x, rg.n_wg);
-    rg.it_begin = static_cast<int>(q4k_div(static_cast<uint32_t>(rg.total) * rg.wg, bt.by_wg));
-    rg.it_end = static_cast<int>(q4k_div(static_cast<uint32_t>(rg.total) * (rg.wg + 1), bt.by_wg));
+    rg.it_begin = static_cast<int>(q4k_div(static_cast<uint32_t>(rg.total) * rg.wg, by_wg));
+    rg.it_end = static_cast<int>(q4k_div(static_cast<uint32_t>(rg.total) * (rg.wg + 1), by_wg));
     const int len = rg.it_end - rg.it_begin;  // <= kSlabStages (host)
     if (len <= 0) return;
     DFL_TR(0);
-    rg.first_group = static_cast<int>(q4k_div(rg.it_begin, bt.by_nb));
+    rg.first_group = static_cast<int>(q4k_div(rg.it_begin, by_nb));
     const int b0 = rg.it_begin - rg.first_group * nb;
     const uint32_t n_in = static_cast<uint32_t>(nb) * DFL_QK_K;
 
@@ -1368,7 +1444,7 @@ __global__ void __launch_bounds__(64 * kSlabWaves)
                 acc = q4k_again<XT, false>(w + (static_cast<size_t>(gc) * nb + bs) * kTiledStageBytes + wave * kTiledTileBytes + n * DFL_Q4_K_BYTES,
                                            kTiledStageBytes, x + static_cast<size_t>(min(n, n_rows - 1)) * n_in + bs * DFL_QK_K, bc - bs, g,
                                            sc_sel, magic);
-            q4k_flush<kW>(rg, bt, gc, acc, stash, y, partials, n_out, n_rows, tid);
+            q4k_flush<kW, false>(rg, bt, gc, acc, stash, y, partials, n_out, n_rows, tid);
             acc = float4_t{0, 0, 0, 0};
             bc = bs = 0;
             gc++;
@@ -1450,9 +1526,13 @@ __device__ __forceinline__ void q4k_experts_compute(const u32x4_t *blk, const ui
 
 template <typename XT, typename YT, bool kRoute>
 __global__ void __launch_bounds__(64 * kSlabWaves)
-    gemm_q4k_experts_kernel(const uint8_t *__restrict__ w, const XT *__restrict__ x, YT *__restrict__ y, int n_out, int nb,
-                            int n_rows, Q4KBatch bt, int upm, Q4KDiv by_upm, int max_slots, int early_ids) {
+    gemm_q4k_experts_kernel(const XT *__restrict__ x, const float *__restrict__ logits, int32_t *ids, int32_t *n_slots_at,
+                            const uint8_t *__restrict__ w, int nb, uint32_t rows_route, int n_out, int max_slots, YT *__restrict__ y, int n_wg,
+                            int upm, Q4KDiv by_upm, int early_ids, Q4KBatch bt) {
+    // (The arguments in the order of their use: the first fourteen words come preloaded with the wave, the others are asked for
+    // under the first loads.  rows_route = n_rows | picks per row << 8 | experts << 16 | shared expert << 31.)
     constexpr int kW = kSlabWaves;
+    const int n_rows = rows_route & 255;
     constexpr int kItems = kExpChunk * 8 / kW;  // activation items (eight values of one row) per thread and refill: 2
     constexpr int kXInstr = kItems * Q4KX8<XT>::kLoads;
     static_assert(3 * (kSlabRing - 1) + kXInstr <= 10 && 3 * kSlabRing <= 10, "q4k_wait_vm_few");
@@ -1461,7 +1541,7 @@ __global__ void __launch_bounds__(64 * kSlabWaves)
     half8_t *ring = reinterpret_cast<half8_t *>(slab + kExpChunk * kTiledStageX);  // [wave][kSlabRing][144]
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const bool per_slot_x = bt.x_stride != 0;
+    const bool per_slot_x = !kRoute && bt.x_stride != 0;
     DFL_TRE_DECL;
     DFL_TRE(0);
     // ---- activations: items as in gemm_q4k_tiled_kernel (virtual wave v = wave + 16 r: stage v / 8 of the chunk) ----
@@ -1477,7 +1557,7 @@ __global__ void __launch_bounds__(64 * kSlabWaves)
     }
     auto chunk_len = [&](int c) { return min(kExpChunk, nb - c * kExpChunk); };
     auto load_x = [&](int xslot, int c) {  // stages past the chunk's end re-read its last stage (never converted)
-        const uint8_t *xb = q4k_uniform(xbytes + static_cast<size_t>(xslot) * bt.x_stride * sizeof(XT));
+        const uint8_t *xb = q4k_uniform(xbytes + (kRoute ? 0 : static_cast<size_t>(xslot) * bt.x_stride * sizeof(XT)));
         const int last = chunk_len(c) - 1;
 #pragma unroll
         for (int r = 0; r < kItems; r++) {
@@ -1498,10 +1578,11 @@ __global__ void __launch_bounds__(64 * kSlabWaves)
         // are asm loads with their own wait, like the activations': a wait the compiler placed at the logits' first use
         // would stand behind the activation loads again.
         unsigned long long *row_mask = reinterpret_cast<unsigned long long *>(reinterpret_cast<uint8_t *>(lds) + kExpXchgEnd);
-        const int E = bt.route_experts, used = bt.route_used;
+        const int E = rows_route >> 16 & 0x1ff, used = rows_route >> 8 & 255;
+        const bool with_shared = rows_route >> 31;
         float lgv[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
         if (wave < n_rows) {
-            const float *lrow = bt.route_logits + static_cast<size_t>(wave) * E + lane;
+            const float *lrow = logits + static_cast<size_t>(wave) * E + lane;
 #pragma unroll
             for (int j = 0; j < 4; j++)
                 if (lane + 64 * j < E) asm volatile("global_load_dword %0, %1, off" : "+v"(lgv[j]) : "v"(lrow + 64 * j) : "memory");
@@ -1510,6 +1591,8 @@ __global__ void __launch_bounds__(64 * kSlabWaves)
 #pragma unroll
         for (int j = 0; j < 4; j++) asm volatile("" : "+v"(lgv[j]));
         load_x(0, 0);
+        dfl_have(y, n_wg, upm, by_upm.mul, by_upm.shift, bt.w2, bt.extra_w, bt.extra_w2, bt.w_stride, bt.y_stride, bt.by_wg.mul, bt.by_wg.shift,
+                 bt.pair, bt.route_sel_e, bt.route_sel_w, bt.route_slot_of);
         dfl_route::RowPicks pk;
         pk.my_e = 0;
         pk.my_w = 0.0f;
@@ -1521,17 +1604,16 @@ __global__ void __launch_bounds__(64 * kSlabWaves)
         unsigned long long un[4];
         dfl_route::union_of_rows(row_mask, lane, un);
         const int total = __popcll(un[0]) + __popcll(un[1]) + __popcll(un[2]) + __popcll(un[3]);
-        n_slots = min(total + (bt.route_shared ? 1 : 0), max_slots);
+        n_slots = min(total + (with_shared ? 1 : 0), max_slots);
         const bool listed = tid < E && ((dfl_route::pick4(un, tid >> 6) >> (tid & 63)) & 1);
         const int my_slot = listed ? dfl_route::slot_below(un, tid) : 0;
         if (listed) ids_lds[my_slot] = tid;
-        if (tid == 0 && bt.route_shared) ids_lds[total] = -1;
+        if (tid == 0 && with_shared) ids_lds[total] = -1;
         if (blockIdx.x == 0) {  // one copy for the launches that follow
-            int32_t *ids_out = const_cast<int32_t *>(bt.ids);
-            if (listed) ids_out[my_slot] = tid;
+            if (listed) ids[my_slot] = tid;
             if (tid == 0) {
-                if (bt.route_shared) ids_out[total] = -1;
-                *const_cast<int32_t *>(bt.n_slots) = n_slots;
+                if (with_shared) ids[total] = -1;
+                *n_slots_at = n_slots;
             }
             if (wave < n_rows && lane < used) {
                 bt.route_sel_e[wave * used + lane] = pk.my_e;
@@ -1543,10 +1625,12 @@ __global__ void __launch_bounds__(64 * kSlabWaves)
         __builtin_amdgcn_s_barrier();
     } else {
         if (early_ids) {  // the first window of the list travels with the slot count: one trip to memory instead of two
-            ids_window = bt.ids[min(lane, max_slots - 1)];
+            ids_window = ids[min(lane, max_slots - 1)];
             slot_base = 0;
         }
-        n_slots = min(*bt.n_slots, max_slots);  // (the bound the host sized the buffers for)
+        n_slots = min(*n_slots_at, max_slots);  // (the bound the host sized the buffers for)
+        dfl_have(y, n_wg, upm, by_upm.mul, by_upm.shift, bt.w2, bt.extra_w, bt.extra_w2, bt.w_stride, bt.x_stride, bt.y_stride, bt.by_wg.mul,
+                 bt.by_wg.shift, bt.pair);
         // one wait for both, stated here on every path so that none is implied at the window's later uses
         __builtin_amdgcn_s_waitcnt(q4k_vmcnt(0));
         asm volatile("" : "+v"(ids_window));
@@ -1557,7 +1641,7 @@ __global__ void __launch_bounds__(64 * kSlabWaves)
     const int n_chunks = (nb + kExpChunk - 1) / kExpChunk;
     // units: (slot, tile) with shared x, (slot, group of sixteen tiles) with x per slot; upm = units per matrix
     const uint32_t units = static_cast<uint32_t>(n_slots) * static_cast<uint32_t>(upm);
-    const int wg = q4k_range_index(blockIdx.x, gridDim.x);
+    const int wg = q4k_range_index(blockIdx.x, n_wg);
     const int u0 = static_cast<int>(q4k_div(units * wg, bt.by_wg)), u1 = static_cast<int>(q4k_div(units * (wg + 1), bt.by_wg));
     if (u0 >= u1) return;  // more workgroups than work (the whole workgroup leaves: no barrier is missed)
     // Pair mode with at most eight units for this workgroup: gate and up of a unit go to two waves (w and w + 8)
@@ -1574,11 +1658,11 @@ __global__ void __launch_bounds__(64 * kSlabWaves)
     auto slot_id = [&](int j) {
         if constexpr (kRoute) {  // the list is in LDS; whatever it holds, the index stays inside the stack
             const int32_t id = __builtin_amdgcn_readfirstlane(ids_lds[min(max(j, 0), kExpRouteIds - 1)]);
-            return min(max(id, -1), bt.route_experts - 1);
+            return min(max(id, -1), static_cast<int>(rows_route >> 16 & 0x1ff) - 1);
         }
         if (j < slot_base || j >= slot_base + 64) {
             slot_base = j;
-            ids_window = bt.ids[min(j + lane, n_slots - 1)];
+            ids_window = ids[min(j + lane, n_slots - 1)];
             __builtin_amdgcn_s_waitcnt(q4k_vmcnt(0));
             asm volatile("" : "+v"(ids_window));
         }
@@ -1904,8 +1988,10 @@ __device__ __forceinline__ void q6k_store_w(uint8_t *area, const Q6KLane &W, con
 
 template <int kWaves, typename XT>
 __global__ void __launch_bounds__(64 * kWaves)
-    gemm_q6k_stream_kernel(const uint8_t *__restrict__ w, const XT *__restrict__ x, float *__restrict__ y,
-                           float *__restrict__ partials, int n_out, int nb, int n_rows, int n_groups, Q4KBatch bt) {
+    gemm_q6k_stream_kernel(const uint8_t *__restrict__ w, const XT *__restrict__ x, int nb, int n_rows, int n_groups, int n_wg, uint32_t wg_mul,
+                           uint32_t wg_shift, uint32_t nb_mul, uint32_t nb_shift, int n_out, float *__restrict__ y, float *__restrict__ partials) {
+    const Q4KBatch bt = {};
+    const Q4KDiv by_wg = {wg_mul, wg_shift}, by_nb = {nb_mul, nb_shift};
     using G6 = Q6KGeom<kWaves>;
     using G = Q4KGeom<kWaves>;
     extern __shared__ half8_t lds[];
@@ -1913,13 +1999,13 @@ __global__ void __launch_bounds__(64 * kWaves)
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     Q4KRange rg;
     rg.nb = nb;
-    rg.n_wg = gridDim.x;
+    rg.n_wg = n_wg;
     rg.total = n_groups * nb;
     rg.wg = q4k_range_index(blockIdx.x, rg.n_wg);
-    rg.it_begin = static_cast<int>(q4k_div(static_cast<uint32_t>(rg.total) * rg.wg, bt.by_wg));
-    rg.it_end = static_cast<int>(q4k_div(static_cast<uint32_t>(rg.total) * (rg.wg + 1), bt.by_wg));
+    rg.it_begin = static_cast<int>(q4k_div(static_cast<uint32_t>(rg.total) * rg.wg, by_wg));
+    rg.it_end = static_cast<int>(q4k_div(static_cast<uint32_t>(rg.total) * (rg.wg + 1), by_wg));
     if (rg.it_begin >= rg.it_end) return;
-    rg.first_group = static_cast<int>(q4k_div(rg.it_begin, bt.by_nb));
+    rg.first_group = static_cast<int>(q4k_div(rg.it_begin, by_nb));
     const int b0 = rg.it_begin - rg.first_group * nb;
     const uint32_t row_bytes = static_cast<uint32_t>(nb) * DFL_Q6_K_BYTES;
     const uint32_t n_in = static_cast<uint32_t>(nb) * DFL_QK_K;
@@ -2074,7 +2160,7 @@ __global__ void __launch_bounds__(64 * kWaves)
         x_n = tx;
         n_left--;
         if (++bc == nb || n_left == 0) {
-            q4k_flush<kWaves>(rg, bt, gc, acc - acc_off, stash, y, partials, n_out, n_rows, tid);
+            q4k_flush<kWaves, false>(rg, bt, gc, acc - acc_off, stash, y, partials, n_out, n_rows, tid);
             acc = float4_t{0, 0, 0, 0};
             acc_off = float4_t{0, 0, 0, 0};
             bc = 0;
@@ -2673,8 +2759,11 @@ int32_t launch_q4k(dflash_ctx *ctx, const void *w, const void *x, int32_t x_type
         if (const int32_t rc_ = dfl_raise_lds_limit(ctx, reinterpret_cast<const void *>(gemm_q4k_experts_kernel<XT, YT, ROUTE>), kExpLdsBytes)) \
             return rc_;                                                                                                     \
         dfl_timed timer(ctx, st, DFL_T_GEMM);                                                                               \
-        gemm_q4k_experts_kernel<XT, YT, ROUTE><<<n_wg, 64 * kSlabWaves, kExpLdsBytes, st>>>(wb, static_cast<const XT *>(x), reinterpret_cast<YT *>(y), \
-                                                                                           no, nb, n_rows, bt, upm, by_upm, max_slots, early_ids); \
+        const uint32_t rows_route = static_cast<uint32_t>(n_rows) | static_cast<uint32_t>(bt.route_used) << 8 |                                   \
+                                    static_cast<uint32_t>(bt.route_experts) << 16 | (bt.route_shared ? 1u << 31 : 0u);                             \
+        gemm_q4k_experts_kernel<XT, YT, ROUTE><<<n_wg, 64 * kSlabWaves, kExpLdsBytes, st>>>(                                                       \
+            static_cast<const XT *>(x), bt.route_logits, const_cast<int32_t *>(bt.ids), const_cast<int32_t *>(bt.n_slots), wb, nb, rows_route, no, \
+            max_slots, reinterpret_cast<YT *>(y), n_wg, upm, by_upm, early_ids, bt);                                                              \
     } while (0)
         if (bt.route_logits) {
             if (x_type != DFLASH_TYPE_F32 || per_slot_x || !bt.y_f16 || bt.route_experts > 256 || bt.route_experts < 1 || bt.route_used < 1 ||
@@ -2732,6 +2821,7 @@ int32_t launch_q4k(dflash_ctx *ctx, const void *w, const void *x, int32_t x_type
     if (swiglu_out) ctx->swiglu_done = false;
     Q4KBatch bt = {};
     if (batch) bt = *batch;
+    const Q4KSplit sp = q4k_make_split(nb, static_cast<int>(total), n_wg);
     bt.groups_per_mat = gpm;
     bt.by_gpm = q4k_make_div(static_cast<uint32_t>(gpm));
     bt.by_nb = q4k_make_div(static_cast<uint32_t>(nb));
@@ -2743,20 +2833,21 @@ int32_t launch_q4k(dflash_ctx *ctx, const void *w, const void *x, int32_t x_type
         const size_t lds = static_cast<size_t>(Q4KGeom<WAVES>::kLdsPieces) * sizeof(half8_t);                      \
         if (lds > ctx->lds_bytes)                                                                                      \
             return dfl_fail(ctx, DFLASH_ERR_UNSUPPORTED, "gemm_fewrow: %zu bytes of LDS needed", lds);                 \
-        if (const int32_t rc_ = dfl_raise_lds_limit(ctx, reinterpret_cast<const void *>(gemm_q4k_stream_kernel<WAVES, XT>), lds)) \
-            return rc_;                                                                                                \
+        const auto sfn = bt.ids ? gemm_q4k_stream_kernel<WAVES, XT, true> : gemm_q4k_stream_kernel<WAVES, XT, false>;  \
+        if (const int32_t rc_ = dfl_raise_lds_limit(ctx, reinterpret_cast<const void *>(sfn), lds)) return rc_;       \
         {                                                                                                              \
             dfl_timed timer(ctx, st, DFL_T_GEMM);                                                                      \
-            gemm_q4k_stream_kernel<WAVES, XT><<<n_wg, 64 * WAVES, lds, st>>>(wb, static_cast<const XT *>(x), y, partials, \
-                                                                             no, nb, n_rows, groups, bt, tiled ? 1 : 0); \
+            sfn<<<n_wg, 64 * WAVES, lds, st>>>(wb, static_cast<const XT *>(x), nb, n_rows, groups, n_wg, bt.by_wg.mul, bt.by_wg.shift, bt.by_nb.mul, \
+                                               bt.by_nb.shift, no, tiled ? 1 : 0, y, partials, bt);                    \
         }                                                                                                              \
         if (reduce && swiglu_out) {                                                                                    \
             dfl_timed timer(ctx, st, DFL_T_REDUCE);                                                                    \
-            q4k_reduce_swiglu_kernel<WAVES><<<no / 32, 256, 0, st>>>(partials, y, swiglu_out, no / 2, nb, n_rows, groups, n_wg); \
+            q4k_reduce_swiglu_kernel<WAVES><<<no / 32, 256, 0, st>>>(partials, sp.nb, sp.total, sp.n_wg, sp.by_total.mul, sp.by_total.shift, sp.by_wg.mul, sp.by_wg.shift, n_rows, no / 2, y, swiglu_out); \
             ctx->swiglu_done = true;                                                                                   \
         } else if (reduce) {                                                                                           \
             dfl_timed timer(ctx, st, DFL_T_REDUCE);                                                                    \
-            q4k_reduce_kernel<WAVES><<<groups * WAVES, 256, 0, st>>>(partials, y, no, nb, n_rows, groups, n_wg, bt);   \
+            const auto rfn = bt.ids ? q4k_reduce_kernel<WAVES, true> : q4k_reduce_kernel<WAVES, false>;                 \
+            rfn<<<groups * WAVES, 256, 0, st>>>(partials, sp.nb, sp.total, sp.n_wg, sp.by_total.mul, sp.by_total.shift, sp.by_wg.mul, sp.by_wg.shift, n_rows, no, y, bt); \
         }                                                                                                              \
     } while (0)
     if (slab && tiled) {
@@ -2769,23 +2860,25 @@ int32_t launch_q4k(dflash_ctx *ctx, const void *w, const void *x, int32_t x_type
         // (while stamping is on, a dispatch carries start / stop stamps of its own: the kernel's duration as a trace reports it)
         {
             dfl_timed timer(ctx, st, DFL_T_GEMM);
-            const dfl_stamp sp(ctx, DFL_T_KERNEL_Q4K_TILED);
+            const dfl_stamp stamp(ctx, DFL_T_KERNEL_Q4K_TILED);
             if (x_type == DFLASH_TYPE_F32)
-                hipExtLaunchKernelGGL(gemm_q4k_tiled_kernel<float>, dim3(n_wg), dim3(64 * kSlabWaves), kTiledLdsBytes, st, sp.start, sp.stop, 0,
-                                      wb, static_cast<const float *>(x), y, partials, no, nb, n_rows, groups, bt, k_pre);
+                hipExtLaunchKernelGGL(gemm_q4k_tiled_kernel<float>, dim3(n_wg), dim3(64 * kSlabWaves), kTiledLdsBytes, st, stamp.start, stamp.stop, 0,
+                                      wb, static_cast<const float *>(x), nb, n_rows, groups, n_wg, bt.by_wg.mul, bt.by_wg.shift, bt.by_nb.mul, bt.by_nb.shift,
+                                      k_pre, no, y, partials);
             else
-                hipExtLaunchKernelGGL(gemm_q4k_tiled_kernel<_Float16>, dim3(n_wg), dim3(64 * kSlabWaves), kTiledLdsBytes, st, sp.start, sp.stop, 0,
-                                      wb, static_cast<const _Float16 *>(x), y, partials, no, nb, n_rows, groups, bt, k_pre);
+                hipExtLaunchKernelGGL(gemm_q4k_tiled_kernel<_Float16>, dim3(n_wg), dim3(64 * kSlabWaves), kTiledLdsBytes, st, stamp.start, stamp.stop, 0,
+                                      wb, static_cast<const _Float16 *>(x), nb, n_rows, groups, n_wg, bt.by_wg.mul, bt.by_wg.shift, bt.by_nb.mul, bt.by_nb.shift,
+                                      k_pre, no, y, partials);
         }
         if (reduce && swiglu_out) {
             dfl_timed timer(ctx, st, DFL_T_REDUCE);
-            q4k_reduce_swiglu_kernel<16><<<no / 32, 256, 0, st>>>(partials, y, swiglu_out, no / 2, nb, n_rows, groups, n_wg);
+            q4k_reduce_swiglu_kernel<16><<<no / 32, 256, 0, st>>>(partials, sp.nb, sp.total, sp.n_wg, sp.by_total.mul, sp.by_total.shift, sp.by_wg.mul, sp.by_wg.shift, n_rows, no / 2, y, swiglu_out);
             ctx->swiglu_done = true;
         } else if (reduce) {
             dfl_timed timer(ctx, st, DFL_T_REDUCE);
-            const dfl_stamp sp(ctx, DFL_T_KERNEL_Q4K_REDUCE);
-            hipExtLaunchKernelGGL(q4k_reduce_kernel<16>, dim3(groups * 16), dim3(256), 0, st, sp.start, sp.stop, 0, partials, y, no, nb, n_rows,
-                                  groups, n_wg, bt);
+            const dfl_stamp stamp(ctx, DFL_T_KERNEL_Q4K_REDUCE);
+            hipExtLaunchKernelGGL((q4k_reduce_kernel<16, false>), dim3(groups * 16), dim3(256), 0, st, stamp.start, stamp.stop, 0, partials, sp.nb,
+                                  sp.total, sp.n_wg, sp.by_total.mul, sp.by_total.shift, sp.by_wg.mul, sp.by_wg.shift, n_rows, no, y, bt);
         }
     } else if (slab) {
         const void *fn = x_type == DFLASH_TYPE_F32 ? reinterpret_cast<const void *>(gemm_q4k_slab_kernel<float>)
@@ -2793,21 +2886,21 @@ int32_t launch_q4k(dflash_ctx *ctx, const void *w, const void *x, int32_t x_type
         if (const int32_t rc_ = dfl_raise_lds_limit(ctx, fn, kSlabLdsBytes)) return rc_;
         {
             dfl_timed timer(ctx, st, DFL_T_GEMM);
-            const dfl_stamp sp(ctx, DFL_T_KERNEL_Q4K_TILED);  // (the same slot as the tiled kernel: one of the two runs)
+            const dfl_stamp stamp(ctx, DFL_T_KERNEL_Q4K_TILED);  // (the same slot as the tiled kernel: one of the two runs)
             if (x_type == DFLASH_TYPE_F32)
-                hipExtLaunchKernelGGL(gemm_q4k_slab_kernel<float>, dim3(n_wg), dim3(64 * kSlabWaves), kSlabLdsBytes, st, sp.start, sp.stop, 0, wb,
+                hipExtLaunchKernelGGL(gemm_q4k_slab_kernel<float>, dim3(n_wg), dim3(64 * kSlabWaves), kSlabLdsBytes, st, stamp.start, stamp.stop, 0, wb,
                                       static_cast<const float *>(x), y, partials, no, nb, n_rows, groups, bt);
             else
-                hipExtLaunchKernelGGL(gemm_q4k_slab_kernel<_Float16>, dim3(n_wg), dim3(64 * kSlabWaves), kSlabLdsBytes, st, sp.start, sp.stop, 0, wb,
+                hipExtLaunchKernelGGL(gemm_q4k_slab_kernel<_Float16>, dim3(n_wg), dim3(64 * kSlabWaves), kSlabLdsBytes, st, stamp.start, stamp.stop, 0, wb,
                                       static_cast<const _Float16 *>(x), y, partials, no, nb, n_rows, groups, bt);
         }
         if (reduce && swiglu_out) {
             dfl_timed timer(ctx, st, DFL_T_REDUCE);
-            q4k_reduce_swiglu_kernel<16><<<no / 32, 256, 0, st>>>(partials, y, swiglu_out, no / 2, nb, n_rows, groups, n_wg);
+            q4k_reduce_swiglu_kernel<16><<<no / 32, 256, 0, st>>>(partials, sp.nb, sp.total, sp.n_wg, sp.by_total.mul, sp.by_total.shift, sp.by_wg.mul, sp.by_wg.shift, n_rows, no / 2, y, swiglu_out);
             ctx->swiglu_done = true;
         } else if (reduce) {
             dfl_timed timer(ctx, st, DFL_T_REDUCE);
-            q4k_reduce_kernel<16><<<groups * 16, 256, 0, st>>>(partials, y, no, nb, n_rows, groups, n_wg, bt);
+            q4k_reduce_kernel<16, false><<<groups * 16, 256, 0, st>>>(partials, sp.nb, sp.total, sp.n_wg, sp.by_total.mul, sp.by_total.shift, sp.by_wg.mul, sp.by_wg.shift, n_rows, no, y, bt);
         }
     } else if (waves == 16 && x_type == DFLASH_TYPE_F32)
         DFL_LAUNCH_Q4K(16, float);
@@ -2861,10 +2954,8 @@ int32_t launch_q6k_stream(dflash_ctx *ctx, const void *w, const void *x, int32_t
     float *partials = reinterpret_cast<float *>(ctx->partials);
     const bool split = groups % n_wg != 0;
     Q4KBatch bt = {};
-    bt.groups_per_mat = groups;
-    bt.by_gpm = q4k_make_div(static_cast<uint32_t>(groups));
-    bt.by_nb = q4k_make_div(static_cast<uint32_t>(nb));
-    bt.by_wg = q4k_make_div(static_cast<uint32_t>(n_wg));
+    const Q4KSplit sp = q4k_make_split(nb, static_cast<int>(total), n_wg);
+    const Q4KDiv by_nb = q4k_make_div(static_cast<uint32_t>(nb));
     const uint8_t *wb = static_cast<const uint8_t *>(w);
     const int no = static_cast<int>(n_out);
 #define DFL_LAUNCH_Q6K(WAVES, XT)                                                                                      \
@@ -2876,12 +2967,12 @@ int32_t launch_q6k_stream(dflash_ctx *ctx, const void *w, const void *x, int32_t
             return rc_;                                                                                                \
         {                                                                                                              \
             dfl_timed timer(ctx, st, DFL_T_GEMM);                                                                      \
-            gemm_q6k_stream_kernel<WAVES, XT><<<n_wg, 64 * WAVES, lds, st>>>(wb, static_cast<const XT *>(x), y, partials, \
-                                                                             no, nb, n_rows, groups, bt);              \
+            gemm_q6k_stream_kernel<WAVES, XT><<<n_wg, 64 * WAVES, lds, st>>>(wb, static_cast<const XT *>(x), nb, n_rows, groups, n_wg, sp.by_wg.mul, \
+                                                                             sp.by_wg.shift, by_nb.mul, by_nb.shift, no, y, partials); \
         }                                                                                                              \
         if (split) {                                                                                                   \
             dfl_timed timer(ctx, st, DFL_T_REDUCE);                                                                    \
-            q4k_reduce_kernel<WAVES><<<groups * WAVES, 256, 0, st>>>(partials, y, no, nb, n_rows, groups, n_wg, bt);   \
+            q4k_reduce_kernel<WAVES, false><<<groups * WAVES, 256, 0, st>>>(partials, sp.nb, sp.total, sp.n_wg, sp.by_total.mul, sp.by_total.shift, sp.by_wg.mul, sp.by_wg.shift, n_rows, no, y, bt); \
         }                                                                                                              \
     } while (0)
     if (waves == 16 && x_type == DFLASH_TYPE_F32)
