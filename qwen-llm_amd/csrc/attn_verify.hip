@@ -898,7 +898,8 @@ __global__ void __launch_bounds__(256)
 // weights need no LDS and no barrier (a wave shuffles them to where they are used), and the only barrier stands between
 // the split lanes' sums and their total: 5.1 -> 3.6 us inside a verify's graph (24 splits, 32 heads of 128, 16 rows).
 // A wave's 64 lanes cover 64 / (HD / 4) split lanes, four dims per lane.
-template <int HD>
+// kEights: eights of splits, by the launch's most.
+template <int HD, int kEights>
 __global__ void __launch_bounds__(HD == 64 ? 128 : 256)
     attn_combine_few_kernel(const float *__restrict__ part_o, const float *__restrict__ part_ml, int64_t ctx_len, int n_q, int n_rows_total, int max_splits,
                             int min_chunk, int want, float *__restrict__ out, void *__restrict__ out_xf, int out_xf_kind, int64_t part_slots,
@@ -915,12 +916,11 @@ __global__ void __launch_bounds__(HD == 64 ? 128 : 256)
     const float2 *ml = reinterpret_cast<const float2 *>(part_ml) + slot0;
     const float *po = part_o + slot0 * HD + 4 * (lane % kLanes);
     const float2 own = ml[min(lane, max_splits - 1) * slot_stride];
-    float4_t o[kSteps][6];
+    float4_t o[kSteps][kEights];
 #pragma unroll
     for (int j = 0; j < kSteps; j++)
 #pragma unroll
-        for (int i = 0; i < 6; i++) {
-            if (8 * i >= max_splits) continue;  // (uniform; a lane past the last split re-reads it)
+        for (int i = 0; i < kEights; i++) {  // (a lane past the last split re-reads it)
             const int s = min(wave * kPerWave + lane / kLanes + j * kPerWave * kWaves + 8 * i, max_splits - 1);
             o[j][i] = *reinterpret_cast<const float4_t *>(po + s * slot_stride * HD);
         }
@@ -937,10 +937,10 @@ __global__ void __launch_bounds__(HD == 64 ? 128 : 256)
         float4_t acc = {0, 0, 0, 0};
         float l = 0.0f;
 #pragma unroll
-        for (int i = 0; i < 6; i++) {
-            if (8 * i >= max_splits) continue;
+        for (int i = 0; i < kEights; i++) {
             const int s = sl + 8 * i;
-            const float w = __shfl(wgt, s, 64), ls = __shfl(own.y, s, 64);
+            float w = __shfl(wgt, s, 64), ls = __shfl(own.y, s, 64);
+            asm volatile("" : "+v"(w), "+v"(ls));  // (read on every path)
             if (s < n_splits) {
                 acc += w * o[j][i];
                 l = __builtin_fmaf(w, ls, l);
@@ -971,7 +971,7 @@ __global__ void __launch_bounds__(HD == 64 ? 128 : 256)
 // (the maximum of the splits before it is a scan over the lanes); a thread adds up one dim, with the factors read from the lane
 // they are in: no LDS, no barrier.
 constexpr int kOrderedSplits = 32;
-template <int HD>
+template <int HD, int kEights>
 __global__ void __launch_bounds__(HD)
     attn_combine_ordered_kernel(const float *__restrict__ part_o, const float *__restrict__ part_ml, int64_t ctx_len, int n_q, int n_rows_total,
                                 int max_splits, int min_chunk, int want, float *__restrict__ out, void *__restrict__ out_xf, int out_xf_kind,
@@ -985,10 +985,9 @@ __global__ void __launch_bounds__(HD)
     const float2 *ml = reinterpret_cast<const float2 *>(part_ml) + slot0;
     const float *po = part_o + slot0 * HD + d;
     const float2 own = ml[min(lane, max_splits - 1) * slot_stride];
-    float o[kOrderedSplits];
+    float o[8 * kEights];
 #pragma unroll
-    for (int s = 0; s < kOrderedSplits; s++) {
-        if ((s & ~7) >= max_splits) continue;  // (uniform; past the last split it is read again)
+    for (int s = 0; s < 8 * kEights; s++) {  // (past the last split it is read again)
         o[s] = po[min(s, max_splits - 1) * slot_stride * HD];
     }
     dfl_have(out, out_xf, out_xf_kind, xf_stride);
@@ -1011,8 +1010,7 @@ __global__ void __launch_bounds__(HD)
     auto at = [](float v, int s) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), s)); };
     float acc = 0.0f, l = 0.0f;
 #pragma unroll
-    for (int s = 0; s < kOrderedSplits; s++) {
-        if ((s & ~7) >= max_splits) continue;
+    for (int s = 0; s < 8 * kEights; s++) {
         if (s < n_splits) {
             const float old = at(w.old, s), next = at(w.next, s);
             acc = __builtin_fmaf(next, o[s], old * acc);
@@ -1427,7 +1425,12 @@ static int32_t attn_rows(dflash_ctx *ctx, const void *q, int32_t q_type, const v
     if (rc) return rc;
     const bool known = n_blocks == 1 && !ctx_len_dev;  // (the number of splits: the one block's)
     if (policy.ordered) {
-        const auto fn = head_dim == 64 ? attn_combine_ordered_kernel<64> : attn_combine_ordered_kernel<128>;
+        typedef decltype(&attn_combine_ordered_kernel<64, 1>) fn_t;
+        static const fn_t fns[2][4] = {
+            {attn_combine_ordered_kernel<64, 1>, attn_combine_ordered_kernel<64, 2>, attn_combine_ordered_kernel<64, 3>, attn_combine_ordered_kernel<64, 4>},
+            {attn_combine_ordered_kernel<128, 1>, attn_combine_ordered_kernel<128, 2>, attn_combine_ordered_kernel<128, 3>, attn_combine_ordered_kernel<128, 4>}};
+        static_assert(kOrderedSplits == 32, "as many eights");
+        const fn_t fn = fns[head_dim == 128][(n_splits - 1) / 8];
         fn<<<dim3(n_q, n_rows, n_blocks), head_dim, 0, st>>>(part_o, part_ml, ctx_len_dev ? -1 : ctx_len, n_q, n_rows_total, n_splits, known ? n_splits : static_cast<int>(min_chunk),
                                                             known ? 0 : want, out, out_xf, out_xf_kind, part_slots,
                                                             dfl_xf_bytes(static_cast<int64_t>(n_q) * head_dim), ctx_len_dev);
@@ -1436,7 +1439,13 @@ static int32_t attn_rows(dflash_ctx *ctx, const void *q, int32_t q_type, const v
     }
     // (more splits than that and the shuffles of the weights cost more than the barriers they replace)
     if (n_splits <= 48) {
-        const auto fn = head_dim == 64 ? attn_combine_few_kernel<64> : head_dim == 128 ? attn_combine_few_kernel<128> : attn_combine_few_kernel<256>;
+        typedef decltype(&attn_combine_few_kernel<64, 1>) fn_t;
+#define DFL_FEW(HD)                                                                                                       \
+    {attn_combine_few_kernel<HD, 1>, attn_combine_few_kernel<HD, 2>, attn_combine_few_kernel<HD, 3>, attn_combine_few_kernel<HD, 4>, \
+     attn_combine_few_kernel<HD, 5>, attn_combine_few_kernel<HD, 6>}
+        static const fn_t fns[3][6] = {DFL_FEW(64), DFL_FEW(128), DFL_FEW(256)};
+#undef DFL_FEW
+        const fn_t fn = fns[head_dim / 128][(n_splits - 1) / 8];
         fn<<<dim3(n_q, n_rows, n_blocks), head_dim == 64 ? 128 : 256, 0, st>>>(part_o, part_ml, ctx_len_dev ? -1 : ctx_len, n_q, n_rows_total, n_splits,
                                                                               known ? n_splits : static_cast<int>(min_chunk), known ? 0 : want, out, out_xf,
                                                                               out_xf_kind, part_slots, dfl_xf_bytes(static_cast<int64_t>(n_q) * head_dim),
