@@ -7,6 +7,8 @@
 #include "device_quant.h"
 #include "sampler_chain.h"
 
+#include <algorithm>
+
 // The walk's scores follow the reference's scalar loop: every product and every addition is
 // rounded on its own: plain operators with contraction switched off (the __f*_rn intrinsics do not
 // stop the compiler from fusing them).
@@ -80,70 +82,137 @@ struct SampledOut {
 // where the raw rows sit in the scores kernel's LDS, behind the decoded ones (bytes)
 __host__ __device__ inline size_t sel_raw_pred_bytes(size_t row_bytes) { return (row_bytes + 15) / 16 * 16; }
 __host__ __device__ inline size_t sel_raw_succ_stride(size_t row_bytes) { return (row_bytes + 3) / 4 * 4; }
-// floats of the decoded rows in front of them: gate[rank], succ[top_k][rank + 1], rounded up to a 16-byte boundary
-__host__ __device__ inline size_t sel_decoded_floats(int top_k, int rank) {
-    return (static_cast<size_t>(rank) + static_cast<size_t>(top_k) * (rank + 1) + 3) / 4 * 4;
-}
+// floats in front of them: gate[rank], products[top_k][sel_prod_stride(rank)], rounded up to a 16-byte boundary
+// (a row of products every stride: the sixteen scoring threads read four of sixteen rows at once, and rows a multiple of 64
+// floats apart would all sit in one bank)
+__host__ __device__ inline int sel_prod_stride(int rank) { return (rank + 3) / 4 * 4 + 4; }
+__host__ __device__ inline size_t sel_gate_floats(int rank) { return (static_cast<size_t>(rank) + 3) / 4 * 4; }
+__host__ __device__ inline size_t sel_decoded_floats(int top_k, int rank) { return sel_gate_floats(rank) + static_cast<size_t>(top_k) * sel_prod_stride(rank); }
 
 // The walk's scores do not have to wait for the walk: the predecessor of position pos is one of the top_k candidates
 // of position pos - 1 (the carry token for pos = 1), so score(pos, a, b) for every candidate a of the previous position
 // and every candidate b of this one is known work up front: (n - 1) x top_k workgroups, all at once, each with the
-// reference's arithmetic for its sixteen scores.  Workgroup (a, pos): all threads dequantise the predecessor row of
-// candidate a and the successor rows of position pos's candidates and form gate = pred * sel_h[pos] in LDS; thread b
-// then scores candidate b with the reference's scalar loop (products and additions rounded separately, rank order):
-// table[pos - 1][a][b] = vals[pos][b] + sum_r gate[r] * succ_b[r], NaN for a candidate without a successor row.  A
-// previous candidate without a predecessor row gets no scores: the walk stops when it picks one.
-__global__ void __launch_bounds__(kSelThreads)
-    dflash2_scores_kernel(Codebook pred_cb, Codebook succ_cb, int top_k, int rank, int carry, int n,
-                          const int32_t *__restrict__ ids, const float *__restrict__ vals, const float *__restrict__ sel_h,
-                          float *__restrict__ table) {
-    extern __shared__ float lds[];  // gate[rank], succ[top_k][rank + 1], then the raw rows: predecessor, top_k successors
-    // (a successor row every rank + 1 floats: the sixteen scoring threads read element r of sixteen rows at once, and rows
-    // a power of two apart would all sit in one bank)
-    float *gate = lds, *succ = lds + rank;
-    const int srow = rank + 1;
-    const int tid = threadIdx.x;
+// reference's arithmetic for its sixteen scores.  Workgroup (a, pos): the predecessor row of candidate a gives gate = pred *
+// sel_h[pos] in LDS, the successor rows of position pos's candidates the products gate[r] * succ_b[r], all elements at once;
+// thread b then adds up candidate b's products as the reference's scalar loop does (products and additions rounded
+// separately, rank order): table[pos - 1][a][b] = vals[pos][b] + sum_r gate[r] * succ_b[r], NaN for a candidate without a
+// successor row.  A previous candidate without a predecessor row gets no scores: the walk stops when it picks one.
+// What bounds it: two trips to memory (the candidates, then their rows) and the sum's chain of `rank` additions.  So a wave
+// takes whole rows, whose bytes it asks for together (an index that is divided into row and word, and the candidate looked up again
+// per word, were 15.7 us a launch; now 6.5), and in Q4_K a thread decodes sixteen elements of two sub-blocks' scales.
+constexpr int kScoreThreads = 512;
+__global__ void __launch_bounds__(kScoreThreads)
+    dflash2_scores_kernel(const int32_t *__restrict__ ids, const uint8_t *__restrict__ pred_rows, const uint8_t *__restrict__ succ_rows,
+                          const float *__restrict__ sel_h, int carry, int top_k, int rank, uint32_t n_pred, uint32_t n_succ, int pred_bytes,
+                          int succ_bytes, int pred_type, int succ_type, const float *__restrict__ vals, float *__restrict__ table) {
+    extern __shared__ float lds[];  // gate, products, then the raw rows: predecessor, top_k successors
+    constexpr int kWaves = kScoreThreads / 64, kRows = kSelMaxTopK / kWaves;  // rows a wave has at most
+    float *gate = lds, *prod = lds + sel_gate_floats(rank);
+    const int ps = sel_prod_stride(rank);
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int a = blockIdx.x, pos = 1 + blockIdx.y;
     if (pos == 1 && a != 0) return;  // (one predecessor only: the carry token)
+    const int32_t cands = ids[pos * top_k + min(lane, top_k - 1)];  // lane b: candidate b
     const int32_t prev = pos == 1 ? carry : ids[(pos - 1) * top_k + a];
-    if (prev < 0 || prev >= pred_cb.n_rows) return;
+    const float *hrow = sel_h + static_cast<size_t>(pos) * rank;
+    float h[kSelMaxRank / kScoreThreads];
+#pragma unroll
+    for (int i = 0; i < kSelMaxRank / kScoreThreads; i++) h[i] = hrow[min(tid + kScoreThreads * i, rank - 1)];
+    dfl_have(vals, table);
+    if (static_cast<uint32_t>(prev) >= n_pred) return;  // (a negative one, too)
     // The rows' bytes come in with coalesced loads first (decoding element by element straight from memory cost a cold
     // trip per field of every element).  Rows of every codebook type are a whole number of 2-byte words and start on
     // one; in LDS the predecessor row sits first and the successor rows follow, each on a 4-byte boundary.
     uint8_t *raw = reinterpret_cast<uint8_t *>(lds + sel_decoded_floats(top_k, rank));
-    const int pw = static_cast<int>(pred_cb.row_bytes / 2), sw = static_cast<int>(succ_cb.row_bytes / 2);
-    const size_t succ_at = sel_raw_pred_bytes(pred_cb.row_bytes), succ_stride = sel_raw_succ_stride(succ_cb.row_bytes);
-    {
-        const uint16_t *src = reinterpret_cast<const uint16_t *>(pred_cb.data + static_cast<size_t>(prev) * pred_cb.row_bytes);
-        for (int i = tid; i < pw; i += kSelThreads) reinterpret_cast<uint16_t *>(raw)[i] = src[i];
+    const int pw = pred_bytes / 2, sw = succ_bytes / 2;
+    const size_t succ_at = sel_raw_pred_bytes(pred_bytes), succ_stride = sel_raw_succ_stride(succ_bytes);
+    bool live[kRows];
+    const uint16_t *src[kRows];
+#pragma unroll
+    for (int i = 0; i < kRows; i++) {
+        const int b = wave + kWaves * i;
+        const int32_t cand = __builtin_amdgcn_readlane(cands, b);
+        live[i] = b < top_k && static_cast<uint32_t>(cand) < n_succ;
+        src[i] = reinterpret_cast<const uint16_t *>(succ_rows + static_cast<size_t>(live[i] ? cand : 0) * succ_bytes);
     }
-    for (int e = tid; e < top_k * sw; e += kSelThreads) {
-        const int b = e / sw, i = e - b * sw;
-        const int32_t cand = ids[pos * top_k + b];
-        if (cand >= 0 && cand < succ_cb.n_rows)
-            reinterpret_cast<uint16_t *>(raw + succ_at + b * succ_stride)[i] =
-                reinterpret_cast<const uint16_t *>(succ_cb.data + static_cast<size_t>(cand) * succ_cb.row_bytes)[i];
+    const uint16_t *psrc = reinterpret_cast<const uint16_t *>(pred_rows + static_cast<size_t>(prev) * pred_bytes);
+    uint16_t p0 = psrc[min(tid, pw - 1)];
+    constexpr int kWords = 3;  // of a lane at once: rows of 384 bytes
+    for (int at = 0; at < sw; at += 64 * kWords) {
+        uint16_t v[kRows][kWords];
+#pragma unroll
+        for (int i = 0; i < kRows; i++)
+#pragma unroll
+            for (int k = 0; k < kWords; k++) v[i][k] = src[i][min(at + lane + 64 * k, sw - 1)];
+#pragma unroll
+        for (int i = 0; i < kRows; i++)
+#pragma unroll
+            for (int k = 0; k < kWords; k++)
+                if (live[i] && at + lane + 64 * k < sw)
+                    reinterpret_cast<uint16_t *>(raw + succ_at + (wave + kWaves * i) * succ_stride)[at + lane + 64 * k] = v[i][k];
     }
+    if (tid < pw) reinterpret_cast<uint16_t *>(raw)[tid] = p0;
+    for (int i = tid + kScoreThreads; i < pw; i += kScoreThreads) reinterpret_cast<uint16_t *>(raw)[i] = psrc[i];
     __syncthreads();
-    Codebook pred_l = pred_cb, succ_l = succ_cb;  // the same rows, now rows of an LDS copy
-    pred_l.data = raw;
-    succ_l.data = raw + succ_at;
-    succ_l.row_bytes = succ_stride;
-    const float *hrow = sel_h + static_cast<size_t>(pos) * rank;
-    for (int r = tid; r < rank; r += kSelThreads) gate[r] = codebook_elem(pred_l, 0, r) * hrow[r];
-    for (int e = tid; e < top_k * rank; e += kSelThreads) {
-        const int b = e / rank, r = e - b * rank;
-        const int32_t cand = ids[pos * top_k + b];
-        if (cand >= 0 && cand < succ_cb.n_rows) succ[b * srow + r] = codebook_elem(succ_l, b, r);
+    Codebook pred_l = {pred_type, rank, 1, raw, static_cast<size_t>(pred_bytes)}, succ_l = {succ_type, rank, top_k, raw + succ_at, succ_stride};
+#pragma unroll
+    for (int i = 0; i < kSelMaxRank / kScoreThreads; i++)
+        if (tid + kScoreThreads * i < rank) gate[tid + kScoreThreads * i] = codebook_elem(pred_l, 0, tid + kScoreThreads * i) * h[i];
+    __syncthreads();
+    if (succ_type == DFLASH_TYPE_Q4_K) {
+        // eight bytes of quants a thread: eight elements of sub-block 2 p, eight of 2 p + 1 (dfl_dequant_elem's arithmetic)
+        const int per_row = rank / 16;  // (a multiple of sixteen)
+#pragma unroll
+        for (int i = 0; i < kRows; i++) {
+            if (!live[i]) continue;
+            const int b = wave + kWaves * i;
+            for (int c = lane; c < per_row; c += 64) {
+                const int sb = c >> 4, p = (c >> 2) & 3, l0 = (c & 3) * 8;
+                const uint8_t *blk = raw + succ_at + b * succ_stride + sb * DFL_Q4_K_BYTES;
+                const uint2 q = *reinterpret_cast<const uint2 *>(blk + 16 + 32 * p + l0);
+                float d1[2], m1[2];
+#pragma unroll
+                for (int u = 0; u < 2; u++) {
+                    int sc, m;
+                    dfl_q4k_scale_min(blk + 4, 2 * p + u, &sc, &m);
+                    d1[u] = __fmul_rn(dfl_h2f(blk), static_cast<float>(sc));
+                    m1[u] = __fmul_rn(dfl_h2f(blk + 2), static_cast<float>(m));
+                }
+                const int r0 = 256 * sb + 64 * p + l0;
+#pragma unroll
+                for (int u = 0; u < 2; u++)
+#pragma unroll
+                    for (int k = 0; k < 8; k++) {
+                        const uint32_t word = k < 4 ? q.x : q.y;
+                        const float e = __fsub_rn(__fmul_rn(d1[u], static_cast<float>((word >> (8 * (k & 3) + 4 * u)) & 15)), m1[u]);
+                        prod[b * ps + r0 + 32 * u + k] = gate[r0 + 32 * u + k] * e;
+                    }
+            }
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < kRows; i++) {
+            if (!live[i]) continue;
+            const int b = wave + kWaves * i;
+            for (int r = lane; r < rank; r += 64) prod[b * ps + r] = gate[r] * codebook_elem(succ_l, b, r);
+        }
     }
     __syncthreads();
     if (tid < top_k) {
-        const int32_t cand = ids[pos * top_k + tid];
         float sc = __builtin_nanf("");  // skipped candidates never compare greater
-        if (cand >= 0 && cand < succ_cb.n_rows) {
+        if (static_cast<uint32_t>(cands) < n_succ) {
             float dot = 0.0f;
-            const float *sr = succ + tid * srow;
-            for (int r = 0; r < rank; r++) dot += gate[r] * sr[r];  // two roundings each (contraction is off in this file)
+            const float *pr = prod + tid * ps;
+            int r = 0;
+#pragma unroll 8
+            for (; r + 4 <= rank; r += 4) {  // (every product and every sum rounded on its own: contraction is off in this file)
+                const float4 v = *reinterpret_cast<const float4 *>(pr + r);
+                dot += v.x;
+                dot += v.y;
+                dot += v.z;
+                dot += v.w;
+            }
+            for (; r < rank; r++) dot += pr[r];
             sc = vals[pos * top_k + tid] + dot;
         }
         table[(static_cast<size_t>(pos - 1) * top_k + a) * top_k + tid] = sc;
@@ -161,6 +230,7 @@ __global__ void __launch_bounds__(kSelThreads)
                           float temperature, const double *__restrict__ uniforms, SampledOut *__restrict__ sampled) {
     __shared__ float table_s[15 * kSelMaxTopK * kSelMaxTopK];
     __shared__ int32_t ids_s[16 * kSelMaxTopK];
+    __shared__ __attribute__((aligned(16))) uint8_t next_s[16][16];
     __shared__ RowDist dist;
     const int tid = threadIdx.x;
     if (tid == 0) {
@@ -178,37 +248,55 @@ __global__ void __launch_bounds__(kSelThreads)
         if (tid == 0) *status = 1;
         return;
     }
-    for (int e = tid; e < (n - 1) * top_k * top_k; e += kSelThreads) table_s[e] = table[e];
-    for (int e = tid; e < n * top_k; e += kSelThreads) ids_s[e] = ids[e];
+    {
+        const int n_table = (n - 1) * top_k * top_k;
+        float t[15];
+#pragma unroll
+        for (int i = 0; i < 15; i++) t[i] = table[min(tid + kSelThreads * i, n_table - 1)];
+        const int32_t id = ids[min(tid, n * top_k - 1)];
+#pragma unroll
+        for (int i = 0; i < 15; i++)
+            if (tid + kSelThreads * i < n_table) table_s[tid + kSelThreads * i] = t[i];
+        if (tid < n * top_k) ids_s[tid] = id;
+    }
     __syncthreads();
     if (!SAMPLED) {
-        // greedy: lane b holds candidate b of the position; the first strict maximum over the candidates with a successor
-        // row, as the scalar loop `if (score[b] > best)` from best = -inf keeps it (a NaN or -inf score is never greater:
-        // with none greater, candidate 0 stands)
-        if (tid >= 64) return;
-        int prev_a = 0;
+        // greedy.  Which candidate follows candidate a of the position before is known for every (position, a) without the walk: the
+        // first strict maximum over the candidates with a successor row, as the scalar loop `if (score[b] > best)` from best =
+        // -inf keeps it (a NaN or -inf score is never greater: with none greater, candidate 0 stands).  Sixteen lanes a
+        // previous candidate find it for all positions (the maximum crosses them by DPP moves), and the walk itself
+        // is a look-up per position out of scalar registers.  (A maximum over shuffles per position, one after the other: 9.7 us
+        // a launch; now 6.1.)
+        const int b = tid & 15, a = tid >> 4;  // (256 threads: sixteen previous candidates)
         for (int pos = 1; pos < n; pos++) {
-            float sc = -INFINITY;
-            int32_t cand = -1;
-            if (tid < top_k) {
-                cand = ids_s[pos * top_k + tid];
-                const float v = table_s[(static_cast<size_t>(pos - 1) * top_k + prev_a) * top_k + tid];
-                if (cand >= 0 && cand < n_succ_rows && v > -INFINITY) sc = v;
-            }
+            const int32_t cand = b < top_k ? ids_s[pos * top_k + b] : -1;
+            const float v = b < top_k && a < top_k ? table_s[(static_cast<size_t>(pos - 1) * top_k + a) * top_k + b] : -INFINITY;
+            const float sc = cand >= 0 && cand < n_succ_rows && v > -INFINITY ? v : -INFINITY;
             float best = sc;
-#pragma unroll
-            for (int off = 1; off < 16; off <<= 1) best = fmaxf(best, __shfl_xor(best, off, 64));
-            best = __shfl(best, 0, 64);  // (lanes 0..15 agree; the others hold -inf)
-            const unsigned long long at = __ballot(tid < top_k && sc == best && best > -INFINITY);
-            const int best_b = at ? __builtin_ctzll(at) : 0;
-            const int32_t chosen = __shfl(cand, best_b, 64);
-            if (tid == 0) out[pos] = chosen;
-            if (chosen < 0 || chosen >= n_pred_rows) {
-                if (tid == 0) *status = 1;
-                return;
-            }
-            prev_a = best_b;
+            best = fmaxf(best, dfl_dpp<0x128>(best));  // row_ror:8, 4, 2, 1
+            best = fmaxf(best, dfl_dpp<0x124>(best));
+            best = fmaxf(best, dfl_dpp<0x122>(best));
+            best = fmaxf(best, dfl_dpp<0x121>(best));
+            const unsigned long long at = __ballot(sc == best && best > -INFINITY);
+            const uint32_t mine = static_cast<uint32_t>(at >> (16 * (a & 3))) & 0xffffu;
+            if (b == 0) next_s[pos][a] = static_cast<uint8_t>(mine ? __builtin_ctz(mine) : 0);
         }
+        __syncthreads();
+        if (tid >= 64) return;
+        const uint4 next = *reinterpret_cast<const uint4 *>(next_s[min(tid, 15)]);  // lane pos: the sixteen of a position
+        int picked = 0, prev_a = 0;  // lane pos: its pick
+        for (int pos = 1; pos < n; pos++) {
+            const uint32_t w = prev_a < 8 ? (prev_a < 4 ? __builtin_amdgcn_readlane(next.x, pos) : __builtin_amdgcn_readlane(next.y, pos))
+                                          : (prev_a < 12 ? __builtin_amdgcn_readlane(next.z, pos) : __builtin_amdgcn_readlane(next.w, pos));
+            prev_a = w >> (8 * (prev_a & 3)) & 255;
+            picked = tid == pos ? prev_a : picked;
+        }
+        // the walk ends behind the first pick without a predecessor row
+        const int32_t chosen = tid >= 1 && tid < n ? ids_s[tid * top_k + picked] : 0;
+        const unsigned long long bad = __ballot(tid >= 1 && tid < n && (chosen < 0 || chosen >= n_pred_rows));
+        const int last = bad ? __builtin_ctzll(bad) : n - 1;
+        if (tid >= 1 && tid <= last) out[tid] = chosen;
+        if (bad && tid == 0) *status = 1;
         return;
     }
     if (tid != 0) return;
@@ -217,17 +305,7 @@ __global__ void __launch_bounds__(kSelThreads)
         const float *score = table_s + (static_cast<size_t>(pos - 1) * top_k + prev_a) * top_k;
         const int32_t *cands = ids_s + pos * top_k;
         int best_b = 0;
-        if (!SAMPLED) {
-            float best = -INFINITY;
-            for (int b = 0; b < top_k; b++) {
-                const int32_t cand = cands[b];
-                if (cand < 0 || cand >= n_succ_rows) continue;
-                if (score[b] > best) {
-                    best = score[b];
-                    best_b = b;
-                }
-            }
-        } else {
+        {
             // scores of skipped candidates are -inf; the "tokens" of the distribution are candidate indices
             uint64_t keys[kSelMaxTopK];
             int nan_at = -1;
@@ -303,7 +381,10 @@ int32_t launch_walk(dflash_ctx *ctx, size_t *ws_off, const Codebook &pc, const C
         if (lds > 48 * 1024) {
             if (const int32_t rc_ = dfl_raise_lds_limit(ctx, reinterpret_cast<const void *>(dflash2_scores_kernel), lds)) return rc_;
         }
-        dflash2_scores_kernel<<<dim3(top_k, n - 1), kSelThreads, lds, st>>>(pc, sc, top_k, rank, carry, n, ids, vals, sel_h, table);
+        auto rows = [](int64_t n_rows) { return static_cast<uint32_t>(std::min<int64_t>(n_rows, int64_t(1) << 31)); };  // (tokens are below 2^31)
+        dflash2_scores_kernel<<<dim3(top_k, n - 1), kScoreThreads, lds, st>>>(ids, pc.data, sc.data, sel_h, carry, top_k, rank, rows(pc.n_rows),
+                                                                             rows(sc.n_rows), static_cast<int>(pc.row_bytes),
+                                                                             static_cast<int>(sc.row_bytes), pc.type, sc.type, vals, table);
     }
     dflash2_select_kernel<SAMPLED><<<1, kSelThreads, 0, st>>>(pc.n_rows, sc.n_rows, top_k, carry, n, ids, table, out, status, temperature,
                                                                uniforms, sampled);
