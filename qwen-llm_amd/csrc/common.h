@@ -293,6 +293,13 @@ bool dfl_q4k_tiled_split(const dflash_ctx *ctx, int64_t n_in, int64_t n_out, int
 int32_t dfl_dflash2_conv(dflash_ctx *ctx, const float *x, const float *dyn, const float *base, float *y, int32_t n_tokens, int32_t h,
                          int32_t kernel_size, int32_t group_size, int32_t side, dflash_stream_t stream, void *y_xf, int y_xf_kind);
 
+// A DFlash-2 sublayer's coefficient projection (a tiled Q4_K matrix whose rows are in fragment order at xf) and its side-0
+// convolution in one launch: the convolved rows to y_xf in fragment order (which must not overlap xf), side 1's coefficients to dyn, whose
+// side 0 is left as it is.  The bits of dfl_gemm_whole followed by dfl_dflash2_conv.
+bool dfl_gemm_conv_takes(const dflash_ctx *ctx, int32_t w_type, int64_t h, int32_t kernel_size, int32_t group_size, int32_t y_xf_kind);
+int32_t dfl_gemm_conv(dflash_ctx *ctx, const void *w, const void *xf, const float *x, const float *base, int64_t h, int32_t group_size, int32_t n_rows,
+                      float *dyn, void *y_xf, int y_xf_kind, hipStream_t stream);
+
 // Device scratch of the mixture-of-experts FFN (owned by the target session).
 struct dfl_moe_scratch {
     float *probs = nullptr;   // [16][n_expert] router logits

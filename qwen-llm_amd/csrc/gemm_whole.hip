@@ -632,6 +632,78 @@ __global__ void __launch_bounds__(1024) gemm_whole_kernel(DFL_WHOLE_PARAMS) {
     }
 }
 
+// A DFlash-2 sublayer's coefficient projection and its side-0 convolution (kernel size 2) as one launch: dyn[row][side][tap][group] =
+// row . W^T as gemm_whole_kernel has it, then y[row][c] = sum_tap (base[0][tap][c] + dyn[row][0][tap][c / group_size]) * x[row - tap][c] as
+// dflash2_conv_kernel has it, in fragment order for the projection that reads it.  Workgroup (part, j), j < n_groups / 16: the
+// coefficients of groups 16 j .. + 15 for both taps (two tiles, its waves share K), then the convolution of 256 of their channels
+// (every part computes the coefficients again: 64 KB of rows and two tiles of weights out of L2).  Behind those, part 0 of j >= n_groups / 16
+// stores two tiles of side 1, which the norm that adds the sublayer's result reads (side 0's go nowhere else).
+// What bounds it: the product's launch; the convolution's operands arrive under it.  4.8 + 3.4 us as two launches, 5.9 now
+// (CONVNEW).
+__global__ void __launch_bounds__(1024)
+    gemm_conv_kernel(const uint8_t *w, const uint8_t *xf, const float *x, const float *base, int nb, int n_groups, uint32_t by_group, int group_size,
+                     int n_rows, int n_waves, float *dyn, uint8_t *y_xf, int y_xf_kind) {
+    __shared__ float4_t red[16 * 64];
+    __shared__ float coef[2][16][16];  // [tap][row][group]
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n = lane & 15, g = lane >> 4, jj = n_groups >> 4, h = nb * DFL_QK_K;
+    const int half = wave >= nb, kslice = half ? wave - nb : wave;
+    const bool conv = static_cast<int>(blockIdx.y) < jj;
+    if (!conv && blockIdx.x) return;
+    const int tile = conv ? half * jj + blockIdx.y : 2 * jj + 2 * (blockIdx.y - jj) + half;
+    WholeArgs a = {};
+    a.w = w;
+    a.nb = nb;
+    Q4W wt;
+    load_w(wt, a, tile, kslice, lane);
+    half8_t af[8];
+    load_xf(af, xf, kslice, lane);
+    // the convolution's operands of this wave's first row: four channels a lane
+    const int c0 = 256 * blockIdx.x + 4 * lane, c = conv ? 16 * group_size * blockIdx.y + c0 : 0, t0 = min(wave, n_rows - 1);
+    float4_t b0 = {0, 0, 0, 0}, b1 = b0, x0 = b0, x1 = b0;
+    if (conv) {
+        b0 = *reinterpret_cast<const float4_t *>(base + c);
+        b1 = *reinterpret_cast<const float4_t *>(base + h + c);
+        x0 = *reinterpret_cast<const float4_t *>(x + static_cast<size_t>(t0) * h + c);
+        x1 = *reinterpret_cast<const float4_t *>(x + static_cast<size_t>(max(t0 - 1, 0)) * h + c);
+    }
+    dfl_have(dyn, y_xf, y_xf_kind);
+    float4_t acc = {0, 0, 0, 0}, acc_sub = {0, 0, 0, 0};
+    compute(wt, af, lane, nullptr, (lane & 16) ? 0x04030402u : 0x04010400u, q4k_magic(), acc, acc_sub);
+    red[wave * 64 + lane] = acc - acc_sub;
+    __syncthreads();
+    if (kslice == 0) {
+        float4_t sum = red[wave * 64 + lane];
+        for (int s = 1; s < nb; s++) sum += red[(wave + s) * 64 + lane];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int row = 4 * g + i;
+            if (conv)
+                coef[half][row][n] = sum[i];
+            else if (row < n_rows)
+                dyn[static_cast<size_t>(row) * (4 * n_groups) + tile * 16 + n] = sum[i];
+        }
+    }
+    if (!conv) return;
+    __syncthreads();
+    const int grp = static_cast<int>(__umulhi(c0, by_group));  // c0 / group_size
+    for (int t = wave; t < n_rows; t += n_waves) {
+        if (t != wave) {
+            x0 = *reinterpret_cast<const float4_t *>(x + static_cast<size_t>(t) * h + c);
+            x1 = *reinterpret_cast<const float4_t *>(x + static_cast<size_t>(t - 1) * h + c);
+        }
+        const float d0 = coef[0][t][grp], d1 = coef[1][t][grp];
+        float4_t y;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            y[e] = __builtin_fmaf(b0[e] + d0, x0[e], 0.0f);
+            if (t) y[e] = __builtin_fmaf(b1[e] + d1, x1[e], y[e]);
+        }
+        dfl_xf_store_pair(y_xf, y_xf_kind, t, c & ~7, y[0], y[1], y[2], y[3]);
+    }
+}
+
 // The same product for a matrix of many more tiles than one round of the chip (an output head: 151936 rows), K of at
 // most 16 super-blocks: a workgroup walks units blockIdx.x * tl + tlane, + gridDim.x * tl, ...  A wave's K slice is
 // the same super-block in every unit, so its eight activation fragments are loaded ONCE and stay in registers; the
@@ -1090,6 +1162,30 @@ int32_t dfl_gemm_whole_blocks(dflash_ctx *ctx, int32_t w_type, const void *w, co
         if (const int32_t rc = dfl_raise_lds_limit(ctx, reinterpret_cast<const void *>(fn), lds)) return rc;
     dfl_timed timer(ctx, st, DFL_T_GEMM);
     whole_launch(fn, p.n_wg, threads, lds, st, a);
+    DFL_HIP_CHECK(ctx, hipGetLastError());
+    return DFLASH_OK;
+}
+
+bool dfl_gemm_conv_takes(const dflash_ctx *ctx, int32_t w_type, int64_t h, int32_t kernel_size, int32_t group_size, int32_t y_xf_kind) {
+    if (w_type != DFLASH_TYPE_Q4_K_TILED || y_xf_kind == DFL_XF_NONE || kernel_size != 2 || h < 256 || h % 256 || h > 8 * DFL_QK_K) return false;
+    if (group_size < 16 || group_size % 16 || h % group_size || (h / group_size) % 16) return false;
+    return whole_plan(ctx, w_type, h, 4 * (h / group_size), 0).kind == DFL_XF_Q4K;
+}
+
+int32_t dfl_gemm_conv(dflash_ctx *ctx, const void *w, const void *xf, const float *x, const float *base, int64_t h, int32_t group_size, int32_t n_rows,
+                      float *dyn, void *y_xf, int y_xf_kind, hipStream_t st) {
+    if (!dfl_gemm_conv_takes(ctx, DFLASH_TYPE_Q4_K_TILED, h, 2, group_size, y_xf_kind) || n_rows < 1 || n_rows > 16)
+        return dfl_fail(ctx, DFLASH_ERR_UNSUPPORTED, "gemm_conv: %lld channels in groups of %d, %d rows", static_cast<long long>(h), group_size, n_rows);
+    if (!w || !xf || !x || !base || !dyn || !y_xf) return dfl_fail(ctx, DFLASH_ERR_INVALID_INPUT, "gemm_conv: null pointer");
+    for (const void *p : {w, xf, static_cast<const void *>(x), static_cast<const void *>(base), static_cast<const void *>(y_xf)})
+        if (reinterpret_cast<uintptr_t>(p) % 16) return dfl_fail(ctx, DFLASH_ERR_ALIGNMENT, "gemm_conv: operand alignment");
+    if (dfl_ranges_overlap(xf, dfl_xf_bytes(h), y_xf, dfl_xf_bytes(h))) return dfl_fail(ctx, DFLASH_ERR_ALIAS, "gemm_conv: the result overlaps the rows");
+    const int nb = static_cast<int>(h / DFL_QK_K), groups = static_cast<int>(h / group_size);
+    const uint32_t by_group = static_cast<uint32_t>(((1ull << 32) + group_size - 1) / group_size);  // (exact for channels below 16 group_size <= h <= 2048)
+    dfl_timed timer(ctx, st, DFL_T_GEMM);
+    gemm_conv_kernel<<<dim3(16 * group_size / 256, 2 * (groups / 16)), 128 * nb, 0, st>>>(
+        static_cast<const uint8_t *>(w), static_cast<const uint8_t *>(xf), x, base, nb, groups, by_group, group_size, n_rows, 2 * nb, dyn,
+        static_cast<uint8_t *>(y_xf), y_xf_kind);
     DFL_HIP_CHECK(ctx, hipGetLastError());
     return DFLASH_OK;
 }

@@ -1921,13 +1921,25 @@ int32_t draft_block_impl(dflash_ctx *ctx, const dflash_model *target, const dfla
         // the convolution then writes q/k/v's over them, later in the stream)
         const int cp_attn = conv && fast ? dfl_whole_kind(ctx, L.conv_attn_proj.type, H, conv_dyn_dim, 0) : DFL_XF_NONE;
         const int cp_ffn = conv && fast ? dfl_whole_kind(ctx, L.conv_ffn_proj.type, H, conv_dyn_dim, 0) : DFL_XF_NONE;
+        // (where both are one launch, the norm's rows for the coefficients sit in conv_buf, which nothing else uses then: the
+        // launch writes q/k/v's rows while other workgroups still read them)
+        auto one_launch = [&](int cp, const dflash_qtensor &proj, const float *base, int kind) {
+            return cp && conv_in_norm && reinterpret_cast<uintptr_t>(base) % 16 == 0 &&
+                   dfl_gemm_conv_takes(ctx, proj.type, H, c.conv_kernel_size, c.conv_group_size, kind);
+        };
+        const bool one_attn = one_launch(cp_attn, L.conv_attn_proj, L.conv_attn_base, s->pk ? xk.qkv : DFL_XF_NONE);
+        const bool one_ffn = one_launch(cp_ffn, L.conv_ffn_proj, L.conv_ffn_base, xk.gate_up);
         const int norm1_kind = conv ? cp_attn : xk.qkv;
         rms_norm(N, st, s->x, pending_resid, L.attn_norm, s->cur, H, c.eps, nullptr, nullptr,
-                                           norm1_kind ? s->xf_cur : nullptr, norm1_kind, 0, pending_conv);
+                 norm1_kind ? (one_attn ? reinterpret_cast<uint8_t *>(s->conv_buf) : s->xf_cur) : nullptr, norm1_kind, 0, pending_conv);
         // DFlash-2 attention convolution (metal_dflash.rs:16210-16262): the dynamic coefficients come
         // from the normed input and serve both sides; q/k/v read the side-0 result
         const float *attn_src = s->cur;
-        if (conv) {
+        if (one_attn) {
+            if ((rc = dfl_gemm_conv(ctx, L.conv_attn_proj.data, s->conv_buf, s->cur, L.conv_attn_base, H, c.conv_group_size, N, s->conv_dyn, s->xf_cur,
+                                    xk.qkv, st)))
+                return rc;
+        } else if (conv) {
             rc = cp_attn ? dfl_gemm_whole(ctx, L.conv_attn_proj.type, L.conv_attn_proj.data, s->xf_cur, s->conv_dyn, H, conv_dyn_dim, N, 0,
                                           nullptr, DFL_XF_NONE, st)
                          : gemm(ctx, L.conv_attn_proj, s->cur, s->conv_dyn, H, conv_dyn_dim, N, st);
@@ -1980,9 +1992,13 @@ int32_t draft_block_impl(dflash_ctx *ctx, const dflash_model *target, const dfla
         }
         const int norm2_kind = conv ? cp_ffn : xk.gate_up;
         rms_norm(N, st, s->x, resid, L.post_norm, s->cur, H, c.eps, nullptr, nullptr,
-                                           norm2_kind ? s->xf_cur : nullptr, norm2_kind, 0, resid_conv);
+                 norm2_kind ? (one_ffn ? reinterpret_cast<uint8_t *>(s->conv_buf) : s->xf_cur) : nullptr, norm2_kind, 0, resid_conv);
         const float *ffn_src = s->cur;
-        if (conv) {  // the FFN pair (:16836-16885, 17003-17022)
+        if (one_ffn) {
+            if ((rc = dfl_gemm_conv(ctx, L.conv_ffn_proj.data, s->conv_buf, s->cur, L.conv_ffn_base, H, c.conv_group_size, N, s->conv_dyn, s->xf_cur,
+                                    xk.gate_up, st)))
+                return rc;
+        } else if (conv) {  // the FFN pair (:16836-16885, 17003-17022)
             rc = cp_ffn ? dfl_gemm_whole(ctx, L.conv_ffn_proj.type, L.conv_ffn_proj.data, s->xf_cur, s->conv_dyn, H, conv_dyn_dim, N, 0,
                                          nullptr, DFL_XF_NONE, st)
                         : gemm(ctx, L.conv_ffn_proj, s->cur, s->conv_dyn, H, conv_dyn_dim, N, st);
