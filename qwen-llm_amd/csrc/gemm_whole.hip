@@ -638,8 +638,7 @@ __global__ void __launch_bounds__(1024) gemm_whole_kernel(DFL_WHOLE_PARAMS) {
 // coefficients of groups 16 j .. + 15 for both taps (two tiles, its waves share K), then the convolution of 256 of their channels
 // (every part computes the coefficients again: 64 KB of rows and two tiles of weights out of L2).  Behind those, part 0 of j >= n_groups / 16
 // stores two tiles of side 1, which the norm that adds the sublayer's result reads (side 0's go nowhere else).
-// What bounds it: the product's launch; the convolution's operands arrive under it.  4.8 + 3.4 us as two launches, 5.9 now
-// (CONVNEW).
+// What bounds it: the product's launch; the convolution's operands arrive under it.  4.8 + 3.4 us as two launches, 6.2 now.
 __global__ void __launch_bounds__(1024)
     gemm_conv_kernel(const uint8_t *w, const uint8_t *xf, const float *x, const float *base, int nb, int n_groups, uint32_t by_group, int group_size,
                      int n_rows, int n_waves, float *dyn, uint8_t *y_xf, int y_xf_kind) {

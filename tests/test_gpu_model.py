@@ -396,6 +396,41 @@ def test_dflash2_identity_convolutions_equal_dflash1_on_the_device(ctx, target):
     assert np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32))
 
 
+@pytest.mark.parametrize("hidden,group,block", [(256, 16, 1), (1024, 64, 8), (1024, 16, 16), (2048, 64, 16)])
+def test_dflash2_coefficients_and_convolution_in_one_launch(ctx, hidden, group, block):
+    """Base kernels at a 16-byte boundary let a sublayer's coefficients and its side-0 convolution go out as one launch; four bytes
+    further on they are two.  Same products, same taps in the same order: the logits are the same bits.  Over the narrowest and the
+    widest stream the launch takes, one and several tiles of a wave's groups, and blocks of one row, some rows and all."""
+    import torch
+
+    tcfg = dfl.ModelConfig(n_layers=1, hidden=hidden, n_q=4, n_kv=2, head_dim=128, ffn=512, vocab=2048)
+    dcfg = dfl.DraftConfig(n_layers=2, hidden=hidden, n_q=4, n_kv=2, head_dim=128, ffn=512, block_size=block, n_taps=2,
+                           conv_kernel_size=2, conv_group_size=group)
+    model = dfl.TargetModel(ctx, tcfg, dfl.synth_target_weights(tcfg, seed=3))
+    dw = dfl.synth_draft_weights(dcfg, seed=4)
+    toks = np.random.default_rng(5).integers(0, tcfg.vocab, 16).tolist()
+    got, shifted = [], []
+    for shift in (0, 1):
+        head = dfl.DraftHead(ctx, dcfg, dw)
+        for L, Lw in zip(head._layers, dw["layers"]):
+            for name in ("conv_attn_base", "conv_ffn_base"):
+                flat = torch.from_numpy(Lw[name]).reshape(-1)
+                buf = torch.zeros(flat.numel() + 1, device="cuda")
+                buf[shift:shift + flat.numel()] = flat.cuda()
+                shifted.append(buf)
+                setattr(L, name, buf.data_ptr() + 4 * shift)
+        sess = dfl.Session(ctx, model, 64, [0, 0])
+        dsess = dfl.DraftSession(ctx, head, model, 64)
+        out = sess.encode_packed_verify_layer_major(toks, 0)
+        dsess.append_target_ctx_columns(out.hidden_capture, list(range(16)))
+        _, logits, _ = dsess.draft_block(11, tcfg.vocab - 1, 16, want_logits=True)
+        got.append(logits.cpu().numpy())
+        dsess.close()
+        sess.close()
+    assert np.all(np.isfinite(got[0])) and np.ptp(got[0]) > 0
+    assert np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32))
+
+
 MOE_CASES = {
     # hidden 512: 16 sub-blocks per row (half-wave rows); hidden 2048 / F_exp 768: the end-to-end shape's widths
     "small": dfl.ModelConfig(n_layers=2, hidden=512, n_q=8, n_kv=2, head_dim=64, ffn=0, vocab=4096, n_expert=16,
