@@ -13,13 +13,14 @@
 //    workgroups cover the chip in one round; each workgroup streams its chunk once with coalesced loads;
 //  * order decisions use the reference's integer keys (descending f32 total order above ascending
 //    token id), so the selected candidates and their order are exact, not approximately sorted;
-//  * top-k of a chunk: the k-th best of the 1024 per-thread bests bounds every winner, so only the elements of the
-//    k winning threads are ranked; ranks come from counting (keys are distinct), not from sorting networks in LDS,
-//    whose every step is a workgroup barrier;
+//  * top-k of a chunk: a bound per wave on its share of the winners, the largest of those on all of them; only what is
+//    below it is ranked, by counting (keys are distinct), not by sorting networks in LDS, whose every step is a workgroup barrier;
 //  * everything that feeds a comparison with a uniform draw is f64 and added in the order of the reference's
 //    loops; what is independent per candidate (conversions, exponentials) is done a candidate per lane;
-//  * a block with dense draft proposals is three launches: selection of both logit tensors, the rows' chains
-//    together with the draft rows' tile sums, the decision (written straight to pinned host memory).
+//  * a block with dense draft proposals is three launches: selection of both logit tensors, the rows' chains with their
+//    draws and draft weights together with the draft rows' tile sums, the decision (written straight to pinned host memory): 7.2 + 9.3 +
+//    5.3 us at 16 rows of 151936 and k = 20 (14.3 + 13.1 + 13.2 with a digit search per chunk, a barrier per tree level and the
+//    walk's scans in one wave; the whole call 57 -> 39 us).
 #include "common.h"
 #include "sampler_chain.h"
 #include "accept_select.h"
@@ -103,273 +104,345 @@ __global__ void top2_final_kernel(const Top2 *__restrict__ part, int n_chunks, i
 // ------------------------------------------------------------------------------------------
 // chunk selection: best K keys of a chunk (sorted), lowest NaN index, optional second row set
 // ------------------------------------------------------------------------------------------
-struct ChunkOut {
-    uint64_t keys[kMaxK];
-    int32_t nan_first;
-    int32_t pad;
-};
+// A chunk's list is k keys, ascending, at out[(row * n_chunks + chunk) * k], filled up with kNoKey.  A chunk with a NaN has
+// the lowest NaN's token id, with nothing above it, as its first key: that is below every candidate's key (only a NaN's
+// bits order as 0), so the least key of a row says whether it holds a NaN and which.
+__device__ __forceinline__ bool key_is_nan(uint64_t key) { return (key >> 32) == 0; }
 
-// min over the workgroup of a key / an int, result broadcast
-__device__ uint64_t block_min_u64(uint64_t v, uint64_t *sh) {
-    for (int off = 32; off > 0; off >>= 1) {
-        uint64_t o = __shfl_xor(v, off, 64);
-        v = o < v ? o : v;
-    }
+// min over the workgroup of a key, result in the first wave
+__device__ __forceinline__ uint64_t block_min_u64(uint64_t v, uint64_t *sh) {
+    const int lane = threadIdx.x & 63, n_waves = blockDim.x >> 6;
+    v = wave_min_u64(v);
+    if (lane == 0) sh[threadIdx.x >> 6] = v;
     __syncthreads();
-    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
-    __syncthreads();
-    uint64_t r = sh[0];
-    for (int w = 1; w < static_cast<int>(blockDim.x >> 6); w++) r = sh[w] < r ? sh[w] : r;
-    return r;
+    return threadIdx.x < 64 ? wave_min_u64(lane < n_waves ? sh[lane] : kNoKey) : kNoKey;
 }
 
-// below[j] = number of keys below x[j] in the ascending list of 1 <= n <= kMaxK keys at base + off[j], four binary
-// searches in lockstep: a probe is an LDS read the next one depends on, and a thread that runs its searches one
-// after the other spends its time waiting for them.  step0 = the largest power of two <= n.
-__device__ __forceinline__ void count_below4(const uint64_t *base, const int (&off)[4], int n, int step0, const uint64_t (&x)[4],
-                                             int (&below)[4]) {
+// A chunk's tokens j * kSelThreads + tid, all asked for at once (past the vocabulary: its last token again).
+constexpr int kSelPer = kSelChunk / kSelThreads;
+__device__ __forceinline__ void load_chunk(const float *__restrict__ x, int vocab, int base, float (&v)[kSelPer]) {
 #pragma unroll
-    for (int j = 0; j < 4; j++) below[j] = 0;
-    for (int step = step0; step >= 1; step >>= 1) {
-        uint64_t v[4];
-        int probe[4];
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            probe[j] = below[j] + step;
-            v[j] = base[off[j] + (probe[j] <= n ? probe[j] : n) - 1];
-        }
-#pragma unroll
-        for (int j = 0; j < 4; j++) below[j] = (probe[j] <= n && v[j] < x[j]) ? probe[j] : below[j];
-    }
+    for (int j = 0; j < kSelPer; j++) v[j] = x[min(base + j * kSelThreads, vocab - 1)];
 }
 
-// K == 1 fast path is the greedy / draft-max case: only the minimum key is needed.
-//
-// K > 1, without a sort: the k-th best of the 1024 per-thread bests bounds every winner of the chunk (block_kth); the at
-// most 16 k elements at or below that bound are then ranked by counting the candidates below each, and a candidate of
-// rank r < k is output r.  Keys are distinct (the token id is in the low bits), so ranks are too.  (The bound by sorting
-// every wave's bests between its lanes and merging the sixteen lists was 21 rounds of shuffles through LDS and k
-// dependent steps: 16.8 -> 14.6 us for 31 rows of 151936, k = 20 on 16 of them.)
-__device__ __forceinline__ void select_chunk_body(const float *__restrict__ logits, int64_t vocab, int64_t stride, int k,
-                                                  ChunkOut *__restrict__ out, bool nan_is_candidate, int row) {
-    constexpr int kMaxCand = (kSelChunk / kSelThreads) * kMaxK;
-    __shared__ uint64_t cand[kMaxCand];
-    __shared__ uint64_t outk[kMaxK];
-    __shared__ KthShared<kSelThreads> kth;
-    __shared__ int rank_sh[kMaxCand];
-    __shared__ int cnt;
-    __shared__ int nan_sh;
-    const int chunk = blockIdx.x, tid = threadIdx.x;
-    const float *x = logits + row * stride;
-    uint64_t keys[kSelChunk / kSelThreads];
+// the best key alone: greedy targets, and the largest logit of a draft row
+__device__ __forceinline__ void best_of_chunk(const float *__restrict__ x, int vocab, uint64_t *__restrict__ out) {
+    __shared__ uint64_t red[kSelThreads / 64];
+    const int base = blockIdx.x * kSelChunk + threadIdx.x;
+    float v[kSelPer];
+    load_chunk(x, vocab, base, v);
     uint64_t best = kNoKey;
-    int nan_first = kNoNan;
+#pragma unroll
+    for (int j = 0; j < kSelPer; j++) {
+        const int i = base + j * kSelThreads;  // (a repeated last token is passed over: its key would be another token's)
+        const uint64_t key = v[j] != v[j] ? static_cast<uint64_t>(i) : cand_key(static_cast<uint32_t>(i), v[j]);
+        best = i < vocab && key < best ? key : best;
+    }
+    best = block_min_u64(best, red);
+    if (threadIdx.x == 0) *out = best;
+}
+
+// The k best, without a sort and without finding the k-th: of every wave's 64 per-thread bests the m-th least ordering word,
+// m = ceil(k / waves), bounds m of them, so the largest of the waves' bounds bounds at least k keys of the chunk, and few more
+// than that (k = 20: about a hundred).  What is below it is ranked by counting the candidates below each, and the candidate of
+// rank r < k is output r.  Keys are distinct (the token id is in the low bits), so ranks are too.  Where more than kSelThreads
+// tokens are below the bound (logits ordered by thread, or alike), the k-th best is looked for digit by digit.  (That search
+// for every chunk was 4.7 of its workgroup's 11.3 us, the collecting of what it bounds another 1.8.)
+__device__ __forceinline__ void select_chunk_body(const float *__restrict__ x, int vocab, int k, uint64_t *__restrict__ out,
+                                                  bool nan_is_candidate) {
+    __shared__ uint64_t cand[kSelThreads];
+    __shared__ KthShared<kSelThreads> kth;
+    __shared__ int rank_sh[kSelThreads];
+    __shared__ uint32_t bounds[kSelThreads / 64];
+    __shared__ int cnt[2];
+    __shared__ int nan_sh;
+    constexpr int kWaves = kSelThreads / 64;
+    const int tid = threadIdx.x, lane = tid & 63, base = blockIdx.x * kSelChunk + tid;
+    float v[kSelPer];
+    load_chunk(x, vocab, base, v);
+    rank_sh[tid] = 0;
     if (tid == 0) {
-        cnt = 0;
+        cnt[0] = cnt[1] = 0;
         nan_sh = kNoNan;
     }
+    // (a token that is no candidate orders last; so does one NaN, which is why the collecting asks for the token, too)
+    uint32_t d[kSelPer], best = 0xffffffffu;
+    int nan_first = kNoNan;
 #pragma unroll
-    for (int j = 0; j < kSelChunk / kSelThreads; j++) {
-        int64_t i = static_cast<int64_t>(chunk) * kSelChunk + j * kSelThreads + tid;
-        uint64_t key = kNoKey;
-        if (i < vocab) {
-            float v = x[i];
-            if (v != v) {
-                nan_first = nan_first < static_cast<int>(i) ? nan_first : static_cast<int>(i);
-                if (nan_is_candidate) key = cand_key(static_cast<uint32_t>(i), v);
-            } else {
-                key = cand_key(static_cast<uint32_t>(i), v);
+    for (int j = 0; j < kSelPer; j++) {
+        const int i = base + j * kSelThreads;
+        const bool nan = v[j] != v[j];
+        d[j] = i < vocab && (nan_is_candidate || !nan) ? desc_bits(__float_as_uint(v[j])) : 0xffffffffu;
+        nan_first = nan && i < vocab ? min(nan_first, i) : nan_first;
+        best = min(best, d[j]);
+    }
+    {
+        uint32_t left = best, least = 0xffffffffu;
+        for (int m = 0; m < k; m += kWaves) {
+            least = wave_min_u32(left);
+            left = left == least ? 0xffffffffu : left;
+        }
+        if (lane == 0) bounds[tid >> 6] = least;
+    }
+    __syncthreads();
+    if (!nan_is_candidate && nan_first != kNoNan) atomicMin(&nan_sh, nan_first);
+    const uint32_t bound = wave_max_u32(lane < kWaves ? bounds[lane] : 0);
+    // a thread with candidates asks for their slots at once (a bound above every number: all that are tokens)
+    auto collect = [&](auto is_candidate) {
+        int n = 0;
+#pragma unroll
+        for (int j = 0; j < kSelPer; j++) n += is_candidate(j);
+        int at = n ? atomicAdd(&cnt[0], n) : 0;
+#pragma unroll
+        for (int j = 0; j < kSelPer; j++) {
+            if (is_candidate(j)) {
+                if (at < kSelThreads) cand[at] = (static_cast<uint64_t>(d[j]) << 32) | static_cast<uint32_t>(base + j * kSelThreads);
+                at++;
             }
         }
-        keys[j] = key;
-        best = key < best ? key : best;
-    }
+    };
+    if (bound == 0xffffffffu)
+        collect([&](int j) { return base + j * kSelThreads < vocab; });
+    else if (best <= bound)
+        collect([&](int j) { return d[j] <= bound; });
     __syncthreads();
-    if (nan_first != kNoNan) atomicMin(&nan_sh, nan_first);
-    ChunkOut *o = out + (row * gridDim.x + chunk);
-    if (k == 1) {
-        uint64_t m = block_min_u64(best, outk);
-        if (tid == 0) {
-            o->keys[0] = m;
-            o->nan_first = nan_sh;
+    int n_cand = cnt[0];
+    if (n_cand > kSelThreads) {
+        uint64_t keys[kSelPer];
+#pragma unroll
+        for (int j = 0; j < kSelPer; j++) {
+            const int i = base + j * kSelThreads;
+            keys[j] = i < vocab ? (static_cast<uint64_t>(d[j]) << 32) | static_cast<uint32_t>(i) : kNoKey;
         }
-        return;
+        const uint64_t kth_key = block_kth<kSelPer>(keys, kNoKey - 1, k, kSelThreads, kth);
+        compact_keys(keys, kth_key, cand, kSelThreads, &cnt[1]);
+        __syncthreads();
+        n_cand = cnt[1];
     }
-    if (tid < kMaxK) outk[tid] = kNoKey;
-    rank_sh[tid] = 0;
-    const uint64_t mine[1] = {best};
-    const uint64_t bound = block_kth<1>(mine, kNoKey - 1, k, kth);
-    compact_keys(keys, bound, cand, kMaxCand, &cnt);
-    __syncthreads();
-    const int n_cand = cnt;  // <= 16 k <= kSelThreads
-    if (n_cand > 0) {
-        // candidate i = tid % n_cand counts the candidates below it in slice tid / n_cand of the list
-        const int slices = kSelThreads / n_cand, i = tid % n_cand, sl = tid / n_cand;
-        if (sl < slices) {
-            const int per = (n_cand + slices - 1) / slices, j0 = sl * per, j1 = min(n_cand, j0 + per);
+    const bool nan_row = nan_sh != kNoNan;
+    {
+        // candidate i = tid % 2^log_n, 2^log_n >= n_cand, counts the candidates below it in slice tid / 2^log_n of the list
+        const int log_n = n_cand > 1 ? 32 - __clz(n_cand - 1) : 0, log_slices = 10 - log_n, i = tid & ((1 << log_n) - 1);
+        if (i < n_cand) {
+            const int per = (n_cand + (1 << log_slices) - 1) >> log_slices, j0 = (tid >> log_n) * per, j1 = min(n_cand, j0 + per);
             const uint64_t key = cand[i];
             int c = 0;
+#pragma unroll 4
             for (int j = j0; j < j1; j++) c += cand[j] < key;
             if (c) atomicAdd(&rank_sh[i], c);
         }
     }
     __syncthreads();
-    if (tid < n_cand && rank_sh[tid] < k) outk[rank_sh[tid]] = cand[tid];
-    __syncthreads();
-    if (tid < k) o->keys[tid] = outk[tid];
-    if (tid == 0) o->nan_first = nan_sh;
+    if (tid < n_cand && rank_sh[tid] < k && !(nan_row && rank_sh[tid] == 0)) out[rank_sh[tid]] = cand[tid];
+    if (tid < k && tid >= n_cand) out[tid] = kNoKey;
+    if (tid == 0 && nan_row) out[0] = static_cast<uint64_t>(nan_sh);
 }
 
-__global__ void __launch_bounds__(kSelThreads)
-    select_chunk_kernel(const float *__restrict__ logits, int64_t vocab, int64_t stride, int k,
-                        ChunkOut *__restrict__ out, bool nan_is_candidate) {
-    select_chunk_body(logits, vocab, stride, k, out, nan_is_candidate, blockIdx.y);
+__global__ void __launch_bounds__(kSelThreads, 8)
+    select_chunk_kernel(const float *__restrict__ logits, int64_t stride, uint64_t *__restrict__ out, int vocab, int k, bool nan_is_candidate) {
+    const int row = blockIdx.y;
+    out += static_cast<int64_t>(row) * gridDim.x * k + blockIdx.x * k;
+    if (k == 1)
+        best_of_chunk(logits + row * stride, vocab, out);
+    else
+        select_chunk_body(logits + row * stride, vocab, k, out, nan_is_candidate);
 }
 
 // Two row sets in one launch: rows [0, n_a) of a (best k_a keys of every chunk), then the rows of b (best key).
-__global__ void __launch_bounds__(kSelThreads)
-    select_pair_kernel(const float *__restrict__ a, int n_a, int k_a, ChunkOut *__restrict__ out_a, const float *__restrict__ b,
-                       ChunkOut *__restrict__ out_b, int64_t vocab, int64_t stride) {
+__global__ void __launch_bounds__(kSelThreads, 8)
+    select_pair_kernel(const float *__restrict__ a, const float *__restrict__ b, int64_t stride, uint64_t *__restrict__ out_a,
+                       uint64_t *__restrict__ out_b, int vocab, int n_a, int k_a) {
     const int row = blockIdx.y;
-    if (row < n_a)
-        select_chunk_body(a, vocab, stride, k_a, out_a, false, row);
+    if (row >= n_a)
+        best_of_chunk(b + (row - n_a) * stride, vocab, out_b + static_cast<int64_t>(row - n_a) * gridDim.x + blockIdx.x);
+    else if (k_a == 1)
+        best_of_chunk(a + row * stride, vocab, out_a + static_cast<int64_t>(row) * gridDim.x + blockIdx.x);
     else
-        select_chunk_body(b, vocab, stride, 1, out_b, false, row - n_a);
+        select_chunk_body(a + row * stride, vocab, k_a, out_a + (static_cast<int64_t>(row) * gridDim.x + blockIdx.x) * k_a, false);
 }
 
-// The dense proposal's side of a row: its largest draft logit (scaled) and NaN / no-candidate errors.
-__device__ void merge_draft_side(const ChunkOut *__restrict__ draft_chunks, int n_chunks, int row, const ChainCfg &cfg, RowDist *d) {
+// Number of keys below x in the ascending list of 1 <= n keys; step0 = the largest power of two <= n.
+__device__ __forceinline__ int count_below(const uint64_t *list, int n, int step0, uint64_t x) {
+    int below = 0;
+    for (int step = step0; step >= 1; step >>= 1) {
+        const int probe = below + step;
+        const uint64_t v = list[min(probe, n) - 1];
+        below = probe <= n && v < x ? probe : below;
+    }
+    return below;
+}
+
+// A lane's share of a draft row's chunk minima, and from the wave's lanes the row's largest logit, scaled; NaN where the row
+// holds one, its token in *nan_token.
+__device__ __forceinline__ uint64_t draft_best_of(const uint64_t *__restrict__ draft_best, int n_chunks, int row) {
     uint64_t best = kNoKey;
-    int dn = kNoNan;
-    for (int c = 0; c < n_chunks; c++) {
-        const ChunkOut &dc = draft_chunks[row * n_chunks + c];
-        best = dc.keys[0] < best ? dc.keys[0] : best;
-        dn = dc.nan_first < dn ? dc.nan_first : dn;
+    for (int c = threadIdx.x & 63; c < n_chunks; c += 64) {
+        const uint64_t key = draft_best[static_cast<int64_t>(row) * n_chunks + c];
+        best = key < best ? key : best;
     }
-    d->d_err = 0;
-    d->d_err_index = -1;
-    d->d_max_scaled = static_cast<double>(key_logit(best)) / static_cast<double>(cfg.draft_temperature);
-    if (dn != kNoNan) {
-        d->d_err = DFLASH_ERR_NAN_LOGIT;
-        d->d_err_index = dn;
-    } else if (!isfinite(d->d_max_scaled)) {
-        d->d_err = DFLASH_ERR_NO_CANDIDATES;
-    }
+    return best;
+}
+__device__ __forceinline__ double draft_max_scaled(uint64_t best, float draft_temperature, int *nan_token) {
+    best = wave_min_u64(best);
+    *nan_token = key_is_nan(best) ? key_token(best) : -1;
+    return static_cast<double>(key_logit(best)) / static_cast<double>(draft_temperature);
 }
 
-// One workgroup per row: merge the chunk lists, order the best k, run the chain (wave 0, a candidate per lane).
-__device__ __forceinline__ void row_merge_body(const ChunkOut *__restrict__ chunks, int n_chunks,
-                                               const ChunkOut *__restrict__ draft_chunks, const ChainCfg &cfg,
-                                               RowDist *__restrict__ rows, int32_t *__restrict__ greedy_out, bool draft_only,
-                                               int row) {
-    __shared__ uint64_t sk[2 * kSelThreads];
-    const int tid = threadIdx.x;
+// One workgroup per row: merge the chunk lists, order the best k, run the chain (wave 0, a candidate per lane).  With dense
+// proposals the second wave takes the draft row's side (its maximum, its errors, the draft's own weight) and the first one, behind
+// the chain, the draft row's weights of the kept candidates: what of the decision is independent per row and does not
+// need the draft row's sum.
+__device__ __forceinline__ void row_merge_body(const uint64_t *__restrict__ chunks, int n_chunks, const uint64_t *__restrict__ draft_best,
+                                               const float *__restrict__ draft, int64_t draft_stride, int k, int n_tokens, const ChainCfg &cfg,
+                                               const BlockWalk &walk, RowDist *__restrict__ rows, int32_t *__restrict__ greedy_out,
+                                               bool draft_only, int row) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     RowDist *d = rows + row;
+    const bool drafted = row + 1 < n_tokens, dense = draft_best && drafted;
+    const int32_t draft_token = drafted ? walk.verified[row + 1] : -1;
+    // the draft row's own side, by one wave: asked for ahead of the lists, worked out behind their merge
+    const int draft_wave = draft_only ? 0 : 1;
+    float draft_token_logit = 0.0f;
+    uint64_t best_draft = kNoKey;
+    auto draft_side = [&]() {
+        int nan_token;
+        const double mx = draft_max_scaled(best_draft, cfg.draft_temperature, &nan_token);
+        const double q = exp(static_cast<double>(draft_token_logit) / static_cast<double>(cfg.draft_temperature) - mx);
+        if (lane == 0) {
+            d->d_err = nan_token >= 0 ? DFLASH_ERR_NAN_LOGIT : isfinite(mx) ? 0 : DFLASH_ERR_NO_CANDIDATES;
+            d->d_err_index = nan_token;
+            d->d_max_scaled = mx;
+            d->q_draft = q;
+        }
+    };
+    const int n_in = n_chunks * k;  // <= 2048, checked on the host
+    uint64_t in0 = kNoKey, in1 = kNoKey;
+    if (!draft_only) {
+        const uint64_t *mine = chunks + static_cast<int64_t>(row) * n_in;
+        in0 = mine[min(tid, n_in - 1)];
+        in1 = mine[min(tid + kSelThreads, n_in - 1)];
+    }
+    if (dense && wave < 2) {
+        if (wave == draft_wave) draft_token_logit = draft[row * draft_stride + draft_token];
+        best_draft = draft_best_of(draft_best, n_chunks, row);
+    }
     if (draft_only) {  // the target side of these rows was filled by the wide chain
-        if (tid == 0) merge_draft_side(draft_chunks, n_chunks, row, cfg, d);
+        if (dense && wave == 0) draft_side();
         return;
     }
     // The chunks' lists are ascending: the rank of a key among all of them is the sum, over the lists, of the keys
-    // below it (binary searches); the keys of rank < k, in rank order, are the row's candidates, best first.
-    const int k = cfg.k;
-    const int n_in = n_chunks * k;  // <= 2048, checked on the host
-    __shared__ uint64_t lists[2 * kSelThreads];
+    // below it (binary searches); the keys of rank < k, in rank order, are the row's candidates, best first.  Only keys up to the
+    // largest of the full lists' m-th, m = ceil(k / lists), can be among them: those lists hold k keys up to there.
+    // (Ranking all of the lists' keys: 3.2 us of the row's 6.8 at ten lists of 20.)
+    __shared__ uint64_t sk[kMaxK];
+    __shared__ uint64_t lists[2 * kSelThreads], cand[2 * kSelThreads];
     __shared__ int rank_sh[2 * kSelThreads];
     __shared__ uint64_t red[kSelThreads / 64];
-    if (tid < kMaxK) sk[tid] = kNoKey;
-    uint64_t mine = kNoKey;
-    for (int i = tid; i < n_in; i += kSelThreads) {
-        const uint64_t key = chunks[row * n_chunks + i / k].keys[i % k];
-        lists[i] = key;
-        rank_sh[i] = 0;
-        mine = key < mine ? key : mine;
-    }
+    __shared__ int cnt;
     if (k == 1) {
-        mine = block_min_u64(mine, red);
-        if (tid == 0) sk[0] = mine;
+        const uint64_t best = block_min_u64(min(in0, in1), red);
+        if (tid == 0) sk[0] = best;
     } else {
+        lists[tid] = in0;
+        lists[tid + kSelThreads] = in1;
+        rank_sh[tid] = rank_sh[tid + kSelThreads] = 0;
+        if (tid < kMaxK) sk[tid] = kNoKey;
+        if (tid == 0) cnt = 0;
         __syncthreads();
-        // (key, list) pairs over all threads: a thread's searches are independent of each other
-        // (consecutive threads: consecutive keys against the same list, so that a wave's probes fall on different
-        // banks and its additions on different counters)
-        const int step0 = 1 << (31 - __clz(k));
-        for (int p0 = tid; p0 < n_in * n_chunks; p0 += 4 * kSelThreads) {
-            int off[4], slot[4], below[4];
-            uint64_t key[4];
+        const int n_full = n_chunks - (lists[n_in - 1] == kNoKey);
+        uint32_t top = n_full ? 0 : 0xffffffffu;
+        if (n_full) {
+            const int m = (k + n_full - 1) / n_full;
+            for (int c = lane; c < n_full; c += 64) top = max(top, static_cast<uint32_t>(lists[c * k + m - 1] >> 32));
+            top = wave_max_u32(top);
+        }
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const int p = p0 + j * kSelThreads;
-                const bool live = p < n_in * n_chunks;
-                const int c = live ? p / n_in : 0;
-                slot[j] = live ? p - c * n_in : 0;
-                off[j] = c * k;
-                key[j] = live ? lists[slot[j]] : 0;  // (nothing is below key 0)
-            }
-            count_below4(lists, off, k, step0, key, below);
-#pragma unroll
-            for (int j = 0; j < 4; j++)
-                if (below[j] && key[j] != kNoKey) atomicAdd(&rank_sh[slot[j]], below[j]);
+        for (int u = 0; u < 2; u++) {
+            const int i = tid + u * kSelThreads;
+            const uint64_t key = u ? in1 : in0;
+            if (i < n_in && key != kNoKey && static_cast<uint32_t>(key >> 32) <= top) cand[atomicAdd(&cnt, 1)] = key;
         }
         __syncthreads();
-        for (int i = tid; i < n_in; i += kSelThreads)
-            if (lists[i] != kNoKey && rank_sh[i] < k) sk[rank_sh[i]] = lists[i];
+        // (key, list) pairs: neighbouring threads take a key's lists
+        const int n_cand = cnt, step0 = 1 << (31 - __clz(k)), log_c = n_chunks > 1 ? 32 - __clz(n_chunks - 1) : 0;  // n_chunks <= 2^log_c <= kSelThreads
+        const int c = tid & ((1 << log_c) - 1);
+        for (int i = tid >> log_c; i < n_cand && c < n_chunks; i += kSelThreads >> log_c) {
+            const int below = count_below(lists + c * k, k, step0, cand[i]);
+            if (below) atomicAdd(&rank_sh[i], below);
+        }
+        __syncthreads();
+        for (int i = tid; i < n_cand; i += kSelThreads)
+            if (rank_sh[i] < k) sk[rank_sh[i]] = cand[i];
     }
     __syncthreads();
-    if (tid >= 64) {
-        // the dense proposal's side is independent of the target's: the first lane of the second wave takes it
-        if (tid == 64 && draft_chunks) merge_draft_side(draft_chunks, n_chunks, row, cfg, d);
+    if (dense && wave == 1) draft_side();
+    if (wave > 0) return;
+    const uint64_t first = sk[0];
+    const int nan_token = key_is_nan(first) ? key_token(first) : -1;
+    if (greedy_out) {  // (the greedy argmax wants nothing else of the row)
+        if (tid == 0) greedy_out[row] = nan_token >= 0 ? ~nan_token : key_token(first);
         return;
     }
-    int nan_first = kNoNan;
-    for (int c = tid; c < n_chunks; c += 64) {
-        int nf = chunks[row * n_chunks + c].nan_first;
-        nan_first = nf < nan_first ? nf : nan_first;
+    const uint64_t key = tid < k ? sk[tid < kMaxK ? tid : 0] : kNoKey;
+    const int n_keys = __popcll(__builtin_amdgcn_ballot_w64(key != kNoKey));  // (missing keys sort last)
+    const int32_t token = key != kNoKey ? key_token(key) : 0;
+    float draft_logit = 0.0f;
+    if (dense && nan_token < 0) draft_logit = draft[row * draft_stride + token];  // (used behind the chain)
+    WaveChain ch = {0, 0.0, 0.0, 0.0};
+    int32_t pick = 0;
+    double draft_weight = -0.0;
+    if (nan_token < 0) {
+        if (cfg.temperature == 0.0f) {  // greedy target: one-hot on the total-order argmax (sampling.rs:391-400)
+            ch = {1, 1.0, 1.0, 1.0};
+            pick = key_token(first);
+        } else {
+            ch = run_chain_wave(key_logit(key), n_keys, cfg);
+            if (ch.len) {
+                const double drawn = walk.uniforms[row] * ch.total;
+                pick = __builtin_amdgcn_readlane(token, wave_first(drawn < ch.upto, ch.len));
+            }
+        }
+        const uint64_t at = __builtin_amdgcn_ballot_w64(drafted && lane < ch.len && token == draft_token);  // (tokens are distinct)
+        if (at) draft_weight = chain_bcast(ch.w, static_cast<int>(__builtin_ctzll(at)));
     }
-    for (int off = 32; off > 0; off >>= 1) nan_first = min(nan_first, __shfl_xor(nan_first, off, 64));
-    if (tid == 0) {
-        d->n_keep = 0;
-        d->err = 0;
-        d->err_index = -1;
-        d->total = 0.0;
-        if (!draft_chunks) {
+    if (dense && ch.len) {
+        int none;
+        const double mx = draft_max_scaled(best_draft, cfg.draft_temperature, &none);
+        const double q = exp(static_cast<double>(draft_logit) / static_cast<double>(cfg.draft_temperature) - mx);
+        if (lane < ch.len) d->q[lane] = q;
+    }
+    if (lane < ch.len) {
+        d->tokens[lane] = token;
+        d->weights[lane] = ch.w;
+    }
+    if (lane == 0) {
+        d->n_keep = ch.len;
+        d->err = nan_token >= 0 ? DFLASH_ERR_NAN_LOGIT : ch.len ? 0 : DFLASH_ERR_NO_CANDIDATES;
+        d->err_index = nan_token;
+        d->total = ch.total;
+        d->pick = pick;
+        d->draft_weight = draft_weight;
+        if (!dense) {
             d->d_err = 0;
             d->d_err_index = -1;
         }
-        if (greedy_out) greedy_out[row] = nan_first != kNoNan ? ~nan_first : key_token(sk[0]);
-    }
-    if (nan_first != kNoNan) {
-        if (tid == 0) {
-            d->err = DFLASH_ERR_NAN_LOGIT;
-            d->err_index = nan_first;
-        }
-    } else if (cfg.temperature == 0.0f) {
-        // greedy target: one-hot on the total-order argmax (sampling.rs:391-400)
-        if (tid == 0) {
-            d->n_keep = 1;
-            d->total = 1.0;
-            d->tokens[0] = key_token(sk[0]);
-            d->weights[0] = 1.0;
-        }
-    } else {
-        const int len = __popcll(__builtin_amdgcn_ballot_w64(tid < k && sk[tid < k ? tid : 0] != kNoKey));  // (missing keys sort last)
-        run_chain_wave(sk, len, cfg, d);
     }
 }
 
 __global__ void __launch_bounds__(kSelThreads)
-    row_merge_kernel(const ChunkOut *__restrict__ chunks, int n_chunks, const ChunkOut *__restrict__ draft_chunks,
-                     ChainCfg cfg, RowDist *__restrict__ rows, int32_t *__restrict__ greedy_out, bool draft_only) {
-    row_merge_body(chunks, n_chunks, draft_chunks, cfg, rows, greedy_out, draft_only, blockIdx.x);
+    row_merge_kernel(const uint64_t *__restrict__ chunks, RowDist *__restrict__ rows, int32_t *__restrict__ greedy_out, int n_chunks, int k,
+                     ChainCfg cfg, BlockWalk walk) {
+    row_merge_body(chunks, n_chunks, nullptr, nullptr, 0, k, walk.n_tokens, cfg, walk, rows, greedy_out, false, blockIdx.x);
 }
 
 // top-16 output from the merged order
 __global__ void __launch_bounds__(kSelThreads)
-    top16_merge_kernel(const ChunkOut *__restrict__ chunks, int n_chunks, int32_t *__restrict__ ids,
+    top16_merge_kernel(const uint64_t *__restrict__ chunks, int n_chunks, int32_t *__restrict__ ids,
                        float *__restrict__ vals) {
     __shared__ uint64_t lists[2 * kSelThreads], sk[16];
     const int row = blockIdx.x, tid = threadIdx.x;
     const int n_in = n_chunks * 16;  // <= 2048, checked on the host
-    for (int i = tid; i < n_in; i += kSelThreads) lists[i] = chunks[row * n_chunks + i / 16].keys[i % 16];
+    for (int i = tid; i < n_in; i += kSelThreads) lists[i] = chunks[static_cast<int64_t>(row) * n_in + i];
     if (tid < 16) sk[tid] = kNoKey;
     __syncthreads();
     // a key's rank by counting the keys below it, sixteen lanes a key: a chunk's list each, sixteen chunks a round
@@ -393,68 +466,70 @@ __global__ void __launch_bounds__(kSelThreads)
 }
 
 // The rows' chains and the dense proposal's tile sums in one launch (neither needs the other; both need only the
-// chunk selection): workgroups [0, n_rows) are row_merge_kernel's, the rest take eight 1024-token tiles each of draft
-// row (workgroup - n_rows) / blocks_per_row.  A tile sum is the sum of exp(d/T - max/T) in a fixed shape: slot t of
+// chunk selection): of a row's workgroups the first is row_merge_kernel's, the rest take four 1024-token tiles each of its
+// draft row.  A tile sum is the sum of exp(d/T - max/T) in a fixed shape: slot t of
 // a tile holds ((e[4t]+e[4t+1])+e[4t+2])+e[4t+3], then a halving tree over the 256 slots; max is the row's largest
-// draft logit, which every tile workgroup takes from the chunk minima itself.
+// draft logit, which every wave takes from the chunk minima itself, with its logits on their way.  The tree's two widest levels
+// are one trip through LDS, the rest a wave's.  (A barrier per level and tile, and the logits asked for behind the maximum: 8.8 us of
+// a workgroup.)
+struct __attribute__((packed, aligned(4))) Logits4 {  // (rows start wherever the vocabulary puts them)
+    float v[4];
+};
 __global__ void __launch_bounds__(kSelThreads)
-    rows_and_tiles_kernel(const ChunkOut *__restrict__ chunks, int n_chunks, const ChunkOut *__restrict__ draft_chunks, ChainCfg cfg,
-                          RowDist *__restrict__ rows, int n_rows, bool draft_only, const float *__restrict__ draft, int64_t vocab,
-                          int64_t stride, int n_tiles, int blocks_per_row, double *__restrict__ tile_sums) {
-    if (static_cast<int>(blockIdx.x) < n_rows) {
-        row_merge_body(chunks, n_chunks, draft_chunks, cfg, rows, nullptr, draft_only, blockIdx.x);
+    rows_and_tiles_kernel(const uint64_t *__restrict__ chunks, const float *__restrict__ draft, const uint64_t *__restrict__ draft_best,
+                          double *__restrict__ tile_sums, int vocab, int n_chunks, int k, int n_tokens, float draft_temperature, int n_tiles,
+                          RowDist *__restrict__ rows, bool draft_only, ChainCfg cfg, BlockWalk walk) {
+    const int row = blockIdx.x;
+    if (blockIdx.y == 0) {
+        row_merge_body(chunks, n_chunks, draft_best, draft, vocab, k, n_tokens, cfg, walk, rows, nullptr, draft_only, row);
         return;
     }
+    if (row == n_tokens - 1) return;  // (the last row has no draft)
     __shared__ double slot[4][256];
-    __shared__ uint64_t red[kSelThreads / 64];
-    const int b = blockIdx.x - n_rows, row = b / blocks_per_row, q = threadIdx.x >> 8, t = threadIdx.x & 255;
-    uint64_t best = kNoKey;
-    for (int c = threadIdx.x; c < n_chunks; c += kSelThreads) {
-        const uint64_t key = draft_chunks[row * n_chunks + c].keys[0];
-        best = key < best ? key : best;
-    }
-    best = block_min_u64(best, red);
-    const double T = static_cast<double>(cfg.draft_temperature);
-    const double mx = static_cast<double>(key_logit(best)) / T;  // merge_draft_side's d_max_scaled
-    const float *x = draft + row * stride;
-    // (eight tiles per workgroup, two per quarter: with four, a 15-row block is more workgroups than the chip holds
-    // at once)
-    for (int half = 0; half < 2; half++) {
-        const int tile = (b - row * blocks_per_row) * 8 + 4 * half + q;
-        const int64_t base = static_cast<int64_t>(tile) * 1024 + 4 * t;
-        double acc = 0.0;
+    const int tid = threadIdx.x, q = tid >> 8, t = tid & 255, tile0 = (blockIdx.y - 1) * 4, i = (tile0 + q) * 1024 + 4 * t;
+    const float *x = draft + static_cast<int64_t>(row) * vocab;
+    Logits4 in;
+    if (i + 3 < vocab)
+        in = *reinterpret_cast<const Logits4 *>(x + i);
+    else
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            int64_t i = base + e;
-            double v = (tile < n_tiles && i < vocab) ? exp(static_cast<double>(x[i]) / T - mx) : 0.0;
-            acc = (e == 0) ? v : acc + v;
-        }
-        __syncthreads();  // (the previous half's sums have been read)
-        slot[q][t] = acc;
-        for (int s = 128; s >= 1; s >>= 1) {
-            __syncthreads();
-            if (t < s) slot[q][t] += slot[q][t + s];
-        }
-        if (t == 0 && tile < n_tiles) tile_sums[row * n_tiles + tile] = slot[q][0];
+        for (int e = 0; e < 4; e++) in.v[e] = x[min(i + e, vocab - 1)];
+    int nan_token;
+    const double mx = draft_max_scaled(draft_best_of(draft_best, n_chunks, row), draft_temperature, &nan_token);
+    // x / T as x * (1 / T) and one correction by the exact remainder: T and x have 24 bits, so the quotient is no closer than 2^-78
+    // of itself to a value where rounding turns, and the corrected one is within 2^-104 of it before its own rounding.
+    // (An infinite x has no remainder and stays as it is.)
+    const double T = static_cast<double>(draft_temperature), inv_T = 1.0 / T;
+    double acc = 0.0;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const double xe = static_cast<double>(in.v[e]), q0 = xe * inv_T, rem = __builtin_fma(-q0, T, xe);
+        const double scaled = rem == rem ? __builtin_fma(rem, inv_T, q0) : q0;
+        const double v = i + e < vocab ? exp(scaled - mx) : 0.0;
+        acc = (e == 0) ? v : acc + v;
     }
+    slot[q][t] = acc;
+    __syncthreads();
+    const int tile = tid >> 6, lane = tid & 63;  // a wave per tile
+    if (tile >= 4) return;
+    double sum = (slot[tile][lane] + slot[tile][lane + 128]) + (slot[tile][lane + 64] + slot[tile][lane + 192]);
+#pragma unroll
+    for (int s = 32; s >= 1; s >>= 1) sum += __shfl_xor(sum, s, 64);
+    if (lane == 0 && tile0 + tile < n_tiles) tile_sums[row * n_tiles + tile0 + tile] = sum;
 }
 
 struct DecideArgs {
-    int32_t n_tokens, n_stop, mode, vocab;
+    int32_t n_stop;
     int64_t budget;
     // The block's small host inputs travel by value, in the kernel arguments: a pageable host-to-device copy
     // of a few bytes costs several microseconds of idle GPU each.
-    int32_t verified[kMaxRows];      // [n_tokens]
-    double uniforms[kMaxRows + 2];   // [n_tokens + 1]
+    BlockWalk walk;
     int32_t prop_offsets[kMaxRows], prop_counts[kMaxRows];  // sparse proposals: row r's candidates in prop_cands
     const int32_t *stop_ids;   // [n_stop]
-    const RowDist *rows;
     const dflash_weighted_candidate *prop_cands;
     // dense proposals
     const float *draft;
     int64_t draft_stride;
-    const double *tile_sums;
-    int32_t n_tiles;
     float temperature, draft_temperature;
     // wide candidate sets (effective top-k above kMaxK): row r's kept candidates are the first n_keep ordered keys
     // / weights at r * wide_stride of these arrays instead of the arrays inside RowDist; null otherwise
@@ -463,165 +538,141 @@ struct DecideArgs {
     int64_t wide_stride;
 };
 
-// A row's kept candidates, wherever they live.
-struct DistView {
-    const RowDist *rd;
-    const uint64_t *keys;  // null: inline arrays of rd
-    const double *w;
-    __device__ int32_t token(int i) const { return keys ? static_cast<int32_t>(keys[i] & kWideTokenMask) : rd->tokens[i]; }
-    __device__ double weight(int i) const { return w ? w[i] : rd->weights[i]; }
-};
-
-__device__ bool in_list(const int32_t *ids, int n, int32_t v) {
-    for (int i = 0; i < n; i++)
-        if (ids[i] == v) return true;
-    return false;
-}
-
 // What one row of the walk comes to, given that every row before it accepted.
 struct RowOutcome {
     int32_t acc;         // the draft is accepted (draft rows only)
+    int32_t stop;        // the draft is a stop id (draft rows only)
     int32_t token;       // correction token (rejected draft row) or bonus token (last row)
     int32_t draws;       // random draws this row consumes
     int32_t err;         // DFLASH_ERR_* of this row, 0 if none
-    int64_t err_index;
-    // a rejected row under a stochastic proposal: its correction token is still to be drawn from the residual
-    // distribution (residual_pick, by the whole wave, for the one row the walk stops at)
+    // wide sets: a rejected row's correction token is still to be drawn from the residual distribution
+    // (residual_pick, for the one row the walk stops at)
     int32_t need_residual;
-    int32_t residual_draw;  // index of the uniform draw the pick uses
-    double prop_total;
+    int64_t err_index;
+    double prop_total, u_residual;  // u_residual: the draw the pick uses
 };
 
-// One row of accept.rs:147-183 with the couplings of sampling.rs:692-790.  A row that is reached has seen only
-// accepting rows before it, and an accepting row consumes exactly one draw (none when greedy): row r therefore
+// One row of accept.rs:147-183 with the couplings of sampling.rs:692-790, by one whole wave.  A row that is reached has seen
+// only accepting rows before it, and an accepting row consumes exactly one draw (none when greedy): row r therefore
 // starts at draw r whatever the rows before it held, which is what lets every row be evaluated at once.
-__device__ RowOutcome decide_row(const DecideArgs &a, const RowDist *rows, int row, const double *p_total,
-                                 const float *draft_tok_logit) {
-    RowOutcome o = {0, 0, 0, 0, -1, 0, 0, 0.0};
-    const int n_drafts = a.n_tokens - 1;
+// rd: the row; token / p / q: lane i's candidate, its probability and its draft weight; target_probability: the draft's;
+// u, u_residual: the row's draw and the one behind it; dense_total: the draft row's sum.
+__device__ __forceinline__ RowOutcome decide_row(const DecideArgs &a, int mode, const RowDist &rd, int row, int32_t token, double p, double q,
+                                                 double target_probability, double u, double u_residual, double dense_total) {
+    RowOutcome o = {0, 0, 0, 0, 0, 0, -1, 0.0, 0.0};
+    const int lane = threadIdx.x & 63, n_drafts = a.walk.n_tokens - 1;
     const bool greedy = a.temperature == 0.0f;
-    const RowDist &rd = rows[row];
-    int draws = greedy ? 0 : row;
-    const int draws0 = draws;
-    // the target token that draw `row` falls on (wide sets: the row's chain has walked its order with that draw)
-    auto target_token = [&]() {
-        if (a.wide_keys) {
-            draws++;
-            return rd.pick;
-        }
-        return rd.tokens[greedy ? 0 : pick_index(rd.weights, rd.n_keep, a.uniforms[draws++] * rd.total)];
-    };
-    if (row == n_drafts) {  // bonus = sample(last reached row)
-        if (rd.err) {
-            o.err = rd.err;
-            o.err_index = rd.err_index;
-            return o;
-        }
-        o.token = target_token();
-        o.draws = draws - draws0;
+    if (row == n_drafts || mode == 0) {
+        // bonus = sample(last reached row); deterministic coupling: draw the target token, accept iff it is the draft
+        o.err = rd.err;
+        o.err_index = rd.err_index;
+        if (o.err) return o;
+        o.token = rd.pick;
+        o.draws = !greedy || a.wide_keys;
+        o.acc = row < n_drafts && o.token == a.walk.verified[row + 1];
         return o;
     }
-    const int32_t draft = a.verified[row + 1];
-    if (a.mode == 0) {  // deterministic coupling: draw the target token, accept iff it is the draft
-        if (rd.err) {
-            o.err = rd.err;
-            o.err_index = rd.err_index;
-            return o;
-        }
-        o.token = target_token();
-        o.acc = o.token == draft;
-        o.draws = draws - draws0;
-        return o;
-    }
+    const int32_t draft = a.walk.verified[row + 1];
     // proposal probability q(draft) and, per target candidate, q(candidate)
     double prop_total = 0.0, prop_tok_w = 0.0;
-    const dflash_weighted_candidate *pc = nullptr;
-    int n_pc = 0;
-    if (a.mode == 1) {
-        pc = a.prop_cands + a.prop_offsets[row];
-        n_pc = a.prop_counts[row];
+    const dflash_weighted_candidate *pc = a.prop_cands + a.prop_offsets[row];
+    const int n_pc = a.prop_counts[row];
+    if (mode == 1) {
         if (n_pc == 0) o.err = DFLASH_ERR_NO_CANDIDATES;
-        for (int j = 0; j < n_pc && !o.err; j++) {
-            if (!isfinite(pc[j].weight) || pc[j].weight < 0.0) {
+        for (int base = 0; base < n_pc && !o.err; base += 64) {
+            const int m = min(64, n_pc - base);
+            const int32_t t = lane < m ? pc[base + lane].token : -1;
+            const double w = lane < m ? pc[base + lane].weight : 0.0;
+            const uint64_t bad = __builtin_amdgcn_ballot_w64(!isfinite(w) || w < 0.0);
+            if (bad) {
                 o.err = DFLASH_ERR_INVALID_PROPOSAL_WEIGHT;
-                o.err_index = pc[j].token;
+                o.err_index = __builtin_amdgcn_readlane(t, static_cast<int>(__builtin_ctzll(bad)));
                 break;
             }
-            prop_total += pc[j].weight;
-            if (pc[j].token == draft) prop_tok_w += pc[j].weight;
-        }
-        if (!o.err && !(isfinite(prop_total) && prop_total > 0.0)) o.err = DFLASH_ERR_NO_CANDIDATES;
-        if (!o.err && !(isfinite(prop_tok_w) && prop_tok_w > 0.0)) {
-            o.err = DFLASH_ERR_MISSING_PROPOSAL_TOKEN;
-            o.err_index = draft;
+            prop_total = chain_bcast(wave_running_sum(prop_total, w, m), m - 1);
+            for (uint64_t at = __builtin_amdgcn_ballot_w64(lane < m && t == draft); at; at &= at - 1)
+                prop_tok_w += chain_bcast(w, static_cast<int>(__builtin_ctzll(at)));
         }
     } else {
-        if (rd.d_err) {
-            o.err = rd.d_err;
-            o.err_index = rd.d_err_index;
-        }
-        prop_total = p_total[row];
-        if (!o.err && !(isfinite(prop_total) && prop_total > 0.0)) o.err = DFLASH_ERR_NO_CANDIDATES;
-        if (!o.err) {
-            // (draft_tok_logit[row] = a.draft[row][draft], fetched ahead)
-            prop_tok_w = exp(static_cast<double>(draft_tok_logit[row]) / static_cast<double>(a.draft_temperature) - rd.d_max_scaled);
-            if (!(isfinite(prop_tok_w) && prop_tok_w > 0.0)) {
-                o.err = DFLASH_ERR_MISSING_PROPOSAL_TOKEN;
-                o.err_index = draft;
-            }
-        }
+        o.err = rd.d_err;
+        o.err_index = rd.d_err_index;
+        prop_total = dense_total;
+        prop_tok_w = rd.q_draft;
+    }
+    if (!o.err && !(isfinite(prop_total) && prop_total > 0.0)) o.err = DFLASH_ERR_NO_CANDIDATES;
+    if (!o.err && !(isfinite(prop_tok_w) && prop_tok_w > 0.0)) {
+        o.err = DFLASH_ERR_MISSING_PROPOSAL_TOKEN;
+        o.err_index = draft;
     }
     if (!o.err && rd.err) {
         o.err = rd.err;
         o.err_index = rd.err_index;
     }
     if (o.err) return o;
-    double tp = -0.0;
-    if (a.wide_keys)
-        tp = rd.draft_weight;
-    else
-        for (int i = 0; i < rd.n_keep; i++)
-            if (rd.tokens[i] == draft) tp += rd.weights[i];
-    const double target_probability = tp / rd.total;
     const double proposal_probability = prop_tok_w / prop_total;
     const double acceptance = fmin(target_probability / proposal_probability, 1.0);
-    if (a.uniforms[draws++] < acceptance) {
+    if (u < acceptance) {
         o.acc = 1;
-    } else {
-        // the correction token comes from the residual distribution: one more draw
-        o.need_residual = 1;
-        o.residual_draw = draws++;
-        o.prop_total = prop_total;
+        o.draws = 1;
+        return o;
     }
-    o.draws = draws - draws0;
+    // The correction token comes from the residual distribution: weights max(p_i - q_i, 0) in the target's order
+    // (sampling.rs:752-790), and one more draw.  A candidate per lane; their running sums give the total and the pick.
+    o.draws = 2;
+    o.u_residual = u_residual;
+    o.prop_total = prop_total;
+    if (a.wide_keys) {
+        o.need_residual = 1;
+        return o;
+    }
+    if (mode == 1) {
+        q = -0.0;
+        for (int base = 0; base < n_pc; base += 64) {
+            const int m = min(64, n_pc - base);
+            const int32_t t = lane < m ? pc[base + lane].token : -1;
+            const double w = lane < m ? pc[base + lane].weight : 0.0;
+            for (int j = 0; j < m; j++) {
+                const double wj = chain_bcast(w, j);
+                if (__builtin_amdgcn_readlane(t, j) == token) q += wj;
+            }
+        }
+    }
+    const int n_keep = rd.n_keep;
+    const double residual = lane < n_keep ? fmax(p - q / prop_total, 0.0) : 0.0;
+    const double upto = wave_running_sum(0.0, residual, n_keep), residual_total = chain_bcast(upto, n_keep - 1);
+    if (!(isfinite(residual_total) && residual_total > 0.0)) {
+        o.err = DFLASH_ERR_NO_CANDIDATES;
+        return o;
+    }
+    const double x = u_residual * residual_total;
+    o.token = __builtin_amdgcn_readlane(token, wave_first(x < upto, n_keep));
     return o;
 }
 
-// The correction token of rejected row `row`: residual weights max(p_i - q_i, 0) in the target's order
-// (sampling.rs:752-790), summed first, then walked again for the pick; the second pass recomputes the same values,
+// The correction token of rejected row `row` where its candidates are a wide set, as in decide_row: the residual weights
+// are summed first, then walked again for the pick; the second pass recomputes the same values,
 // so no per-candidate array is needed.  By the whole wave: lane j computes the weight of candidate base + j (one f64
 // exponential each under a dense proposal, the expensive part), and the sums add those values in candidate order,
 // one addition after the other.
-__device__ void residual_pick(const DecideArgs &a, const RowDist *rows, int row, RowOutcome &o, const float *draft_logit_of) {
+__device__ __forceinline__ void residual_pick(const DecideArgs &a, int mode, const RowDist &rd, int row, RowOutcome &o) {
     const int lane = threadIdx.x & 63;
-    const RowDist &rd = rows[row];
-    const DistView dv = {&rd, a.wide_keys ? a.wide_keys + row * a.wide_stride : nullptr,
-                         a.wide_w ? a.wide_w + row * a.wide_stride : nullptr};
-    const dflash_weighted_candidate *pc = a.mode == 1 ? a.prop_cands + a.prop_offsets[row] : nullptr;
-    const int n_pc = a.mode == 1 ? a.prop_counts[row] : 0;
+    const uint64_t *keys = a.wide_keys + row * a.wide_stride;
+    const double *weights = a.wide_w + row * a.wide_stride;
+    const dflash_weighted_candidate *pc = mode == 1 ? a.prop_cands + a.prop_offsets[row] : nullptr;
+    const int n_pc = mode == 1 ? a.prop_counts[row] : 0;
     const double prop_total = o.prop_total;
+    auto token_at = [&](int i) { return static_cast<int32_t>(keys[i] & kWideTokenMask); };
     auto residual_at = [&](int i) {
-        const double p = dv.weight(i) / rd.total;
+        const double p = weights[i] / rd.total;
         double q;
-        if (a.mode == 1) {
-            const int32_t ti = dv.token(i);
+        if (mode == 1) {
+            const int32_t ti = token_at(i);
             double qs = -0.0;
             for (int j = 0; j < n_pc; j++)
                 if (pc[j].token == ti) qs += pc[j].weight;
             q = qs / prop_total;
         } else {
-            // (draft_logit_of: the row's candidates' draft logits, fetched ahead; else they are read here)
-            const float dl = draft_logit_of ? draft_logit_of[i] : a.draft[row * a.draft_stride + dv.token(i)];
+            const float dl = a.draft[row * a.draft_stride + token_at(i)];
             q = exp(static_cast<double>(dl) / static_cast<double>(a.draft_temperature) - rd.d_max_scaled) / prop_total;
         }
         return fmax(p - q, 0.0);
@@ -631,181 +682,137 @@ __device__ void residual_pick(const DecideArgs &a, const RowDist *rows, int row,
     for (int base = 0; base < n_keep; base += 64) {
         const double r = base + lane < n_keep ? residual_at(base + lane) : 0.0;
         const int m = min(64, n_keep - base);
-        for (int j = 0; j < m; j++) residual_total += chain_bcast(r, j);
+        residual_total = chain_bcast(wave_running_sum(residual_total, r, m), m - 1);
     }
     if (!(isfinite(residual_total) && residual_total > 0.0)) {
         o.err = DFLASH_ERR_NO_CANDIDATES;
         return;
     }
-    const double x = a.uniforms[o.residual_draw] * residual_total;
+    const double x = o.u_residual * residual_total;
     int pick = n_keep - 1;
     double cumulative = 0.0;
-    bool found = false;
-    for (int base = 0; base < n_keep && !found; base += 64) {
+    for (int base = 0; base < n_keep; base += 64) {
         const double r = base + lane < n_keep ? residual_at(base + lane) : 0.0;
         const int m = min(64, n_keep - base);
-        for (int j = 0; j < m; j++) {
-            cumulative += chain_bcast(r, j);
-            if (x < cumulative) {
-                pick = base + j;
-                found = true;
-                break;
-            }
+        const double upto = wave_running_sum(cumulative, r, m);
+        const uint64_t above = __builtin_amdgcn_ballot_w64(lane < m && x < upto);
+        if (above) {
+            pick = base + static_cast<int>(__builtin_ctzll(above));
+            break;
         }
+        cumulative = chain_bcast(upto, m - 1);
     }
-    o.token = dv.token(pick);
+    o.token = token_at(pick);
 }
 
-// Thread r evaluates row r (all rows at once); thread 0 then walks the outcomes in order exactly as the serial
-// loop of accept.rs:147-183 does: rows behind the first rejection, stop or error are never looked at.
-// What it spends its time on is the way to its data and its own code: a single wave made sixty requests of tile sums,
-// each with its own branch, out of 16 KB of instructions that nothing has fetched before.  Eight waves ask for
-// everything in eight requests each; the first one decides (16.3 -> 10.2 us for a 16-row block with dense proposals).
-constexpr int kDecThreads = 512;
-__global__ void __launch_bounds__(kDecThreads) decide_kernel(DecideArgs a, dflash_accept_decision *__restrict__ out) {
+// Wave r evaluates row r (all rows at once); the first wave then finds the row at which the serial
+// loop of accept.rs:147-183 stops: rows behind the first rejection, stop or error are never looked at.
+// A chain of latencies: what the kernel reads was written by other XCDs and comes from memory at about two microseconds a
+// trip, so everything is asked for at once, and a draft row's tile sums are 150 dependent additions.  (Rows walked by one wave, each
+// scan over its candidates a loop over LDS, the exponentials and the residual of the row it stops at behind the walk: 13.2 us for
+// a 16-row block with dense proposals.)
+constexpr int kDecThreads = 64 * kMaxRows;
+__global__ void __launch_bounds__(kDecThreads)
+    decide_kernel(const RowDist *__restrict__ rows, const double *__restrict__ tile_sums, dflash_accept_decision *__restrict__ out, int mode,
+                  int n_tiles, int n_tokens, DecideArgs a) {
     constexpr int kStage = 256;  // tile sums per row and round
     __shared__ double p_total[kMaxRows];
-    __shared__ RowOutcome outcome[kMaxRows + 1];
-    // the rows' distributions are walked element by element: they are copied to LDS once, coalesced
-    __shared__ RowDist rows_sh[kMaxRows];
-    __shared__ double staged[kMaxRows][kStage + 1];  // (a row per lane is read: the lanes' banks differ)
-    __shared__ float draft_tok_logit[kMaxRows];
-    __shared__ float resid_logit[kMaxRows][kMaxK];
-    static_assert(sizeof(RowDist) % 8 == 0, "copied as double words");
-    const int tid = threadIdx.x;
-    const int n_drafts = a.n_tokens - 1;
-    const bool dense = a.mode == 2;
-    // What the kernel reads from memory is written by other XCDs and comes from memory at about two microseconds a
-    // trip: everything whose address is known is requested before anything is waited for (the first round of tile
-    // sums, each draft row's logit of its own draft token, the rows), the candidates' draft logits as soon as the
-    // rows are there, and the arithmetic runs on LDS copies.
-    constexpr int kPerRow = kDecThreads / kStage;  // rows a round of requests covers
-    auto tile_sum = [&](int r, int t) { return r < n_drafts && t < a.n_tiles ? a.tile_sums[r * a.n_tiles + t] : 0.0; };
-    double tsum[kMaxRows / kPerRow];
-    float my_logit = 0.0f;
+    __shared__ RowOutcome outcome[kMaxRows];
+    __shared__ alignas(16) double staged[kMaxRows][kStage + 2];  // (a row per lane is read, two sums at a time: the lanes' banks differ)
+    const int tid = threadIdx.x, lane = tid & 63, row = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n_drafts = n_tokens - 1;
+    const bool dense = mode == 2, live = row < n_tokens;
+    const RowDist &rd = rows[live ? row : 0];
+    double sums[kStage / 64];
+#pragma unroll
+    for (int j = 0; j < kStage / 64; j++) sums[j] = dense && row < n_drafts && 64 * j + lane < n_tiles ? tile_sums[row * n_tiles + 64 * j + lane] : 0.0;
+    const int32_t token = rd.tokens[lane];
+    const double weight = rd.weights[lane], q = rd.q[lane];
+    const int draw = a.temperature == 0.0f || !live ? 0 : row;
+    const double u = a.walk.uniforms[draw], u_residual = a.walk.uniforms[draw + 1];
+    bool stop = false;
+    if (row < n_drafts)
+        for (int base = 0; base < a.n_stop; base += 64)
+            stop = stop || __builtin_amdgcn_ballot_w64(base + lane < a.n_stop && a.stop_ids[base + lane < a.n_stop ? base + lane : 0] == a.walk.verified[row + 1]) != 0;
+    const double total = rd.total, p = weight / total, target_probability = rd.draft_weight / total;  // (while the last wave adds)
     if (dense) {
-#pragma unroll
-        for (int j = 0; j < kMaxRows / kPerRow; j++) tsum[j] = tile_sum(kPerRow * j + tid / kStage, tid % kStage);
-        if (tid < n_drafts) my_logit = a.draft[tid * a.draft_stride + a.verified[tid + 1]];
-    }
-    {
-        const uint64_t *src = reinterpret_cast<const uint64_t *>(a.rows);
-        uint64_t *dst = reinterpret_cast<uint64_t *>(rows_sh);
-        const int n_words = a.n_tokens * static_cast<int>(sizeof(RowDist) / 8);
-        constexpr int kRounds = (kMaxRows * static_cast<int>(sizeof(RowDist) / 8) + kDecThreads - 1) / kDecThreads;
-        uint64_t v[kRounds];
-#pragma unroll
-        for (int u = 0; u < kRounds; u++) v[u] = src[min(u * kDecThreads + tid, n_words - 1)];
-#pragma unroll
-        for (int u = 0; u < kRounds; u++)
-            if (u * kDecThreads + tid < n_words) dst[u * kDecThreads + tid] = v[u];
-    }
-    if (dense) {
-#pragma unroll
-        for (int j = 0; j < kMaxRows / kPerRow; j++) staged[kPerRow * j + tid / kStage][tid % kStage] = tsum[j];
-        if (tid < n_drafts) draft_tok_logit[tid] = my_logit;
-    }
-    __syncthreads();
-    const bool prefetched = dense && !a.wide_keys;
-    if (prefetched) {
-#pragma unroll
-        for (int j = 0; j < kMaxRows / (kDecThreads / 64); j++) {
-            const int r = kDecThreads / 64 * j + (tid >> 6), i = tid & 63;
-            resid_logit[r][i] = (r < n_drafts && i < rows_sh[r].n_keep) ? a.draft[r * a.draft_stride + rows_sh[r].tokens[i]] : 0.0f;
-        }
-    }
-    if (dense) {
-        // P = sequential sum of a row's tile sums, in tile order, by thread r from the LDS copies
+        // P = sequential sum of a row's tile sums, in tile order, by lane r of the last wave (its own row has no draft) from the LDS copies
         double P = 0.0;
-        for (int t0 = 0; t0 < a.n_tiles; t0 += kStage) {
-            if (t0 > 0) {  // further rounds (vocabularies above 262144 tokens)
-                __syncthreads();
-                for (int r = tid / kStage; r < n_drafts; r += kPerRow) staged[r][tid % kStage] = tile_sum(r, t0 + tid % kStage);
-                __syncthreads();
-            }
-            if (tid < n_drafts) {
-                // (sixteen read ahead of their additions; past the last tile is +0, which changes no sum of exponentials)
-                const int n = min(kStage, a.n_tiles - t0);
-                for (int i = 0; i < n; i += 16) {
-                    double v[16];
+        for (int t0 = 0;; t0 += kStage) {
 #pragma unroll
-                    for (int j = 0; j < 16; j++) v[j] = staged[tid][i + j];
+            for (int j = 0; j < kStage / 64; j++) staged[row][64 * j + lane] = sums[j];
+            __syncthreads();
+            if (row == kMaxRows - 1 && lane < n_drafts) {
+                // (the next sixteen are read ahead of these sixteen's additions; past the last tile is +0, which changes no sum of
+                // exponentials; the last read ahead is of the next row, which is there: lane 15 has none)
+                const int n = min(kStage, n_tiles - t0);
+                double v[16], next[16];
+#pragma unroll
+                for (int j = 0; j < 16; j++) v[j] = staged[lane][j];
+                for (int i = 0; i < n; i += 16) {
+#pragma unroll
+                    for (int j = 0; j < 16; j++) next[j] = staged[lane][i + 16 + j];
 #pragma unroll
                     for (int j = 0; j < 16; j++) P += v[j];
+#pragma unroll
+                    for (int j = 0; j < 16; j++) v[j] = next[j];
                 }
             }
+            if (t0 + kStage >= n_tiles) break;  // (more rounds: vocabularies above 262144 tokens)
+#pragma unroll
+            for (int j = 0; j < kStage / 64; j++) {
+                const int t = t0 + kStage + 64 * j + lane;
+                sums[j] = row < n_drafts && t < n_tiles ? tile_sums[row * n_tiles + t] : 0.0;
+            }
+            __syncthreads();
         }
-        if (tid < n_drafts) p_total[tid] = P;
+        if (row == kMaxRows - 1 && lane < n_drafts) p_total[lane] = P;
+        __syncthreads();
+    }
+    if (live) {
+        RowOutcome o = decide_row(a, mode, rd, row, token, p, q, target_probability, u, u_residual, dense && row < n_drafts ? p_total[row] : 0.0);
+        o.stop = stop;
+        if (lane == 0) outcome[row] = o;
     }
     __syncthreads();
-    if (tid <= n_drafts) outcome[tid] = decide_row(a, rows_sh, tid, p_total, draft_tok_logit);
-    __syncthreads();
-    if (tid >= 64) return;
-    // The walk, by every lane alike (one wave; everything it reads is uniform): at the row it stops
-    // at, a rejected draft's correction token is drawn by the whole wave.  The decision is put together in LDS and
+    if (row > 0) return;
+    // The decision is put together in LDS and
     // leaves as one coalesced store: `out` may be host memory, where every separate store is a transaction over the
     // bus.
     __shared__ dflash_accept_decision d_sh;
     static_assert(sizeof(dflash_accept_decision) % 4 == 0, "copied as words");
-    int accepted = 0, draws = 0, carry_kind = DFLASH_CARRY_NONE, stop = DFLASH_STOP_NONE, carry_token = 0;
-    int err = 0, err_row = -1;
-    int64_t err_index = -1;
-    for (;;) {
-        const int row = accepted;
-        RowOutcome o = outcome[row];
-        if (!o.err && o.need_residual) residual_pick(a, rows_sh, row, o, prefetched ? resid_logit[row] : nullptr);
-        if (o.err) {
-            err = o.err;
-            err_index = o.err_index;
-            err_row = row;
-            break;
-        }
-        draws += o.draws;
-        if (row == n_drafts) {
-            carry_kind = DFLASH_CARRY_BONUS;
-            carry_token = o.token;
-            break;
-        }
-        if (!o.acc) {
-            carry_kind = DFLASH_CARRY_CORRECTION;
-            carry_token = o.token;
-            break;
-        }
-        const int32_t draft = a.verified[row + 1];
-        accepted++;
-        if (in_list(a.stop_ids, a.n_stop, draft)) {
-            stop = DFLASH_STOP_EOS;
-            break;
-        }
-        if (accepted == a.budget) {
-            stop = DFLASH_STOP_TOKEN_LIMIT;
-            break;
-        }
-    }
-    if (threadIdx.x == 0) {
-        dflash_accept_decision &d = d_sh;
-        memset(&d, 0, sizeof(d));
-        d.err_row = err_row;
-        d.err_index = err_index;
-        if (err) {
-            d.err_code = err;
-        } else {
-            for (int i = 0; i < accepted; i++) d.accepted_drafts[i] = a.verified[i + 1];
-            d.n_accepted = accepted;
-            d.carry_kind = carry_kind;
-            d.carry_token = carry_token;
-            d.stop_reason = stop;
-            d.retain_input_count = 1 + accepted - (stop != DFLASH_STOP_NONE ? 1 : 0);
-            d.draws_used = draws;
+    constexpr int kWords = sizeof(dflash_accept_decision) / 4;
+    static_assert(kWords <= 64, "a word per lane");
+    const RowOutcome &mine = outcome[min(lane, n_drafts)];
+    const int my_draws = mine.draws;
+    const bool ends = lane >= n_drafts || mine.err || !mine.acc || mine.stop || lane + 1 == a.budget;
+    const int at = static_cast<int>(__builtin_ctzll(__builtin_amdgcn_ballot_w64(ends)));
+    RowOutcome o = outcome[at];
+    if (o.need_residual) residual_pick(a, mode, rows[at], at, o);  // (its row has no error of its own)
+    const uint64_t reached = (uint64_t(2) << at) - 1;
+    const int draws = __popcll(__builtin_amdgcn_ballot_w64(my_draws & 1) & reached) + 2 * __popcll(__builtin_amdgcn_ballot_w64(my_draws & 2) & reached);
+    const bool bonus = at == n_drafts, accepted_last = !bonus && o.acc;
+    const int accepted = at + accepted_last, stop_reason = !accepted_last ? DFLASH_STOP_NONE : o.stop ? DFLASH_STOP_EOS : DFLASH_STOP_TOKEN_LIMIT;
+    if (lane < kWords) reinterpret_cast<uint32_t *>(&d_sh)[lane] = 0;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    if (lane < accepted && !o.err) d_sh.accepted_drafts[lane] = a.walk.verified[lane + 1];
+    if (lane == 0) {
+        d_sh.err_row = o.err ? at : -1;
+        d_sh.err_index = o.err ? o.err_index : -1;
+        d_sh.err_code = o.err;
+        if (!o.err) {
+            d_sh.n_accepted = accepted;
+            d_sh.carry_kind = bonus ? DFLASH_CARRY_BONUS : accepted_last ? DFLASH_CARRY_NONE : DFLASH_CARRY_CORRECTION;
+            d_sh.carry_token = accepted_last ? 0 : o.token;
+            d_sh.stop_reason = stop_reason;
+            d_sh.retain_input_count = 1 + accepted - (stop_reason != DFLASH_STOP_NONE ? 1 : 0);
+            d_sh.draws_used = draws;
         }
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
-    {
-        const uint32_t *src = reinterpret_cast<const uint32_t *>(&d_sh);
-        uint32_t *dst = reinterpret_cast<uint32_t *>(out);
-        for (int i = threadIdx.x; i < static_cast<int>(sizeof(dflash_accept_decision) / 4); i += 64) dst[i] = src[i];
-    }
+    if (lane < kWords) reinterpret_cast<uint32_t *>(out)[lane] = reinterpret_cast<const uint32_t *>(&d_sh)[lane];
 }
 
 // ------------------------------------------------------------------------------------------
@@ -905,14 +912,13 @@ int32_t dflash_argmax_greedy(dflash_ctx *ctx, const float *logits, int32_t n_row
     const int n_chunks = static_cast<int>((vocab + kSelChunk - 1) / kSelChunk);
     if (n_chunks > 2 * kSelThreads) return dfl_fail(ctx, DFLASH_ERR_UNSUPPORTED, "argmax_greedy: vocabulary too large");
     size_t off = 0;
-    ChunkOut *chunks = dfl_ws_take<ChunkOut>(ctx, &off, sizeof(ChunkOut) * n_rows * n_chunks);
-    RowDist *rows = dfl_ws_take<RowDist>(ctx, &off, sizeof(RowDist) * n_rows);
-    if (!chunks || !rows) return dfl_fail(ctx, DFLASH_ERR_WORKSPACE, "argmax_greedy: workspace too small");
+    uint64_t *chunks = dfl_ws_take<uint64_t>(ctx, &off, sizeof(uint64_t) * n_rows * n_chunks);
+    if (!chunks) return dfl_fail(ctx, DFLASH_ERR_WORKSPACE, "argmax_greedy: workspace too small");
     ChainCfg cfg = {};
     cfg.k = 1;
     dfl_timed timer(ctx, st, DFL_T_ARGMAX);
-    select_chunk_kernel<<<dim3(n_chunks, n_rows), kSelThreads, 0, st>>>(logits, vocab, stride, 1, chunks, false);
-    row_merge_kernel<<<n_rows, kSelThreads, 0, st>>>(chunks, n_chunks, nullptr, cfg, rows, idx, false);
+    select_chunk_kernel<<<dim3(n_chunks, n_rows), kSelThreads, 0, st>>>(logits, stride, chunks, static_cast<int>(vocab), 1, false);
+    row_merge_kernel<<<n_rows, kSelThreads, 0, st>>>(chunks, nullptr, idx, n_chunks, 1, cfg, BlockWalk{});
     DFL_HIP_CHECK(ctx, hipGetLastError());
     return DFLASH_OK;
 }
@@ -927,10 +933,10 @@ int32_t dflash_top16(dflash_ctx *ctx, const float *logits, int32_t n_rows, int64
     const int n_chunks = static_cast<int>((vocab + kSelChunk - 1) / kSelChunk);
     if (n_chunks * 16 > 2 * kSelThreads) return dfl_fail(ctx, DFLASH_ERR_UNSUPPORTED, "top16: vocabulary too large");
     size_t off = 0;
-    ChunkOut *chunks = dfl_ws_take<ChunkOut>(ctx, &off, sizeof(ChunkOut) * n_rows * n_chunks);
+    uint64_t *chunks = dfl_ws_take<uint64_t>(ctx, &off, sizeof(uint64_t) * 16 * n_rows * n_chunks);
     if (!chunks) return dfl_fail(ctx, DFLASH_ERR_WORKSPACE, "top16: workspace too small");
     dfl_timed timer(ctx, st, DFL_T_ARGMAX);
-    select_chunk_kernel<<<dim3(n_chunks, n_rows), kSelThreads, 0, st>>>(logits, vocab, stride, 16, chunks, true);
+    select_chunk_kernel<<<dim3(n_chunks, n_rows), kSelThreads, 0, st>>>(logits, stride, chunks, static_cast<int>(vocab), 16, true);
     top16_merge_kernel<<<n_rows, kSelThreads, 0, st>>>(chunks, n_chunks, ids, vals);
     DFL_HIP_CHECK(ctx, hipGetLastError());
     return DFLASH_OK;
@@ -1048,22 +1054,24 @@ int32_t dflash_accept_prefix(dflash_ctx *ctx, const int32_t *verified, int32_t n
     hipStream_t st = static_cast<hipStream_t>(stream);
     const int n_tiles = static_cast<int>((vocab + 1023) / 1024);
     size_t off = 0;
-    ChunkOut *chunks = dfl_ws_take<ChunkOut>(ctx, &off, sizeof(ChunkOut) * n_tokens * n_chunks);
-    ChunkOut *dchunks = dfl_ws_take<ChunkOut>(ctx, &off, sizeof(ChunkOut) * n_tokens * n_chunks);
+    // (wide sets order their candidates elsewhere: no lists of the target's chunks)
+    uint64_t *chunks = dfl_ws_take<uint64_t>(ctx, &off, sizeof(uint64_t) * (wide ? 0 : k_eff) * n_tokens * n_chunks);
+    uint64_t *draft_best = dfl_ws_take<uint64_t>(ctx, &off, sizeof(uint64_t) * n_tokens * n_chunks);
     RowDist *rows = dfl_ws_take<RowDist>(ctx, &off, sizeof(RowDist) * n_tokens);
     double *tile_sums = dfl_ws_take<double>(ctx, &off, sizeof(double) * n_tokens * n_tiles);
     int32_t *d_stop = dfl_ws_take<int32_t>(ctx, &off, sizeof(int32_t) * (n_stop + 8));
     dflash_weighted_candidate *d_cands =
         dfl_ws_take<dflash_weighted_candidate>(ctx, &off, sizeof(dflash_weighted_candidate) * (n_cands + 1));
     dflash_accept_decision *d_out = dfl_ws_take<dflash_accept_decision>(ctx, &off, sizeof(dflash_accept_decision));
-    if (!chunks || !dchunks || !rows || !tile_sums || !d_stop || !d_cands || !d_out)
+    if (!chunks || !draft_best || !rows || !tile_sums || !d_stop || !d_cands || !d_out)
         return dfl_fail(ctx, DFLASH_ERR_WORKSPACE, "accept_prefix: workspace too small");
 
     // small host inputs: by value in the decision kernel's arguments; only the variable-length lists are copied
     DecideArgs a;
     memset(&a, 0, sizeof(a));
-    dflash_sampler_peek(sampler, n_tokens + 1, a.uniforms);
-    for (int i = 0; i < n_tokens; i++) a.verified[i] = verified[i];
+    dflash_sampler_peek(sampler, n_tokens + 1, a.walk.uniforms);
+    a.walk.n_tokens = n_tokens;
+    for (int i = 0; i < n_tokens; i++) a.walk.verified[i] = verified[i];
     for (int r = 0; r < n_drafts && mode == 1; r++) {
         a.prop_offsets[r] = prop_offsets[r];
         a.prop_counts[r] = prop_counts[r];
@@ -1088,43 +1096,33 @@ int32_t dflash_accept_prefix(dflash_ctx *ctx, const int32_t *verified, int32_t n
         const uint64_t *wide_keys = nullptr;
         const double *wide_w = nullptr;
         if (wide) {
-            WideWalk walk = {};
-            walk.n_tokens = n_tokens;
-            for (int i = 0; i < n_tokens; i++) walk.verified[i] = verified[i];
-            for (int i = 0; i <= n_tokens; i++) walk.uniforms[i] = a.uniforms[i];
-            if (const int32_t rc_ = dfl_accept_wide_rows(ctx, target_logits, n_tokens, vocab, vocab, cfg, walk, rows, &off, &wide_keys, &wide_w,
+            if (const int32_t rc_ = dfl_accept_wide_rows(ctx, target_logits, n_tokens, vocab, vocab, cfg, a.walk, rows, &off, &wide_keys, &wide_w,
                                                          &a.wide_stride, st))
                 return rc_;
-            if (dense) select_chunk_kernel<<<dim3(n_chunks, n_drafts), kSelThreads, 0, st>>>(draft_logits, vocab, vocab, 1, dchunks, false);
+            if (dense) select_chunk_kernel<<<dim3(n_chunks, n_drafts), kSelThreads, 0, st>>>(draft_logits, vocab, draft_best, static_cast<int>(vocab), 1, false);
         } else if (dense) {
-            select_pair_kernel<<<dim3(n_chunks, n_tokens + n_drafts), kSelThreads, 0, st>>>(target_logits, n_tokens, cfg.k, chunks,
-                                                                                         draft_logits, dchunks, vocab, vocab);
+            select_pair_kernel<<<dim3(n_chunks, n_tokens + n_drafts), kSelThreads, 0, st>>>(target_logits, draft_logits, vocab, chunks, draft_best,
+                                                                                         static_cast<int>(vocab), n_tokens, cfg.k);
         } else {
-            select_chunk_kernel<<<dim3(n_chunks, n_tokens), kSelThreads, 0, st>>>(target_logits, vocab, vocab, cfg.k, chunks, false);
+            select_chunk_kernel<<<dim3(n_chunks, n_tokens), kSelThreads, 0, st>>>(target_logits, vocab, chunks, static_cast<int>(vocab), cfg.k, false);
         }
-        // the rows' chains and, for dense proposals, the tile sums of the draft rows: one launch
+        // the rows' chains and, for dense proposals, the tile sums of the draft rows: one launch (wide: the chain has run; only the
+        // draft side is merged)
         if (dense) {
-            const int blocks_per_row = (n_tiles + 7) / 8;
-            const int n_row_wgs = wide ? n_drafts : n_tokens;  // (wide: the chain has run; only the draft side is merged)
-            rows_and_tiles_kernel<<<n_row_wgs + n_drafts * blocks_per_row, kSelThreads, 0, st>>>(
-                chunks, n_chunks, dchunks, cfg, rows, n_row_wgs, wide, draft_logits, vocab, vocab, n_tiles, blocks_per_row, tile_sums);
+            rows_and_tiles_kernel<<<dim3(n_tokens, 1 + (n_tiles + 3) / 4), kSelThreads, 0, st>>>(
+                chunks, draft_logits, draft_best, tile_sums, static_cast<int>(vocab), n_chunks, cfg.k, n_tokens, draft_temperature, n_tiles, rows, wide,
+                cfg, a.walk);
         } else if (!wide) {
-            row_merge_kernel<<<n_tokens, kSelThreads, 0, st>>>(chunks, n_chunks, nullptr, cfg, rows, nullptr, false);
+            row_merge_kernel<<<n_tokens, kSelThreads, 0, st>>>(chunks, rows, nullptr, n_chunks, cfg.k, cfg, a.walk);
         }
         a.wide_keys = wide_keys;
         a.wide_w = wide_w;
-        a.n_tokens = n_tokens;
         a.n_stop = n_stop;
-        a.mode = mode;
-        a.vocab = static_cast<int32_t>(vocab);
         a.budget = budget;
         a.stop_ids = d_stop;
-        a.rows = rows;
         a.prop_cands = d_cands;
         a.draft = draft_logits;
         a.draft_stride = vocab;
-        a.tile_sums = tile_sums;
-        a.n_tiles = n_tiles;
         a.temperature = sc.temperature;
         a.draft_temperature = draft_temperature;
         // the decision goes straight to the context's pinned page when the device can address it (one copy less
@@ -1133,7 +1131,8 @@ int32_t dflash_accept_prefix(dflash_ctx *ctx, const int32_t *verified, int32_t n
         void *pinned_dev = nullptr;
         const bool direct = ctx->pinned && hipHostGetDevicePointer(&pinned_dev, ctx->pinned, 0) == hipSuccess && pinned_dev;
         if (!direct) (void)hipGetLastError();
-        decide_kernel<<<1, kDecThreads, 0, st>>>(a, direct ? static_cast<dflash_accept_decision *>(pinned_dev) : d_out);
+        decide_kernel<<<1, kDecThreads, 0, st>>>(rows, tile_sums, direct ? static_cast<dflash_accept_decision *>(pinned_dev) : d_out, mode, n_tiles,
+                                                 n_tokens, a);
         DFL_HIP_CHECK(ctx, hipGetLastError());
         if (!direct) DFL_HIP_CHECK(ctx, hipMemcpyAsync(ctx->pinned, d_out, sizeof(*out), hipMemcpyDeviceToHost, st));
     }

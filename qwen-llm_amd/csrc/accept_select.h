@@ -15,13 +15,13 @@ struct KthShared {
     int n[THREADS / 64];
 };
 
-// A bound B <= limit such that exactly k of the workgroup's keys are <= B; limit if no more than k are <= limit.
+// A bound B <= limit such that at least k and at most `most` >= k of the workgroup's keys are <= B; limit if no more than k are <= limit.
 // Digit by digit from the first bit in which the keys differ (most share sign and most of the exponent: a digit
-// above it would put every key on one counter), and no further than until a digit's counts end at k.  Keys are
-// distinct, so the last digit ends there at the latest.  One barrier per digit: every wave adds up the counters by
+// above it would put every key on one counter), and no further than until a digit's counts end there.  Keys are
+// distinct, so the last digit ends at k at the latest.  One barrier per digit: every wave adds up the counters by
 // itself, and of three sets of counters one is counted in, one may still be read, one is cleared for the next digit.
 template <int PER, int THREADS>
-__device__ uint64_t block_kth(const uint64_t (&key)[PER], uint64_t limit, int k, KthShared<THREADS> &sh) {
+__device__ uint64_t block_kth(const uint64_t (&key)[PER], uint64_t limit, int k, int most, KthShared<THREADS> &sh) {
     constexpr int kWaves = THREADS / 64;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     uint64_t lo = kNoKey, hi = 0;
@@ -46,6 +46,7 @@ __device__ uint64_t block_kth(const uint64_t (&key)[PER], uint64_t limit, int k,
     hi = ~wave_min_u64(lane < kWaves ? ~sh.hi[lane] : kNoKey);
     n = __builtin_amdgcn_readlane(wave_scan_i32(lane < kWaves ? sh.n[lane] : 0), 63);
     if (n <= k) return limit;
+    const int slack = most - k;
     int shift = 64 - __clzll(static_cast<long long>(lo ^ hi));  // 1 .. 64: n > k >= 1 distinct keys
     uint64_t prefix = (lo >> 1) >> (shift - 1);
     for (int set = 0;; set = set == 2 ? 0 : set + 1) {
@@ -66,36 +67,67 @@ __device__ uint64_t block_kth(const uint64_t (&key)[PER], uint64_t limit, int k,
         k -= __builtin_amdgcn_readlane(below, from);
         prefix = (prefix << (shift - digit)) | static_cast<uint64_t>(__builtin_amdgcn_readlane(bin, from));
         shift = digit;
-        if (__builtin_amdgcn_readlane(count, from) == k) return (prefix << shift) | ((uint64_t(1) << shift) - 1);
+        if (__builtin_amdgcn_readlane(count, from) - k <= slack) return (prefix << shift) | ((uint64_t(1) << shift) - 1);
     }
 }
 
-template <int PER>
-__device__ __forceinline__ uint64_t thread_best(const uint64_t (&key)[PER]) {
-    uint64_t best = kNoKey;
-#pragma unroll
-    for (int j = 0; j < PER; j++) best = key[j] < best ? key[j] : best;
-    return best;
+// The same over ordering words, one a thread, which may be alike: a bound that at least k of them are at or below (the largest word
+// if there are no k) and, as far as the words differ, at most `most`.  Bins of the words' own range, 128 to 256 of them, so that
+// one round is nearly always the last; a word is one instruction a step where a key is five (2.2 -> 1.1 us of a workgroup of 512).
+template <int THREADS>
+__device__ __forceinline__ uint32_t block_kth_word(uint32_t word, int k, int most, KthShared<THREADS> &sh) {
+    constexpr int kWaves = THREADS / 64;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, slack = most - k;
+    {
+        const uint32_t lo = wave_min_u32(word), hi = wave_max_u32(word);
+        if (lane == 0) sh.lo[wave] = (static_cast<uint64_t>(hi) << 32) | lo;
+    }
+    if (tid < 256) sh.hist[0][tid] = 0;
+    __syncthreads();
+    const uint64_t ends = sh.lo[lane < kWaves ? lane : 0];
+    uint32_t lo = wave_min_u32(static_cast<uint32_t>(ends));
+    const uint32_t hi = wave_max_u32(static_cast<uint32_t>(ends >> 32));
+    if (k >= THREADS || lo == hi) return hi;
+    int shift = max(0, 24 - __clz(hi - lo));  // ((hi - lo) >> shift < 256)
+    for (int set = 0;; set = set == 2 ? 0 : set + 1) {
+        const uint32_t bin_of = (word - lo) >> shift;
+        if (word >= lo && bin_of < 256) atomicAdd(&sh.hist[set][bin_of], 1);
+        if (tid < 256) sh.hist[set == 2 ? 0 : set + 1][tid] = 0;
+        __syncthreads();
+        const int4 c = *reinterpret_cast<const int4 *>(&sh.hist[set][4 * lane]);
+        const int upto = wave_scan_i32(c.x + c.y + c.z + c.w);
+        int below = upto - (c.x + c.y + c.z + c.w), bin = 4 * lane, count = c.x;
+        const bool here = below < k && k <= upto;  // in one lane
+        if (below + count < k) below += count, bin++, count = c.y;
+        if (bin == 4 * lane + 1 && below + count < k) below += count, bin++, count = c.z;
+        if (bin == 4 * lane + 2 && below + count < k) below += count, bin++, count = c.w;
+        const int from = __builtin_ctzll(__builtin_amdgcn_ballot_w64(here));
+        k -= __builtin_amdgcn_readlane(below, from);
+        lo += static_cast<uint32_t>(__builtin_amdgcn_readlane(bin, from)) << shift;
+        if (shift == 0 || __builtin_amdgcn_readlane(count, from) - k <= slack) return lo + min((uint32_t(1) << shift) - 1, hi - lo);  // (the last bin may end above every word)
+        shift = max(0, shift - 8);
+    }
 }
 
 // The workgroup's keys <= bound to the slots [0, cap) of out, in no order, as far as they fit; *cnt (0 before) becomes
-// their number.  A wave asks for its slots with one addition.
+// their number.  A wave asks for its slots with one addition, and a thread's are next to each other.
 template <int PER>
-__device__ void compact_keys(const uint64_t (&key)[PER], uint64_t bound, uint64_t *out, int cap, int *cnt) {
+__device__ __forceinline__ void compact_keys(const uint64_t (&key)[PER], uint64_t bound, uint64_t *out, int cap, int *cnt) {
     const int lane = threadIdx.x & 63;
     int n = 0;
 #pragma unroll
-    for (int j = 0; j < PER; j++) n += __popcll(__builtin_amdgcn_ballot_w64(key[j] <= bound));
-    if (n == 0) return;
+    for (int j = 0; j < PER; j++) n += key[j] <= bound;
+    const int upto = wave_scan_i32(n), all = __builtin_amdgcn_readlane(upto, 63);
+    if (all == 0) return;
     int at = 0;
-    if (lane == 0) at = atomicAdd(cnt, n);
-    at = __builtin_amdgcn_readfirstlane(at);
+    if (lane == 0) at = atomicAdd(cnt, all);
+    at = __builtin_amdgcn_readfirstlane(at) + upto - n;
 #pragma unroll
     for (int j = 0; j < PER; j++) {
-        const uint64_t m = __builtin_amdgcn_ballot_w64(key[j] <= bound);
-        const int slot = at + __popcll(m & ((uint64_t(1) << lane) - 1));
-        if (key[j] <= bound && slot < cap) out[slot] = key[j];
-        at += __popcll(m);
+        if (key[j] <= bound) {
+            if (at < cap) out[at] = key[j];
+            at++;
+        }
     }
 }
 

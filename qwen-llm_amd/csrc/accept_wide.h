@@ -8,18 +8,10 @@
 constexpr int kWideTokenBits = 28;
 constexpr uint64_t kWideTokenMask = (uint64_t(1) << kWideTokenBits) - 1;
 
-// What the block's decision asks of a row's ordered candidates: row r's draw is uniforms[r] (every row before it
-// accepted, each with one draw) and its draft verified[r + 1].
-struct WideWalk {
-    int32_t n_tokens;
-    int32_t verified[16];
-    double uniforms[17];
-};
-
 // Orders every row of logits [n_rows][stride] (n_rows <= 16, vocab < 2^28) and runs the sampler chain on it for
 // an effective top-k above kMaxK.  rows[r] receives n_keep / err / err_index / total / pick / draft_weight; row r's
 // kept candidates are, best first, the tokens (key & kWideTokenMask) of (*keys_out)[r * *out_stride ..] with weights
 // (*weights_out)[r * *out_stride ..].  Device arrays come from the context workspace at *ws_off.  Enqueue only.
 int32_t dfl_accept_wide_rows(dflash_ctx *ctx, const float *logits, int32_t n_rows, int64_t vocab, int64_t stride, const ChainCfg &cfg,
-                             const WideWalk &walk, RowDist *rows, size_t *ws_off, const uint64_t **keys_out, const double **weights_out,
+                             const BlockWalk &walk, RowDist *rows, size_t *ws_off, const uint64_t **keys_out, const double **weights_out,
                              int64_t *out_stride, hipStream_t st);

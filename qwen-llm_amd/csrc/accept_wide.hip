@@ -8,8 +8,8 @@
 // Two ways.  A set of at most kPickMax candidates (the chat preset's 200) is selected, not sorted: a workgroup per
 // 8192 tokens finds its own k smallest keys, a workgroup per row the k smallest of those, ranks them by counting and
 // runs the chain with a candidate per thread.  Two launches that read the logits once, each bound
-// by its chain of barriers and LDS round trips (the logits take 2 us): 16 rows x 151936 tokens, k = 200: 11.2 + 12.9 us
-// where the sort, its 17 clears and its chain take 316; the whole call 334 -> 44.5 us.
+// by its chain of barriers and LDS round trips (the logits take 2 us): 16 rows x 151936 tokens, k = 200: 8.4 + 9.4 us
+// where the sort, its 17 clears and its chain take 316; the whole call 334 -> 38 us.
 // Anything larger (the whole vocabulary) is ordered by ONE device-wide radix sort: a key is
 //   row << 60 | descending_logit_bits << 28 | token          (token < 2^28, row < 16)
 // and ascending key order is (row, descending logit in f32 total order, ascending token id): row r's
@@ -65,6 +65,12 @@ constexpr int kPickChunk = 8192;  // tokens per workgroup: 16 rows of 151936 are
 constexpr int kPickMax = 1024;    // threads of the row kernel: a candidate each
 constexpr int kPickSlots = 16 * kPickMax;  // chunk winners of a row that its workgroup holds in registers
 
+// The largest key of a row with at most this ordering word.
+__device__ __forceinline__ uint64_t wide_bound(int row, uint32_t word) {
+    const uint64_t bound = (static_cast<uint64_t>(row) << 60) | (static_cast<uint64_t>(word) << kWideTokenBits) | kWideTokenMask;
+    return bound < kNoKey ? bound : kNoKey - 1;
+}
+
 // A chunk's winners, the k best keys and at most cap >= k, in no order, at out[(row * n_chunks + chunk) * cap], filled up
 // with kNoKey; the chunk's lowest NaN token.  The k-th best of the per-thread bests bounds every winner, and what is
 // below it usually fits the slots (k = 200: about 250 keys); only where it does not, the k best of all are looked for.
@@ -86,6 +92,7 @@ __global__ void __launch_bounds__(kPickThreads)
     }
     __syncthreads();
     uint64_t key[kPer];
+    uint32_t best = 0xffffffffu;
 #pragma unroll
     for (int j = 0; j < kPer; j++) {
         const int64_t i = base + j * kPickThreads;
@@ -94,16 +101,16 @@ __global__ void __launch_bounds__(kPickThreads)
         key[j] = i < vocab && !nan ? (static_cast<uint64_t>(row) << 60) |
                                          (static_cast<uint64_t>(desc_bits(__float_as_uint(v[j]))) << kWideTokenBits) | static_cast<uint64_t>(i)
                                    : kNoKey;
+        best = min(best, static_cast<uint32_t>(key[j] >> kWideTokenBits));
     }
-    const uint64_t best[1] = {thread_best(key)};
-    uint64_t bound = block_kth<1>(best, kNoKey - 1, k, sh);
+    uint64_t bound = wide_bound(row, block_kth_word(best, k, k + k / 8, sh));
     const int64_t at = static_cast<int64_t>(row) * gridDim.x + blockIdx.x;
     uint64_t *o = out + at * cap;
     compact_keys(key, bound, o, cap, &cnt[0]);
     __syncthreads();
     int n = cnt[0];
     if (n > cap) {
-        bound = block_kth<kPer>(key, bound, k, sh);
+        bound = block_kth<kPer>(key, bound, k, k, sh);
         compact_keys(key, bound, o, cap, &cnt[1]);
         n = k;
     }
@@ -116,7 +123,7 @@ __global__ void __launch_bounds__(kPickThreads)
 template <int PER>
 __global__ void __launch_bounds__(kPickMax)
     pick_row_kernel(const uint64_t *__restrict__ chunk_keys, const int32_t *__restrict__ chunk_nan, int n_chunks, int cap, ChainCfg cfg,
-                    WideWalk walk, RowDist *__restrict__ rows, uint64_t *__restrict__ keys_out, double *__restrict__ weights) {
+                    BlockWalk walk, RowDist *__restrict__ rows, uint64_t *__restrict__ keys_out, double *__restrict__ weights) {
     constexpr int kFold = 16;  // additions per round of the sum
     __shared__ KthShared<kPickMax> sh;
     __shared__ uint64_t cand[kPickMax], sorted[kPickMax];
@@ -126,11 +133,13 @@ __global__ void __launch_bounds__(kPickMax)
     const int row = blockIdx.x, tid = threadIdx.x, k = cfg.k, n_in = n_chunks * cap;
     RowDist *d = rows + row;
     uint64_t key[PER];
+    uint32_t best = 0xffffffffu;
 #pragma unroll
     for (int j = 0; j < PER; j++) {
         const int i = j * kPickMax + tid;
         const uint64_t got = chunk_keys[static_cast<int64_t>(row) * n_in + (i < n_in ? i : 0)];
         key[j] = i < n_in ? got : kNoKey;
+        best = min(best, static_cast<uint32_t>(key[j] >> kWideTokenBits));
     }
     const int nan = tid < n_chunks ? chunk_nan[row * n_chunks + tid] : kNoNanW;  // (n_chunks <= kPickSlots / k < kPickMax)
     rank_sh[tid] = 0;
@@ -140,8 +149,7 @@ __global__ void __launch_bounds__(kPickMax)
     }
     __syncthreads();
     if (nan != kNoNanW) atomicMin(&nan_sh, nan);
-    const uint64_t best[1] = {thread_best(key)};
-    uint64_t bound = block_kth<1>(best, kNoKey - 1, k, sh);  // (its barriers are behind the minimum)
+    uint64_t bound = wide_bound(row, block_kth_word(best, k, k + k / 8, sh));  // (its barriers are behind the minimum)
     auto finish = [&](int32_t err, int64_t err_index, int n_keep, double total, int32_t pick, double draft_weight) {
         if (tid == 0) {
             d->n_keep = n_keep;
@@ -159,21 +167,29 @@ __global__ void __launch_bounds__(kPickMax)
     __syncthreads();
     int n = cnt[0];
     if (n > kPickMax) {
-        bound = block_kth<PER>(key, bound, k, sh);
+        bound = block_kth<PER>(key, bound, k, kPickMax, sh);
         compact_keys(key, bound, cand, kPickMax, &cnt[1]);
         __syncthreads();
         n = cnt[1];
     }
     {
-        // candidate i = tid % n counts the candidates below it in slice tid / n of the list
-        const int slices = kPickMax / n, i = tid % n, sl = tid / n;
-        if (sl < slices) {
-            const int per = (n + slices - 1) / slices, j0 = sl * per, j1 = min(n, j0 + per);
-            const uint64_t x = cand[i];
-            int c = 0;
-#pragma unroll 8
-            for (int j = j0; j < j1; j++) c += cand[j] < x;
-            if (c) atomicAdd(&rank_sh[i], c);
+        // A wave takes a sixteenth of the list and counts, for four candidates a lane, those of it that are below them: an element is
+        // read from LDS once for 256 candidates (each thread with one candidate and a longer slice: 2.2 us for 228 of them, 1.1 now).
+        const int lane = tid & 63, per = (n + kPickMax / 64 - 1) / (kPickMax / 64), j0 = (tid >> 6) * per, j1 = min(n, j0 + per);
+        for (int i0 = 0; i0 < n; i0 += 256) {
+            uint64_t x[4];
+            int c[4] = {0, 0, 0, 0};
+#pragma unroll
+            for (int u = 0; u < 4; u++) x[u] = cand[min(i0 + 64 * u + lane, n - 1)];
+#pragma unroll 4
+            for (int j = j0; j < j1; j++) {
+                const uint64_t y = cand[j];
+#pragma unroll
+                for (int u = 0; u < 4; u++) c[u] += y < x[u];
+            }
+#pragma unroll
+            for (int u = 0; u < 4; u++)
+                if (c[u] && i0 + 64 * u + lane < n) atomicAdd(&rank_sh[i0 + 64 * u + lane], c[u]);
         }
     }
     __syncthreads();
@@ -192,8 +208,7 @@ __global__ void __launch_bounds__(kPickMax)
     } else {
         const double temperature = static_cast<double>(cfg.temperature), max_logit = l0 / temperature;
         if (max_logit == -INFINITY) return finish(DFLASH_ERR_NO_CANDIDATES, -1, 0, 0.0, 0, -0.0);
-        if (tid < len) w = exp(l / temperature - max_logit);
-        if (__syncthreads_or(!isfinite(w))) return finish(DFLASH_ERR_NO_CANDIDATES, -1, 0, 0.0, 0, -0.0);
+        if (tid < len) w = exp(l / temperature - max_logit);  // (no logit is above the first, which is finite: at most 1)
     }
     w_sh[tid] = w;
     if (tid < len) {
@@ -309,7 +324,7 @@ __device__ double sequential_fold(const double *__restrict__ w, int64_t n, doubl
 
 // sampling.rs:1541-1615 on the ordered candidates of one row; weights[row * vocab + i] receives candidate i's weight
 __global__ void __launch_bounds__(kWideThreads)
-    wide_chain_kernel(const uint64_t *__restrict__ keys_sorted, int64_t vocab, ChainCfg cfg, WideWalk walk,
+    wide_chain_kernel(const uint64_t *__restrict__ keys_sorted, int64_t vocab, ChainCfg cfg, BlockWalk walk,
                       const int32_t *__restrict__ nan_first, RowDist *__restrict__ rows, double *__restrict__ weights) {
     __shared__ double tile[kWideTile];
     __shared__ int64_t red[kWideThreads / 64];
@@ -388,7 +403,7 @@ __global__ void __launch_bounds__(kWideThreads)
 }  // namespace
 
 int32_t dfl_accept_wide_rows(dflash_ctx *ctx, const float *logits, int32_t n_rows, int64_t vocab, int64_t stride, const ChainCfg &cfg,
-                             const WideWalk &walk, RowDist *rows, size_t *ws_off, const uint64_t **keys_out, const double **weights_out,
+                             const BlockWalk &walk, RowDist *rows, size_t *ws_off, const uint64_t **keys_out, const double **weights_out,
                              int64_t *out_stride, hipStream_t st) {
     if (n_rows > 16 || vocab >= (int64_t(1) << kWideTokenBits))
         return dfl_fail(ctx, DFLASH_ERR_UNSUPPORTED, "accept_prefix: wide top-k needs <= 16 rows and a vocabulary below 2^28");

@@ -26,10 +26,20 @@ struct RowDist {
     double weights[kMaxK];
     // dense proposal side
     int32_t d_err;
-    int32_t pick;  // wide sets: the token the row's draw falls on
+    int32_t pick;  // the token the row's draw falls on
     int64_t d_err_index;
     double d_max_scaled;  // f64(max draft logit) / T
-    double draft_weight;  // wide sets: weight of the row's draft among the kept candidates, -0 if it is not one
+    double draft_weight;  // weight of the row's draft among the kept candidates, -0 if it is not one
+    double q_draft;       // exp(draft's draft logit / T - d_max_scaled)
+    double q[kMaxK];      // the same of the kept candidates (inline sets)
+};
+
+// What the block's decision asks of a row's candidates: row r's draw is uniforms[r] (every row before it accepted,
+// each with one draw) and its draft verified[r + 1].
+struct BlockWalk {
+    int32_t n_tokens;
+    int32_t verified[16];
+    double uniforms[17];
 };
 
 struct ChainCfg {
@@ -93,6 +103,24 @@ __device__ __forceinline__ int wave_scan_i32(int v) {
 #undef DFL_SUM_STEP
     return v;
 }
+
+// Minimum / maximum of a word over the wave, in every lane: the same moves, one instruction each.
+__device__ __forceinline__ uint32_t wave_min_u32(uint32_t v) {
+#define DFL_MIN_STEP(ctrl, row_mask)                                                                                            \
+    do {                                                                                                                        \
+        const uint32_t o = __builtin_amdgcn_update_dpp(0xffffffffu, v, ctrl, row_mask, 0xf, false);                             \
+        v = o < v ? o : v;                                                                                                      \
+    } while (0)
+    DFL_MIN_STEP(0x111, 0xf);
+    DFL_MIN_STEP(0x112, 0xf);
+    DFL_MIN_STEP(0x114, 0xf);
+    DFL_MIN_STEP(0x118, 0xf);
+    DFL_MIN_STEP(0x142, 0xa);
+    DFL_MIN_STEP(0x143, 0xc);
+#undef DFL_MIN_STEP
+    return __builtin_amdgcn_readlane(v, 63);
+}
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) { return ~wave_min_u32(~v); }
 
 // sampling.rs:1541-1615 on the ordered candidates of one row (keys ascending = best first)
 // Work arrays of the chain (kMaxK entries each): a caller that runs the chain on one thread of a workgroup
@@ -195,63 +223,65 @@ __device__ __forceinline__ double chain_bcast(double v, int src) {
     return __longlong_as_double(static_cast<long long>((static_cast<unsigned long long>(hi) << 32) | lo));
 }
 
+// Lane i: start + w[0] + .. + w[i], added in that order, one after the other; w of the lanes from len on is +0 (len <= 64,
+// uniform).  The lanes' values are read at constant positions, sixteen a round, and move down by sixteen for the next: a
+// read at a position that is itself in a register, with its loop, is 70 cycles an addition, this is 30.
+__device__ __forceinline__ double wave_running_sum(double start, double w, int len) {
+    const int lane = threadIdx.x & 63;
+    double acc = start, mine = start;
+#pragma unroll 1
+    for (int base = 0; base < len; base += 16) {
+#pragma unroll
+        for (int j = 0; j < 16; j++) {
+            acc += chain_bcast(w, j);
+            mine = lane - base >= j ? acc : mine;
+        }
+        w = __shfl(w, lane + 16, 64);
+    }
+    return mine;
+}
+// The first lane of [0, len) for which `reached` holds, or len - 1.
+__device__ __forceinline__ int wave_first(bool reached, int len) {
+    const uint64_t m = __builtin_amdgcn_ballot_w64(static_cast<int>(threadIdx.x & 63) < len && reached);
+    return m ? static_cast<int>(__builtin_ctzll(m)) : len - 1;
+}
+
 // run_chain by one whole wave (len <= 64): lane i holds candidate i.  What the reference does element by element
 // without carrying anything from one element to the next (the conversions, the division by the temperature, the
 // exponentials, the filters' comparisons) is done by all lanes at once; every sum that is compared with something is
-// still added in candidate order, one addition after the other, on values that are the same bits as run_chain's.
-// The candidates are in descending logit order, so what min-p and the +inf rule keep is a prefix: its length is a
-// population count.
-__device__ void run_chain_wave(const uint64_t *keys, int len, const ChainCfg &c, RowDist *d) {
+// still added in candidate order, one addition after the other: each is one of the running sums of the weights (from
+// +0 or -0 is the same, no weight is below +0), so they are added up once.  The candidates are in descending logit
+// order, so what min-p and the +inf rule keep is a prefix: its length is a population count.
+struct WaveChain {
+    int len;          // candidates kept, 0 = none (uniform)
+    double w, upto;   // lane i: its weight, the running sum up to it
+    double total;     // of the kept ones (uniform)
+};
+__device__ __forceinline__ WaveChain run_chain_wave(float logit, int len, const ChainCfg &c) {
     const int lane = threadIdx.x & 63;
-    double l = lane < len ? static_cast<double>(key_logit(keys[lane])) : 0.0;
-    const int tok = lane < len ? key_token(keys[lane]) : 0;
-    auto fail = [&]() {
-        if (lane == 0) d->err = DFLASH_ERR_NO_CANDIDATES;
-    };
-    if (c.min_p > 0.0f && len > 0) {
-        const double max_logit = chain_bcast(l, 0);
-        if (isfinite(max_logit)) {
-            const double threshold = max_logit + c.ln_min_p;
-            len = __popcll(__builtin_amdgcn_ballot_w64(lane < len && l >= threshold));
-        }
-    }
-    if (len == 0) return fail();
-    if (chain_bcast(l, 0) == INFINITY) len = __popcll(__builtin_amdgcn_ballot_w64(lane < len && l == INFINITY));
+    WaveChain r = {0, 0.0, 0.0, 0.0};
+    double l = lane < len ? static_cast<double>(logit) : 0.0;
+    const double l0 = chain_bcast(l, 0);
+    if (c.min_p > 0.0f && len > 0 && isfinite(l0)) len = __popcll(__builtin_amdgcn_ballot_w64(lane < len && l >= l0 + c.ln_min_p));
+    if (len == 0) return r;
+    if (l0 == INFINITY) len = __popcll(__builtin_amdgcn_ballot_w64(lane < len && l == INFINITY));
     l = l / static_cast<double>(c.temperature);
-    const int n_inf = __popcll(__builtin_amdgcn_ballot_w64(lane < len && l == INFINITY));
-    double w;
-    if (n_inf > 0) {
-        w = (l == INFINITY) ? 1.0 : 0.0;
+    const double max_logit = chain_bcast(l, 0);
+    if (max_logit == INFINITY) {
+        r.w = lane < len && l == INFINITY ? 1.0 : 0.0;
     } else {
-        const double max_logit = chain_bcast(l, 0);
-        if (max_logit == -INFINITY) return fail();
-        w = lane < len ? exp(l - max_logit) : 0.0;
-        if (__builtin_amdgcn_ballot_w64(lane < len && !isfinite(w)) != 0) return fail();
+        if (max_logit == -INFINITY) return r;
+        r.w = lane < len ? exp(l - max_logit) : 0.0;
+        if (__builtin_amdgcn_ballot_w64(!isfinite(r.w)) != 0) return r;
     }
+    r.upto = wave_running_sum(0.0, r.w, len);
     if (c.top_p < 1.0f) {
-        double total = -0.0;
-        for (int i = 0; i < len; i++) total += chain_bcast(w, i);
-        const double target = total * static_cast<double>(c.top_p);
-        double cumulative = 0.0;
-        int keep = 0;
-        for (int i = 0; i < len; i++) {
-            cumulative += chain_bcast(w, i);
-            keep++;
-            if (cumulative >= target) break;
-        }
-        len = keep < 1 ? 1 : keep;
+        const double target = chain_bcast(r.upto, len - 1) * static_cast<double>(c.top_p);
+        len = wave_first(r.upto >= target, len) + 1;
     }
-    double total_weight = -0.0;
-    for (int i = 0; i < len; i++) total_weight += chain_bcast(w, i);
-    if (!(isfinite(total_weight) && total_weight > 0.0)) return fail();
-    if (lane == 0) {
-        d->n_keep = len;
-        d->total = total_weight;
-    }
-    if (lane < len) {
-        d->tokens[lane] = tok;
-        d->weights[lane] = w;
-    }
+    r.total = chain_bcast(r.upto, len - 1);
+    if (isfinite(r.total) && r.total > 0.0) r.len = len;
+    return r;
 }
 
 // the same with private work arrays

@@ -346,6 +346,45 @@ def test_selection_at_chunk_boundaries(ctx, oracle, vocab, top_k):
     assert len(lengths) > 1
 
 
+@pytest.mark.parametrize("kind", ["alike", "by_thread", "short_chunk", "infinite_drafts", "long_lists", "late_nan"])
+@pytest.mark.parametrize("top_k", [1, 17, 64])
+def test_selection_and_decision_off_their_short_paths(ctx, oracle, kind, top_k):
+    """Logits whose selection needs more than a bound per wave (all alike; the best tokens of a 16384-token chunk all with the same few
+    threads), a last chunk of fewer tokens than threads, draft logits that are infinite, proposals and stop ids beyond a wave's 64
+    lanes, a NaN in a later chunk of a target or a draft row: decisions, errors and sampler state equal the oracle's."""
+    vocab, n, T = 2 * 16384 + 700, 4, 0.7
+    rng = np.random.default_rng(top_k)
+    tl = (rng.standard_normal((n, vocab)) * 3.0).astype(np.float32)
+    thread, turn = np.arange(vocab) % 1024, np.arange(vocab) // 1024
+    if kind == "alike":
+        tl[:2] = 0.5
+    elif kind == "by_thread":
+        tl[:] = (-thread + turn * 1e-3)[None, :] * 0.25
+    elif kind == "short_chunk":
+        tl[:, 2 * 16384:] += 8.0
+    dl = (tl[: n - 1] + rng.standard_normal((n - 1, vocab)) * 0.5).astype(np.float32)
+    drafts = [int(np.argmax(dl[r])) for r in range(n - 1)]
+    stops = []
+    if kind == "infinite_drafts":
+        dl[:, ::3] = -np.inf
+        drafts = [int(np.argmax(dl[r])) for r in range(n - 1)]
+    props = [(d, [(d, 0.7), ((d + 1) % vocab, 0.3)]) for d in drafts]
+    if kind == "long_lists":
+        props = [(d, [((d + 1 + j) % vocab, 0.001 * (j + 1)) for j in range(90)] + [(d, 0.4)]) for d in drafts]
+        stops = [(drafts[1] + 1 + j) % vocab for j in range(70)] + [drafts[1]]
+    skw = dict(temperature=T, top_k=top_k, top_p=0.95)
+    for seed in range(6):
+        toks = [3] + drafts
+        for mode in ("deterministic", "sparse", "dense"):
+            t, d = tl, dl
+            if kind == "late_nan":
+                t, d = tl.copy(), dl.copy()
+                (t if seed % 2 else d)[seed // 2, 16384 + 5] = np.nan
+            r = both(ctx, oracle, toks, t, vocab, props if mode == "sparse" else None, 100, stops, draft=d if mode == "dense" else None,
+                     draft_T=T if mode == "dense" else 0.0, seed=seed, **skw)
+            assert_same(oracle, *r)
+
+
 @pytest.mark.parametrize("kind,n_trials", [(dfl.RNG_PHILOX, 10000), (dfl.RNG_XOSHIRO, 2000)])
 def test_seeded_trials_full_vocab_dense(ctx, oracle, kind, n_trials):
     """Stochastic acceptance at its benchmark size: vocabulary 151936, block 16, target logits N(0, 3), draft = target +
