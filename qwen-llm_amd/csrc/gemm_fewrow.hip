@@ -1468,8 +1468,8 @@ __global__ void __launch_bounds__(64 * kSlabWaves)
 //   * x shared by every slot (gate/up, a drafter's per-layer projections of the same columns): a workgroup takes a
 //     contiguous run of (slot, tile) units, sixteen per round, one per wave; the slab is refilled only when K is
 //     longer than four stages (twice per round for K = 2048);
-//   * x per slot (down: every expert has its own SwiGLU rows): a unit is (slot, sixteen tiles) and the slab is
-//     refilled when the slot changes.
+//   * x per slot (down: every expert has its own SwiGLU rows): a unit is (slot, sixteen tiles, or eight where the
+//     list is short) and the slab is refilled when the slot changes.
 // A (row, matrix) result never depends on which other matrices take part: whole K per wave, fixed order.
 constexpr int kExpChunk = 4;  // stages of activations in LDS at a time
 constexpr size_t kExpRingEnd = static_cast<size_t>(kExpChunk) * kTiledStageX +
@@ -1524,15 +1524,133 @@ __device__ __forceinline__ void q4k_experts_compute(const u32x4_t *blk, const ui
     }
 }
 
-template <typename XT, typename YT, bool kRoute>
+// One stage's weights as B operands, ahead of the activations and of the accumulator they meet (the same values as in
+// q4k_experts_compute, which makes them on the way).
+struct Q4KStageW {
+    half4_t mn;
+    half8_t lo[4], hi[4];
+};
+__device__ __forceinline__ void q4k_stage_weights(const u32x4_t *blk, int g, uint32_t sc_sel, Q4KMagic magic, Q4KStageW &b) {
+    const u32x4_t hdr = blk[0], q0 = blk[1 + 2 * g], q1 = blk[2 + 2 * g];
+    const uint32_t upper = 0u - static_cast<uint32_t>(g >> 1);
+    const uint32_t sc_lo = hdr.y & 0x3F3F3F3Fu, sc_hi = (hdr.w & 0x0F0F0F0Fu) | ((hdr.y >> 2) & 0x30303030u);
+    const uint32_t mn_lo = hdr.z & 0x3F3F3F3Fu, mn_hi = ((hdr.w >> 4) & 0x0F0F0F0Fu) | ((hdr.z >> 2) & 0x30303030u);
+    const uint32_t sc_word = (sc_hi & upper) | (sc_lo & ~upper), mn_word = (mn_hi & upper) | (mn_lo & ~upper);
+    const half2_t dm = __builtin_bit_cast(half2_t, hdr.x);
+    const half2_t p_sc = as_half2(__builtin_amdgcn_perm(0x64646464u, sc_word, sc_sel));
+    const half2_t p_mn = as_half2(__builtin_amdgcn_perm(0x64646464u, mn_word, sc_sel));
+    const half2_t neg = dm * splat(static_cast<_Float16>(-1024.0f));
+    const half2_t S = __builtin_elementwise_fma(p_sc, splat(dm[0]), splat(neg[0]));
+    const half2_t M = __builtin_elementwise_fma(p_mn, splat(-dm[1]), splat(-neg[1]));
+    const half2_t unbias = {static_cast<_Float16>(-1024.0f), static_cast<_Float16>(-64.0f)};
+    const half2_t Cs = S * unbias;
+    const half2_t s2l = splat(S[0]), c2l = splat(Cs[0]);
+    const half2_t s2h = splat(S[1]), c2h = splat(Cs[1]);
+    const uint32_t qw[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
+    b.mn = half4_t{M[0], M[1], M[0], M[1]};
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+        b.lo[t] = unpack_scale<false>(qw[2 * t], qw[2 * t + 1], s2l, c2l, magic.lo);
+        b.hi[t] = unpack_scale<true>(qw[2 * t], qw[2 * t + 1], s2h, c2h, magic.hi);
+    }
+}
+// q4k_experts_compute's nine products, in its order
+__device__ __forceinline__ uint32_t q4k_lds_at(const void *p) {
+    return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const void *)(p)));
+}
+struct Q4KStageX {
+    half4_t tw;
+    half8_t af[8];
+};
+__device__ __forceinline__ void q4k_stage_activations(const uint8_t *stage, int lane, Q4KStageX &x) {
+    x.tw = *reinterpret_cast<const half4_t *>(stage + 8 * kTiledFragStride + lane * 8);
+#pragma unroll
+    for (int t = 0; t < 8; t++) x.af[t] = *reinterpret_cast<const half8_t *>(stage + t * kTiledFragStride + lane * 16);
+}
+// (kNext: each activation fragment is replaced by the next stage's once its product has been asked for; the compiler would read
+// those one product ahead of their use, a quarter of the way there)
+template <bool kNext>
+__device__ __forceinline__ void q4k_stage_products(const Q4KStageW &b, Q4KStageX &x, const uint8_t *next, int lane, float4_t &acc) {
+    const _Float16 zero = static_cast<_Float16>(0.0f);
+    const half8_t a_min = {x.tw[0], x.tw[1], x.tw[2], x.tw[3], zero, zero, zero, zero};
+    const half8_t b_min = {b.mn[0], b.mn[1], b.mn[2], b.mn[3], zero, zero, zero, zero};
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a_min, b_min, acc, 0, 0, 0);
+    if constexpr (kNext) {
+        x.tw = *reinterpret_cast<const half4_t *>(next + 8 * kTiledFragStride + lane * 8);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int t = 0; t < 8; t++) {
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(x.af[t], t < 4 ? b.lo[t & 3] : b.hi[t & 3], acc, 0, 0, 0);
+        if constexpr (kNext) {
+            x.af[t] = *reinterpret_cast<const half8_t *>(next + t * kTiledFragStride + lane * 16);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+}
+
+// The slab of a launch of few rows: an octet of values (the c-th of row m) with its share of the sub-block sums, four neighbouring
+// lanes to a sub-block; and zeros for the rows that are not there, a fragment set or the sums of a stage a wave and turn.
+__device__ __forceinline__ void q4k_few_octet(uint8_t *slab, int m, int c, const _Float16 (&h)[8]) {
+    const int j = (c & 31) >> 2, quarter = c & 3;
+    uint8_t *stage = slab + (c >> 5) * kTiledStageX;
+    const half8_t frag = {h[0], h[2], h[1], h[3], h[4], h[6], h[5], h[7]};
+    *reinterpret_cast<half8_t *>(stage + (4 * (j & 1) + quarter) * kTiledFragStride + (16 * (j >> 1) + m) * 16) = frag;
+    const float sum = q4k_quad_sum(q4k_octet_sum_seq(h));
+    if (quarter == 0) {
+        const _Float16 hi = static_cast<_Float16>(sum), lo = static_cast<_Float16>(sum - static_cast<float>(hi));
+        _Float16 *tw = reinterpret_cast<_Float16 *>(stage + 8 * kTiledFragStride) + (m + 16 * (j >> 1)) * 4 + (j & 1);
+        tw[0] = hi;
+        tw[2] = lo;
+    }
+}
+__device__ __forceinline__ void q4k_few_zero(uint8_t *slab, int stages, int n_rows, int lane, int first, int step) {
+    for (int p = first; p < 9 * stages; p += step) {
+        uint8_t *stage = slab + p / 9 * kTiledStageX;
+        const int t = p % 9;
+        if ((lane & 15) >= n_rows) {
+            if (t < 8)
+                *reinterpret_cast<float4_t *>(stage + t * kTiledFragStride + lane * 16) = float4_t{0, 0, 0, 0};
+            else
+                *reinterpret_cast<uint2 *>(stage + 8 * kTiledFragStride + lane * 8) = uint2{0, 0};
+        }
+    }
+}
+// The accumulator of a chain that goes from wave to wave, and whose turn it is.  They are written and read in this order by one
+// wave each, and a wave's LDS accesses stay in order: a reader that sees its turn has the accumulator.  (A part waits for the part
+// before it, and the first for none: every wait ends.)
+__device__ __forceinline__ float4_t q4k_chain_await(uint32_t acc_at, uint32_t turn_at, int turn) {
+    float4_t v;
+    int32_t seen;
+    do {
+        asm volatile("ds_read_b32 %0, %2\n\tds_read_b128 %1, %3\n\ts_waitcnt lgkmcnt(0)" : "=&v"(seen), "=&v"(v) : "v"(turn_at), "v"(acc_at) : "memory");
+    } while (__builtin_amdgcn_readfirstlane(seen) != turn);
+    return v;
+}
+__device__ __forceinline__ void q4k_chain_pass(uint32_t acc_at, uint32_t turn_at, int turn, const float4_t &acc) {
+    *reinterpret_cast<__attribute__((address_space(3))) float4_t *>(acc_at) = acc;
+    asm volatile("" ::: "memory");
+    *reinterpret_cast<volatile __attribute__((address_space(3))) int32_t *>(turn_at) = turn;
+}
+
+// kFew: a routed launch of one or two units a workgroup (the host's bound on the list says so) and K of two chunks: one row's nine
+// matrices of 768 x 2048 are 432 units on 256 workgroups.  The chain of a unit's eight stages, gate and up, is what such a launch
+// would wait for: a stage is 0.4 us of LDS reads, unpacking and nine products for a wave that has its SIMD to itself, and only
+// the products, 0.15, have to follow one another.  So a tile has four waves (wave 8 u + 4 half + part, two stages each), which bring
+// in and unpack their stages at the same time; the accumulator goes through them in the order of the stages (in LDS,
+// with whose turn it is), so the sum is the one wave's, bit for bit.  All of x is in LDS, in the room of the third ring buffers, converted by
+// the waves that have no row to route while the others route (three rows leave enough of them for an octet a lane).  One row of
+// the 35B-A3B-shaped stack: 15.3 us a launch with a tile a wave, 10.3 now.
+template <typename XT, typename YT, bool kRoute, bool kFew = false>
 __global__ void __launch_bounds__(64 * kSlabWaves)
     gemm_q4k_experts_kernel(const XT *__restrict__ x, const float *__restrict__ logits, int32_t *ids, int32_t *n_slots_at,
                             const uint8_t *__restrict__ w, int nb, uint32_t rows_route, int n_out, int max_slots, YT *__restrict__ y, int n_wg,
-                            int upm, Q4KDiv by_upm, int early_ids, Q4KBatch bt) {
+                            int upm, Q4KDiv by_upm, int early_group, Q4KBatch bt) {
     // (The arguments in the order of their use: the first fourteen words come preloaded with the wave, the others are asked for
-    // under the first loads.  rows_route = n_rows | picks per row << 8 | experts << 16 | shared expert << 31.)
+    // under the first loads.  rows_route = n_rows | picks per row << 8 | experts << 16 | shared expert << 31; early_group = tiles of a
+    // unit with x per slot | read the list ahead << 8.)
     constexpr int kW = kSlabWaves;
-    const int n_rows = rows_route & 255;
+    const int n_rows = rows_route & 255, group = early_group & 255;
     constexpr int kItems = kExpChunk * 8 / kW;  // activation items (eight values of one row) per thread and refill: 2
     constexpr int kXInstr = kItems * Q4KX8<XT>::kLoads;
     static_assert(3 * (kSlabRing - 1) + kXInstr <= 10 && 3 * kSlabRing <= 10, "q4k_wait_vm_few");
@@ -1565,6 +1683,8 @@ __global__ void __launch_bounds__(64 * kSlabWaves)
             q4k_load_x8(xb + static_cast<size_t>(sb) * (DFL_QK_K * sizeof(XT)), x_off[r], raw_a[r], raw_b[r]);
         }
     };
+    // kFew: how many parts of a chain are done, behind the accumulators that go through it
+    int32_t *chain_turn = reinterpret_cast<int32_t *>(reinterpret_cast<uint8_t *>(lds) + kExpRingEnd + 4 * 64 * sizeof(float4_t));
     int32_t *ids_lds = reinterpret_cast<int32_t *>(reinterpret_cast<uint8_t *>(lds) + kExpXchgEnd + 16 * 4 * sizeof(unsigned long long));
     int slot_base = -64;  // no window of the list yet: the first use (before any weight load is issued) reads it
     int32_t ids_window = 0;
@@ -1590,7 +1710,7 @@ __global__ void __launch_bounds__(64 * kSlabWaves)
         __builtin_amdgcn_s_waitcnt(q4k_vmcnt(0));
 #pragma unroll
         for (int j = 0; j < 4; j++) asm volatile("" : "+v"(lgv[j]));
-        load_x(0, 0);
+        if constexpr (!kFew) load_x(0, 0);
         dfl_have(y, n_wg, upm, by_upm.mul, by_upm.shift, bt.w2, bt.extra_w, bt.extra_w2, bt.w_stride, bt.y_stride, bt.by_wg.mul, bt.by_wg.shift,
                  bt.pair, bt.route_sel_e, bt.route_sel_w, bt.route_slot_of);
         dfl_route::RowPicks pk;
@@ -1598,6 +1718,20 @@ __global__ void __launch_bounds__(64 * kSlabWaves)
         pk.my_w = 0.0f;
         pk.m[0] = pk.m[1] = pk.m[2] = pk.m[3] = 0;
         if (wave < n_rows) pk = dfl_route::route_row_from(lgv, E, used, lane);
+        if constexpr (kFew) {
+            if (wave >= n_rows) {  // the waves without a row: an octet of x a lane, and zeros for the rows that are not there
+                const int item = (wave - n_rows) * 64 + lane, m = item >> 8, c = item & 255;
+                const float4_t *src = reinterpret_cast<const float4_t *>(x + static_cast<size_t>(min(m, n_rows - 1)) * n_in + 8 * c);
+                const float4_t xa = src[0], xb = src[1];
+                if (wave == n_rows && lane < 4) chain_turn[lane] = 0;
+                q4k_few_zero(slab, 2 * kExpChunk, n_rows, lane, wave - n_rows, kW - n_rows);
+                if (m < n_rows) {
+                    _Float16 h[8];
+                    q4k_x8_to_half(xa, xb, h);
+                    q4k_few_octet(slab, m, c, h);
+                }
+            }
+        }
         if (lane < 4) row_mask[wave * 4 + lane] = dfl_route::pick4(pk.m, lane);
         __builtin_amdgcn_s_waitcnt(kWaitLds);
         __builtin_amdgcn_s_barrier();
@@ -1624,7 +1758,7 @@ __global__ void __launch_bounds__(64 * kSlabWaves)
         __builtin_amdgcn_s_waitcnt(kWaitLds);
         __builtin_amdgcn_s_barrier();
     } else {
-        if (early_ids) {  // the first window of the list travels with the slot count: one trip to memory instead of two
+        if (early_group >> 8) {  // the first window of the list travels with the slot count: one trip to memory instead of two
             ids_window = ids[min(lane, max_slots - 1)];
             slot_base = 0;
         }
@@ -1639,7 +1773,7 @@ __global__ void __launch_bounds__(64 * kSlabWaves)
     const int tiles = (n_out + 15) >> 4;
     const int halves = bt.pair ? 2 : 1;
     const int n_chunks = (nb + kExpChunk - 1) / kExpChunk;
-    // units: (slot, tile) with shared x, (slot, group of sixteen tiles) with x per slot; upm = units per matrix
+    // units: (slot, tile) with shared x, (slot, group of tiles, one a wave) with x per slot; upm = units per matrix
     const uint32_t units = static_cast<uint32_t>(n_slots) * static_cast<uint32_t>(upm);
     const int wg = q4k_range_index(blockIdx.x, n_wg);
     const int u0 = static_cast<int>(q4k_div(units * wg, bt.by_wg)), u1 = static_cast<int>(q4k_div(units * (wg + 1), bt.by_wg));
@@ -1673,10 +1807,10 @@ __global__ void __launch_bounds__(64 * kSlabWaves)
         if (per_slot_x) {
             const int g = u0 + r;
             slot = static_cast<int>(q4k_div(g, by_upm));
-            tile = (g - slot * upm) * kW + wave;
-            return tile < tiles;
+            tile = (g - slot * upm) * group + wave;
+            return wave < group && tile < tiles;
         }
-        const int u = hsplit ? u0 + (wave & 7) : u0 + r * kW + wave;
+        const int u = kFew ? u0 + (wave >> 3) : hsplit ? u0 + (wave & 7) : u0 + r * kW + wave;
         slot = static_cast<int>(q4k_div(min(u, u1 - 1), by_upm));
         tile = u - slot * upm;
         return u < u1;
@@ -1761,16 +1895,18 @@ __global__ void __launch_bounds__(64 * kSlabWaves)
 
     // ---- prologue: the first activations (oldest loads), two weight stages, then the slab ----
     int slab_slot = xslot_of(0), slab_chunk = 0;
-    if (!kRoute) load_x(slab_slot, 0);
-    it_seek();
-    for (int t = 0; t < 2; t++)
-        if (it_valid) issue();
-    DFL_TRE(2);
-    q4k_wait_vm_few(3 * w_issued);  // the activations are older than every weight load
-    convert(0);
-    __builtin_amdgcn_s_waitcnt(kWaitLds);
-    __builtin_amdgcn_s_barrier();
-    DFL_TRE(3);
+    if (!kFew) {
+        if (!kRoute) load_x(slab_slot, 0);
+        it_seek();
+        for (int t = 0; t < 2; t++)
+            if (it_valid) issue();
+        DFL_TRE(2);
+        q4k_wait_vm_few(3 * w_issued);  // the activations are older than every weight load
+        convert(0);
+        __builtin_amdgcn_s_waitcnt(kWaitLds);
+        __builtin_amdgcn_s_barrier();
+        DFL_TRE(3);
+    }
     bool x_pending = false;  // activations of the next refill are on their way (issued when w_issued was x_pos)
     int x_pos = 0;
 
@@ -1796,7 +1932,52 @@ __global__ void __launch_bounds__(64 * kSlabWaves)
         return q4k_any_nan(res);
     };
     bool again = false;
-    for (int r = 0; r < n_rounds; r++) {
+    if constexpr (kFew) {
+        int slot = 0, tile = 0;
+        const bool active = unit_of(0, slot, tile);
+        const int half = (wave >> 2) & 1, part = wave & 3;
+        static_assert(2 * kExpChunk * kTiledStageX + kW * 2 * kSlabWavePieces * 16 <= kExpRingEnd, "the slab in the rings' place");
+        half8_t *buf = reinterpret_cast<half8_t *>(slab + 2 * kExpChunk * kTiledStageX) + wave * (2 * kSlabWavePieces);
+        if (active) {
+            const uint8_t *src = tile_base(slot, tile, half) + static_cast<size_t>(2 * part) * kTiledStageBytes + static_cast<size_t>(lane) * 16;
+#pragma unroll
+            for (int t = 0; t < 2; t++, src += kTiledStageBytes, buf += kSlabWavePieces) {
+                __builtin_amdgcn_global_load_lds((gptr_t)(src), (lptr_t)(buf), 16, 0, DFL_W_AUX);
+                __builtin_amdgcn_global_load_lds((gptr_t)(src + 1024), (lptr_t)(buf + 64), 16, 0, DFL_W_AUX);
+                if (lane < 16) __builtin_amdgcn_global_load_lds((gptr_t)(src + 2048), (lptr_t)(buf + 128), 16, 0, DFL_W_AUX);
+            }
+            buf -= 2 * kSlabWavePieces;
+        }
+        DFL_TRE(2);
+        __builtin_amdgcn_s_waitcnt(q4k_vmcnt(0));
+        DFL_TRE(4);
+        if (active) {
+            float4_t acc = {0, 0, 0, 0};
+            Q4KStageW w0, w1;
+            Q4KStageX xs;
+            const u32x4_t *blk = reinterpret_cast<const u32x4_t *>(buf) + n * 9;
+            q4k_stage_weights(blk, g, sc_sel, magic, w0);
+            q4k_stage_weights(blk + kSlabWavePieces, g, sc_sel, magic, w1);
+            q4k_stage_activations(slab + 2 * part * kTiledStageX, lane, xs);
+            // (unpacked here and not between the products, as the compiler would have it)
+#pragma unroll
+            for (int t = 0; t < 4; t++) asm volatile("" : "+v"(w0.lo[t]), "+v"(w0.hi[t]), "+v"(w1.lo[t]), "+v"(w1.hi[t]));
+            asm volatile("" : "+v"(w0.mn), "+v"(w1.mn));
+            const int chain = wave >> 2;
+            const uint32_t at = q4k_lds_at(reinterpret_cast<uint8_t *>(lds) + kExpRingEnd) + (chain * 64 + lane) * 16;
+            const uint32_t turn_at = q4k_lds_at(chain_turn + chain);
+            if (part > 0) acc = q4k_chain_await(at, turn_at, part);
+            q4k_stage_products<true>(w0, xs, slab + (2 * part + 1) * kTiledStageX, lane, acc);
+            q4k_stage_products<false>(w1, xs, nullptr, lane, acc);
+            if (half == 0 && part == 3) {
+                DFL_TRE(5);
+                again = put(slot, tile, acc, q4k_chain_await(at + 64 * 16, turn_at + 4, 4));
+            } else {
+                q4k_chain_pass(at, turn_at, part + 1, acc);
+            }
+        }
+    }
+    for (int r = 0; !kFew && r < n_rounds; r++) {
         int slot = 0, tile = 0;
         const bool active = unit_of(r, slot, tile);
         const int xslot = xslot_of(r);
@@ -1879,6 +2060,83 @@ __global__ void __launch_bounds__(64 * kSlabWaves)
     }
     DFL_TRE(6);
     DFL_TRE_FLUSH;
+}
+
+// The few rows' product of a list of matrices with K of at most four stages and rows of its own per slot (down: one row's nine
+// matrices of 2048 x 768), as kFew above: a stage a wave, the accumulator handed from stage to stage.  A unit is (slot, 16 / stages
+// tiles) and a workgroup has one, so its rows and its place in the list are known at once, and the weights are asked for one trip
+// to memory after the start.  A CU takes in about 30 KB per microsecond: units of sixteen whole tiles were 110 KB in 72 workgroups
+// (9.3 us), of eight 55 KB in 144 (7.1); 35 KB in 234, with a stage and not a tile a wave, 4.8.
+__global__ void __launch_bounds__(1024)
+    gemm_q4k_few_slots_kernel(const _Float16 *__restrict__ x, const int32_t *__restrict__ ids, const int32_t *__restrict__ n_slots_at,
+                              const uint8_t *__restrict__ w, const uint8_t *__restrict__ extra_w, uint32_t stages_rows, int upm, Q4KDiv by_upm,
+                              size_t w_stride, size_t x_stride, size_t y_stride, float *__restrict__ y, int n_out) {
+    extern __shared__ half8_t lds[];
+    const int nb = stages_rows & 255, n_rows = stages_rows >> 8 & 255, n_in = nb * DFL_QK_K;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    uint8_t *slab = reinterpret_cast<uint8_t *>(lds);                                      // [nb][kTiledStageX]
+    uint8_t *buf = slab + nb * kTiledStageX + wave * kTiledTileBytes;                      // [wave]: its stage of its tile
+    uint8_t *accs = slab + nb * kTiledStageX + kSlabWaves * kTiledTileBytes;               // [tile][64] accumulators, [tile] turns
+    int32_t *turns = reinterpret_cast<int32_t *>(accs + kSlabWaves * 64 * sizeof(float4_t));
+    auto by_nb = [&](int v) { return v * static_cast<int>(stages_rows >> 16) >> 5; };  // v / nb, v < 32
+    const int slot = static_cast<int>(q4k_div(blockIdx.x, by_upm)), in_unit = by_nb(wave), part = wave - in_unit * nb;
+    const int tpu = by_nb(kSlabWaves), tile = (blockIdx.x - slot * upm) * tpu + in_unit;
+    // the rows' octets, one a thread (n_rows * nb * 32 <= 1024, checked on the host)
+    const int m = by_nb(tid >> 5), c = tid - m * nb * 32;
+    const half8_t xv = *reinterpret_cast<const half8_t *>(x + slot * x_stride + static_cast<size_t>(min(m, n_rows - 1)) * n_in + 8 * c);
+    const int32_t id = ids[slot], n_slots = *n_slots_at;
+    dfl_have(w_stride, y_stride, y, n_out);
+    // (what goes to LDS by itself goes there ahead of the weights, which the compiler would wait for)
+    if (tid < kSlabWaves) turns[tid] = 0;
+    q4k_few_zero(slab, nb, n_rows, lane, wave, kSlabWaves);
+    dfl_have(id, n_slots);
+    if (slot >= n_slots) return;  // (the whole workgroup)
+    if (m < n_rows) {
+        _Float16 h[8];
+        q4k_x8_to_half(xv, xv, h);
+        q4k_few_octet(slab, m, c, h);
+    }
+    const bool active = in_unit < tpu && tile * 16 < n_out;
+    const uint8_t *tile_w = (id < 0 ? extra_w : w + static_cast<size_t>(id) * w_stride) + static_cast<size_t>(tile >> 4) * nb * kTiledStageBytes +
+                            static_cast<size_t>(tile & 15) * kTiledTileBytes;
+    if (active) {
+        const uint8_t *src = tile_w + static_cast<size_t>(part) * kTiledStageBytes + static_cast<size_t>(lane) * 16;
+        __builtin_amdgcn_global_load_lds((gptr_t)(src), (lptr_t)(buf), 16, 0, DFL_W_AUX);
+        __builtin_amdgcn_global_load_lds((gptr_t)(src + 1024), (lptr_t)(buf + 1024), 16, 0, DFL_W_AUX);
+        if (lane < 16) __builtin_amdgcn_global_load_lds((gptr_t)(src + 2048), (lptr_t)(buf + 2048), 16, 0, DFL_W_AUX);
+    }
+    __builtin_amdgcn_s_waitcnt(kWaitLds);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_s_waitcnt(q4k_vmcnt(0));
+    if (!active) return;
+    const int n = lane & 15, g = lane >> 4;
+    const uint32_t sc_sel = (lane & 16) ? 0x04030402u : 0x04010400u;
+    const Q4KMagic magic = q4k_magic();
+    float4_t acc = {0, 0, 0, 0};
+    Q4KStageW sw;
+    Q4KStageX sx;
+    q4k_stage_weights(reinterpret_cast<const u32x4_t *>(buf) + n * 9, g, sc_sel, magic, sw);
+    q4k_stage_activations(slab + part * kTiledStageX, lane, sx);
+#pragma unroll
+    for (int t = 0; t < 4; t++) asm volatile("" : "+v"(sw.lo[t]), "+v"(sw.hi[t]));
+    asm volatile("" : "+v"(sw.mn));
+    const uint32_t at = q4k_lds_at(accs) + (in_unit * 64 + lane) * 16, turn_at = q4k_lds_at(turns + in_unit);
+    if (part > 0) acc = q4k_chain_await(at, turn_at, part);
+    q4k_stage_products<false>(sw, sx, nullptr, lane, acc);
+    if (part < nb - 1) {
+        q4k_chain_pass(at, turn_at, part + 1, acc);
+        return;
+    }
+    if (__builtin_expect(q4k_any_nan(acc), 0))
+        acc = q4k_again<_Float16, true>(tile_w + n * DFL_Q4_K_BYTES, kTiledStageBytes, x + slot * x_stride + static_cast<size_t>(min(n, n_rows - 1)) * n_in,
+                                        nb, g, sc_sel, magic);
+    float *yo = y + slot * y_stride + tile * 16 + n;  // (n_out is a multiple of 16)
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+        if (4 * g + i < n_rows) yo[static_cast<size_t>(4 * g + i) * n_out] = acc[i];
+}
+inline size_t q4k_few_slots_lds(int nb) {
+    return static_cast<size_t>(nb) * kTiledStageX + kSlabWaves * (kTiledTileBytes + 64 * sizeof(float4_t) + sizeof(int32_t));
 }
 
 // ----------------------------------------------------------------------------
@@ -2742,34 +3000,57 @@ int32_t launch_q4k(dflash_ctx *ctx, const void *w, const void *x, int32_t x_type
         if (reinterpret_cast<uintptr_t>(x) % 16)
             return dfl_fail(ctx, DFLASH_ERR_ALIGNMENT, "gemm_q4k_batched: activations must be 16-byte aligned");
         const bool per_slot_x = batch->x_stride != 0;
-        const int upm = per_slot_x ? (tiles + 15) / 16 : tiles;  // units per matrix
         int n_wg = env_int("DFLASH_MOE_WGS", ctx->batch_wgs > 0 ? ctx->batch_wgs : ctx->n_cu);
         if (n_wg < 1) n_wg = 1;
+        const uint8_t *wb = static_cast<const uint8_t *>(w);
+        const int no = static_cast<int>(n_out);
+        // Rows of their own per slot, K of at most four stages and so few matrices that every unit of 16 / stages tiles has a workgroup of
+        // its own: a stage a wave (one row of the 35B-A3B-shaped stack 4.8 us a launch, against 7.1 with eight whole tiles a workgroup).
+        if (per_slot_x && x_type == DFLASH_TYPE_F16 && !batch->y_f16 && !batch->pair && nb <= 4 && n_out % 16 == 0 && n_rows * nb * 32 <= 1024) {
+            const int tpu = kSlabWaves / nb, upm = (tiles + tpu - 1) / tpu;
+            if (static_cast<int64_t>(max_slots) * upm <= n_wg) {
+                if (const int32_t rc_ = dfl_raise_lds_limit(ctx, reinterpret_cast<const void *>(gemm_q4k_few_slots_kernel), q4k_few_slots_lds(nb))) return rc_;
+                dfl_timed timer(ctx, st, DFL_T_GEMM);
+                gemm_q4k_few_slots_kernel<<<max_slots * upm, 64 * kSlabWaves, q4k_few_slots_lds(nb), st>>>(
+                    static_cast<const _Float16 *>(x), batch->ids, batch->n_slots, wb, batch->extra_w,
+                    static_cast<uint32_t>(nb) | static_cast<uint32_t>(n_rows) << 8 | ((32u + nb - 1) / nb) << 16, upm, q4k_make_div(static_cast<uint32_t>(upm)), batch->w_stride,
+                    batch->x_stride, batch->y_stride, y, no);
+                DFL_HIP_CHECK(ctx, hipGetLastError());
+                return DFLASH_OK;
+            }
+        }
+        // Sixteen tiles a unit, one a wave, or eight where the longest list still gives no workgroup a second unit: a CU takes in
+        // about 30 KB per microsecond, and a short list in large units leaves most of them without any (one row's nine matrices of
+        // 2048 x 768: 72 units of 110 KB 9.3 us, 144 of 55 KB 7.1).
+        int group = 16;
+        if (static_cast<int64_t>(max_slots) * ((tiles + 7) / 8) <= n_wg) group = 8;
+        const int upm = per_slot_x ? (tiles + group - 1) / group : tiles;  // units per matrix
         if (static_cast<int64_t>(max_slots) * upm * (n_wg + 1) >= (int64_t(1) << 31) || nb > 4096)
             return dfl_fail(ctx, DFLASH_ERR_BAD_SHAPE, "gemm_fewrow: batch too large for 32-bit work indices");
         Q4KBatch bt = *batch;
         bt.by_wg = q4k_make_div(static_cast<uint32_t>(n_wg));
         const Q4KDiv by_upm = q4k_make_div(static_cast<uint32_t>(upm));
         // the first 64 list entries are loaded together with the slot count (0.5 us per down launch at light load)
-        const int early_ids = env_int("DFLASH_EXP_EARLY_IDS", 1);
-        const uint8_t *wb = static_cast<const uint8_t *>(w);
-        const int no = static_cast<int>(n_out);
-#define DFL_LAUNCH_EXPERTS(XT, YT, ROUTE)                                                                                   \
+        const int early_group = group | (env_int("DFLASH_EXP_EARLY_IDS", 1) ? 256 : 0);
+#define DFL_LAUNCH_EXPERTS(XT, YT, ...)                                                                                     \
     do {                                                                                                                    \
-        if (const int32_t rc_ = dfl_raise_lds_limit(ctx, reinterpret_cast<const void *>(gemm_q4k_experts_kernel<XT, YT, ROUTE>), kExpLdsBytes)) \
+        if (const int32_t rc_ = dfl_raise_lds_limit(ctx, reinterpret_cast<const void *>(gemm_q4k_experts_kernel<XT, YT, __VA_ARGS__>), kExpLdsBytes)) \
             return rc_;                                                                                                     \
         dfl_timed timer(ctx, st, DFL_T_GEMM);                                                                               \
         const uint32_t rows_route = static_cast<uint32_t>(n_rows) | static_cast<uint32_t>(bt.route_used) << 8 |                                   \
                                     static_cast<uint32_t>(bt.route_experts) << 16 | (bt.route_shared ? 1u << 31 : 0u);                             \
-        gemm_q4k_experts_kernel<XT, YT, ROUTE><<<n_wg, 64 * kSlabWaves, kExpLdsBytes, st>>>(                                                       \
+        gemm_q4k_experts_kernel<XT, YT, __VA_ARGS__><<<n_wg, 64 * kSlabWaves, kExpLdsBytes, st>>>(                                                 \
             static_cast<const XT *>(x), bt.route_logits, const_cast<int32_t *>(bt.ids), const_cast<int32_t *>(bt.n_slots), wb, nb, rows_route, no, \
-            max_slots, reinterpret_cast<YT *>(y), n_wg, upm, by_upm, early_ids, bt);                                                              \
+            max_slots, reinterpret_cast<YT *>(y), n_wg, upm, by_upm, early_group, bt);                                                              \
     } while (0)
         if (bt.route_logits) {
             if (x_type != DFLASH_TYPE_F32 || per_slot_x || !bt.y_f16 || bt.route_experts > 256 || bt.route_experts < 1 || bt.route_used < 1 ||
                 bt.route_used > 64 || bt.route_used > bt.route_experts || max_slots + 0 > kExpRouteIds - 1)
                 return dfl_fail(ctx, DFLASH_ERR_UNSUPPORTED, "gemm_q4k_batched: routing inside the launch needs f32 shared activations, f16 output and at most 256 experts");
-            DFL_LAUNCH_EXPERTS(float, _Float16, true);
+            if (bt.pair && nb == 2 * kExpChunk && n_rows <= 3 && static_cast<int64_t>(max_slots) * upm <= 2ll * n_wg)
+                DFL_LAUNCH_EXPERTS(float, _Float16, true, true);
+            else
+                DFL_LAUNCH_EXPERTS(float, _Float16, true, false);
         } else if (x_type == DFLASH_TYPE_F32 && !bt.y_f16) {
             DFL_LAUNCH_EXPERTS(float, float, false);
         } else if (x_type == DFLASH_TYPE_F32) {

@@ -9,6 +9,8 @@
 
 #include <cstdint>
 
+#include "common.h"
+
 namespace dfl_route {
 
 // Maximum of a float over the wave, in every lane: data-parallel-primitive moves within rows of 16 lanes (shift right
@@ -143,19 +145,29 @@ __device__ __forceinline__ unsigned long long pick4(const unsigned long long v[4
     return i == 0 ? v[0] : i == 1 ? v[1] : i == 2 ? v[2] : v[3];
 }
 
-// The union of the sixteen rows' masks (row_mask[row * 4 + j] in LDS, complete): lane l reads word l, four xor-shuffle
-// steps OR the rows together, and words 0..3 are read back out of lanes 0..3.  Called by a whole wave.
+// v | v of the lanes 4, 8, 16 and 32 away and of all combinations of those: lanes alike in their last two bits have the same then
+__device__ __forceinline__ unsigned or_of_rows(unsigned v) {
+    float a = __uint_as_float(v), b = a;  // (moved, never computed with)
+    dfl_swap32(a, b);
+    v = __float_as_uint(a) | __float_as_uint(b);
+    a = b = __uint_as_float(v);
+    dfl_swap16(a, b);
+    v = __float_as_uint(a) | __float_as_uint(b);
+    v |= static_cast<unsigned>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x128, 0xF, 0xF, true));  // row_ror:8
+    v |= static_cast<unsigned>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x124, 0xF, 0xF, true));  // row_ror:4
+    return v;
+}
+
+// The union of the sixteen rows' masks (row_mask[row * 4 + j] in LDS, complete): lane l reads word l, the rows are ORed together
+// without a trip through LDS, and words 0..3 are read back out of lanes 0..3.  Called by a whole wave.
 __device__ __forceinline__ void union_of_rows(const unsigned long long *row_mask, int lane, unsigned long long un[4]) {
-    unsigned long long v = row_mask[lane];
-    for (int off = 4; off < 64; off <<= 1) {
-        const unsigned lo = __shfl_xor(static_cast<unsigned>(v), off, 64), hi = __shfl_xor(static_cast<unsigned>(v >> 32), off, 64);
-        v |= (static_cast<unsigned long long>(hi) << 32) | lo;
-    }
+    const unsigned long long mine = row_mask[lane];
+    const unsigned v_lo = or_of_rows(static_cast<unsigned>(mine)), v_hi = or_of_rows(static_cast<unsigned>(mine >> 32));
 #pragma unroll
     for (int j = 0; j < 4; j++) {
         // (readlane returns int: through unsigned, or a low word with bit 31 set would smear over the high word)
-        const unsigned lo = static_cast<unsigned>(__builtin_amdgcn_readlane(static_cast<unsigned>(v), j));
-        const unsigned hi = static_cast<unsigned>(__builtin_amdgcn_readlane(static_cast<unsigned>(v >> 32), j));
+        const unsigned lo = static_cast<unsigned>(__builtin_amdgcn_readlane(v_lo, j));
+        const unsigned hi = static_cast<unsigned>(__builtin_amdgcn_readlane(v_hi, j));
         un[j] = (static_cast<unsigned long long>(hi) << 32) | lo;
     }
 }

@@ -465,6 +465,31 @@ def test_moe_verify_matches_oracle(ctx, oracle, name, wtype):
     sess.close()
 
 
+@pytest.mark.parametrize("hidden,n_expert,used,ffn,shared,rows", [
+    (2048, 32, 8, 768, 768, 1),   # the end-to-end shape's widths: 16 tiles a matrix and three stages of K, a wave of each five tiles idle
+    (2048, 16, 2, 256, 256, 3),   # three rows: every octet of x has a lane of its own; K of one stage
+    (2048, 16, 4, 512, 512, 2),
+    (2048, 16, 2, 1024, 1024, 2),  # K of four stages
+    (2048, 16, 1, 1280, 1280, 1),  # K of five: units of whole tiles, eight to a workgroup
+    (2048, 16, 2, 768, 512, 4),   # four rows: gate and up in the kernel of the large lists, down not
+    (512, 16, 2, 256, 512, 1),    # K of two stages in front of gate and up
+])
+def test_short_expert_lists_give_the_bits_of_long_ones(ctx, hidden, n_expert, used, ffn, shared, rows):
+    """One to four rows' expert products hand a tile's accumulator from wave to wave, stage by stage; a block of sixteen rows keeps it in
+    one wave.  The sums are the same, in the same order, so the first rows of a block are the bits they are by themselves."""
+    cfg = dfl.ModelConfig(n_layers=1, hidden=hidden, n_q=4, n_kv=2, head_dim=64, ffn=0, vocab=4096, n_expert=n_expert, n_expert_used=used,
+                          ffn_expert=ffn, ffn_shared=shared)
+    model = dfl.TargetModel(ctx, cfg, dfl.synth_target_weights(cfg, seed=ffn + rows))
+    toks = np.random.default_rng(rows).integers(0, cfg.vocab, 16).tolist()
+    got = []
+    for n in (rows, 16):
+        sess = dfl.Session(ctx, model, 32, [0])
+        got.append(sess.encode_packed_verify_layer_major(toks[:n], 0).hidden_capture.cpu().numpy()[:rows])
+        sess.close()
+    assert np.all(np.isfinite(got[0])) and np.ptp(got[0]) > 0
+    assert np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32))
+
+
 def test_draft_block_general_positions(ctx, oracle, target):
     """Context columns at arbitrary positions and a block that does not start right behind them: the
     general f32 drafter attention (the MFMA path needs positions 0, 1, 2, ... and start == ctx_len)."""
