@@ -2666,6 +2666,84 @@ __global__ void __launch_bounds__(64 * kMaxSplit)
     }
 }
 
+// The same product for the many rows of a prefill group: a workgroup has sixteen rows and 64 weight rows instead of 16, so the
+// rows are read and converted by a quarter of the workgroups, straight into the MFMA operands (every wave has four steps of K for
+// itself, a line of each row a step), while the weights come through LDS, a row in whole lines.  Waves and steps are cut as above with
+// sixteen waves, so are the bits.  (2048 rows x 2048 to 128 experts: 34 us in 1024 workgroups of the kernel above, four rounds of
+// 163 KB each, 15.4 in 256 of this one.)
+constexpr int kQ8RowsOut = 64;
+constexpr size_t kQ8RowsLds = kQ8RowsOut * static_cast<size_t>(kQ8WRowStride);
+static_assert(kMaxSplit * 4 * 256 * sizeof(float) <= kQ8RowsLds, "the waves' sums in the weights' place");
+
+__global__ void __launch_bounds__(64 * kMaxSplit)
+    gemm_q8_0_rows_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x, float *__restrict__ y, int n_out, int n_steps, int n_rows_total) {
+    extern __shared__ __attribute__((aligned(16))) float red[];  // the weight rows, then [wave][tile][256] sums
+    uint8_t *ws = reinterpret_cast<uint8_t *>(red);
+    const int n_rows = min(16, n_rows_total - 16 * static_cast<int>(blockIdx.y)), n0 = blockIdx.x * kQ8RowsOut;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), n = lane & 15, g = lane >> 4;
+    const size_t n_in = static_cast<size_t>(n_steps) * 32;
+    x += static_cast<size_t>(blockIdx.y) * 16 * n_in;
+    y += static_cast<size_t>(blockIdx.y) * 16 * n_out;
+    const int s0 = n_steps * wave / kMaxSplit, s1 = n_steps * (wave + 1) / kMaxSplit;
+    constexpr int kSteps = kQ8ChunkSteps / kMaxSplit;
+    // four weight rows a wave, in whole lines (past n_out the last one again)
+    const int row_bytes = n_steps * DFL_Q8_0_BYTES, pieces = row_bytes / 16;
+    constexpr int kPieces = (kQ8ChunkSteps * DFL_Q8_0_BYTES / 16 + 63) / 64;
+    u32x4_t wr[4][kPieces];
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        const uint8_t *src = w + static_cast<size_t>(min(n0 + 4 * wave + r, n_out - 1)) * row_bytes;
+#pragma unroll
+        for (int c = 0; c < kPieces; c++) wr[r][c] = *reinterpret_cast<const u32x4_t *>(src + 16 * min(lane + 64 * c, pieces - 1));
+    }
+    // this wave's steps of its lanes' row (past n_rows the last one again)
+    RawX8<float> xr[kSteps];
+    {
+        const float *row = x + static_cast<size_t>(min(n, n_rows - 1)) * n_in + 8 * g;
+#pragma unroll
+        for (int i = 0; i < kSteps; i++) xr[i] = load_rawx8(row + static_cast<size_t>(min(s0 + i, n_steps - 1)) * 32);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+#pragma unroll
+        for (int c = 0; c < kPieces; c++)
+            if (lane + 64 * c < pieces) *reinterpret_cast<u32x4_t *>(ws + (4 * wave + r) * kQ8WRowStride + 16 * (lane + 64 * c)) = wr[r][c];
+    half8_t xf[kSteps];
+#pragma unroll
+    for (int i = 0; i < kSteps; i++) xf[i] = convert_rawx8(xr[i]);
+    __syncthreads();
+    float4_t acc[4] = {{0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}};
+#pragma unroll
+    for (int i = 0; i < kSteps; i++) {
+        if (s0 + i >= s1) break;
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            // (a block starts at a multiple of two: its quants by the words they lie in, a third one where they start inside one)
+            const uint8_t *blk = ws + (16 * t + n) * kQ8WRowStride + (s0 + i) * DFL_Q8_0_BYTES;
+            const uint32_t in_word = 2u & ~(static_cast<uint32_t>(s0 + i) << 1);
+            const uint32_t *words = reinterpret_cast<const uint32_t *>(blk + 2 + 8 * g - in_word);
+            const uint32_t q0 = words[0], q1 = words[1], q2 = words[2];
+            Raw8<DFLASH_TYPE_Q8_0> rw;
+            rw.d = static_cast<float>(__builtin_bit_cast(_Float16, *reinterpret_cast<const uint16_t *>(blk)));
+            rw.q = static_cast<uint64_t>(__builtin_amdgcn_alignbyte(q1, q0, in_word)) |
+                   static_cast<uint64_t>(__builtin_amdgcn_alignbyte(q2, q1, in_word)) << 32;
+            acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[i], convert_raw8<DFLASH_TYPE_Q8_0>(rw), acc[t], 0, 0, 0);
+        }
+    }
+    __syncthreads();  // the weights have been read
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) red[(wave * 4 + t) * 256 + (4 * g + i) * 16 + n] = acc[t][i];
+    __syncthreads();
+    // output (row m, weight row o) by thread 64 m + o: a row's 64 are one store
+    const int m = tid >> 6, o = tid & 63;
+    float sum = 0.0f;
+#pragma unroll
+    for (int wv = 0; wv < kMaxSplit; wv++) sum += red[(wv * 4 + (o >> 4)) * 256 + m * 16 + (o & 15)];
+    if (m < n_rows && n0 + o < n_out) y[static_cast<size_t>(m) * n_out + n0 + o] = sum;
+}
+
 // The router of a mixture-of-experts layer together with the residual add, the RMSNorm and the shared-expert gate
 // that precede it (rms_norm_kernel of the model followed by the kernel above, as one launch).  One workgroup per
 // (16 experts, block row): it normalises its row of x + add exactly as the norm kernel does (256 threads, the row in
@@ -3306,8 +3384,18 @@ int32_t dfl_router_rows(dflash_ctx *ctx, const void *router_w, const float *cur,
         reinterpret_cast<uintptr_t>(cur) % 16)
         return dfl_fail(ctx, DFLASH_ERR_UNSUPPORTED, "router_rows: hidden %lld / %d experts / %d rows", static_cast<long long>(hidden), n_expert,
                         n_rows);
+    const int n_steps = static_cast<int>(hidden / DFL_QK8_0), blocks = (n_rows + 15) / 16;
+    // (from where the smaller workgroups are more than one round of the chip; us, them : these, 2048 to 128 experts: 512 rows 9.6 : 11, 544 14.8 : 11.3,
+    // 800 16.2 : 12.0, 1088 23.2 : 12.7, 2048 34 : 15.4)
+    if (static_cast<int64_t>(blocks) * ((n_expert + 15) / 16) > ctx->n_cu) {
+        if (const int32_t rc_ = dfl_raise_lds_limit(ctx, reinterpret_cast<const void *>(gemm_q8_0_rows_kernel), kQ8RowsLds)) return rc_;
+        dfl_timed timer(ctx, st, DFL_T_GEMM);
+        gemm_q8_0_rows_kernel<<<dim3((n_expert + kQ8RowsOut - 1) / kQ8RowsOut, blocks), 64 * kMaxSplit, kQ8RowsLds, st>>>(
+            static_cast<const uint8_t *>(router_w), cur, logits, n_expert, n_steps, n_rows);
+        DFL_HIP_CHECK(ctx, hipGetLastError());
+        return DFLASH_OK;
+    }
     if (const int32_t rc_ = dfl_raise_lds_limit(ctx, reinterpret_cast<const void *>(gemm_q8_0_staged_kernel<float>), kQ8StagedLds)) return rc_;
-    const int n_steps = static_cast<int>(hidden / DFL_QK8_0);
     dfl_timed timer(ctx, st, DFL_T_GEMM);
     // sixteen waves split the 64 steps of a row, as the few-row product of a router does for one block
     gemm_q8_0_staged_kernel<float><<<dim3((n_expert + 15) / 16, (n_rows + 15) / 16), 64 * kMaxSplit, kQ8StagedLds, st>>>(

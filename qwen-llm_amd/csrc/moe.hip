@@ -501,8 +501,11 @@ constexpr int kGroupPicksPerThread = 16;
 __global__ void __launch_bounds__(1024)
     moe_group_slots_kernel(const int32_t *__restrict__ sel_e, int n_rows, int n_used, int n_expert, int32_t *__restrict__ n_slots,
                            int32_t *__restrict__ slot_rows, int32_t *__restrict__ pick_pos, int4 *__restrict__ tiles,
-                           int32_t *__restrict__ n_tiles, int max_slots, int tile_slots) {
+                           int32_t *__restrict__ n_tiles, int max_slots, int tile_slots, uint32_t by_used) {
     __shared__ int cnt[256], base[257], wave_s[4], wave_t[4];
+    // the experts' slot rows are put together here and leave in whole lines: a row's place is anywhere, and 16384 stores of four
+    // bytes to a line each were 7 us of one CU's address path (16.4 us a launch, 12.5 now, at 2048 rows of 8 picks)
+    extern __shared__ __attribute__((aligned(16))) int32_t rows_sh[];
     const int tid = threadIdx.x, lane = tid & 63;
     if (tid < 256) cnt[tid] = 0;
     __syncthreads();
@@ -553,7 +556,7 @@ __global__ void __launch_bounds__(1024)
             tiles[pt - nt + t] = int4{tid, b + first, ns * (t + 1) / nt - first, 0};
         }
         if (c & 15)
-            for (int m = c & 15; m < 16; m++) slot_rows[(b + (c >> 4)) * 16 + m] = 0;
+            for (int m = c & 15; m < 16; m++) rows_sh[(b + (c >> 4)) * 16 + m] = 0;
     }
     for (int t = tid; t < shared_t; t += 1024) {
         const int first = n_blocks * t / shared_t;
@@ -566,30 +569,51 @@ __global__ void __launch_bounds__(1024)
         if (my_e[j] >= 0) {
             const int p = tid + 1024 * j;
             const int at = (base[my_e[j]] + (my_place[j] >> 4)) * 16 + (my_place[j] & 15);
-            slot_rows[at] = p / n_used;
+            rows_sh[at] = n_used == 1 ? p : static_cast<int>(__umulhi(p, by_used));  // p / n_used
             pick_pos[p] = at;
         }
     }
+    __syncthreads();
+    for (int i = tid; i < 4 * total; i += 1024) reinterpret_cast<int4 *>(slot_rows)[i] = reinterpret_cast<const int4 *>(rows_sh)[i];
 }
 
 // A slot's rows in fragment order (kind Q4K) with their sub-block sums, rounded to f16 as every few-row kernel rounds its
-// activations: one wave per (super-block, slot), lane (m, g) takes the 64 values of chunk g of the slot's row m.
+// activations: one wave per (super-block, slot).  Lane (m, q) reads sixteenths of 64 bytes of row m, the q-th 16 of each, so a load
+// takes half lines of sixteen rows; in the output it has the 64 values of chunk q, the (4 x 4) blocks of the four lanes of a row
+// being exchanged by swaps of lanes 32 and 16 apart.  (Each lane its own 64 values: 64 lines a load, the address path's 16 us of 30
+// at 2048 rows of 8 picks; 25.5 now, the 90 MB it writes being most of it.)
 __global__ void __launch_bounds__(64)
     moe_group_gather_kernel(const float *__restrict__ cur, const int32_t *__restrict__ slot_rows, const int32_t *__restrict__ n_slots,
                             int hidden, uint8_t *__restrict__ xg, uint8_t *__restrict__ sums) {
-    const int b = blockIdx.x, slot = blockIdx.y, lane = threadIdx.x, m = lane & 15, g = lane >> 4, nb = hidden >> 8;
+    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+    const int b = blockIdx.x, slot = blockIdx.y, lane = threadIdx.x, m = lane & 15, q = lane >> 4, nb = hidden >> 8;
     if (slot >= *n_slots) return;
-    const float4_t *src = reinterpret_cast<const float4_t *>(cur + static_cast<size_t>(slot_rows[slot * 16 + m]) * hidden + 256 * b + 64 * g);
+    const float4_t *src = reinterpret_cast<const float4_t *>(cur + static_cast<size_t>(slot_rows[slot * 16 + m]) * hidden + 256 * b) + q;
     half8_t *dst = reinterpret_cast<half8_t *>(xg + (static_cast<size_t>(slot) * nb + b) * 8192) + lane;
     float4_t v[16];
 #pragma unroll
-    for (int i = 0; i < 16; i++) v[i] = src[i];
+    for (int i = 0; i < 16; i++) v[i] = src[4 * i];
+    // p[c][2 j + k]: pair k of the four values 64 c + 16 j + 4 q
+    float p[4][8];
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+        p[i >> 2][2 * (i & 3)] = __builtin_bit_cast(float, h2{static_cast<_Float16>(v[i][0]), static_cast<_Float16>(v[i][1])});
+        p[i >> 2][2 * (i & 3) + 1] = __builtin_bit_cast(float, h2{static_cast<_Float16>(v[i][2]), static_cast<_Float16>(v[i][3])});
+    }
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        dfl_swap32(p[0][e], p[2][e]);  // chunks 0 and 1 to the lower lanes, 2 and 3 to the upper, of the other half's lane in p[2], p[3]
+        dfl_swap32(p[1][e], p[3][e]);
+        dfl_swap16(p[0][e], p[1][e]);
+        dfl_swap16(p[2][e], p[3][e]);
+    }
+    // p[k]: what lane k of the row had of this lane's chunk
     float o[8];
 #pragma unroll
     for (int t = 0; t < 8; t++) {
-        _Float16 h[8];
-#pragma unroll
-        for (int i = 0; i < 8; i++) h[i] = static_cast<_Float16>(v[2 * t + (i >> 2)][i & 3]);
+        const h2 a = __builtin_bit_cast(h2, p[2 * (t & 1)][t & ~1]), c = __builtin_bit_cast(h2, p[2 * (t & 1)][(t & ~1) + 1]);
+        const h2 d = __builtin_bit_cast(h2, p[2 * (t & 1) + 1][t & ~1]), f = __builtin_bit_cast(h2, p[2 * (t & 1) + 1][(t & ~1) + 1]);
+        const _Float16 h[8] = {a[0], a[1], c[0], c[1], d[0], d[1], f[0], f[1]};
         const half8_t frag = {h[0], h[2], h[1], h[3], h[4], h[6], h[5], h[7]};
         dst[t * 64] = frag;
         o[t] = q4k_octet_sum_seq(h);
@@ -793,8 +817,11 @@ int32_t dfl_moe_ffn_group(dflash_ctx *ctx, const dflash_model_cfg &c, const dfla
     //               385 : 385, 468 : 468, 575 : 590
     const int narrow_ct = std::min(fe / 128, H / 256);  // column tiles of the narrower product, gate and up or down
     const int tile_slots = n_rows * used >= 85 * E && E * narrow_ct >= 2 * ctx->n_cu ? 8 : 4;
-    moe_group_slots_kernel<<<1, 1024, 0, st>>>(s.sel_e, n_rows, used, E, s.n_slots, s.slot_rows, s.pick_pos, reinterpret_cast<int4 *>(s.tiles),
-                                             s.n_tiles, max_slots, tile_slots);
+    const size_t slots_lds = static_cast<size_t>(max_slots - (n_rows + 15) / 16) * 16 * sizeof(int32_t);  // (at most 1280 slots of experts)
+    if ((rc = dfl_raise_lds_limit(ctx, reinterpret_cast<const void *>(moe_group_slots_kernel), slots_lds))) return rc;
+    moe_group_slots_kernel<<<1, 1024, slots_lds, st>>>(s.sel_e, n_rows, used, E, s.n_slots, s.slot_rows, s.pick_pos, reinterpret_cast<int4 *>(s.tiles),
+                                                     s.n_tiles, max_slots, tile_slots,
+                                                     static_cast<uint32_t>(((1ull << 32) + used - 1) / used));  // (exact: picks x used < 2^32)
     moe_group_gather_kernel<<<dim3(H / DFL_QK_K, max_slots), 64, 0, st>>>(cur, s.slot_rows, s.n_slots, H, s.xg, s.xg_sums);
     const size_t stride_in = dflash_q4k_tiled_bytes(H, fe), stride_dn = dflash_q4k_tiled_bytes(fe, H);
     // most row tiles the list can have: one per tile_slots slots, and a short one per expert and for the shared one

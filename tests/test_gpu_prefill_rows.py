@@ -180,6 +180,15 @@ def test_expert_tiles_of_eight_blocks_equal_block_by_block(ctx, rows):
     test_many_row_prefill_equals_block_by_block(ctx, "experts128", rows)
 
 
+@pytest.mark.parametrize("hidden,n_expert,used,rows", [(512, 72, 3, 832), (512, 72, 3, 850), (2048, 200, 1, 321), (256, 129, 2, 530)])
+def test_routers_of_many_rows_equal_block_by_block(ctx, hidden, n_expert, used, rows):
+    """Routers whose last workgroup of 64 weight rows has eight of them or one, one to four steps of K a wave or none for some waves, row
+    counts from the first that takes them, a last block of two rows and of one; slots of one, two and three picks a row."""
+    SHAPES["router"] = (dfl.ModelConfig(n_layers=2, hidden=hidden, n_q=4, n_kv=2, head_dim=128, ffn=0, vocab=2048, n_expert=n_expert,
+                                        n_expert_used=used, ffn_expert=256, ffn_shared=256), dfl.synth.Q6_K)
+    test_many_row_prefill_equals_block_by_block(ctx, "router", rows)
+
+
 @pytest.mark.parametrize("rows", [17, 192, 200, 530])
 def test_a_mixture_with_q4k_projections_equals_block_by_block(ctx, rows):
     """Its output projection's minima go by sums made ahead of the product: past held weights up to their last count, and split."""
