@@ -2746,9 +2746,9 @@ __global__ void __launch_bounds__(64 * kMaxSplit)
 
 // The router of a mixture-of-experts layer together with the residual add, the RMSNorm and the shared-expert gate
 // that precede it (rms_norm_kernel of the model followed by the kernel above, as one launch).  One workgroup per
-// (16 experts, block row): it normalises its row of x + add exactly as the norm kernel does (256 threads, the row in
+// (OUT experts, block row): it normalises its row of x + add exactly as the norm kernel does (256 threads, the row in
 // registers), keeps the f16 copy in LDS as the one live row of the MFMA's X operand (the other fifteen are zeros: a
-// row's products do not depend on its neighbours) and multiplies it with its 16 weight rows.  The kernel
+// row's products do not depend on its neighbours) and multiplies it with its weight rows.  The kernel
 // above gives a workgroup all 16 rows, 162 KB to take in where this one takes 50 KB, and a CU takes in only 20-30 KB
 // per microsecond: 16 x 8 small workgroups instead of 8 large ones, and no launch for the norm.  (Measured first
 // with the norm of all 16 rows inside each of the 8 workgroups, 290 KB each: slower than the two launches.)  The
@@ -2757,6 +2757,10 @@ __global__ void __launch_bounds__(64 * kMaxSplit)
 // residual.  Sums are taken in rms_norm_kernel's order (the first four waves do the norm) and the product in the order
 // of the kernel above with 16 waves, so cur, gate_out and y have the bits of the two separate launches.  One 64-step
 // chunk: hidden <= 2048.
+// OUT of the 16 weight rows an MFMA takes are there (the other lanes repeat the last one, their products are not
+// written): a lane's eight weights and their scale are two loads of two bytes' alignment, sixteen rows of 34-byte blocks are
+// some 24 lines a load, and 128 such loads a workgroup are 1.3 us of a CU's address path, beside the 35 KB.
+template <int OUT>
 __global__ void __launch_bounds__(64 * kMaxSplit)
     q8_0_norm_router_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x, const float *__restrict__ add,
                             const float *__restrict__ norm_w, const float *__restrict__ gate_w, int n_out, int n_steps, float eps,
@@ -2768,7 +2772,7 @@ __global__ void __launch_bounds__(64 * kMaxSplit)
     __shared__ float sq_part[4], dot_part[4];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int n = lane & 15, g = lane >> 4;
-    const int n0 = blockIdx.x * 16, r = blockIdx.y;
+    const int n0 = blockIdx.x * OUT, r = blockIdx.y;
     const int hidden = 32 * n_steps;
     const bool first_tile = blockIdx.x == 0;
     const bool norm_wave = wave < 4;  // the norm is the work of 256 threads, as in rms_norm_kernel; the row's loads go out first
@@ -2791,7 +2795,7 @@ __global__ void __launch_bounds__(64 * kMaxSplit)
     constexpr int kSteps = kQ8ChunkSteps / kMaxSplit;
     Raw8<DFLASH_TYPE_Q8_0> rw[kSteps];
     {
-        const uint8_t *wrow = w + static_cast<size_t>(min(n0 + n, n_out - 1)) * (n_steps * DFL_Q8_0_BYTES);
+        const uint8_t *wrow = w + static_cast<size_t>(min(n0 + min(n, OUT - 1), n_out - 1)) * (n_steps * DFL_Q8_0_BYTES);
 #pragma unroll
         for (int i = 0; i < kSteps; i++) rw[i] = load_raw8<DFLASH_TYPE_Q8_0>(wrow, static_cast<int64_t>(min(s0 + i, n_steps - 1)) * 32 + 8 * g);
     }
@@ -2861,7 +2865,7 @@ __global__ void __launch_bounds__(64 * kMaxSplit)
     DFL_TRR(5);
     __syncthreads();
     DFL_TRR(6);
-    if (tid < 16 && n0 + tid < n_out) {
+    if (tid < OUT && n0 + tid < n_out) {
         float sum = 0.0f;
         for (int wv = 0; wv < kMaxSplit; wv++) sum += red[wv][tid];
         y[static_cast<size_t>(r) * n_out + n0 + tid] = sum;
@@ -3370,10 +3374,21 @@ int32_t dfl_router_norm(dflash_ctx *ctx, const void *router_w, const float *x, c
         if (reinterpret_cast<uintptr_t>(p) % 16)
             return dfl_fail(ctx, DFLASH_ERR_ALIGNMENT, "router_norm: rows and weights must be 16-byte aligned");
     const int n_steps = static_cast<int>(hidden / DFL_QK8_0);
-    const int tiles = (n_expert + 15) / 16;
     dfl_timed timer(ctx, st, DFL_T_GEMM);
-    q8_0_norm_router_kernel<<<dim3(tiles, n_rows), 64 * kMaxSplit, 0, st>>>(static_cast<const uint8_t *>(router_w), x, add, norm_w, gate_w, n_expert,
-                                                                 n_steps, eps, cur, gate_out, logits);
+#define DFL_ROUTER(OUT)                                                                                                                     \
+    q8_0_norm_router_kernel<OUT><<<dim3((n_expert + OUT - 1) / OUT, n_rows), 64 * kMaxSplit, 0, st>>>(                                       \
+        static_cast<const uint8_t *>(router_w), x, add, norm_w, gate_w, n_expert, n_steps, eps, cur, gate_out, logits)
+    // The fewest experts a workgroup with which the launch is one workgroup a CU.  2048 to 128 experts, 16 : 8 : 4 : 2 experts: one row,
+    // decode step of 40 layers 2156 : 2151 : 2032 : 2079 us; 16 rows, verify 3601 : 3550 : 3648 : 3848
+    // (8 experts: 256 workgroups).
+    const int64_t logits_n = static_cast<int64_t>(n_rows) * n_expert;
+    if (logits_n <= 4 * ctx->n_cu)
+        DFL_ROUTER(4);
+    else if (logits_n <= 8 * ctx->n_cu)
+        DFL_ROUTER(8);
+    else
+        DFL_ROUTER(16);
+#undef DFL_ROUTER
     DFL_HIP_CHECK(ctx, hipGetLastError());
     return DFLASH_OK;
 }

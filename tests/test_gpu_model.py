@@ -490,6 +490,28 @@ def test_short_expert_lists_give_the_bits_of_long_ones(ctx, hidden, n_expert, us
     assert np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32))
 
 
+@pytest.mark.parametrize("hidden,n_expert", [(2048, 130), (256, 133), (1024, 200), (2048, 9)])
+def test_routers_split_over_more_workgroups_give_the_same_bits(ctx, hidden, n_expert):
+    """A router's launch takes four, eight or sixteen experts a workgroup by rows times experts: rows of blocks of different sizes,
+    on both sides of both lines, are the bits they are by themselves, last workgroups of one to ten experts included."""
+    import torch
+
+    cfg = dfl.ModelConfig(n_layers=1, hidden=hidden, n_q=4, n_kv=2, head_dim=64, ffn=0, vocab=4096, n_expert=n_expert, n_expert_used=3,
+                          ffn_expert=256, ffn_shared=256)
+    model = dfl.TargetModel(ctx, cfg, dfl.synth_target_weights(cfg, seed=hidden + n_expert))
+    toks = np.random.default_rng(n_expert).integers(0, cfg.vocab, 16).tolist()
+    n_cu = torch.cuda.get_device_properties(0).multi_processor_count
+    lines = [min(16, per * n_cu // n_expert) for per in (4, 8)]
+    got = []
+    for n in sorted({1, 16, *lines, *(min(16, at + 1) for at in lines)}):
+        sess = dfl.Session(ctx, model, 32, [0])
+        got.append(sess.encode_packed_verify_layer_major(toks[:n], 0).hidden_capture.cpu().numpy())
+        sess.close()
+    assert np.all(np.isfinite(got[-1])) and np.ptp(got[-1]) > 0
+    for g in got:
+        assert np.array_equal(g.view(np.uint32), got[-1][: len(g)].view(np.uint32))
+
+
 def test_draft_block_general_positions(ctx, oracle, target):
     """Context columns at arbitrary positions and a block that does not start right behind them: the
     general f32 drafter attention (the MFMA path needs positions 0, 1, 2, ... and start == ctx_len)."""
