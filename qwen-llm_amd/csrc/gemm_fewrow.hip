@@ -2666,6 +2666,81 @@ __global__ void __launch_bounds__(64 * kMaxSplit)
     }
 }
 
+// The same product for few tiles, over more of the chip: a workgroup has four of the block's rows and OUT weight rows, and the next
+// chunk's bytes are on their way while this one is multiplied.  (The kernel above is bound by what one of its few workgroups
+// takes in, all sixteen rows and sixteen weight rows, a chunk at a time with nothing under way in between: 18 us for 16 rows 8192 ->
+// 1024, 12 here.)  Sixteen waves and the
+// chunks cut K as above, so a product has the bits it has there.
+constexpr int kQ8SplitRows = 4;
+template <typename XT, int OUT>
+__global__ void __launch_bounds__(64 * kMaxSplit)
+    gemm_q8_0_split_kernel(const uint8_t *__restrict__ w, const XT *__restrict__ x, int n_out, int n_steps, int n_rows, float *__restrict__ y) {
+    constexpr int kPer = kMaxSplit / OUT, kRow = kQ8ChunkSteps * DFL_Q8_0_BYTES / 16, kPieces = (kRow + 64 * kPer - 1) / (64 * kPer);
+    static_assert(kMaxSplit * 64 == kQ8SplitRows * 4 * kQ8ChunkSteps, "a piece of the activations per thread and chunk");
+    __shared__ __attribute__((aligned(16))) uint8_t ws[OUT * kQ8WRowStride];
+    __shared__ half8_t xs[4 * kQ8ChunkSteps * (kQ8SplitRows + 1)];  // [step][k-group][row], a group's rows padded by one
+    __shared__ float red[kMaxSplit][kQ8SplitRows][OUT];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n = lane & 15, g = lane >> 4;
+    const int n0 = blockIdx.x * OUT, row0 = blockIdx.y * kQ8SplitRows;
+    // this thread's pieces of a chunk: of one weight row (past n_out the last one) and of one activation row (past n_rows the last one)
+    const int wr_row = wave / kPer, wr_at = (wave % kPer) * 64 + lane, xr_row = wave >> 2, xr_at = (wave & 3) * 64 + lane;
+    const uint8_t *wsrc = w + static_cast<size_t>(min(n0 + wr_row, n_out - 1)) * (static_cast<size_t>(n_steps) * DFL_Q8_0_BYTES);
+    const XT *xsrc = x + static_cast<size_t>(min(row0 + xr_row, n_rows - 1)) * (static_cast<size_t>(n_steps) * 32);
+    u32x4_t wr[kPieces];
+    RawX8<XT> xr;
+    auto fetch = [&](int c0) {
+        const int cs = min(kQ8ChunkSteps, n_steps - c0), pieces = cs * DFL_Q8_0_BYTES / 16;
+        const uint8_t *wp = wsrc + static_cast<size_t>(c0) * DFL_Q8_0_BYTES;
+#pragma unroll
+        for (int i = 0; i < kPieces; i++) wr[i] = *reinterpret_cast<const u32x4_t *>(wp + 16 * min(wr_at + 64 * kPer * i, pieces - 1));
+        xr = load_rawx8(xsrc + static_cast<size_t>(c0) * 32 + 8 * min(xr_at, 4 * cs - 1));
+    };
+    // LDS only: the next chunk's loads stay in flight across it
+    auto barrier = [] {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    float4_t acc = {0, 0, 0, 0};
+    fetch(0);
+    for (int c0 = 0; c0 < n_steps; c0 += kQ8ChunkSteps) {
+        const int cs = min(kQ8ChunkSteps, n_steps - c0), pieces = cs * DFL_Q8_0_BYTES / 16;
+        if (c0) barrier();  // the previous chunk's fragments have been read
+#pragma unroll
+        for (int i = 0; i < kPieces; i++) {
+            const int at = wr_at + 64 * kPer * i;
+            if (at < pieces) *reinterpret_cast<u32x4_t *>(ws + wr_row * kQ8WRowStride + 16 * at) = wr[i];
+        }
+        if (xr_at < 4 * cs) xs[xr_at * (kQ8SplitRows + 1) + xr_row] = convert_rawx8(xr);
+        if (c0 + kQ8ChunkSteps < n_steps) fetch(c0 + kQ8ChunkSteps);
+        barrier();
+        const int s0 = cs * wave / kMaxSplit, s1 = cs * (wave + 1) / kMaxSplit;
+        const uint8_t *rowp = ws + min(n, OUT - 1) * kQ8WRowStride;
+        for (int s = s0; s < s1; s++) {
+            const uint8_t *blk = rowp + s * DFL_Q8_0_BYTES;  // 2-byte aligned
+            const uint16_t *q16 = reinterpret_cast<const uint16_t *>(blk + 2 + 8 * g);
+            Raw8<DFLASH_TYPE_Q8_0> r;
+            r.d = static_cast<float>(__builtin_bit_cast(_Float16, *reinterpret_cast<const uint16_t *>(blk)));
+            r.q = static_cast<uint64_t>(q16[0]) | (static_cast<uint64_t>(q16[1]) << 16) | (static_cast<uint64_t>(q16[2]) << 32) |
+                  (static_cast<uint64_t>(q16[3]) << 48);
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(xs[(4 * s + g) * (kQ8SplitRows + 1) + (n & (kQ8SplitRows - 1))],
+                                                         convert_raw8<DFLASH_TYPE_Q8_0>(r), acc, 0, 0, 0);
+        }
+    }
+    // (the MFMA's sixteen rows are the four, four times: the first four are in lane group 0)
+    if (g == 0 && n < OUT)
+#pragma unroll
+        for (int i = 0; i < kQ8SplitRows; i++) red[wave][i][n] = acc[i];
+    __syncthreads();
+    const int m = tid / OUT, nn = tid % OUT;
+    if (m < kQ8SplitRows && row0 + m < n_rows && n0 + nn < n_out) {
+        float sum = 0.0f;
+#pragma unroll
+        for (int wv = 0; wv < kMaxSplit; wv++) sum += red[wv][m][nn];
+        y[static_cast<size_t>(row0 + m) * n_out + n0 + nn] = sum;
+    }
+}
+
 // The same product for the many rows of a prefill group: a workgroup has sixteen rows and 64 weight rows instead of 16, so the
 // rows are read and converted by a quarter of the workgroups, straight into the MFMA operands (every wave has four steps of K for
 // itself, a line of each row a step), while the weights come through LDS, a row in whole lines.  Waves and steps are cut as above with
@@ -3613,6 +3688,26 @@ int32_t gemm_fewrow_impl(dflash_ctx *ctx, int32_t w_type, const void *w, const v
             DFL_LAUNCH_GENERIC(DFLASH_TYPE_F16);
         else if (n_in % 256 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
             env_int("DFLASH_Q8_STAGED", 1)) {
+            // Four rows and four, eight or sixteen weight rows a workgroup, the fewest that are one round of the chip; past that its rounds cost
+            // more than they save.  us a call, below : here (7.2 to 8 is the host): 16 rows 8192 -> 1024 18.2 : 11.8, 8192 -> 128 18.0 : 10.0,
+            // 11 rows 5632 -> 1024 12.8 : 8.7, one row 8192 -> 1024 17.5 : 10.1; two rounds, 16 rows 8192 -> 2170 17.8 : 27.2.
+            const int groups = (n_rows + kQ8SplitRows - 1) / kQ8SplitRows;
+            if (split == kMaxSplit && groups * tiles <= ctx->n_cu) {
+#define DFL_Q8_SPLIT(XT, OUT)                                                                                                                \
+    gemm_q8_0_split_kernel<XT, OUT><<<dim3(static_cast<unsigned>((n_out + OUT - 1) / OUT), groups), 64 * kMaxSplit, 0, st>>>(                \
+        wb, static_cast<const XT *>(x), static_cast<int>(n_out), static_cast<int>(n_steps), n_rows, y)
+#define DFL_Q8_SPLIT_OUT(OUT) (x_type == DFLASH_TYPE_F32 ? DFL_Q8_SPLIT(float, OUT) : DFL_Q8_SPLIT(_Float16, OUT))
+                if (groups * ((n_out + 3) / 4) <= ctx->n_cu)
+                    DFL_Q8_SPLIT_OUT(4);
+                else if (groups * ((n_out + 7) / 8) <= ctx->n_cu)
+                    DFL_Q8_SPLIT_OUT(8);
+                else
+                    DFL_Q8_SPLIT_OUT(16);
+#undef DFL_Q8_SPLIT_OUT
+#undef DFL_Q8_SPLIT
+                DFL_HIP_CHECK(ctx, hipGetLastError());
+                return DFLASH_OK;
+            }
             if (const int32_t rc_ = dfl_raise_lds_limit(ctx, x_type == DFLASH_TYPE_F32
                                                                  ? reinterpret_cast<const void *>(gemm_q8_0_staged_kernel<float>)
                                                                  : reinterpret_cast<const void *>(gemm_q8_0_staged_kernel<_Float16>),

@@ -405,3 +405,28 @@ def test_repack_declines_a_tensor_out_of_range(ctx):
     with pytest.raises(dfl.DFlashError) as e:
         ctx.repack_q4k_tiled(dev(w), n_in, n_out)
     assert e.value.status == 2
+
+
+@pytest.mark.parametrize("n_in,n_out", [(512, 5), (2048, 128), (2304, 777), (4352, 1024), (8192, 1031), (2560, 2049), (6144, 4)])
+@pytest.mark.parametrize("rows,x_dtype", [(1, "f32"), (4, "f16"), (5, "f32"), (13, "f16"), (16, "f32")])
+def test_q8_0_split_over_the_chip_gives_the_bits_of_sixteen_rows_a_workgroup(ctx, oracle, canaries, n_in, n_out, rows, x_dtype):
+    """Few tiles of Q8_0 take four rows and four to sixteen weight rows a workgroup: one to four chunks of K, the last of 8 steps or more,
+    ragged tiles and row groups; the same bits as in a matrix of 136 tiles, whose sixteen rows stay together, and for a row alone."""
+    import torch
+
+    blocks = dfl.synth.random_blocks(dfl.synth.Q8_0, n_out * n_in // 32, seed=n_in + n_out).reshape(n_out, -1)
+    w = dev(blocks)
+    x = np.random.default_rng(rows).standard_normal((16, n_in)).astype(np.float32)
+    xd = dev(x.astype(np.float16 if x_dtype == "f16" else np.float32))
+    y = ctx.gemm_fewrow(w, dfl.TYPE_Q8_0, xd[:rows].clone(), n_in, n_out)
+    canaries.check()
+    wide = torch.cat([w, w[:1].expand(2176 - n_out, -1)]).contiguous()
+    together = ctx.gemm_fewrow(wide, dfl.TYPE_Q8_0, xd, n_in, 2176)[:rows, :n_out].contiguous()
+    assert torch.equal(together.view(torch.int32), y.view(torch.int32))
+    alone = ctx.gemm_fewrow(w, dfl.TYPE_Q8_0, xd[rows - 1:rows].clone(), n_in, n_out)
+    assert torch.equal(alone.view(torch.int32), y[rows - 1:].view(torch.int32))
+    wf = oracle.dequant(dfl.synth.Q8_0, blocks, n_out * n_in).reshape(n_out, n_in).astype(np.float64)
+    ref = x[:rows].astype(np.float16).astype(np.float64) @ wf.T
+    # a weight d * q rounded to f16: 2^-11 of itself at most, so of the sum of its terms' sizes; f32 sums on top
+    bound = np.abs(x[:rows].astype(np.float16)).astype(np.float64) @ np.abs(wf).T * (2.0 ** -11 + n_in * 2.0 ** -24)
+    assert np.all(np.abs(y.cpu().numpy() - ref) <= bound)
