@@ -788,10 +788,10 @@ def main():
                    "weight_footprint_bytes": n_sets * sum(w_bytes)},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS, "traffic": measured_traffic(),
-                     "kernel": "gemm_q4k_tiled_kernel", "bytes_per_launch": k_bytes, "us_per_launch": k_us,
+                     "kernel": "gemm_q4k_wide_kernel / gemm_q4k_tiled_kernel", "bytes_per_launch": k_bytes, "us_per_launch": k_us,
                      "read_probe_GBps": ceiling, "frac_of_read_probe": achieved / ceiling,
                      "note": "the streaming kernel's own duration (start / stop stamps of the dispatch, as a kernel trace reports "
-                             "it), mean over the three shapes; its split-K reduction is another kernel; every launch streams "
+                             "it), mean over the three shapes; the split-K reduction of those that have one is another kernel; every launch streams "
                              "from HBM (each shape rotates over more than 256 MB of copies); the whole call is "
                              "shapes[].call_us_with_reduction, the whole step is `value`",
                      "whole_call_frac": k_bytes / (sum(call_us) / len(call_us) * 1e-6) / 1e9 / HBM_PEAK_GBS},
