@@ -2825,7 +2825,7 @@ __global__ void __launch_bounds__(64 * kMaxSplit)
 // registers), keeps the f16 copy in LDS as the one live row of the MFMA's X operand (the other fifteen are zeros: a
 // row's products do not depend on its neighbours) and multiplies it with its weight rows.  The kernel
 // above gives a workgroup all 16 rows, 162 KB to take in where this one takes 50 KB, and a CU takes in only 20-30 KB
-// per microsecond: 16 x 8 small workgroups instead of 8 large ones, and no launch for the norm.  (Measured first
+// per microsecond: 16 x 8 small workgroups, or more, instead of 8 large ones, and no launch for the norm.  (Measured first
 // with the norm of all 16 rows inside each of the 8 workgroups, 290 KB each: slower than the two launches.)  The
 // workgroups of tile 0 write the row's f32 copy (cur, read by the expert products) and its gate.  x itself is NOT
 // updated (other workgroups are still reading the row): the caller adds `add` again where it next updates the
