@@ -36,7 +36,7 @@ constexpr int kChunk = 8192;       // tokens per workgroup of the argmax / top-2
 // per workgroup that is 589 workgroups of 1024 threads, more than the chip holds at once (two per CU), and the kernel
 // takes two rounds of a workgroup whose time is mostly latency; at 16384 it is 310 and one round.
 constexpr int kSelChunk = 16384;
-constexpr int kSelThreads = 1024;  // 8 tokens per thread
+constexpr int kSelThreads = 1024;  // 16 tokens per thread
 constexpr int kMaxRows = 16;
 constexpr int kNoNan = 0x7fffffff;
 
@@ -715,10 +715,13 @@ constexpr int kDecThreads = 64 * kMaxRows;
 __global__ void __launch_bounds__(kDecThreads)
     decide_kernel(const RowDist *__restrict__ rows, const double *__restrict__ tile_sums, dflash_accept_decision *__restrict__ out, int mode,
                   int n_tiles, int n_tokens, DecideArgs a) {
-    constexpr int kStage = 256;  // tile sums per row and round
+    constexpr int kStage = 256, kAhead = 16;  // tile sums per row and round, and of those that are read ahead of their additions
     __shared__ double p_total[kMaxRows];
     __shared__ RowOutcome outcome[kMaxRows];
-    __shared__ alignas(16) double staged[kMaxRows][kStage + 2];  // (a row per lane is read, two sums at a time: the lanes' banks differ)
+    // (a row's last read ahead is behind its sums, never used; a row per lane is read, two sums at a time: two more words a row make
+    // the lanes' banks differ)
+    __shared__ alignas(16) double staged[kMaxRows][kStage + kAhead + 2];
+    static_assert(kStage % kAhead == 0 && sizeof(staged[0]) >= (kStage + kAhead) * sizeof(double), "the last read ahead stays in its row");
     const int tid = threadIdx.x, lane = tid & 63, row = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n_drafts = n_tokens - 1;
     const bool dense = mode == 2, live = row < n_tokens;
@@ -744,18 +747,18 @@ __global__ void __launch_bounds__(kDecThreads)
             __syncthreads();
             if (row == kMaxRows - 1 && lane < n_drafts) {
                 // (the next sixteen are read ahead of these sixteen's additions; past the last tile is +0, which changes no sum of
-                // exponentials; the last read ahead is of the next row, which is there: lane 15 has none)
+                // exponentials)
                 const int n = min(kStage, n_tiles - t0);
-                double v[16], next[16];
+                double v[kAhead], next[kAhead];
 #pragma unroll
-                for (int j = 0; j < 16; j++) v[j] = staged[lane][j];
-                for (int i = 0; i < n; i += 16) {
+                for (int j = 0; j < kAhead; j++) v[j] = staged[lane][j];
+                for (int i = 0; i < n; i += kAhead) {
 #pragma unroll
-                    for (int j = 0; j < 16; j++) next[j] = staged[lane][i + 16 + j];
+                    for (int j = 0; j < kAhead; j++) next[j] = staged[lane][i + kAhead + j];
 #pragma unroll
-                    for (int j = 0; j < 16; j++) P += v[j];
+                    for (int j = 0; j < kAhead; j++) P += v[j];
 #pragma unroll
-                    for (int j = 0; j < 16; j++) v[j] = next[j];
+                    for (int j = 0; j < kAhead; j++) v[j] = next[j];
                 }
             }
             if (t0 + kStage >= n_tiles) break;  // (more rounds: vocabularies above 262144 tokens)

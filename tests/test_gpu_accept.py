@@ -385,6 +385,24 @@ def test_selection_and_decision_off_their_short_paths(ctx, oracle, kind, top_k):
             assert_same(oracle, *r)
 
 
+@pytest.mark.parametrize("n_tiles", [255, 256, 257, 513])
+def test_dense_sums_of_whole_rounds_of_tiles(ctx, oracle, n_tiles):
+    """A draft row's sum is taken in rounds of 256 tiles of 1024 tokens, sixteen of them read ahead of their additions: one round less a
+    tile, exactly one, one and a tile, two and a tile, the last tile ragged but for the full round, at a block of sixteen rows (the last
+    draft row is the last row of the sums) and one of three."""
+    vocab, T = 1024 * n_tiles - (0 if n_tiles == 256 else 1000), 0.7
+    rng = np.random.default_rng(n_tiles)
+    for n in (16, 3):
+        tl = (rng.standard_normal((n, vocab)) * 3.0).astype(np.float32)
+        dl = (tl[: n - 1] + rng.standard_normal((n - 1, vocab)) * 0.5).astype(np.float32)
+        dl[:, -50:] += 4.0  # (the last tile weighs in the sum)
+        tl[: n - 1, -50:] += 4.0
+        for seed in range(6):
+            drafts = [int(np.argmax(dl[r])) if (r + seed) % 5 else vocab - 1 - r for r in range(n - 1)]
+            r = both(ctx, oracle, [3] + drafts, tl, vocab, None, 100, [], draft=dl, draft_T=T, seed=seed, temperature=T, top_k=20)
+            assert_same(oracle, *r)
+
+
 @pytest.mark.parametrize("kind,n_trials", [(dfl.RNG_PHILOX, 10000), (dfl.RNG_XOSHIRO, 2000)])
 def test_seeded_trials_full_vocab_dense(ctx, oracle, kind, n_trials):
     """Stochastic acceptance at its benchmark size: vocabulary 151936, block 16, target logits N(0, 3), draft = target +
