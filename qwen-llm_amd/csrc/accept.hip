@@ -145,9 +145,11 @@ __device__ __forceinline__ void best_of_chunk(const float *__restrict__ x, int v
 // The k best, without a sort and without finding the k-th: of every wave's 64 per-thread bests the m-th least ordering word,
 // m = ceil(k / waves), bounds m of them, so the largest of the waves' bounds bounds at least k keys of the chunk, and few more
 // than that (k = 20: about a hundred).  What is below it is ranked by counting the candidates below each, and the candidate of
-// rank r < k is output r.  Keys are distinct (the token id is in the low bits), so ranks are too.  Where more than kSelThreads
-// tokens are below the bound (logits ordered by thread, or alike), the k-th best is looked for digit by digit.  (That search
-// for every chunk was 4.7 of its workgroup's 11.3 us, the collecting of what it bounds another 1.8.)
+// rank r < k is output r.  Keys are distinct (the token id is in the low bits), so ranks are too.  (The k-th of the threads' best keys
+// digit by digit in every chunk was 4.7 of its workgroup's 11.3 us, the collecting of what it bounds another 1.8.)
+// Where more than kSelThreads tokens are below the bound (a vocabulary of which a mask has left a few; logits ordered by thread, or
+// alike), the k-th best of the threads' best keys is what bounds them, and with the winners no more than the kSelPer tokens of k threads.
+// (16 rows of 151936, k = 20, one token in a thousand left: 14.8 us, 7.3 unmasked; a digit search over all of the tokens: about 110.)
 __device__ __forceinline__ void select_chunk_body(const float *__restrict__ x, int vocab, int k, uint64_t *__restrict__ out,
                                                   bool nan_is_candidate) {
     __shared__ uint64_t cand[kSelThreads];
@@ -157,6 +159,7 @@ __device__ __forceinline__ void select_chunk_body(const float *__restrict__ x, i
     __shared__ int cnt[2];
     __shared__ int nan_sh;
     constexpr int kWaves = kSelThreads / 64;
+    static_assert(kSelPer * kMaxK <= kSelThreads, "the tokens of k threads are candidates of a thread each");
     const int tid = threadIdx.x, lane = tid & 63, base = blockIdx.x * kSelChunk + tid;
     float v[kSelPer];
     load_chunk(x, vocab, base, v);
@@ -178,7 +181,7 @@ __device__ __forceinline__ void select_chunk_body(const float *__restrict__ x, i
     }
     {
         uint32_t left = best, least = 0xffffffffu;
-        for (int m = 0; m < k; m += kWaves) {
+        for (int m = 0; m < k; m = kWaves * __popcll(__builtin_amdgcn_ballot_w64(best <= least))) {
             least = wave_min_u32(left);
             left = left == least ? 0xffffffffu : left;
         }
@@ -208,13 +211,15 @@ __device__ __forceinline__ void select_chunk_body(const float *__restrict__ x, i
     __syncthreads();
     int n_cand = cnt[0];
     if (n_cand > kSelThreads) {
-        uint64_t keys[kSelPer];
+        uint64_t keys[kSelPer], first = kNoKey;
 #pragma unroll
         for (int j = 0; j < kSelPer; j++) {
             const int i = base + j * kSelThreads;
             keys[j] = i < vocab ? (static_cast<uint64_t>(d[j]) << 32) | static_cast<uint32_t>(i) : kNoKey;
+            first = keys[j] < first ? keys[j] : first;
         }
-        const uint64_t kth_key = block_kth<kSelPer>(keys, kNoKey - 1, k, kSelThreads, kth);
+        const uint64_t limit = bound < 0xffffffffu ? (static_cast<uint64_t>(bound) << 32) | 0xffffffffu : kNoKey - 1;
+        const uint64_t kth_key = block_kth_first(first, best, bound, limit, k, kth);
         compact_keys(keys, kth_key, cand, kSelThreads, &cnt[1]);
         __syncthreads();
         n_cand = cnt[1];

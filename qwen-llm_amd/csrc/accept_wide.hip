@@ -10,6 +10,7 @@
 // runs the chain with a candidate per thread.  Two launches that read the logits once, each bound
 // by its chain of barriers and LDS round trips (the logits take 2 us): 16 rows x 151936 tokens, k = 200: 8.4 + 9.4 us
 // where the sort, its 17 clears and its chain take 316; the whole call 334 -> 38 us.
+// (Of a vocabulary that a mask has left one token in a thousand of, most words are alike: 13.8 + 15.8 us.)
 // Anything larger (the whole vocabulary) is ordered by ONE device-wide radix sort: a key is
 //   row << 60 | descending_logit_bits << 28 | token          (token < 2^28, row < 16)
 // and ascending key order is (row, descending logit in f32 total order, ascending token id): row r's
@@ -71,9 +72,18 @@ __device__ __forceinline__ uint64_t wide_bound(int row, uint32_t word) {
     return bound < kNoKey ? bound : kNoKey - 1;
 }
 
+template <int PER>
+__device__ __forceinline__ uint64_t first_key(const uint64_t (&key)[PER]) {
+    uint64_t first = kNoKey;
+#pragma unroll
+    for (int j = 0; j < PER; j++) first = key[j] < first ? key[j] : first;
+    return first;
+}
+
 // A chunk's winners, the k best keys and at most cap >= k, in no order, at out[(row * n_chunks + chunk) * cap], filled up
-// with kNoKey; the chunk's lowest NaN token.  The k-th best of the per-thread bests bounds every winner, and what is
-// below it usually fits the slots (k = 200: about 250 keys); only where it does not, the k best of all are looked for.
+// with kNoKey; the chunk's lowest NaN token.  The k-th best of the per-thread best words bounds every winner, and what is
+// below it usually fits the slots (k = 200: about 250 keys); only where it does not, the threads' best keys bound them, and only where
+// that does not do either, as many of all as fit are looked for.
 __global__ void __launch_bounds__(kPickThreads)
     pick_chunk_kernel(const float *__restrict__ logits, int64_t vocab, int64_t stride, int k, int cap, uint64_t *__restrict__ out,
                       int32_t *__restrict__ nan_first) {
@@ -103,16 +113,20 @@ __global__ void __launch_bounds__(kPickThreads)
                                    : kNoKey;
         best = min(best, static_cast<uint32_t>(key[j] >> kWideTokenBits));
     }
-    uint64_t bound = wide_bound(row, block_kth_word(best, k, k + k / 8, sh));
+    const uint32_t word = block_kth_word(best, k, k + k / 8, sh);
+    uint64_t bound = wide_bound(row, word);
     const int64_t at = static_cast<int64_t>(row) * gridDim.x + blockIdx.x;
     uint64_t *o = out + at * cap;
     compact_keys(key, bound, o, cap, &cnt[0]);
     __syncthreads();
     int n = cnt[0];
     if (n > cap) {
-        bound = block_kth<kPer>(key, bound, k, k, sh);
+        bound = block_kth_first(first_key(key), best, word, bound, k, sh);
+        __syncthreads();  // (the counters have been read)
+        bound = block_kth<kPer>(key, bound, k, cap, sh);
         compact_keys(key, bound, o, cap, &cnt[1]);
-        n = k;
+        __syncthreads();
+        n = cnt[1];
     }
     for (int i = n + tid; i < cap; i += kPickThreads) o[i] = kNoKey;
     if (tid == 0) nan_first[at] = nan_sh;
@@ -149,7 +163,8 @@ __global__ void __launch_bounds__(kPickMax)
     }
     __syncthreads();
     if (nan != kNoNanW) atomicMin(&nan_sh, nan);
-    uint64_t bound = wide_bound(row, block_kth_word(best, k, k + k / 8, sh));  // (its barriers are behind the minimum)
+    const uint32_t word = block_kth_word(best, k, k + k / 8, sh);  // (its barriers are behind the minimum)
+    uint64_t bound = wide_bound(row, word);
     auto finish = [&](int32_t err, int64_t err_index, int n_keep, double total, int32_t pick, double draft_weight) {
         if (tid == 0) {
             d->n_keep = n_keep;
@@ -167,6 +182,8 @@ __global__ void __launch_bounds__(kPickMax)
     __syncthreads();
     int n = cnt[0];
     if (n > kPickMax) {
+        bound = block_kth_first(first_key(key), best, word, bound, k, sh);
+        __syncthreads();  // (the counters have been read)
         bound = block_kth<PER>(key, bound, k, kPickMax, sh);
         compact_keys(key, bound, cand, kPickMax, &cnt[1]);
         __syncthreads();

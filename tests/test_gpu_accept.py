@@ -2,6 +2,7 @@
 longest-prefix, deterministic coupling, sparse and vocabulary-wide rejection sampling) against
 the CPU oracle on the same logits and the same random stream."""
 import math
+import time
 
 import numpy as np
 import pytest
@@ -383,6 +384,59 @@ def test_selection_and_decision_off_their_short_paths(ctx, oracle, kind, top_k):
             r = both(ctx, oracle, toks, t, vocab, props if mode == "sparse" else None, 100, stops, draft=d if mode == "dense" else None,
                      draft_T=T if mode == "dense" else 0.0, seed=seed, **skw)
             assert_same(oracle, *r)
+
+
+def masked_rows(rng, n, vocab, low, keep):
+    """Logits of which a mask has left one token in 1 / keep: the others are all `low`."""
+    rows = (rng.standard_normal((n, vocab)) * 3.0).astype(np.float32)
+    mask = rng.random(vocab) < keep
+    rows[:, ~mask] = low
+    return rows
+
+
+@pytest.mark.parametrize("low", [-np.inf, np.finfo(np.float32).min, 1.0])
+@pytest.mark.parametrize("top_k", [1, 20, 64, 200, 1000])
+def test_masked_vocabularies(ctx, oracle, low, top_k):
+    """Rows of which a mask has left fewer tokens than k, about as many, and many more, the others all alike at -inf, at the type's lowest
+    value or in the middle of the others; a ragged last chunk of masked tokens only: decisions and sampler state equal the oracle's."""
+    vocab, n, T = 3 * 16384 + 77, 4, 0.7
+    rng = np.random.default_rng(top_k)
+    for keep in (8 / vocab, 0.001, 0.05):
+        tl = masked_rows(rng, n, vocab, low, keep)
+        tl[:, 3 * 16384:] = low
+        tl[:, 11] = 12.0
+        dl = np.where(np.isfinite(tl[: n - 1]), tl[: n - 1], -30.0).astype(np.float32)
+        for seed in range(3):
+            drafts = [int(np.argmax(tl[r])) if seed else int(rng.integers(vocab)) for r in range(n - 1)]
+            for dense in (False, True):
+                r = both(ctx, oracle, [3] + drafts, tl, vocab, None, 100, [], draft=dl if dense else None, draft_T=T if dense else 0.0,
+                         seed=seed, temperature=T, top_k=top_k, top_p=0.95)
+                assert_same(oracle, *r)
+
+
+@pytest.mark.parametrize("top_k", [20, 200])
+def test_a_masked_vocabulary_takes_no_search_over_all_of_its_tokens(ctx, top_k):
+    """A block's decision on 151936 tokens of which a mask has left one in a thousand, against the same block unmasked: at most twice as
+    long.  (A digit search over all tokens that are alike, thousands of them on one counter, is four times as long.)"""
+    import torch
+
+    vocab, n = 151936, 16
+    rng = np.random.default_rng(top_k)
+    plain = (rng.standard_normal((n, vocab)) * 3.0).astype(np.float32)
+    times = []
+    for rows in (plain, masked_rows(rng, n, vocab, -np.inf, 0.001)):
+        t = dev(rows)
+        toks = [int(rows[0].argmax())] + [int(rows[r].argmax()) for r in range(n - 1)]
+        s = dfl.Sampler(temperature=0.7, top_k=top_k, seed=1)
+        best = np.inf
+        for _ in range(5):
+            torch.cuda.synchronize()
+            t0 = time.perf_counter()
+            for _ in range(20):
+                ctx.decide_dflash_accept_prefix(toks, t, vocab, None, s.clone(), 100, [])
+            best = min(best, time.perf_counter() - t0)
+        times.append(best)
+    assert times[1] <= 2 * times[0], [f"{x / 20 * 1e6:.1f} us" for x in times]
 
 
 @pytest.mark.parametrize("n_tiles", [255, 256, 257, 513])
