@@ -1197,6 +1197,8 @@ namespace {
 //   one tile per wave   Q6_K 2048 -> 512   7.3 : 4.2   7.9 : 4.9   7.9 : 5.4    tiled Q4_K 4096 -> 4096  8.4 : 4.4   9.7 : 5.5   9.7 : 6.1
 //                       Q6_K 6144 -> 2048 10.0 : 8.1  11.1 :10.3  11.1 :11.1    Q4_K in row order 6144 -> 2048  8.9 : 6.5  10.0 : 8.2   9.9 : 9.2
 //     beyond 24 super-blocks  Q6_K 8192 -> 1024   9.9 : 8.8  10.7 :11.0  10.8 :12.4 (two stages a wave, each with its rows to bring in)
+//     beyond 22, few tiles, us a call  Q6_K 6144 -> 512  9.0 : 7.9   9.1 :10.0   9.0 :11.2   -> 1024  9.1 : 8.1   9.2 :10.1   9.0 :11.3
+//                                      from half a round of tiles on a single row gains what sixteen lose:  -> 2048  9.4 : 8.3  10.2 :11.2  10.3 :11.5
 //   two tiles per wave  tiled Q4_K 4096 -> 5120  8.9 : 5.8  10.1 : 7.1  10.2 : 7.7    in row order  9.1 : 6.6  10.8 : 8.0  10.8 : 8.9
 //     beyond 16 super-blocks  5120 -> 5120  8.7 : 8.3  10.1 :10.2  10.2 :10.7    Q6_K, 4096 -> 5120  11.5 :13.4 (its registers spill)
 WholePlan rows_direct_plan(const dflash_ctx *ctx, int32_t w_type, int64_t n_in, int64_t n_out) {
@@ -1205,6 +1207,7 @@ WholePlan rows_direct_plan(const dflash_ctx *ctx, int32_t w_type, int64_t n_in, 
     const int nb = static_cast<int>(n_in / DFL_QK_K);
     if (kind == DFL_XF_NONE || n_in % DFL_QK_K || nb < 1 || nb > 24 || n_out < 1 || n_out >= (1 << 24)) return p;
     const int ksplit = nb < 16 ? nb : 16, tiles = static_cast<int>((n_out + 15) / 16);
+    if (kind == DFL_XF_Q6K && nb > 22 && 2 * tiles < ctx->n_cu) return p;
     for (int R = 1; R <= (kind == DFL_XF_Q4K && nb <= 16 ? 2 : 1); R++)
         for (int tl = 1; tl <= 16 / ksplit; tl++) {
             const int units = (tiles + R - 1) / R, n_wg = (units + tl - 1) / tl;

@@ -242,6 +242,28 @@ def test_rows_in_row_order_give_the_bits_of_packed_rows(ctx, oracle, canaries, q
     check(y[:, torch.from_numpy(cols).cuda()].cpu().numpy(), ref, f"{n_in}->{n_out} x{rows}")
 
 
+def reductions(ctx, w, w_type, x, n_in, n_out):
+    """Split-K reductions launched by one call of the public operator: one on the streaming kernels, none in one launch."""
+    ctx.set_kernel_timing(1)
+    ctx.gemm_fewrow(w, w_type, x, n_in, n_out)
+    n = ctx.kernel_timing(4)[1]
+    ctx.set_kernel_timing(0)
+    return n
+
+
+@pytest.mark.parametrize("n_in,n_out,streamed", [(5632, 512, 0), (5888, 512, 1), (6144, 1024, 1), (6144, 2032, 1), (6144, 2033, 0), (6144, 4096, 0),
+                                                 (6400, 4096, 1)])
+def test_q6k_of_many_super_blocks_and_few_tiles_streams(ctx, oracle, n_in, n_out, streamed):
+    """Beyond 22 super-blocks one launch pays from half a round of tiles on; both sides of the line against the f64 product."""
+    w, w_type, blocks, _ = upload(ctx, dfl.synth.Q6_K, n_in, n_out, seed=n_out)
+    x = np.random.default_rng(n_in).standard_normal((16, n_in)).astype(np.float32)
+    assert reductions(ctx, w, w_type, dev(x), n_in, n_out) == streamed
+    y = ctx.gemm_fewrow(w, w_type, dev(x), n_in, n_out).cpu().numpy()
+    cols = np.unique(np.concatenate([np.arange(40), np.arange(n_out - 40, n_out)]))
+    wf = oracle.dequant(dfl.synth.Q6_K, np.ascontiguousarray(blocks[cols]), len(cols) * n_in).reshape(len(cols), n_in).astype(np.float64)
+    check(y[:, cols], x.astype(np.float16).astype(np.float64) @ wf.T, f"{n_in}->{n_out}")
+
+
 # many rounds of tiles: K of one super-block (sixteen tiles a workgroup), of one and two super-blocks a wave, an odd split of K
 # (17: nine waves, one of them with one super-block), the widest (24); a ragged last tile, a last round that few workgroups have
 WIDE_SHAPES = [(256, 140001), (768, 45000), (1024, 33000), (2048, 16400), (2560, 8200), (4096, 8193), (4352, 12300), (5120, 17408), (6144, 12289)]
