@@ -3062,6 +3062,11 @@ struct EnvInt {
 };
 #define env_int(name, fallback) ([]() -> const EnvInt & { static const EnvInt e(name); return e; }().get(fallback))
 
+// Whether a switch that shapes the streaming kernels' launches is set: a matrix that such a switch speaks of goes to them.
+bool streaming_asked_for(bool q4k_row_order) {
+    return env_int("DFLASH_GEMM_WGS", -1) != -1 || env_int("DFLASH_GEMM_WAVES", -1) != -1 || (q4k_row_order && !env_int("DFLASH_Q4K_SLAB", 1));
+}
+
 int32_t launch_q6k(dflash_ctx *ctx, Q6KSet set, const void *x, int32_t x_type, int64_t n_in, int32_t n_rows, hipStream_t st) {
     if (reinterpret_cast<uintptr_t>(x) % (x_type == DFLASH_TYPE_F32 ? 16 : 8))
         return dfl_fail(ctx, DFLASH_ERR_ALIGNMENT, "gemm_fewrow: activations must be 16-byte (f32) / 8-byte (f16) aligned");
@@ -3646,10 +3651,11 @@ int32_t gemm_fewrow_impl(dflash_ctx *ctx, int32_t w_type, const void *w, const v
     } else if (w_type == DFLASH_TYPE_Q4_K) {
         if (tiled && reinterpret_cast<uintptr_t>(w) % 128)
             return dfl_fail(ctx, DFLASH_ERR_ALIGNMENT, "gemm_fewrow: tiled Q4_K weights must be 128-byte aligned");
-        if (direct && dfl_gemm_direct_takes(ctx, w_type, n_in, n_out))
+        if (direct && !streaming_asked_for(!tiled) && dfl_gemm_direct_takes(ctx, w_type, n_in, n_out))
             return dfl_gemm_direct(ctx, tiled ? DFLASH_TYPE_Q4_K_TILED : DFLASH_TYPE_Q4_K, w, x, x_type, y, n_in, n_out, n_rows, st);
         return launch_q4k(ctx, w, x, x_type, y, n_in, n_out, n_rows, st, nullptr, 1, tiled);
-    } else if (w_type == DFLASH_TYPE_Q6_K && direct && env_int("DFLASH_Q6K_STREAM", 1) && dfl_gemm_direct_takes(ctx, w_type, n_in, n_out)) {
+    } else if (w_type == DFLASH_TYPE_Q6_K && direct && env_int("DFLASH_Q6K_STREAM", 1) && !streaming_asked_for(false) &&
+               dfl_gemm_direct_takes(ctx, w_type, n_in, n_out)) {
         return dfl_gemm_direct(ctx, w_type, w, x, x_type, y, n_in, n_out, n_rows, st);
     } else if (w_type == DFLASH_TYPE_Q6_K && env_int("DFLASH_Q6K_STREAM", 1)) {
         const int32_t rc = launch_q6k_stream(ctx, w, x, x_type, y, n_in, n_out, n_rows, st);

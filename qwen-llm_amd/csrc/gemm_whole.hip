@@ -1203,6 +1203,7 @@ namespace {
 //     beyond 16 super-blocks  5120 -> 5120  8.7 : 8.3  10.1 :10.2  10.2 :10.7    Q6_K, 4096 -> 5120  11.5 :13.4 (its registers spill)
 WholePlan rows_direct_plan(const dflash_ctx *ctx, int32_t w_type, int64_t n_in, int64_t n_out) {
     WholePlan p = {DFL_XF_NONE, 0, 0, 0, 0, 0, false};
+    if (!env_int("DFLASH_GEMM_WHOLE", 1)) return p;
     const int kind = w_type == DFLASH_TYPE_Q6_K ? DFL_XF_Q6K : (w_type == DFLASH_TYPE_Q4_K || w_type == DFLASH_TYPE_Q4_K_TILED) ? DFL_XF_Q4K : DFL_XF_NONE;
     const int nb = static_cast<int>(n_in / DFL_QK_K);
     if (kind == DFL_XF_NONE || n_in % DFL_QK_K || nb < 1 || nb > 24 || n_out < 1 || n_out >= (1 << 24)) return p;
@@ -1225,6 +1226,7 @@ struct WidePlan {
 };
 WidePlan rows_wide_plan(const dflash_ctx *ctx, int32_t w_type, int64_t n_in, int64_t n_out) {
     WidePlan p = {0, 0, 0, 0};
+    if (!env_int("DFLASH_GEMM_WHOLE", 1) || !env_int("DFLASH_GEMM_WHOLE_LOOP", 1)) return p;
     const int nb = static_cast<int>(n_in / DFL_QK_K);
     if ((w_type != DFLASH_TYPE_Q4_K && w_type != DFLASH_TYPE_Q4_K_TILED) || n_in % DFL_QK_K || nb < 1 || nb > 24 || n_out < 1 || n_out >= (1 << 24)) return p;
     const int tiles = static_cast<int>((n_out + 15) / 16);

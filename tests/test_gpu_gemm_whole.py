@@ -264,6 +264,49 @@ def test_q6k_of_many_super_blocks_and_few_tiles_streams(ctx, oracle, n_in, n_out
     check(y[:, cols], x.astype(np.float16).astype(np.float64) @ wf.T, f"{n_in}->{n_out}")
 
 
+# (type, tiled order, n_in, n_out): one round of tiles, in both orders of Q4_K, many rounds in both, Q6_K
+SWITCHED = [(dfl.synth.Q4_K, True, 4096, 4096), (dfl.synth.Q4_K, False, 4096, 4096), (dfl.synth.Q4_K, True, 2560, 16384), (dfl.synth.Q4_K, False, 2560, 16384),
+            (dfl.synth.Q6_K, False, 2048, 1024)]
+
+
+def switched_routes(ctx):
+    """For each of SWITCHED the split-K reductions of a call."""
+    routes = []
+    for qtype, tiled, n_in, n_out in SWITCHED:
+        w, w_type, _, w_rows = upload(ctx, qtype, n_in, n_out, seed=1)
+        if not tiled:
+            w, w_type = w_rows, ctx.checked_type(qtype, w_rows)
+        routes.append(reductions(ctx, w, w_type, dev(np.ones((5, n_in), np.float32)), n_in, n_out))
+    return routes
+
+
+_SWITCH_PROBE = """
+import sys
+sys.path.insert(0, "tests")
+import qwen_llm_amd as dfl
+import test_gpu_gemm_whole as t
+print(t.switched_routes(dfl.Context(0)))
+"""
+
+
+@pytest.mark.parametrize("name,value,streamed", [
+    ("DFLASH_GEMM_WHOLE", "0", [1, 1, 1, 1, 1]), ("DFLASH_GEMM_WHOLE_LOOP", "0", [0, 0, 1, 1, 0]), ("DFLASH_GEMM_WGS", "200", [1, 1, 1, 1, 1]),
+    ("DFLASH_GEMM_WAVES", "8", [1, 1, 1, 1, 1]), ("DFLASH_Q4K_SLAB", "0", [0, 1, 0, 1, 0])])
+def test_switches_of_the_streaming_kernels_reach_the_public_operator(ctx, name, value, streamed):
+    """What a switch says of a matrix holds for the public operator's call on it: with the whole-K kernels off, or with a launch geometry
+    of the streaming kernels asked for, the matrix streams.  (The switches are read once per process.)"""
+    import os
+    import subprocess
+    import sys
+
+    assert switched_routes(ctx) == [0, 0, 0, 0, 0]
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    env = dict(os.environ, PYTHONPATH=root + os.pathsep + os.environ.get("PYTHONPATH", ""), **{name: value})
+    r = subprocess.run([sys.executable, "-c", _SWITCH_PROBE], env=env, cwd=root, capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stderr[-2000:]
+    assert r.stdout.split("\n")[-2] == str(streamed)
+
+
 # many rounds of tiles: K of one super-block (sixteen tiles a workgroup), of one and two super-blocks a wave, an odd split of K
 # (17: nine waves, one of them with one super-block), the widest (24); a ragged last tile, a last round that few workgroups have
 WIDE_SHAPES = [(256, 140001), (768, 45000), (1024, 33000), (2048, 16400), (2560, 8200), (4096, 8193), (4352, 12300), (5120, 17408), (6144, 12289)]
