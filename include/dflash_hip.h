@@ -76,8 +76,8 @@ const char *dflash_version(void);
 /* Per-kernel GPU timers: enable_phase_timers / maybe_record (metal_dflash.rs:5181-5190, 5622).
  * While enabled, each call brackets its dominant kernel with events on the call's stream and
  * waits for it, accumulating into a slot: 0 few-row GEMM, 1 verify attention, 2 acceptance,
- * 3 argmax/top-k, 4 split-K reduction of the few-row GEMM.  enable == 2 instead: nothing waits; the single-matrix
- * Q4_K streaming kernel (slot 5) and its reduction (slot 6) are dispatched with start / stop stamps of their own - the
+ * 3 argmax/top-k, 4 split-K reduction of the few-row GEMM.  enable == 2 instead: nothing waits; the kernel of a single-matrix
+ * Q4_K product (slot 5) and the tiled order's reduction, if it has one (slot 6), are dispatched with start / stop stamps of their own - the
  * duration a kernel trace reports, without the dispatch latency an event pair around a launch includes, and with the
  * kernels still running back to back - which dflash_ctx_kernel_timing waits for and adds up when it is called.
  * Changing the mode clears the slots. */

@@ -267,7 +267,7 @@ class Context:
 
     def set_kernel_timing(self, enable):
         """False / 0: off; True / 1: event pairs around the dominant kernels (each timed launch waits); 2: dispatch stamps
-        of the Q4_K streaming kernel and its reduction (slots 5 and 6), read when kernel_timing() is called."""
+        of the kernel of a Q4_K product and its reduction, if any (slots 5 and 6), read when kernel_timing() is called."""
         self._lib.dflash_ctx_set_kernel_timing(self._h, int(enable))
 
     def set_draft_graphs(self, enable: bool):

@@ -63,7 +63,7 @@ enum { DFL_PINNED_BYTES = 8192 };
 
 // Slots of the per-kernel timers.
 enum { DFL_T_GEMM = 0, DFL_T_ATTN = 1, DFL_T_ACCEPT = 2, DFL_T_ARGMAX = 3, DFL_T_REDUCE = 4,
-       // the tiled Q4_K streaming kernel and its reduction by the device's own start / stop stamps of that one dispatch (what a
+       // the kernel of a single Q4_K product and the tiled order's reduction by the device's own start / stop stamps of that one dispatch (what a
        // kernel trace reports as its duration), not by events recorded around the launch (which add the dispatch latency)
        DFL_T_KERNEL_Q4K_TILED = 5, DFL_T_KERNEL_Q4K_REDUCE = 6 };
 

@@ -1303,7 +1303,13 @@ int32_t dfl_gemm_direct(dflash_ctx *ctx, int32_t w_type, const void *w, const vo
     if (lds > 48 * 1024)
         if (const int32_t rc = dfl_raise_lds_limit(ctx, reinterpret_cast<const void *>(fn), lds)) return rc;
     dfl_timed timer(ctx, st, DFL_T_GEMM);
-    whole_launch(fn, p.n_wg, 64 * p.ksplit * p.tl, lds, st, a);
+    hipEvent_t start = nullptr, stop = nullptr;
+    if (!q6) {  // (Q4_K's slot, whichever kernel the matrix takes)
+        const dfl_stamp stamp(ctx, DFL_T_KERNEL_Q4K_TILED);
+        start = stamp.start;
+        stop = stamp.stop;
+    }
+    whole_launch(fn, p.n_wg, 64 * p.ksplit * p.tl, lds, st, a, start, stop);
     DFL_HIP_CHECK(ctx, hipGetLastError());
     return DFLASH_OK;
 }

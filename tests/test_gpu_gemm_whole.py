@@ -280,6 +280,20 @@ def switched_routes(ctx):
     return routes
 
 
+@pytest.mark.parametrize("qtype,tiled,n_in,n_out,stamps", [(*s, [1, 0] if s[0] == dfl.synth.Q4_K else [0, 0]) for s in SWITCHED] +
+                         [(dfl.synth.Q4_K, True, 8192, 528, [1, 1])])
+def test_dispatch_stamps_of_a_q4k_product(ctx, qtype, tiled, n_in, n_out, stamps):
+    """Stamps of single dispatches: the kernel of a Q4_K product whichever it is, and the tiled order's reduction where it has one."""
+    w, w_type, _, w_rows = upload(ctx, qtype, n_in, n_out, seed=1)
+    if not tiled:
+        w, w_type = w_rows, ctx.checked_type(qtype, w_rows)
+    ctx.set_kernel_timing(2)
+    ctx.gemm_fewrow(w, w_type, dev(np.ones((5, n_in), np.float32)), n_in, n_out)
+    got = [ctx.kernel_timing(slot) for slot in (5, 6)]
+    ctx.set_kernel_timing(0)
+    assert [n for _, n in got] == stamps and all((ms > 0) == (n > 0) for ms, n in got)
+
+
 _SWITCH_PROBE = """
 import sys
 sys.path.insert(0, "tests")
