@@ -27,10 +27,12 @@ FLAGS = [
 # Kernels that keep loads in flight across many instructions with hand-placed s_waitcnt (the loads are inline asm, so
 # the compiler does not know their destination registers are still being filled).  If register pressure makes the
 # compiler spill, it can save such a register to scratch BEFORE its data has arrived and restore the stale value
-# later: silently wrong activations or weights.  The build therefore refuses any of them that uses scratch at all.
+# later: silently wrong activations or weights.  The build therefore refuses any of them that uses scratch at all; so it does where
+# the loads go to LDS and only the waits are placed by hand (a spill's own loads and stores would be counted among them).
 NO_SCRATCH_BY_FILE = {
     "gemm_fewrow.hip": ("gemm_q4k_stream_kernel", "gemm_q4k_slab_kernel", "gemm_q4k_tiled_kernel", "gemm_q4k_experts_kernel",
-                        "gemm_q6k_stream_kernel"),
+                        "gemm_q4k_few_slots_kernel", "gemm_q6k_stream_kernel"),
+    "gemm_whole.hip": ("gemm_q6t_loop_kernel", "gemm_q4k_wide_kernel"),
     "attn_verify.hip": ("attn_split_kernel", "attn_rows_kernel", "attn_rows_pair_kernel"),
     "gemm_rows.hip": ("gemm_rows_kernel",),
 }
@@ -41,7 +43,8 @@ NO_SCRATCH_KERNELS = tuple(k for kernels in NO_SCRATCH_BY_FILE.values() for k in
 INSPECTED_SPILLS = {}
 # Files whose generated code is checked for a register that is touched while a load still fills it (inflight.py): reads from
 # LDS in all of their kernels, loads from memory in the kernels named (the others count theirs at run time).
-CHECKED_CODE = {"gemm_rows.hip": ("gemm_rows_kernel",), "attn_verify.hip": ("attn_rows_pair_kernel",), "gemm_fewrow.hip": ()}
+CHECKED_CODE = {"gemm_rows.hip": ("gemm_rows_kernel",), "attn_verify.hip": ("attn_rows_pair_kernel",), "gemm_fewrow.hip": ("gemm_q4k_few_slots_kernel",),
+                "gemm_whole.hip": ("gemm_q6t_loop_kernel",)}
 RESOURCE_FLAG = "-Rpass-analysis=kernel-resource-usage"
 REMARK = r"remark: (?:\S+:\d+:\d+: )?\s*"  # (the place stands ahead of the word, or behind it where the assembly is kept)
 

@@ -57,6 +57,28 @@ def test_a_guarded_kernel_missing_from_the_remarks_fails_the_guard():
     assert b.check_no_scratch("nothing of the kind\n", expect=("gemm_q4k_tiled_kernel",)) != []
 
 
+def test_every_kernel_that_waits_for_memory_by_hand_is_guarded():
+    """A kernel with an s_waitcnt of its own on vector memory, or a call of a function that waits, is named in the build's list, and a
+    file that such a kernel lives in has its generated code checked."""
+    import re
+
+    b = _build_module()
+    found = set()
+    for src in b.sources():
+        with open(src) as f:
+            text = re.sub(r"//[^\n]*", "", f.read())
+        name = os.path.basename(src)
+        for at in [m.end() for m in re.finditer("__global__", text)]:
+            kernel = re.compile(r"(\w+_kernel)\s*\(").search(text, at)
+            body = text[kernel.end():text.index("\n}\n", at)]
+            # (a wait for LDS alone, or for everything, is none of this)
+            if re.search(r"__builtin_amdgcn_s_waitcnt\((?!kWaitLds\)|0\)|0xC07F\))|\b\w*wait_(?:vm\w*|groups)\(|\b(?:wide|attn)_wait\(", body):
+                found.add(kernel.group(1))
+                assert kernel.group(1) in b.NO_SCRATCH_BY_FILE.get(name, ()), f"{name}: {kernel.group(1)}"
+                assert name in b.CHECKED_CODE, name
+    assert len(found) >= 8
+
+
 def test_inspected_exceptions_hold_only_at_their_recorded_counts():
     b = _build_module()
     b.INSPECTED_SPILLS = {"gemm_q6k_stream_kernelILi16EfE": 13}
