@@ -28,6 +28,16 @@ def gemm_fast(ctx, w, qtype, x, n_in, n_out):
     return ctx.gemm_fewrow(w, ctx.checked_type(qtype, w), x, n_in, n_out)
 
 
+def reductions(ctx, w, w_type, x, n_in, n_out):
+    """Split-K reductions launched by one call on a checked tensor: one on the streaming kernels, none in one launch."""
+    tag = w_type if w_type == dfl.TYPE_Q4_K_TILED else ctx.checked_type(w_type, w)
+    ctx.set_kernel_timing(1)
+    ctx.gemm_fewrow(w, tag, x, n_in, n_out)
+    n = ctx.kernel_timing(4)[1]
+    ctx.set_kernel_timing(0)
+    return n
+
+
 @pytest.mark.parametrize("qtype", QTYPES)
 @pytest.mark.parametrize("kind", ["random", "extreme", "quantised"])
 def test_dequant_bit_exact(ctx, oracle, qtype, kind):
@@ -143,23 +153,26 @@ def test_gemm_deterministic_and_linear(ctx):
 
 
 @pytest.mark.parametrize("qtype", [dfl.synth.Q4_K, dfl.synth.Q6_K])
-@pytest.mark.parametrize("n_in,n_out", [(2048, 5120), (4096, 2048), (2048, 12288), (6144, 2048)])
+@pytest.mark.parametrize("n_in,n_out", [(2048, 5120), (4096, 2048), (2048, 12288), (6144, 2048), (6656, 2048), (7168, 5003)])
 def test_gemm_small_split_k_repeats(ctx, oracle, qtype, n_in, n_out, canaries):
-    """Products of a few MB (the projections of a decoder layer) are split over K across workgroups, their
-    partial tiles living in a scratch buffer that every launch shares.  Forty launches in a row, alternating
-    with another shape: every result bit-identical to the first and within the GEMM bar of the f64 reference."""
+    """Products of a few MB (the projections of a decoder layer), of one launch or split over K across workgroups, their
+    partial tiles then living in a scratch buffer that every launch shares.  Forty launches in a row, alternating
+    with a shape that is split (the longest K here are, too): every result bit-identical to the first and within the GEMM bar of the f64
+    reference."""
     import torch
 
     w = dev(dfl.synth.random_weight(qtype, n_out, n_in, seed=5))
-    w2 = dev(dfl.synth.random_weight(qtype, 1024, 2048, seed=6))
+    w2 = dev(dfl.synth.random_weight(qtype, 272, 8192, seed=6))
     g = torch.Generator(device="cuda").manual_seed(2)
     x = torch.randn((16, n_in), device="cuda", generator=g, dtype=torch.float32)
-    x2 = torch.randn((16, 2048), device="cuda", generator=g, dtype=torch.float32)
+    x2 = torch.randn((16, 8192), device="cuda", generator=g, dtype=torch.float32)
+    assert reductions(ctx, w2, qtype, x2, 8192, 272) == 1
+    assert n_in <= 6144 or reductions(ctx, w, qtype, x, n_in, n_out) == 1
     first = gemm_fast(ctx, w, qtype, x, n_in, n_out).clone()
-    other = gemm_fast(ctx, w2, qtype, x2, 2048, 1024).clone()
+    other = gemm_fast(ctx, w2, qtype, x2, 8192, 272).clone()
     for _ in range(20):
         assert torch.equal(gemm_fast(ctx, w, qtype, x, n_in, n_out), first)
-        assert torch.equal(gemm_fast(ctx, w2, qtype, x2, 2048, 1024), other)
+        assert torch.equal(gemm_fast(ctx, w2, qtype, x2, 8192, 272), other)
     ref = f64_reference(oracle, qtype, w.cpu().numpy(), x.cpu().numpy(), n_in, n_out)
     check_gemm(first.cpu().numpy(), ref, f"split-K {n_in}x{n_out}")
 
@@ -201,7 +214,8 @@ def test_gemm_guards(ctx):
 
 TILED_SHAPES = [(256, 16, 16), (256, 250, 3), (768, 257, 16), (1024, 4096, 7), (1280, 1000, 16), (2048, 5120, 1),
                 (5120, 6144, 16), (5120, 17408, 16), (17408, 5120, 16),
-                (2048, 50000, 16), (8192, 16384, 5)]  # the last two: ranges longer than six stages (the per-stage-barrier kernel)
+                (2048, 50000, 16),   # the looping kernel
+                (8192, 16384, 5)]    # ranges longer than six stages (the per-stage-barrier kernel)
 
 
 @pytest.mark.parametrize("n_in,n_out,n_rows", TILED_SHAPES)
@@ -226,12 +240,13 @@ def test_gemm_q4k_tiled_order_is_bit_identical(ctx, n_in, n_out, n_rows, x_dtype
     assert torch.isnan(buf[:guard]).all() and torch.isnan(buf[-guard:]).all()
 
 
-@pytest.mark.parametrize("n_in,n_out", [(256, 16), (1280, 1000), (5120, 6144), (17408, 512), (2048, 50000)])
+@pytest.mark.parametrize("n_in,n_out", [(256, 16), (1280, 1000), (5120, 6144), (17408, 512), (2048, 50000), (8192, 16384)])
 @pytest.mark.parametrize("x_dtype", [np.float32, np.float16])
 def test_gemm_q4k_sums_past_f16(ctx, oracle, n_in, n_out, x_dtype, canaries):
     """Rows whose sub-block sums lie on both sides of 65520, where a sum no longer rounds to an f16, and at the most that
-    f16 activations can reach (32 x 60000), beside ordinary rows: the slab, the tiled and the streaming kernel (2048 ->
-    50000) against the f64 product, row order and tiled order bit for bit, and an ordinary row with the bits it has alone."""
+    f16 activations can reach (32 x 60000), beside ordinary rows: the whole-K, the slab, the tiled, the looping (2048 -> 50000) and the
+    streaming kernel (8192 -> 16384) against the f64 product, row order and tiled order bit for bit, and an ordinary row with the
+    bits it has alone."""
     import torch
     rng = np.random.default_rng(n_in + n_out)
     w = dfl.synth.random_blocks(dfl.synth.Q4_K, n_out * n_in // 256, n_in + n_out)
@@ -248,6 +263,49 @@ def test_gemm_q4k_sums_past_f16(ctx, oracle, n_in, n_out, x_dtype, canaries):
     ref = f64_reference(oracle, dfl.synth.Q4_K, w.reshape(n_out, -1)[cols], x.astype(np.float32), n_in, len(cols))
     for r in range(len(level)):
         check_gemm(y[r:r + 1, cols].cpu().numpy(), ref[r:r + 1], f"{n_in}x{n_out} row around {level[r]}")
+
+
+# K of more than 24 super-blocks, or of 17 to 24 between one round of tiles and three: few tiles, one and several tile groups with a ragged last one,
+# ranges that wrap over tile groups, ranges longer than six stages
+STREAMED_SHAPES = [(6656, 5), (6656, 250), (7168, 1003), (17408, 777), (5120, 4109), (6656, 20003)]
+
+
+@pytest.mark.parametrize("n_in,n_out", STREAMED_SHAPES)
+@pytest.mark.parametrize("n_rows,x_dtype", [(1, "f32"), (3, "f16"), (5, "f32"), (16, "f16"), (16, "f32")])
+def test_gemm_q4k_streamed_and_ragged(ctx, oracle, n_in, n_out, n_rows, x_dtype, canaries):
+    """Q4_K products that no single launch takes: the slab, tiled and per-stage-barrier kernels, their split over workgroups and the
+    reduction of the partial tiles, at ragged edges, in both orders of the weights (the same bits), against f64."""
+    import torch
+
+    w = dfl.synth.random_blocks(dfl.synth.Q4_K, n_out * n_in // 256, n_in + n_out)
+    x = np.random.default_rng(n_rows + n_out).standard_normal((n_rows, n_in)).astype(np.float32 if x_dtype == "f32" else np.float16)
+    wd, xd = dev(w), dev(x)
+    wt = ctx.repack_q4k_tiled(wd, n_in, n_out)
+    assert reductions(ctx, wd, dfl.TYPE_Q4_K, xd, n_in, n_out) == reductions(ctx, wt, dfl.TYPE_Q4_K_TILED, xd, n_in, n_out) == 1
+    y = gemm_fast(ctx, wd, dfl.TYPE_Q4_K, xd, n_in, n_out)
+    yt = ctx.gemm_fewrow(wt, dfl.TYPE_Q4_K_TILED, xd, n_in, n_out)
+    canaries.check()
+    assert torch.equal(y.view(torch.int32), yt.view(torch.int32))
+    cols = np.unique(np.concatenate([np.arange(min(n_out, 300)), np.random.default_rng(1).integers(0, n_out, 300), np.arange(max(0, n_out - 300), n_out)]))
+    ref = f64_reference(oracle, dfl.synth.Q4_K, w.reshape(n_out, -1)[cols], x.astype(np.float32), n_in, len(cols))
+    check_gemm(y[:, torch.from_numpy(cols).cuda()].cpu().numpy(), ref, f"streamed {n_in}x{n_out}x{n_rows} {x_dtype}")
+
+
+@pytest.mark.parametrize("n_in,n_out", [(6656, 5), (6656, 250), (7168, 1003), (2048, 12305)])
+@pytest.mark.parametrize("n_rows,x_dtype", [(1, "f32"), (5, "f16"), (16, "f32")])
+def test_gemm_q6k_streamed_and_ragged(ctx, oracle, n_in, n_out, n_rows, x_dtype, canaries):
+    """The same of Q6_K: K of more than 24 super-blocks, and many rounds of tiles."""
+    import torch
+
+    w = dfl.synth.random_blocks(dfl.synth.Q6_K, n_out * n_in // 256, n_in + n_out)
+    x = np.random.default_rng(n_rows + n_out).standard_normal((n_rows, n_in)).astype(np.float32 if x_dtype == "f32" else np.float16)
+    wd, xd = dev(w), dev(x)
+    assert reductions(ctx, wd, dfl.TYPE_Q6_K, xd, n_in, n_out) == 1
+    y = gemm_fast(ctx, wd, dfl.TYPE_Q6_K, xd, n_in, n_out)
+    canaries.check()
+    cols = np.unique(np.concatenate([np.arange(min(n_out, 300)), np.arange(max(0, n_out - 300), n_out)]))
+    ref = f64_reference(oracle, dfl.synth.Q6_K, w.reshape(n_out, -1)[cols], x.astype(np.float32), n_in, len(cols))
+    check_gemm(y[:, torch.from_numpy(cols).cuda()].cpu().numpy(), ref, f"streamed q6k {n_in}x{n_out}x{n_rows} {x_dtype}")
 
 
 def test_q4k_tiled_repack_layout(ctx):

@@ -1,7 +1,7 @@
 """GPU parity of the whole-K few-row GEMM over activations in fragment order (dflash_pack_xf,
 dflash_gemm_fewrow_xf): against float64 of the oracle's dequant (<= 1e-2 relative, f32 accumulation), and
-against dflash_gemm_fewrow on the same weights (same operands rounded the same way: the two may differ only in
-the order of the f32 sums)."""
+against dflash_gemm_fewrow on the same weights, which streams the larger ones (same operands rounded the same way: the two may
+differ only in the order of the f32 sums) and takes the same kernels, with the rows brought in by themselves, for the others."""
 import numpy as np
 import pytest
 
@@ -35,6 +35,8 @@ def check(y, ref, label):
 # (n_in, n_out, rows): one stage per wave (n_in <= 4096), two (up to 8192), ragged tile and row counts, two tiles per wave
 SHAPES = [(256, 16, 16), (256, 40, 1), (1024, 272, 16), (2048, 5120, 16), (2048, 1000, 7), (4096, 2048, 16), (6144, 2048, 16),
           (5120, 6144, 16), (2048, 12288, 16), (3072, 100, 3), (8192, 48, 16)]
+# of those and of these the public operator streams what has more than 24 super-blocks (and what is 17 to 24 in more than one round of tiles)
+STREAMED_SHAPES = [(6656, 1000, 16), (6656, 17, 3), (7168, 2047, 5), (8192, 4096, 16)]
 
 
 def upload(ctx, qtype, n_in, n_out, seed, extreme=False):
@@ -49,8 +51,17 @@ def upload(ctx, qtype, n_in, n_out, seed, extreme=False):
     return wd, ctx.checked_type(dfl.TYPE_Q6_K, wd), blocks, wd
 
 
+def reductions(ctx, w, w_type, x, n_in, n_out):
+    """Split-K reductions launched by one call of the public operator: one on the streaming kernels, none in one launch."""
+    ctx.set_kernel_timing(1)
+    ctx.gemm_fewrow(w, w_type, x, n_in, n_out)
+    n = ctx.kernel_timing(4)[1]
+    ctx.set_kernel_timing(0)
+    return n
+
+
 @pytest.mark.parametrize("qtype", [dfl.synth.Q4_K, dfl.synth.Q6_K])
-@pytest.mark.parametrize("n_in,n_out,rows", SHAPES)
+@pytest.mark.parametrize("n_in,n_out,rows", SHAPES + STREAMED_SHAPES)
 @pytest.mark.parametrize("x_dtype", [np.float32, np.float16])
 def test_whole_k_gemm_matches_oracle_and_streaming_kernels(ctx, oracle, canaries, qtype, n_in, n_out, rows, x_dtype):
     w, w_type, blocks, w_rows = upload(ctx, qtype, n_in, n_out, seed=n_in + n_out)
@@ -64,7 +75,8 @@ def test_whole_k_gemm_matches_oracle_and_streaming_kernels(ctx, oracle, canaries
     wf = oracle.dequant(qtype, blocks, n_in * n_out).reshape(n_out, n_in).astype(np.float64)
     ref = x.astype(np.float16).astype(np.float64) @ wf.T  # every few-row kernel rounds its activations to f16
     check(y, ref, f"{n_in}->{n_out} x{rows}")
-    # the streaming kernels on the same operands: same products, other order of the f32 sums
+    # the public operator on the same operands, for the longer K the streaming kernels: same products, other order of the f32 sums
+    assert n_in <= 6144 or reductions(ctx, w, w_type, xd, n_in, n_out) == 1
     y2 = ctx.gemm_fewrow(w, w_type, xd, n_in, n_out).cpu().numpy()
     assert np.max(np.abs(y - y2)) <= 2e-5 * max(np.max(np.abs(ref)), 1.0) + 1e-4 * np.sqrt(np.mean(ref ** 2))
 
@@ -240,15 +252,6 @@ def test_rows_in_row_order_give_the_bits_of_packed_rows(ctx, oracle, canaries, q
     wf = oracle.dequant(qtype, np.ascontiguousarray(blocks[cols]), len(cols) * n_in).reshape(len(cols), n_in).astype(np.float64)
     ref = x.half().cpu().numpy().astype(np.float64) @ wf.T
     check(y[:, torch.from_numpy(cols).cuda()].cpu().numpy(), ref, f"{n_in}->{n_out} x{rows}")
-
-
-def reductions(ctx, w, w_type, x, n_in, n_out):
-    """Split-K reductions launched by one call of the public operator: one on the streaming kernels, none in one launch."""
-    ctx.set_kernel_timing(1)
-    ctx.gemm_fewrow(w, w_type, x, n_in, n_out)
-    n = ctx.kernel_timing(4)[1]
-    ctx.set_kernel_timing(0)
-    return n
 
 
 @pytest.mark.parametrize("n_in,n_out,streamed", [(5632, 512, 0), (5888, 512, 1), (6144, 1024, 1), (6144, 2032, 1), (6144, 2033, 0), (6144, 4096, 0),

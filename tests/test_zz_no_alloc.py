@@ -28,6 +28,12 @@ def _run_pair(ctx, L, qtype, n_in, n_out, n_rows, seed, x_f16):
     assert rc == 0, L.dflash_gemm_fewrow_noalloc_error().decode()
     torch.cuda.synchronize()
     assert torch.equal(got.view(torch.int32), want.view(torch.int32)), (qtype, n_in, n_out, n_rows)
+    # what goes through the scratch array, by the context's own count of reductions
+    ctx.set_kernel_timing(1)
+    ctx.gemm_fewrow(w, qtype, x, n_in, n_out)
+    split = ctx.kernel_timing(4)[1]
+    ctx.set_kernel_timing(0)
+    return split
 
 
 def test_noalloc_gemm_equals_context_gemm_twice_in_a_row():
@@ -53,7 +59,11 @@ def test_noalloc_gemm_equals_context_gemm_twice_in_a_row():
         torch.cuda.synchronize()
         assert torch.cuda.mem_get_info(0)[0] == free_before, "the no-allocation entry point allocated device memory"
         # split-K shapes (partial tiles go through the scratch array), larger then smaller, for both streaming kernels
-        _run_pair(ctx, L, dfl.TYPE_Q4_K, 5120, 6144, 16, 1, True)
+        assert _run_pair(ctx, L, dfl.TYPE_Q4_K, 5120, 6144, 16, 1, True) == 1
+        assert _run_pair(ctx, L, dfl.TYPE_Q4_K, 8192, 272, 5, 6, False) == 1
+        assert _run_pair(ctx, L, dfl.TYPE_Q6_K, 2048, 12304, 16, 7, False) == 1
+        assert _run_pair(ctx, L, dfl.TYPE_Q6_K, 8192, 48, 1, 8, True) == 1
+        # products of one launch, without scratch
         _run_pair(ctx, L, dfl.TYPE_Q4_K, 1024, 272, 5, 2, False)
         _run_pair(ctx, L, dfl.TYPE_Q6_K, 2048, 4096, 16, 3, False)
         _run_pair(ctx, L, dfl.TYPE_Q6_K, 512, 48, 1, 4, True)
