@@ -1554,7 +1554,6 @@ __device__ __forceinline__ void q4k_stage_weights(const u32x4_t *blk, int g, uin
         b.hi[t] = unpack_scale<true>(qw[2 * t], qw[2 * t + 1], s2h, c2h, magic.hi);
     }
 }
-// q4k_experts_compute's nine products, in its order
 __device__ __forceinline__ uint32_t q4k_lds_at(const void *p) {
     return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const void *)(p)));
 }
@@ -1567,7 +1566,7 @@ __device__ __forceinline__ void q4k_stage_activations(const uint8_t *stage, int 
 #pragma unroll
     for (int t = 0; t < 8; t++) x.af[t] = *reinterpret_cast<const half8_t *>(stage + t * kTiledFragStride + lane * 16);
 }
-// (kNext: each activation fragment is replaced by the next stage's once its product has been asked for; the compiler would read
+// q4k_experts_compute's nine products, in its order (kNext: each activation fragment is replaced by the next stage's once its product has been asked for; the compiler would read
 // those one product ahead of their use, a quarter of the way there)
 template <bool kNext>
 __device__ __forceinline__ void q4k_stage_products(const Q4KStageW &b, Q4KStageX &x, const uint8_t *next, int lane, float4_t &acc) {
@@ -1633,8 +1632,9 @@ __device__ __forceinline__ void q4k_chain_pass(uint32_t acc_at, uint32_t turn_at
     *reinterpret_cast<volatile __attribute__((address_space(3))) int32_t *>(turn_at) = turn;
 }
 
-// kFew: a routed launch of one or two units a workgroup (the host's bound on the list says so) and K of two chunks: one row's nine
-// matrices of 768 x 2048 are 432 units on 256 workgroups.  The chain of a unit's eight stages, gate and up, is what such a launch
+// kFew: a routed launch of one or two units a workgroup (the host's bound on the list says so) and K of exactly two chunks, 2048, the two
+// stages of each of four waves: one row's nine matrices of 768 x 2048 are 432 units on 256 workgroups.  (Two rows' seventeen are 816
+// and keep a tile a wave; mixtures of fewer or smaller experts get here with up to three rows.)  The chain of a unit's eight stages, gate and up, is what such a launch
 // would wait for: a stage is 0.4 us of LDS reads, unpacking and nine products for a wave that has its SIMD to itself, and only
 // the products, 0.15, have to follow one another.  So a tile has four waves (wave 8 u + 4 half + part, two stages each), which bring
 // in and unpack their stages at the same time; the accumulator goes through them in the order of the stages (in LDS,
@@ -2667,10 +2667,9 @@ __global__ void __launch_bounds__(64 * kMaxSplit)
 }
 
 // The same product for few tiles, over more of the chip: a workgroup has four of the block's rows and OUT weight rows, and the next
-// chunk's bytes are on their way while this one is multiplied.  (The kernel above is bound by what one of its few workgroups
-// takes in, all sixteen rows and sixteen weight rows, a chunk at a time with nothing under way in between: 18 us for 16 rows 8192 ->
-// 1024, 12 here.)  Sixteen waves and the
-// chunks cut K as above, so a product has the bits it has there.
+// chunk's bytes are on their way while this one is multiplied.  Sixteen waves and the chunks cut K as above, so a product has
+// the bits it has there.  (The kernel above is bound by what one of its few workgroups takes in, all sixteen rows and sixteen
+// weight rows, a chunk at a time with nothing under way in between: 18 us for 16 rows 8192 -> 1024, 12 here.)
 constexpr int kQ8SplitRows = 4;
 template <typename XT, int OUT>
 __global__ void __launch_bounds__(64 * kMaxSplit)
@@ -3167,7 +3166,8 @@ int32_t launch_q4k(dflash_ctx *ctx, const void *w, const void *x, int32_t x_type
         const uint8_t *wb = static_cast<const uint8_t *>(w);
         const int no = static_cast<int>(n_out);
         // Rows of their own per slot, K of at most four stages and so few matrices that every unit of 16 / stages tiles has a workgroup of
-        // its own: a stage a wave (one row of the 35B-A3B-shaped stack 4.8 us a launch, against 7.1 with eight whole tiles a workgroup).
+        // its own: a stage a wave (one row of the 35B-A3B-shaped stack, 9 matrices of 26 units, 4.8 us a launch, against 7.1 with eight whole tiles a
+        // workgroup; two rows of it, 17 x 26, are more units than workgroups).
         if (per_slot_x && x_type == DFLASH_TYPE_F16 && !batch->y_f16 && !batch->pair && nb <= 4 && n_out % 16 == 0 && n_rows * nb * 32 <= 1024) {
             const int tpu = kSlabWaves / nb, upm = (tiles + tpu - 1) / tpu;
             if (static_cast<int64_t>(max_slots) * upm <= n_wg) {
@@ -3183,7 +3183,7 @@ int32_t launch_q4k(dflash_ctx *ctx, const void *w, const void *x, int32_t x_type
         }
         // Sixteen tiles a unit, one a wave, or eight where the longest list still gives no workgroup a second unit: a CU takes in
         // about 30 KB per microsecond, and a short list in large units leaves most of them without any (one row's nine matrices of
-        // 2048 x 768: 72 units of 110 KB 9.3 us, 144 of 55 KB 7.1).
+        // 2048 x 768: 72 units of 110 KB 9.3 us, 144 of 55 KB 7.1; two rows' are 17 x 16, more than a workgroup a CU, and stay at sixteen).
         int group = 16;
         if (static_cast<int64_t>(max_slots) * ((tiles + 7) / 8) <= n_wg) group = 8;
         const int upm = per_slot_x ? (tiles + group - 1) / group : tiles;  // units per matrix

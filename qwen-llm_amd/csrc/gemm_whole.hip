@@ -832,7 +832,7 @@ __global__ void __launch_bounds__(1024) gemm_q6t_loop_kernel(DFL_WHOLE_PARAMS) {
     }
 }
 
-// The public operator on a Q4_K matrix of many rounds of tiles, K of at most 32 super-blocks, rows in row order: one workgroup per
+// The public operator on a Q4_K matrix of many rounds of tiles, K of at most 24 super-blocks, rows in row order: one workgroup per
 // CU walks units of one tile, its waves share K.  A wave keeps the fragments and the sub-block sums of its one or two
 // super-blocks in registers for every tile, so a tile costs it nothing but weights, which it streams through a private
 // ring of LDS slots (a slot: one super-block of the tile, 144 pieces of 16 bytes, three direct-to-LDS loads); the slices' partial tiles
@@ -842,8 +842,10 @@ __global__ void __launch_bounds__(1024) gemm_q6t_loop_kernel(DFL_WHOLE_PARAMS) {
 // us a call, weights cold, streaming kernel and reduction : this one, 1 row f32 / 16 rows f16 / 16 rows f32:
 //   tiled Q4_K  5120 -> 17408 17.9 :17.0 20.2 :17.2 20.5 :19.4   2560 -> 16384 12.2 : 9.2 13.3 :10.2 13.4 :10.8   2048 -> 40000 17.0 :13.0 20.3 :14.4 20.3 :15.9
 //   row order   5120 -> 17408 18.1 :17.7 19.8 :18.2 19.9 :20.3   2560 -> 16384 12.6 : 9.4 14.4 :10.1 14.4 :11.3   2048 -> 40000 17.0 :13.5 19.2 :15.1 19.2 :16.6
+// Sixteen f32 rows are twice the bytes to bring in ahead of the first product, and against weights in row order, two super-blocks a wave,
+// that is all that the launch saves, or 2 % more; the line looks at the matrix alone, so that a row has its bits whatever its type and company.
 // (no stage ahead of the rows, or four: 18.3 and 18.5 for 16 f16 rows, 5120 -> 17408).
-// `landed` is an s_waitcnt vmcnt of the loads behind: they return in order, and a Y store among them only makes it stricter.
+// A stage has landed when no more loads are under way than were issued behind it: they return in order, and a Y store among them only makes it stricter.
 constexpr int kWideSlot = 16 * DFL_Q4_K_BYTES;  // 2304 bytes
 constexpr int kWideSlots = 6;                        // at most (the counts below)
 __device__ __forceinline__ void wide_wait(int ahead) {  // at most `ahead` stages (three loads each) still under way, ahead uniform
