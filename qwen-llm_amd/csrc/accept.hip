@@ -147,8 +147,9 @@ __device__ __forceinline__ void best_of_chunk(const float *__restrict__ x, int v
 // than that (k = 20: about a hundred).  What is below it is ranked by counting the candidates below each, and the candidate of
 // rank r < k is output r.  Keys are distinct (the token id is in the low bits), so ranks are too.  (The k-th of the threads' best keys
 // digit by digit in every chunk was 4.7 of its workgroup's 11.3 us, the collecting of what it bounds another 1.8.)
-// Where more than kSelThreads tokens are below the bound (a vocabulary of which a mask has left a few; logits ordered by thread, or
-// alike), the k-th best of the threads' best keys is what bounds them, and with the winners no more than the kSelPer tokens of k threads.
+// Where many tokens are below the bound (a vocabulary of which a mask has left a few; logits ordered by token, or alike), the
+// k-th best of the threads' best keys is what bounds them, and with the winners no more than the kSelPer tokens of k threads.  From 512 on the
+// ranking costs more than that search (logits that fall from token to token, k = 20, 960 below the bound: a call of 62 us, now 41).
 // (16 rows of 151936, k = 20, one token in a thousand left: 14.8 us, 7.3 unmasked; a digit search over all of the tokens: about 110.)
 __device__ __forceinline__ void select_chunk_body(const float *__restrict__ x, int vocab, int k, uint64_t *__restrict__ out,
                                                   bool nan_is_candidate) {
@@ -210,7 +211,7 @@ __device__ __forceinline__ void select_chunk_body(const float *__restrict__ x, i
         collect([&](int j) { return d[j] <= bound; });
     __syncthreads();
     int n_cand = cnt[0];
-    if (n_cand > kSelThreads) {
+    if (n_cand > kSelThreads / 2) {
         uint64_t keys[kSelPer], first = kNoKey;
 #pragma unroll
         for (int j = 0; j < kSelPer; j++) {

@@ -347,11 +347,11 @@ def test_selection_at_chunk_boundaries(ctx, oracle, vocab, top_k):
     assert len(lengths) > 1
 
 
-@pytest.mark.parametrize("kind", ["alike", "by_thread", "short_chunk", "infinite_drafts", "long_lists", "late_nan"])
+@pytest.mark.parametrize("kind", ["alike", "by_thread", "descending", "short_chunk", "infinite_drafts", "long_lists", "late_nan"])
 @pytest.mark.parametrize("top_k", [1, 17, 64])
 def test_selection_and_decision_off_their_short_paths(ctx, oracle, kind, top_k):
     """Logits whose selection needs more than a bound per wave (all alike; the best tokens of a 16384-token chunk all with the same few
-    threads), a last chunk of fewer tokens than threads, draft logits that are infinite, proposals and stop ids beyond a wave's 64
+    threads, or all of a chunk's first), a last chunk of fewer tokens than threads, draft logits that are infinite, proposals and stop ids beyond a wave's 64
     lanes, a NaN in a later chunk of a target or a draft row: decisions, errors and sampler state equal the oracle's."""
     vocab, n, T = 2 * 16384 + 700, 4, 0.7
     rng = np.random.default_rng(top_k)
@@ -361,6 +361,8 @@ def test_selection_and_decision_off_their_short_paths(ctx, oracle, kind, top_k):
         tl[:2] = 0.5
     elif kind == "by_thread":
         tl[:] = (-thread + turn * 1e-3)[None, :] * 0.25
+    elif kind == "descending":
+        tl[:] = np.arange(vocab)[None, :] * -1e-3 * np.array([1, -1, 1, -1])[:, None]
     elif kind == "short_chunk":
         tl[:, 2 * 16384:] += 8.0
     dl = (tl[: n - 1] + rng.standard_normal((n - 1, vocab)) * 0.5).astype(np.float32)
@@ -414,17 +416,19 @@ def test_masked_vocabularies(ctx, oracle, low, top_k):
                 assert_same(oracle, *r)
 
 
-@pytest.mark.parametrize("top_k", [20, 200])
-def test_a_masked_vocabulary_takes_no_search_over_all_of_its_tokens(ctx, top_k):
-    """A block's decision on 151936 tokens of which a mask has left one in a thousand, against the same block unmasked: at most twice as
-    long.  (A digit search over all tokens that are alike, thousands of them on one counter, is four times as long.)"""
+@pytest.mark.parametrize("kind,top_k,limit", [("masked", 20, 2.0), ("masked", 200, 2.0), ("falling", 20, 1.5)])
+def test_logits_off_the_short_path_take_no_search_over_all_of_the_tokens(ctx, kind, top_k, limit):
+    """A block's decision on 151936 tokens of which a mask has left one in a thousand, and on logits that fall from token to token, against the
+    same block of random logits, by the call's time: 1.35 and 1.2 times as long.  (A digit search over all tokens that are alike,
+    thousands of them on one counter, is four times as long, the ranking of a thousand tokens 1.8 times.)"""
     import torch
 
     vocab, n = 151936, 16
     rng = np.random.default_rng(top_k)
     plain = (rng.standard_normal((n, vocab)) * 3.0).astype(np.float32)
+    other = masked_rows(rng, n, vocab, -np.inf, 0.001) if kind == "masked" else np.tile(np.arange(vocab, dtype=np.float32) * np.float32(-1e-3), (n, 1))
     times = []
-    for rows in (plain, masked_rows(rng, n, vocab, -np.inf, 0.001)):
+    for rows in (plain, other):
         t = dev(rows)
         toks = [int(rows[0].argmax())] + [int(rows[r].argmax()) for r in range(n - 1)]
         s = dfl.Sampler(temperature=0.7, top_k=top_k, seed=1)
@@ -436,7 +440,7 @@ def test_a_masked_vocabulary_takes_no_search_over_all_of_its_tokens(ctx, top_k):
                 ctx.decide_dflash_accept_prefix(toks, t, vocab, None, s.clone(), 100, [])
             best = min(best, time.perf_counter() - t0)
         times.append(best)
-    assert times[1] <= 2 * times[0], [f"{x / 20 * 1e6:.1f} us" for x in times]
+    assert times[1] <= limit * times[0], [f"{x / 20 * 1e6:.1f} us" for x in times]
 
 
 @pytest.mark.parametrize("n_tiles", [255, 256, 257, 513])
