@@ -35,6 +35,7 @@ NO_SCRATCH_BY_FILE = {
     "gemm_whole.hip": ("gemm_q6t_loop_kernel", "gemm_q4k_wide_kernel"),
     "attn_verify.hip": ("attn_split_kernel", "attn_rows_kernel", "attn_rows_pair_kernel"),
     "gemm_rows.hip": ("gemm_rows_kernel",),
+    "gemm_dense.hip": ("gemm_q4k_dense_pair_kernel",),
 }
 NO_SCRATCH_KERNELS = tuple(k for kernels in NO_SCRATCH_BY_FILE.values() for k in kernels)
 # Inspected exceptions, by mangled-name fragment -> spilled VGPRs: none at present.  An entry belongs here only after
@@ -44,7 +45,7 @@ INSPECTED_SPILLS = {}
 # Files whose generated code is checked for a register that is touched while a load still fills it (inflight.py): reads from
 # LDS in all of their kernels, loads from memory in the kernels named (the others count theirs at run time).
 CHECKED_CODE = {"gemm_rows.hip": ("gemm_rows_kernel",), "attn_verify.hip": ("attn_rows_pair_kernel",), "gemm_fewrow.hip": ("gemm_q4k_few_slots_kernel",),
-                "gemm_whole.hip": ("gemm_q6t_loop_kernel",)}
+                "gemm_whole.hip": ("gemm_q6t_loop_kernel",), "gemm_dense.hip": ()}
 RESOURCE_FLAG = "-Rpass-analysis=kernel-resource-usage"
 REMARK = r"remark: (?:\S+:\d+:\d+: )?\s*"  # (the place stands ahead of the word, or behind it where the assembly is kept)
 

@@ -225,7 +225,7 @@ __device__ static inline float dfl_wave_max(float v) {
 // Lanes (2 p, 2 p + 1) of a wave hold values i .. i + 3 and i + 4 .. i + 7 of row m (i a multiple of 8 on the even lane):
 // the even lane stores the octet.  Every lane of the wave must call it.
 __device__ static inline void dfl_xf_store_pair(void *xf, int kind, int m, int i, float a, float b, float c, float d) {
-    const float e = __shfl_down(a, 1, 64), f = __shfl_down(b, 1, 64), g = __shfl_down(c, 1, 64), h = __shfl_down(d, 1, 64);
+    const float e = dfl_dpp<0x101>(a), f = dfl_dpp<0x101>(b), g = dfl_dpp<0x101>(c), h = dfl_dpp<0x101>(d);  // row_shl:1
     if ((threadIdx.x & 1) == 0) dfl_xf_store(xf, kind, m, i, a, b, c, d, e, f, g, h);
 }
 #endif
@@ -257,6 +257,13 @@ bool dfl_whole_holds_weights(const dflash_ctx *ctx, int32_t w_type, int64_t n_in
 bool dfl_gemm_direct_takes(const dflash_ctx *ctx, int32_t w_type, int64_t n_in, int64_t n_out);
 int32_t dfl_gemm_direct(dflash_ctx *ctx, int32_t w_type, const void *w, const void *x, int32_t x_type, float *y, int64_t n_in, int64_t n_out,
                         int32_t n_rows, hipStream_t stream);
+
+// silu(x . gate^T) * (x . up^T) of up to sixteen rows as f16, [n_rows][ffn], in one launch (gemm_dense.hip): the fused gate | up matrix of a
+// dense layer in the tiled order, of more tiles than a whole-K launch takes.  xf, xs: the rows in fragment order (Q4K) and their
+// sub-block sums.
+bool dfl_gemm_dense_pair_takes(const dflash_ctx *ctx, int32_t w_type, int64_t n_in, int64_t ffn);
+int32_t dfl_gemm_dense_pair(dflash_ctx *ctx, int32_t w_type, const void *w, const void *xf, const void *xs, void *y_f16, int64_t n_in, int64_t ffn,
+                            int32_t n_rows, hipStream_t stream);
 
 // ---- many rows at once (gemm_rows.hip): the products of a prompt's prefill ----
 // Every row gets the bits the 16-row kernels give it in its own block: dfl_gemm_rows_plan says which of their

@@ -699,6 +699,13 @@ dfl_rows_plan dfl_gemm_rows_plan(const dflash_ctx *ctx, int32_t w_type, int64_t 
         return p;
     }
     if (w_type != DFLASH_TYPE_Q4_K_TILED) return p;
+    if (pair_ffn && dfl_gemm_dense_pair_takes(ctx, w_type, n_in, pair_ffn)) {  // (one sum over the whole K)
+        p.kind = DFL_XF_Q4K;
+        p.sums = 1;
+        p.total = nb;
+        p.n_cut = 1;
+        return p;
+    }
     int total = 0, n_wg = 0;
     if (!dfl_q4k_tiled_split(ctx, n_in, n_out, &total, &n_wg)) return p;
     p.kind = DFL_XF_Q4K;

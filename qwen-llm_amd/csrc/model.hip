@@ -44,7 +44,7 @@ __device__ float block_sum(float v, float *sh) {
 // kernel_rms_norm_batched_f32 (attn.metal:35-69), optionally preceded by the residual add that
 // feeds it (kernel_add, elementwise.metal): x += add (add may be null), then
 // y = x * rsqrt(mean(x^2) + eps) * w.  One row per workgroup; a row of up to 8192 values (n a
-// multiple of 4) is read once and stays in registers between the two passes.  With gate_w, the row's
+// multiple of 4) is read once and stays in registers between the two passes.  y may be null where only fragment order is asked for.  With gate_w, the row's
 // sigmoid(y . gate_w) also goes to gate_out[row] (the shared-expert gate of a mixture-of-experts
 // layer, forward.rs:749-824: the normalised row is at hand here, in registers).  With y_xf (n a multiple of 256, at most
 // 8192: every width the whole-K GEMMs take), y also goes there as f16 in the fragment order a whole-K GEMM reads (common.h, "XF").
@@ -154,7 +154,7 @@ __global__ void __launch_bounds__(256) rms_norm_kernel(float *__restrict__ x, co
         const int i = 4 * (tid + 256 * j);
         if (i < n) {
             const f4 o = v[j] * scale * wv[j];
-            *reinterpret_cast<f4 *>(yr + i) = o;
+            if (y) *reinterpret_cast<f4 *>(yr + i) = o;
             // (the host passes y_xf only for n a multiple of 256: whole waves are inside or outside the row)
             // (more than sixteen rows: block b of sixteen at y_xf + b * xf_stride bytes)
             if (y_xf)
@@ -173,15 +173,10 @@ __global__ void __launch_bounds__(256) rms_norm_kernel(float *__restrict__ x, co
                 sub += dfl_dpp<0xB1>(sub);
                 sub += dfl_dpp<0x4E>(sub);
                 sub += dfl_xor4(sub);
-                if ((tid & 7) == 0) {
-                    const int jj = (i >> 5) & 7;
-                    _Float16 *to = static_cast<_Float16 *>(y_xs) + (static_cast<size_t>(t >> 4) * (n >> 8) + (i >> 8)) * 512 + ((t & 15) + 16 * (jj >> 1)) * 8 + (jj & 1);
-                    const Q4KSumParts parts = q4k_sum_parts(sub);
-                    to[0] = parts.hi;
-                    to[2] = parts.lo;
-                    to[4] = parts.over;
-                    to[6] = static_cast<_Float16>(0.0f);
-                }
+                const float next = dfl_dpp<0x128>(sub);  // of the sub-block eight lanes on
+                if ((tid & 15) == 0)
+                    *reinterpret_cast<half8_t *>(static_cast<uint8_t *>(y_xs) + (static_cast<size_t>(t >> 4) * (n >> 8) + (i >> 8)) * 1024 +
+                                                 ((t & 15) + 16 * ((i >> 6) & 3)) * 16) = q4k_sum_operand(sub, next);
             }
             if (gate_w) dot += (o[0] * gw[j][0] + o[1] * gw[j][1]) + (o[2] * gw[j][2] + o[3] * gw[j][3]);
         }
@@ -721,6 +716,15 @@ LayerXf layer_xf(const dflash_ctx *ctx, const LayerT &L, bool packed_qkv_allowed
     return k;
 }
 
+// Whether a dense layer's gate | up is one launch of gemm_dense.hip (a prompt's rows get its bits: dfl_gemm_rows_plan asks the same).
+bool takes_dense_pair(const dflash_ctx *ctx, const dflash_model_cfg &c, const dflash_layer &L) {
+    const bool quants = L.down.type == DFLASH_TYPE_Q4_K || L.down.type == DFLASH_TYPE_Q4_K_TILED || L.down.type == DFLASH_TYPE_Q6_K ||
+                        L.down.type == DFLASH_TYPE_Q6_K_TILED;
+    return quants && c.ffn % DFL_QK_K == 0 && adjacent(L.gate, c.ffn, L.up, c.hidden) &&
+           dfl_whole_kind(ctx, L.gate.type, c.hidden, 2ll * c.ffn, c.ffn) == DFL_XF_NONE && norm_in_registers(c.hidden) &&
+           dfl_gemm_dense_pair_takes(ctx, L.gate.type, c.hidden, c.ffn);
+}
+
 // The q, k and v projections of a layer.  Returns in *packed whether they went out as one GEMM into
 // pk[n][q_dim + 2 kv_dim] (adjacent weights) or as separate ones into q, k, v.  xf_kind != DFL_XF_NONE (from
 // layer_xf: implies adjacent weights): the rows are in x_xf in fragment order and the whole-K kernel takes them.
@@ -794,6 +798,7 @@ struct dflash_session {
     float *pk = nullptr;  // [16][max(q_dim + 2 kv_dim, 2 ffn)]: output of a fused q/k/v or gate/up GEMM
     // cur and attn once more, as f16 in MFMA fragment order, for the projections that take the whole-K kernel
     uint8_t *xf_cur = nullptr, *xf_attn = nullptr, *xf_g = nullptr;
+    uint8_t *xs_cur = nullptr;  // the sub-block sums of xf_cur's rows (a wide dense layer's gate | up)
     float *hidden = nullptr;  // [16][n_taps][hidden] capture slots of the speculative step
     int32_t *ids = nullptr, *pos = nullptr, *argmax = nullptr;
     dfl_moe_scratch moe;
@@ -909,7 +914,7 @@ int32_t dflash_session_create(dflash_ctx *ctx, const dflash_model_cfg *cfg, int6
               bufs.want(&s->k, 16 * kv_dim) && bufs.want(&s->v, 16 * kv_dim) && bufs.want(&s->attn, 16 * q_dim) &&
               bufs.want(&s->mix, 16 * cfg->hidden) && bufs.want(&s->g, 16 * f) && bufs.want(&s->u, 16 * f) &&
               bufs.want(&s->pk, 16 * std::max(q_dim + 2 * kv_dim, 2 * f)) &&
-              bufs.want(&s->xf_cur, dfl_xf_bytes((cfg->hidden + 255) / 256 * 256)) &&
+              bufs.want(&s->xf_cur, dfl_xf_bytes((cfg->hidden + 255) / 256 * 256)) && bufs.want(&s->xs_cur, dfl_xs_bytes((cfg->hidden + 255) / 256 * 256)) &&
               bufs.want(&s->xf_attn, dfl_xf_bytes((static_cast<int64_t>(q_dim) + 255) / 256 * 256)) &&
               bufs.want(&s->xf_g, dfl_xf_bytes((static_cast<int64_t>(f) + 255) / 256 * 256)) &&
               bufs.want(&s->logits, 16 * static_cast<size_t>(cfg->vocab)) && bufs.want(&s->gap, 16) &&
@@ -1118,8 +1123,7 @@ int32_t verify_enqueue(dflash_ctx *ctx, const dflash_model *model, dflash_sessio
         const bool moe = c.n_expert > 0;
         const LayerXf xk = layer_kinds(il);
         if (!cur_ready)
-            rms_norm(n, st, s->x, pending_resid, L.attn_norm, s->cur, H, c.eps, nullptr, nullptr,
-                                               xk.qkv ? s->xf_cur : nullptr, xk.qkv);
+            rms_norm(n, st, s->x, pending_resid, L.attn_norm, xk.qkv ? nullptr : s->cur, H, c.eps, nullptr, nullptr, xk.qkv ? s->xf_cur : nullptr, xk.qkv);
         pending_resid = nullptr;
         cur_ready = false;
         bool packed;
@@ -1157,9 +1161,12 @@ int32_t verify_enqueue(dflash_ctx *ctx, const dflash_model *model, dflash_sessio
         // (where the router's launch can take the add and the norm along, they are left to it; s->x then gets its
         // s->mix together with the experts' sum)
         const bool norm_in_router = moe && dfl_moe_norm_fusable(ctx, c, L, n);
+        // (a wide dense layer's gate | up reads fragment order and sums, and leaves f16 rows: what every product rounds its rows to)
+        const bool dense_pair = !moe && takes_dense_pair(ctx, c, L);
         if (!norm_in_router)
-            rms_norm(n, st, s->x, s->mix, L.post_norm, s->cur, H, c.eps, moe ? L.shexp_gate : nullptr,
-                                               moe ? s->moe.sg : nullptr, xk.gate_up ? s->xf_cur : nullptr, xk.gate_up);
+            rms_norm(n, st, s->x, s->mix, L.post_norm, xk.gate_up || dense_pair ? nullptr : s->cur, H, c.eps, moe ? L.shexp_gate : nullptr, moe ? s->moe.sg : nullptr,
+                     xk.gate_up || dense_pair ? s->xf_cur : nullptr, dense_pair ? DFL_XF_Q4K : xk.gate_up, 0, ConvResid(),
+                     dense_pair ? s->xs_cur : nullptr);
         if (moe) {
             const float *next_w = il + 1 < c.n_layers ? model->layers[il + 1].attn_norm : model->output_norm;
             const int next_kind = layer_kinds(il + 1).qkv;  // (the next layer's q/k/v read what this layer's last kernel normalises)
@@ -1170,9 +1177,14 @@ int32_t verify_enqueue(dflash_ctx *ctx, const dflash_model *model, dflash_sessio
         } else {
             // the down projection reads fragment-order rows only where the gate/up launch can write them
             const int down_kind = xk.gate_up ? xk.down : DFL_XF_NONE;
-            if ((rc = gemm_gate_up(ctx, L.gate, L.up, s->cur, s->g, s->u, s->pk, H, c.ffn, n, st, s->xf_cur, xk.gate_up, s->xf_g, down_kind, true)))
-                return rc;
-            if (down_kind)
+            if (dense_pair)
+                rc = dfl_gemm_dense_pair(ctx, L.gate.type, L.gate.data, s->xf_cur, s->xs_cur, s->g, H, c.ffn, n, st);
+            else
+                rc = gemm_gate_up(ctx, L.gate, L.up, s->cur, s->g, s->u, s->pk, H, c.ffn, n, st, s->xf_cur, xk.gate_up, s->xf_g, down_kind, true);
+            if (rc) return rc;
+            if (dense_pair)
+                rc = dfl_gemm_fewrow_checked(ctx, L.down.type, L.down.data, s->g, DFLASH_TYPE_F16, s->mix, c.ffn, H, n, st);
+            else if (down_kind)
                 rc = dfl_gemm_whole(ctx, L.down.type, L.down.data, s->xf_g, s->mix, c.ffn, H, n, 0, nullptr, DFL_XF_NONE, st, true);
             else
                 rc = gemm(ctx, L.down, s->g, s->mix, c.ffn, H, n, st);
@@ -1191,8 +1203,8 @@ int32_t verify_enqueue(dflash_ctx *ctx, const dflash_model *model, dflash_sessio
     }
     if (want_head) {  // (not for a caller that asked for no output of it: a prefill block wants K/V and the taps only)
         if (!cur_ready)
-            rms_norm(n, st, s->x, pending_resid, model->output_norm, s->cur, H, c.eps, nullptr, nullptr,
-                                               head_kind ? s->xf_cur : nullptr, head_kind);
+            rms_norm(n, st, s->x, pending_resid, model->output_norm, head_kind ? nullptr : s->cur, H, c.eps, nullptr, nullptr, head_kind ? s->xf_cur : nullptr,
+                     head_kind);
         if (head_kind)
             rc = dfl_gemm_whole(ctx, model->output.type, model->output.data, s->xf_cur, lg, H, c.vocab, n, 0, nullptr, DFL_XF_NONE, st);
         else
@@ -1495,7 +1507,7 @@ int32_t prefill_group_enqueue(dflash_ctx *ctx, const dflash_model *model, dflash
         _Float16 *kc = s->k_cache + il * per_layer, *vtc = s->vt_cache + il * per_layer;
         next_rows = il + 1 < c.n_layers ? layer_rows(ctx, c, model->layers[il + 1]) : LayerRows();
         if (!moe || il == 0)  // (a mixture's later layers: the experts' last kernel has normalised their input)
-            rms_norm(n, st, g.x, pending_resid, L.attn_norm, g.cur, H, c.eps, nullptr, nullptr, g.xf_cur, rows.qkv.kind, xf_h, ConvResid(),
+            rms_norm(n, st, g.x, pending_resid, L.attn_norm, nullptr, H, c.eps, nullptr, nullptr, g.xf_cur, rows.qkv.kind, xf_h, ConvResid(),
                      rows.qkv.sums ? g.xs_cur : nullptr);
         pending_resid = nullptr;
         if ((rc = product(rows.qkv, L.wq, g.xf_cur, g.xs_cur, moe && il, g.pk, H, tot))) return rc;
@@ -1516,7 +1528,7 @@ int32_t prefill_group_enqueue(dflash_ctx *ctx, const dflash_model *model, dflash
                                         st)))
                 return rc;
         } else {
-            rms_norm(n, st, g.x, g.mix, L.post_norm, g.cur, H, c.eps, nullptr, nullptr, g.xf_cur, rows.gate_up.kind, xf_h, ConvResid(),
+            rms_norm(n, st, g.x, g.mix, L.post_norm, nullptr, H, c.eps, nullptr, nullptr, g.xf_cur, rows.gate_up.kind, xf_h, ConvResid(),
                      rows.gate_up.sums ? g.xs_cur : nullptr);
             // silu(gate) * up straight into fragment order, with the sums the down product wants
             if ((rc = dfl_gemm_rows(ctx, rows.gate_up, L.gate.type, L.gate.data, g.xf_cur, g.xs_cur, false, nullptr, H, 2ll * c.ffn, n, c.ffn, g.xf_g,
