@@ -474,6 +474,16 @@ int32_t dflash_prefill_blocks(dflash_ctx *ctx, const dflash_model *model, dflash
                               const int32_t *tap_layers_host, int32_t n_taps, float *hidden_capture,
                               dflash_stream_t stream);
 
+/* A whole prompt: dflash_prefill_blocks over all n_tokens, and the argmax behind the last one (on the host; the call waits).  Where the
+ * rows pass through the layers together the last block goes along with the others, and only the last layer (unless it is tapped) and the head
+ * are run for it alone; else it is a dflash_verify_block behind the others.  K/V rows, hidden rows and the argmax are those of
+ * the two calls.  Guards as dflash_prefill_blocks; on an error kv_n_pos is unchanged.  (The reference's prefill ends the same way: the last
+ * chunk's logits, metal_dflash.rs:10779-15648.) */
+int32_t dflash_prefill_prompt(dflash_ctx *ctx, const dflash_model *model, dflash_session *session,
+                              const int32_t *tokens_host, int32_t n_tokens, int64_t start_position,
+                              const int32_t *tap_layers_host, int32_t n_taps, float *hidden_capture,
+                              int32_t *last_argmax_host, dflash_stream_t stream);
+
 /* ---- block drafter ----------------------------------------------------------------------
  * DFlashConfig / DFlashHead / DFlashLayer (loader.rs:342-399), MetalDFlashSession
  * (metal_dflash.rs:5053-5191). */

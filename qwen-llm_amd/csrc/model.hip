@@ -486,6 +486,11 @@ __global__ void set_group_ids_kernel(IntGroupArgs ids, int n, int32_t *__restric
     if (i < n) ids_dst[i] = ids.v[i];
 }
 
+__global__ void set_range_kernel(int32_t first, int n, int32_t *__restrict__ dst) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) dst[i] = first + i;
+}
+
 // kernel_add_inplace_f32 (elementwise.metal:89)
 __global__ void add_kernel(float *__restrict__ x, const float *__restrict__ y, size_t n) {
     size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -1093,14 +1098,22 @@ uint64_t hash_model(const dflash_model *m) {
 // Every launch of one packed verify, from the embedding rows to the argmax, on `st`: no host
 // reads, no synchronisation, nothing that depends on the position except through pos[] on the
 // device, so the sequence can be captured once and replayed.
+// resume: the rows have been through the layers ahead of the last one, and through its K/V rows, as a prompt's group: what is
+// left of that layer, and the head.
+struct VerifyResume {
+    float *x;        // [n][hidden], the residual; rewritten
+    const float *q;  // [n][q_dim], normed and rotated (null: the last layer is done as well)
+};
 int32_t verify_enqueue(dflash_ctx *ctx, const dflash_model *model, dflash_session *s, int32_t n, int64_t start,
                        const int32_t *tap_layers, int32_t n_taps, float *hidden_capture, float *lg, int32_t *am, float *gp,
-                       hipStream_t st, bool want_head = true, const PrefillLane *lane = nullptr) {
+                       hipStream_t st, bool want_head = true, const PrefillLane *lane = nullptr, const VerifyResume *resume = nullptr) {
     const dflash_model_cfg &c = model->cfg;
     const int H = c.hidden, hd = c.head_dim;
     const size_t q_dim = static_cast<size_t>(c.n_q) * hd, kv_dim = static_cast<size_t>(c.n_kv) * hd;
-    int32_t rc = embed_rows(ctx, model->token_embd, s->ids, n, H, s->x, st);
-    if (rc) return rc;
+    float *const x = resume ? resume->x : s->x;
+    const float *const q = resume ? resume->q : s->q;
+    int32_t rc;
+    if (!resume && (rc = embed_rows(ctx, model->token_embd, s->ids, n, H, x, st))) return rc;
     const float scale = 1.0f / sqrtf(static_cast<float>(hd));
     const size_t per_layer = static_cast<size_t>(s->capacity) * kv_dim;
     bool cur_ready = false;  // s->cur already holds this layer's normalised input
@@ -1115,24 +1128,26 @@ int32_t verify_enqueue(dflash_ctx *ctx, const dflash_model *model, dflash_sessio
         head.qkv = head_kind;
         return head;
     };
-    for (int il = 0; il < c.n_layers; il++) {
+    for (int il = !resume ? 0 : resume->q ? c.n_layers - 1 : c.n_layers; il < c.n_layers; il++) {
         const dflash_layer &L = model->layers[il];
         _Float16 *kc = s->k_cache + il * per_layer, *vtc = s->vt_cache + il * per_layer;
         // (a mixture-of-experts layer leaves the next layer's normalised input behind)
         // (a dense layer leaves its FFN output in s->mix: the residual add is folded into this norm)
         const bool moe = c.n_expert > 0;
         const LayerXf xk = layer_kinds(il);
-        if (!cur_ready)
-            rms_norm(n, st, s->x, pending_resid, L.attn_norm, xk.qkv ? nullptr : s->cur, H, c.eps, nullptr, nullptr, xk.qkv ? s->xf_cur : nullptr, xk.qkv);
-        pending_resid = nullptr;
-        cur_ready = false;
-        bool packed;
-        if ((rc = gemm_qkv(ctx, L.wq, L.wk, L.wv, s->cur, s->q, s->k, s->v, s->pk, true, &packed, H, q_dim, kv_dim, n, st, s->xf_cur, xk.qkv, true)))
-            return rc;
-        const int64_t tot = q_dim + 2 * kv_dim;
-        qk_norm_rope(hd, c.n_q + 2 * c.n_kv, n, st, packed ? s->pk : s->q, packed ? tot : q_dim, packed ? s->pk + q_dim : s->k, packed ? tot : kv_dim, s->q, s->k, L.q_norm,
-            L.k_norm, kc, s->pos, c.n_q, c.n_kv, c.eps, c.rope_theta, packed ? s->pk + q_dim + kv_dim : s->v,
-            packed ? tot : kv_dim, vtc, s->capacity);
+        if (!resume) {
+            if (!cur_ready)
+                rms_norm(n, st, x, pending_resid, L.attn_norm, xk.qkv ? nullptr : s->cur, H, c.eps, nullptr, nullptr, xk.qkv ? s->xf_cur : nullptr, xk.qkv);
+            pending_resid = nullptr;
+            cur_ready = false;
+            bool packed;
+            if ((rc = gemm_qkv(ctx, L.wq, L.wk, L.wv, s->cur, s->q, s->k, s->v, s->pk, true, &packed, H, q_dim, kv_dim, n, st, s->xf_cur, xk.qkv, true)))
+                return rc;
+            const int64_t tot = q_dim + 2 * kv_dim;
+            qk_norm_rope(hd, c.n_q + 2 * c.n_kv, n, st, packed ? s->pk : s->q, packed ? tot : q_dim, packed ? s->pk + q_dim : s->k, packed ? tot : kv_dim, s->q, s->k, L.q_norm,
+                L.k_norm, kc, s->pos, c.n_q, c.n_kv, c.eps, c.rope_theta, packed ? s->pk + q_dim + kv_dim : s->v,
+                packed ? tot : kv_dim, vtc, s->capacity);
+        }
         if (lane) {
             // This block's K/V rows of the layer are written; the earlier blocks' must be before the attention reads
             // them.  The wait for the previous block comes first and the record behind it: the event then stands for
@@ -1149,7 +1164,7 @@ int32_t verify_enqueue(dflash_ctx *ctx, const dflash_model *model, dflash_sessio
         }
         // under capture the context length is read from pos[0] on the device: the same launches then serve every
         // position of the bucket
-        if ((rc = dfl_attn_block(ctx, s->q, DFLASH_TYPE_F32, kc, vtc, 1, start, n, c.n_q, c.n_kv, hd, s->capacity, scale,
+        if ((rc = dfl_attn_block(ctx, q, DFLASH_TYPE_F32, kc, vtc, 1, start, n, c.n_q, c.n_kv, hd, s->capacity, scale,
                                  s->attn, st, 0, 0, ctx->capturing ? s->pos : nullptr, xk.wo ? s->xf_attn : nullptr, xk.wo)))
             return rc;
         if (xk.wo)
@@ -1164,13 +1179,13 @@ int32_t verify_enqueue(dflash_ctx *ctx, const dflash_model *model, dflash_sessio
         // (a wide dense layer's gate | up reads fragment order and sums, and leaves f16 rows: what every product rounds its rows to)
         const bool dense_pair = !moe && takes_dense_pair(ctx, c, L);
         if (!norm_in_router)
-            rms_norm(n, st, s->x, s->mix, L.post_norm, xk.gate_up || dense_pair ? nullptr : s->cur, H, c.eps, moe ? L.shexp_gate : nullptr, moe ? s->moe.sg : nullptr,
+            rms_norm(n, st, x, s->mix, L.post_norm, xk.gate_up || dense_pair ? nullptr : s->cur, H, c.eps, moe ? L.shexp_gate : nullptr, moe ? s->moe.sg : nullptr,
                      xk.gate_up || dense_pair ? s->xf_cur : nullptr, dense_pair ? DFL_XF_Q4K : xk.gate_up, 0, ConvResid(),
                      dense_pair ? s->xs_cur : nullptr);
         if (moe) {
             const float *next_w = il + 1 < c.n_layers ? model->layers[il + 1].attn_norm : model->output_norm;
             const int next_kind = layer_kinds(il + 1).qkv;  // (the next layer's q/k/v read what this layer's last kernel normalises)
-            if ((rc = dfl_moe_ffn(ctx, c, L, s->cur, n, s->moe, s->x, L.shexp_gate != nullptr, next_w, s->cur, &cur_ready, st,
+            if ((rc = dfl_moe_ffn(ctx, c, L, s->cur, n, s->moe, x, L.shexp_gate != nullptr, next_w, s->cur, &cur_ready, st,
                                   norm_in_router ? s->mix : nullptr, norm_in_router ? L.post_norm : nullptr,
                                   next_kind ? s->xf_cur : nullptr, next_kind)))
                 return rc;
@@ -1193,17 +1208,17 @@ int32_t verify_enqueue(dflash_ctx *ctx, const dflash_model *model, dflash_sessio
             bool tapped = false;
             for (int t = 0; t < n_taps; t++) tapped = tapped || tap_layers[t] == il;
             if (tapped)
-                add_kernel<<<blocks_for(static_cast<size_t>(n) * H), 256, 0, st>>>(s->x, s->mix, static_cast<size_t>(n) * H);
+                add_kernel<<<blocks_for(static_cast<size_t>(n) * H), 256, 0, st>>>(x, s->mix, static_cast<size_t>(n) * H);
             else
                 pending_resid = s->mix;
         }
         for (int t = 0; t < n_taps; t++)
             if (tap_layers[t] == il)
-                capture_kernel<<<dim3(blocks_for(H), n), 256, 0, st>>>(s->x, hidden_capture, H, n_taps, t);
+                capture_kernel<<<dim3(blocks_for(H), n), 256, 0, st>>>(x, hidden_capture, H, n_taps, t);
     }
     if (want_head) {  // (not for a caller that asked for no output of it: a prefill block wants K/V and the taps only)
         if (!cur_ready)
-            rms_norm(n, st, s->x, pending_resid, model->output_norm, head_kind ? nullptr : s->cur, H, c.eps, nullptr, nullptr, head_kind ? s->xf_cur : nullptr,
+            rms_norm(n, st, x, pending_resid, model->output_norm, head_kind ? nullptr : s->cur, H, c.eps, nullptr, nullptr, head_kind ? s->xf_cur : nullptr,
                      head_kind);
         if (head_kind)
             rc = dfl_gemm_whole(ctx, model->output.type, model->output.data, s->xf_cur, lg, H, c.vocab, n, 0, nullptr, DFL_XF_NONE, st);
@@ -1476,9 +1491,11 @@ bool prefill_group_takes(const dflash_ctx *ctx, const dflash_model *model, const
 // One group of n rows (positions start .. start + n - 1) through every layer, on `st`: K/V rows into the session's
 // cache, tapped residuals into hidden_capture.  A row gets the bits verify_enqueue gives it in its own 16-row block:
 // every operator here is that block's operator over more rows.
+// with_head: also the head of the last block's rows (argmax and gap to the session's buffers); what the last layer is for is
+// then the block path's, for those rows alone.
 int32_t prefill_group_enqueue(dflash_ctx *ctx, const dflash_model *model, dflash_session *s, PrefillGroup &g, const int32_t *tokens,
                               int32_t n, int64_t start, const int32_t *tap_layers, int32_t n_taps, float *hidden_capture,
-                              hipStream_t st) {
+                              hipStream_t st, bool with_head = false) {
     const dflash_model_cfg &c = model->cfg;
     const int H = c.hidden, hd = c.head_dim;
     const bool moe = c.n_expert > 0;
@@ -1502,6 +1519,7 @@ int32_t prefill_group_enqueue(dflash_ctx *ctx, const dflash_model *model, dflash
     };
     const float *pending_resid = nullptr;  // a dense layer's FFN output still to be added to g.x
     LayerRows rows = layer_rows(ctx, c, model->layers[0]), next_rows;
+    bool last_done = false;
     for (int il = 0; il < c.n_layers; il++, rows = next_rows) {
         const dflash_layer &L = model->layers[il];
         _Float16 *kc = s->k_cache + il * per_layer, *vtc = s->vt_cache + il * per_layer;
@@ -1516,6 +1534,7 @@ int32_t prefill_group_enqueue(dflash_ctx *ctx, const dflash_model *model, dflash
         for (int t = 0; t < n_taps; t++) tapped = tapped || tap_layers[t] == il;
         // nothing of the last layer beyond its K/V rows is needed unless its residual is tapped (as in verify_enqueue)
         if (il == c.n_layers - 1 && !tapped) break;
+        last_done = il == c.n_layers - 1;
         if ((rc = dfl_attn_blocks(ctx, g.q, DFLASH_TYPE_F32, kc, vtc, start, n, c.n_q, c.n_kv, hd, s->capacity, scale, g.attn, st, g.xf_attn,
                                   rows.wo.kind)))
             return rc;
@@ -1546,14 +1565,17 @@ int32_t prefill_group_enqueue(dflash_ctx *ctx, const dflash_model *model, dflash
                 capture_kernel<<<dim3(blocks_for(H), n), 256, 0, st>>>(g.x, hidden_capture, H, n_taps, t);
     }
     DFL_HIP_CHECK(ctx, hipGetLastError());
-    return DFLASH_OK;
+    if (!with_head) return DFLASH_OK;
+    const int first = (n - 1) / 16 * 16;  // of the last block
+    const VerifyResume resume = {g.x + static_cast<size_t>(first) * H, last_done ? nullptr : g.q + static_cast<size_t>(first) * q_dim};
+    return verify_enqueue(ctx, model, s, n - first, start + first, nullptr, 0, nullptr, s->logits, s->argmax, s->gap, st, true, nullptr, &resume);
 }
 
 }  // namespace
 
-int32_t dflash_prefill_blocks(dflash_ctx *ctx, const dflash_model *model, dflash_session *s, const int32_t *tokens,
-                              int32_t n_tokens, int64_t start, const int32_t *tap_layers, int32_t n_taps,
-                              float *hidden_capture, dflash_stream_t stream) {
+namespace {
+int32_t prefill_check(dflash_ctx *ctx, const dflash_model *model, const dflash_session *s, const int32_t *tokens, int32_t n_tokens, int64_t start,
+                      const int32_t *tap_layers, int32_t n_taps, const float *hidden_capture) {
     if (!ctx) return DFLASH_ERR_INVALID_INPUT;
     if (!model || !s || !tokens) return dfl_fail(ctx, DFLASH_ERR_INVALID_INPUT, "prefill_blocks: null argument");
     if (const int32_t rc_ = model_tensors_checked(ctx, model)) return rc_;
@@ -1571,6 +1593,15 @@ int32_t dflash_prefill_blocks(dflash_ctx *ctx, const dflash_model *model, dflash
     if (n_taps < 0 || n_taps > s->n_taps || (n_taps > 0 && (!tap_layers || !hidden_capture)))
         return dfl_fail(ctx, DFLASH_ERR_INVALID_INPUT, "prefill_blocks: hidden capture arguments");
     if (memcmp(&c, &s->cfg, sizeof(c)) != 0) return dfl_fail(ctx, DFLASH_ERR_STATE, "prefill_blocks: session/model shape mismatch");
+    return DFLASH_OK;
+}
+}  // namespace
+
+int32_t dflash_prefill_blocks(dflash_ctx *ctx, const dflash_model *model, dflash_session *s, const int32_t *tokens,
+                              int32_t n_tokens, int64_t start, const int32_t *tap_layers, int32_t n_taps,
+                              float *hidden_capture, dflash_stream_t stream) {
+    if (const int32_t rc_ = prefill_check(ctx, model, s, tokens, n_tokens, start, tap_layers, n_taps, hidden_capture)) return rc_;
+    const dflash_model_cfg &c = model->cfg;
     int32_t rc = DFLASH_OK;
     if (!s->pipe && (rc = prefill_pipe_create(ctx, s))) return rc;
     PrefillPipe *p = s->pipe;
@@ -1662,6 +1693,51 @@ int32_t dflash_prefill_blocks(dflash_ctx *ctx, const dflash_model *model, dflash
     return DFLASH_OK;
 }
 
+int32_t dflash_prefill_prompt(dflash_ctx *ctx, const dflash_model *model, dflash_session *s, const int32_t *tokens, int32_t n_tokens,
+                              int64_t start, const int32_t *tap_layers, int32_t n_taps, float *hidden_capture, int32_t *last_argmax_host,
+                              dflash_stream_t stream) {
+    if (const int32_t rc_ = prefill_check(ctx, model, s, tokens, n_tokens, start, tap_layers, n_taps, hidden_capture)) return rc_;
+    if (!last_argmax_host) return dfl_fail(ctx, DFLASH_ERR_INVALID_INPUT, "prefill_prompt: null argument");
+    const dflash_model_cfg &c = model->cfg;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    int32_t rc = DFLASH_OK, ids[16];
+    if (!s->pipe && (rc = prefill_pipe_create(ctx, s))) return rc;
+    PrefillGroup &g = s->pipe->group;
+    const size_t cap_row = static_cast<size_t>(std::max(n_taps, 0)) * c.hidden;
+    auto capture = [&](int32_t row) { return hidden_capture ? hidden_capture + static_cast<size_t>(row) * cap_row : nullptr; };
+    // The last pass, whose last block has the head, is a group wherever that is more than a block: the block by itself reads every weight
+    // again.  ms, blocks and verify : this one, 17, 64, 300 and 2048 tokens: ten layers of the 35B-A3B shape 1.40 : 1.24, 2.41 : 1.61,
+    // 3.23 : 2.39, 7.58 : 6.60; six of the 27B shape 1.13 : 0.96, 1.47 : 1.08, 2.46 : 2.10, 8.86 : 8.28; ten of a 1024-wide one
+    // 0.70 : 0.51, 0.90 : 0.61, 1.26 : 0.93, 3.16 : 2.76.
+    int32_t body = 0;
+    bool tail_group = n_tokens > 16 && start + n_tokens <= 0x7fffffffll && prefill_group_takes(ctx, model, g);
+    if (tail_group) body = (n_tokens - 1) / g.rows * g.rows;
+    tail_group = tail_group && n_tokens - body > 16;
+    if (!tail_group) body = (n_tokens - 1) / 16 * 16;
+    if (body && (rc = dflash_prefill_blocks(ctx, model, s, tokens, body, start, tap_layers, n_taps, hidden_capture, stream))) return rc;
+    const int32_t n = n_tokens - body;
+    if (!tail_group) {
+        if ((rc = dflash_verify_block(ctx, model, s, tokens + body, n, start + body, tap_layers, n_taps, nullptr, nullptr, capture(body), nullptr, ids,
+                                      stream))) {
+            s->kv_n_pos = start;  // (rows written past it are overwritten by the next block)
+            return rc;
+        }
+        *last_argmax_host = ids[n - 1];
+        return DFLASH_OK;
+    }
+    rc = prefill_group_enqueue(ctx, model, s, g, tokens + body, n, start + body, tap_layers, n_taps, capture(body), st, true);
+    hipError_t err = hipSuccess;
+    if (!rc) err = hipMemcpyAsync(ctx->pinned, s->argmax + (n - 1) % 16, sizeof(int32_t), hipMemcpyDeviceToHost, st);
+    const hipError_t done = hipStreamSynchronize(st);
+    if (rc || err != hipSuccess || done != hipSuccess) {
+        s->kv_n_pos = start;
+        return rc ? rc : dfl_fail(ctx, DFLASH_ERR_HIP, "prefill_prompt: %s", hipGetErrorString(err != hipSuccess ? err : done));
+    }
+    memcpy(last_argmax_host, ctx->pinned, sizeof(int32_t));
+    s->kv_n_pos = start + n_tokens;
+    return DFLASH_OK;
+}
+
 int32_t dflash_draft_session_create(dflash_ctx *ctx, const dflash_draft_cfg *cfg, int64_t ctx_capacity, int64_t vocab,
                                     dflash_draft_session **out) {
     if (!ctx || !cfg || !out) return DFLASH_ERR_INVALID_INPUT;
@@ -1742,8 +1818,11 @@ int32_t dflash_draft_append_ctx(dflash_ctx *ctx, dflash_draft_session *s, const 
         return dfl_fail(ctx, DFLASH_ERR_STATE, "append_ctx: %lld + %d columns exceed the context capacity %lld",
                         static_cast<long long>(s->ctx_len), n_cols, static_cast<long long>(s->capacity));
     if (n_cols == 0) return DFLASH_OK;
-    for (int i = 0; i < n_cols; i++)
+    bool range = true;  // each position one past the one before it
+    for (int i = 0; i < n_cols; i++) {
         if (positions[i] != s->ctx_len + i) s->contiguous = false;
+        range = range && static_cast<int64_t>(positions[i]) == static_cast<int64_t>(positions[0]) + i;
+    }
     hipStream_t st = static_cast<hipStream_t>(stream);
     const size_t feat = static_cast<size_t>(s->cfg.n_taps) * s->cfg.hidden;
     DFL_HIP_CHECK(ctx, hipMemcpyAsync(s->ctx_raw + s->ctx_len * feat, hidden_capture, n_cols * feat * sizeof(float),
@@ -1752,6 +1831,9 @@ int32_t dflash_draft_append_ctx(dflash_ctx *ctx, dflash_draft_session *s, const 
         Int16Args none = {}, pos_arg = {};
         for (int i = 0; i < n_cols; i++) pos_arg.v[i] = positions[i];
         set_ids_pos_kernel<<<1, 64, 0, st>>>(none, pos_arg, n_cols, nullptr, s->pos_ctx + s->ctx_len, nullptr, 0);
+    } else if (range) {
+        set_range_kernel<<<blocks_for(n_cols), 256, 0, st>>>(positions[0], n_cols, s->pos_ctx + s->ctx_len);
+        DFL_HIP_CHECK(ctx, hipGetLastError());
     } else {
         DFL_HIP_CHECK(ctx, hipMemcpyAsync(s->pos_ctx + s->ctx_len, positions, n_cols * sizeof(int32_t), hipMemcpyHostToDevice, st));
     }

@@ -573,6 +573,25 @@ class Session:
                                                 hidden.data_ptr() if hidden is not None else None, _stream_ptr()))
         return hidden
 
+    def prefill_prompt(self, tokens, start_position: int, want_hidden=True):
+        """A whole prompt (dflash_prefill_prompt): the tapped hidden rows of every token as ``prefill_blocks`` returns them (or
+        None), and the argmax behind the last one."""
+        torch = _torch()
+        n = len(tokens)
+        L = self._L
+        L.dflash_prefill_prompt.restype = C.c_int32
+        L.dflash_prefill_prompt.argtypes = [C.c_void_p, C.POINTER(ModelC), C.c_void_p, C.POINTER(C.c_int32), C.c_int32, C.c_int64,
+                                            C.POINTER(C.c_int32), C.c_int32, C.c_void_p, C.POINTER(C.c_int32), C.c_void_p]
+        toks = (C.c_int32 * max(n, 1))(*[int(t) for t in tokens])
+        n_taps = len(self.tap_layers) if want_hidden else 0
+        taps = (C.c_int32 * max(n_taps, 1))(*self.tap_layers[:n_taps])
+        hidden = (_binding._empty((n, n_taps, self.model.cfg.hidden), dtype=torch.float32, device=f"cuda:{self.ctx.device}")
+                  if n_taps else None)
+        last = C.c_int32()
+        self.ctx._check(L.dflash_prefill_prompt(self.ctx._h, C.byref(self.model.c), self._h, toks, n, start_position, taps, n_taps,
+                                                hidden.data_ptr() if hidden is not None else None, C.byref(last), _stream_ptr()))
+        return hidden, last.value
+
     @property
     def graph_replays(self) -> int:
         return int(self._L.dflash_session_graph_replays(self._h))
@@ -814,23 +833,16 @@ class SpeculativeDecoder:
         self.draft_session.close()
 
     def prefill(self, prompt):
-        """Run the prompt through the packed verify in blocks of 16, feed the tapped hidden rows to
+        """Run the prompt through the target (many blocks per pass where it takes them so), feed the tapped hidden rows to
         the drafter context, and return the argmax after the last prompt token."""
         assert len(prompt) > 0 and self.position == 0
-        # every block but the last: K/V and the tapped rows only (many blocks per pass, or several in flight); the last one with its head
-        body = (len(prompt) - 1) // 16 * 16
-        if body:
-            hidden = self.session.prefill_blocks(list(prompt[:body]), 0)
-            for s in range(0, body, 16):
-                self.draft_session.append_target_ctx_columns(hidden[s:s + 16], list(range(s, s + 16)))
-        blk = list(prompt[body:])
-        last = self.session.encode_packed_verify_layer_major(blk, body)
-        self.draft_session.append_target_ctx_columns(last.hidden_capture, list(range(body, body + len(blk))))
+        hidden, first = self.session.prefill_prompt(list(prompt), 0)
+        self.draft_session.append_target_ctx_columns(hidden, list(range(len(prompt))))
         # the drafter's pass over the prompt's columns belongs to the prefill, not to the first step
         self.draft_session.prepare_ctx()
         _torch().cuda.synchronize()
         self.position = len(prompt)
-        return last.argmax_host[-1]
+        return first
 
     def step(self, carry: int, budget: int, draft_override=None, replay_only: bool = False) -> StepResultC:
         """One speculative transition.  ``replay_only``: a prefix-replay step, ``draft_override`` holds every draft

@@ -233,3 +233,58 @@ def test_a_prepared_session_allocates_nothing_for_its_first_prompt(ctx, shape):
         taken = free - torch.cuda.mem_get_info()[0]
         sess.close()
     assert taken == 0
+
+
+@pytest.mark.parametrize("head", [0, 37])
+@pytest.mark.parametrize("taps", [[0], [0, 1]], ids=["last layer not tapped", "tapped"])
+@pytest.mark.parametrize("shape,adjacent,rows", [("experts", True, 1), ("experts", True, 16), ("experts", True, 17), ("experts", True, 300), ("experts", True, 2050),
+                                                 ("experts", True, 2070), ("wide", True, 33), ("narrow", True, 130), ("narrow", False, 70), ("heads64", True, 500)])
+def test_a_prompt_in_one_call_equals_its_blocks_and_their_last_one(ctx, shape, adjacent, rows, taps, head):
+    """Hidden rows, the argmax behind the last token, and what a block behind the prompt computes from its K/V rows: a prompt of one block, of a few, of
+    a group and a rest of a block or of more, and a target that has no groups (separate projections: its blocks go by lanes)."""
+    cfg, attn_type = SHAPES[shape]
+    model = dfl.TargetModel(ctx, cfg, dfl.synth_target_weights_device(cfg, 5, "cuda", attn_type=attn_type), adjacent=adjacent)
+    two, one = dfl.Session(ctx, model, head + rows + 32, taps), dfl.Session(ctx, model, head + rows + 32, taps)
+    tokens = np.random.default_rng(rows).integers(0, cfg.vocab, head + rows).tolist()
+    if head:
+        for s in (two, one):
+            s.prefill_blocks(tokens[:head], 0, want_hidden=False)
+    body = head + (rows - 1) // 16 * 16
+    want = [two.prefill_blocks(tokens[head:body], head)] if body > head else []
+    last = two.encode_packed_verify_layer_major(tokens[body:], body)
+    got, token = one.prefill_prompt(tokens[head:], head)
+    assert torch.equal(got, torch.cat(want + [last.hidden_capture])) and token == last.argmax_host[-1]
+    assert one.kv_n_pos == two.kv_n_pos == head + rows
+    a, b = (s.encode_packed_verify_layer_major([token, 3, 5], head + rows, want_logits=True) for s in (two, one))
+    assert torch.equal(a.logits, b.logits)
+    two.close()
+    one.close()
+
+
+def test_a_prompt_in_one_call_keeps_the_guards(ctx):
+    cfg, attn_type = SHAPES["narrow"]
+    model = dfl.TargetModel(ctx, cfg, dfl.synth_target_weights_device(cfg, 5, "cuda", attn_type=attn_type))
+    sess = dfl.Session(ctx, model, 64, [0])
+    for tokens, start, status in (([1, 2], 5, 10), ([1, cfg.vocab], 0, 8), ([1] * 65, 0, 10), ([], 0, 1)):
+        with pytest.raises(dfl.DFlashError) as e:
+            sess.prefill_prompt(tokens, start)
+        assert e.value.status == status and sess.kv_n_pos == 0
+    sess.close()
+
+
+@pytest.mark.parametrize("first", [0, 7])
+def test_context_columns_appended_at_once_equal_columns_in_blocks(ctx, first):
+    """More than sixteen columns of consecutive positions: from zero (the mirror's case) and off it."""
+    cfg = dfl.ModelConfig(n_layers=1, hidden=512, n_q=4, n_kv=2, head_dim=64, ffn=512, vocab=1024)
+    dcfg = dfl.DraftConfig(n_layers=2, hidden=512, n_q=4, n_kv=2, head_dim=64, ffn=512, block_size=8, n_taps=2)
+    model = dfl.TargetModel(ctx, cfg, dfl.synth_target_weights_device(cfg, 5, "cuda"))
+    drafter = dfl.DraftHead(ctx, dcfg, dfl.synth_draft_weights_device(dcfg, 6, "cuda", vocab=cfg.vocab))
+    cols = torch.randn((45, 2, 512), generator=torch.Generator(device="cuda").manual_seed(3), device="cuda")
+    out = []
+    for step in (16, 45):
+        d = dfl.DraftSession(ctx, drafter, model, 64)
+        for i in range(0, 45, step):
+            d.append_target_ctx_columns(cols[i:i + step], list(range(first + i, first + min(i + step, 45))))
+        out.append(d.draft_block(5, cfg.vocab - 1, first + 45, want_logits=True)[1].clone())
+        d.close()
+    assert torch.equal(out[0], out[1])
