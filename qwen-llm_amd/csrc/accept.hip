@@ -60,45 +60,66 @@ __device__ __forceinline__ Top2 top2_merge(Top2 a, Top2 b) {
     return a;
 }
 
+__device__ __forceinline__ Top2 top2_wave(Top2 t) {  // over a wave, in every lane
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        Top2 o;
+        o.v1 = __shfl_xor(t.v1, off, 64);
+        o.i1 = static_cast<uint32_t>(__shfl_xor(static_cast<int>(t.i1), off, 64));
+        o.v2 = __shfl_xor(t.v2, off, 64);
+        t = top2_merge(t, o);
+    }
+    return t;
+}
+// What bounds it and the launch that follows it: their chains (the merges are of maxima and of the lowest token among equals, so any order
+// gives the same).  All of a thread's tokens are asked for at once, waves merge by lane moves; the last launch has a chunk a lane.
+// 6.4 + 5.0 us a 16 x 151936 block with a tree through LDS and one thread a row behind it, 5.0 + 2.7 now.
 __global__ void __launch_bounds__(kSelThreads)
     top2_chunk_kernel(const float *__restrict__ logits, int64_t vocab, int64_t stride, Top2 *__restrict__ part) {
-    __shared__ Top2 sh[kSelThreads];
+    __shared__ Top2 sh[kSelThreads / 64];
     const int row = blockIdx.y, chunk = blockIdx.x;
     const float *x = logits + row * stride;
+    const int64_t base = static_cast<int64_t>(chunk) * kChunk + threadIdx.x;
+    float v[kChunk / kSelThreads];
+#pragma unroll
+    for (int j = 0; j < kChunk / kSelThreads; j++) v[j] = x[min(base + j * kSelThreads, vocab - 1)];
     Top2 t = {-INFINITY, 0xffffffffu, -INFINITY};
 #pragma unroll
     for (int j = 0; j < kChunk / kSelThreads; j++) {
-        int64_t i = static_cast<int64_t>(chunk) * kChunk + j * kSelThreads + threadIdx.x;
+        const int64_t i = base + j * kSelThreads;  // (a thread's tokens ascend: among equals the first stands)
         if (i < vocab) {
-            float v = x[i];
-            if (v > t.v1) {
+            if (v[j] > t.v1 || (v[j] == t.v1 && t.i1 == 0xffffffffu)) {
                 t.v2 = t.v1;
-                t.v1 = v;
+                t.v1 = v[j];
                 t.i1 = static_cast<uint32_t>(i);
-            } else if (v == t.v1 && static_cast<uint32_t>(i) < t.i1) {
-                t.v2 = t.v1;
-                t.i1 = static_cast<uint32_t>(i);
-            } else if (v > t.v2) {
-                t.v2 = v;
+            } else if (v[j] > t.v2) {
+                t.v2 = v[j];
             }
         }
     }
-    sh[threadIdx.x] = t;
-    for (int s = kSelThreads / 2; s > 0; s >>= 1) {
-        __syncthreads();
-        if (threadIdx.x < s) sh[threadIdx.x] = top2_merge(sh[threadIdx.x], sh[threadIdx.x + s]);
-    }
-    if (threadIdx.x == 0) part[row * gridDim.x + chunk] = sh[0];
+    t = top2_wave(t);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = t;
+    __syncthreads();
+    if (threadIdx.x >= 64) return;
+    t = top2_wave(threadIdx.x < kSelThreads / 64 ? sh[threadIdx.x] : Top2{-INFINITY, 0xffffffffu, -INFINITY});
+    if (threadIdx.x == 0) part[row * gridDim.x + chunk] = t;
 }
 
-__global__ void top2_final_kernel(const Top2 *__restrict__ part, int n_chunks, int32_t *__restrict__ idx,
-                                  float *__restrict__ gap) {
-    const int row = blockIdx.x;
-    if (threadIdx.x != 0) return;
-    Top2 t = part[row * n_chunks];
-    for (int c = 1; c < n_chunks; c++) t = top2_merge(t, part[row * n_chunks + c]);
+__global__ void __launch_bounds__(64) top2_final_kernel(const Top2 *__restrict__ part, int n_chunks, int32_t *__restrict__ idx, float *__restrict__ gap,
+                                                        int32_t *page, const int32_t *__restrict__ also) {
+    const int row = blockIdx.x, lane = threadIdx.x;
+    Top2 t = {-INFINITY, 0xffffffffu, -INFINITY};
+    for (int c = lane; c < n_chunks; c += 64) t = top2_merge(t, part[row * n_chunks + c]);
+    t = top2_wave(t);
+    if (lane != 0) return;
+    const float d = t.v1 - t.v2;
     idx[row] = static_cast<int32_t>(t.i1);
-    gap[row] = t.v1 - t.v2;
+    gap[row] = d;
+    if (page) {
+        page[row] = static_cast<int32_t>(t.i1);
+        if (also) page[16 + row] = also[row];
+        page[32 + row] = __float_as_int(d);
+    }
 }
 
 // ------------------------------------------------------------------------------------------
@@ -891,24 +912,28 @@ int32_t check_rows(dflash_ctx *ctx, const char *what, const float *logits, int32
 
 }  // namespace
 
-extern "C" {
-
-int32_t dflash_argmax_top2(dflash_ctx *ctx, const float *logits, int32_t n_rows, int64_t vocab, int64_t stride,
-                           int32_t *idx, float *gap, dflash_stream_t stream) {
+int32_t dfl_argmax_top2(dflash_ctx *ctx, const float *logits, int32_t n_rows, int64_t vocab, int64_t stride, int32_t *idx, float *gap,
+                        int32_t *page, const int32_t *also, hipStream_t st) {
     if (!ctx) return DFLASH_ERR_INVALID_INPUT;
     int32_t rc = check_rows(ctx, "argmax_top2", logits, n_rows, vocab, stride);
     if (rc) return rc;
     if (!idx || !gap) return dfl_fail(ctx, DFLASH_ERR_INVALID_INPUT, "argmax_top2: null output");
-    hipStream_t st = static_cast<hipStream_t>(stream);
     const int n_chunks = static_cast<int>((vocab + kChunk - 1) / kChunk);
     size_t off = 0;
     Top2 *part = dfl_ws_take<Top2>(ctx, &off, sizeof(Top2) * n_rows * n_chunks);
     if (!part) return dfl_fail(ctx, DFLASH_ERR_WORKSPACE, "argmax_top2: workspace too small");
     dfl_timed timer(ctx, st, DFL_T_ARGMAX);
     top2_chunk_kernel<<<dim3(n_chunks, n_rows), kSelThreads, 0, st>>>(logits, vocab, stride, part);
-    top2_final_kernel<<<n_rows, 64, 0, st>>>(part, n_chunks, idx, gap);
+    top2_final_kernel<<<n_rows, 64, 0, st>>>(part, n_chunks, idx, gap, page, also);
     DFL_HIP_CHECK(ctx, hipGetLastError());
     return DFLASH_OK;
+}
+
+extern "C" {
+
+int32_t dflash_argmax_top2(dflash_ctx *ctx, const float *logits, int32_t n_rows, int64_t vocab, int64_t stride,
+                           int32_t *idx, float *gap, dflash_stream_t stream) {
+    return dfl_argmax_top2(ctx, logits, n_rows, vocab, stride, idx, gap, nullptr, nullptr, static_cast<hipStream_t>(stream));
 }
 
 int32_t dflash_argmax_greedy(dflash_ctx *ctx, const float *logits, int32_t n_rows, int64_t vocab, int64_t stride,
@@ -1137,8 +1162,8 @@ int32_t dflash_accept_prefix(dflash_ctx *ctx, const int32_t *verified, int32_t n
         // the decision goes straight to the context's pinned page when the device can address it (one copy less
         // between the last kernel and the host)
         static_assert(sizeof(dflash_accept_decision) <= DFL_PINNED_BYTES, "the decision is read back through the pinned page");
-        void *pinned_dev = nullptr;
-        const bool direct = ctx->pinned && hipHostGetDevicePointer(&pinned_dev, ctx->pinned, 0) == hipSuccess && pinned_dev;
+        void *const pinned_dev = ctx->pinned_dev;
+        const bool direct = pinned_dev != nullptr;
         if (!direct) (void)hipGetLastError();
         decide_kernel<<<1, kDecThreads, 0, st>>>(rows, tile_sums, direct ? static_cast<dflash_accept_decision *>(pinned_dev) : d_out, mode, n_tiles,
                                                  n_tokens, a);

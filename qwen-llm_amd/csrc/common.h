@@ -53,6 +53,7 @@ struct dflash_ctx {
     // pinned host staging for the few words a blocking call reads back (a device-to-host copy into pageable
     // memory is staged by the runtime and costs several microseconds each); one page, owned
     void *pinned = nullptr;
+    void *pinned_dev = nullptr;  // its address on the device (null: the device cannot write it)
     // kernels whose dynamic-LDS limit has already been raised for this context (the attribute is kept per
     // device by the runtime, so the record lives with the context, not in process-wide flags)
     const void *lds_attr_fn[96] = {nullptr};
@@ -325,7 +326,8 @@ struct dfl_moe_scratch {
 // already holds sigmoid(cur . shexp_gate) per row (the norm kernel that wrote cur computed it).
 // next_norm_w / next_cur / next_done (all or none): the RMSNorm that reads x_resid next may be done
 // in the same pass, next_cur = rms_norm(x_resid) * next_norm_w; *next_done says whether it was.
-// next_xf / next_xf_kind: where that norm is done here, its rows also go to next_xf in fragment order (XF).
+// next_xf / next_xf_kind: where that norm is done here, its rows go to next_xf in fragment order (XF) instead.  cap / cap_ld: where it is
+// done here, x_resid's new rows also go to cap, cap_ld floats apart (16-byte aligned, cap_ld a multiple of 4).
 // pre_add / pre_norm_w (both or neither; only where dfl_moe_norm_fusable() holds): the layer's input has not been
 // normalised yet, x_resid still lacks pre_add (the attention's output projection), and `cur` is where the normalised rows
 // go: cur = rms_norm(x_resid + pre_add) * pre_norm_w, computed inside the router's launch with the shared-expert gate
@@ -333,7 +335,7 @@ struct dfl_moe_scratch {
 int32_t dfl_moe_ffn(dflash_ctx *ctx, const dflash_model_cfg &cfg, const dflash_layer &layer, float *cur, int n,
                     const dfl_moe_scratch &scratch, float *x_resid, bool gate_done, const float *next_norm_w,
                     float *next_cur, bool *next_done, hipStream_t stream, const float *pre_add = nullptr,
-                    const float *pre_norm_w = nullptr, void *next_xf = nullptr, int next_xf_kind = 0);
+                    const float *pre_norm_w = nullptr, void *next_xf = nullptr, int next_xf_kind = 0, float *cap = nullptr, int cap_ld = 0);
 bool dfl_moe_norm_fusable(const dflash_ctx *ctx, const dflash_model_cfg &cfg, const dflash_layer &layer, int n);
 
 // The same FFN for the rows of several consecutive 16-row blocks at once (a prompt's prefill): the rows are regrouped
@@ -363,7 +365,7 @@ int dfl_moe_group_max_picks();  // rows * picks per row that one pass takes
 bool dfl_moe_group_fits(const dflash_ctx *ctx, const dflash_model_cfg &cfg, const dflash_layer &layer, int n_rows);
 int32_t dfl_moe_ffn_group(dflash_ctx *ctx, const dflash_model_cfg &cfg, const dflash_layer &layer, float *x_resid,
                           float *cur, int n_rows, const dfl_moe_group_scratch &scratch, const float *next_norm_w, void *next_xf,
-                          int next_xf_kind, size_t next_xf_stride, hipStream_t stream);
+                          int next_xf_kind, size_t next_xf_stride, hipStream_t stream, float *cap = nullptr, int cap_ld = 0);
 
 // Residual add + RMSNorm + shared-expert gate + Q8_0 router product of a mixture-of-experts layer as one launch:
 // cur[n_rows][hidden] = rms_norm(x + add) * norm_w, gate_out[r] = sigmoid(cur[r] . gate_w),
@@ -395,6 +397,15 @@ inline int64_t dfl_attn_bucket(int64_t n_pos) {
     while (2 * b <= n_pos) b *= 2;
     return b;
 }
+// dflash_argmax_top2 whose results also go to page (a host page the device can write, as the context's pinned one; may be null): [16] indices,
+// [16] of also (null: left alone), [16] gaps.
+int32_t dfl_argmax_top2(dflash_ctx *ctx, const float *logits, int32_t n_rows, int64_t vocab, int64_t stride, int32_t *idx, float *gap,
+                        int32_t *page, const int32_t *also, hipStream_t stream);
+// dflash_select_draft_path whose tokens also go to page (as above; may be null).
+int32_t dfl_select_draft_path(dflash_ctx *ctx, const dflash_codebook *predecessor, const dflash_codebook *successor, int32_t rank, int32_t top_k,
+                              int32_t carry_token, int32_t n, const int32_t *topk_ids, const float *topk_vals, const float *sel_h, int32_t *out_tokens,
+                              int32_t *out_tokens_host, int32_t *page, dflash_stream_t stream);
+
 int32_t dfl_attn_block(dflash_ctx *ctx, const void *q, int32_t q_type, const void *k_cache, const void *v_cache,
                        int32_t v_layout, int64_t ctx_len, int32_t n_rows, int32_t n_q, int32_t n_kv, int32_t head_dim,
                        int64_t kv_capacity, float scale, float *out, dflash_stream_t stream, int32_t full_block,

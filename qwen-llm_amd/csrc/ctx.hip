@@ -74,6 +74,10 @@ int32_t dflash_ctx_create(int32_t device, size_t workspace_bytes, dflash_ctx **o
         dflash_ctx_destroy(ctx);
         return DFLASH_ERR_HIP;
     }
+    if (hipHostGetDevicePointer(&ctx->pinned_dev, ctx->pinned, 0) != hipSuccess) {
+        (void)hipGetLastError();
+        ctx->pinned_dev = nullptr;
+    }
     if (const char *e = getenv("DFLASH_GRAPHS")) ctx->graphs = atoi(e) != 0;
     if (const char *e = getenv("DFLASH_DRAFT_GRAPH")) ctx->draft_graphs = atoi(e) != 0;
     *out = ctx;

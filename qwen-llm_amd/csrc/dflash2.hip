@@ -227,7 +227,8 @@ template <bool SAMPLED>
 __global__ void __launch_bounds__(kSelThreads)
     dflash2_select_kernel(int64_t n_pred_rows, int64_t n_succ_rows, int top_k, int carry, int n, const int32_t *__restrict__ ids,
                           const float *__restrict__ table, int32_t *__restrict__ out, int32_t *__restrict__ status,
-                          float temperature, const double *__restrict__ uniforms, SampledOut *__restrict__ sampled) {
+                          float temperature, const double *__restrict__ uniforms, SampledOut *__restrict__ sampled, int32_t *page) {
+    // page (may be null): where the tokens go as well, a host page; a place the walk does not reach gets what out holds there
     __shared__ float table_s[15 * kSelMaxTopK * kSelMaxTopK];
     __shared__ int32_t ids_s[16 * kSelMaxTopK];
     __shared__ __attribute__((aligned(16))) uint8_t next_s[16][16];
@@ -243,9 +244,9 @@ __global__ void __launch_bounds__(kSelThreads)
             for (int p = 1; p < n; p++) out[p] = ids[0];  // the reference pre-fills every slot with the anchor's top-1
         }
     }
-    if (n < 2) return;
-    if (carry < 0 || carry >= n_pred_rows) {
-        if (tid == 0) *status = 1;
+    if (n < 2 || carry < 0 || carry >= n_pred_rows) {
+        if (n >= 2 && tid == 0) *status = 1;
+        if (page && tid < n) page[tid] = tid == 0 ? ids[0] : out[tid];
         return;
     }
     {
@@ -295,6 +296,7 @@ __global__ void __launch_bounds__(kSelThreads)
         const int32_t chosen = tid >= 1 && tid < n ? ids_s[tid * top_k + picked] : 0;
         const unsigned long long bad = __ballot(tid >= 1 && tid < n && (chosen < 0 || chosen >= n_pred_rows));
         const int last = bad ? __builtin_ctzll(bad) : n - 1;
+        if (page && tid < n) page[tid] = tid == 0 ? ids_s[0] : tid <= last ? chosen : out[tid];
         if (tid >= 1 && tid <= last) out[tid] = chosen;
         if (bad && tid == 0) *status = 1;
         return;
@@ -369,7 +371,7 @@ __global__ void __launch_bounds__(kSelThreads)
 template <bool SAMPLED>
 int32_t launch_walk(dflash_ctx *ctx, size_t *ws_off, const Codebook &pc, const Codebook &sc, int top_k, int rank, int carry, int n,
                     const int32_t *ids, const float *vals, const float *sel_h, int32_t *out, int32_t *status, float temperature,
-                    const double *uniforms, SampledOut *sampled, hipStream_t st) {
+                    const double *uniforms, SampledOut *sampled, hipStream_t st, int32_t *page = nullptr) {
     float *table = dfl_ws_take<float>(ctx, ws_off, static_cast<size_t>(15) * kSelMaxTopK * kSelMaxTopK * sizeof(float));
     if (!table) return dfl_fail(ctx, DFLASH_ERR_WORKSPACE, "select_draft_path: workspace too small");
     if (n > 1) {
@@ -387,7 +389,7 @@ int32_t launch_walk(dflash_ctx *ctx, size_t *ws_off, const Codebook &pc, const C
                                                                              static_cast<int>(sc.row_bytes), pc.type, sc.type, vals, table);
     }
     dflash2_select_kernel<SAMPLED><<<1, kSelThreads, 0, st>>>(pc.n_rows, sc.n_rows, top_k, carry, n, ids, table, out, status, temperature,
-                                                               uniforms, sampled);
+                                                               uniforms, sampled, page);
     DFL_HIP_CHECK(ctx, hipGetLastError());
     return DFLASH_OK;
 }
@@ -441,6 +443,13 @@ extern "C" int32_t dflash_select_draft_path(dflash_ctx *ctx, const dflash_codebo
                                             const dflash_codebook *successor, int32_t rank, int32_t top_k, int32_t carry_token,
                                             int32_t n, const int32_t *topk_ids, const float *topk_vals, const float *sel_h,
                                             int32_t *out_tokens, int32_t *out_tokens_host, dflash_stream_t stream) {
+    return dfl_select_draft_path(ctx, predecessor, successor, rank, top_k, carry_token, n, topk_ids, topk_vals, sel_h, out_tokens, out_tokens_host,
+                                 nullptr, stream);
+}
+
+int32_t dfl_select_draft_path(dflash_ctx *ctx, const dflash_codebook *predecessor, const dflash_codebook *successor, int32_t rank, int32_t top_k,
+                              int32_t carry_token, int32_t n, const int32_t *topk_ids, const float *topk_vals, const float *sel_h, int32_t *out_tokens,
+                              int32_t *out_tokens_host, int32_t *page, dflash_stream_t stream) {
     if (!ctx) return DFLASH_ERR_INVALID_INPUT;
     if (!topk_ids || !topk_vals || !sel_h || !out_tokens)
         return dfl_fail(ctx, DFLASH_ERR_INVALID_INPUT, "select_draft_path: null pointer");
@@ -455,7 +464,7 @@ extern "C" int32_t dflash_select_draft_path(dflash_ctx *ctx, const dflash_codebo
     if (!status) return dfl_fail(ctx, DFLASH_ERR_WORKSPACE, "select_draft_path: workspace too small");
     hipStream_t st = static_cast<hipStream_t>(stream);
     if ((rc = launch_walk<false>(ctx, &off, pc, sc, top_k, rank, carry_token, n, topk_ids, topk_vals, sel_h, out_tokens, status, 0.0f,
-                                 nullptr, nullptr, st)))
+                                 nullptr, nullptr, st, page)))
         return rc;
     if (out_tokens_host) {
         // the blocking form also reports an invalid predecessor row, as the reference's CPU walk does

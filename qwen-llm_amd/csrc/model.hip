@@ -44,7 +44,8 @@ __device__ float block_sum(float v, float *sh) {
 // kernel_rms_norm_batched_f32 (attn.metal:35-69), optionally preceded by the residual add that
 // feeds it (kernel_add, elementwise.metal): x += add (add may be null), then
 // y = x * rsqrt(mean(x^2) + eps) * w.  One row per workgroup; a row of up to 8192 values (n a
-// multiple of 4) is read once and stays in registers between the two passes.  y may be null where only fragment order is asked for.  With gate_w, the row's
+// multiple of 4) is read once and stays in registers between the two passes.  y may be null where only fragment order is asked for;
+// cap (may be null; rows that stay in registers only): the rows of x with add in them also go there, cap_ld floats apart.  With gate_w, the row's
 // sigmoid(y . gate_w) also goes to gate_out[row] (the shared-expert gate of a mixture-of-experts
 // layer, forward.rs:749-824: the normalised row is at hand here, in registers).  With y_xf (n a multiple of 256, at most
 // 8192: every width the whole-K GEMMs take), y also goes there as f16 in the fragment order a whole-K GEMM reads (common.h, "XF").
@@ -71,7 +72,8 @@ __global__ void __launch_bounds__(256) rms_norm_kernel(float *__restrict__ x, co
                                                        int conv_ks, const float *__restrict__ conv_dyn, const float *__restrict__ conv_base,
                                                        int conv_groups, uint32_t by_group, float *__restrict__ y, float eps,
                                                        const float *__restrict__ gate_w, float *__restrict__ gate_out, void *__restrict__ y_xf,
-                                                       int y_xf_kind, size_t xf_stride, void *__restrict__ y_xs) {
+                                                       int y_xf_kind, size_t xf_stride, void *__restrict__ y_xs, float *__restrict__ cap,
+                                                       int cap_ld) {
     typedef norm_f4 f4;
     __shared__ float sh[4], sh_dot[4];
     const int t = blockIdx.x, tid = threadIdx.x;
@@ -129,7 +131,7 @@ __global__ void __launch_bounds__(256) rms_norm_kernel(float *__restrict__ x, co
 #pragma unroll
         for (int j = 0; j < V; j++) gw[j] = *reinterpret_cast<const f4 *>(gate_w + at[j]);
     }
-    dfl_have(y, eps, gate_out, y_xf, y_xf_kind, xf_stride, y_xs);
+    dfl_have(y, eps, gate_out, y_xf, y_xf_kind, xf_stride, y_xs, cap, cap_ld);
     float s = 0.0f;
 #pragma unroll
     for (int j = 0; j < V; j++) {
@@ -144,6 +146,11 @@ __global__ void __launch_bounds__(256) rms_norm_kernel(float *__restrict__ x, co
 #pragma unroll
         for (int j = 0; j < V; j++)
             if (4 * (tid + 256 * j) < n) *reinterpret_cast<f4 *>(xr + at[j]) = v[j];
+    }
+    if (cap) {
+#pragma unroll
+        for (int j = 0; j < V; j++)
+            if (4 * (tid + 256 * j) < n) *reinterpret_cast<f4 *>(cap + static_cast<size_t>(t) * cap_ld + at[j]) = v[j];
     }
     __syncthreads();
     s = ((sh[0] + sh[1]) + sh[2]) + sh[3];
@@ -223,7 +230,8 @@ __global__ void __launch_bounds__(256) rms_norm_any_kernel(float *__restrict__ x
 }
 
 void rms_norm(int rows, hipStream_t st, float *x, const float *add, const float *w, float *y, int n, float eps, const float *gate_w,
-              float *gate_out, void *y_xf = nullptr, int y_xf_kind = 0, size_t xf_stride = 0, ConvResid conv = ConvResid(), void *y_xs = nullptr) {
+              float *gate_out, void *y_xf = nullptr, int y_xf_kind = 0, size_t xf_stride = 0, ConvResid conv = ConvResid(), void *y_xs = nullptr,
+              float *cap = nullptr, int cap_ld = 0) {
     if (!norm_in_registers(n)) {
         rms_norm_any_kernel<<<rows, 256, 0, st>>>(x, add, w, y, n, eps, gate_w, gate_out);
         return;
@@ -235,7 +243,7 @@ void rms_norm(int rows, hipStream_t st, float *x, const float *add, const float 
     do {                                                                                                                     \
         const auto fn = conv.dyn && add ? rms_norm_kernel<V, true> : rms_norm_kernel<V, false>;                              \
         fn<<<rows, 256, 0, st>>>(x, add, w, n, conv.kernel_size, conv.dyn, conv.base, groups, by_group, y, eps, gate_w, gate_out, y_xf, y_xf_kind, \
-                                 xf_stride, y_xs);                                                                           \
+                                 xf_stride, y_xs, cap, cap_ld);                                                              \
     } while (0)
     switch ((n + 1023) / 1024) {
         case 1: DFL_NORM(1); break;
@@ -475,6 +483,24 @@ __global__ void set_ids_pos_kernel(Int16Args ids, Int16Args pos, int n, int32_t 
     }
 }
 
+// A block's ids and positions to the device, as set_ids_pos_kernel, and its embedding rows, as get_rows_kernel: one launch at the head of a
+// block (1.5 + 3.0 us as two).
+__global__ void __launch_bounds__(256)
+    begin_rows_kernel(int type, const uint8_t *__restrict__ table, size_t row_bytes, int hidden, float *__restrict__ out, Int16Args ids, Int16Args pos,
+                      int32_t *__restrict__ ids_dst, int32_t *__restrict__ pos_dst, const int32_t *__restrict__ dev_ids, int vocab) {
+    const int r = blockIdx.y, e = blockIdx.x * blockDim.x + threadIdx.x;
+    int id = ids.v[r];
+    if (dev_ids && id < 0) {
+        id = dev_ids[r];
+        if (id < 0 || id >= vocab) id = 0;
+    }
+    if (e == 0) {
+        ids_dst[r] = id;
+        pos_dst[r] = pos.v[r];
+    }
+    if (e < hidden) out[static_cast<size_t>(r) * hidden + e] = dfl_dequant_elem(type, table + static_cast<size_t>(id) * row_bytes, e);
+}
+
 // The same for the rows of a prefill group, 512 token ids by value at a time: positions start, start + 1, ...
 constexpr int kMaxGroupRows = 2048;
 constexpr int kGroupIdsPerLaunch = 512;
@@ -614,7 +640,7 @@ __global__ void step_readback_kernel(const int32_t *__restrict__ argmax, const f
     const int i = threadIdx.x;
     if (i < n) {
         out[i] = argmax[i];
-        out[16 + i] = draft[i];
+        if (draft) out[16 + i] = draft[i];
         out[32 + i] = __float_as_int(gap[i]);
     }
 }
@@ -788,6 +814,25 @@ int32_t embed_rows(dflash_ctx *ctx, const dflash_qtensor &t, const int32_t *ids_
     get_rows_kernel<<<dim3(blocks_for(hidden), n), 256, 0, st>>>(t.type, static_cast<const uint8_t *>(t.data), rb, ids_dev,
                                                                hidden, out);
     return DFLASH_OK;
+}
+
+// What a block starts from, where its first launch may take it by value (no captured graph).
+struct BlockBegin {
+    Int16Args ids, pos;
+    const int32_t *dev_ids;  // (see set_ids_pos_kernel)
+};
+int32_t begin_rows(dflash_ctx *ctx, const dflash_qtensor &t, const BlockBegin &b, int n, int hidden, int vocab, float *out, int32_t *ids_dst,
+                   int32_t *pos_dst, hipStream_t st) {
+    const size_t rb = dflash_row_bytes(t.type, hidden);
+    if (rb == 0) return dfl_fail(ctx, DFLASH_ERR_UNSUPPORTED, "embedding type %d", t.type);
+    begin_rows_kernel<<<dim3(blocks_for(hidden), n), 256, 0, st>>>(t.type, static_cast<const uint8_t *>(t.data), rb, hidden, out, b.ids, b.pos, ids_dst,
+                                                                 pos_dst, b.dev_ids, vocab);
+    return DFLASH_OK;
+}
+// A few rows through a small matrix in one launch, where the public operator has one for it (whose cuts of K a prompt's products do not share).
+int32_t gemm_one(dflash_ctx *ctx, const dflash_qtensor &w, const float *x, float *y, int64_t n_in, int64_t n_out, int n, hipStream_t st) {
+    if (dfl_gemm_direct_takes(ctx, w.type, n_in, n_out)) return dfl_gemm_direct(ctx, w.type, w.data, x, DFLASH_TYPE_F32, y, n_in, n_out, n, st);
+    return gemm(ctx, w, x, y, n_in, n_out, n, st);
 }
 
 }  // namespace
@@ -1095,6 +1140,35 @@ uint64_t hash_model(const dflash_model *m) {
     return h;
 }
 
+// Where the tapped layers' residuals go.
+struct Captures {
+    const int32_t *layers;
+    int n, hidden, ld;  // ld: floats between rows
+    float *to;
+    float *next = nullptr;  // the rows that the next norm captures
+    Captures(const int32_t *tap_layers, int n_taps, float *capture, int h) : layers(tap_layers), n(n_taps), hidden(h), ld(n_taps * h), to(capture) {}
+    bool tapped(int il) const {
+        for (int t = 0; t < n; t++)
+            if (layers[t] == il) return true;
+        return false;
+    }
+    // the layer's slot where it has one alone and the kernels that have the rows in registers may write it (16-byte vectors)
+    float *own(int il) const {
+        int at = -1;
+        for (int t = 0; t < n; t++)
+            if (layers[t] == il) {
+                if (at >= 0) return nullptr;
+                at = t;
+            }
+        return at >= 0 && hidden % 4 == 0 && reinterpret_cast<uintptr_t>(to) % 16 == 0 ? to + static_cast<size_t>(at) * hidden : nullptr;
+    }
+    float *take() {
+        float *p = next;
+        next = nullptr;
+        return p;
+    }
+};
+
 // Every launch of one packed verify, from the embedding rows to the argmax, on `st`: no host
 // reads, no synchronisation, nothing that depends on the position except through pos[] on the
 // device, so the sequence can be captured once and replayed.
@@ -1106,14 +1180,18 @@ struct VerifyResume {
 };
 int32_t verify_enqueue(dflash_ctx *ctx, const dflash_model *model, dflash_session *s, int32_t n, int64_t start,
                        const int32_t *tap_layers, int32_t n_taps, float *hidden_capture, float *lg, int32_t *am, float *gp,
-                       hipStream_t st, bool want_head = true, const PrefillLane *lane = nullptr, const VerifyResume *resume = nullptr) {
+                       hipStream_t st, bool want_head = true, const PrefillLane *lane = nullptr, const VerifyResume *resume = nullptr,
+                       const BlockBegin *begin = nullptr, int32_t *page = nullptr, const int32_t *page_also = nullptr) {
     const dflash_model_cfg &c = model->cfg;
     const int H = c.hidden, hd = c.head_dim;
     const size_t q_dim = static_cast<size_t>(c.n_q) * hd, kv_dim = static_cast<size_t>(c.n_kv) * hd;
     float *const x = resume ? resume->x : s->x;
     const float *const q = resume ? resume->q : s->q;
     int32_t rc;
-    if (!resume && (rc = embed_rows(ctx, model->token_embd, s->ids, n, H, x, st))) return rc;
+    if (!resume && (rc = begin ? begin_rows(ctx, model->token_embd, *begin, n, H, c.vocab, x, s->ids, s->pos, st)
+                               : embed_rows(ctx, model->token_embd, s->ids, n, H, x, st)))
+        return rc;
+    Captures caps(tap_layers, n_taps, hidden_capture, H);
     const float scale = 1.0f / sqrtf(static_cast<float>(hd));
     const size_t per_layer = static_cast<size_t>(s->capacity) * kv_dim;
     bool cur_ready = false;  // s->cur already holds this layer's normalised input
@@ -1137,7 +1215,8 @@ int32_t verify_enqueue(dflash_ctx *ctx, const dflash_model *model, dflash_sessio
         const LayerXf xk = layer_kinds(il);
         if (!resume) {
             if (!cur_ready)
-                rms_norm(n, st, x, pending_resid, L.attn_norm, xk.qkv ? nullptr : s->cur, H, c.eps, nullptr, nullptr, xk.qkv ? s->xf_cur : nullptr, xk.qkv);
+                rms_norm(n, st, x, pending_resid, L.attn_norm, xk.qkv ? nullptr : s->cur, H, c.eps, nullptr, nullptr, xk.qkv ? s->xf_cur : nullptr, xk.qkv, 0,
+                         ConvResid(), nullptr, caps.take(), caps.ld);
             pending_resid = nullptr;
             cur_ready = false;
             bool packed;
@@ -1187,8 +1266,9 @@ int32_t verify_enqueue(dflash_ctx *ctx, const dflash_model *model, dflash_sessio
             const int next_kind = layer_kinds(il + 1).qkv;  // (the next layer's q/k/v read what this layer's last kernel normalises)
             if ((rc = dfl_moe_ffn(ctx, c, L, s->cur, n, s->moe, x, L.shexp_gate != nullptr, next_w, s->cur, &cur_ready, st,
                                   norm_in_router ? s->mix : nullptr, norm_in_router ? L.post_norm : nullptr,
-                                  next_kind ? s->xf_cur : nullptr, next_kind)))
+                                  next_kind ? s->xf_cur : nullptr, next_kind, caps.own(il), caps.ld)))
                 return rc;
+            if (cur_ready && caps.own(il)) continue;  // (its rows are captured)
         } else {
             // the down projection reads fragment-order rows only where the gate/up launch can write them
             const int down_kind = xk.gate_up ? xk.down : DFL_XF_NONE;
@@ -1204,13 +1284,14 @@ int32_t verify_enqueue(dflash_ctx *ctx, const dflash_model *model, dflash_sessio
             else
                 rc = gemm(ctx, L.down, s->g, s->mix, c.ffn, H, n, st);
             if (rc) return rc;
-            // x += mix: by the next norm, unless this layer's residual is captured first
-            bool tapped = false;
-            for (int t = 0; t < n_taps; t++) tapped = tapped || tap_layers[t] == il;
-            if (tapped)
-                add_kernel<<<blocks_for(static_cast<size_t>(n) * H), 256, 0, st>>>(x, s->mix, static_cast<size_t>(n) * H);
-            else
+            // x += mix: by the next norm, which also captures the sum; where there is none, or the layer is captured more than once, here
+            const bool norm_follows = norm_in_registers(H) && (il + 1 < c.n_layers || want_head);
+            if (!caps.tapped(il) || (caps.own(il) && norm_follows)) {
                 pending_resid = s->mix;
+                caps.next = caps.own(il);
+                continue;
+            }
+            add_kernel<<<blocks_for(static_cast<size_t>(n) * H), 256, 0, st>>>(x, s->mix, static_cast<size_t>(n) * H);
         }
         for (int t = 0; t < n_taps; t++)
             if (tap_layers[t] == il)
@@ -1219,13 +1300,13 @@ int32_t verify_enqueue(dflash_ctx *ctx, const dflash_model *model, dflash_sessio
     if (want_head) {  // (not for a caller that asked for no output of it: a prefill block wants K/V and the taps only)
         if (!cur_ready)
             rms_norm(n, st, x, pending_resid, model->output_norm, head_kind ? nullptr : s->cur, H, c.eps, nullptr, nullptr, head_kind ? s->xf_cur : nullptr,
-                     head_kind);
+                     head_kind, 0, ConvResid(), nullptr, caps.take(), caps.ld);
         if (head_kind)
             rc = dfl_gemm_whole(ctx, model->output.type, model->output.data, s->xf_cur, lg, H, c.vocab, n, 0, nullptr, DFL_XF_NONE, st);
         else
             rc = gemm(ctx, model->output, s->cur, lg, H, c.vocab, n, st);
         if (rc) return rc;
-        if ((rc = dflash_argmax_top2(ctx, lg, n, c.vocab, c.vocab, am, gp, st))) return rc;
+        if ((rc = dfl_argmax_top2(ctx, lg, n, c.vocab, c.vocab, am, gp, page, page_also, st))) return rc;
     }
     DFL_HIP_CHECK(ctx, hipGetLastError());
     return DFLASH_OK;
@@ -1237,7 +1318,7 @@ namespace {
 int32_t verify_block_impl(dflash_ctx *ctx, const dflash_model *model, dflash_session *s, const int32_t *tokens,
                           const int32_t *dev_tokens, int32_t n, int64_t start, const int32_t *tap_layers, int32_t n_taps,
                           int32_t *argmax, float *gap, float *hidden_capture, float *logits, int32_t *argmax_host,
-                          dflash_stream_t stream, bool want_head = true);
+                          dflash_stream_t stream, bool want_head = true, int32_t *page = nullptr, const int32_t *page_also = nullptr);
 }
 
 int32_t dflash_verify_block(dflash_ctx *ctx, const dflash_model *model, dflash_session *s, const int32_t *tokens,
@@ -1258,7 +1339,7 @@ namespace {
 int32_t verify_block_impl(dflash_ctx *ctx, const dflash_model *model, dflash_session *s, const int32_t *tokens,
                           const int32_t *dev_tokens, int32_t n, int64_t start, const int32_t *tap_layers, int32_t n_taps,
                           int32_t *argmax, float *gap, float *hidden_capture, float *logits, int32_t *argmax_host,
-                          dflash_stream_t stream, bool want_head) {
+                          dflash_stream_t stream, bool want_head, int32_t *page, const int32_t *page_also) {
     if (!ctx) return DFLASH_ERR_INVALID_INPUT;
     if (!model || !s || !tokens) return dfl_fail(ctx, DFLASH_ERR_INVALID_INPUT, "verify_block: null argument");
     if (const int32_t rc_ = model_tensors_checked(ctx, model)) return rc_;
@@ -1280,19 +1361,21 @@ int32_t verify_block_impl(dflash_ctx *ctx, const dflash_model *model, dflash_ses
     if (memcmp(&c, &s->cfg, sizeof(c)) != 0) return dfl_fail(ctx, DFLASH_ERR_STATE, "verify_block: session/model shape mismatch");
 
     hipStream_t st = static_cast<hipStream_t>(stream);
-    Int16Args ids_arg = {}, pos_arg = {};
+    BlockBegin begin = {{}, {}, dev_tokens};
     for (int i = 0; i < n; i++) {
-        ids_arg.v[i] = tokens[i];
-        pos_arg.v[i] = static_cast<int32_t>(start + i);
+        begin.ids.v[i] = tokens[i];
+        begin.pos.v[i] = static_cast<int32_t>(start + i);
     }
-    set_ids_pos_kernel<<<1, 64, 0, st>>>(ids_arg, pos_arg, n, s->ids, s->pos, dev_tokens, c.vocab);
     float *lg = logits ? logits : s->logits;
     int32_t *am = argmax ? argmax : s->argmax;
     float *gp = gap ? gap : s->gap;
     int32_t rc = DFLASH_OK;
     const bool use_graph = ctx->graphs && !ctx->timing && ctx->gstream;
+    // (a graph's launches read the ids from the device, and its results are read back behind it)
+    int32_t *const host_page = argmax_host && want_head && !use_graph ? static_cast<int32_t *>(ctx->pinned_dev) : nullptr;
     uint64_t key = 0;
     if (use_graph) {
+        set_ids_pos_kernel<<<1, 64, 0, st>>>(begin.ids, begin.pos, n, s->ids, s->pos, dev_tokens, c.vocab);
         key = hash_model(model);
         const uintptr_t outs[4] = {reinterpret_cast<uintptr_t>(hidden_capture), reinterpret_cast<uintptr_t>(lg),
                                    reinterpret_cast<uintptr_t>(am), reinterpret_cast<uintptr_t>(gp)};
@@ -1330,12 +1413,14 @@ int32_t verify_block_impl(dflash_ctx *ctx, const dflash_model *model, dflash_ses
         s->graph_replays++;
         DFL_HIP_CHECK(ctx, hipEventRecord(ctx->g_out, ctx->gstream));
         DFL_HIP_CHECK(ctx, hipStreamWaitEvent(st, ctx->g_out, 0));
-    } else if ((rc = verify_enqueue(ctx, model, s, n, start, tap_layers, n_taps, hidden_capture, lg, am, gp, st, want_head))) {
+    } else if ((rc = verify_enqueue(ctx, model, s, n, start, tap_layers, n_taps, hidden_capture, lg, am, gp, st, want_head, nullptr, nullptr,
+                                   use_graph ? nullptr : &begin, page ? page : host_page, page_also))) {
         return rc;
     }
+    if (page && use_graph) step_readback_kernel<<<1, 64, 0, st>>>(am, gp, page_also, n, page);
     s->kv_n_pos = start + n;
     if (argmax_host) {
-        DFL_HIP_CHECK(ctx, hipMemcpyAsync(ctx->pinned, am, n * sizeof(int32_t), hipMemcpyDeviceToHost, st));
+        if (!host_page) DFL_HIP_CHECK(ctx, hipMemcpyAsync(ctx->pinned, am, n * sizeof(int32_t), hipMemcpyDeviceToHost, st));
         DFL_HIP_CHECK(ctx, hipStreamSynchronize(st));
         memcpy(argmax_host, ctx->pinned, n * sizeof(int32_t));
     }
@@ -1518,6 +1603,7 @@ int32_t prefill_group_enqueue(dflash_ctx *ctx, const dflash_model *model, dflash
         return dfl_gemm_rows(ctx, p, w.type, w.data, xf, xs, make_sums, y, n_in, n_out, n, 0, nullptr, nullptr, 0, st);
     };
     const float *pending_resid = nullptr;  // a dense layer's FFN output still to be added to g.x
+    Captures caps(tap_layers, n_taps, hidden_capture, H);
     LayerRows rows = layer_rows(ctx, c, model->layers[0]), next_rows;
     bool last_done = false;
     for (int il = 0; il < c.n_layers; il++, rows = next_rows) {
@@ -1526,7 +1612,7 @@ int32_t prefill_group_enqueue(dflash_ctx *ctx, const dflash_model *model, dflash
         next_rows = il + 1 < c.n_layers ? layer_rows(ctx, c, model->layers[il + 1]) : LayerRows();
         if (!moe || il == 0)  // (a mixture's later layers: the experts' last kernel has normalised their input)
             rms_norm(n, st, g.x, pending_resid, L.attn_norm, nullptr, H, c.eps, nullptr, nullptr, g.xf_cur, rows.qkv.kind, xf_h, ConvResid(),
-                     rows.qkv.sums ? g.xs_cur : nullptr);
+                     rows.qkv.sums ? g.xs_cur : nullptr, caps.take(), caps.ld);
         pending_resid = nullptr;
         if ((rc = product(rows.qkv, L.wq, g.xf_cur, g.xs_cur, moe && il, g.pk, H, tot))) return rc;
         group_norm_rope(hd, st, g.pk, tot, g.q, L.q_norm, L.k_norm, kc, start, n, c.n_q, c.n_kv, c.eps, c.rope_theta, vtc, s->capacity);
@@ -1544,8 +1630,10 @@ int32_t prefill_group_enqueue(dflash_ctx *ctx, const dflash_model *model, dflash
             // x += mix, the experts' norm and the shared-expert gates: the block path's norm kernel over all the rows
             rms_norm(n, st, g.x, g.mix, L.post_norm, g.cur, H, c.eps, L.shexp_gate, g.moe.sg);
             if ((rc = dfl_moe_ffn_group(ctx, c, L, g.x, g.cur, n, g.moe, next_w, next_rows.qkv.kind ? g.xf_cur : nullptr, next_rows.qkv.kind, xf_h,
-                                        st)))
+                                        st,
+                                        caps.own(il), caps.ld)))
                 return rc;
+            if (caps.own(il)) continue;  // (its rows are captured)
         } else {
             rms_norm(n, st, g.x, g.mix, L.post_norm, nullptr, H, c.eps, nullptr, nullptr, g.xf_cur, rows.gate_up.kind, xf_h, ConvResid(),
                      rows.gate_up.sums ? g.xs_cur : nullptr);
@@ -1555,10 +1643,13 @@ int32_t prefill_group_enqueue(dflash_ctx *ctx, const dflash_model *model, dflash
                 return rc;
             if ((rc = dfl_gemm_rows(ctx, rows.down, L.down.type, L.down.data, g.xf_g, g.xs_g, false, g.mix, c.ffn, H, n, 0, nullptr, nullptr, 0, st)))
                 return rc;
-            if (tapped)  // (the residual is captured below; else the next norm adds it)
-                add_kernel<<<blocks_for(static_cast<size_t>(n) * H), 256, 0, st>>>(g.x, g.mix, static_cast<size_t>(n) * H);
-            else
+            // the next norm adds the residual and captures the sum, where there is one and the layer is captured once
+            if (!tapped || (caps.own(il) && il + 1 < c.n_layers)) {
                 pending_resid = g.mix;
+                caps.next = caps.own(il);
+                continue;
+            }
+            add_kernel<<<blocks_for(static_cast<size_t>(n) * H), 256, 0, st>>>(g.x, g.mix, static_cast<size_t>(n) * H);
         }
         for (int t = 0; t < n_taps; t++)
             if (tap_layers[t] == il)
@@ -1568,7 +1659,8 @@ int32_t prefill_group_enqueue(dflash_ctx *ctx, const dflash_model *model, dflash
     if (!with_head) return DFLASH_OK;
     const int first = (n - 1) / 16 * 16;  // of the last block
     const VerifyResume resume = {g.x + static_cast<size_t>(first) * H, last_done ? nullptr : g.q + static_cast<size_t>(first) * q_dim};
-    return verify_enqueue(ctx, model, s, n - first, start + first, nullptr, 0, nullptr, s->logits, s->argmax, s->gap, st, true, nullptr, &resume);
+    return verify_enqueue(ctx, model, s, n - first, start + first, nullptr, 0, nullptr, s->logits, s->argmax, s->gap, st, true, nullptr, &resume, nullptr,
+                          static_cast<int32_t *>(ctx->pinned_dev));
 }
 
 }  // namespace
@@ -1606,14 +1698,14 @@ int32_t dflash_prefill_blocks(dflash_ctx *ctx, const dflash_model *model, dflash
     if (!s->pipe && (rc = prefill_pipe_create(ctx, s))) return rc;
     PrefillPipe *p = s->pipe;
     if (n_tokens <= 16) {  // a lone block: the verify's own launches, without its head
-        Int16Args ids_arg = {}, pos_arg = {};
+        BlockBegin begin = {};
         for (int i = 0; i < n_tokens; i++) {
-            ids_arg.v[i] = tokens[i];
-            pos_arg.v[i] = static_cast<int32_t>(start + i);
+            begin.ids.v[i] = tokens[i];
+            begin.pos.v[i] = static_cast<int32_t>(start + i);
         }
         hipStream_t st = static_cast<hipStream_t>(stream);
-        set_ids_pos_kernel<<<1, 64, 0, st>>>(ids_arg, pos_arg, n_tokens, s->ids, s->pos, nullptr, c.vocab);
-        if ((rc = verify_enqueue(ctx, model, s, n_tokens, start, tap_layers, n_taps, hidden_capture, s->logits, s->argmax, s->gap, st, false))) {
+        if ((rc = verify_enqueue(ctx, model, s, n_tokens, start, tap_layers, n_taps, hidden_capture, s->logits, s->argmax, s->gap, st, false, nullptr,
+                                 nullptr, &begin))) {
             (void)hipStreamSynchronize(st);
             return rc;
         }
@@ -1664,16 +1756,15 @@ int32_t dflash_prefill_blocks(dflash_ctx *ctx, const dflash_model *model, dflash
         const int lane_i = block % n_lanes, prev_i = (block + n_lanes - 1) % n_lanes;
         const int32_t n = std::min<int32_t>(16, n_tokens - t0);
         dflash_session *ls = lanes_s[lane_i];
-        Int16Args ids_arg = {}, pos_arg = {};
+        BlockBegin begin = {};
         for (int i = 0; i < n; i++) {
-            ids_arg.v[i] = tokens[t0 + i];
-            pos_arg.v[i] = static_cast<int32_t>(start + t0 + i);
+            begin.ids.v[i] = tokens[t0 + i];
+            begin.pos.v[i] = static_cast<int32_t>(start + t0 + i);
         }
-        set_ids_pos_kernel<<<1, 64, 0, lanes_st[lane_i]>>>(ids_arg, pos_arg, n, ls->ids, ls->pos, nullptr, c.vocab);
         const PrefillLane lane = {p->kv_done[lane_i].data(), p->kv_done[prev_i].data(), block > 0 && n_lanes > 1};
         rc = verify_enqueue(lanes_ctx[lane_i], model, ls, n, start + t0, tap_layers, n_taps,
                             hidden_capture ? hidden_capture + static_cast<size_t>(t0) * cap_row : nullptr, ls->logits, ls->argmax, ls->gap,
-                            lanes_st[lane_i], false, &lane);
+                            lanes_st[lane_i], false, &lane, nullptr, &begin);
         if (rc && lane_i > 0) rc = dfl_fail(ctx, rc, "prefill_blocks: %s", dflash_last_error(lanes_ctx[lane_i]));
     }
     ctx->batch_wgs = owner_wgs;
@@ -1727,13 +1818,13 @@ int32_t dflash_prefill_prompt(dflash_ctx *ctx, const dflash_model *model, dflash
     }
     rc = prefill_group_enqueue(ctx, model, s, g, tokens + body, n, start + body, tap_layers, n_taps, capture(body), st, true);
     hipError_t err = hipSuccess;
-    if (!rc) err = hipMemcpyAsync(ctx->pinned, s->argmax + (n - 1) % 16, sizeof(int32_t), hipMemcpyDeviceToHost, st);
+    if (!rc && !ctx->pinned_dev) err = hipMemcpyAsync(ctx->pinned, s->argmax, 16 * sizeof(int32_t), hipMemcpyDeviceToHost, st);
     const hipError_t done = hipStreamSynchronize(st);
     if (rc || err != hipSuccess || done != hipSuccess) {
         s->kv_n_pos = start;
         return rc ? rc : dfl_fail(ctx, DFLASH_ERR_HIP, "prefill_prompt: %s", hipGetErrorString(err != hipSuccess ? err : done));
     }
-    memcpy(last_argmax_host, ctx->pinned, sizeof(int32_t));
+    *last_argmax_host = static_cast<const int32_t *>(ctx->pinned)[(n - 1) % 16];
     s->kv_n_pos = start + n_tokens;
     return DFLASH_OK;
 }
@@ -1857,7 +1948,7 @@ int32_t draft_prepare(dflash_ctx *ctx, const dflash_draft_head *head, dflash_dra
     if (s->ctx_h_ready >= s->ctx_len && s->kv_ready >= s->ctx_len) return DFLASH_OK;
     for (int64_t c0 = s->ctx_h_ready; c0 < s->ctx_len; c0 += 16) {
         const int m = static_cast<int>(std::min<int64_t>(16, s->ctx_len - c0));
-        if ((rc = gemm(ctx, head->fc, s->ctx_raw + c0 * feat, s->tmp, feat, H, m, st))) return rc;
+        if ((rc = gemm_one(ctx, head->fc, s->ctx_raw + c0 * feat, s->tmp, feat, H, m, st))) return rc;
         rms_norm(m, st, s->tmp, nullptr, head->hidden_norm, s->ctx_h + c0 * H, H, c.eps, nullptr, nullptr);
     }
     // Every layer's K/V projection reads the same rows (ctx_h): when the layers' [wk; wv] pairs are Q4_K matrices
@@ -2004,20 +2095,24 @@ int32_t draft_block_impl(dflash_ctx *ctx, const dflash_model *target, const dfla
     // phase 1 and the context K/V of the new columns (a no-op if dflash_draft_prepare_ctx ran)
     if ((rc = draft_prepare(ctx, head, s, fast, st))) return rc;
     // phase 2: noise embedding
-    Int16Args ids_arg = {}, pos_arg = {};
+    BlockBegin begin = {};
     for (int i = 0; i < N; i++) {
-        ids_arg.v[i] = i == 0 ? carry : mask_token;
-        pos_arg.v[i] = static_cast<int32_t>(noise_start + i);
+        begin.ids.v[i] = i == 0 ? carry : mask_token;
+        begin.pos.v[i] = static_cast<int32_t>(noise_start + i);
     }
-    set_ids_pos_kernel<<<1, 64, 0, st>>>(ids_arg, pos_arg, N, s->ids, s->pos, nullptr, 0);
+    bool by_value = true;  // (a graph's launches read the ids from the device)
     float *lg = draft_logits ? draft_logits : s->logits;
     int32_t *am = draft_argmax ? draft_argmax : s->argmax;
+    // the walk's tokens go straight to the host's page where the caller waits for them (a walk is never in a graph)
+    int32_t *const walk_page = argmax_host && c.selector_rank > 0 && !skip_selector_walk ? static_cast<int32_t *>(ctx->pinned_dev) : nullptr;
     // Everything from the noise embedding to the argmax, on stream `st`: the launches depend on the call only through
     // device memory (ids, pos; the attention reads the context length from pos[0]) - except the DFlash-2 selector
     // walk, which takes the carry by value - so they can be captured once and replayed.
     auto enqueue = [&](hipStream_t st) -> int32_t {
     int32_t rc;
-    if ((rc = embed_rows(ctx, target->token_embd, s->ids, N, H, s->x, st))) return rc;
+    if ((rc = by_value ? begin_rows(ctx, target->token_embd, begin, N, H, V, s->x, s->ids, s->pos, st)
+                       : embed_rows(ctx, target->token_embd, s->ids, N, H, s->x, st)))
+        return rc;
 
     const float *pending_resid = nullptr;
     // DFlash-2: the side-1 convolution of a sublayer's output is what gets added to the residual; the norm kernel that
@@ -2158,10 +2253,10 @@ int32_t draft_block_impl(dflash_ctx *ctx, const dflash_model *target, const dfla
         // row, the selector gate W_h . h of the output-normed hidden, and the predecessor-conditioned
         // walk, all on the device
         if ((rc = dflash_top16(ctx, lg, N, V, V, s->topk_ids, s->topk_vals, st))) return rc;
-        if ((rc = gemm(ctx, head->selector_hidden, s->cur, s->sel_h, H, c.selector_rank, N, st))) return rc;
+        if ((rc = gemm_one(ctx, head->selector_hidden, s->cur, s->sel_h, H, c.selector_rank, N, st))) return rc;
         if (!skip_selector_walk &&
-            (rc = dflash_select_draft_path(ctx, &head->selector_predecessor, &head->selector_successor, c.selector_rank,
-                                           c.selector_top_k, carry, N, s->topk_ids, s->topk_vals, s->sel_h, am, nullptr, st)))
+            (rc = dfl_select_draft_path(ctx, &head->selector_predecessor, &head->selector_successor, c.selector_rank, c.selector_top_k, carry, N,
+                                        s->topk_ids, s->topk_vals, s->sel_h, am, nullptr, walk_page, st)))
             return rc;
     } else if ((rc = dflash_argmax_greedy(ctx, lg, N, V, V, am, st))) {
         return rc;
@@ -2178,7 +2273,9 @@ int32_t draft_block_impl(dflash_ctx *ctx, const dflash_model *target, const dfla
     const bool walk_by_value = c.selector_rank > 0 && !skip_selector_walk;
     const bool use_graph = ctx->draft_graphs && fast && !walk_by_value && !ctx->timing && ctx->gstream;
     uint64_t key = 0;
+    by_value = !use_graph;
     if (use_graph) {
+        set_ids_pos_kernel<<<1, 64, 0, st>>>(begin.ids, begin.pos, N, s->ids, s->pos, nullptr, 0);
         key = hash_model(target);
         const uintptr_t ptrs[6] = {reinterpret_cast<uintptr_t>(head->layers), reinterpret_cast<uintptr_t>(head->fc.data),
                                    reinterpret_cast<uintptr_t>(head->output_norm), reinterpret_cast<uintptr_t>(lg),
@@ -2231,7 +2328,7 @@ int32_t draft_block_impl(dflash_ctx *ctx, const dflash_model *target, const dfla
     s->ctx_h_ready = s->ctx_len;
     s->kv_ready = s->ctx_len;
     if (argmax_host) {
-        DFL_HIP_CHECK(ctx, hipMemcpyAsync(ctx->pinned, am, N * sizeof(int32_t), hipMemcpyDeviceToHost, st));
+        if (!walk_page) DFL_HIP_CHECK(ctx, hipMemcpyAsync(ctx->pinned, am, N * sizeof(int32_t), hipMemcpyDeviceToHost, st));
         DFL_HIP_CHECK(ctx, hipStreamSynchronize(st));
         memcpy(argmax_host, ctx->pinned, N * sizeof(int32_t));
     }
@@ -2475,20 +2572,14 @@ int32_t dflash_spec_step(dflash_ctx *ctx, const dflash_model *target, const dfla
         for (int i = 1; i < N; i++) tokens_in[i] = (draft_override && draft_override[i - 1] >= 0) ? draft_override[i - 1] : -1;
         const double enqueue_draft_ms = ms_since(t0);
         t0 = std::chrono::steady_clock::now();
-        if ((rc = verify_block_impl(ctx, target, sess, tokens_in, dsess->argmax, N, position, taps, n_taps, nullptr, nullptr,
-                                    sess->hidden, nullptr, nullptr, st)))
-            return undo(rc);
-        if (timed) STEP_HIP(hipEventRecord(ctx->ev1, st));
-        // read back through the context's pinned page, one wait
+        // read back through the context's pinned page, one wait (the verify's last launch writes it, the drafts with it)
         int32_t *pin_argmax = static_cast<int32_t *>(ctx->pinned), *pin_draft = pin_argmax + 16;
         float *pin_gap = reinterpret_cast<float *>(pin_argmax + 32);
-        void *pinned_dev = nullptr;
-        if (hipHostGetDevicePointer(&pinned_dev, ctx->pinned, 0) == hipSuccess && pinned_dev) {
-            // (one launch that writes the pinned page directly instead of three copy commands)
-            step_readback_kernel<<<1, 64, 0, st>>>(sess->argmax, sess->gap, dsess->argmax, N, static_cast<int32_t *>(pinned_dev));
-            STEP_HIP(hipGetLastError());
-        } else {
-            (void)hipGetLastError();
+        if ((rc = verify_block_impl(ctx, target, sess, tokens_in, dsess->argmax, N, position, taps, n_taps, nullptr, nullptr,
+                                    sess->hidden, nullptr, nullptr, st, true, static_cast<int32_t *>(ctx->pinned_dev), dsess->argmax)))
+            return undo(rc);
+        if (timed) STEP_HIP(hipEventRecord(ctx->ev1, st));
+        if (!ctx->pinned_dev) {
             STEP_HIP(hipMemcpyAsync(pin_argmax, sess->argmax, N * sizeof(int32_t), hipMemcpyDeviceToHost, st));
             STEP_HIP(hipMemcpyAsync(pin_gap, sess->gap, N * sizeof(float), hipMemcpyDeviceToHost, st));
             STEP_HIP(hipMemcpyAsync(pin_draft, dsess->argmax, N * sizeof(int32_t), hipMemcpyDeviceToHost, st));

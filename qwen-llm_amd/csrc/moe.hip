@@ -379,7 +379,8 @@ __global__ void __launch_bounds__(256)
                             const float *__restrict__ sg, const float *__restrict__ shared, const int32_t *__restrict__ n_slots,
                             int n_used, int hidden, float *__restrict__ x, const float *__restrict__ norm_w,
                             float *__restrict__ y, float eps, const float *__restrict__ pre_add, void *__restrict__ y_xf,
-                            int y_xf_kind, size_t xf_stride) {
+                            int y_xf_kind, size_t xf_stride, float *__restrict__ cap, int cap_ld) {
+    // (y: null where the rows go to fragment order; cap: the new residual's rows go there as well, cap_ld floats apart)
     typedef float f4 __attribute__((ext_vector_type(4)));
     __shared__ float sh[4];
     const int row = blockIdx.x, tid = threadIdx.x;
@@ -418,7 +419,7 @@ __global__ void __launch_bounds__(256)
                 if (pre_add) pre[j] = *reinterpret_cast<const f4 *>(pre_add + row_at + at[j]);
                 nw[j] = *reinterpret_cast<const f4 *>(norm_w + at[j]);
             }
-            dfl_have(y, eps, y_xf, y_xf_kind, xf_stride);
+            dfl_have(y, eps, y_xf, y_xf_kind, xf_stride, cap, cap_ld);
         }
 #pragma unroll
         for (int k = 0; k < 8; k++) {
@@ -442,7 +443,10 @@ __global__ void __launch_bounds__(256)
     if ((tid & 63) == 0) sh[tid >> 6] = s;
 #pragma unroll
     for (int j = 0; j < V; j++)
-        if (4 * (tid + 256 * j) < hidden) *reinterpret_cast<f4 *>(x + row_at + at[j]) = v[j];
+        if (4 * (tid + 256 * j) < hidden) {
+            *reinterpret_cast<f4 *>(x + row_at + at[j]) = v[j];
+            if (cap) *reinterpret_cast<f4 *>(cap + static_cast<size_t>(row) * cap_ld + at[j]) = v[j];
+        }
     __syncthreads();
     s = ((sh[0] + sh[1]) + sh[2]) + sh[3];
     const float scale = 1.0f / sqrtf(s / static_cast<float>(hidden) + eps);
@@ -451,7 +455,7 @@ __global__ void __launch_bounds__(256)
         const int i = 4 * (tid + 256 * j);
         if (i < hidden) {
             const f4 o = v[j] * scale * nw[j];
-            *reinterpret_cast<f4 *>(y + row_at + i) = o;
+            if (y) *reinterpret_cast<f4 *>(y + row_at + i) = o;
             // (hidden a multiple of 256 here: whole waves are inside or outside the row)
             if (y_xf)
                 dfl_xf_store_pair(static_cast<uint8_t *>(y_xf) + (row >> 4) * xf_stride, y_xf_kind, row & 15, i & ~7, o[0], o[1], o[2], o[3]);
@@ -461,11 +465,11 @@ __global__ void __launch_bounds__(256)
 
 void moe_combine_norm(int rows, hipStream_t st, const float *eo, const int32_t *slot_of, const float *sel_w, const float *sg, const float *shared,
                       const int32_t *n_slots, int n_used, int hidden, float *x, const float *norm_w, float *y, float eps, const float *pre_add,
-                      void *y_xf, int y_xf_kind, bool grouped = false, size_t xf_stride = 0) {
+                      void *y_xf, int y_xf_kind, bool grouped, size_t xf_stride, float *cap, int cap_ld) {
 #define DFL_COMBINE(V) (grouped ? moe_combine_norm_kernel<V, true> : moe_combine_norm_kernel<V, false>)
     const auto fn = hidden <= 1024 ? DFL_COMBINE(1) : hidden <= 2048 ? DFL_COMBINE(2) : DFL_COMBINE(4);
 #undef DFL_COMBINE
-    fn<<<rows, 256, 0, st>>>(eo, slot_of, sel_w, sg, shared, n_slots, n_used, hidden, x, norm_w, y, eps, pre_add, y_xf, y_xf_kind, xf_stride);
+    fn<<<rows, 256, 0, st>>>(eo, slot_of, sel_w, sg, shared, n_slots, n_used, hidden, x, norm_w, y_xf ? nullptr : y, eps, pre_add, y_xf, y_xf_kind, xf_stride, cap, cap_ld);
 }
 
 // ---- rows of several 16-row blocks through one pass over the experts (prefill) ----
@@ -643,7 +647,7 @@ bool dfl_moe_norm_fusable(const dflash_ctx *ctx, const dflash_model_cfg &c, cons
 
 int32_t dfl_moe_ffn(dflash_ctx *ctx, const dflash_model_cfg &c, const dflash_layer &L, float *cur, int n,
                     const dfl_moe_scratch &s, float *x_resid, bool gate_done, const float *next_norm_w, float *next_cur,
-                    bool *next_done, hipStream_t st, const float *pre_add, const float *pre_norm_w, void *next_xf, int next_xf_kind) {
+                    bool *next_done, hipStream_t st, const float *pre_add, const float *pre_norm_w, void *next_xf, int next_xf_kind, float *cap, int cap_ld) {
     if (next_done) *next_done = false;
     if ((pre_add != nullptr) != (pre_norm_w != nullptr) ||
         (pre_add && !(next_norm_w && next_cur && next_done && dfl_moe_norm_fusable(ctx, c, L, n))))
@@ -761,7 +765,7 @@ int32_t dfl_moe_ffn(dflash_ctx *ctx, const dflash_model_cfg &c, const dflash_lay
     if (batched && next_norm_w && next_cur && next_done && H <= 4096 && H % 4 == 0) {
         moe_combine_norm(n, st, s.eo, s.slot_of, s.sel_w, s.sg, folded_shared ? nullptr : s.shared, s.n_distinct,
                                                    used, H, x_resid, next_norm_w, next_cur, c.eps, pre_add,
-                                                   H % DFL_QK_K == 0 ? next_xf : nullptr, next_xf_kind);
+                                                   H % DFL_QK_K == 0 ? next_xf : nullptr, next_xf_kind, false, 0, cap, cap_ld);
         *next_done = true;
     } else if (batched)
         moe_combine_slots_kernel<<<dim3((H + 255) / 256, n), 256, 0, st>>>(s.eo, s.slot_of, s.sel_w, s.sg,
@@ -796,7 +800,7 @@ bool dfl_moe_group_fits(const dflash_ctx *ctx, const dflash_model_cfg &c, const 
 
 int32_t dfl_moe_ffn_group(dflash_ctx *ctx, const dflash_model_cfg &c, const dflash_layer &L, float *x_resid,
                           float *cur, int n_rows, const dfl_moe_group_scratch &s, const float *next_norm_w, void *next_xf,
-                          int next_xf_kind, size_t next_xf_stride, hipStream_t st) {
+                          int next_xf_kind, size_t next_xf_stride, hipStream_t st, float *cap, int cap_ld) {
     if (!dfl_moe_group_fits(ctx, c, L, n_rows) || !x_resid || !cur || !next_norm_w)
         return dfl_fail(ctx, DFLASH_ERR_UNSUPPORTED, "moe group: layer or row count (%d) not taken", n_rows);
     const int E = c.n_expert, used = c.n_expert_used < E ? c.n_expert_used : E, H = c.hidden, fe = c.ffn_expert;
@@ -833,7 +837,7 @@ int32_t dfl_moe_ffn_group(dflash_ctx *ctx, const dflash_model_cfg &c, const dfla
                                     max_tiles, tile_slots, s.eo, fe, H, nullptr, nullptr, st)))
         return rc;
     moe_combine_norm(n_rows, st, s.eo, s.pick_pos, s.sel_w, s.sg, nullptr, s.n_slots, used, H, x_resid, next_norm_w,
-                                                    cur, c.eps, nullptr, next_xf, next_xf_kind, true, next_xf_stride);
+                                                    cur, c.eps, nullptr, next_xf, next_xf_kind, true, next_xf_stride, cap, cap_ld);
     DFL_HIP_CHECK(ctx, hipGetLastError());
     return DFLASH_OK;
 }

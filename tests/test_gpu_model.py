@@ -590,3 +590,40 @@ def test_graph_replay_is_bit_identical_to_launch_by_launch(ctx, target):
         for x, y, name in zip(a, b, ("logits", "hidden", "argmax", "gap")):
             assert np.array_equal(x.view(np.uint32) if x.dtype == np.float32 else x,
                                   y.view(np.uint32) if y.dtype == np.float32 else y), f"call {i}: {name} differs under graph replay"
+
+
+@pytest.mark.parametrize("kind", ["dense", "moe"])
+def test_captured_rows_by_the_norms_equal_those_of_their_own_launch(ctx, kind):
+    """A tapped layer's residual is written by the kernel that has its rows in registers (the next norm, or the experts' combine); tapped
+    twice, or into a buffer that is not 16-byte aligned, by a launch of its own; the last layer's too, with and without the head: the same rows."""
+    import ctypes as C
+    import torch
+
+    cfg = (dfl.ModelConfig(n_layers=3, hidden=512, n_q=4, n_kv=2, head_dim=128, ffn=512, vocab=1024) if kind == "dense" else
+           dfl.ModelConfig(n_layers=3, hidden=512, n_q=4, n_kv=2, head_dim=128, ffn=0, vocab=1024, n_expert=8, n_expert_used=2, ffn_expert=256, ffn_shared=256))
+    model = dfl.TargetModel(ctx, cfg, dfl.synth_target_weights_blocks(cfg, 9))
+    tokens = np.random.default_rng(5).integers(0, cfg.vocab, 40).tolist()
+    rows = {}
+    for name, taps, offset, head in (("own", [0, 1, 2], 0, True), ("off", [0, 1, 2], 1, True), ("twice", [0, 0, 1, 2], 0, True), ("no head", [0, 1, 2], 0, False)):
+        sess = dfl.Session(ctx, model, 64, taps)
+        n_taps, n = len(taps), 13
+        buf = torch.zeros(n * n_taps * cfg.hidden + 4, device="cuda")
+        arg = torch.zeros(16, dtype=torch.int32, device="cuda")
+        host = (C.c_int32 * 16)()
+        rc = sess._L.dflash_verify_block(ctx._h, C.byref(model.c), sess._h, (C.c_int32 * n)(*tokens[:n]), n, 0, (C.c_int32 * n_taps)(*taps), n_taps,
+                                         arg.data_ptr() if head else None, None, buf.data_ptr() + 4 * offset, None, host if head else None, None)
+        assert rc == 0
+        torch.cuda.synchronize()
+        got = buf[offset:offset + n * n_taps * cfg.hidden].view(n, n_taps, cfg.hidden)
+        if head:
+            assert list(host[:n]) == arg[:n].tolist()
+        if name == "twice":
+            assert torch.equal(got[:, 0], got[:, 1])
+            got = got[:, 1:]
+        rows[name] = got.clone()
+        # a prompt's group: the same rows, and a buffer off the alignment
+        many = sess.prefill_prompt(tokens[n:], n)[0]
+        rows[name + " group"] = many[:, 1:] if name == "twice" else many
+        sess.close()
+    for name in ("off", "twice", "no head"):
+        assert torch.equal(rows["own"], rows[name]) and torch.equal(rows["own group"], rows[name + " group"]), name
