@@ -33,7 +33,7 @@ NO_SCRATCH_BY_FILE = {
     "gemm_fewrow.hip": ("gemm_q4k_stream_kernel", "gemm_q4k_slab_kernel", "gemm_q4k_tiled_kernel", "gemm_q4k_experts_kernel",
                         "gemm_q4k_few_slots_kernel", "gemm_q6k_stream_kernel"),
     "gemm_whole.hip": ("gemm_q6t_loop_kernel", "gemm_q4k_wide_kernel"),
-    "attn_verify.hip": ("attn_split_kernel", "attn_rows_kernel", "attn_rows_pair_kernel"),
+    "attn_verify.hip": ("attn_split_kernel", "attn_split_rope_kernel", "attn_rows_kernel", "attn_rows_pair_kernel"),
     "gemm_rows.hip": ("gemm_rows_kernel",),
     "gemm_dense.hip": ("gemm_q4k_dense_pair_kernel",),
 }

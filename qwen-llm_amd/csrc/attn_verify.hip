@@ -26,6 +26,7 @@
 //  * each workgroup writes (m, l, O) partials; a second small kernel merges the splits.
 #include "common.h"
 #include "lds_read.h"
+#include "rope_head.h"
 
 #include <cmath>
 #include <algorithm>
@@ -168,6 +169,153 @@ __device__ __forceinline__ void attn_store_xf(float4_t (&tot)[DT], void *out_xf,
     }
 }
 
+// ROPE: the block's rows come as the projections leave them, [row][query heads | key heads | value heads] in f32.  A wave norms and
+// rotates its head's queries in registers; where a workgroup's keys reach into the block, two waves more make the block's keys and
+// values of its KV head, put them over what the cache still holds there in LDS, and (in the first part of a group) into the
+// cache.  Elsewhere those two waves end at once.  The arithmetic is that of qk_norm_rope_kernel, bit for bit; sines and cosines
+// come from a table of the block, [row][cosines, sines], made once a block, which waits with the norm's weights in the ring's last
+// buffer, ahead of the stage that comes there.
+// What bounds it: the launch of the rotation was one trip to memory with little to do; here that trip is the one the first stages
+// are on anyway, and what is left is 450 vector instructions a wave ahead of the first scores (heads of 256).  Rotation and attention,
+// behind 2 k of context: 16 rows of 16 / 2 heads of 256 3.9 + 11.2 -> 12.5 us, one row 3.5 + 7.9 -> 9.6, 16 rows of 32 / 8 heads
+// of 128 4.9 + 7.7 -> 9.4.  (The block's keys and values by the heads' waves, behind their queries: 14.0, 10.5 and 10.5; by one wave of
+// a workgroup of one, through LDS: 12 us more a launch.)
+struct AttnRope {
+    const float *table, *q_w, *k_w;
+    float eps;
+};
+// A lane of an MFMA's query operand holds elements 32 s + 8 g + j of head row n in r[s][j]: the sum of squares over the row in the order
+// of RopeHead (chains of the elements 64 apart, then lanes 32, 16, 8, 4, 2, 1 apart, of which the first and the last three are this
+// lane's own elements here): the same bits.
+template <int KS>
+__device__ __forceinline__ float attn_row_squares(const float (&r)[KS][8]) {
+    float t[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+        float c0 = r[0][j] * r[0][j], c1 = r[1][j] * r[1][j];
+#pragma unroll
+        for (int k = 1; k < KS / 2; k++) {
+            c0 = __builtin_fmaf(r[2 * k][j], r[2 * k][j], c0);
+            c1 = __builtin_fmaf(r[2 * k + 1][j], r[2 * k + 1][j], c1);
+        }
+        if constexpr (KS == 2) asm volatile("" : "+v"(c0), "+v"(c1));  // (a product and a sum, two roundings: the sum there crosses lanes)
+        t[j] = c0 + c1;
+    }
+    // (elements 16 apart are lanes 32 apart, elements 8 apart lanes 16 apart; j ^ 1 then sits in the other half of the wave, j ^ 2 in
+    // the other half of that)
+    float u[4], w[2];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        dfl_swap32(t[2 * i], t[2 * i + 1]);
+        u[i] = t[2 * i] + t[2 * i + 1];
+    }
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        dfl_swap16(u[2 * i], u[2 * i + 1]);
+        w[i] = u[2 * i] + u[2 * i + 1];
+    }
+    float v = w[0] + w[1], a = v, b = v;
+    dfl_swap16(a, b);
+    v = a + b;
+    a = v, b = v;
+    dfl_swap32(a, b);
+    return a + b;
+}
+// ... and its norm and rotation: tab(c), w(c) are the 16-byte chunk c of the row's cosines and sines, and of the weights; put(s, j, value).
+template <int KS, typename Tab, typename W, typename Put>
+__device__ __forceinline__ void attn_rotate(const float (&r)[KS][8], int g, float eps, Tab tab, W w, Put put) {
+    constexpr int kHalf = 4 * KS;  // chunks of half a head
+    const float by = dfl_head_scale<32 * KS>(attn_row_squares<KS>(r), eps);
+#pragma unroll
+    for (int s = 0; s < KS / 2; s++)
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+            const int c = 8 * s + 2 * g + e;
+            const float4_t cs = tab(c), sn = tab(kHalf + c), wa = w(c), wb = w(kHalf + c);
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                float ra, rb;
+                dfl_rope_pair(r[s][4 * e + i] * by * wa[i], r[s + KS / 2][4 * e + i] * by * wb[i], sn[i], cs[i], ra, rb);
+                put(s, 4 * e + i, ra);
+                put(s + KS / 2, 4 * e + i, rb);
+            }
+        }
+}
+// The wave that makes the block's keys (values: VALUES) of one KV head: row: this lane's row of that head, table and weights in memory;
+// tiles: the ring; cache: key 0 of the split (null: another workgroup writes it).  Keeps the other waves' barriers.
+template <int HD, bool VALUES>
+__device__ __forceinline__ void attn_new_rows(const float *__restrict__ row, const float *__restrict__ table, const float *__restrict__ w, float eps,
+                                              int n_rows, int first_new, int n_keys, int n_steps, half8_t *ring, _Float16 *cache, int64_t stride) {
+    constexpr int KS = HD / 32, CH = HD / 8, kKPieces = 32 * CH;
+    const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
+    float r[KS][8];
+#pragma unroll
+    for (int s = 0; s < KS; s++)
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+            const float4_t x = *reinterpret_cast<const float4_t *>(row + 32 * s + 8 * g + 4 * e);
+#pragma unroll
+            for (int i = 0; i < 4; i++) r[s][4 * e + i] = x[i];
+        }
+    __builtin_amdgcn_s_barrier();  // (the others': what they asked for ahead of the stages is there)
+    half8_t out[KS];
+    if constexpr (VALUES) {
+#pragma unroll
+        for (int s = 0; s < KS; s++)
+#pragma unroll
+            for (int j = 0; j < 8; j++) out[s][j] = static_cast<_Float16>(r[s][j]);
+    } else {
+        // (asked for along with the row, in one trip to memory)
+        const float4_t *t = reinterpret_cast<const float4_t *>(table) + min(n, n_rows - 1) * (HD / 4), *wt = reinterpret_cast<const float4_t *>(w);
+        float4_t tv[2 * KS], wv[2 * KS];
+#pragma unroll
+        for (int i = 0; i < 2 * KS; i++) tv[i] = t[8 * (i >> 1) + 2 * g + (i & 1)];
+#pragma unroll
+        for (int i = 0; i < 2 * KS; i++) wv[i] = wt[8 * (i >> 1) + 2 * g + (i & 1)];
+#pragma unroll
+        for (int i = 0; i < 2 * KS; i++) asm volatile("" : "+v"(tv[i]), "+v"(wv[i]));
+        attn_rotate<KS>(r, g, eps, [&](int c) { return tv[(c - 2 * g) / 8 * 2 + (c - 2 * g) % 8]; },
+                        [&](int c) { return wv[(c - 2 * g) / 8 * 2 + (c - 2 * g) % 8]; }, [&](int s, int j, float v) { out[s][j] = static_cast<_Float16>(v); });
+    }
+    const int at = first_new + n;  // this row's key
+    const bool mine = n < n_rows && at >= 0 && at < n_keys;
+    for (int st = 0; st < n_steps; st++) {
+        __builtin_amdgcn_s_barrier();
+        if (32 * st + 31 < first_new) continue;
+        asm volatile("" ::: "memory");
+        half8_t *kt = ring + (st % kAttnBufs) * (2 * kKPieces);
+        const int key = at - 32 * st;
+        if (mine && key >= 0 && key < 32) {
+#pragma unroll
+            for (int s = 0; s < KS; s++) {
+                if constexpr (VALUES) {
+                    _Float16 *vt = reinterpret_cast<_Float16 *>(kt + kKPieces);
+#pragma unroll
+                    for (int j = 0; j < 8; j++) {
+                        const int d = 32 * s + 8 * g + j;
+                        vt[(d * 4 + ((key >> 3) ^ attn_swz_v(d))) * 8 + (key & 7)] = out[s][j];
+                    }
+                } else {
+                    kt[key * CH + ((4 * s + g) ^ attn_swz<CH>(key))] = out[s];
+                }
+            }
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+    }
+    if (cache && mine) {
+#pragma unroll
+        for (int s = 0; s < KS; s++) {
+            if constexpr (VALUES) {
+#pragma unroll
+                for (int j = 0; j < 8; j++) cache[(32 * s + 8 * g + j) * stride + at] = out[s][j];
+            } else {
+                *reinterpret_cast<half8_t *>(cache + at * stride + 32 * s + 8 * g) = out[s];
+            }
+        }
+    }
+}
+
 // One workgroup = one KV head x one contiguous chunk of keys; wave w = query head w of the GQA
 // group.  Stage = 32 keys: the K tile [32 keys][HD] and the V^T tile [HD dims][32 keys] are copied
 // global -> LDS with direct-to-LDS loads into a ring of kAttnBufs buffers, so the whole group
@@ -182,13 +330,14 @@ __device__ __forceinline__ void attn_store_xf(float4_t (&tot)[DT], void *out_xf,
 // merge: 105.9 -> 98.3 us, both trees in turn (4.2 TB/s of keys and values; a copy reaches 5.03).
 // MERGE: the workgroup takes all of its rows' keys, split by split, and merges the splits as it goes (see
 // attn_rows_kernel); else one split, whose partial result it writes.
-template <int HD, typename TQ, int MAXW, int MAXL, bool MERGE>
+template <int HD, typename TQ, int MAXW, int MAXL, bool MERGE, bool ROPE>
 __device__ __forceinline__ void attn_body(const TQ *__restrict__ q, const _Float16 *__restrict__ k_cache,
                                           const _Float16 *__restrict__ vt_cache, float *__restrict__ part_o, float *__restrict__ part_ml,
                                           int64_t ctx_len, const int32_t *__restrict__ ctx_len_dev, int n_rows_total, int n_kv, int group, int n_waves,
                                           int64_t vt_stride, int want, int min_chunk, float scale, int full_block, int64_t window,
                                           int split_stride, int64_t part_slots, int block, float *__restrict__ out, void *__restrict__ out_xf,
-                                          int out_xf_kind, size_t xf_stride) {
+                                          int out_xf_kind, size_t xf_stride, AttnRope rope = {}) {
+    static_assert(!(MERGE && ROPE) && (!ROPE || sizeof(TQ) == 4), "a lone block's f32 rows");
     const int n_q = n_kv * group;
     // block: which block of sixteen query rows (a prefill group hands over many: block b's rows follow block
     // b - 1's in q and in the cache, its partial tiles sit part_slots slots further on)
@@ -208,11 +357,29 @@ __device__ __forceinline__ void attn_body(const TQ *__restrict__ q, const _Float
     // blockIdx.x = split + split_stride * (part of the GQA group this workgroup serves); split_stride is a multiple
     // of 8, so the workgroups that read one chunk of keys are dispatched to the same XCD and share its L2 copy
     const int split = MERGE ? 0 : blockIdx.x % split_stride;
+    if constexpr (ROPE) {
+        if (wave >= n_waves) {
+            const int64_t from = split * static_cast<int64_t>(min_chunk), to = min(ctx_len + n_rows, from + min_chunk);
+            if (to <= ctx_len || from >= to) return;
+            const bool values = wave > n_waves;
+            const float *row = reinterpret_cast<const float *>(q) + (static_cast<int64_t>(min(n, n_rows - 1)) * (n_q + 2 * n_kv) + n_q + (values ? n_kv : 0) + kvh) * HD;
+            const int first = static_cast<int>(ctx_len - from), keys = static_cast<int>(to - from), steps = (keys + 31) / 32;
+            const bool writes = static_cast<int>(blockIdx.x) < split_stride;
+            if (values)
+                attn_new_rows<HD, true>(row, nullptr, nullptr, 0.0f, n_rows, first, keys, steps, lds,
+                                        writes ? const_cast<_Float16 *>(vt_cache) + static_cast<int64_t>(kvh) * HD * vt_stride + from : nullptr, vt_stride);
+            else
+                attn_new_rows<HD, false>(row, rope.table, rope.k_w, rope.eps, n_rows, first, keys, steps, lds,
+                                         writes ? const_cast<_Float16 *>(k_cache) + (from * n_kv + kvh) * HD : nullptr, static_cast<int64_t>(n_kv) * HD);
+            return;
+        }
+    }
     const int head = kvh * group + (MERGE ? blockIdx.x : blockIdx.x / split_stride) * n_waves + wave;  // this wave's query head
     // Q^T fragments: lane (row n, g) holds Q[n][head][32 s + 8 g ..+8]
     // (rows at or past n_rows repeat the last row: they are never stored)
     AttnQ8<TQ> q_raw[KS];
-    const TQ *qrow = q + (static_cast<int64_t>(min(n, n_rows - 1)) * n_q + head) * HD + 8 * g;
+    const int64_t q_heads = ROPE ? n_q + 2 * n_kv : n_q;  // heads from one row to the next
+    const TQ *qrow = q + (static_cast<int64_t>(min(n, n_rows - 1)) * q_heads + head) * HD + 8 * g;
     attn_load_q<0, KS>(q_raw, qrow);
     if (ctx_len < 0) ctx_len = *ctx_len_dev;
     ctx_len += 16 * static_cast<int64_t>(block);
@@ -266,6 +433,22 @@ __device__ __forceinline__ void attn_body(const TQ *__restrict__ q, const _Float
         issued++;
     };
 
+    // ROPE: the norm's weights (a KB) and the table in the place of the last buffer.  The table's 16-byte chunk c of row r sits at c ^ r:
+    // sixteen lanes read the sixteen rows' at once.
+    constexpr int RP = HD / 4;  // chunks of a row of the table
+    static_assert(!ROPE || 64 + 16 * RP <= 2 * kKPieces, "the ring's last buffer holds the table");
+    half8_t *const raw_w = lds + (kAttnBufs - 1) * (2 * kKPieces), *const raw_tab = raw_w + 64;
+    const bool has_rows = ROPE && c1 > ctx_len;
+    const int first_new = ROPE ? static_cast<int>(min(ctx_len - c0, static_cast<int64_t>(0x3fffffff))) : 0;  // where the block's first key lies, relative to c0
+    if constexpr (ROPE) {
+        const int row_loads = (n_rows * RP + 63) / 64;
+        for (int i = wave; i < row_loads + 1; i += n_waves) {
+            const int p = 64 * i + lane, r = min(p / RP, n_rows - 1);
+            const float *src = i < row_loads ? rope.table + r * HD + 4 * ((p % RP) ^ r) : rope.q_w + 4 * (lane % RP);
+            __builtin_amdgcn_global_load_lds((gptr_t)(src), (lptr_t)(i < row_loads ? raw_tab + 64 * i : raw_w), 16, 0, 0);
+        }
+    }
+
     // prologue: kAttnBufs - 1 stages in flight
 #pragma unroll
     for (int st = 0; st < kAttnBufs - 1; st++)
@@ -283,11 +466,28 @@ __device__ __forceinline__ void attn_body(const TQ *__restrict__ q, const _Float
     {
         const float mult = scale * kLog2e;
         attn_wait(per_wave * issued);
+        if constexpr (!ROPE) {
 #pragma unroll
-        for (int s = 0; s < KS; s++) {
-            q_raw[s].arrived();
+            for (int s = 0; s < KS; s++) {
+                q_raw[s].arrived();
 #pragma unroll
-            for (int i = 0; i < 8; i++) qf[s][i] = static_cast<_Float16>(q_raw[s].get(i) * mult);
+                for (int i = 0; i < 8; i++) qf[s][i] = static_cast<_Float16>(q_raw[s].get(i) * mult);
+            }
+        } else {
+            float r[KS][8];
+#pragma unroll
+            for (int s = 0; s < KS; s++) {
+                q_raw[s].arrived();
+#pragma unroll
+                for (int i = 0; i < 8; i++) r[s][i] = q_raw[s].get(i);
+            }
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_barrier();  // what all waves asked for is there
+            asm volatile("" ::: "memory");
+            const int row = min(n, n_rows - 1);
+            const float4_t *tab = reinterpret_cast<const float4_t *>(raw_tab) + row * RP, *wt = reinterpret_cast<const float4_t *>(raw_w);
+            attn_rotate<KS>(r, g, rope.eps, [&](int c) { return tab[c ^ row]; }, [&](int c) { return wt[c]; },
+                            [&](int s, int j, float v) { qf[s][j] = static_cast<_Float16>(v * mult); });
         }
     }
 
@@ -333,6 +533,11 @@ __device__ __forceinline__ void attn_body(const TQ *__restrict__ q, const _Float
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
+        if constexpr (ROPE) {
+            if (!has_rows || 32 * st + 31 < first_new) return;
+            __builtin_amdgcn_s_barrier();  // the block's own rows are over what the cache still holds there
+            asm volatile("" ::: "memory");
+        }
     };
     // MERGE: what the splits so far come to; the split at hand ends ahead of stage split_end
     float4_t tot[MERGE ? DT : 1];
@@ -434,7 +639,6 @@ __device__ __forceinline__ void attn_body(const TQ *__restrict__ q, const _Float
         if (st < 8) ATT_TR(3 + st);
     }
     ATT_TR(12);
-
     if constexpr (MERGE) {
         float *o = out + ((static_cast<int64_t>(block) * 16 + n) * n_q + head) * HD;
 #pragma unroll
@@ -473,9 +677,20 @@ __global__ void __launch_bounds__(64 * MAXW)
                       const int32_t *__restrict__ ctx_len_dev) {
     // The arguments in the order of their use: the first fourteen words, which the first loads need, come preloaded with the wave.
     // heads = KV heads | group << 20, split_waves = split_stride | waves << 24; ctx_len < 0: it is in device memory; want == 0: min_chunk is the chunk.
-    attn_body<HD, TQ, MAXW, MAXL, false>(q, k_cache, vt_cache, part_o, part_ml, ctx_len, ctx_len_dev, n_rows_total, heads & 0xfffff, heads >> 20,
+    attn_body<HD, TQ, MAXW, MAXL, false, false>(q, k_cache, vt_cache, part_o, part_ml, ctx_len, ctx_len_dev, n_rows_total, heads & 0xfffff, heads >> 20,
                                          split_waves >> 24, vt_stride, want, min_chunk, scale, full_block, window, split_waves & 0xffffff, part_slots,
                                          blockIdx.z, nullptr, nullptr, 0, 0);
+}
+
+// A lone block whose rows are as the projections left them: see AttnRope.  heads: the rows, less one | query heads a KV head << 4 | KV heads << 9;
+// split_waves: split_stride | heads a workgroup << 11 | the chunk, in stages << 16.  (All the first loads need comes preloaded with the wave.)
+template <int HD, int MAXL>
+__global__ void __launch_bounds__(HD == 256 ? 512 : 640)
+    attn_split_rope_kernel(const float *__restrict__ rows, _Float16 *k_cache, _Float16 *vt_cache, const float *__restrict__ table,
+                           const float *__restrict__ q_w, uint32_t heads, uint32_t split_waves, int ctx_len, int vt_stride, const float *__restrict__ k_w, float eps, float scale, float *__restrict__ part_o, float *__restrict__ part_ml, int full_block, int64_t window) {
+    attn_body<HD, float, 8, MAXL, false, true>(rows, k_cache, vt_cache, part_o, part_ml, ctx_len, nullptr, (heads & 15) + 1, heads >> 9, heads >> 4 & 31,
+                                                  split_waves >> 11 & 31, vt_stride, 0, 32 * (split_waves >> 16), scale, full_block, window, split_waves & 0x7ff, 0, 0, nullptr,
+                                                  nullptr, 0, 0, AttnRope{table, q_w, k_w, eps});
 }
 
 // Many blocks of rows at once, a prompt's prefill: the blocks are enough workgroups, so one takes all of its block's keys
@@ -500,7 +715,7 @@ __global__ void __launch_bounds__(512)
         want = runs.want[r];
         min_chunk = runs.min_chunk[r];
     }
-    attn_body<HD, float, 8, MAXL, true>(q, k_cache, vt_cache, nullptr, nullptr, ctx_len, nullptr, n_rows_total, n_kv, n_q / n_kv, blockDim.x >> 6, vt_stride, want, min_chunk,
+    attn_body<HD, float, 8, MAXL, true, false>(q, k_cache, vt_cache, nullptr, nullptr, ctx_len, nullptr, n_rows_total, n_kv, n_q / n_kv, blockDim.x >> 6, vt_stride, want, min_chunk,
                                         scale, 0, 0, 1, 0, block, out, out_xf, out_xf_kind, xf_stride);
 }
 
@@ -1050,7 +1265,7 @@ template <int HD, typename TQ>
 int32_t launch_split(dflash_ctx *ctx, dim3 grid, int threads, hipStream_t st, const void *q, const _Float16 *k, const _Float16 *vt,
                   float *po, float *pml, int64_t ctx_len, const int32_t *ctx_len_dev, int n_rows, int n_q, int n_kv,
                   int64_t vt_stride, int want, int min_chunk, float scale, int full_block, int64_t window, int split_stride,
-                  int64_t part_slots) {
+                  int64_t part_slots, const dfl_attn_rope *rope) {
     const size_t lds = static_cast<size_t>(kAttnBufs) * 2 * (32 * HD / 8) * sizeof(half8_t);
     constexpr int kWaveLoads = 2 * 32 * (HD / 8) / 64;
     const int n_waves = threads / 64, per_wave = (kWaveLoads + n_waves - 1) / n_waves;
@@ -1062,8 +1277,19 @@ int32_t launch_split(dflash_ctx *ctx, dim3 grid, int threads, hipStream_t st, co
         want = 0;
         min_chunk = static_cast<int>(chunk);
     }
+    const uint32_t rope_heads = static_cast<uint32_t>(n_rows - 1) | static_cast<uint32_t>(n_q / n_kv) << 4 | static_cast<uint32_t>(n_kv) << 9;
+    const uint32_t rope_split = static_cast<uint32_t>(split_stride) | static_cast<uint32_t>(n_waves) << 11 | static_cast<uint32_t>(chunk / 32) << 16;
 #define DFL_ATTN_LAUNCH(MAXW, MAXL)                                                                                 \
     do {                                                                                                            \
+        if constexpr (sizeof(TQ) == 4 && MAXW == 8)                                                                 \
+            if (rope) {                                                                                             \
+                if (const int32_t rc_ = dfl_raise_lds_limit(ctx, reinterpret_cast<const void *>(attn_split_rope_kernel<HD, MAXL>), lds)) \
+                    return rc_;                                                                                     \
+                attn_split_rope_kernel<HD, MAXL><<<grid, threads + 128, lds, st>>>(                             \
+                    static_cast<const float *>(q), const_cast<_Float16 *>(k), const_cast<_Float16 *>(vt), rope->table, rope->q_w, rope_heads, \
+                    rope_split, static_cast<int>(ctx_len), static_cast<int>(vt_stride), rope->k_w, rope->eps, scale, po, pml, full_block, window); \
+                break;                                                                                              \
+            }                                                                                                       \
         if (const int32_t rc_ = dfl_raise_lds_limit(ctx, reinterpret_cast<const void *>(attn_split_kernel<HD, TQ, MAXW, MAXL>), lds)) \
             return rc_;                                                                                             \
         attn_split_kernel<HD, TQ, MAXW, MAXL><<<grid, threads, lds, st>>>(static_cast<const TQ *>(q), k, vt, ctx_len_dev ? -1 : ctx_len, vt_stride, \
@@ -1127,16 +1353,20 @@ extern "C" int32_t dflash_attn_verify_block(dflash_ctx *ctx, const void *q, int3
 static int32_t attn_rows(dflash_ctx *ctx, const void *q, int32_t q_type, const void *k_cache, const void *v_cache,
                          int32_t v_layout, int64_t ctx_len, int32_t n_rows_total, int32_t n_q, int32_t n_kv, int32_t head_dim,
                          int64_t kv_capacity, float scale, float *out, dflash_stream_t stream, int32_t full_block,
-                         int64_t window, const int32_t *ctx_len_dev, void *out_xf, int out_xf_kind, int32_t *blocks_done);
+                         int64_t window, const int32_t *ctx_len_dev, void *out_xf, int out_xf_kind, int32_t *blocks_done,
+                         const dfl_attn_rope *rope = nullptr);
 
 int32_t dfl_attn_block(dflash_ctx *ctx, const void *q, int32_t q_type, const void *k_cache, const void *v_cache,
                        int32_t v_layout, int64_t ctx_len, int32_t n_rows, int32_t n_q, int32_t n_kv, int32_t head_dim,
                        int64_t kv_capacity, float scale, float *out, dflash_stream_t stream, int32_t full_block,
-                       int64_t window, const int32_t *ctx_len_dev, void *out_xf, int out_xf_kind) {
+                       int64_t window, const int32_t *ctx_len_dev, void *out_xf, int out_xf_kind, const dfl_attn_rope *rope) {
     if (!ctx) return DFLASH_ERR_INVALID_INPUT;
     if (n_rows < 1 || n_rows > 16) return dfl_fail(ctx, DFLASH_ERR_BAD_SHAPE, "attn_verify: n_rows %d outside 1..16", n_rows);
+    if (rope && (q_type != DFLASH_TYPE_F32 || v_layout != 1 || ctx_len_dev ||
+                 !dfl_attn_rope_takes(ctx, *rope, q, n_q, n_kv, ctx_len, n_rows, head_dim, kv_capacity)))
+        return dfl_fail(ctx, DFLASH_ERR_UNSUPPORTED, "attn_verify: rows as the projections left them are not taken here");
     return attn_rows(ctx, q, q_type, k_cache, v_cache, v_layout, ctx_len, n_rows, n_q, n_kv, head_dim, kv_capacity, scale, out, stream,
-                     full_block, window, ctx_len_dev, out_xf, out_xf_kind, nullptr);
+                     full_block, window, ctx_len_dev, out_xf, out_xf_kind, nullptr, rope);
 }
 
 static int32_t attn_check(dflash_ctx *ctx, const void *q, int32_t q_type, const void *k_cache, const void *v_cache, int32_t v_layout,
@@ -1227,6 +1457,17 @@ static AttnPolicy attn_policy(const dflash_ctx *ctx, int64_t bucket, int n_kv, i
     // launch's: the bits must not depend on it.
     const int64_t max_splits = std::min<int64_t>(want, (2 * bucket - 1 + min_chunk - 1) / min_chunk);
     return {want, min_chunk, hw, head_dim < 256 && max_splits <= kOrderedSplits};
+}
+
+// Loads of rows, table and weights are of 16 bytes; a chunk goes over as sixteen bits of stages.  Beside its heads' waves a workgroup has two more: with
+// heads of 256 a wave holds more than a third of a SIMD's registers, so there are eight at most.
+bool dfl_attn_rope_takes(const dflash_ctx *ctx, const dfl_attn_rope &r, const void *rows, int32_t n_q, int32_t n_kv, int64_t ctx_len, int32_t n_rows,
+                         int32_t head_dim, int64_t kv_capacity) {
+    const uintptr_t at = reinterpret_cast<uintptr_t>(rows) | reinterpret_cast<uintptr_t>(r.table) | reinterpret_cast<uintptr_t>(r.q_w) | reinterpret_cast<uintptr_t>(r.k_w);
+    if (!r.table || !r.q_w || !r.k_w || !rows || at % 16 || n_rows < 1 || n_rows > 16 || ctx_len < 0 || kv_capacity > 65535 * 32 || n_kv < 1 || n_kv >= 1 << 20 || n_q % n_kv ||
+        n_q / n_kv > 16 || (head_dim != 64 && head_dim != 128 && head_dim != 256))
+        return false;
+    return attn_policy(ctx, dfl_attn_bucket(ctx_len + n_rows), n_kv, n_q / n_kv, head_dim).hw <= (head_dim == 256 ? 6 : 8);
 }
 
 int32_t dfl_attn_blocks(dflash_ctx *ctx, const void *q, int32_t q_type, const void *k_cache, const void *vt_cache, int64_t ctx_len,
@@ -1321,7 +1562,8 @@ int32_t dfl_attn_blocks(dflash_ctx *ctx, const void *q, int32_t q_type, const vo
 static int32_t attn_rows(dflash_ctx *ctx, const void *q, int32_t q_type, const void *k_cache, const void *v_cache,
                          int32_t v_layout, int64_t ctx_len, int32_t n_rows_total, int32_t n_q, int32_t n_kv, int32_t head_dim,
                          int64_t kv_capacity, float scale, float *out, dflash_stream_t stream, int32_t full_block,
-                         int64_t window, const int32_t *ctx_len_dev, void *out_xf, int out_xf_kind, int32_t *blocks_done) {
+                         int64_t window, const int32_t *ctx_len_dev, void *out_xf, int out_xf_kind, int32_t *blocks_done,
+                         const dfl_attn_rope *rope) {
     int32_t n_blocks = (n_rows_total + 15) / 16;
     const int32_t n_rows = std::min(16, n_rows_total);  // rows of the first block: what the split policy looks at
     if (const int32_t rc_ = attn_check(ctx, q, q_type, k_cache, v_cache, v_layout, ctx_len, n_rows_total, n_q, n_kv, head_dim, kv_capacity, out,
@@ -1408,11 +1650,11 @@ static int32_t attn_rows(dflash_ctx *ctx, const void *q, int32_t q_type, const v
     if (q_type == DFLASH_TYPE_F32)                                                                                \
         rc = launch_split<HD, float>(ctx, grid, threads, st, q, k, vt, part_o, part_ml, ctx_len, ctx_len_dev, n_rows_total, n_q, n_kv, \
                                      vt_stride, want, static_cast<int>(min_chunk), scale, full_block, window,     \
-                                     split_stride, part_slots);                                                   \
+                                     split_stride, part_slots, rope);                                             \
     else                                                                                                          \
         rc = launch_split<HD, _Float16>(ctx, grid, threads, st, q, k, vt, part_o, part_ml, ctx_len, ctx_len_dev, n_rows_total, n_q, \
                                         n_kv, vt_stride, want, static_cast<int>(min_chunk), scale, full_block, window, \
-                                        split_stride, part_slots)
+                                        split_stride, part_slots, nullptr)
         if (head_dim == 64) {
             DFL_ATTN(64);
         } else if (head_dim == 128) {

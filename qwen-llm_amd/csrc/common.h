@@ -406,10 +406,19 @@ int32_t dfl_select_draft_path(dflash_ctx *ctx, const dflash_codebook *predecesso
                               int32_t carry_token, int32_t n, const int32_t *topk_ids, const float *topk_vals, const float *sel_h, int32_t *out_tokens,
                               int32_t *out_tokens_host, int32_t *page, dflash_stream_t stream);
 
+// A block's rows as the projections leave them, [row][query heads | key heads | value heads] in f32: the attention norms and rotates them itself,
+// and writes the block's rows of both caches (dfl_attn_block with rope; its q is then those rows).
+struct dfl_attn_rope {
+    const float *q_w, *k_w;  // the norms' weights
+    const float *table;      // [row][head_dim / 2 cosines, head_dim / 2 sines] of the rows' positions
+    float eps;
+};
+bool dfl_attn_rope_takes(const dflash_ctx *ctx, const dfl_attn_rope &r, const void *rows, int32_t n_q, int32_t n_kv, int64_t ctx_len, int32_t n_rows,
+                         int32_t head_dim, int64_t kv_capacity);
 int32_t dfl_attn_block(dflash_ctx *ctx, const void *q, int32_t q_type, const void *k_cache, const void *v_cache,
                        int32_t v_layout, int64_t ctx_len, int32_t n_rows, int32_t n_q, int32_t n_kv, int32_t head_dim,
                        int64_t kv_capacity, float scale, float *out, dflash_stream_t stream, int32_t full_block,
-                       int64_t window, const int32_t *ctx_len_dev, void *out_xf = nullptr, int out_xf_kind = 0);
+                       int64_t window, const int32_t *ctx_len_dev, void *out_xf = nullptr, int out_xf_kind = 0, const struct dfl_attn_rope *rope = nullptr);
 
 // Block-causal attention of n_rows_total consecutive query rows, sixteen to a block, each block exactly as
 // dfl_attn_block would run it alone at its own context length (ctx_len + 16 b): the same split of the keys, so the same

@@ -9,6 +9,7 @@
 #include "common.h"
 #include "device_quant.h"
 #include "mfma_unpack.h"
+#include "rope_head.h"
 
 #include <algorithm>
 #include <array>
@@ -257,58 +258,6 @@ void rms_norm(int rows, hipStream_t st, float *x, const float *add, const float 
 #undef DFL_NORM
 }
 
-// A lane's rotation pairs of one head: pair k is elements (i, i + HD/2), i = lane + 64 k (heads of 64: lanes 0..31).
-template <int HD>
-struct RopePairs {
-    static constexpr int N = HD <= 128 ? 1 : 2, kEl = HD / 64;  // pairs, elements per lane
-    float sn[N], cs[N];
-    __device__ __forceinline__ void angles(int lane, float theta, float pos) {
-#pragma unroll
-        for (int k = 0; k < N; k++) {
-            const int i = HD == 64 ? (lane & 31) : lane + 64 * k;
-            const float freq = pos / powf(theta, static_cast<float>(2 * i) / static_cast<float>(HD));
-            sincosf(freq, &sn[k], &cs[k]);
-        }
-    }
-};
-// ... and the head's values: element lane + 64 k in r[k], its norm weight in wr[k] (heads of 64: a lane also holds the
-// other element of its pair)
-template <int HD>
-struct RopeHead {
-    static constexpr int kEl = HD / 64;
-    float r[kEl], wr[kEl], r_far = 0.0f, w_far = 1.0f;
-    __device__ __forceinline__ void load(const float *v, const float *w, int lane) {
-#pragma unroll
-        for (int k = 0; k < kEl; k++) r[k] = v[lane + 64 * k];
-        if (HD == 64) r_far = v[lane ^ 32];
-#pragma unroll
-        for (int k = 0; k < kEl; k++) wr[k] = w ? w[lane + 64 * k] : 1.0f;
-        if (HD == 64) w_far = w ? w[lane ^ 32] : 1.0f;
-    }
-    // norm, weight (where there is one), rotation; put(i, value) for elements i and i + HD / 2 of every pair
-    template <typename Put>
-    __device__ __forceinline__ void finish(const RopePairs<HD> &t, bool weighted, int lane, float eps, Put put) const {
-        float s = r[0] * r[0];
-#pragma unroll
-        for (int k = 1; k < kEl; k++) s = __builtin_fmaf(r[k], r[k], s);
-        s = dfl_wave_sum(s);
-        const float scale = 1.0f / sqrtf(s / static_cast<float>(HD) + eps);
-#pragma unroll
-        for (int k = 0; k < RopePairs<HD>::N; k++) {
-            constexpr int kFar = HD / 128;  // the partner's register, from k on
-            float a = r[k] * scale, b = (HD == 64 ? r_far : r[k + (HD == 64 ? 0 : kFar)]) * scale;
-            if (weighted) {
-                a *= wr[k];
-                b *= HD == 64 ? w_far : wr[k + (HD == 64 ? 0 : kFar)];
-            }
-            // (spelled out, so that the two kernels round alike; and a key's value is rounded to f32 before it is to f16)
-            float ra = __builtin_fmaf(a, t.cs[k], -(b * t.sn[k])), rb = __builtin_fmaf(b, t.cs[k], a * t.sn[k]);
-            asm volatile("" : "+v"(ra), "+v"(rb));
-            if (HD > 64 || lane < 32) put(lane + 64 * k, ra, rb);
-        }
-    }
-};
-
 // kernel_qk_rms_norm_rope_f32_packed_consecutive (attn.metal:137-196) + the f32 -> f16 KV scatter
 // (elementwise.metal:674-685).  One wave per (row, head): per-head RMSNorm (weight may be null),
 // NeoX RoPE over the full head (pairs (i, i + hd/2), angle = pos / theta^(2i/hd)).
@@ -484,10 +433,20 @@ __global__ void set_ids_pos_kernel(Int16Args ids, Int16Args pos, int n, int32_t 
 }
 
 // A block's ids and positions to the device, as set_ids_pos_kernel, and its embedding rows, as get_rows_kernel: one launch at the head of a
-// block (1.5 + 3.0 us as two).
+// block (1.5 + 3.0 us as two).  With rope_table, one workgroup more per row makes the row's sines and cosines (see dfl_attn_rope).
 __global__ void __launch_bounds__(256)
     begin_rows_kernel(int type, const uint8_t *__restrict__ table, size_t row_bytes, int hidden, float *__restrict__ out, Int16Args ids, Int16Args pos,
-                      int32_t *__restrict__ ids_dst, int32_t *__restrict__ pos_dst, const int32_t *__restrict__ dev_ids, int vocab) {
+                      int32_t *__restrict__ ids_dst, int32_t *__restrict__ pos_dst, const int32_t *__restrict__ dev_ids, int vocab,
+                      float *__restrict__ rope_table, int head_dim, float theta) {
+    if (rope_table && blockIdx.x == gridDim.x - 1) {
+        const int i = threadIdx.x;
+        if (i >= head_dim / 2) return;
+        float sn, cs, *row = rope_table + static_cast<size_t>(blockIdx.y) * head_dim + i;
+        dfl_rope_angle(i, head_dim, theta, static_cast<float>(pos.v[blockIdx.y]), &sn, &cs);
+        row[0] = cs;
+        row[head_dim / 2] = sn;
+        return;
+    }
     const int r = blockIdx.y, e = blockIdx.x * blockDim.x + threadIdx.x;
     int id = ids.v[r];
     if (dev_ids && id < 0) {
@@ -822,11 +781,12 @@ struct BlockBegin {
     const int32_t *dev_ids;  // (see set_ids_pos_kernel)
 };
 int32_t begin_rows(dflash_ctx *ctx, const dflash_qtensor &t, const BlockBegin &b, int n, int hidden, int vocab, float *out, int32_t *ids_dst,
-                   int32_t *pos_dst, hipStream_t st) {
+                   int32_t *pos_dst, hipStream_t st, float *rope_table, int head_dim, float theta) {
     const size_t rb = dflash_row_bytes(t.type, hidden);
     if (rb == 0) return dfl_fail(ctx, DFLASH_ERR_UNSUPPORTED, "embedding type %d", t.type);
-    begin_rows_kernel<<<dim3(blocks_for(hidden), n), 256, 0, st>>>(t.type, static_cast<const uint8_t *>(t.data), rb, hidden, out, b.ids, b.pos, ids_dst,
-                                                                 pos_dst, b.dev_ids, vocab);
+    begin_rows_kernel<<<dim3(blocks_for(hidden) + (rope_table ? 1 : 0), n), 256, 0, st>>>(t.type, static_cast<const uint8_t *>(t.data), rb, hidden, out,
+                                                                                         b.ids, b.pos, ids_dst, pos_dst, b.dev_ids, vocab, rope_table,
+                                                                                         head_dim, theta);
     return DFLASH_OK;
 }
 // A few rows through a small matrix in one launch, where the public operator has one for it (whose cuts of K a prompt's products do not share).
@@ -849,6 +809,7 @@ struct dflash_session {
     // cur and attn once more, as f16 in MFMA fragment order, for the projections that take the whole-K kernel
     uint8_t *xf_cur = nullptr, *xf_attn = nullptr, *xf_g = nullptr;
     uint8_t *xs_cur = nullptr;  // the sub-block sums of xf_cur's rows (a wide dense layer's gate | up)
+    float *rope = nullptr;      // a block's sines and cosines, [16][head_dim]
     float *hidden = nullptr;  // [16][n_taps][hidden] capture slots of the speculative step
     int32_t *ids = nullptr, *pos = nullptr, *argmax = nullptr;
     dfl_moe_scratch moe;
@@ -923,6 +884,7 @@ struct dflash_draft_session {
     float *pk = nullptr;  // [16][max(q_dim + 2 kv_dim, 2 ffn)]: output of a fused q/k/v or gate/up GEMM
     // cur, attn and g once more, as f16 in MFMA fragment order, for the projections that take the whole-K kernel
     uint8_t *xf_cur = nullptr, *xf_attn = nullptr, *xf_g = nullptr;
+    float *rope = nullptr;  // a block's sines and cosines, [16][head_dim]
     int32_t *ids = nullptr, *pos = nullptr, *argmax = nullptr;
     // every layer's context K/V projection as ONE batched GEMM (draft_prepare): its output [layer][16][2 kv_dim],
     // the list 0 .. n_layers - 1 and its length for the batched kernel
@@ -965,6 +927,7 @@ int32_t dflash_session_create(dflash_ctx *ctx, const dflash_model_cfg *cfg, int6
               bufs.want(&s->mix, 16 * cfg->hidden) && bufs.want(&s->g, 16 * f) && bufs.want(&s->u, 16 * f) &&
               bufs.want(&s->pk, 16 * std::max(q_dim + 2 * kv_dim, 2 * f)) &&
               bufs.want(&s->xf_cur, dfl_xf_bytes((cfg->hidden + 255) / 256 * 256)) && bufs.want(&s->xs_cur, dfl_xs_bytes((cfg->hidden + 255) / 256 * 256)) &&
+              bufs.want(&s->rope, 16 * static_cast<size_t>(cfg->head_dim)) &&
               bufs.want(&s->xf_attn, dfl_xf_bytes((static_cast<int64_t>(q_dim) + 255) / 256 * 256)) &&
               bufs.want(&s->xf_g, dfl_xf_bytes((static_cast<int64_t>(f) + 255) / 256 * 256)) &&
               bufs.want(&s->logits, 16 * static_cast<size_t>(cfg->vocab)) && bufs.want(&s->gap, 16) &&
@@ -1188,7 +1151,9 @@ int32_t verify_enqueue(dflash_ctx *ctx, const dflash_model *model, dflash_sessio
     float *const x = resume ? resume->x : s->x;
     const float *const q = resume ? resume->q : s->q;
     int32_t rc;
-    if (!resume && (rc = begin ? begin_rows(ctx, model->token_embd, *begin, n, H, c.vocab, x, s->ids, s->pos, st)
+    // (a lane of the pipeline hands its K/V rows to the next block's lane ahead of its attention: they have a launch of their own there)
+    float *const rope_table = begin && !lane ? s->rope : nullptr;
+    if (!resume && (rc = begin ? begin_rows(ctx, model->token_embd, *begin, n, H, c.vocab, x, s->ids, s->pos, st, rope_table, hd, c.rope_theta)
                                : embed_rows(ctx, model->token_embd, s->ids, n, H, x, st)))
         return rc;
     Captures caps(tap_layers, n_taps, hidden_capture, H);
@@ -1213,6 +1178,11 @@ int32_t verify_enqueue(dflash_ctx *ctx, const dflash_model *model, dflash_sessio
         // (a dense layer leaves its FFN output in s->mix: the residual add is folded into this norm)
         const bool moe = c.n_expert > 0;
         const LayerXf xk = layer_kinds(il);
+        // A block nobody asked head outputs of needs nothing of the last layer beyond its K/V rows, unless that layer's
+        // residual is tapped: its attention, output projection and FFN would only feed the head.
+        const bool kv_only = !want_head && il == c.n_layers - 1 && !caps.tapped(il);
+        bool rotates = false;  // the attention norms and rotates the rows, and writes the caches'
+        const dfl_attn_rope rope = {L.q_norm, L.k_norm, rope_table, c.eps};
         if (!resume) {
             if (!cur_ready)
                 rms_norm(n, st, x, pending_resid, L.attn_norm, xk.qkv ? nullptr : s->cur, H, c.eps, nullptr, nullptr, xk.qkv ? s->xf_cur : nullptr, xk.qkv, 0,
@@ -1223,7 +1193,9 @@ int32_t verify_enqueue(dflash_ctx *ctx, const dflash_model *model, dflash_sessio
             if ((rc = gemm_qkv(ctx, L.wq, L.wk, L.wv, s->cur, s->q, s->k, s->v, s->pk, true, &packed, H, q_dim, kv_dim, n, st, s->xf_cur, xk.qkv, true)))
                 return rc;
             const int64_t tot = q_dim + 2 * kv_dim;
-            qk_norm_rope(hd, c.n_q + 2 * c.n_kv, n, st, packed ? s->pk : s->q, packed ? tot : q_dim, packed ? s->pk + q_dim : s->k, packed ? tot : kv_dim, s->q, s->k, L.q_norm,
+            rotates = packed && !kv_only && dfl_attn_rope_takes(ctx, rope, s->pk, c.n_q, c.n_kv, start, n, hd, s->capacity);
+            if (!rotates)
+                qk_norm_rope(hd, c.n_q + 2 * c.n_kv, n, st, packed ? s->pk : s->q, packed ? tot : q_dim, packed ? s->pk + q_dim : s->k, packed ? tot : kv_dim, s->q, s->k, L.q_norm,
                 L.k_norm, kc, s->pos, c.n_q, c.n_kv, c.eps, c.rope_theta, packed ? s->pk + q_dim + kv_dim : s->v,
                 packed ? tot : kv_dim, vtc, s->capacity);
         }
@@ -1234,17 +1206,11 @@ int32_t verify_enqueue(dflash_ctx *ctx, const dflash_model *model, dflash_sessio
             if (lane->wait_other) DFL_HIP_CHECK(ctx, hipStreamWaitEvent(st, lane->other[il], 0));
             DFL_HIP_CHECK(ctx, hipEventRecord(lane->mine[il], st));
         }
-        // A block nobody asked head outputs of needs nothing of the last layer beyond its K/V rows, unless that layer's
-        // residual is tapped: its attention, output projection and FFN would only feed the head.
-        if (!want_head && il == c.n_layers - 1) {
-            bool tapped_last = false;
-            for (int t = 0; t < n_taps; t++) tapped_last = tapped_last || tap_layers[t] == il;
-            if (!tapped_last) break;
-        }
+        if (kv_only) break;
         // under capture the context length is read from pos[0] on the device: the same launches then serve every
         // position of the bucket
-        if ((rc = dfl_attn_block(ctx, q, DFLASH_TYPE_F32, kc, vtc, 1, start, n, c.n_q, c.n_kv, hd, s->capacity, scale,
-                                 s->attn, st, 0, 0, ctx->capturing ? s->pos : nullptr, xk.wo ? s->xf_attn : nullptr, xk.wo)))
+        if ((rc = dfl_attn_block(ctx, rotates ? s->pk : q, DFLASH_TYPE_F32, kc, vtc, 1, start, n, c.n_q, c.n_kv, hd, s->capacity, scale,
+                                 s->attn, st, 0, 0, ctx->capturing ? s->pos : nullptr, xk.wo ? s->xf_attn : nullptr, xk.wo, rotates ? &rope : nullptr)))
             return rc;
         if (xk.wo)
             rc = dfl_gemm_whole(ctx, L.wo.type, L.wo.data, s->xf_attn, s->mix, static_cast<int64_t>(q_dim), H, n, 0, nullptr, DFL_XF_NONE, st, true);
@@ -1865,7 +1831,8 @@ int32_t dflash_draft_session_create(dflash_ctx *ctx, const dflash_draft_cfg *cfg
               bufs.want(&s->layer_ids, static_cast<size_t>(cfg->n_layers)) && bufs.want(&s->n_layers_dev, 1) &&
               bufs.want(&s->xf_cur, dfl_xf_bytes((static_cast<int64_t>(H) + 255) / 256 * 256)) &&
               bufs.want(&s->xf_attn, dfl_xf_bytes((static_cast<int64_t>(q_dim) + 255) / 256 * 256)) &&
-              bufs.want(&s->xf_g, dfl_xf_bytes((static_cast<int64_t>(cfg->ffn) + 255) / 256 * 256));
+              bufs.want(&s->xf_g, dfl_xf_bytes((static_cast<int64_t>(cfg->ffn) + 255) / 256 * 256)) &&
+              bufs.want(&s->rope, 16 * static_cast<size_t>(cfg->head_dim));
     if (ok && cfg->conv_kernel_size > 0)
         ok = bufs.want(&s->conv_buf, 16 * H) &&
              bufs.want(&s->conv_dyn, 16 * static_cast<size_t>(2) * cfg->conv_kernel_size * (H / cfg->conv_group_size));
@@ -2110,7 +2077,8 @@ int32_t draft_block_impl(dflash_ctx *ctx, const dflash_model *target, const dfla
     // walk, which takes the carry by value - so they can be captured once and replayed.
     auto enqueue = [&](hipStream_t st) -> int32_t {
     int32_t rc;
-    if ((rc = by_value ? begin_rows(ctx, target->token_embd, begin, N, H, V, s->x, s->ids, s->pos, st)
+    float *const rope_table = by_value && fast ? s->rope : nullptr;
+    if ((rc = by_value ? begin_rows(ctx, target->token_embd, begin, N, H, V, s->x, s->ids, s->pos, st, rope_table, hd, c.rope_theta)
                        : embed_rows(ctx, target->token_embd, s->ids, N, H, s->x, st)))
         return rc;
 
@@ -2167,16 +2135,19 @@ int32_t draft_block_impl(dflash_ctx *ctx, const dflash_model *target, const dfla
         const int64_t tot = q_dim + 2 * kv_dim;
         if (fast) {
             // the block's own K (normed, rotated) and V go behind the context in the f16 mirror, written by the
-            // same kernel (positions pos[i] = ctx_len + i on this path); one MFMA pass over context and block
-            qk_norm_rope(hd, c.n_q + 2 * c.n_kv, N, st, packed ? s->pk : s->q, packed ? tot : q_dim, packed ? s->pk + q_dim : s->k, packed ? tot : kv_dim, s->q, s->k,
+            // same kernel (positions pos[i] = ctx_len + i on this path); one MFMA pass over context and block, which does all of
+            // that itself where it can
+            const dfl_attn_rope rope = {L.q_norm, L.k_norm, rope_table, c.eps};
+            const bool rotates = packed && dfl_attn_rope_takes(ctx, rope, s->pk, c.n_q, c.n_kv, s->ctx_len, N, hd, s->cap16);
+            if (!rotates) qk_norm_rope(hd, c.n_q + 2 * c.n_kv, N, st, packed ? s->pk : s->q, packed ? tot : q_dim, packed ? s->pk + q_dim : s->k, packed ? tot : kv_dim, s->q, s->k,
                 L.q_norm, L.k_norm, k16, s->pos, c.n_q, c.n_kv, c.eps, c.rope_theta, packed ? s->pk + q_dim + kv_dim : s->v,
                 packed ? tot : kv_dim, vt16, s->cap16);
             // (under capture the context length is pos[0], read on the device: the launches then serve every context
             // of the bucket; chunking, and so the result, is the same either way)
-            if ((rc = dfl_attn_block(ctx, s->q, DFLASH_TYPE_F32, k16, vt16, 1, s->ctx_len, N, c.n_q, c.n_kv, hd, s->cap16,
+            if ((rc = dfl_attn_block(ctx, rotates ? s->pk : s->q, DFLASH_TYPE_F32, k16, vt16, 1, s->ctx_len, N, c.n_q, c.n_kv, hd, s->cap16,
                                      1.0f / sqrtf(static_cast<float>(hd)), s->attn, st, c.causal ? 0 : 1,
                                      L.is_swa ? static_cast<int64_t>(c.swa_window) : 0, ctx->capturing ? s->pos : nullptr,
-                                     xk.wo ? s->xf_attn : nullptr, xk.wo)))
+                                     xk.wo ? s->xf_attn : nullptr, xk.wo, rotates ? &rope : nullptr)))
                 return rc;
         } else {
             qk_norm_rope(hd, c.n_q + c.n_kv, N, st, s->q, q_dim, s->k, kv_dim, s->q, s->k, L.q_norm, L.k_norm, nullptr, s->pos, c.n_q, c.n_kv,

@@ -288,3 +288,26 @@ def test_context_columns_appended_at_once_equal_columns_in_blocks(ctx, first):
         out.append(d.draft_block(5, cfg.vocab - 1, first + 45, want_logits=True)[1].clone())
         d.close()
     assert torch.equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("start", [0, 17, 31, 63, 260, 520, 569])
+@pytest.mark.parametrize("shape", ["narrow", "experts", "heads64", "heads64x12", "heads256x1", "heads256x12"])
+def test_a_lone_block_rotates_its_rows_as_a_group_does(ctx, shape, start):
+    """A lone block's attention norms and rotates its rows itself and puts its keys and values over the cache's (groups of at most
+    eight heads); a group's rows have a launch of their own: the same bits, of every number of rows, where the rows fall into one
+    stage of keys, two, or the splits of two workgroups, and where the next block reads what they left in the cache.  (Starts with
+    64 positions behind them whose splits are of one policy, that of their bucket of context lengths.)"""
+    cfg, attn_type = SHAPES[shape]
+    model = dfl.TargetModel(ctx, cfg, dfl.synth_target_weights_device(cfg, 5, "cuda", attn_type=attn_type))
+    tokens = np.random.default_rng(start).integers(0, cfg.vocab, start + 64).tolist()
+    one, many = dfl.Session(ctx, model, start + 80, [0, 1]), dfl.Session(ctx, model, start + 80, [0, 1])
+    for s in (one, many) if start else ():
+        s.prefill_blocks(tokens[:start], 0)
+    want = many.prefill_blocks(tokens[start:], start)
+    at = start
+    for n in (1, 16, 5, 11, 2, 16):
+        got = one.encode_packed_verify_layer_major(tokens[at:at + n], at).hidden_capture
+        assert torch.equal(got, want[at - start:at - start + n]), (at, n)
+        at += n
+    one.close()
+    many.close()
