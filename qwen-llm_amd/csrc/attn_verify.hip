@@ -727,25 +727,34 @@ __global__ void __launch_bounds__(512)
 // registers, and beside the queries a lane keeps one sum.
 // LDS: three 64-key tiles of K for the first walk; for the second two splits of K and V, the first of them behind the
 // three tiles (it is asked for while the first walk ends), the other in the place of two of them.
-// What bounds it: a wave's products (96 MFMAs a split) and vector work (270 instructions) stand mostly one behind the other, 3.4 us
-// a split with eight waves, 2.6 with four; without the loads 7 % less.  Computing the next split's scores under this
-// one's softmax: 151 -> 160 us (registers).  2048 rows of 16 / 2 heads: 425 us as splits (286 MB of partial results out
-// and as many back), 151 here; 300 rows 36 -> 26 us.
+// What bounds it: the chain of the longest block.  A wave's products (96 MFMAs a split) and vector work (250 instructions) stand mostly
+// one behind the other, 3.4 us a split with eight busy waves, 2.6 to 3.2 with four; without the loads 7 % less, without the first walk's
+// products 14 %, without the second walk's 47 %.  So a workgroup has four heads of a long block and of a short one, which
+// share keys and values as far as the short one reaches, and the longest are mostly alone on their SIMDs: 2048 rows of 16 / 2 heads, where eight
+// heads of one block are a CU's and the longest block's is the last to end, 147 -> 124 us.  As splits they are 425 us (286 MB of partial results
+// out and as many back); 300 rows 36 -> 26 us.
+// Not kept: the next split's scores under this one's softmax (151 -> 160 us, registers); a quarter of the keys for four heads a wave in the first
+// walk, a quarter of its LDS reads, and a tile's second product behind the next tile's first (124 : 124 us).
 constexpr int kPairSplit = 64, kPairKeys = 32 * 1024, kPairLds = 5 * kPairKeys;
 __global__ void __launch_bounds__(512)
     attn_rows_pair_kernel(const float *__restrict__ q, const _Float16 *__restrict__ k_cache, const _Float16 *__restrict__ vt_cache, int64_t ctx_len,
                           int n_rows_total, int n_q, int n_kv, int64_t vt_stride, float scale, float *__restrict__ out, void *__restrict__ out_xf,
-                          int out_xf_kind, size_t xf_stride) {
+                          int out_xf_kind, size_t xf_stride, int heads) {
     constexpr int HD = 256, KS = HD / 32, DT = HD / 16, CH = HD / 8;
     extern __shared__ half8_t lds[];
-    const int block = gridDim.z - 1 - blockIdx.z;  // (the longest first)
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n_waves = blockDim.x >> 6;
+    const int n = lane & 15, g = lane >> 4;
+    // The longest blocks first.  Twice as many waves as heads: the second half of them has the block as far from the first as
+    // this one from the last (none in the middle of an odd number), and goes along with this one's splits as far as its own reach.
+    const int far = (n_rows_total + 15) / 16 - 1 - blockIdx.z, near = blockIdx.z;
+    const bool second = wave >= heads;
+    const int block = second ? near : far;
+    const int n_all = static_cast<int>(ctx_len) + min(16 * far + 16, n_rows_total), all_splits = (n_all + kPairSplit - 1) / kPairSplit;
     const int n_rows = min(16, n_rows_total - 16 * block);
     ctx_len += 16 * static_cast<int64_t>(block);
     const int n_pos = static_cast<int>(ctx_len) + n_rows;
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n_waves = blockDim.x >> 6;
-    const int n = lane & 15, g = lane >> 4;
-    const int kvh = blockIdx.y, head = kvh * (n_q / n_kv) + blockIdx.x * n_waves + wave;
-    const int n_splits = (n_pos + kPairSplit - 1) / kPairSplit;
+    const int kvh = blockIdx.y, head = kvh * (n_q / n_kv) + blockIdx.x * heads + (second ? wave - heads : wave);
+    const int n_splits = second && near == far ? 0 : (n_pos + kPairSplit - 1) / kPairSplit;
     const int64_t kv_dim = static_cast<int64_t>(n_kv) * HD;
     const uint8_t *const k_base = reinterpret_cast<const uint8_t *>(k_cache + static_cast<int64_t>(kvh) * HD);
     const uint8_t *const v_base = reinterpret_cast<const uint8_t *>(vt_cache + static_cast<int64_t>(kvh) * HD * vt_stride);
@@ -757,7 +766,7 @@ __global__ void __launch_bounds__(512)
     const uint32_t k_lane = static_cast<uint32_t>(2 * wave + (lane >> 5)) * static_cast<uint32_t>(kv_dim * 2) +
                             (((lane & 31) ^ attn_swz<CH>(2 * wave + (lane >> 5))) << 4);
     auto load = [&](int split, bool values, uint8_t *dst) {
-        const int total = values ? 64 : 32, c0 = split * kPairSplit, last = n_pos - 1 - c0;
+        const int total = values ? 64 : 32, c0 = split * kPairSplit, last = n_all - 1 - c0;
         auto whole = [&](auto waves) {
             constexpr int NW = decltype(waves)::value;
             const uint8_t *k = k_base + c0 * kv_dim * 2, *v = v_base + static_cast<int64_t>(16 * wave) * vt_stride * 2 + 2 * static_cast<int64_t>(c0);
@@ -802,7 +811,7 @@ __global__ void __launch_bounds__(512)
         const float *qrow = q + (static_cast<int64_t>(block) * 16 + min(n, n_rows - 1)) * n_q * HD + static_cast<int64_t>(head) * HD + 8 * g;
         AttnQ8<float> raw[KS];
         load(0, false, lds_b);
-        if (n_splits > 1)
+        if (all_splits > 1)
             load(1, false, lds_b + kPairKeys);
         else
             load(0, true, lds_b + 3 * kPairKeys);
@@ -853,12 +862,12 @@ __global__ void __launch_bounds__(512)
 
     // first walk: the maximum over every key a row sees
     float m_star = -INFINITY;
-    for (int split = 0, buf = 0; split < n_splits; split++) {
-        landed(split + 1 < n_splits ? per_keys : per_split);
+    for (int split = 0, buf = 0; split < all_splits; split++) {
+        landed(split + 1 < all_splits ? per_keys : per_split);
         uint8_t *const free_buf = lds_b + (buf == 0 ? 2 : buf - 1) * kPairKeys;
-        if (split + 2 < n_splits)
+        if (split + 2 < all_splits)
             load(split + 2, false, free_buf);
-        else if (split + 2 == n_splits)
+        else if (split + 2 == all_splits)
             load(0, true, lds_b + 3 * kPairKeys);
         auto maxima = [&](auto masked) {
             float p[16];
@@ -866,9 +875,9 @@ __global__ void __launch_bounds__(512)
 #pragma unroll
             for (int i = 0; i < 16; i++) m_star = fmaxf(m_star, p[i]);
         };
-        if (edge(split))
+        if (split < n_splits && edge(split))
             maxima(std::true_type());
-        else
+        else if (split < n_splits)
             maxima(std::false_type());
         buf = buf == 2 ? 0 : buf + 1;
     }
@@ -886,12 +895,12 @@ __global__ void __launch_bounds__(512)
     for (int t = 0; t < DT; t++) sum[t] = float4_t{0, 0, 0, 0};
     float l_sum = 0.0f, l_tot = 0.0f;
     const bool few = n_splits <= 8;
-    for (int split = 0, at = 0; at < n_splits; at++) {
+    for (int split = 0, at = 0, next; at < all_splits; at++, split = next) {
         const bool ends = split + 8 >= n_splits;  // the last of this one's eighth
-        const int next = ends ? (split & 7) + 1 : split + 8;
+        next = split + 8 >= all_splits ? (split & 7) + 1 : split + 8;
         landed(0);
         const uint32_t buf = at & 1 ? 0 : 3 * kPairKeys;
-        if (at + 1 < n_splits) load(next, true, lds_b + (at & 1 ? 3 * kPairKeys : 0));
+        if (at + 1 < all_splits) load(next, true, lds_b + (at & 1 ? 3 * kPairKeys : 0));
         auto merge = [&](auto masked, auto of_few) {
             constexpr bool kFew = decltype(of_few)::value;
             float p[16];
@@ -947,6 +956,7 @@ __global__ void __launch_bounds__(512)
                 if constexpr (I + kRing < 4 * KS + 2 * DT) read(std::integral_constant<int, I + kRing>(), buf);
             });
         };
+        if (split >= n_splits) continue;
         if (few && edge(split))
             merge(std::true_type(), std::true_type());
         else if (few)
@@ -976,8 +986,8 @@ __global__ void __launch_bounds__(512)
                 }
             }
         }
-        split = next;
     }
+    if (n_splits == 0) return;
     if (few) l_tot = l_sum;
 #pragma unroll
     for (int t = 0; t < DT; t++) {
@@ -1329,11 +1339,11 @@ int32_t launch_rows(dflash_ctx *ctx, dim3 grid, int n_waves, hipStream_t st, con
     DFL_HIP_CHECK(ctx, hipGetLastError());
     return DFLASH_OK;
 }
-int32_t launch_rows_pair(dflash_ctx *ctx, dim3 grid, int n_waves, hipStream_t st, const float *q, const _Float16 *k, const _Float16 *vt, int64_t ctx_len,
+int32_t launch_rows_pair(dflash_ctx *ctx, dim3 grid, int n_waves, int heads, hipStream_t st, const float *q, const _Float16 *k, const _Float16 *vt, int64_t ctx_len,
                          int n_rows, int n_q, int n_kv, int64_t vt_stride, float scale, float *out, void *out_xf, int out_xf_kind) {
     if (const int32_t rc_ = dfl_raise_lds_limit(ctx, reinterpret_cast<const void *>(attn_rows_pair_kernel), kPairLds)) return rc_;
     attn_rows_pair_kernel<<<grid, 64 * n_waves, kPairLds, st>>>(q, k, vt, ctx_len, n_rows, n_q, n_kv, vt_stride, scale, out, out_xf, out_xf_kind,
-                                                                dfl_xf_bytes(static_cast<int64_t>(n_q) * 256));
+                                                                dfl_xf_bytes(static_cast<int64_t>(n_q) * 256), heads);
     DFL_HIP_CHECK(ctx, hipGetLastError());
     return DFLASH_OK;
 }
@@ -1514,25 +1524,28 @@ int32_t dfl_attn_blocks(dflash_ctx *ctx, const void *q, int32_t q_type, const vo
         int hw = std::min(group, 8);
         while (group % hw) hw--;
         const int32_t rows = std::min(n_rows_total, 16 * taken);
-        // heads of 256, half the waves on a workgroup's splits where those workgroups still fit the chip side by side: 2.6 us a
-        // split instead of 3.4 (16 / 2 heads, 1024 rows 85 -> 67 us; 2048 rows, twice the chip's CUs, 157 : 154)
-        if (head_dim == 256 && hw == 8 && static_cast<int64_t>(taken) * n_kv * (group / 4) <= ctx->n_cu) hw = 4;
-        const int64_t wgs = static_cast<int64_t>(taken) * n_kv * (group / hw), n_steps = (ctx_len + rows + 31) / 32;
+        // Heads of 256: four heads of a block where those workgroups fit the chip side by side, 2.6 us a split (with eight heads 3.4:
+        // 16 / 2 heads, 1024 rows 85 -> 67 us); beyond, four heads of two blocks, a long one and a short one, as
+        // attn_rows_pair_kernel has them: 3.2 us for a split of the longest (1536 rows 117 -> 94 us, 2048 rows 147 -> 124).
+        const bool fours = head_dim == 256 && hw % 4 == 0, two = fours && static_cast<int64_t>(taken) * n_kv * (group / 4) > ctx->n_cu;
+        if (fours) hw = 4;
+        const int32_t units = two ? (taken + 1) / 2 : taken;
+        const int64_t wgs = static_cast<int64_t>(units) * n_kv * (group / hw), n_steps = (ctx_len + rows + 31) / 32;
         const int64_t stages = wgs * (ctx_len + rows / 2) / 32;
         const double as_splits = (head_dim == 256 ? 20.0 : 11.0) * runs.n + (0.5 * stages + 1.1 * partials) / ctx->n_cu;
         double one_launch = 5.5 + 1.15 * n_steps;
-        // Heads of 256 walk the keys twice: 14 us and 2.6, 3.4 or (workgroups of neither four nor eight heads) 4.2 us for a split of
+        // Heads of 256 walk the keys twice: 14 us and 2.6, 3.2 or (workgroups of another number of heads than four) 4.2 us for a split of
         // two stages, 8 us more where the total goes out and back; the two launches of a run 20 us.  Both sides in us, the last layer's worth of 95 measured
         // pairs (splits : one launch): 16 / 2 heads 452 : 154 for 2048 rows behind none, 60 : 36 for 512, 155 : 111 for 512 behind
         // 1520, 71 : 98 for 256 behind 1520, 38 : 149 for 64 behind 3040; 8 / 1 heads 74 : 107 and 161 : 129 for 512 and 1024
         // behind 1520; 32 / 4 heads 43 : 25 for 256 behind none; 5 / 1 heads 191 : 193 for 2048 behind none.
         if (head_dim == 256)
-            one_launch = (n_steps > 16 ? 22.0 : 14.0) + (hw == 4 ? 2.6 : hw == 8 ? 3.4 : 4.2) * std::max(0.5 * n_steps, 0.65 * stages / ctx->n_cu);
+            one_launch = (n_steps > 16 ? 22.0 : 14.0) + (two ? 3.2 : fours ? 2.6 : 4.2) * std::max(0.5 * n_steps, 0.65 * stages / ctx->n_cu);
         if (taken > 1 && one_launch <= as_splits) {
             hipStream_t st = static_cast<hipStream_t>(stream);
             dfl_timed timer(ctx, st, DFL_T_ATTN);
             if (head_dim == 256) {
-                if (const int32_t rc_ = launch_rows_pair(ctx, dim3(group / hw, n_kv, taken), hw, st, static_cast<const float *>(q),
+                if (const int32_t rc_ = launch_rows_pair(ctx, dim3(group / hw, n_kv, units), two ? 8 : hw, hw, st, static_cast<const float *>(q),
                                                          static_cast<const _Float16 *>(k_cache), static_cast<const _Float16 *>(vt_cache), ctx_len, rows, n_q,
                                                          n_kv, kv_capacity, scale, out, out_xf, out_xf_kind))
                     return rc_;

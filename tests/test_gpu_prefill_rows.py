@@ -44,6 +44,7 @@ SHAPES["loop4096"] = (dfl.ModelConfig(n_layers=2, hidden=4096, n_q=64, n_kv=4, h
 # (a mixture's projections in Q4_K: wo of 16 super-blocks, by sums that no kernel ahead of it has left)
 SHAPES["experts_q4k"] = (dfl.ModelConfig(n_layers=3, hidden=2048, n_q=16, n_kv=2, head_dim=256, ffn=0, vocab=2048, n_expert=32, n_expert_used=4,
                                          ffn_expert=768, ffn_shared=768), dfl.synth.Q4_K)
+SHAPES["heads256x64"] = (dfl.ModelConfig(n_layers=2, hidden=1024, n_q=64, n_kv=16, head_dim=256, ffn=3072, vocab=2048), dfl.synth.Q4_K)
 SHAPES["heads256x12"] = (dfl.ModelConfig(n_layers=2, hidden=1024, n_q=12, n_kv=1, head_dim=256, ffn=3072, vocab=2048), dfl.synth.Q4_K)
 
 
@@ -107,6 +108,13 @@ def test_continued_prefill_equals_block_by_block(ctx, shape, head, rows):
 def test_heads_of_256_equal_block_by_block(ctx, shape, head, rows):
     """Keys walked twice in one workgroup against splits and their merge: one, four, five, six and eight waves, up to eight
     splits (the total in registers) and more (in the output rows, also where the last block is short), a last split of one stage and of two."""
+    test_continued_prefill_equals_block_by_block(ctx, shape, head, rows)
+
+
+@pytest.mark.parametrize("shape,head,rows", [("experts", 0, 1030), ("experts", 37, 1041), ("heads256x64", 0, 272), ("heads256x64", 0, 287), ("heads256x64", 450, 318)])
+def test_two_blocks_a_workgroup_equal_block_by_block(ctx, shape, head, rows):
+    """Heads of 256 beyond a workgroup a CU: even and odd numbers of blocks (one in the middle without a second), a short last
+    block, up to eight splits in both blocks of a workgroup, in the second alone and in neither."""
     test_continued_prefill_equals_block_by_block(ctx, shape, head, rows)
 
 
