@@ -1448,7 +1448,17 @@ static AttnPolicy attn_policy(const dflash_ctx *ctx, int64_t bucket, int n_kv, i
     static const int env_hw = [] { const char *e = getenv("DFLASH_ATTN_HW"); return e ? atoi(e) : 0; }();
     if (env_per_cu > 0) per_cu_x2 = 2 * env_per_cu;
     if (env_min_chunk > 0) min_chunk = env_min_chunk;
-    if (env_hw > 0 && group % env_hw == 0) hw = env_hw;
+    // A workgroup of one wave asks for a whole stage by itself, with a table's loads ahead of it where the attention rotates (65 loads a
+    // split, heads of 256), and none of its SIMD's time is another's: two heads at least, with heads of 128 four, where the rule
+    // above divides further.  What covers the chip decides on the split (want) all the same: the same bits.  A call at 330 positions,
+    // one, two and four heads a workgroup, 16 rows / one row: 16 / 2 heads of 256 12.4, 10.5, 11.4 / 11.7, 9.3, 9.3 us; 32 / 8 of
+    // 128 9.1, 8.4, 8.5 / 8.3, 7.5, 7.2; 16 / 8 of 128 8.6, 7.9 / 8.2, 7.4; 16 / 4 of 64 7.2, 6.5, 6.7 / 7.0, 6.2, 6.3; at
+    // 1000 positions by as much.  With the rotation inside, of a layer: 16 / 2 of 256 3.2, 2.5 / 2.7, 3.1 less than with one head, 32 / 8 of 128
+    // 1.1, 2.9 / 1.8, 2.6.  (Six heads of 128 keep their one part or two: 48 / 8 at 1500 positions, 13.7 : 12.3 / 8.4 : 8.8.)
+    int served = hw;
+    const int least = head_dim == 128 ? 4 : 2;
+    while (2 * served <= least && group % (2 * served) == 0) served *= 2;
+    if (env_hw > 0 && group % env_hw == 0) served = hw = env_hw;
     if (per_cu_x2 < 1) per_cu_x2 = 1;
     if (min_chunk < 32) min_chunk = 32;
     const int n_parts = group / hw;
@@ -1466,7 +1476,7 @@ static AttnPolicy attn_policy(const dflash_ctx *ctx, int64_t bucket, int n_kv, i
     // 100 k keys, 101.3 -> 102.7 us with the attention).  By the most splits any context of the bucket can have, not the
     // launch's: the bits must not depend on it.
     const int64_t max_splits = std::min<int64_t>(want, (2 * bucket - 1 + min_chunk - 1) / min_chunk);
-    return {want, min_chunk, hw, head_dim < 256 && max_splits <= kOrderedSplits};
+    return {want, min_chunk, served, head_dim < 256 && max_splits <= kOrderedSplits};
 }
 
 // Loads of rows, table and weights are of 16 bytes; a chunk goes over as sixteen bits of stages.  Beside its heads' waves a workgroup has two more: with

@@ -96,6 +96,21 @@ def test_equals_sixteen_single_query_attentions(ctx, canaries):
         np.testing.assert_allclose(one[0], packed[i], atol=2e-3, rtol=2e-3)
 
 
+@pytest.mark.parametrize("n_q,n_kv,hd", [(16, 2, 256), (6, 2, 256), (24, 2, 256), (32, 8, 128), (10, 5, 128), (12, 2, 128), (24, 3, 128), (16, 4, 64), (10, 1, 64)])
+@pytest.mark.parametrize("L,n_rows", [(0, 1), (33, 16), (330, 16), (640, 1), (671, 16)])
+def test_heads_of_a_workgroup_equal_heads_one_by_one(ctx, n_q, n_kv, hd, L, n_rows, canaries):
+    """Short contexts, where a workgroup has two to four heads of a group (fewer, and more, where they do not come out even):
+    every head has the bits of a call of its own.  (Up to 704 positions: there the eleven splits that 24 heads of three or two groups
+    may have are of 64 keys, as a single head's are.)"""
+    q, k, v, cap = make_case(L + n_q, L, n_rows, n_q, n_kv, hd)
+    scale, vt = 1.0 / math.sqrt(hd), np.ascontiguousarray(v.transpose(1, 2, 0))
+    got = ctx.attn_verify_block(dev(q), dev(k), dev(vt), L, scale, v_transposed=True).cpu().numpy()
+    for head in range(n_q):
+        kv = head * n_kv // n_q
+        one = ctx.attn_verify_block(dev(q[:, head:head + 1]), dev(k[:, kv:kv + 1]), dev(vt[kv:kv + 1]), L, scale, v_transposed=True).cpu().numpy()
+        assert np.array_equal(got[:, head], one[:, 0]), f"head {head}"
+
+
 @pytest.mark.parametrize("L", [32768, 131072])
 def test_attn_long_context(ctx, oracle, L, canaries):
     """production shape: 48 q / 8 kv heads, hd 128; checked on a few heads against the oracle
