@@ -973,6 +973,18 @@ int prefill_group_blocks() {
     return std::max(0, std::min(kMaxGroupRows / 16, v));
 }
 
+// Rows of the next pass where `left` are to come from position `at` on and a pass holds `most`: full passes, but a prompt of two, the
+// second of an eighth at least, goes as two of the same size: the many-row products of few rows leave CUs idle or their tiles half full.
+// (A shorter rest is cheap by itself, and two halves would lose more of the expert tiles' fill.)  ms of full passes : equal ones, 2310, 2500,
+// 2800 and 3000 tokens: five layers of the 27B shape 9.33 : 8.15, 9.90 : 9.00, 10.56 : 9.99, 11.10 : 10.71; eight of the 35B-A3B shape 8.58 :
+// 8.33, 8.95 : 8.71, 9.72 : 9.50, 10.10 : 9.65; eight of a 1024-wide one 3.73 : 3.75, 4.23 : 3.94, 4.52 : 4.48, 4.73 : 4.70.  2100 tokens (52 behind
+// a full pass) 8.30 : 7.79, 7.16 : 7.81, 3.21 : 3.45.  Three passes, 4380 tokens, 16.96 : 15.93, 15.44 : 15.90, 7.79 : 8.09: there a
+// pass of equal size crosses the length from which the attention goes by splits.
+int32_t prefill_pass_rows(int32_t most, int32_t left, int64_t at) {
+    if (at || left < most + most / 8 || left > 2 * most) return std::min(most, left);
+    return ((left + 1) / 2 + 15) / 16 * 16;
+}
+
 // Sets the group scratch up; leaves it empty (no error) where the shape is not one the grouped path takes or the memory
 // is not there.
 void prefill_group_alloc(dflash_session *s, PrefillGroup *g) {
@@ -1681,8 +1693,8 @@ int32_t dflash_prefill_blocks(dflash_ctx *ctx, const dflash_model *model, dflash
     if (start + n_tokens <= 0x7fffffffll && prefill_group_takes(ctx, model, p->group)) {
         // rows of many blocks per pass (see PrefillGroup); the caller's stream alone
         const size_t cap_row = static_cast<size_t>(std::max(n_taps, 0)) * c.hidden;
-        for (int32_t t0 = 0; t0 < n_tokens; t0 += p->group.rows) {
-            const int32_t n = std::min<int32_t>(p->group.rows, n_tokens - t0);
+        for (int32_t t0 = 0, n; t0 < n_tokens; t0 += n) {
+            n = prefill_pass_rows(p->group.rows, n_tokens - t0, start + t0);
             if ((rc = prefill_group_enqueue(ctx, model, s, p->group, tokens + t0, n, start + t0, tap_layers, n_taps,
                                             hidden_capture ? hidden_capture + static_cast<size_t>(t0) * cap_row : nullptr,
                                             static_cast<hipStream_t>(stream)))) {
@@ -1768,7 +1780,8 @@ int32_t dflash_prefill_prompt(dflash_ctx *ctx, const dflash_model *model, dflash
     // 0.70 : 0.51, 0.90 : 0.61, 1.26 : 0.93, 3.16 : 2.76.
     int32_t body = 0;
     bool tail_group = n_tokens > 16 && start + n_tokens <= 0x7fffffffll && prefill_group_takes(ctx, model, g);
-    if (tail_group) body = (n_tokens - 1) / g.rows * g.rows;
+    if (tail_group)
+        for (body = 0; n_tokens - body > g.rows;) body += prefill_pass_rows(g.rows, n_tokens - body, start + body);
     tail_group = tail_group && n_tokens - body > 16;
     if (!tail_group) body = (n_tokens - 1) / 16 * 16;
     if (body && (rc = dflash_prefill_blocks(ctx, model, s, tokens, body, start, tap_layers, n_taps, hidden_capture, stream))) return rc;

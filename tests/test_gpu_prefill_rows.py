@@ -269,6 +269,13 @@ def test_a_prompt_in_one_call_equals_its_blocks_and_their_last_one(ctx, shape, a
     one.close()
 
 
+@pytest.mark.parametrize("shape,rows", [("experts", 2303), ("experts", 2304), ("narrow", 3011), ("narrow", 4361)])
+def test_prompts_of_several_passes_equal_block_by_block(ctx, shape, rows):
+    """More rows than a pass holds (2048): a full pass and a short rest, two passes of the same size, full passes and a rest, in both calls."""
+    test_continued_prefill_equals_block_by_block(ctx, shape, 0, rows)
+    test_a_prompt_in_one_call_equals_its_blocks_and_their_last_one(ctx, shape, True, rows, [0], 0)
+
+
 def test_a_prompt_in_one_call_keeps_the_guards(ctx):
     cfg, attn_type = SHAPES["narrow"]
     model = dfl.TargetModel(ctx, cfg, dfl.synth_target_weights_device(cfg, 5, "cuda", attn_type=attn_type))
