@@ -254,7 +254,8 @@ int32_t dfl_gemm_whole_blocks(dflash_ctx *ctx, int32_t w_type, const void *w, co
 bool dfl_whole_holds_weights(const dflash_ctx *ctx, int32_t w_type, int64_t n_in, int64_t n_out);
 
 // The whole-K kernel on rows in row order (f32 or f16), for the public operator: y[n_rows][n_out] = x . w^T in one launch, for Q4_K in either
-// order and Q6_K in row order; the same bits for both orders.
+// order and Q6_K in row order; the same bits for both orders.  (Null and misaligned weights and overlapping buffers are gemm_fewrow_impl's to refuse,
+// which every caller comes through.)
 bool dfl_gemm_direct_takes(const dflash_ctx *ctx, int32_t w_type, int64_t n_in, int64_t n_out);
 int32_t dfl_gemm_direct(dflash_ctx *ctx, int32_t w_type, const void *w, const void *x, int32_t x_type, float *y, int64_t n_in, int64_t n_out,
                         int32_t n_rows, hipStream_t stream);
@@ -433,6 +434,9 @@ int32_t dfl_attn_blocks(dflash_ctx *ctx, const void *q, int32_t q_type, const vo
 // dflash_gemm_fewrow for a tensor of a model that passed dfl_model_tensors_checked (the fast kernels).
 int32_t dfl_gemm_fewrow_checked(dflash_ctx *ctx, int32_t w_type, const void *w, const void *x, int32_t x_type, float *y,
                                 int64_t n_in, int64_t n_out, int32_t n_rows, dflash_stream_t stream);
+// The same by the public operator's routes: small matrices in one launch, whose cuts of K a prompt's products do not share.
+int32_t dfl_gemm_fewrow_one(dflash_ctx *ctx, int32_t w_type, const void *w, const void *x, int32_t x_type, float *y, int64_t n_in,
+                            int64_t n_out, int32_t n_rows, dflash_stream_t stream);
 
 // Few-row Q6_K GEMMs of up to three matrices over the same activations (a layer's q, k and v
 // projections) as one launch: y[m] = x . w[m]^T, [n_rows][n_out[m]] each.

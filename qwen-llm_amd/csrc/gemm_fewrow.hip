@@ -3595,6 +3595,11 @@ int32_t dfl_gemm_fewrow_checked(dflash_ctx *ctx, int32_t w_type, const void *w, 
     return gemm_fewrow_impl(ctx, w_type | DFLASH_TYPE_RANGE_CHECKED, w, x, x_type, y, n_in, n_out, n_rows, stream, false);
 }
 
+int32_t dfl_gemm_fewrow_one(dflash_ctx *ctx, int32_t w_type, const void *w, const void *x, int32_t x_type, float *y, int64_t n_in,
+                            int64_t n_out, int32_t n_rows, dflash_stream_t stream) {
+    return gemm_fewrow_impl(ctx, w_type | DFLASH_TYPE_RANGE_CHECKED, w, x, x_type, y, n_in, n_out, n_rows, stream, true);
+}
+
 namespace {
 
 int32_t gemm_fewrow_impl(dflash_ctx *ctx, int32_t w_type, const void *w, const void *x, int32_t x_type, float *y, int64_t n_in,

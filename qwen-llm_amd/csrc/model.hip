@@ -641,6 +641,10 @@ int32_t gemm(dflash_ctx *ctx, const dflash_qtensor &w, const float *x, float *y,
              hipStream_t st) {
     return dfl_gemm_fewrow_checked(ctx, w.type, w.data, x, DFLASH_TYPE_F32, y, n_in, n_out, n, st);
 }
+int32_t gemm_one(dflash_ctx *ctx, const dflash_qtensor &w, const float *x, float *y, int64_t n_in, int64_t n_out, int n,
+                 hipStream_t st) {
+    return dfl_gemm_fewrow_one(ctx, w.type, w.data, x, DFLASH_TYPE_F32, y, n_in, n_out, n, st);
+}
 
 // True if b's rows follow a's rows_a rows directly in memory and both have the same type: the two
 // are then one matrix of more rows, and one GEMM serves both (its output rows hold a's columns, then
@@ -789,12 +793,6 @@ int32_t begin_rows(dflash_ctx *ctx, const dflash_qtensor &t, const BlockBegin &b
                                                                                          head_dim, theta);
     return DFLASH_OK;
 }
-// A few rows through a small matrix in one launch, where the public operator has one for it (whose cuts of K a prompt's products do not share).
-int32_t gemm_one(dflash_ctx *ctx, const dflash_qtensor &w, const float *x, float *y, int64_t n_in, int64_t n_out, int n, hipStream_t st) {
-    if (dfl_gemm_direct_takes(ctx, w.type, n_in, n_out)) return dfl_gemm_direct(ctx, w.type, w.data, x, DFLASH_TYPE_F32, y, n_in, n_out, n, st);
-    return gemm(ctx, w, x, y, n_in, n_out, n, st);
-}
-
 }  // namespace
 
 struct dflash_session {

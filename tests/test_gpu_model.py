@@ -308,6 +308,49 @@ def test_separate_and_adjacent_weight_layouts_agree(ctx, oracle, wtype):
     close(outs["adjacent"][2], outs["separate"][2], "adjacent vs separate draft logits")
 
 
+def test_a_drafter_with_a_null_or_misaligned_matrix_is_refused_before_it_is_read(ctx):
+    """The two products that go by the public operator's one-launch routes (fc of the context columns, the selector's gate) keep its
+    guards: a null pointer is DFLASH_ERR_INVALID_INPUT, tiled Q4_K off 128 bytes and row-order Q4_K off 16 DFLASH_ERR_ALIGNMENT, and no
+    product is launched; with the pointer back in its place the block is the one of a session of its own."""
+    import torch
+    cfg = dfl.ModelConfig(n_layers=1, hidden=512, n_q=4, n_kv=2, head_dim=64, ffn=512, vocab=1024)
+    dcfg = dfl.DraftConfig(n_layers=1, hidden=512, n_q=4, n_kv=2, head_dim=64, ffn=512, block_size=8, n_taps=2, conv_kernel_size=2,
+                           conv_group_size=64, selector_rank=256, selector_top_k=16)
+    model = dfl.TargetModel(ctx, cfg, dfl.synth_target_weights_device(cfg, 5, "cuda"))
+    head = dfl.DraftHead(ctx, dcfg, dfl.synth_draft_weights_device(dcfg, 6, "cuda", vocab=cfg.vocab))
+    cols = torch.randn((20, 2, 512), generator=torch.Generator(device="cuda").manual_seed(3), device="cuda")
+
+    def session():
+        d = dfl.DraftSession(ctx, head, model, 64)
+        d.append_target_ctx_columns(cols, list(range(20)))
+        return d
+
+    clean = session()
+    want = clean.draft_block(5, cfg.vocab - 1, 20, want_logits=True)[1].clone()
+    clean.close()
+    assert head.c.fc.type == dfl.TYPE_Q4_K_TILED and head.c.selector_hidden.type == dfl.TYPE_Q4_K
+    d = session()
+    for name, off, calls in (("fc", 64, (d.prepare_ctx, lambda: d.draft_block(5, cfg.vocab - 1, 20))),
+                             ("selector_hidden", 8, (lambda: d.draft_block(5, cfg.vocab - 1, 20),))):
+        tensor = getattr(head.c, name)
+        at = tensor.data
+        for pointer, status in ((None, 7), (at + off, 4)):
+            tensor.data = pointer
+            try:
+                for call in calls:
+                    ctx.set_kernel_timing(1)
+                    with pytest.raises(dfl.DFlashError) as e:
+                        call()
+                    assert e.value.status == status
+                    if name == "fc":
+                        assert ctx.kernel_timing(0)[1] == 0
+            finally:
+                ctx.set_kernel_timing(0)
+                tensor.data = at
+    assert torch.equal(d.draft_block(5, cfg.vocab - 1, 20, want_logits=True)[1], want)
+    d.close()
+
+
 @pytest.mark.parametrize("codebook_type", [dfl.TYPE_Q4_K, dfl.TYPE_Q8_0])
 def test_dflash2_draft_block_matches_oracle(ctx, oracle, target, codebook_type):
     """A DFlash-2 head (two-tap dynamic convolutions around both sublayers, block of 8, selector of rank
