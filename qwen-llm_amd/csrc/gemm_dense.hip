@@ -244,9 +244,10 @@ bool dfl_gemm_dense_pair_takes(const dflash_ctx *ctx, int32_t w_type, int64_t n_
 int32_t dfl_gemm_dense_pair(dflash_ctx *ctx, int32_t w_type, const void *w, const void *xf, const void *xs, void *y_f16, int64_t n_in, int64_t ffn,
                             int32_t n_rows, hipStream_t st) {
     const DensePlan p = dense_plan(ctx, w_type, n_in, ffn);
-    if (!p.units || !w || !xf || !xs || !y_f16 || n_rows < 1 || n_rows > 16 || reinterpret_cast<uintptr_t>(w) % 16 || reinterpret_cast<uintptr_t>(xf) % 16 ||
-        reinterpret_cast<uintptr_t>(xs) % 16)
-        return dfl_fail(ctx, DFLASH_ERR_UNSUPPORTED, "gemm_dense_pair: shape not taken, null or misaligned operand");
+    if (!p.units || n_rows < 1 || n_rows > 16) return dfl_fail(ctx, DFLASH_ERR_UNSUPPORTED, "gemm_dense_pair: shape not taken");
+    if (!w || !xf || !xs || !y_f16) return dfl_fail(ctx, DFLASH_ERR_INVALID_INPUT, "gemm_dense_pair: null pointer");
+    if (reinterpret_cast<uintptr_t>(w) % 128 || reinterpret_cast<uintptr_t>(xf) % 16 || reinterpret_cast<uintptr_t>(xs) % 16)
+        return dfl_fail(ctx, DFLASH_ERR_ALIGNMENT, "gemm_dense_pair: tiled Q4_K weights must be 128-byte aligned, rows 16-byte aligned");
     if (const int32_t rc = dfl_raise_lds_limit(ctx, reinterpret_cast<const void *>(gemm_q4k_dense_pair_kernel), p.lds)) return rc;
     dfl_timed timer(ctx, st, DFL_T_GEMM);
     gemm_q4k_dense_pair_kernel<<<p.n_wg, 64 * (2 * p.per + 1), p.lds, st>>>(

@@ -44,3 +44,19 @@ def test_wide_ffn_matches_oracle_and_the_prompts_rows(ctx, oracle, hidden, ffn):
     assert torch.equal(got, torch.cat(rows))
     one.close()
     many.close()
+
+
+def test_misaligned_weights_are_refused(ctx):
+    """Tiled Q4_K off 128 bytes is refused, as by every other kernel that reads that order, and the session goes on where it was."""
+    cfg = dfl.ModelConfig(n_layers=1, hidden=1280, n_q=4, n_kv=2, head_dim=128, ffn=12544, vocab=512)
+    model = dfl.TargetModel(ctx, cfg, dfl.synth_target_weights_device(cfg, 23, "cuda"))
+    sess = dfl.Session(ctx, model, 64, [0])
+    layer = model.c.layers[0]
+    at = layer.gate.data, layer.up.data
+    layer.gate.data, layer.up.data = at[0] + 64, at[1] + 64
+    with pytest.raises(dfl.DFlashError) as e:
+        sess.encode_packed_verify_layer_major([1, 2, 3], 0)
+    assert e.value.status == 4 and sess.kv_n_pos == 0
+    layer.gate.data, layer.up.data = at
+    sess.encode_packed_verify_layer_major([1, 2, 3], 0)
+    sess.close()
