@@ -770,6 +770,16 @@ int32_t gemm_gate_up(dflash_ctx *ctx, const dflash_qtensor &gate, const dflash_q
     return DFLASH_OK;
 }
 
+// A dense layer's down projection of rows in row order.  A tiled Q6_K matrix is read in fragment order only: its rows are packed first (xf: room for
+// them; kind: the matrix's, from layer_xf), to the bits that a prompt's rows get from a gate | up launch that writes that order.
+int32_t gemm_down(dflash_ctx *ctx, const dflash_qtensor &down, int kind, const void *g, int32_t g_type, void *xf, float *y, int64_t ffn,
+                  int64_t n_out, int n, hipStream_t st) {
+    if (down.type != DFLASH_TYPE_Q6_K_TILED || kind == DFL_XF_NONE)
+        return dfl_gemm_fewrow_checked(ctx, down.type, down.data, g, g_type, y, ffn, n_out, n, st);
+    if (const int32_t rc = dflash_pack_xf(ctx, g, g_type, n, ffn, kind, xf, st)) return rc;
+    return dfl_gemm_whole(ctx, down.type, down.data, xf, y, ffn, n_out, n, 0, nullptr, DFL_XF_NONE, st);
+}
+
 int32_t embed_rows(dflash_ctx *ctx, const dflash_qtensor &t, const int32_t *ids_dev, int n, int hidden, float *out,
                    hipStream_t st) {
     size_t rb = dflash_row_bytes(t.type, hidden);
@@ -1253,12 +1263,10 @@ int32_t verify_enqueue(dflash_ctx *ctx, const dflash_model *model, dflash_sessio
             else
                 rc = gemm_gate_up(ctx, L.gate, L.up, s->cur, s->g, s->u, s->pk, H, c.ffn, n, st, s->xf_cur, xk.gate_up, s->xf_g, down_kind, true);
             if (rc) return rc;
-            if (dense_pair)
-                rc = dfl_gemm_fewrow_checked(ctx, L.down.type, L.down.data, s->g, DFLASH_TYPE_F16, s->mix, c.ffn, H, n, st);
-            else if (down_kind)
+            if (down_kind)
                 rc = dfl_gemm_whole(ctx, L.down.type, L.down.data, s->xf_g, s->mix, c.ffn, H, n, 0, nullptr, DFL_XF_NONE, st, true);
             else
-                rc = gemm(ctx, L.down, s->g, s->mix, c.ffn, H, n, st);
+                rc = gemm_down(ctx, L.down, xk.down, s->g, dense_pair ? DFLASH_TYPE_F16 : DFLASH_TYPE_F32, s->xf_g, s->mix, c.ffn, H, n, st);
             if (rc) return rc;
             // x += mix: by the next norm, which also captures the sum; where there is none, or the layer is captured more than once, here
             const bool norm_follows = norm_in_registers(H) && (il + 1 < c.n_layers || want_head);
@@ -2208,7 +2216,7 @@ int32_t draft_block_impl(dflash_ctx *ctx, const dflash_model *target, const dfla
         if (down_kind)
             rc = dfl_gemm_whole(ctx, L.down.type, L.down.data, s->xf_g, s->mix, c.ffn, H, N, 0, nullptr, DFL_XF_NONE, st);
         else
-            rc = gemm(ctx, L.down, s->g, s->mix, c.ffn, H, N, st);
+            rc = gemm_down(ctx, L.down, xk.down, s->g, DFLASH_TYPE_F32, s->xf_g, s->mix, c.ffn, H, N, st);
         if (rc) return rc;
         resid = s->mix;
         pending_conv = ConvResid();

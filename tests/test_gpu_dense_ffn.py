@@ -46,6 +46,43 @@ def test_wide_ffn_matches_oracle_and_the_prompts_rows(ctx, oracle, hidden, ffn):
     many.close()
 
 
+@pytest.mark.parametrize("adjacent", [True, False], ids=["one launch", "separate products"])
+@pytest.mark.parametrize("tiled", [True, False], ids=["tiled", "row order"])
+@pytest.mark.parametrize("hidden,ffn", [(2304, 4608), (1280, 8192)])
+def test_down_in_q6k_behind_rows_in_row_order(ctx, oracle, hidden, ffn, tiled, adjacent):
+    """A Q6_K down projection in both orders behind a gate | up that leaves its rows in row order (the one launch, as f16; separate products, as
+    f32): blocks, a prompt's rows and a prompt in one call.  Only fragment-order rows go through the tiled order, so a block packs them."""
+    cfg = dfl.ModelConfig(n_layers=2, hidden=hidden, n_q=4, n_kv=2, head_dim=128, ffn=ffn, vocab=512)
+    w, rng = dfl.synth_target_weights_blocks(cfg, 29), np.random.default_rng(31)
+    for layer in w["layers"]:
+        layer["down"] = (dfl.TYPE_Q6_K, dfl.synth.random_blocks_scaled(dfl.TYPE_Q6_K, hidden, ffn, ffn ** -0.5, rng))
+    model = dfl.TargetModel(ctx, cfg, w, adjacent=adjacent)
+    tensors = []
+    for il, layer in enumerate(w["layers"] if tiled else ()):
+        assert ctx.xf_kind(dfl.TYPE_Q6_K_TILED, ffn, hidden) == dfl.XF_Q6K
+        tensors.append(ctx.repack_q6k_tiled(torch.from_numpy(layer["down"][1]).cuda(), ffn, hidden))
+        model.c.layers[il].down = type(model.c.layers[il].down)(dfl.TYPE_Q6_K_TILED, model.c.layers[il].down.flags, tensors[-1].data_ptr())
+    omodel, _keep = oracle.build_model(cfg.as_dict(), w)
+    one, many, prompt = (dfl.Session(ctx, model, 64, [0, 1]) for _ in range(3))
+    ostate = oracle.TargetState(cfg.as_dict(), 64)
+    tokens = np.random.default_rng(ffn).integers(0, cfg.vocab, 40).tolist()
+    rows = []
+    for at, n in ((0, 16), (16, 16), (32, 1), (33, 7)):
+        out = one.encode_packed_verify_layer_major(tokens[at:at + n], at)
+        _, want = oracle.target_verify(omodel, ostate, tokens[at:at + n], at, [0, 1])
+        rows.append(out.hidden_capture)
+        # (as above, two layers of it)
+        d = rows[-1].cpu().numpy().astype(np.float64) - want
+        rms = np.sqrt(np.mean(np.square(want, dtype=np.float64)))
+        assert np.linalg.norm(d) / np.linalg.norm(want) <= 5e-3
+        assert np.max(np.abs(d) / np.maximum(np.abs(want), rms)) <= 3e-2
+    assert torch.equal(many.prefill_blocks(tokens, 0), torch.cat(rows))
+    hidden_rows, last = prompt.prefill_prompt(tokens, 0)
+    assert torch.equal(hidden_rows, torch.cat(rows)) and last == out.argmax_host[-1]
+    for s in (one, many, prompt):
+        s.close()
+
+
 def test_misaligned_weights_are_refused(ctx):
     """Tiled Q4_K off 128 bytes is refused, as by every other kernel that reads that order, and the session goes on where it was."""
     cfg = dfl.ModelConfig(n_layers=1, hidden=1280, n_q=4, n_kv=2, head_dim=128, ffn=12544, vocab=512)
