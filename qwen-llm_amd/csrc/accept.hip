@@ -1164,7 +1164,6 @@ int32_t dflash_accept_prefix(dflash_ctx *ctx, const int32_t *verified, int32_t n
         static_assert(sizeof(dflash_accept_decision) <= DFL_PINNED_BYTES, "the decision is read back through the pinned page");
         void *const pinned_dev = ctx->pinned_dev;
         const bool direct = pinned_dev != nullptr;
-        if (!direct) (void)hipGetLastError();
         decide_kernel<<<1, kDecThreads, 0, st>>>(rows, tile_sums, direct ? static_cast<dflash_accept_decision *>(pinned_dev) : d_out, mode, n_tiles,
                                                  n_tokens, a);
         DFL_HIP_CHECK(ctx, hipGetLastError());
