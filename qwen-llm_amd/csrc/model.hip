@@ -599,7 +599,7 @@ __global__ void step_readback_kernel(const int32_t *__restrict__ argmax, const f
     const int i = threadIdx.x;
     if (i < n) {
         out[i] = argmax[i];
-        if (draft) out[16 + i] = draft[i];
+        out[16 + i] = draft[i];
         out[32 + i] = __float_as_int(gap[i]);
     }
 }
