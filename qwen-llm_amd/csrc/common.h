@@ -288,6 +288,8 @@ int32_t dfl_xf_sums(dflash_ctx *ctx, const void *xf, int64_t n_in, int32_t n_blo
 // sums to y_xs unless null) instead.  make_sums: xs is to be computed first, where the plan needs it.
 int32_t dfl_gemm_rows(dflash_ctx *ctx, const dfl_rows_plan &plan, int32_t w_type, const void *w, const void *xf, void *xs, bool make_sums, float *y,
                       int64_t n_in, int64_t n_out, int32_t n_rows, int64_t pair_ffn, void *y_xf, void *y_xs, int y_kind, hipStream_t stream);
+// What a product of n_rows rows costs by the measure that picks its tiles: rounds of the chip times what a tile takes, over its super-blocks.
+double dfl_gemm_rows_cost(const dflash_ctx *ctx, const dfl_rows_plan &p, int64_t n_in, int64_t n_out, int32_t n_rows, int64_t pair_ffn);
 // The experts' products over row tiles listed on the device, tiles[i] = {expert (-1: the extra matrix), first block,
 // blocks (1..tile_blocks, which is 4 or 8), -}: the arithmetic of gemm_q4k_experts_kernel.  w_up != null: silu(x . w^T) * (x . w_up^T) to y_xf / y_xs.
 int32_t dfl_gemm_rows_experts(dflash_ctx *ctx, const void *w, const void *w_extra, const void *w_up, const void *w_up_extra, size_t w_stride,

@@ -740,7 +740,7 @@ int32_t rows_launch(dflash_ctx *ctx, const RowsArgs &a, int64_t tiles, hipStream
 
 // Row blocks per tile: the largest tile (the fewest unpackings per product) unless a smaller one leaves less of the last
 // round of the chip idle: cost = rounds x (row blocks of a tile + what a tile costs besides).
-int rows_pick_rb(const dflash_ctx *ctx, int n_blocks, int n_ct, int most) {
+int rows_pick_rb(const dflash_ctx *ctx, int n_blocks, int n_ct, int most, int64_t *cost_of = nullptr) {
     int rb = most;
     int64_t best = -1;
     for (int r = most; r >= 2; r--) {
@@ -751,6 +751,7 @@ int rows_pick_rb(const dflash_ctx *ctx, int n_blocks, int n_ct, int most) {
             rb = r;
         }
     }
+    if (cost_of) *cost_of = best;
     return rb;
 }
 
@@ -758,7 +759,7 @@ int rows_pick_rb(const dflash_ctx *ctx, int n_blocks, int n_ct, int most) {
 // of the longest share, and the weights are read by fewer row tiles.  The tile by whole rounds (2 blocks) : this one.  Q4_K,
 // 100 rows, 5120 -> 6144, 4096 -> 5120 and 17408 -> 5120 on average 28.1 : 23.8 us (6 and 3 blocks); 200 rows, 4096 -> 5120 26.5 :
 // 23.2 (4).  Q6_K, 300 rows, 4096 -> 2048 27.4 : 20.2 (4).
-int rows_pick_split_rb(const dflash_ctx *ctx, int n_blocks, int n_ct, int most, int ranges) {
+int rows_pick_split_rb(const dflash_ctx *ctx, int n_blocks, int n_ct, int most, int ranges, int64_t *cost_of = nullptr) {
     int rb = 2;
     int64_t best = -1;
     for (int r = most; r >= 2; r--) {
@@ -771,7 +772,15 @@ int rows_pick_split_rb(const dflash_ctx *ctx, int n_blocks, int n_ct, int most, 
             rb = r;
         }
     }
+    if (cost_of) *cost_of = best;
     return rb;
+}
+
+// What decides on a product's launch besides its rows: the most row blocks of a tile (a twin product has second accumulators) and the ranges K falls into.
+int rows_most(const dfl_rows_plan &p) { return p.sums ? 8 : 4; }
+int rows_columns(int64_t n_out, int64_t pair_ffn) { return static_cast<int>(pair_ffn ? pair_ffn / 128 : (n_out + 255) / 256); }
+int rows_ranges(const dfl_rows_plan &p, int nb) {
+    return p.by_group ? std::max(1, static_cast<int>(static_cast<int64_t>(nb) * p.n_cut / p.total)) : p.n_cut;
 }
 
 template <typename Tile, bool kTwin, int kEpi>
@@ -794,6 +803,19 @@ int32_t rows_dispatch(dflash_ctx *ctx, const RowsArgs &a, int rb, int64_t tiles,
     return dfl_fail(ctx, DFLASH_ERR_UNSUPPORTED, "gemm_rows: %d row blocks per tile", rb);
 }
 }  // namespace
+
+double dfl_gemm_rows_cost(const dflash_ctx *ctx, const dfl_rows_plan &p, int64_t n_in, int64_t n_out, int32_t n_rows, int64_t pair_ffn) {
+    const int n_blocks = (n_rows + 15) / 16, n_ct = rows_columns(n_out, pair_ffn), nb = static_cast<int>(n_in / DFL_QK_K), ranges = rows_ranges(p, nb);
+    if (n_blocks < 1 || n_ct < 1) return 0.0;
+    const double twin = p.sums ? 1.0 : 2.0;  // (two MFMAs a product)
+    int64_t cost = 0;
+    const int rb = rows_pick_rb(ctx, n_blocks, n_ct, rows_most(p), &cost);
+    if (!pair_ffn && ranges > 1 && 2ll * n_ct * ((n_blocks + rb - 1) / rb) <= ctx->n_cu) {
+        rows_pick_split_rb(ctx, n_blocks, n_ct, rows_most(p), ranges, &cost);
+        return twin * nb * static_cast<double>(cost) / ranges;
+    }
+    return twin * nb * static_cast<double>(cost);
+}
 
 int32_t dfl_gemm_rows(dflash_ctx *ctx, const dfl_rows_plan &p, int32_t w_type, const void *w, const void *xf, void *xs, bool make_sums, float *y,
                       int64_t n_in, int64_t n_out, int32_t n_rows, int64_t pair_ffn, void *y_xf, void *y_xs, int y_kind, hipStream_t st) {
@@ -819,9 +841,9 @@ int32_t dfl_gemm_rows(dflash_ctx *ctx, const dfl_rows_plan &p, int32_t w_type, c
     a.y_xs = static_cast<uint8_t *>(y_xs);
     a.y_kind = y_kind;
     a.nb_out = static_cast<int>(pair_ffn / DFL_QK_K);
-    a.n_ct = static_cast<int>(pair_ffn ? pair_ffn / 128 : (n_out + 255) / 256);
+    a.n_ct = rows_columns(n_out, pair_ffn);
     const bool q6 = w_type == DFLASH_TYPE_Q6_K_TILED;
-    const int most = p.sums ? 8 : 4;  // (a twin product's second accumulators)
+    const int most = rows_most(p);
     int rb = rows_pick_rb(ctx, a.n_blocks, a.n_ct, most);
     a.n_rt = (a.n_blocks + rb - 1) / rb;
     int64_t tiles = static_cast<int64_t>(a.n_ct) * a.n_rt;
@@ -832,7 +854,7 @@ int32_t dfl_gemm_rows(dflash_ctx *ctx, const dfl_rows_plan &p, int32_t w_type, c
     }
     // Tiles for less than half the chip: K is shared by several workgroups, each range between two cuts on its own (as
     // many as there are at least in every tile group), where the workspace holds the partial products.
-    const int ranges = p.by_group ? std::max(1, static_cast<int>(static_cast<int64_t>(a.nb) * a.n_cut / a.total)) : a.n_cut;
+    const int ranges = rows_ranges(p, a.nb);
     const int most_ranges = p.by_group ? static_cast<int>((static_cast<int64_t>(a.nb) * a.n_cut + a.total - 1) / a.total) + 1 : a.n_cut;
     if (2 * tiles <= ctx->n_cu && ranges > 1) {
         // The whole-K kernel does the few blocks of a short prompt in one launch, one block after the other: 1.5 us each past

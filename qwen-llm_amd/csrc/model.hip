@@ -981,18 +981,6 @@ int prefill_group_blocks() {
     return std::max(0, std::min(kMaxGroupRows / 16, v));
 }
 
-// Rows of the next pass where `left` are to come from position `at` on and a pass holds `most`: full passes, but a prompt of two, the
-// second of an eighth at least, goes as two of the same size: the many-row products of few rows leave CUs idle or their tiles half full.
-// (A shorter rest is cheap by itself, and two halves would lose more of the expert tiles' fill.)  ms of full passes : equal ones, 2310, 2500,
-// 2800 and 3000 tokens: five layers of the 27B shape 9.33 : 8.15, 9.90 : 9.00, 10.56 : 9.99, 11.10 : 10.71; eight of the 35B-A3B shape 8.58 :
-// 8.33, 8.95 : 8.71, 9.72 : 9.50, 10.10 : 9.65; eight of a 1024-wide one 3.73 : 3.75, 4.23 : 3.94, 4.52 : 4.48, 4.73 : 4.70.  2100 tokens (52 behind
-// a full pass) 8.30 : 7.79, 7.16 : 7.81, 3.21 : 3.45.  Three passes, 4380 tokens, 16.96 : 15.93, 15.44 : 15.90, 7.79 : 8.09: there a
-// pass of equal size crosses the length from which the attention goes by splits.
-int32_t prefill_pass_rows(int32_t most, int32_t left, int64_t at) {
-    if (at || left < most + most / 8 || left > 2 * most) return std::min(most, left);
-    return ((left + 1) / 2 + 15) / 16 * 16;
-}
-
 // Sets the group scratch up; leaves it empty (no error) where the shape is not one the grouped path takes or the memory
 // is not there.
 void prefill_group_alloc(dflash_session *s, PrefillGroup *g) {
@@ -1557,6 +1545,41 @@ bool prefill_group_takes(const dflash_ctx *ctx, const dflash_model *model, const
     return true;
 }
 
+// What a pass of that many rows costs a dense model in its projections, by the measure that picks their tiles.
+double prefill_pass_cost(const dflash_ctx *ctx, const dflash_model *model, int32_t rows) {
+    const dflash_model_cfg &c = model->cfg;
+    const int64_t H = c.hidden, q_dim = static_cast<int64_t>(c.n_q) * c.head_dim, kv_dim = static_cast<int64_t>(c.n_kv) * c.head_dim;
+    double cost = 0.0;
+    for (int il = 0; il < c.n_layers; il++) {
+        const LayerRows r = layer_rows(ctx, c, model->layers[il]);
+        cost += dfl_gemm_rows_cost(ctx, r.qkv, H, q_dim + 2 * kv_dim, rows, 0) + dfl_gemm_rows_cost(ctx, r.wo, q_dim, H, rows, 0) +
+                dfl_gemm_rows_cost(ctx, r.gate_up, H, 2ll * c.ffn, rows, c.ffn) + dfl_gemm_rows_cost(ctx, r.down, c.ffn, H, rows, 0);
+    }
+    return cost;
+}
+// Rows of the next pass where `left` are to come from position `at` on and a pass holds `most`: full passes, but where two are left and the
+// projections take at least 1 % less of the chip's rounds in two of the same size, those.  (A rest's products leave CUs idle or their tiles
+// half full; so do two halves' where a matrix has few column tiles, or just more than a round of them.)  ms of full passes : equal ones, five
+// dense layers from position 0, in brackets what the rounds say, in percent:
+//   equal  5120 / 17408, 2100, 2310, 2500 and 3000 tokens 7.28 : 6.96 (-2), 8.33 : 7.57 (-6), 8.69 : 8.21 (-5), 10.00 : 9.79 (-1)
+//          5120 / 8192, 2310 and 2500 5.49 : 5.04 (-3), 5.73 : 5.46 (-3)     4608 / 12288, 2500 6.40 : 6.03 (-4)
+//   full   1024 / 3072, 2100, 2310, 2500 and 3000 1.62 : 1.89 (+46), 1.92 : 2.03 (+37), 2.18 : 2.16 (+32), 2.45 : 2.57 (+19)
+//          2048 / 6144 2.70 : 3.03 (+35), 3.07 : 3.26 (+22), 3.47 : 3.42 (+15), 3.86 : 4.02 (+6)
+//          8192 / 22016 13.39 : 14.44 (+16), 15.24 : 15.59 (+8), 16.07 : 16.36 (+3), 19.03 : 19.76 (+4)
+//          5120 / 17408, 3500 11.66 : 11.88 (+5); and where they say too little: 4096 / 14336, 2310 6.13 : 5.74 (0)
+// A mixture's experts fill their tiles either way: eight layers of the 35B-A3B shape 6.59 : 7.17, 7.53 : 7.51, 7.99 : 7.98, 9.03 : 8.96.
+// Behind a context the same keys come on top, over fewer rows at once: 5120 / 17408, 2310 and 2500 tokens behind 1024 positions 8.66 : 8.04,
+// 9.19 : 8.66, behind 2048 8.92 : 8.57, 9.48 : 9.29, behind 4096 9.62 : 9.69, 10.37 : 10.37, behind 8192 11.15 : 11.82, 11.92 : 12.44;
+// so: up to the positions of two passes.
+int32_t prefill_pass_rows(const dflash_ctx *ctx, const dflash_model *model, int32_t most, int32_t left, int64_t at) {
+    if (left <= most) return left;
+    if (model->cfg.n_expert || at + left > 2ll * most) return most;
+    const int32_t half = ((left + 1) / 2 + 15) / 16 * 16;
+    const double full = prefill_pass_cost(ctx, model, most) + prefill_pass_cost(ctx, model, left - most);
+    const double equal = prefill_pass_cost(ctx, model, half) + prefill_pass_cost(ctx, model, left - half);
+    return equal <= 0.99 * full ? half : most;
+}
+
 // One group of n rows (positions start .. start + n - 1) through every layer, on `st`: K/V rows into the session's
 // cache, tapped residuals into hidden_capture.  A row gets the bits verify_enqueue gives it in its own 16-row block:
 // every operator here is that block's operator over more rows.
@@ -1700,7 +1723,7 @@ int32_t dflash_prefill_blocks(dflash_ctx *ctx, const dflash_model *model, dflash
         // rows of many blocks per pass (see PrefillGroup); the caller's stream alone
         const size_t cap_row = static_cast<size_t>(std::max(n_taps, 0)) * c.hidden;
         for (int32_t t0 = 0, n; t0 < n_tokens; t0 += n) {
-            n = prefill_pass_rows(p->group.rows, n_tokens - t0, start + t0);
+            n = prefill_pass_rows(ctx, model, p->group.rows, n_tokens - t0, start + t0);
             if ((rc = prefill_group_enqueue(ctx, model, s, p->group, tokens + t0, n, start + t0, tap_layers, n_taps,
                                             hidden_capture ? hidden_capture + static_cast<size_t>(t0) * cap_row : nullptr,
                                             static_cast<hipStream_t>(stream)))) {
@@ -1787,7 +1810,7 @@ int32_t dflash_prefill_prompt(dflash_ctx *ctx, const dflash_model *model, dflash
     int32_t body = 0;
     bool tail_group = n_tokens > 16 && start + n_tokens <= 0x7fffffffll && prefill_group_takes(ctx, model, g);
     if (tail_group)
-        for (body = 0; n_tokens - body > g.rows;) body += prefill_pass_rows(g.rows, n_tokens - body, start + body);
+        for (body = 0; n_tokens - body > g.rows;) body += prefill_pass_rows(ctx, model, g.rows, n_tokens - body, start + body);
     tail_group = tail_group && n_tokens - body > 16;
     if (!tail_group) body = (n_tokens - 1) / 16 * 16;
     if (body && (rc = dflash_prefill_blocks(ctx, model, s, tokens, body, start, tap_layers, n_taps, hidden_capture, stream))) return rc;

@@ -269,11 +269,13 @@ def test_a_prompt_in_one_call_equals_its_blocks_and_their_last_one(ctx, shape, a
     one.close()
 
 
-@pytest.mark.parametrize("shape,rows", [("experts", 2303), ("experts", 2304), ("narrow", 3011), ("narrow", 4361)])
-def test_prompts_of_several_passes_equal_block_by_block(ctx, shape, rows):
-    """More rows than a pass holds (2048): a full pass and a short rest, two passes of the same size, full passes and a rest, in both calls."""
-    test_continued_prefill_equals_block_by_block(ctx, shape, 0, rows)
-    test_a_prompt_in_one_call_equals_its_blocks_and_their_last_one(ctx, shape, True, rows, [0], 0)
+@pytest.mark.parametrize("shape,rows,head", [("experts", 2303, 0), ("experts", 2304, 0), ("narrow", 3011, 0), ("narrow", 4361, 0), ("wide", 2310, 0),
+                                             ("wide", 2505, 37)])
+def test_prompts_of_several_passes_equal_block_by_block(ctx, shape, rows, head):
+    """More rows than a pass holds (2048): a full pass and a rest, full passes and a rest, two passes of the same size (the wide shape, from position
+    0 and behind a context), in both calls."""
+    test_continued_prefill_equals_block_by_block(ctx, shape, head, rows)
+    test_a_prompt_in_one_call_equals_its_blocks_and_their_last_one(ctx, shape, True, rows, [0], head)
 
 
 def test_a_prompt_in_one_call_keeps_the_guards(ctx):
