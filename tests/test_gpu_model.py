@@ -638,7 +638,8 @@ def test_graph_replay_is_bit_identical_to_launch_by_launch(ctx, target):
 @pytest.mark.parametrize("kind", ["dense", "moe"])
 def test_captured_rows_by_the_norms_equal_those_of_their_own_launch(ctx, kind):
     """A tapped layer's residual is written by the kernel that has its rows in registers (the next norm, or the experts' combine); tapped
-    twice, or into a buffer that is not 16-byte aligned, by a launch of its own; the last layer's too, with and without the head: the same rows."""
+    twice, or into a buffer that is not 16-byte aligned, by a launch of its own; the last layer's too, with and without the head: the same rows,
+    in a block and in a prompt's group, and nothing beside them."""
     import ctypes as C
     import torch
 
@@ -646,27 +647,51 @@ def test_captured_rows_by_the_norms_equal_those_of_their_own_launch(ctx, kind):
            dfl.ModelConfig(n_layers=3, hidden=512, n_q=4, n_kv=2, head_dim=128, ffn=0, vocab=1024, n_expert=8, n_expert_used=2, ffn_expert=256, ffn_shared=256))
     model = dfl.TargetModel(ctx, cfg, dfl.synth_target_weights_blocks(cfg, 9))
     tokens = np.random.default_rng(5).integers(0, cfg.vocab, 40).tolist()
-    rows = {}
+    rows, launched = {}, {}
     for name, taps, offset, head in (("own", [0, 1, 2], 0, True), ("off", [0, 1, 2], 1, True), ("twice", [0, 0, 1, 2], 0, True), ("no head", [0, 1, 2], 0, False)):
         sess = dfl.Session(ctx, model, 64, taps)
         n_taps, n = len(taps), 13
-        buf = torch.zeros(n * n_taps * cfg.hidden + 4, device="cuda")
+        taps_c = (C.c_int32 * n_taps)(*taps)
         arg = torch.zeros(16, dtype=torch.int32, device="cuda")
         host = (C.c_int32 * 16)()
-        rc = sess._L.dflash_verify_block(ctx._h, C.byref(model.c), sess._h, (C.c_int32 * n)(*tokens[:n]), n, 0, (C.c_int32 * n_taps)(*taps), n_taps,
+
+        def buffer(count):  # (and what stands ahead of it and behind it)
+            return torch.full((count * n_taps * cfg.hidden + 8,), -7.0, device="cuda")
+
+        def captured(buf, count):
+            end = offset + count * n_taps * cfg.hidden
+            assert torch.all(buf[:offset] == -7.0) and torch.all(buf[end:] == -7.0)
+            got = buf[offset:end].view(count, n_taps, cfg.hidden)
+            if name == "twice":
+                assert torch.equal(got[:, 0], got[:, 1])
+                got = got[:, 1:]
+            return got.clone()
+
+        buf = buffer(n)
+        rc = sess._L.dflash_verify_block(ctx._h, C.byref(model.c), sess._h, (C.c_int32 * n)(*tokens[:n]), n, 0, taps_c, n_taps,
                                          arg.data_ptr() if head else None, None, buf.data_ptr() + 4 * offset, None, host if head else None, None)
         assert rc == 0
         torch.cuda.synchronize()
-        got = buf[offset:offset + n * n_taps * cfg.hidden].view(n, n_taps, cfg.hidden)
         if head:
             assert list(host[:n]) == arg[:n].tolist()
-        if name == "twice":
-            assert torch.equal(got[:, 0], got[:, 1])
-            got = got[:, 1:]
-        rows[name] = got.clone()
-        # a prompt's group: the same rows, and a buffer off the alignment
-        many = sess.prefill_prompt(tokens[n:], n)[0]
-        rows[name + " group"] = many[:, 1:] if name == "twice" else many
+        rows[name] = captured(buf, n)
+        # a prompt's group, with the head of its last block and without: the rows of the blocks
+        rest, last = len(tokens) - n, C.c_int32()
+        toks = (C.c_int32 * rest)(*tokens[n:])
+        blocks = [sess.encode_packed_verify_layer_major(tokens[i:i + 16], i) for i in range(n, len(tokens), 16)]
+        rows[name + " blocks"] = torch.cat([o.hidden_capture for o in blocks])[:, 1 if name == "twice" else 0:]
+        sess.encode_restore_after_partial_accept(n, rest, 0)
+        buf = buffer(rest)
+        ctx.set_kernel_timing(1)
+        args = [ctx._h, C.byref(model.c), sess._h, toks, rest, C.c_int64(n), taps_c, n_taps, C.c_void_p(buf.data_ptr() + 4 * offset)]
+        rc = (sess._L.dflash_prefill_prompt(*args, C.byref(last), C.c_void_p()) if head else sess._L.dflash_prefill_blocks(*args, C.c_void_p()))
+        torch.cuda.synchronize()
+        launched[name] = ctx.kernel_timing(ctx.T_ATTN)[1]
+        ctx.set_kernel_timing(0)
+        assert rc == 0 and (not head or last.value == blocks[-1].argmax_host[-1])
+        rows[name + " group"] = captured(buf, rest)
         sess.close()
-    for name in ("off", "twice", "no head"):
-        assert torch.equal(rows["own"], rows[name]) and torch.equal(rows["own group"], rows[name + " group"]), name
+    # (both blocks' rows went through the layers together: an attention launch a layer)
+    assert set(launched.values()) == {cfg.n_layers}
+    for name in rows:
+        assert torch.equal(rows["own" if " " not in name or name == "no head" else "own blocks"], rows[name]), name
