@@ -2,7 +2,9 @@
 prompt's rows against their own blocks bit for bit.
 
 A unit is sixteen columns; what is left over when each of 256 workgroups has as many units is cut into 16, 8, 4 or 2 parts by weight rows, or not
-at all.  The shapes bring each cut, none left over, two rounds of units, and K whose last chunk of four super-blocks is not full."""
+at all.  The shapes bring each cut, none left over, two rounds of units, K whose last chunk of four super-blocks is not full, and K of up to
+32 super-blocks, the most that a norm leaves in fragment order.  Each is one that the launch takes: of the layer's products only down has a
+reduction then."""
 import numpy as np
 import pytest
 import torch
@@ -11,7 +13,7 @@ import qwen_llm_amd as dfl
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = [(2304, 4352), (2304, 4608), (2304, 5120), (2304, 6144), (2560, 7168), (2304, 8192), (1280, 12544), (1280, 28928)]
+SHAPES = [(2304, 4352), (2304, 4608), (2304, 5120), (2304, 6144), (2560, 7168), (2304, 8192), (1280, 12544), (1280, 28928), (5120, 4608), (8192, 4608)]
 
 
 @pytest.fixture(scope="module")
@@ -19,6 +21,15 @@ def ctx():
     c = dfl.Context(0, workspace_bytes=256 << 20)
     yield c
     c.close()
+
+
+def verified(ctx, sess, tokens, at):
+    """The tapped rows of a block, and how many of its products were followed by a reduction."""
+    ctx.set_kernel_timing(1)
+    out = sess.encode_packed_verify_layer_major(tokens, at, want_head=False)
+    n = ctx.kernel_timing(ctx.T_REDUCE)[1]
+    ctx.set_kernel_timing(0)
+    return out.hidden_capture, n
 
 
 @pytest.mark.parametrize("hidden,ffn", SHAPES)
@@ -32,7 +43,8 @@ def test_wide_ffn_matches_oracle_and_the_prompts_rows(ctx, oracle, hidden, ffn):
     tokens = np.random.default_rng(ffn).integers(0, cfg.vocab, 40).tolist()
     rows = []
     for at, n in ((0, 16), (16, 16), (32, 1), (33, 7)):
-        got = one.encode_packed_verify_layer_major(tokens[at:at + n], at).hidden_capture
+        got, reductions = verified(ctx, one, tokens[at:at + n], at)
+        assert reductions == 1
         _, want = oracle.target_verify(omodel, ostate, tokens[at:at + n], at, [0])
         rows.append(got)
         # f16 operands (2^-11) in the six products that a row passes through: 5e-3 in the 2-norm, 3e-2 in an element (as for whole stacks)
@@ -44,6 +56,28 @@ def test_wide_ffn_matches_oracle_and_the_prompts_rows(ctx, oracle, hidden, ffn):
     assert torch.equal(got, torch.cat(rows))
     one.close()
     many.close()
+
+
+@pytest.mark.parametrize("hidden,ffn", [(2304, 4608), (2560, 9728), (5120, 4608)])
+def test_one_launch_is_as_near_the_oracle_as_separate_products(ctx, oracle, hidden, ffn):
+    """One f32 sum over K in place of several that are added, of the same f16 operands, and silu(gate) * up held in the f16 that down rounds it to:
+    what differs is f32 rounding, 2^-24 a step, next to the operands' 2^-11 that both have: their errors agree to a percent."""
+    cfg = dfl.ModelConfig(n_layers=1, hidden=hidden, n_q=4, n_kv=2, head_dim=128, ffn=ffn, vocab=512)
+    w = dfl.synth_target_weights_blocks(cfg, 37)
+    omodel, _keep = oracle.build_model(cfg.as_dict(), w)
+    tokens = np.random.default_rng(ffn).integers(0, cfg.vocab, 16).tolist()
+    _, want = oracle.target_verify(omodel, oracle.TargetState(cfg.as_dict(), 64), tokens, 0, [0])
+    errors, model = [], dfl.TargetModel(ctx, cfg, w)
+    up = ctx.repack_q4k_tiled(torch.from_numpy(w["layers"][0]["up"][1]).cuda(), hidden, ffn)
+    for one_launch in (True, False):
+        if not one_launch:  # up somewhere else than behind gate
+            model.c.layers[0].up.data = up.data_ptr()
+        sess = dfl.Session(ctx, model, 64, [0])
+        got, reductions = verified(ctx, sess, tokens, 0)
+        assert (reductions == 1) == one_launch
+        errors.append(np.linalg.norm(got.cpu().numpy().astype(np.float64) - want))
+        sess.close()
+    assert errors[0] <= 1.01 * errors[1], errors
 
 
 @pytest.mark.parametrize("adjacent", [True, False], ids=["one launch", "separate products"])
