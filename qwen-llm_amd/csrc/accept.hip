@@ -73,7 +73,8 @@ __device__ __forceinline__ Top2 top2_wave(Top2 t) {  // over a wave, in every la
 }
 // What bounds it and the launch that follows it: their chains (the merges are of maxima and of the lowest token among equals, so any order
 // gives the same).  All of a thread's tokens are asked for at once, waves merge by lane moves; the last launch has a chunk a lane.
-// 6.4 + 5.0 us a 16 x 151936 block with a tree through LDS and one thread a row behind it, 5.0 + 2.7 now.
+// With a tree through LDS and one thread a row behind it : this, medians of traces: a 16 x 151936 block by itself 6.0 + 4.6 : 6.5 + 2.6 us, one row
+// 5.0 + 3.4 : 4.9 + 1.8; at the end of a verify of 16 rows 6.5 + 4.8 : 6.8 + 4.2.
 __global__ void __launch_bounds__(kSelThreads)
     top2_chunk_kernel(const float *__restrict__ logits, int64_t vocab, int64_t stride, Top2 *__restrict__ part) {
     __shared__ Top2 sh[kSelThreads / 64];
